@@ -356,16 +356,12 @@ hipError_t launch_k_sliced(GemmF32Args args, size_t slices, size_t k_steps, int 
     void *workspace = nullptr;
     hipError_t rc = stream_workspace(stream, slices * plane * sizeof(float), &workspace);
     if (rc != hipSuccess) return rc;
-    SliceReduceArgs reduce;
-    reduce.partial = static_cast<const float *>(workspace);
-    reduce.C = args.C;
-    reduce.bias = args.bias;
-    reduce.residual = args.residual;
-    reduce.plane = plane;
-    reduce.N = args.N;
-    reduce.slices = static_cast<int>(slices);
-    reduce.scale = args.scale;
-    reduce.activation = args.activation;
+    GemmEpilogue epilogue;
+    epilogue.scale = args.scale;
+    epilogue.bias = args.bias;
+    epilogue.residual = args.residual;
+    epilogue.activation = args.activation;
+    float *const out = args.C;
     args.C = static_cast<float *>(workspace);
     args.bias = nullptr;
     args.residual = nullptr;
@@ -374,13 +370,7 @@ hipError_t launch_k_sliced(GemmF32Args args, size_t slices, size_t k_steps, int 
     args.slice_k = static_cast<int>(steps_per_slice) * bk;
     rc = launch(args, static_cast<unsigned>(slices));
     if (rc != hipSuccess) return rc;
-    if (slices >= 32 && plane <= 65536)
-        hipLaunchKernelGGL(gemm_f32_slice_reduce_wide_kernel, dim3(static_cast<unsigned>((plane + 15) / 16)), dim3(256), 0, stream,
-                           reduce);
-    else
-        hipLaunchKernelGGL(gemm_f32_slice_reduce_kernel, dim3(static_cast<unsigned>((plane + 255) / 256)), dim3(256), 0, stream,
-                           reduce);
-    return hipGetLastError();
+    return launch_f32_slice_reduce(args.M, args.N, slices, static_cast<const float *>(workspace), out, epilogue, stream);
 }
 
 template <int BM, int BN, int WM, int WN>
@@ -896,14 +886,70 @@ hipError_t launch_pad_f32_pair(const PadJobF32 &first, const PadJobF32 &second, 
 
 }  // namespace
 
+hipError_t launch_f32_slice_reduce(size_t m, size_t n, size_t slices, const float *partial, float *out, const GemmEpilogue &epilogue,
+                                   hipStream_t stream)
+{
+    SliceReduceArgs reduce;
+    reduce.partial = partial;
+    reduce.C = out;
+    reduce.bias = epilogue.bias;
+    reduce.residual = epilogue.residual;
+    reduce.plane = m * n;
+    reduce.N = static_cast<int>(n);
+    reduce.slices = static_cast<int>(slices);
+    reduce.scale = epilogue.scale;
+    reduce.activation = epilogue.activation;
+    if (slices >= 32 && reduce.plane <= 65536)
+        hipLaunchKernelGGL(gemm_f32_slice_reduce_wide_kernel, dim3(static_cast<unsigned>((reduce.plane + 15) / 16)), dim3(256), 0, stream,
+                           reduce);
+    else
+        hipLaunchKernelGGL(gemm_f32_slice_reduce_kernel, dim3(static_cast<unsigned>((reduce.plane + 255) / 256)), dim3(256), 0, stream,
+                           reduce);
+    return hipGetLastError();
+}
+
+namespace {
+
+// What the f32 matrix-core kernels below need for a product, in µs: within a fifth of what was measured over some hundred
+// shapes from 64 to 4096.  On whole 16-wide k-tiles with aligned rows they run at 100 to 115 TFLOP/s beside a launch's
+// fixed time.  Other shapes take the general kernel, which walks k at 0.6 (aligned rows) or 0.75 µs a k-tile however few tiles there are, unless
+// it can slice k over workgroups; a prepacked B is unpacked for it first.
+double f32_kernels_us(size_t m, size_t n, size_t k, bool lhs_transposed, bool rhs_packed, const float *lhs, const float *rhs, bool scratch_free)
+{
+    const double flops = 2.0 * m * n * k;
+    const bool aligned = aligned16(lhs) && aligned16(rhs) && (lhs_transposed ? m : k) % 4 == 0 && (rhs_packed ? k : n) % 4 == 0;
+    if (aligned && k % 16 == 0) return lhs_transposed ? 8.0 + flops / 118.0e6 : rhs_packed ? 5.0 + flops / 105.0e6 : 4.0 + flops / 108.0e6;
+    const double k_tiles = static_cast<double>((k + 15) / 16);
+    const size_t tiles = ((m + 63) / 64) * ((n + 63) / 64);
+    if (!rhs_packed && scratch_free && tiles <= 128 && k_tiles >= 32) return 12.0 + flops / 45.0e6;
+    const double unpack = rhs_packed ? 8.0 * k * n / 5.0e6 : 0.0;
+    return 5.0 + unpack + std::max(flops / (aligned ? 80.0e6 : 60.0e6), (aligned ? 0.6 : 0.75) * k_tiles) + flops / 200.0e6;
+}
+
+hipError_t launch_gemm_f32_native(size_t m, size_t n, size_t k, bool lhs_transposed, const float *lhs, const float *rhs, float *out,
+                                  const GemmEpilogue &epilogue, hipStream_t stream, bool scratch_free);
+
+}  // namespace
+
 hipError_t launch_gemm_f32(size_t m, size_t n, size_t k, bool lhs_transposed, const float *lhs,
                            const float *rhs, float *out, const GemmEpilogue &epilogue, hipStream_t stream, bool scratch_free)
 {
     if (m == 0 || n == 0) return hipSuccess;
     if (!lhs_transposed && gemv_f32_applies(m, n, k, lhs, rhs)) return launch_gemv_f32(m, n, k, lhs, rhs, out, epilogue, stream);
     if (lhs_transposed && scratch_free && gemv_t_f32_applies(m, n, k)) return launch_gemv_t_f32(m, n, k, lhs, rhs, out, epilogue, stream);
-    // A k that is not a multiple of 4 (a vocabulary of 50257 as the reduction of a backward product): the rows of A start
-    // at odd addresses, which the direct-to-LDS kernels do not take, and the general kernel runs at about 0.6 of their
+    if (gemm_f32_split_applies(m, n, k, f32_kernels_us(m, n, k, lhs_transposed, false, lhs, rhs, scratch_free), scratch_free)) {
+        const hipError_t rc = launch_gemm_f32_split(m, n, k, lhs_transposed, lhs, false, rhs, out, epilogue, stream, scratch_free);
+        if (!scratch_unavailable(rc)) return rc;
+    }
+    return launch_gemm_f32_native(m, n, k, lhs_transposed, lhs, rhs, out, epilogue, stream, scratch_free);
+}
+
+namespace {
+
+hipError_t launch_gemm_f32_native(size_t m, size_t n, size_t k, bool lhs_transposed, const float *lhs, const float *rhs, float *out,
+                                  const GemmEpilogue &epilogue, hipStream_t stream, bool scratch_free)
+{
+    // A k that is not a multiple of 4 in a product too large for the split kernels: the rows of A start at odd addresses, which the direct-to-LDS kernels do not take, and the general kernel runs at about 0.6 of their
     // speed (1024×1024×4099: 140 µs against 80 µs at 4096).  Where the product is large against its operands, copies
     // of A and B zero-padded along k to a multiple of 16 (exact: the new terms are 0·0) go into the stream's second
     // scratch buffer, one launch for both, and the product runs on them.
@@ -925,7 +971,7 @@ hipError_t launch_gemm_f32(size_t m, size_t n, size_t k, bool lhs_transposed, co
         rc = launch_pad_f32_pair(lhs_transposed ? job(k, m, k_pad, m, lhs, a_pad) : job(m, k, m, k_pad, lhs, a_pad),
                                  job(k, n, k_pad, n, rhs, b_pad), stream);
         if (rc != hipSuccess) return rc;
-        return launch_gemm_f32(m, n, k_pad, lhs_transposed, a_pad, b_pad, out, epilogue, stream, true);
+        return launch_gemm_f32_native(m, n, k_pad, lhs_transposed, a_pad, b_pad, out, epilogue, stream, true);
     }
     // An A of 2 GiB or more (the direct-to-LDS kernels address their operands through 32-bit byte offsets): row blocks
     // of A are independent products, so the launch is cut into blocks that fit and each takes the fast path.
@@ -935,7 +981,7 @@ hipError_t launch_gemm_f32(size_t m, size_t n, size_t k, bool lhs_transposed, co
             const size_t rows = std::min(block, m - row);
             GemmEpilogue part = epilogue;
             if (part.residual) part.residual += row * n;
-            const hipError_t rc = launch_gemm_f32(rows, n, k, false, lhs + row * k, rhs, out + row * n, part, stream, scratch_free);
+            const hipError_t rc = launch_gemm_f32_native(rows, n, k, false, lhs + row * k, rhs, out + row * n, part, stream, scratch_free);
             if (rc != hipSuccess) return rc;
         }
         return hipSuccess;
@@ -990,6 +1036,8 @@ hipError_t launch_gemm_f32(size_t m, size_t n, size_t k, bool lhs_transposed, co
     return launch_tile<64, 64, 2, 2>(args, lhs_transposed, vec, stream);
 }
 
+}  // namespace
+
 hipError_t launch_gemm_f32_batched(size_t batch, size_t m, size_t n, size_t k, bool lhs_transposed, const float *lhs,
                                    size_t lhs_stride, const float *rhs, float *out, size_t out_stride, hipStream_t stream)
 {
@@ -1038,6 +1086,10 @@ hipError_t launch_gemm_f32_packed(size_t m, size_t n, size_t k, const float *lhs
                                   const GemmEpilogue &epilogue, hipStream_t stream)
 {
     if (m == 0 || n == 0) return hipSuccess;
+    if (gemm_f32_split_applies(m, n, k, f32_kernels_us(m, n, k, false, true, lhs, packed_rhs, true), true)) {
+        const hipError_t rc = launch_gemm_f32_split(m, n, k, false, lhs, true, packed_rhs, out, epilogue, stream, true);
+        if (!scratch_unavailable(rc)) return rc;
+    }
     const bool ring_ok = k >= 16 && k % 16 == 0 && aligned16(lhs) && aligned16(packed_rhs) && m * k * 4 < (1ull << 31) &&
                          k * n * 4 < (1ull << 31);
     if (!ring_ok) {

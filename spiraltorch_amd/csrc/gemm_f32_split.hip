@@ -1,0 +1,564 @@
+// Large f32 products on the bf16 matrix cores: every f32 operand value is written as the sum of three bf16 values,
+// x = hi + mid + lo (hi = bf16(x), mid = bf16(x - hi), lo = x - hi - mid, each difference exact: 3 × 8 mantissa bits hold
+// all 24 of an f32), and a product a·b is accumulated in f32 from six of the nine piece products,
+//     lo·hi, mid·hi, mid·mid, hi·mid, hi·lo, hi·hi.
+// What is left out (mid·lo, lo·mid, lo·lo) is below 2^-26 of |a·b|, a quarter of what rounding one f32 product costs.
+// v_mfma_f32_32x32x16_bf16 multiplies exactly and adds into f32 accumulators, and the result carries one rounding of the
+// large sum per sixteen terms where the f32 instruction rounds after every term, so it is closer to the exact sum than the
+// f32 matrix cores' (rms error against float64, N(0,1) operands, of the result's rms: k = 768 1.6e-7 against 5.0e-7,
+// k = 3072 1.6e-7 to 2.3e-7 against 5.0e-7 to 7.0e-7, k = 4096 4.0e-7 against 1.1e-6).
+//
+// Six bf16 products take 6/16 of the f32 instruction's time at their nominal rates.  What bounds the product kernel is the
+// power the matrix cores draw on random operands: a 32×32×16 instruction takes 21 ns of a SIMD here, 19 in a loop of
+// nothing else, 13 on zeros; then come the splitting pass (memory: 4 bytes read and 6 written a value, ~6 TB/s), and 11 µs
+// of launches, first loads and stores.  Measured with the pass, f32 matrix cores -> here: 4096³ 1014 -> 615 µs
+// (223 TFLOP/s), 1576×3072×768 70 -> 48, A stored k×m 3072×768×1576 100 -> 62, B prepacked 2384×1120×3708 243 -> 133,
+// and where rows are unaligned or k is no multiple of 16 853×1399×1747 114 -> 43, 182×425×2895 161 -> 20 µs.
+//
+// Values for which the three pieces are not exact (non-finite, 2^127 and more, whole operand rows below 2^-100) are found
+// by the splitting pass; the tiles they touch are computed with f32 multiply-adds from the original operands.
+#include <algorithm>
+#include <type_traits>
+
+#include "device_math.h"
+#include "kernels.h"
+
+namespace sthip {
+
+namespace {
+
+typedef __attribute__((address_space(3))) void *lds_void_ptr;
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+
+#define ST_SPLIT_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (7 << 4) | (15 << 8) | ((((n) >> 4) & 3) << 14))
+#define ST_SPLIT_FENCE() __builtin_amdgcn_sched_barrier(0)
+
+// ---- the splitting pass ------------------------------------------------------------------------------------------
+// An operand of `rows` rows along a reduction of `k` terms becomes blocks of 32 rows × 16 terms.  A block is three
+// fragments (hi, mid, lo) of 1 KB, each in the order the matrix instruction wants its operand: lane l holds row l % 32,
+// terms 8·(l / 32) .. + 7.  Block (rb, ks) starts at (rb·ksteps + ks)·3 KB; rows and terms past the end are zeros, so the
+// product kernel needs no edge cases, and any m, n, k and alignment of the operands is served alike.
+//
+// Beside every pair of blocks along k, 16 bytes of status: bit r of word 0 is set when row r holds a non-zero value
+// there, bit r of word 1 when it holds one of at least 2^-100, word 2 is non-zero when some value is 2^127 or more or not
+// finite.
+struct SplitJob {
+    const float *src;
+    unsigned char *blocks;
+    uint4 *status;
+    int rows, k, ld;
+    int transposed;  // 0: src[row·ld + term], 1: src[term·ld + row]
+    int ksteps;  // ceil(k / 16), rounded up to even
+    unsigned groups_k;  // workgroups along k: 128 terms each (32 when transposed)
+};
+
+__device__ __forceinline__ float4 load4_guarded(const float *row, int first, int limit)
+{
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (first + 4 <= limit) {
+        const f32x4_a4 w = *reinterpret_cast<const f32x4_a4 *>(row + first);
+        v = make_float4(w[0], w[1], w[2], w[3]);
+    } else {
+        if (first + 0 < limit) v.x = row[first + 0];
+        if (first + 1 < limit) v.y = row[first + 1];
+        if (first + 2 < limit) v.z = row[first + 2];
+    }
+    return v;
+}
+
+// A workgroup splits 32 rows × 128 terms (128 rows × 32 terms when the source runs along the rows): 512-byte pieces of the
+// source go through LDS, a wavefront then owns two neighbouring blocks and writes their 6 KB contiguously.
+__global__ __launch_bounds__(256) void split_operands_kernel(SplitJob first, SplitJob second, unsigned first_groups)
+{
+    constexpr int STRIDE = 132;
+    __shared__ __attribute__((aligned(16))) float tile[32 * STRIDE];
+    const bool is_first = blockIdx.x < first_groups;
+    const SplitJob &job = is_first ? first : second;
+    const unsigned group = blockIdx.x - (is_first ? 0u : first_groups);
+    const int gk = static_cast<int>(group % job.groups_k), gr = static_cast<int>(group / job.groups_k);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int li = lane & 31, lh = lane >> 5;
+    const int r0 = gr * (job.transposed ? 128 : 32), k0 = gk * (job.transposed ? 32 : 128);
+    {
+        const int line0 = job.transposed ? k0 : r0, lines = job.transposed ? job.k : job.rows;
+        const int along0 = (job.transposed ? r0 : k0) + (tid & 31) * 4, along = job.transposed ? job.rows : job.k;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int line = i * 8 + (tid >> 5);
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (line0 + line < lines) v = load4_guarded(job.src + static_cast<size_t>(line0 + line) * job.ld, along0, along);
+            *reinterpret_cast<float4 *>(&tile[line * STRIDE + (tid & 31) * 4]) = v;
+        }
+    }
+    __syncthreads();
+    const int rb = job.transposed ? gr * 4 + wave : gr;
+    const int pair = job.transposed ? gk : gk * 4 + wave;
+    if (rb * 32 >= job.rows || pair * 2 >= job.ksteps) return;
+    unsigned nonzero = 0, ordinary = 0, wild = 0;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        const int ks = pair * 2 + half;
+        float x[8];
+        if (job.transposed) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = tile[(half * 16 + lh * 8 + e) * STRIDE + wave * 32 + li];
+        } else {
+            const float *src = &tile[li * STRIDE + (wave * 2 + half) * 16 + lh * 8];
+            const float4 v0 = *reinterpret_cast<const float4 *>(src), v1 = *reinterpret_cast<const float4 *>(src + 4);
+            x[0] = v0.x; x[1] = v0.y; x[2] = v0.z; x[3] = v0.w; x[4] = v1.x; x[5] = v1.y; x[6] = v1.z; x[7] = v1.w;
+        }
+        uint32_t piece[3][4];
+        bool nz = false, ord = false;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float a = x[2 * e], b = x[2 * e + 1];
+            piece[0][e] = pack_bf16x2_rne(a, b);
+            const float ra = a - __uint_as_float(piece[0][e] << 16), rb_ = b - __uint_as_float(piece[0][e] & 0xffff0000u);
+            piece[1][e] = pack_bf16x2_rne(ra, rb_);
+            const float la = ra - __uint_as_float(piece[1][e] << 16), lb = rb_ - __uint_as_float(piece[1][e] & 0xffff0000u);
+            piece[2][e] = pack_bf16x2_rne(la, lb);
+            const float most = fmaxf(fabsf(a), fabsf(b));
+            nz |= most > 0.0f;
+            ord |= most >= 0x1p-100f;
+            // (a NaN fails the comparison; fmaxf alone would drop it)
+            wild |= !(fabsf(a) < 0x1p127f) | !(fabsf(b) < 0x1p127f);
+        }
+        const unsigned long long nz64 = __ballot(nz), ord64 = __ballot(ord);
+        nonzero |= static_cast<unsigned>(nz64) | static_cast<unsigned>(nz64 >> 32);
+        ordinary |= static_cast<unsigned>(ord64) | static_cast<unsigned>(ord64 >> 32);
+        unsigned char *dst = job.blocks + (static_cast<size_t>(rb) * job.ksteps + ks) * 3072 + lane * 16;
+#pragma unroll
+        for (int plane = 0; plane < 3; ++plane)
+            *reinterpret_cast<uint4 *>(dst + plane * 1024) = make_uint4(piece[plane][0], piece[plane][1], piece[plane][2], piece[plane][3]);
+    }
+    const unsigned any_wild = __ballot(wild != 0) != 0 ? 1u : 0u;
+    if (lane == 0) job.status[static_cast<size_t>(rb) * (job.ksteps / 2) + pair] = make_uint4(nonzero, ordinary, any_wild, 0u);
+}
+
+// ---- the product -------------------------------------------------------------------------------------------------
+struct SplitGemmArgs {
+    const unsigned char *blocks;  // A's blocks, then B's at b_base
+    unsigned b_base, bytes;
+    const uint4 *status_a, *status_b;
+    float *C;  // the result, or plane `split` of the partial sums
+    const float *bias, *residual;
+    const float *A, *B;  // the original operands, for the tiles the splitting pass marked
+    int a_row, a_k, b_col, b_k;  // their strides
+    int M, N, K, ksteps;  // ksteps: even
+    int tiles_m, tiles_n, steps_per_split;
+    float scale;
+    int activation;
+};
+
+// Whether A's 32-row blocks [ra, ra + TM) or B's [rb, rb + TN) hold anything the three pieces cannot carry, over block
+// pairs [pair0, pair1): wavefront-uniform.
+template <int TM, int TN>
+__device__ __forceinline__ bool split_status_bad(const SplitGemmArgs &p, int ra, int rb, int pair0, int pair1, int lane)
+{
+    constexpr int COUNT = TM + TN;
+    const int pairs = p.ksteps / 2, blocks_a = (p.M + 31) / 32, blocks_b = (p.N + 31) / 32;
+    const uint4 *line[COUNT];
+#pragma unroll
+    for (int b = 0; b < COUNT; ++b)  // (blocks past the end repeat the last one)
+        line[b] = b < TM ? p.status_a + static_cast<size_t>(min(ra + b, blocks_a - 1)) * pairs
+                         : p.status_b + static_cast<size_t>(min(rb + b - TM, blocks_b - 1)) * pairs;
+    unsigned nonzero[COUNT], ordinary[COUNT], wild = 0;
+#pragma unroll
+    for (int b = 0; b < COUNT; ++b) nonzero[b] = ordinary[b] = 0;
+    for (int i = pair0 + lane; i < pair1; i += 64) {
+        uint4 s[COUNT];
+#pragma unroll
+        for (int b = 0; b < COUNT; ++b) s[b] = line[b][i];
+#pragma unroll
+        for (int b = 0; b < COUNT; ++b) {
+            nonzero[b] |= s[b].x;
+            ordinary[b] |= s[b].y;
+            wild |= s[b].z;
+        }
+    }
+    unsigned suspect = 0;
+#pragma unroll
+    for (int b = 0; b < COUNT; ++b) suspect |= nonzero[b] & ~ordinary[b];
+    if (__any(wild != 0)) return true;
+    if (!__any(suspect != 0)) return false;
+    // A row may be small in one stretch and ordinary in another: only rows that are small throughout count.
+    unsigned bad = 0;
+#pragma unroll 1
+    for (int b = 0; b < COUNT; ++b) {
+        unsigned nz = 0, ord = 0;
+        for (int i = pair0; i < pair1; ++i) {
+            const uint4 s = line[b][i];
+            nz |= s.x;
+            ord |= s.y;
+        }
+        bad |= nz & ~ord;
+    }
+    return bad != 0;
+}
+
+template <int BM, int BN, int WM, int WN, int STAGES>
+__device__ __forceinline__ void gemm_f32_split_body(const SplitGemmArgs &p)
+{
+    constexpr int WAVES = WM * WN;
+    constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN = WTN / 32;
+    constexpr int PIECES = (BM + BN) / 32 * 3;  // 1 KB pieces of a 16-term stage
+    constexpr int LOADS = (PIECES + WAVES - 1) / WAVES;
+    constexpr int STAGE = PIECES * 1024;
+    constexpr int SLOTS = TM * TN, SPREAD = TM + TN;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds_bytes[];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / WN, wn = wave % WN;
+    const int li = lane & 31, lh = lane >> 5;
+
+    // Every XCD takes one contiguous run of tiles, walked in groups of 4 tile rows, so that what is resident on an XCD at
+    // a time shares its A and B panels through that L2.
+    const int grid = static_cast<int>(gridDim.x), xcd = static_cast<int>(blockIdx.x) & 7;
+    int logical = xcd * (grid >> 3) + min(xcd, grid & 7) + (static_cast<int>(blockIdx.x) >> 3);
+    const int tiles = p.tiles_m * p.tiles_n;
+    const int split = logical / tiles;
+    logical -= split * tiles;
+    constexpr int GROUP_M = 4;
+    const int width = GROUP_M * p.tiles_n;
+    const int group = logical / width;
+    const int first_m = group * GROUP_M;
+    const int group_size = min(p.tiles_m - first_m, GROUP_M);
+    const int m0 = (first_m + (logical % width) % group_size) * BM, n0 = (logical % width) / group_size * BN;
+    const int step0 = split * p.steps_per_split;
+    const int steps = min(p.steps_per_split, p.ksteps - step0);
+
+    const __amdgpu_buffer_rsrc_t rsrc =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char *>(p.blocks), 0, static_cast<int>(p.bytes), 0x00020000);
+    // Piece q of a stage: fragment q % 3 of row block q / 3 of the tile (A's blocks first).  Row blocks past the end of A
+    // read B's, those past the end of B read zeros; neither reaches a stored value.
+    unsigned piece_off[LOADS];
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+        const int q = min(wave * LOADS + i, PIECES - 1);
+        const int block = q / 3, plane = q % 3;
+        const unsigned row_block = block < BM / 32 ? m0 / 32 + block : n0 / 32 + block - BM / 32;
+        piece_off[i] = (block < BM / 32 ? 0u : p.b_base) + (row_block * p.ksteps + step0) * 3072u + plane * 1024u;
+    }
+    const unsigned lane_off = lane * 16;
+    auto load = [&](int stage, int i, int step, unsigned off) {
+        const int q = min(wave * LOADS + i, PIECES - 1);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_ptr)(lds_bytes + stage * STAGE + q * 1024), 16, off,
+                                                 piece_off[i] + step * 3072u, 0, 0);
+    };
+
+    // hi·hi and the five small products accumulate apart and are added at the end: a small product then never rounds
+    // against the large sum, and the result carries one rounding per sixteen terms.
+    f32x16 acc[TM][TN], fine[TM][TN];
+#pragma unroll
+    for (int a = 0; a < TM; ++a)
+#pragma unroll
+        for (int b = 0; b < TN; ++b)
+            acc[a][b] = fine[a][b] = f32x16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+
+    bf16x8 a_hi[TM], a_mid[TM], a_lo[TM], b_hi[2][TN], b_mid[TN], b_lo[TN];
+    const unsigned a_frag = wm * TM * 3072 + lane_off, b_frag = (BM / 32 + wn * TN) * 3072 + lane_off;
+    auto frag_a = [&](int stage, int t, int plane) {
+        return *reinterpret_cast<const bf16x8 *>(lds_bytes + stage * STAGE + a_frag + t * 3072 + plane * 1024);
+    };
+    auto frag_b = [&](int stage, int t, int plane) {
+        return *reinterpret_cast<const bf16x8 *>(lds_bytes + stage * STAGE + b_frag + t * 3072 + plane * 1024);
+    };
+    // The product is formed transposed (B's fragment first), so register 4g + j of lane (li, lh) is
+    // C[32·tm + li][32·tn + 8g + 4·lh + j]: four neighbouring columns of a row.
+    auto product = [&](f32x16 (&sum)[TM][TN], const bf16x8 (&a)[TM], const bf16x8 (&b)[TN], auto &&memory) {
+#pragma unroll
+        for (int slot = 0; slot < SLOTS; ++slot) {
+            sum[slot / TN][slot % TN] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[slot % TN], a[slot / TN], sum[slot / TN][slot % TN], 0, 0, 0);
+            ST_SPLIT_FENCE();
+            memory(slot);
+            ST_SPLIT_FENCE();
+        }
+    };
+
+    // Step t (16 terms).  On entry the fragments lo and mid of A and hi and mid of B are in registers; the rest is read
+    // during the first product, so that every LDS read of a stage is behind its barrier, after which the stage takes
+    // the loads of step t + STAGES.  Behind the barrier come those loads and the next step's fragments, each into
+    // registers whose last use is past: one memory instruction behind an MFMA, never a burst.
+    int stage = 0;
+    auto iteration = [&](auto buf_tag, int t) {
+        constexpr int BUF = decltype(buf_tag)::value;
+        const int next = stage + 1 == STAGES ? 0 : stage + 1;
+        product(fine, a_lo, b_hi[BUF], [&](int slot) {
+            if (slot < SPREAD) {
+                if (slot < TM) a_hi[slot] = frag_a(stage, slot, 0);
+                else b_lo[slot - TM] = frag_b(stage, slot - TM, 2);
+            }
+            if (SLOTS < SPREAD && slot == SLOTS - 1) {
+#pragma unroll
+                for (int i = SLOTS; i < SPREAD; ++i) {
+                    if (i < TM) a_hi[i] = frag_a(stage, i, 0);
+                    else b_lo[i - TM] = frag_b(stage, i - TM, 2);
+                }
+            }
+        });
+        product(fine, a_mid, b_hi[BUF], [&](int) {});
+        // This wavefront's loads of step t + 1 have landed, and its LDS reads of step t have returned; the barrier extends
+        // both to every wavefront.
+        ST_SPLIT_WAIT_VMCNT((STAGES - 2) * LOADS);
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        // Past the last step the loads fall outside the buffer (zeros, no memory access) and the fragments read are
+        // never used: every step runs the same code.
+        const unsigned off = t + STAGES < steps ? lane_off : 0x80000000u;
+        // the memory instructions of the last four products: loads, then A's lo and B's hi, spread over three of them ...
+        auto tail = [&](int slot) {
+            constexpr int ALL = LOADS + SPREAD, PER = (ALL + 3 * SLOTS - 1) / (3 * SLOTS);
+#pragma unroll
+            for (int e = 0; e < PER; ++e) {
+                const int i = slot * PER + e, r = i - LOADS;
+                if (i < LOADS) load(stage, i, t + STAGES, off);
+                else if (r < TM) a_lo[r] = frag_a(next, r, 2);
+                else if (r < SPREAD) b_hi[BUF ^ 1][r - TM] = frag_b(next, r - TM, 0);
+            }
+        };
+        product(fine, a_mid, b_mid, [&](int slot) { tail(slot); });
+        product(fine, a_hi, b_mid, [&](int slot) { tail(SLOTS + slot); });
+        product(fine, a_hi, b_lo, [&](int slot) { tail(2 * SLOTS + slot); });
+        // ... and the mid fragments behind the last one that reads them
+        product(acc, a_hi, b_hi[BUF], [&](int slot) {
+            constexpr int PER = (SPREAD + SLOTS - 1) / SLOTS;
+#pragma unroll
+            for (int e = 0; e < PER; ++e) {
+                const int i = slot * PER + e;
+                if (i < TM) a_mid[i] = frag_a(next, i, 1);
+                else if (i < SPREAD) b_mid[i - TM] = frag_b(next, i - TM, 1);
+            }
+        });
+        stage = next;
+    };
+
+#pragma unroll
+    for (int s = 0; s < STAGES; ++s) {
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) load(s, i, s, s < steps ? lane_off : 0x80000000u);
+    }
+    const bool bad = split_status_bad<TM, TN>(p, m0 / 32 + wm * TM, n0 / 32 + wn * TN, step0 / 2, (step0 + steps) / 2, lane);
+    ST_SPLIT_WAIT_VMCNT(0);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+        a_lo[i] = frag_a(0, i, 2);
+        a_mid[i] = frag_a(0, i, 1);
+    }
+#pragma unroll
+    for (int i = 0; i < TN; ++i) {
+        b_hi[0][i] = frag_b(0, i, 0);
+        b_mid[i] = frag_b(0, i, 1);
+    }
+    for (int t = 0; t < steps; t += 2) {
+        iteration(std::integral_constant<int, 0>{}, t);
+        iteration(std::integral_constant<int, 1>{}, t + 1);
+    }
+
+#pragma unroll
+    for (int a = 0; a < TM; ++a)
+#pragma unroll
+        for (int b = 0; b < TN; ++b) acc[a][b] += fine[a][b];
+
+    // Epilogue through a strip of LDS per wavefront, so that stores and residual loads cover whole row segments.
+    __syncthreads();
+    constexpr int C_STRIDE = WTN + 4;
+    constexpr int LPR = WTN / 4, ROWS_PER_PASS = 64 / LPR, PASSES = 32 / ROWS_PER_PASS;
+    float *strip = reinterpret_cast<float *>(lds_bytes) + wave * (32 * C_STRIDE);
+    const int row_first = m0 + wm * WTM, col_first = n0 + wn * WTN;
+    const int col0 = col_first + (lane & (LPR - 1)) * 4;
+    float *const C = p.C + static_cast<size_t>(split) * p.M * p.N;
+    float bias[4] = {-0.0f, -0.0f, -0.0f, -0.0f};  // x + -0.0f == x for every x
+    if (p.bias) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (col0 + e < p.N) bias[e] = p.bias[col0 + e];
+    }
+    with_epilogue_ops(p.activation, p.residual != nullptr, [&](auto &&act, auto has_residual) {
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm) {
+            const int row_base = row_first + tm * 32;
+            if (!bad) {
+#pragma unroll
+                for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g)
+                        *reinterpret_cast<float4 *>(&strip[li * C_STRIDE + tn * 32 + g * 8 + lh * 4]) = make_float4(
+                            acc[tm][tn][4 * g], acc[tm][tn][4 * g + 1], acc[tm][tn][4 * g + 2], acc[tm][tn][4 * g + 3]);
+            } else {
+                const int k_end = min(p.K, (step0 + steps) * 16);
+                for (int e = lane; e < 32 * WTN; e += 64) {
+                    const int row = row_base + e / WTN, col = col_first + e % WTN;
+                    float sum = 0.0f;
+                    if (row < p.M && col < p.N)
+                        for (int k = step0 * 16; k < k_end; ++k)
+                            sum = fmaf(p.A[static_cast<size_t>(row) * p.a_row + static_cast<size_t>(k) * p.a_k],
+                                       p.B[static_cast<size_t>(col) * p.b_col + static_cast<size_t>(k) * p.b_k], sum);
+                    strip[e / WTN * C_STRIDE + e % WTN] = sum;
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < PASSES; ++j) {
+                const int local_row = j * ROWS_PER_PASS + lane / LPR;
+                const int row = row_base + local_row;
+                const float4 s4 = *reinterpret_cast<const float4 *>(&strip[local_row * C_STRIDE + (lane & (LPR - 1)) * 4]);
+                if (row >= p.M || col0 >= p.N) continue;
+                const size_t idx = static_cast<size_t>(row) * p.N + col0;
+                const float v[4] = {s4.x * p.scale + bias[0], s4.y * p.scale + bias[1], s4.z * p.scale + bias[2], s4.w * p.scale + bias[3]};
+                if (col0 + 4 <= p.N) {
+                    f32x4_a4 out = {v[0], v[1], v[2], v[3]};
+                    if constexpr (decltype(has_residual)::value) out += *reinterpret_cast<const f32x4_a4 *>(p.residual + idx);
+                    *reinterpret_cast<f32x4_a4 *>(C + idx) = f32x4_a4{act(out[0]), act(out[1]), act(out[2]), act(out[3])};
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 3; ++e) {
+                        if (col0 + e >= p.N) continue;
+                        float value = v[e];
+                        if constexpr (decltype(has_residual)::value) value += p.residual[idx + e];
+                        C[idx + e] = act(value);
+                    }
+                }
+            }
+        }
+    });
+}
+
+// (Plain kernels around the templated body: a kernel template whose body uses the LDS-load builtins loses its host-side
+// launch stub with this compiler.)
+__global__ __launch_bounds__(512) void gemm_f32_split_256x128_kernel(SplitGemmArgs p) { gemm_f32_split_body<256, 128, 4, 2, 3>(p); }
+__global__ __launch_bounds__(256) void gemm_f32_split_160x128_kernel(SplitGemmArgs p) { gemm_f32_split_body<160, 128, 1, 4, 5>(p); }
+__global__ __launch_bounds__(256, 2) void gemm_f32_split_128x128_kernel(SplitGemmArgs p) { gemm_f32_split_body<128, 128, 2, 2, 3>(p); }
+__global__ __launch_bounds__(256) void gemm_f32_split_96x128_kernel(SplitGemmArgs p) { gemm_f32_split_body<96, 128, 1, 4, 3>(p); }
+__global__ __launch_bounds__(256, 2) void gemm_f32_split_64x128_kernel(SplitGemmArgs p) { gemm_f32_split_body<64, 128, 2, 2, 4>(p); }
+__global__ __launch_bounds__(256, 2) void gemm_f32_split_64x64_kernel(SplitGemmArgs p) { gemm_f32_split_body<64, 64, 2, 2, 6>(p); }
+
+// The tile shapes, and what one 32×32 block of a tile costs per 16-term step (measured on N(0,1) operands with the chip
+// full; the matrix pipe alone needs 19 ns of the four it shares between SIMDs at the clock that data allows).
+struct SplitConfig {
+    void (*kernel)(SplitGemmArgs);
+    int bm, bn, threads, stages;
+    double block_ns;
+};
+const SplitConfig kSplitConfigs[] = {
+    {gemm_f32_split_256x128_kernel, 256, 128, 512, 3, 32.5}, {gemm_f32_split_160x128_kernel, 160, 128, 256, 5, 32.0},
+    {gemm_f32_split_128x128_kernel, 128, 128, 256, 3, 33.5}, {gemm_f32_split_96x128_kernel, 96, 128, 256, 3, 35.0},
+    {gemm_f32_split_64x128_kernel, 64, 128, 256, 4, 38.0},   {gemm_f32_split_64x64_kernel, 64, 64, 256, 6, 42.0},
+};
+
+struct SplitPlan {
+    const SplitConfig *config = nullptr;
+    int splits = 1, steps_per_split = 0;
+    double us = 0.0;  // estimate, the splitting pass included
+};
+
+constexpr double kCopyBytesPerUs = 5.0e6;  // what streaming kernels reach here
+
+// Tile shape and k-split with the least estimated time.  Work is handed out by whole tiles, so what counts is the
+// fullest of the 256 compute units: 1576×3072×768 is 240 tiles of 160×128 (one round, 41 µs) but 312 of 128×128 (two,
+// 50 µs).  A k-split costs its partial planes (written and read once) and a launch.
+SplitPlan plan_split(size_t m, size_t n, size_t k, bool may_split_k)
+{
+    const size_t ksteps = (k + 31) / 32 * 2;
+    SplitPlan best;
+    for (const SplitConfig &c : kSplitConfigs) {
+        const size_t tiles = ((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn);
+        const double blocks = c.bm / 32 * (c.bn / 32);
+        for (size_t splits = 1; splits <= 8; ++splits) {
+            if (splits > 1 && (!may_split_k || ksteps / splits < 16 || tiles * splits > 1024)) break;
+            const size_t steps = (ksteps / 2 + splits - 1) / splits * 2;
+            if (splits > 1 && (splits - 1) * steps >= ksteps) continue;
+            const double rounds = static_cast<double>((tiles * splits + 255) / 256);
+            double us = 4.5 + rounds * (steps * std::max(blocks * c.block_ns * 1e-3, 0.16) + 1.0) + 4.0 * m * n * splits / kCopyBytesPerUs;
+            if (splits > 1) us += 3.0 + 4.0 * m * n * (splits + 1) / kCopyBytesPerUs;
+            if (best.config == nullptr || us < best.us) {
+                best.config = &c;
+                best.splits = static_cast<int>(splits);
+                best.steps_per_split = static_cast<int>(steps);
+                best.us = us;
+            }
+        }
+    }
+    best.us += 4.5 + 10.0 * (static_cast<double>(m) + n) * k / 7.0e6;  // the splitting pass: 4 bytes read, 6 written a value
+    return best;
+}
+
+unsigned split_groups(SplitJob &job)
+{
+    job.groups_k = static_cast<unsigned>(job.transposed ? (job.k + 31) / 32 : (job.k + 127) / 128);
+    return job.groups_k * static_cast<unsigned>(job.transposed ? (job.rows + 127) / 128 : (job.rows + 31) / 32);
+}
+
+}  // namespace
+
+bool gemm_f32_split_applies(size_t m, size_t n, size_t k, double other_us, bool may_split_k)
+{
+    if (k < 64 || m < 32 || n < 32) return false;
+    // all block offsets below 2^31, so that the ones past the end can be marked by bit 31
+    const double bytes = (static_cast<double>(m) + n + 64) * (static_cast<double>(k) + 32) * 6.0;
+    if (bytes >= static_cast<double>(1ull << 31)) return false;
+    return plan_split(m, n, k, may_split_k).us < 0.9 * other_us;  // a tenth for the error of both estimates
+}
+
+hipError_t launch_gemm_f32_split(size_t m, size_t n, size_t k, bool lhs_transposed, const float *lhs, bool rhs_packed, const float *rhs,
+                                 float *out, const GemmEpilogue &epilogue, hipStream_t stream, bool may_split_k)
+{
+    const SplitPlan plan = plan_split(m, n, k, may_split_k);
+    const SplitConfig &config = *plan.config;
+    const size_t ksteps = (k + 31) / 32 * 2, rows_a = (m + 31) / 32, rows_b = (n + 31) / 32;
+    const size_t bytes_a = rows_a * ksteps * 3072, bytes_b = rows_b * ksteps * 3072;
+    void *blocks = nullptr, *planes = nullptr;
+    hipError_t rc = stream_workspace_slot(stream, 1, bytes_a + bytes_b + (rows_a + rows_b) * (ksteps / 2) * sizeof(uint4), &blocks);
+    if (rc == hipSuccess && plan.splits > 1) rc = stream_workspace(stream, plan.splits * m * n * sizeof(float), &planes);
+    if (rc != hipSuccess) return rc;
+    unsigned char *const base = static_cast<unsigned char *>(blocks);
+    uint4 *const status = reinterpret_cast<uint4 *>(base + bytes_a + bytes_b);
+
+    SplitJob job_a{lhs, base, status, static_cast<int>(m), static_cast<int>(k), static_cast<int>(lhs_transposed ? m : k),
+                   lhs_transposed ? 1 : 0, static_cast<int>(ksteps), 0};
+    SplitJob job_b{rhs, base + bytes_a, status + rows_a * (ksteps / 2), static_cast<int>(n), static_cast<int>(k),
+                   static_cast<int>(rhs_packed ? k : n), rhs_packed ? 0 : 1, static_cast<int>(ksteps), 0};
+    const unsigned groups_a = split_groups(job_a), groups_b = split_groups(job_b);
+    hipLaunchKernelGGL(split_operands_kernel, dim3(groups_a + groups_b), dim3(256), 0, stream, job_a, job_b, groups_a);
+    rc = hipGetLastError();
+    if (rc != hipSuccess) return rc;
+
+    SplitGemmArgs args;
+    args.blocks = base;
+    args.b_base = static_cast<unsigned>(bytes_a);
+    args.bytes = static_cast<unsigned>(bytes_a + bytes_b);
+    args.status_a = job_a.status;
+    args.status_b = job_b.status;
+    args.A = lhs;
+    args.B = rhs;
+    args.a_row = static_cast<int>(lhs_transposed ? 1 : k);
+    args.a_k = static_cast<int>(lhs_transposed ? m : 1);
+    args.b_col = static_cast<int>(rhs_packed ? k : 1);
+    args.b_k = static_cast<int>(rhs_packed ? 1 : n);
+    args.M = static_cast<int>(m);
+    args.N = static_cast<int>(n);
+    args.K = static_cast<int>(k);
+    args.ksteps = static_cast<int>(ksteps);
+    args.tiles_m = static_cast<int>((m + config.bm - 1) / config.bm);
+    args.tiles_n = static_cast<int>((n + config.bn - 1) / config.bn);
+    args.steps_per_split = plan.steps_per_split;
+    const bool split = plan.splits > 1;
+    args.C = split ? static_cast<float *>(planes) : out;
+    args.bias = split ? nullptr : epilogue.bias;
+    args.residual = split ? nullptr : epilogue.residual;
+    args.scale = split ? 1.0f : epilogue.scale;
+    args.activation = split ? ST_HIP_ACT_NONE : epilogue.activation;
+    const size_t lds = static_cast<size_t>(config.bm + config.bn) / 32 * 3072 * config.stages;
+    rc = hipFuncSetAttribute(reinterpret_cast<const void *>(config.kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+    if (rc != hipSuccess) return rc;
+    const size_t groups = static_cast<size_t>(args.tiles_m) * args.tiles_n * plan.splits;
+    hipLaunchKernelGGL(config.kernel, dim3(static_cast<unsigned>(groups)), dim3(config.threads), lds, stream, args);
+    rc = hipGetLastError();
+    if (rc != hipSuccess || !split) return rc;
+    return launch_f32_slice_reduce(m, n, static_cast<size_t>(plan.splits), args.C, out, epilogue, stream);
+}
+
+}  // namespace sthip

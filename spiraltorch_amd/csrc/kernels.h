@@ -42,6 +42,16 @@ hipError_t launch_gemm_f32_batched(size_t batch, size_t m, size_t n, size_t k, b
 // Same with B prepacked as n×k (column-major packing, crates/st-tensor/src/pure.rs:1285-1323).
 hipError_t launch_gemm_f32_packed(size_t m, size_t n, size_t k, const float *lhs, const float *packed_rhs,
                                   float *out, const GemmEpilogue &epilogue, hipStream_t stream);
+// The same products on the bf16 matrix cores, every f32 value as the exact sum of three bf16 values (gemm_f32_split.hip): any
+// shape, layout and alignment.  `applies`: operands that fit its 32-bit offsets and an estimated time below `other_us`.
+// Keeps the split operands in slot 1 of the stream's scratch memory and, where k is split over workgroups (only if
+// `may_split_k`), partial sums in slot 0.
+bool gemm_f32_split_applies(size_t m, size_t n, size_t k, double other_us, bool may_split_k);
+hipError_t launch_gemm_f32_split(size_t m, size_t n, size_t k, bool lhs_transposed, const float *lhs, bool rhs_packed, const float *rhs,
+                                 float *out, const GemmEpilogue &epilogue, hipStream_t stream, bool may_split_k);
+// out = epilogue(sum of `slices` partial planes of m×n values, added in slice order).
+hipError_t launch_f32_slice_reduce(size_t m, size_t n, size_t slices, const float *partial, float *out, const GemmEpilogue &epilogue,
+                                   hipStream_t stream);
 // out(cols×rows) = in(rows×cols) transposed.
 hipError_t launch_transpose_f32(size_t rows, size_t cols, const float *in, float *out, hipStream_t stream);
 
@@ -173,6 +183,9 @@ hipError_t stream_workspace(hipStream_t stream, size_t bytes, void **out);
 // A second buffer of the same kind (slot 1) for re-laid copies of a call's operands, which must stay where they are
 // while the kernels that read them take scratch from slot 0.
 hipError_t stream_workspace_slot(hipStream_t stream, int slot, size_t bytes, void **out);
+// Whether a launcher failed only because scratch memory could not grow (out of memory, or the stream is being captured):
+// nothing has been launched then, and a route that needs no scratch may still run.
+inline bool scratch_unavailable(hipError_t rc) { return rc == hipErrorOutOfMemory || rc == hipErrorStreamCaptureUnsupported; }
 void release_stream_workspace(hipStream_t stream);
 size_t stream_workspace_entry_count();
 // Host<->device copies made by the library, for tests that check where tensors live.

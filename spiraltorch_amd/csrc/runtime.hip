@@ -139,6 +139,13 @@ struct ThreadScratchGuard {
 };
 thread_local ThreadScratchGuard thread_scratch_guard;
 
+// A stream under capture can neither be waited for nor followed by an allocation.
+bool being_captured(hipStream_t stream)
+{
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(stream, &status) == hipSuccess && status != hipStreamCaptureStatusNone;
+}
+
 WorkspaceEntry *find_entry(hipStream_t stream, std::thread::id owner, int slot)
 {
     for (WorkspaceEntry &e : workspace_entries())
@@ -168,6 +175,7 @@ hipError_t stream_workspace_slot(hipStream_t stream, int slot, size_t bytes, voi
                 *out = e->ptr;
                 return hipSuccess;
             }
+            if (being_captured(stream)) return hipErrorStreamCaptureUnsupported;
             // Grow: outside the lock (the wait for the stream must not stall other threads' launches).  The entry stays
             // in the table, owned by this thread and empty, so nobody else touches it meanwhile.
             old = e->ptr;
@@ -187,8 +195,10 @@ hipError_t stream_workspace_slot(hipStream_t stream, int slot, size_t bytes, voi
             return rc;
         }
     }
+    if (!adopted_or_own && being_captured(stream)) return hipErrorStreamCaptureUnsupported;
     void *fresh = nullptr;
     const hipError_t rc = hipMalloc(&fresh, wanted);
+    if (rc != hipSuccess) (void)hipGetLastError();  // the caller may go on without scratch
     std::lock_guard<std::mutex> lock(workspace_mutex());
     WorkspaceEntry *e = find_entry(stream, me, slot);
     if (rc != hipSuccess) {
