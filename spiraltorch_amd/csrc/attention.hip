@@ -36,7 +36,7 @@ struct AttnArgs {
     const float *attn_bias;
     float *out;
     int contexts, S, D;
-    int q_tiles;
+    int bq, q_tiles;  // query rows per tile, ceil(S / bq)
     int swizzle;
     float scale;
     // Keys split over workgroups (non-causal fast kernel only): workgroup (…, split) covers keys_per_split keys
@@ -314,7 +314,8 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(AttnArgs p)
 }
 
 // -------------------------------------------------------------------------------------------------
-// Fast path: head_dim a multiple of 4, 16-byte aligned operands; BIAS adds z_bias / attn_bias where their rows can
+// Fast path on the f32 matrix cores (head sizes above 64, and calls whose logits are large: see sums_in_reference_order):
+// head_dim a multiple of 4, 16-byte aligned operands; BIAS adds z_bias / attn_bias where their rows can
 // be read 128 bits at a time (sequence a multiple of 4), otherwise biased calls take the general kernel above.
 //
 // Same transposed formulation as the general kernel above, tuned for the matrix pipe:
@@ -639,6 +640,435 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DPAD <= 64 
 }
 
 // -------------------------------------------------------------------------------------------------
+// Head sizes up to 64, with or without biases: both products on the bf16 matrix cores, every f32 value (Q, K, V and the
+// probabilities) as the exact sum of three bf16 values, x = hi + mid + lo, and a product as the six piece products
+//     lo·hi, mid·hi, mid·mid, hi·mid, hi·lo, hi·hi
+// accumulated in f32; what is left out is below 2^-26 of the product.  (gemm_f32_split.hip does the same for matrix
+// products, with its error measurements.)  Six bf16 instructions replace eight f32 ones of twice their duration.
+//
+// Same transposed formulation, masks and running maximum as the kernel above.  A stage of 64 keys is split into its pieces
+// by the workgroup on the way from global memory to LDS — a thread owns eight values along the reduction: eight
+// dimensions of a key for K, eight keys of a dimension for V — and stored in fragment order: 1 KB per (32 rows × 16 terms,
+// piece), lane l's 16 bytes at 16·l, so that writes and reads are conflict-free and nothing is padded.  V's reduction runs
+// over the keys in the order the first product leaves the probabilities in the accumulators.  With eight wavefronts (256
+// queries) a value is split once per 256 queries; with four (few query tiles) once per 128.
+//
+// What bounds it: a 64-key stage of 32 queries is 96 matrix instructions (2.0 µs of a SIMD at the rate random operands allow,
+// 21 ns each) beside some 450 vector ones (softmax, the pieces of the probabilities and of the staged values), two
+// wavefronts per SIMD take 5.2 µs for theirs.  Measured, f32 matrix cores -> here: 128 × 2048 × 64 causal 615 -> 382 µs,
+// non-causal 1070 -> 665, 128 × 1024 causal 163 -> 106; biased 1 × 1000 26 -> 16 µs, 16 × 1024 60 -> 51, biases on rows of
+// 777 (no 16-byte alignment: the general kernel) 162 -> 16.  Errors against float64 are 0.7 to 0.85 of the f32 kernel's.
+//
+// Values the pieces cannot carry — 2^40 and more in Q or K (2^127 in V), or a column of V below 2^-110 throughout — make
+// the workgroup redo its rows with f32 multiply-adds (redo_rows below).
+// -------------------------------------------------------------------------------------------------
+__device__ __forceinline__ void split_pair(float a, float b, uint32_t &hi, uint32_t &mid, uint32_t &lo)
+{
+    hi = pack_bf16x2_rne(a, b);
+    const float ra = a - __uint_as_float(hi << 16), rb = b - __uint_as_float(hi & 0xffff0000u);
+    mid = pack_bf16x2_rne(ra, rb);
+    lo = pack_bf16x2_rne(ra - __uint_as_float(mid << 16), rb - __uint_as_float(mid & 0xffff0000u));
+}
+
+__device__ __forceinline__ void split8(const float (&x)[8], u32x4_t (&piece)[3])
+{
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        uint32_t hi, mid, lo;
+        split_pair(x[2 * e], x[2 * e + 1], hi, mid, lo);
+        piece[0][e] = hi;
+        piece[1][e] = mid;
+        piece[2][e] = lo;
+    }
+}
+
+__device__ __forceinline__ float largest8(const float (&x)[8], float so_far)
+{
+#pragma unroll
+    for (int e = 0; e < 4; ++e) so_far = fmaxf(fmaxf(fabsf(x[2 * e]), fabsf(x[2 * e + 1])), so_far);
+    return so_far;
+}
+
+// One thread per query row, f32 multiply-adds throughout: what the split kernel's workgroups fall back to for operands its
+// pieces cannot carry.  Rows q0 .. q0 + count - 1 over keys [key_first, key_end), in the units of the split kernel.
+template <int DPAD, bool CAUSAL, bool BIAS>
+__device__ void redo_rows(const AttnArgs &p, int ctx, int q0, int count, int threads, int tid, int split, int key_first, int key_end,
+                          float scale_log2e, float exp_scale)
+{
+    const int S = p.S, D = p.D;
+    const size_t first = static_cast<size_t>(ctx) * S * D;
+    for (int i = tid; i < count; i += threads) {
+        const int row = q0 + i;
+        if (row >= S) continue;
+        // (four dimensions at a time: D is a multiple of 4 here)
+        float4 q[DPAD / 4], o[DPAD / 4];
+        const float *q_row = p.q + first + static_cast<size_t>(row) * D;
+#pragma unroll
+        for (int g = 0; g < DPAD / 4; ++g) {
+            q[g] = o[g] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (g * 4 < D) q[g] = *reinterpret_cast<const float4 *>(q_row + g * 4);
+            if (p.scale < 0.0f) q[g] = make_float4(-q[g].x, -q[g].y, -q[g].z, -q[g].w);
+        }
+        float top = -INFINITY, sum = 0.0f;
+        const int end = CAUSAL ? min(key_end, row + 1) : key_end;
+        for (int key = key_first; key < end; ++key) {
+            const float *k = p.k + first + static_cast<size_t>(key) * D, *v = p.v + first + static_cast<size_t>(key) * D;
+            float logit = 0.0f;
+#pragma unroll
+            for (int g = 0; g < DPAD / 4; ++g) {
+                if (g * 4 >= D) break;
+                const float4 k4 = *reinterpret_cast<const float4 *>(k + g * 4);
+                logit = fmaf(k4.w, q[g].w, fmaf(k4.z, q[g].z, fmaf(k4.y, q[g].y, fmaf(k4.x, q[g].x, logit))));
+            }
+            if constexpr (BIAS) {
+                float bias = p.attn_bias ? p.attn_bias[(static_cast<size_t>(ctx) * S + row) * S + key] : 0.0f;
+                if (p.z_bias) bias += p.z_bias[static_cast<size_t>(ctx) * S + key];
+                logit = fmaf(logit, scale_log2e, bias * kLog2e);
+            }
+            const float new_top = fmaxf(top, logit);
+            const float safe = new_top == -INFINITY ? 0.0f : new_top;
+            const float alpha = __builtin_amdgcn_exp2f((top - safe) * exp_scale);
+            const float w = __builtin_amdgcn_exp2f(fmaf(logit, exp_scale, -safe * exp_scale));
+            sum = fmaf(sum, alpha, w);
+#pragma unroll
+            for (int g = 0; g < DPAD / 4; ++g) {
+                if (g * 4 >= D) break;
+                const float4 v4 = *reinterpret_cast<const float4 *>(v + g * 4);
+                o[g] = make_float4(fmaf(w, v4.x, o[g].x * alpha), fmaf(w, v4.y, o[g].y * alpha), fmaf(w, v4.z, o[g].z * alpha),
+                                   fmaf(w, v4.w, o[g].w * alpha));
+            }
+            top = new_top;
+        }
+        const bool partial = p.key_splits > 1;
+        const size_t at = (static_cast<size_t>(split) * p.contexts + ctx) * S + row;
+        float *out = partial ? p.part_o + at * D : p.out + first + static_cast<size_t>(row) * D;
+        const float inv = partial ? 1.0f : sum > 0.0f ? 1.0f / sum : 0.0f;
+#pragma unroll
+        for (int g = 0; g < DPAD / 4; ++g)
+            if (g * 4 < D) *reinterpret_cast<float4 *>(out + g * 4) = make_float4(o[g].x * inv, o[g].y * inv, o[g].z * inv, o[g].w * inv);
+        if (partial) *reinterpret_cast<float2 *>(p.part_ml + at * 2) = make_float2(top, sum);
+    }
+}
+
+template <int DPAD, bool CAUSAL, bool BIAS, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void attention_f32_split_kernel(AttnArgs p)
+{
+    constexpr int BKV = 64, THREADS = 64 * WAVES, BQ = 32 * WAVES;
+    constexpr int QSTEPS = DPAD / 16, DT = DPAD / 32;
+    constexpr int CHAINS = DT == 1 ? 2 : 1;  // a single chain of dependent matrix instructions would wait for each
+    constexpr int K_BYTES = 2 * QSTEPS * 3072, V_BYTES = DT * 4 * 3072, STAGE = K_BYTES + V_BYTES;
+    constexpr int ITEMS = 64 * DPAD / 8;  // groups of eight values of K (and of V) in a stage
+    constexpr int PER = ITEMS > THREADS ? ITEMS / THREADS : 1;
+    // Eight wavefronts (one workgroup per compute unit): two stages.  Four: one, so that two workgroups fit a compute unit.
+    constexpr int BUFFERS = WAVES == 8 ? 2 : 1;
+    constexpr float kWild = 0x1p40f, kWildV = 0x1p127f, kTiny = 0x1p-110f;
+    extern __shared__ __attribute__((aligned(16))) unsigned char split_lds[];
+    __shared__ unsigned column_top[DPAD];
+    __shared__ int any_wild;
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 31, lh = lane >> 5;
+    const int S = p.S, D = p.D;
+    const bool stages_items = ITEMS >= THREADS || tid < ITEMS;  // (head size 32 leaves half of eight wavefronts without any)
+
+    const FastItem item = decode_fast_block<CAUSAL>(p.contexts, p.q_tiles, p.swizzle, p.key_splits, p.keys_per_split,
+                                                    p.causal_items, static_cast<int>(blockIdx.x));
+    const int ctx = item.ctx, unit = item.unit, split = item.split;
+    const int split_tile = item.split_tile;
+    const size_t ctx_elem0 = static_cast<size_t>(ctx) * S * D;
+    const unsigned ctx_bytes = static_cast<unsigned>(S) * static_cast<unsigned>(D) * 4u;
+    const __amdgpu_buffer_rsrc_t rsrc_q =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.q + ctx_elem0), 0, static_cast<int>(ctx_bytes), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc_k =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.k + ctx_elem0), 0, static_cast<int>(ctx_bytes), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc_v =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.v + ctx_elem0), 0, static_cast<int>(ctx_bytes), 0x00020000);
+    constexpr unsigned kOutside = 0x80000000u;  // beyond every context: reads as zero
+
+    auto load8 = [&](const __amdgpu_buffer_rsrc_t &rsrc, int row, int d, float (&x)[8]) {
+        const unsigned at = (static_cast<unsigned>(row) * D + d) * 4u;
+        const u32x4_t a = __builtin_amdgcn_raw_buffer_load_b128(rsrc, d < D ? at : kOutside, 0, 0);
+        const u32x4_t b = __builtin_amdgcn_raw_buffer_load_b128(rsrc, d + 4 < D ? at + 16u : kOutside, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            x[e] = __uint_as_float(a[e]);
+            x[4 + e] = __uint_as_float(b[e]);
+        }
+    };
+
+    const int passes = (CAUSAL && split_tile < 0 && unit != p.q_tiles - 1 - unit) ? 2 : 1;
+    for (int pass = 0; pass < passes; ++pass) {
+    const int q_tile = !CAUSAL ? unit : split_tile >= 0 ? split_tile : (pass == 0 ? p.q_tiles - 1 - unit : unit);  // the long tile first
+    const int q0 = q_tile * BQ;
+    const int wq0 = q0 + wave * 32;
+    const int my_q = wq0 + li;
+    float top_qk = 0.0f, top_v[PER];  // largest magnitudes this thread has split
+#pragma unroll
+    for (int r = 0; r < PER; ++r) top_v[r] = 0.0f;
+    // Q pieces: fragment c holds Q[my_q][16c + 8·lh .. + 7]; rows past the end read as zero.  A negative scale is moved
+    // into Q, as in the kernel above.
+    bf16x8 qf[QSTEPS][3];
+#pragma unroll
+    for (int c = 0; c < QSTEPS; ++c) {
+        float x[8];
+        load8(rsrc_q, my_q, c * 16 + lh * 8, x);
+        top_qk = largest8(x, top_qk);
+        if (p.scale < 0.0f) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = -x[e];
+        }
+        u32x4_t piece[3];
+        split8(x, piece);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) qf[c][i] = __builtin_bit_cast(bf16x8, piece[i]);
+    }
+
+    f32x16 oacc[DT * CHAINS];
+#pragma unroll
+    for (int t = 0; t < DT * CHAINS; ++t)
+        oacc[t] = f32x16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float run_max = -INFINITY;
+    float run_sum = 0.0f;
+
+    const bool split_keys = !CAUSAL || split_tile >= 0;
+    const int key_first = split_keys ? split * p.keys_per_split : 0;
+    const int key_end = min(CAUSAL ? min(S, q0 + BQ) : S, split_keys ? key_first + p.keys_per_split : S);
+    const int stages = (key_end - key_first + BKV - 1) / BKV;
+
+    float rk[PER][8], rv[PER][8];
+    auto load_global = [&](int key0) {
+        if (!stages_items) return;
+#pragma unroll
+        for (int r = 0; r < PER; ++r) {
+            const int f = tid + THREADS * r;
+            load8(rsrc_k, key0 + (f & 63), (f >> 6) * 8, rk[r]);
+            const int d = f % DPAD, group = f / DPAD;  // group: 16-key step group / 2, accumulator half group % 2
+            const int key = key0 + (group >> 1) * 16 + (group & 1) * 4;
+            const unsigned at = d < D ? (static_cast<unsigned>(key) * D + d) * 4u : kOutside;
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                rv[r][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc_v, at + ((e >> 2) * 8 + (e & 3)) * (D * 4u), 0, 0));
+        }
+    };
+    auto store_lds = [&](int stage) {
+        if (!stages_items) return;
+        unsigned char *ks = split_lds + stage * STAGE, *vs = ks + K_BYTES;
+#pragma unroll
+        for (int r = 0; r < PER; ++r) {
+            const int f = tid + THREADS * r;
+            u32x4_t piece[3];
+            split8(rk[r], piece);
+            top_qk = largest8(rk[r], top_qk);
+            const int key = f & 63, chunk = f >> 6;
+            unsigned char *dst = ks + ((key >> 5) * QSTEPS + (chunk >> 1)) * 3072 + ((chunk & 1) * 32 + (key & 31)) * 16;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x4_t *>(dst + i * 1024) = piece[i];
+            split8(rv[r], piece);
+            top_v[r] = largest8(rv[r], top_v[r]);
+            const int d = f % DPAD, group = f / DPAD;
+            dst = vs + ((d >> 5) * 4 + (group >> 1)) * 3072 + ((group & 1) * 32 + (d & 31)) * 16;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x4_t *>(dst + i * 1024) = piece[i];
+        }
+    };
+
+    // The maximum in units of the raw dot product and the scale in the exponent, as above; with biases everything after
+    // the logits is in log2 units.
+    const float scale_log2e = fmaxf(fabsf(p.scale) * kLog2e, 1e-30f);
+    const float exp_scale = BIAS ? 1.0f : scale_log2e;
+    const float lag = 8.0f / exp_scale;
+    // The biases come through buffer descriptors that cover this context's: a group of four keys is one 16-byte load at
+    // whatever alignment the row has, past the end of the tensor it reads zeros, and past the end of a row whatever is
+    // there — those keys are masked.  Without a tensor the range is empty.
+    const unsigned long long bias_values = static_cast<unsigned long long>(S) * S;
+    const __amdgpu_buffer_rsrc_t rsrc_ab = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(p.attn_bias + (BIAS && p.attn_bias ? ctx * bias_values : 0)), 0,
+        BIAS && p.attn_bias ? static_cast<int>(bias_values * 4) : 0, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc_zb = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(p.z_bias + (BIAS && p.z_bias ? static_cast<size_t>(ctx) * S : 0)), 0, BIAS && p.z_bias ? S * 4 : 0, 0x00020000);
+    // the six piece products, smallest first: (piece of the first operand, piece of the second)
+    constexpr int kFirst[6] = {2, 1, 1, 0, 0, 0}, kSecond[6] = {0, 0, 1, 1, 2, 0};
+    auto compute = [&](auto nt_tag, auto may_mask_tag, int stage, int key0) {
+        constexpr int NT = decltype(nt_tag)::value;
+        constexpr bool MAY_MASK = decltype(may_mask_tag)::value;
+        const unsigned char *ks = split_lds + stage * STAGE + lane * 16, *vs = ks + K_BYTES;
+        f32x16 sacc[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+            sacc[t] = f32x16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        u32x4_t ab4[BIAS ? NT : 1][4], zb4[BIAS ? NT : 1][4];
+        if constexpr (BIAS) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const unsigned key = key0 + t * 32 + g * 8 + lh * 4;
+                    ab4[t][g] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_ab, (static_cast<unsigned>(my_q) * S + key) * 4u, 0, 0);
+                    zb4[t][g] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_zb, key * 4u, 0, 0);
+                }
+        }
+#pragma unroll
+        for (int c = 0; c < QSTEPS; ++c) {
+            bf16x8 kf[NT][3];
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int i = 0; i < 3; ++i) kf[t][i] = *reinterpret_cast<const bf16x8 *>(ks + (t * QSTEPS + c) * 3072 + i * 1024);
+#pragma unroll
+            for (int i = 0; i < 6; ++i)
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+                    sacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[t][kFirst[i]], qf[c][kSecond[i]], sacc[t], 0, 0, 0);
+        }
+        if constexpr (BIAS) {
+            // logit = (dot·scale + z_bias) + attn_bias of pure.rs:11870-11880, in log2 units
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const float bias = __uint_as_float(ab4[t][r >> 2][r & 3]) + __uint_as_float(zb4[t][r >> 2][r & 3]);
+                    sacc[t][r] = fmaf(sacc[t][r], scale_log2e, bias * kLog2e);
+                }
+        }
+        const bool need_mask = MAY_MASK && ((key0 + NT * 32 > S) || (CAUSAL && key0 + NT * 32 - 1 > wq0));
+        float tile_max = -INFINITY;
+        const int last_key = CAUSAL ? min(my_q, S - 1) : S - 1;
+        if (need_mask) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int key = key0 + t * 32 + (r >> 2) * 8 + lh * 4 + (r & 3);
+                    float v = sacc[t][r];
+                    if (key > last_key) v = -INFINITY;
+                    sacc[t][r] = v;
+                    tile_max = fmaxf(tile_max, v);
+                }
+        } else {
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) tile_max = fmaxf(tile_max, sacc[t][r]);
+        }
+        tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32));
+        if (__any(tile_max > run_max + lag)) {  // wavefront-uniform; the maximum may lag by up to 2^8, as above
+            const float new_max = fmaxf(run_max, tile_max);
+            const float new_safe = new_max == -INFINITY ? 0.0f : new_max;
+            const float alpha = __builtin_amdgcn_exp2f((run_max - new_safe) * exp_scale);
+            run_sum *= alpha;
+#pragma unroll
+            for (int t = 0; t < DT * CHAINS; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) oacc[t][r] *= alpha;
+            run_max = new_max;
+        }
+        const float safe_max = run_max == -INFINITY ? 0.0f : run_max;
+        const float shift = -safe_max * exp_scale;
+        float tile_sum = 0.0f;
+        // Oᵀ += Vᵀ·Pᵀ, sixteen keys at a time: registers 8j .. 8j + 7 of a score tile are this lane's half of the operand.
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                float pr[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    pr[e] = __builtin_amdgcn_exp2f(fmaf(sacc[t][8 * j + e], exp_scale, shift));
+                    tile_sum += pr[e];
+                }
+                u32x4_t piece[3];
+                split8(pr, piece);
+                bf16x8 pf[3];
+#pragma unroll
+                for (int i = 0; i < 3; ++i) pf[i] = __builtin_bit_cast(bf16x8, piece[i]);
+                bf16x8 vf[DT][3];
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                    for (int i = 0; i < 3; ++i)
+                        vf[dt][i] = *reinterpret_cast<const bf16x8 *>(vs + (dt * 4 + t * 2 + j) * 3072 + i * 1024);
+#pragma unroll
+                for (int i = 0; i < 6; ++i)
+#pragma unroll
+                    for (int dt = 0; dt < DT; ++dt) {
+                        const int at = CHAINS == 1 ? dt : i & 1;
+                        oacc[at] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[dt][kFirst[i]], pf[kSecond[i]], oacc[at], 0, 0, 0);
+                    }
+            }
+        run_sum += tile_sum;
+    };
+
+    if (tid < DPAD) column_top[tid] = 0u;
+    if (tid == 0) any_wild = 0;
+    if (stages > 0) {
+        load_global(key_first);
+        store_lds(0);
+    }
+    __syncthreads();
+    // Unmasked stages first, in a loop with one path through it (see the kernel above).
+    const int limit = wq0 >= S ? 0 : CAUSAL ? min(S, wq0 + 32) : S;
+    const int plain_end = wq0 >= S ? key_first : CAUSAL ? min(S, wq0 + 1) : S;
+    const int plain_stages = max(0, min(stages, (plain_end - key_first) / BKV));
+    int t = 0;
+    for (; t < plain_stages; ++t) {
+        const bool more = t + 1 < stages;
+        if (more) load_global(key_first + (t + 1) * BKV);
+        compute(std::integral_constant<int, 2>{}, std::false_type{}, t % BUFFERS, key_first + t * BKV);
+        if (BUFFERS == 1) __syncthreads();
+        if (more) store_lds((t + 1) % BUFFERS);
+        __syncthreads();
+    }
+    for (; t < stages; ++t) {
+        const bool more = t + 1 < stages;
+        if (more) load_global(key_first + (t + 1) * BKV);
+        const int key0 = key_first + t * BKV;
+        if (key0 + 32 < limit) compute(std::integral_constant<int, 2>{}, std::true_type{}, t % BUFFERS, key0);
+        else if (key0 < limit) compute(std::integral_constant<int, 1>{}, std::true_type{}, t % BUFFERS, key0);
+        if (BUFFERS == 1) __syncthreads();
+        if (more) store_lds((t + 1) % BUFFERS);
+        __syncthreads();
+    }
+
+    bool wild = top_qk >= kWild;
+    if (stages_items) {
+#pragma unroll
+        for (int r = 0; r < PER; ++r) {
+            wild |= top_v[r] >= kWildV;
+            atomicMax(&column_top[(tid + THREADS * r) % DPAD], __float_as_uint(top_v[r]));
+        }
+    }
+    if (wild) any_wild = 1;
+    __syncthreads();
+    const float column = lane < DPAD ? __uint_as_float(column_top[lane % DPAD]) : 0.0f;
+    const bool redo = any_wild != 0 || __any(column > 0.0f && column < kTiny);
+
+    const float total = run_sum + __shfl_xor(run_sum, 32);
+    if constexpr (CHAINS == 2) oacc[0] += oacc[1];
+    if (redo) {
+        redo_rows<DPAD, CAUSAL, BIAS>(p, ctx, q0, BQ, THREADS, tid, split, key_first, key_end, scale_log2e, exp_scale);
+    } else if (my_q < S) {
+        const bool partial = p.key_splits > 1;
+        const size_t row = (static_cast<size_t>(split) * p.contexts + ctx) * S + my_q;
+        float *orow = partial ? p.part_o + row * D : p.out + ctx_elem0 + static_cast<size_t>(my_q) * D;
+        const float inv = partial ? 1.0f : total > 0.0f ? 1.0f / total : 0.0f;
+#pragma unroll
+        for (int t = 0; t < DT; ++t)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int d = t * 32 + g * 8 + lh * 4;
+                if (d < D)
+                    *reinterpret_cast<float4 *>(orow + d) = make_float4(oacc[t][g * 4 + 0] * inv, oacc[t][g * 4 + 1] * inv,
+                                                                        oacc[t][g * 4 + 2] * inv, oacc[t][g * 4 + 3] * inv);
+            }
+        if (partial && lh == 0) *reinterpret_cast<float2 *>(p.part_ml + row * 2) = make_float2(run_max, total);
+    }
+    if (pass + 1 < passes) __syncthreads();  // column_top and the stages are written again
+    }  // pass
+}
+
+// -------------------------------------------------------------------------------------------------
 // Many short contexts (windowed attention: thousands of contexts of 16 to 64 positions).  The kernels above give a
 // context a workgroup and a 128-row query tile, which is mostly padding here, and such launches are memory-bound:
 // 16384 contexts of 16 × 64 took 218 µs, 1.2 TB/s.  Here ONE WAVEFRONT owns a context of up to 64 positions: it stages
@@ -895,7 +1325,50 @@ size_t plan_fast(AttnArgs &args, const bool causal, int *causal_r)
     args.causal_items = 0;
     *causal_r = 0;
     constexpr size_t kTargetBlocks = 512;
-    if (blocks * 2 > kTargetBlocks || args.S < 256) return blocks;
+    if (blocks * 2 > kTargetBlocks || args.S < 256 || args.bq != kBQ) return blocks;
+    // The split kernel (head sizes up to 64): a stage of 64 keys costs a workgroup about 2 µs, its start and end 3, merging
+    // 2 and a quarter per chunk, and what counts is the fullest of the 256 compute units.  3 contexts of 1180 (30 query
+    // tiles): 7 chunks of 192 keys are 210 workgroups, 14.8 µs; 10 of 128 are 300, two on some units, 17.7.
+    if (args.D <= 64) {
+        const size_t tiles = static_cast<size_t>(args.q_tiles), contexts = static_cast<size_t>(args.contexts);
+        auto cost = [](size_t workgroups, double stages, size_t chunks) {
+            return static_cast<double>((workgroups + 255) / 256) * (2.0 * stages + 3.0) + (chunks > 1 ? 2.0 + 0.25 * chunks : 0.0);
+        };
+        if (causal) {
+            auto items = [&](size_t r) {
+                size_t total = 0;
+                for (size_t j = 0; j < tiles; ++j) total += j / r + 1;
+                return total;
+            };
+            double best = cost(blocks, 2.0 * (tiles + 1), 1);
+            for (size_t r = 1; r < tiles; ++r) {
+                const double us = cost(contexts * items(r), 2.0 * r, (tiles - 1) / r + 1);
+                if (contexts * items(r) <= blocks || us >= best) continue;
+                best = us;
+                *causal_r = static_cast<int>(r);
+            }
+            if (*causal_r > 0) {
+                const size_t r = static_cast<size_t>(*causal_r);
+                args.keys_per_split = static_cast<int>(r) * kBQ;
+                args.key_splits = static_cast<int>((tiles - 1) / r + 1);
+                args.causal_items = static_cast<int>(items(r));
+                blocks = contexts * items(r);
+            }
+        } else {
+            double best = cost(blocks, (args.S + 63) / 64, 1);
+            for (size_t per = 128; per < static_cast<size_t>(args.S); per += 64) {
+                const size_t splits = (static_cast<size_t>(args.S) + per - 1) / per;
+                const double us = cost(contexts * tiles * splits, per / 64, splits);
+                if (us >= best) continue;
+                best = us;
+                args.keys_per_split = static_cast<int>(per);
+                args.key_splits = static_cast<int>(splits);
+            }
+            blocks *= static_cast<size_t>(args.key_splits);
+        }
+        if (args.key_splits > 1) args.swizzle = 0;
+        return blocks;
+    }
     if (causal) {
         // Few contexts: pairs of query tiles leave most of the chip idle (8 contexts of 2048: 64 workgroups, slower than
         // the non-causal call that does twice the work).  Split every tile's keys into chunks of 128·r instead, with the
@@ -923,9 +1396,9 @@ size_t plan_fast(AttnArgs &args, const bool causal, int *causal_r)
         // split the keys over workgroups until the launch offers about two workgroups per compute unit, 128 keys at least
         // per split, and merge the partial rows in a second kernel.
         const size_t want = (kTargetBlocks + blocks - 1) / blocks;
-        const size_t most = static_cast<size_t>(args.S) / 128;
+        const size_t most = (static_cast<size_t>(args.S) + 127) / 128;
         const size_t splits = std::min(want, most);
-        const size_t per = ((static_cast<size_t>(args.S) + splits - 1) / splits + 63) / 64 * 64;
+        const size_t per = std::max<size_t>(128, ((static_cast<size_t>(args.S) + splits - 1) / splits + 63) / 64 * 64);
         args.keys_per_split = static_cast<int>(per);
         args.key_splits = static_cast<int>((static_cast<size_t>(args.S) + per - 1) / per);
         blocks *= static_cast<size_t>(args.key_splits);
@@ -962,18 +1435,29 @@ bool fast_plan_consistent(const AttnArgs &args, const bool causal, const size_t 
     return fast_block_in_range(args, causal, 0) && fast_block_in_range(args, causal, blocks - 1);
 }
 
-template <int DPAD, bool CAUSAL, bool BIAS = false>
-hipError_t launch_fast(AttnArgs args, hipStream_t stream)
+// Calls whose logits are large (the usual scale is 1/sqrt(head_dim)) stay on the f32 matrix cores: the exponential turns the
+// last bits of a logit of 100 into a relative 1e-5 of its weight, so two correct f32 evaluations differ visibly, and the f32
+// instruction adds the products of a logit in the reference's order.
+bool sums_in_reference_order(size_t head_dim, float scale) { return !(fabsf(scale) * sqrtf(static_cast<float>(head_dim)) <= 4.0f); }
+
+// Query rows per workgroup: the split kernel (head sizes up to 64) takes 256 where such tiles still give every compute
+// unit one, 128 otherwise and on every other kernel.
+int query_rows(size_t contexts, size_t sequence, size_t head_dim, bool causal)
 {
-    constexpr size_t lds_bytes = 2 * static_cast<size_t>(64) * ((DPAD + 4) + (DPAD + 8)) * sizeof(float);
-    auto kernel = attention_f32_fast_kernel<DPAD, CAUSAL, BIAS>;
-    hipError_t rc = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes));
-    if (rc != hipSuccess) return rc;
+    if (head_dim > 64 || sequence <= 256) return kBQ;
+    const size_t tiles = (sequence + 255) / 256;
+    return contexts * (causal ? (tiles + 1) / 2 : tiles) >= 256 ? 256 : kBQ;
+}
+
+// Plans, checks and launches a kernel whose workgroups decode their items with decode_fast_block, and merges the key splits.
+hipError_t launch_planned(void (*kernel)(AttnArgs), unsigned threads, size_t lds_bytes, AttnArgs args, bool causal, bool bias,
+                          hipStream_t stream)
+{
     args.part_o = args.part_ml = nullptr;
     int causal_r = 0;
-    const size_t blocks = plan_fast(args, CAUSAL, &causal_r);
-    if (!fast_plan_consistent(args, CAUSAL, blocks)) return hipErrorInvalidConfiguration;
+    const size_t blocks = plan_fast(args, causal, &causal_r);
+    if (!fast_plan_consistent(args, causal, blocks)) return hipErrorInvalidConfiguration;
+    hipError_t rc = hipSuccess;
     if (args.key_splits > 1) {
         const size_t rows = static_cast<size_t>(args.contexts) * args.S;
         const size_t o_bytes = static_cast<size_t>(args.key_splits) * rows * args.D * sizeof(float);
@@ -984,14 +1468,43 @@ hipError_t launch_fast(AttnArgs args, hipStream_t stream)
         args.part_o = static_cast<float *>(workspace);
         args.part_ml = reinterpret_cast<float *>(static_cast<unsigned char *>(workspace) + o_bytes);
     }
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), lds_bytes, stream, args);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(threads), lds_bytes, stream, args);
     rc = hipGetLastError();
     if (rc != hipSuccess || args.key_splits == 1) return rc;
     const float scale_log2e = fmaxf(fabsf(args.scale) * kLog2e, 1e-30f);
     const size_t work = static_cast<size_t>(args.contexts) * args.S * (args.D / 4);
     hipLaunchKernelGGL(attention_merge_splits_kernel, dim3(static_cast<unsigned>((work + 255) / 256)), dim3(256), 0, stream, args,
-                       BIAS ? 1.0f : scale_log2e, causal_r);
+                       bias ? 1.0f : scale_log2e, causal_r);
     return hipGetLastError();
+}
+
+template <int DPAD, bool CAUSAL, bool BIAS = false>
+hipError_t launch_fast(AttnArgs args, hipStream_t stream)
+{
+    constexpr size_t lds_bytes = 2 * static_cast<size_t>(64) * ((DPAD + 4) + (DPAD + 8)) * sizeof(float);
+    auto kernel = attention_f32_fast_kernel<DPAD, CAUSAL, BIAS>;
+    const hipError_t rc = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                              static_cast<int>(lds_bytes));
+    if (rc != hipSuccess) return rc;
+    return launch_planned(kernel, 256, lds_bytes, args, CAUSAL, BIAS, stream);
+}
+
+template <int DPAD, bool CAUSAL, bool BIAS, int WAVES>
+hipError_t launch_split_rows(AttnArgs args, hipStream_t stream)
+{
+    constexpr size_t lds_bytes = (WAVES == 8 ? 2 : 1) * static_cast<size_t>(2 * (DPAD / 16) + 4 * (DPAD / 32)) * 3072;
+    auto kernel = attention_f32_split_kernel<DPAD, CAUSAL, BIAS, WAVES>;
+    const hipError_t rc = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                              static_cast<int>(lds_bytes));
+    if (rc != hipSuccess) return rc;
+    return launch_planned(kernel, 64 * WAVES, lds_bytes, args, CAUSAL, BIAS, stream);
+}
+
+template <int DPAD, bool CAUSAL, bool BIAS>
+hipError_t launch_split(AttnArgs args, hipStream_t stream)
+{
+    if (args.bq == 256) return launch_split_rows<DPAD, CAUSAL, BIAS, 8>(args, stream);
+    return launch_split_rows<DPAD, CAUSAL, BIAS, 4>(args, stream);
 }
 
 template <int DPAD, int BKV, bool CAUSAL, bool BIAS, bool VEC>
@@ -1032,7 +1545,8 @@ AttentionPlanReport attention_f32_plan_report(size_t contexts, size_t sequence, 
     args.contexts = static_cast<int>(contexts);
     args.S = static_cast<int>(sequence);
     args.D = static_cast<int>(head_dim);
-    args.q_tiles = static_cast<int>((sequence + kBQ - 1) / kBQ);
+    args.bq = query_rows(contexts, sequence, head_dim, causal);
+    args.q_tiles = static_cast<int>((sequence + args.bq - 1) / args.bq);
     args.swizzle = (contexts % 8 == 0) ? 1 : 0;
     args.key_splits = 1;
     args.keys_per_split = args.S;
@@ -1046,7 +1560,8 @@ AttentionPlanReport attention_f32_plan_report(size_t contexts, size_t sequence, 
         report.items = report.items_expected = contexts;
         return report;
     }
-    const bool fast = vec && fits_buffer && (biased ? head_dim <= 64 && sequence % 4 == 0 : head_dim <= 128);
+    const bool bias_fits = sequence * (sequence + 256) * sizeof(float) < (1ull << 31);
+    const bool fast = vec && fits_buffer && (biased ? head_dim <= 64 && bias_fits : head_dim <= 128);
     if (!fast) {
         report.kernel = ST_HIP_ATTN_KERNEL_GENERAL;  // one workgroup per (context, query tile), decoded by division
         report.workgroups = contexts * static_cast<size_t>(args.q_tiles);
@@ -1112,6 +1627,7 @@ hipError_t launch_attention_f32(size_t contexts, size_t sequence, size_t head_di
     args.contexts = static_cast<int>(contexts);
     args.S = static_cast<int>(sequence);
     args.D = static_cast<int>(head_dim);
+    args.bq = kBQ;
     args.q_tiles = static_cast<int>((sequence + kBQ - 1) / kBQ);
     const size_t blocks = contexts * static_cast<size_t>(args.q_tiles);
     if (blocks > 0x7fffffffu) return hipErrorInvalidConfiguration;
@@ -1126,18 +1642,30 @@ hipError_t launch_attention_f32(size_t contexts, size_t sequence, size_t head_di
     const bool vec = (head_dim % 4 == 0) && aligned(q) && aligned(k) && aligned(v) && aligned(out);
     // The fast kernel addresses one context through a 32-bit buffer range.
     const bool fits_buffer = sequence * head_dim * sizeof(float) < (1ull << 31);
+    const bool bias_fits = sequence * (sequence + 256) * sizeof(float) < (1ull << 31);  // rows past the end included
     // Many contexts of at most 64 positions: a wavefront per context.
     if (!bias && vec && fits_buffer && head_dim <= 128 && sequence <= 64 && contexts >= 256) {
         if (head_dim <= 32) return causal ? launch_tiny<32, true>(args, stream) : launch_tiny<32, false>(args, stream);
         if (head_dim <= 64) return causal ? launch_tiny<64, true>(args, stream) : launch_tiny<64, false>(args, stream);
         return causal ? launch_tiny<128, true>(args, stream) : launch_tiny<128, false>(args, stream);
     }
+    // Head sizes up to 64 on the bf16 matrix cores.
+    if (vec && fits_buffer && head_dim <= 64 && !sums_in_reference_order(head_dim, scale) && (!bias || bias_fits)) {
+        args.bq = query_rows(contexts, sequence, head_dim, causal);
+        args.q_tiles = static_cast<int>((sequence + args.bq - 1) / args.bq);
+        if (head_dim <= 32) {
+            if (bias) return causal ? launch_split<32, true, true>(args, stream) : launch_split<32, false, true>(args, stream);
+            return causal ? launch_split<32, true, false>(args, stream) : launch_split<32, false, false>(args, stream);
+        }
+        if (bias) return causal ? launch_split<64, true, true>(args, stream) : launch_split<64, false, true>(args, stream);
+        return causal ? launch_split<64, true, false>(args, stream) : launch_split<64, false, false>(args, stream);
+    }
     if (!bias && vec && fits_buffer && head_dim <= 128) {
         if (head_dim <= 32) return causal ? launch_fast<32, true>(args, stream) : launch_fast<32, false>(args, stream);
         if (head_dim <= 64) return causal ? launch_fast<64, true>(args, stream) : launch_fast<64, false>(args, stream);
         return causal ? launch_fast<128, true>(args, stream) : launch_fast<128, false>(args, stream);
     }
-    // The same kernel with the additive biases folded in, where their rows can be read 128 bits at a time.
+    // The same with the additive biases folded in, where their rows can be read 128 bits at a time.
     const bool bias_vec = sequence % 4 == 0 && aligned(z_bias) && aligned(attn_bias);
     if (bias && bias_vec && vec && fits_buffer && head_dim <= 64) {
         if (head_dim <= 32) return causal ? launch_fast<32, true, true>(args, stream) : launch_fast<32, false, true>(args, stream);

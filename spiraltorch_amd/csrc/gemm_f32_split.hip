@@ -15,7 +15,7 @@
 // (223 TFLOP/s), 1576×3072×768 70 -> 48, A stored k×m 3072×768×1576 100 -> 62, B prepacked 2384×1120×3708 243 -> 133,
 // and where rows are unaligned or k is no multiple of 16 853×1399×1747 114 -> 43, 182×425×2895 161 -> 20 µs.
 //
-// Values for which the three pieces are not exact (non-finite, 2^127 and more, whole operand rows below 2^-100) are found
+// Values for which the three pieces are not exact (non-finite, 2^127 and more, whole operand rows below 2^-110) are found
 // by the splitting pass; the tiles they touch are computed with f32 multiply-adds from the original operands.
 #include <algorithm>
 #include <type_traits>
@@ -40,7 +40,7 @@ typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 // product kernel needs no edge cases, and any m, n, k and alignment of the operands is served alike.
 //
 // Beside every pair of blocks along k, 16 bytes of status: bit r of word 0 is set when row r holds a non-zero value
-// there, bit r of word 1 when it holds one of at least 2^-100, word 2 is non-zero when some value is 2^127 or more or not
+// there, bit r of word 1 when it holds one of at least 2^-110, word 2 is non-zero when some value is 2^127 or more or not
 // finite.
 struct SplitJob {
     const float *src;
@@ -119,7 +119,7 @@ __global__ __launch_bounds__(256) void split_operands_kernel(SplitJob first, Spl
             piece[2][e] = pack_bf16x2_rne(la, lb);
             const float most = fmaxf(fabsf(a), fabsf(b));
             nz |= most > 0.0f;
-            ord |= most >= 0x1p-100f;
+            ord |= most >= 0x1p-110f;
             // (a NaN fails the comparison; fmaxf alone would drop it)
             wild |= !(fabsf(a) < 0x1p127f) | !(fabsf(b) < 0x1p127f);
         }

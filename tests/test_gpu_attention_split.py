@@ -1,0 +1,74 @@
+"""f32 attention on the bf16 matrix cores (head sizes up to 64), every value as three exact bf16 pieces, against float64."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def exact(q, k, v, scale, causal, z_bias=None, attn_bias=None):
+    logits = (q.astype(np.float64) @ k.astype(np.float64).T) * scale
+    if z_bias is not None:
+        logits = logits + z_bias.astype(np.float64)[None]
+    if attn_bias is not None:
+        logits = logits + attn_bias.astype(np.float64)
+    if causal:
+        logits = np.where(np.tril(np.ones(logits.shape, bool)), logits, -np.inf)
+    w = np.exp(logits - logits.max(axis=1, keepdims=True))
+    return (w / w.sum(axis=1, keepdims=True)) @ v.astype(np.float64)
+
+
+def run(hip, q, k, v, scale, causal, z_bias=None, attn_bias=None):
+    contexts, seq, dim = q.shape
+    up = lambda a: None if a is None else hip.DeviceBuffer.from_array(a)
+    d_out = hip.DeviceBuffer.from_array(np.full(q.size + 64, 7.5, np.float32))
+    keep = [up(a) for a in (q, k, v, z_bias, attn_bias)]
+    hip.attention_f32_dev(contexts, seq, dim, scale, causal, *keep, d_out)
+    hip.device_synchronize()
+    out = d_out.to_array(np.float32, q.size + 64)
+    assert (out[q.size:] == 7.5).all(), "wrote past the end of the result"
+    return out[:q.size].reshape(q.shape)
+
+
+# Query tiles of 128 and (from 256 workgroups on) of 256 rows, one key past a stage, short heads, biases on rows of any
+# length (a row's last group of four keys reaches into the next row or past the tensor), keys split over workgroups.
+@pytest.mark.parametrize("contexts,seq,dim,causal,biased", [
+    (1, 1, 64, False, True), (2, 65, 64, True, False), (3, 129, 60, False, True), (2, 191, 36, True, True), (1, 777, 64, False, True),
+    (5, 333, 32, False, False), (4, 1001, 64, True, True), (2, 1025, 20, False, True), (128, 513, 64, True, False), (90, 641, 64, False, False),
+    (128, 385, 32, True, False), (86, 515, 64, False, True)])
+def test_against_float64(hip, contexts, seq, dim, causal, biased):
+    rng = np.random.default_rng(seq + dim)
+    q, k, v = (rng.normal(size=(contexts, seq, dim)).astype(np.float32) for _ in range(3))
+    zb = rng.normal(0, 0.5, (contexts, seq)).astype(np.float32) if biased else None
+    ab = rng.normal(0, 0.5, (contexts, seq, seq)).astype(np.float32) if biased else None
+    for scale in (1.0 / np.sqrt(dim), -0.3):
+        got = run(hip, q, k, v, scale, causal, zb, ab)
+        for c in sorted({0, contexts // 2, contexts - 1}):
+            want = exact(q[c], k[c], v[c], float(np.float32(scale)), causal, None if zb is None else zb[c], None if ab is None else ab[c])
+            # Logits of magnitude L (under 16 here) carry a few roundings of 2^-24·L, which the exponential turns into
+            # relative errors of the weights; the weighted sum averages them.  A missing piece costs 2^-17 and more.
+            error = got[c] - want
+            assert np.sqrt(np.mean(error ** 2)) <= 2.0 ** -20 * np.sqrt(np.mean(want ** 2))
+            assert np.abs(error).max() <= 2.0 ** -15
+
+
+def test_values_the_pieces_cannot_carry(hip):
+    rng = np.random.default_rng(9)
+    q, k, v = (rng.normal(size=(4, 300, 64)).astype(np.float32) for _ in range(3))
+    clean = run(hip, q, k, v, 0.125, True)
+    q2, k2, v2 = q.copy(), k.copy(), v.copy()
+    k2[0, 290] = -np.inf          # seen by the last rows only: weight 0 or NaN, as in f32 arithmetic
+    q2[0, 290:] = np.abs(q2[0, 290:])
+    v2[1, 40, 3] = np.inf
+    v2[2, :, 7] *= np.float32(2.0 ** -121)
+    q2[3, 5] *= np.float32(2.0 ** 45)
+    k2[3, :6] *= np.float32(2.0 ** -45)
+    got = run(hip, q2, k2, v2, 0.125, True)
+    assert np.isfinite(got[0, :290]).all() and (got[0, :256] == clean[0, :256]).all() and np.isfinite(got[0, 290:]).all()
+    want = exact(q2[0, 290:291], k2[0, :290], v2[0, :290], 0.125, False)
+    assert np.abs(got[0, 290] - want[0]).max() <= 2.0 ** -15
+    assert not np.isfinite(got[1, 40:, 3]).any() and np.isfinite(got[1, :40]).all() and np.isfinite(np.delete(got[1], 3, axis=1)).all()
+    want = exact(q2[2], k2[2], v2[2], 0.125, True)
+    assert (np.abs(got[2, :, 7] - want[:, 7]) <= 2.0 ** -18 * 2.0 ** -119).all()  # its own magnitude, not that of the other columns
+    assert np.abs(got[2] - want).max() <= 2.0 ** -15
+    want = exact(q2[3], k2[3], v2[3], 0.125, True)
+    assert np.abs(got[3] - want).max() <= 2.0 ** -15
