@@ -709,77 +709,97 @@ __global__ __launch_bounds__(256) void row_softmax_split_write_kernel(int cols, 
     }
 }
 
-// The same for softmax: the row stays in the registers of a 1024-thread workgroup through all three phases.
-template <int CH>
-__global__ __launch_bounds__(1024) void row_softmax_block_kernel(int cols, const float *in, float *out)
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+// The same for softmax: the row stays in the registers of a 512-thread workgroup through all three phases.  A launch is
+// bound by memory, and a workgroup only uses it in its first and last phase: what counts is that a compute unit holds two
+// rows at a time, so that one is loaded or stored while the other is reduced.  25 pieces a thread (51200 values) still do
+// (128 registers a wavefront, four wavefronts per SIMD); with 1024 threads and the row padded to 65536 values one row
+// filled the unit.  The index a row without a usable sum needs is found by reading the row again: no row of ordinary
+// values pays for it.
+// 1024 × 50257 115 -> 102 µs, × 40000 78 -> 63, × 32000 53 -> 39 (6.7 TB/s), 2048 × 5001 20.5 -> 14.3, 4 × 50257 14 -> 9.7.
+template <int CH, int THREADS>
+__device__ __forceinline__ void row_softmax_block_body(int cols, const float *in, float *out)
 {
-    __shared__ float scratch_f[16];
-    __shared__ int scratch_i[16];
+    __shared__ float scratch_f[THREADS / 64];
+    __shared__ int scratch_i[THREADS / 64];
     const int tid = threadIdx.x;
     const float *x = in + static_cast<size_t>(blockIdx.x) * cols;
     float *y = out + static_cast<size_t>(blockIdx.x) * cols;
+    // (Buffer accesses: an offset register each instead of a 64-bit address, of which the compiler keeps one per piece.)
+    const __amdgpu_buffer_rsrc_t rsrc_x = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(x), 0, cols * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc_y = __builtin_amdgcn_make_buffer_rsrc(y, 0, cols * 4, 0x00020000);
+    // A piece that would pass the end of the row is read from the row's last four values instead; the ones before the
+    // piece's own start are another thread's and count as -inf here, as NaN entries do (skipped: a weight of zero).
     float v[CH][4];
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
-        const int c = (tid + 1024 * i) * 4;
-        if (c + 4 <= cols) {
-            const f32x4_a4 t = *reinterpret_cast<const f32x4_a4 *>(x + c);
-            v[i][0] = t[0]; v[i][1] = t[1]; v[i][2] = t[2]; v[i][3] = t[3];
-        } else {
+        const f32x4 t = __builtin_bit_cast(
+            f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_x, min((tid + THREADS * i) * 4, cols - 4) * 4, 0, 0));
+        v[i][0] = t[0]; v[i][1] = t[1]; v[i][2] = t[2]; v[i][3] = t[3];
+    }
+    // The piece offsets of each phase are computed anew from a copy of the thread index the compiler takes for another
+    // value: it would keep all of them from the first phase to the last, a register per piece.
+    int tid_mask = tid;
+    asm volatile("" : "+v"(tid_mask));
+    float best = -INFINITY;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[i][e] = c + e < cols ? x[c + e] : __builtin_nanf("");  // skipped like NaN entries
+    for (int i = 0; i < CH; ++i) {
+        const int ahead = (tid_mask + THREADS * i) * 4 - (cols - 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[i][e] = e >= ahead ? fmaxf(v[i][e], -INFINITY) : -INFINITY;
+            best = fmaxf(best, v[i][e]);
         }
     }
-    float best = -INFINITY;
-    int best_index = 0x7fffffff;
-#pragma unroll
-    for (int i = 0; i < CH; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {  // ascending columns per thread: the first occurrence wins
-            const float value = v[i][e];
-            if (value != value) continue;
-            if (best_index == 0x7fffffff || value > best) {
-                best = value;
-                best_index = (tid + 1024 * i) * 4 + e;
-            }
-        }
-    const float row_max = block_reduce<1024>(best_index == 0x7fffffff ? -INFINITY : best, scratch_f,
-                                             [](float a, float b) { return fmaxf(a, b); });
-    const int candidate = block_reduce<1024>((best_index != 0x7fffffff && best == row_max) ? best_index : 0x7fffffff, scratch_i,
-                                             [](int a, int b) { return min(a, b); });
-    const bool found = candidate != 0x7fffffff;
-    const float base = (found && isfinite(row_max)) ? row_max : 0.0f;
+    const float row_max = block_reduce<THREADS>(best, scratch_f, [](float a, float b) { return fmaxf(a, b); });
+    const float base = isfinite(row_max) ? row_max : 0.0f;
     float denom = 0.0f;
 #pragma unroll
     for (int i = 0; i < CH; ++i)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const float value = v[i][e];
-            const float weight = (!found || value != value) ? 0.0f : __expf(value - base);
-            v[i][e] = weight;
-            denom += weight;
+            v[i][e] = __expf(v[i][e] - base);
+            denom += v[i][e];
         }
-    denom = block_reduce<1024>(denom, scratch_f, [](float a, float b) { return a + b; });
-    const bool normal = isfinite(denom) && denom > 1.1920929e-7f;
-    const float inv = normal ? 1.0f / denom : 0.0f;
+    denom = block_reduce<THREADS>(denom, scratch_f, [](float a, float b) { return a + b; });
+    if (!(isfinite(denom) && denom > 1.1920929e-7f)) {
+        // one at the first entry that holds the maximum, if there is an entry at all
+        int first = 0x7fffffff;
+        for (int c = tid; c < cols; c += THREADS)
+            if (x[c] == row_max) {
+                first = c;
+                break;
+            }
+        first = block_reduce<THREADS>(first, scratch_i, [](int a, int b) { return min(a, b); });
+        for (int c = tid; c < cols; c += THREADS) y[c] = c == first ? 1.0f : 0.0f;
+        return;
+    }
+    const float inv = 1.0f / denom;
+    int tid_store = tid;
+    asm volatile("" : "+v"(tid_store));
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
-        const int c = (tid + 1024 * i) * 4;
-        if (c >= cols) continue;
-        float o[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            o[e] = v[i][e] * inv;
-            if (found && !normal) o[e] = (c + e == candidate) ? 1.0f : 0.0f;
-        }
+        const int c = (tid_store + THREADS * i) * 4;
         if (c + 4 <= cols) {
-            *reinterpret_cast<f32x4_a4 *>(y + c) = f32x4_a4{o[0], o[1], o[2], o[3]};
+            const f32x4 o = {v[i][0] * inv, v[i][1] * inv, v[i][2] * inv, v[i][3] * inv};
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), rsrc_y, c * 4, 0, 0);
         } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                if (c + e < cols) y[c + e] = o[e];
+                if (c < cols && e >= c - (cols - 4)) y[cols - 4 + e] = v[i][e] * inv;
         }
     }
+}
+template <int CH>
+__global__ __launch_bounds__(512, 4) void row_softmax_block_kernel(int cols, const float *in, float *out)
+{
+    row_softmax_block_body<CH, 512>(cols, in, out);
+}
+// Up to 65536 values: more than 25 pieces a thread do not leave room for a second row.
+__global__ __launch_bounds__(1024) void row_softmax_block_wide_kernel(int cols, const float *in, float *out)
+{
+    row_softmax_block_body<16, 1024>(cols, in, out);
 }
 
 // Gelu::forward, crates/st-nn/src/layers/gelu.rs:78-94 (the tanh form of crates/st-tensor/src/pure.rs:12026-12031).
@@ -1199,14 +1219,15 @@ hipError_t launch_row_softmax_f32(size_t rows, size_t cols, const float *in, flo
         hipLaunchKernelGGL(row_softmax_split_partial_kernel, split_grid, dim3(256), 0, stream, c, seg, in, parts);
         hipLaunchKernelGGL(row_softmax_split_write_kernel, split_grid, dim3(256), 0, stream, c, seg, in, parts, out);
     } else if (cols > 4096 && cols <= 65536) {
-        // The row in the registers of a 1024-thread workgroup: 2 to 16 pieces of 16 bytes per thread.
+        // The row in the registers of a workgroup: 4 to 25 pieces of 16 bytes per thread, 16 in the wide kernel.
         const dim3 rows_grid(static_cast<unsigned>(rows));
-        const size_t pieces = (cols + 4095) / 4096;
-        if (pieces <= 2) hipLaunchKernelGGL(row_softmax_block_kernel<2>, rows_grid, dim3(1024), 0, stream, c, in, out);
-        else if (pieces <= 4) hipLaunchKernelGGL(row_softmax_block_kernel<4>, rows_grid, dim3(1024), 0, stream, c, in, out);
-        else if (pieces <= 8) hipLaunchKernelGGL(row_softmax_block_kernel<8>, rows_grid, dim3(1024), 0, stream, c, in, out);
-        else if (pieces <= 12) hipLaunchKernelGGL(row_softmax_block_kernel<12>, rows_grid, dim3(1024), 0, stream, c, in, out);
-        else hipLaunchKernelGGL(row_softmax_block_kernel<16>, rows_grid, dim3(1024), 0, stream, c, in, out);
+        const size_t pieces = (cols + 2047) / 2048;
+        if (pieces <= 4) hipLaunchKernelGGL(row_softmax_block_kernel<4>, rows_grid, dim3(512), 0, stream, c, in, out);
+        else if (pieces <= 8) hipLaunchKernelGGL(row_softmax_block_kernel<8>, rows_grid, dim3(512), 0, stream, c, in, out);
+        else if (pieces <= 16) hipLaunchKernelGGL(row_softmax_block_kernel<16>, rows_grid, dim3(512), 0, stream, c, in, out);
+        else if (pieces <= 20) hipLaunchKernelGGL(row_softmax_block_kernel<20>, rows_grid, dim3(512), 0, stream, c, in, out);
+        else if (pieces <= 25) hipLaunchKernelGGL(row_softmax_block_kernel<25>, rows_grid, dim3(512), 0, stream, c, in, out);
+        else hipLaunchKernelGGL(row_softmax_block_wide_kernel, rows_grid, dim3(1024), 0, stream, c, in, out);
     } else if (cols > 2048) {
         // A workgroup per row: 1024 threads while the rows are few, 256 once the rows alone fill the chip.
         const bool vec_long = cols % 4 == 0 && ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0;
