@@ -160,7 +160,10 @@ int st_hip_conv2d_bias_act_f32(size_t batch, size_t c_in, size_t h, size_t w, si
 
 /* Which kernel the dispatcher runs for a convolution.  The choice is made from the shape alone (plus 16-byte
  * alignment of the weight and output pointers, assumed here); st_hip_conv2d_planned_kernel reports it for the forward
- * pass (direction 0) or for grad_input of that forward shape (direction 1) as one of ST_HIP_CONV_KERNEL_*.
+ * pass (direction 0) or for grad_input of that forward shape (direction 1) as one of ST_HIP_CONV_KERNEL_*.  Large layers
+ * run on the bf16 matrix cores instead, as products of three exact bf16 pieces per value, while no family is forced and
+ * the stream's scratch memory can hold the pieces; the query then names the kernel that serves them where it cannot (under
+ * capture before a first call, or out of memory).
  * st_hip_conv2d_force_family is a process-wide diagnostic switch (the parity tests use it to run every family on
  * small shapes): with a family forced, a convolution whose shape that family cannot serve fails with
  * ST_HIP_ERR_UNSUPPORTED instead of silently running another kernel, and the query reports 0 for it.  No reference
@@ -323,7 +326,8 @@ int st_hip_conv2d_grad_input_f32_dev(size_t batch, size_t c_in, size_t h, size_t
  * layers whose adjoint gather is wasteful do not go through the per-image GEMM + col2im route (reported as
  * ST_HIP_CONV_KERNEL_COL2IM: the gather kernel runs instead, correct but up to three orders of magnitude slower on
  * patch-embedding-like shapes — such callers should give the allocating entry point one warm-up call outside the
- * capture instead).  For every other shape the kernels, and the result bits, are those of the allocating entry point.
+ * capture instead).  Nor are large layers run as products of bf16 pieces (closer to the exact sum, not the same bits).  For
+ * every other shape the kernels, and the result bits, are those of the allocating entry point.
  * c_out*c_in*kh*kw*4 bytes must fit the array, otherwise ST_HIP_ERR_UNSUPPORTED (nothing is launched).  Every call on a
  * GPU shares that GPU's array: calls that overlap on one GPU (different streams or threads) race; calls on one stream
  * are ordered and safe.  st_hip_init must have succeeded first. */

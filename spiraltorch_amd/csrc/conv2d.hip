@@ -24,6 +24,7 @@
 #include "kernels.h"
 
 #include <atomic>
+#include <cmath>
 #include <type_traits>
 
 namespace sthip {
@@ -1095,6 +1096,32 @@ int choose_conv_kernel(const ConvShape &shape, bool weight_aligned, bool out_ali
 
 void set_conv_forced_family(int family) { g_forced_family.store(family, std::memory_order_relaxed); }
 
+// What the f32 kernels take for a layer, from below (measured: 64 -> 128 channels on 56×56, batch 32, strip kernel 144 µs;
+// 256 -> 256 on 14×14 ring kernel 99, 512 -> 512 on 7×7 in slices 119, 24 -> 96 5×5 on 112×112, batch 4, general kernel 105):
+// a rate per kernel over what its tiles of 64 pixels of an image and 64 or 128 channels cover.
+bool conv2d_f32_split_preferred(const ConvShape &s, bool weight_aligned, bool out_aligned, bool keep_strip)
+{
+    if (g_forced_family.load(std::memory_order_relaxed) != ST_HIP_CONV_FAMILY_AUTO) return false;
+    if (s.batch == 0 || s.c_out == 0 || s.oh == 0 || s.ow == 0) return false;
+    StripArgs strip;
+    const int kernel = choose_conv_kernel(s, weight_aligned, out_aligned, ST_HIP_CONV_FAMILY_AUTO, strip);
+    const double spatial = static_cast<double>(s.oh) * s.ow, terms = static_cast<double>(s.c_in) * s.kh * s.kw;
+    const double tile_oc = s.c_out > 64 ? 128.0 : 64.0;
+    const double covered = 2.0 * s.batch * (std::ceil(spatial / 64.0) * 64.0) * (std::ceil(s.c_out / tile_oc) * tile_oc) * terms;
+    double us;
+    switch (kernel) {
+    case ST_HIP_CONV_KERNEL_RING: us = 5.0 + covered / 95.0e6; break;
+    case ST_HIP_CONV_KERNEL_TILE: us = 10.0 + covered / 80.0e6; break;
+    case ST_HIP_CONV_KERNEL_TILE_KSLICED: us = 12.0 + covered / 72.0e6; break;
+    case ST_HIP_CONV_KERNEL_DIRECT: return false;
+    default:
+        if (keep_strip) return false;
+        us = 5.0 + 2.0 * s.batch * spatial * s.c_out * terms / 112.0e6;
+        break;
+    }
+    return conv2d_f32_split_applies(s, us);
+}
+
 int planned_conv_kernel(const ConvShape &shape, bool weight_aligned, bool out_aligned)
 {
     StripArgs strip;
@@ -1131,6 +1158,10 @@ hipError_t launch_conv2d_f32(const ConvShape &shape, int activation, const float
         return hipErrorInvalidValue;
     const bool weight_aligned = (reinterpret_cast<uintptr_t>(weight) & 15u) == 0;
     const bool out_aligned = (reinterpret_cast<uintptr_t>(out) & 15u) == 0;
+    if (scratch == kConvScratchStream && scratch_offset == 0 && conv2d_f32_split_preferred(shape, weight_aligned, out_aligned, false)) {
+        const hipError_t rc = launch_conv2d_f32_split(shape, activation, input, weight, false, bias, out, stream);
+        if (!scratch_unavailable(rc)) return rc;
+    }
     StripArgs strip;
     const int kernel = choose_conv_kernel(shape, weight_aligned, out_aligned,
                                           g_forced_family.load(std::memory_order_relaxed), strip, scratch == kConvScratchStream);

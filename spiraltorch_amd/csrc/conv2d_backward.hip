@@ -584,6 +584,10 @@ hipError_t launch_conv2d_grad_input_f32(const ConvShape &shape, const float *gra
     ConvShape t;
     const bool as_forward = grad_input_as_forward(shape, t);
     hipError_t rc;
+    if (as_forward && weight_scratch == nullptr && conv2d_f32_split_preferred(t, true, (reinterpret_cast<uintptr_t>(grad_input) & 15u) == 0, true)) {
+        rc = launch_conv2d_f32_split(t, ST_HIP_ACT_NONE, grad_output, weight, true, nullptr, grad_input, stream);
+        if (!scratch_unavailable(rc)) return rc;
+    }
     if (!as_forward && weight_scratch == nullptr && grad_input_by_col2im(shape)) {
         const size_t m = static_cast<size_t>(shape.oh) * shape.ow, S = static_cast<size_t>(shape.c_in) * shape.kh * shape.kw;
         const size_t image_cols = m * S;

@@ -22,6 +22,7 @@
 
 #include "device_math.h"
 #include "kernels.h"
+#include "split_product.h"
 
 namespace sthip {
 
@@ -29,9 +30,6 @@ namespace {
 
 typedef __attribute__((address_space(3))) void *lds_void_ptr;
 typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
-
-#define ST_SPLIT_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (7 << 4) | (15 << 8) | ((((n) >> 4) & 3) << 14))
-#define ST_SPLIT_FENCE() __builtin_amdgcn_sched_barrier(0)
 
 // ---- the splitting pass ------------------------------------------------------------------------------------------
 // An operand of `rows` rows along a reduction of `k` terms becomes blocks of 32 rows × 16 terms.  A block is three
@@ -108,20 +106,14 @@ __global__ __launch_bounds__(256) void split_operands_kernel(SplitJob first, Spl
             x[0] = v0.x; x[1] = v0.y; x[2] = v0.z; x[3] = v0.w; x[4] = v1.x; x[5] = v1.y; x[6] = v1.z; x[7] = v1.w;
         }
         uint32_t piece[3][4];
+        split_pieces(x, piece);
         bool nz = false, ord = false;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float a = x[2 * e], b = x[2 * e + 1];
-            piece[0][e] = pack_bf16x2_rne(a, b);
-            const float ra = a - __uint_as_float(piece[0][e] << 16), rb_ = b - __uint_as_float(piece[0][e] & 0xffff0000u);
-            piece[1][e] = pack_bf16x2_rne(ra, rb_);
-            const float la = ra - __uint_as_float(piece[1][e] << 16), lb = rb_ - __uint_as_float(piece[1][e] & 0xffff0000u);
-            piece[2][e] = pack_bf16x2_rne(la, lb);
-            const float most = fmaxf(fabsf(a), fabsf(b));
+        for (int e = 0; e < 8; e += 2) {
+            const float most = fmaxf(fabsf(x[e]), fabsf(x[e + 1]));
             nz |= most > 0.0f;
-            ord |= most >= 0x1p-110f;
-            // (a NaN fails the comparison; fmaxf alone would drop it)
-            wild |= !(fabsf(a) < 0x1p127f) | !(fabsf(b) < 0x1p127f);
+            ord |= most >= kSplitOrdinary;
+            wild |= split_wild(x[e]) | split_wild(x[e + 1]);
         }
         const unsigned long long nz64 = __ballot(nz), ord64 = __ballot(ord);
         nonzero |= static_cast<unsigned>(nz64) | static_cast<unsigned>(nz64 >> 32);
@@ -199,12 +191,9 @@ __device__ __forceinline__ bool split_status_bad(const SplitGemmArgs &p, int ra,
 template <int BM, int BN, int WM, int WN, int STAGES>
 __device__ __forceinline__ void gemm_f32_split_body(const SplitGemmArgs &p)
 {
-    constexpr int WAVES = WM * WN;
-    constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN = WTN / 32;
-    constexpr int PIECES = (BM + BN) / 32 * 3;  // 1 KB pieces of a 16-term stage
-    constexpr int LOADS = (PIECES + WAVES - 1) / WAVES;
-    constexpr int STAGE = PIECES * 1024;
-    constexpr int SLOTS = TM * TN, SPREAD = TM + TN;
+    using Tile = SplitTile<BM, BN, WM, WN, STAGES>;
+    constexpr int WTM = Tile::WTM, WTN = Tile::WTN, TM = Tile::TM, TN = Tile::TN;
+    constexpr int PIECES = Tile::PIECES, LOADS = Tile::LOADS, STAGE = Tile::STAGE;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_bytes[];
 
     const int tid = threadIdx.x;
@@ -242,127 +231,19 @@ __device__ __forceinline__ void gemm_f32_split_body(const SplitGemmArgs &p)
         piece_off[i] = (block < BM / 32 ? 0u : p.b_base) + (row_block * p.ksteps + step0) * 3072u + plane * 1024u;
     }
     const unsigned lane_off = lane * 16;
-    auto load = [&](int stage, int i, int step, unsigned off) {
+    struct Where {
+        unsigned step_off, lane_off;  // past the last step: outside the buffer (zeros, no memory access)
+    };
+    auto load = [&](int stage, int i, const Where &where) {
         const int q = min(wave * LOADS + i, PIECES - 1);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_ptr)(lds_bytes + stage * STAGE + q * 1024), 16, off,
-                                                 piece_off[i] + step * 3072u, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_ptr)(lds_bytes + stage * STAGE + q * 1024), 16, where.lane_off,
+                                                 piece_off[i] + where.step_off, 0, 0);
     };
 
-    // hi·hi and the five small products accumulate apart and are added at the end: a small product then never rounds
-    // against the large sum, and the result carries one rounding per sixteen terms.
-    f32x16 acc[TM][TN], fine[TM][TN];
-#pragma unroll
-    for (int a = 0; a < TM; ++a)
-#pragma unroll
-        for (int b = 0; b < TN; ++b)
-            acc[a][b] = fine[a][b] = f32x16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-
-    bf16x8 a_hi[TM], a_mid[TM], a_lo[TM], b_hi[2][TN], b_mid[TN], b_lo[TN];
-    const unsigned a_frag = wm * TM * 3072 + lane_off, b_frag = (BM / 32 + wn * TN) * 3072 + lane_off;
-    auto frag_a = [&](int stage, int t, int plane) {
-        return *reinterpret_cast<const bf16x8 *>(lds_bytes + stage * STAGE + a_frag + t * 3072 + plane * 1024);
-    };
-    auto frag_b = [&](int stage, int t, int plane) {
-        return *reinterpret_cast<const bf16x8 *>(lds_bytes + stage * STAGE + b_frag + t * 3072 + plane * 1024);
-    };
-    // The product is formed transposed (B's fragment first), so register 4g + j of lane (li, lh) is
-    // C[32·tm + li][32·tn + 8g + 4·lh + j]: four neighbouring columns of a row.
-    auto product = [&](f32x16 (&sum)[TM][TN], const bf16x8 (&a)[TM], const bf16x8 (&b)[TN], auto &&memory) {
-#pragma unroll
-        for (int slot = 0; slot < SLOTS; ++slot) {
-            sum[slot / TN][slot % TN] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[slot % TN], a[slot / TN], sum[slot / TN][slot % TN], 0, 0, 0);
-            ST_SPLIT_FENCE();
-            memory(slot);
-            ST_SPLIT_FENCE();
-        }
-    };
-
-    // Step t (16 terms).  On entry the fragments lo and mid of A and hi and mid of B are in registers; the rest is read
-    // during the first product, so that every LDS read of a stage is behind its barrier, after which the stage takes
-    // the loads of step t + STAGES.  Behind the barrier come those loads and the next step's fragments, each into
-    // registers whose last use is past: one memory instruction behind an MFMA, never a burst.
-    int stage = 0;
-    auto iteration = [&](auto buf_tag, int t) {
-        constexpr int BUF = decltype(buf_tag)::value;
-        const int next = stage + 1 == STAGES ? 0 : stage + 1;
-        product(fine, a_lo, b_hi[BUF], [&](int slot) {
-            if (slot < SPREAD) {
-                if (slot < TM) a_hi[slot] = frag_a(stage, slot, 0);
-                else b_lo[slot - TM] = frag_b(stage, slot - TM, 2);
-            }
-            if (SLOTS < SPREAD && slot == SLOTS - 1) {
-#pragma unroll
-                for (int i = SLOTS; i < SPREAD; ++i) {
-                    if (i < TM) a_hi[i] = frag_a(stage, i, 0);
-                    else b_lo[i - TM] = frag_b(stage, i - TM, 2);
-                }
-            }
-        });
-        product(fine, a_mid, b_hi[BUF], [&](int) {});
-        // This wavefront's loads of step t + 1 have landed, and its LDS reads of step t have returned; the barrier extends
-        // both to every wavefront.
-        ST_SPLIT_WAIT_VMCNT((STAGES - 2) * LOADS);
-        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        // Past the last step the loads fall outside the buffer (zeros, no memory access) and the fragments read are
-        // never used: every step runs the same code.
-        const unsigned off = t + STAGES < steps ? lane_off : 0x80000000u;
-        // the memory instructions of the last four products: loads, then A's lo and B's hi, spread over three of them ...
-        auto tail = [&](int slot) {
-            constexpr int ALL = LOADS + SPREAD, PER = (ALL + 3 * SLOTS - 1) / (3 * SLOTS);
-#pragma unroll
-            for (int e = 0; e < PER; ++e) {
-                const int i = slot * PER + e, r = i - LOADS;
-                if (i < LOADS) load(stage, i, t + STAGES, off);
-                else if (r < TM) a_lo[r] = frag_a(next, r, 2);
-                else if (r < SPREAD) b_hi[BUF ^ 1][r - TM] = frag_b(next, r - TM, 0);
-            }
-        };
-        product(fine, a_mid, b_mid, [&](int slot) { tail(slot); });
-        product(fine, a_hi, b_mid, [&](int slot) { tail(SLOTS + slot); });
-        product(fine, a_hi, b_lo, [&](int slot) { tail(2 * SLOTS + slot); });
-        // ... and the mid fragments behind the last one that reads them
-        product(acc, a_hi, b_hi[BUF], [&](int slot) {
-            constexpr int PER = (SPREAD + SLOTS - 1) / SLOTS;
-#pragma unroll
-            for (int e = 0; e < PER; ++e) {
-                const int i = slot * PER + e;
-                if (i < TM) a_mid[i] = frag_a(next, i, 1);
-                else if (i < SPREAD) b_mid[i - TM] = frag_b(next, i - TM, 1);
-            }
-        });
-        stage = next;
-    };
-
-#pragma unroll
-    for (int s = 0; s < STAGES; ++s) {
-#pragma unroll
-        for (int i = 0; i < LOADS; ++i) load(s, i, s, s < steps ? lane_off : 0x80000000u);
-    }
-    const bool bad = split_status_bad<TM, TN>(p, m0 / 32 + wm * TM, n0 / 32 + wn * TN, step0 / 2, (step0 + steps) / 2, lane);
-    ST_SPLIT_WAIT_VMCNT(0);
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-        a_lo[i] = frag_a(0, i, 2);
-        a_mid[i] = frag_a(0, i, 1);
-    }
-#pragma unroll
-    for (int i = 0; i < TN; ++i) {
-        b_hi[0][i] = frag_b(0, i, 0);
-        b_mid[i] = frag_b(0, i, 1);
-    }
-    for (int t = 0; t < steps; t += 2) {
-        iteration(std::integral_constant<int, 0>{}, t);
-        iteration(std::integral_constant<int, 1>{}, t + 1);
-    }
-
-#pragma unroll
-    for (int a = 0; a < TM; ++a)
-#pragma unroll
-        for (int b = 0; b < TN; ++b) acc[a][b] += fine[a][b];
+    f32x16 acc[TM][TN];
+    const bool bad = split_product_loop<BM, BN, WM, WN, STAGES>(
+        lds_bytes, wave, lane, steps, acc, [&](int t) { return Where{t * 3072u, t < steps ? lane_off : 0x80000000u}; }, load,
+        [&] { return split_status_bad<TM, TN>(p, m0 / 32 + wm * TM, n0 / 32 + wn * TN, step0 / 2, (step0 + steps) / 2, lane); });
 
     // Epilogue through a strip of LDS per wavefront, so that stores and residual loads cover whole row segments.
     __syncthreads();

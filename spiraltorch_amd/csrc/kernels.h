@@ -93,7 +93,19 @@ hipError_t launch_conv2d_f32(const ConvShape &shape, int activation, const float
 // Bytes of the stream's scratch buffer launch_conv2d_f32 uses for `shape` (0 for most shapes).
 size_t conv2d_scratch_bytes(const ConvShape &shape, bool weight_aligned, bool out_aligned);
 
-// Which kernel launch_conv2d_f32 would run for `shape` (one of ST_HIP_CONV_KERNEL_*; 0 when the family forced with
+// The same layer on the bf16 matrix cores, operands as three exact bf16 pieces (conv2d_split.hip): a large share of what
+// launch_conv2d_f32 would serve.  `adjoint_weight`: `weight` is the forward layer's, [c_in][c_out][taps] seen from `shape`,
+// and its taps are flipped.  Fails with an error scratch_unavailable() knows, before anything is launched, where the
+// stream's scratch buffers cannot grow.  `other_us`: what the f32 kernels would take.
+bool conv2d_f32_split_applies(const ConvShape &shape, double other_us);
+hipError_t launch_conv2d_f32_split(const ConvShape &shape, int activation, const float *input, const float *weight, bool adjoint_weight,
+                                   const float *bias, float *out, hipStream_t stream);
+// The decision for a layer whose weights and output are 16-byte aligned or not; false while a kernel family is forced.
+// `keep_strip`: not where a strip kernel serves it (grad_input: a strip kernel's result for an image is promised to be the
+// same bits whatever the batch).
+bool conv2d_f32_split_preferred(const ConvShape &shape, bool weight_aligned, bool out_aligned, bool keep_strip);
+
+// Which of its kernels launch_conv2d_f32 would run for `shape` when the split product does not serve it (one of ST_HIP_CONV_KERNEL_*; 0 when the family forced with
 // set_conv_forced_family cannot serve it), and the same for launch_conv2d_grad_input_f32 on the forward `shape`.
 int planned_conv_kernel(const ConvShape &shape, bool weight_aligned, bool out_aligned);
 int planned_conv_grad_input_kernel(const ConvShape &shape);
