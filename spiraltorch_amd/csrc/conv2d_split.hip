@@ -13,7 +13,8 @@
 // pass), 128 -> 128 on 28×28 93 -> 65, 256 -> 256 on 14×14 99 -> 64, 512 -> 512 on 7×7 119 -> 72,
 // 250 -> 250 on 14×15, batch 31, 189 -> 64, 24 -> 96 5×5 on 112×112, batch 4, 105 -> 67, 256 -> 256 on 28×28, batch 2, 41 -> 30.
 // 64 -> 64 on 56×56 and one-tap layers stay on the f32 kernels (70 against 69 µs, 46 against 51): the pass costs what the
-// matrix cores save.
+// matrix cores save.  Errors against float64 are 0.34 to 0.62 of those of the kernels that ran before (rms, six layers with
+// rectified N(0,1) images).
 //
 // Values the pieces cannot carry (non-finite, 2^127 and more, whole rows below 2^-110) are found by the pass; the rows of
 // a marked tile are looked at in the original operands, and tiles that do hold such rows are computed with f32
