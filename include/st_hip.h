@@ -242,6 +242,17 @@ typedef struct {
     uint64_t workgroups, items, out_of_range, duplicates;
 } st_hip_gemm_tile_plan;
 int st_hip_gemm_bf16_tile_plan(size_t m, size_t n, size_t k, st_hip_gemm_tile_plan *plan);
+/* Whether the f32 GEMM entry points run an m×n×k product of 16-byte aligned operands on the bf16 matrix cores, as products of
+ * three exact bf16 pieces per value (`served`; the rest is 0 if not), and how it is cut: tiles, workgroups along k, 16-term
+ * steps each of them walks, the size of the split operands in the stream's scratch memory and how far into each the
+ * kernel's loads reach (`*_reach` must not exceed `*_bytes`). */
+typedef struct {
+    int served;
+    int tile_rows, tile_cols, tiles_m, tiles_n;
+    int k_splits, steps_per_split;
+    uint64_t a_bytes, a_reach, b_bytes, b_reach;
+} st_hip_gemm_split_plan;
+int st_hip_gemm_f32_split_plan(size_t m, size_t n, size_t k, int lhs_transposed, int rhs_packed, st_hip_gemm_split_plan *plan);
 /* Rows of A per launch when a GEMM whose A is 2 GiB or larger is cut into row blocks for the kernels that address
  * operands through 32-bit byte offsets: a multiple of 256 with rows*k*element_bytes < 2^31, or 0 when 256 rows do not
  * fit (such products run on the kernels with 64-bit addressing). */

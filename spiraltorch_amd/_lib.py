@@ -48,6 +48,11 @@ class GemmTilePlan(ctypes.Structure):
                 ("duplicates", c_uint64)]
 
 
+class GemmSplitPlan(ctypes.Structure):
+    _fields_ = [(name, c_int) for name in ("served", "tile_rows", "tile_cols", "tiles_m", "tiles_n", "k_splits", "steps_per_split")] + \
+        [(name, c_uint64) for name in ("a_bytes", "a_reach", "b_bytes", "b_reach")]
+
+
 class DecoderConfig(ctypes.Structure):
     _fields_ = [
         ("vocab", c_size_t),
@@ -99,6 +104,7 @@ SIGNATURES = {
     "st_hip_conv2d_planned_kernel": (c_int, [c_size_t] * 13 + [c_int, POINTER(c_int)]),
     "st_hip_attention_f32_launch_plan": (c_int, [c_size_t, c_size_t, c_size_t, c_int, c_int, POINTER(AttentionPlan)]),
     "st_hip_gemm_row_block": (c_size_t, [c_size_t, c_size_t]),
+    "st_hip_gemm_f32_split_plan": (c_int, [c_size_t, c_size_t, c_size_t, c_int, c_int, POINTER(GemmSplitPlan)]),
     "st_hip_probe_mfma_bf16_dev": (c_int, [c_size_t, c_size_t, c_void_p, c_void_p, c_void_p]),
     "st_hip_probe_mfma_f32_dev": (c_int, [c_size_t, c_size_t, c_void_p, c_void_p, c_void_p]),
     "st_hip_probe_stream_lds_dev": (c_int, [c_size_t, c_size_t, c_void_p, c_size_t, c_void_p]),

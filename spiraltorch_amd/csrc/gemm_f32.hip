@@ -926,10 +926,23 @@ double f32_kernels_us(size_t m, size_t n, size_t k, bool lhs_transposed, bool rh
     return 5.0 + unpack + std::max(flops / (aligned ? 80.0e6 : 60.0e6), (aligned ? 0.6 : 0.75) * k_tiles) + flops / 200.0e6;
 }
 
+bool f32_split_preferred(size_t m, size_t n, size_t k, bool lhs_transposed, bool rhs_packed, const float *lhs, const float *rhs, bool scratch_free)
+{
+    return gemm_f32_split_applies(m, n, k, f32_kernels_us(m, n, k, lhs_transposed, rhs_packed, lhs, rhs, scratch_free), scratch_free);
+}
+
 hipError_t launch_gemm_f32_native(size_t m, size_t n, size_t k, bool lhs_transposed, const float *lhs, const float *rhs, float *out,
                                   const GemmEpilogue &epilogue, hipStream_t stream, bool scratch_free);
 
 }  // namespace
+
+bool gemm_f32_split_served(size_t m, size_t n, size_t k, bool lhs_transposed, bool rhs_packed)
+{
+    const float *const aligned = reinterpret_cast<const float *>(16);
+    if (m == 0 || n == 0) return false;
+    if (!rhs_packed && (lhs_transposed ? gemv_t_f32_applies(m, n, k) : gemv_f32_applies(m, n, k, aligned, aligned))) return false;
+    return f32_split_preferred(m, n, k, lhs_transposed, rhs_packed, aligned, aligned, true);
+}
 
 hipError_t launch_gemm_f32(size_t m, size_t n, size_t k, bool lhs_transposed, const float *lhs,
                            const float *rhs, float *out, const GemmEpilogue &epilogue, hipStream_t stream, bool scratch_free)
@@ -937,7 +950,7 @@ hipError_t launch_gemm_f32(size_t m, size_t n, size_t k, bool lhs_transposed, co
     if (m == 0 || n == 0) return hipSuccess;
     if (!lhs_transposed && gemv_f32_applies(m, n, k, lhs, rhs)) return launch_gemv_f32(m, n, k, lhs, rhs, out, epilogue, stream);
     if (lhs_transposed && scratch_free && gemv_t_f32_applies(m, n, k)) return launch_gemv_t_f32(m, n, k, lhs, rhs, out, epilogue, stream);
-    if (gemm_f32_split_applies(m, n, k, f32_kernels_us(m, n, k, lhs_transposed, false, lhs, rhs, scratch_free), scratch_free)) {
+    if (f32_split_preferred(m, n, k, lhs_transposed, false, lhs, rhs, scratch_free)) {
         const hipError_t rc = launch_gemm_f32_split(m, n, k, lhs_transposed, lhs, false, rhs, out, epilogue, stream, scratch_free);
         if (!scratch_unavailable(rc)) return rc;
     }
@@ -1086,7 +1099,7 @@ hipError_t launch_gemm_f32_packed(size_t m, size_t n, size_t k, const float *lhs
                                   const GemmEpilogue &epilogue, hipStream_t stream)
 {
     if (m == 0 || n == 0) return hipSuccess;
-    if (gemm_f32_split_applies(m, n, k, f32_kernels_us(m, n, k, false, true, lhs, packed_rhs, true), true)) {
+    if (f32_split_preferred(m, n, k, false, true, lhs, packed_rhs, true)) {
         const hipError_t rc = launch_gemm_f32_split(m, n, k, false, lhs, true, packed_rhs, out, epilogue, stream, true);
         if (!scratch_unavailable(rc)) return rc;
     }

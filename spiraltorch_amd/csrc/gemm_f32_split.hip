@@ -128,6 +128,16 @@ __global__ __launch_bounds__(256) void split_operands_kernel(SplitJob first, Spl
 }
 
 // ---- the product -------------------------------------------------------------------------------------------------
+// Where the row block `block` of a tile that starts at row `first` lies for reduction step `step`, in bytes from the start
+// of its operand's blocks.  Tiles reach past the last row block; they read the last one again (what that gives is not
+// stored).  These offsets go into a load's scalar offset, which its bounds check does not see: every one of them has to lie
+// inside the buffer.
+__host__ __device__ inline unsigned split_block_offset(int first, int block, int rows, int ksteps, int step)
+{
+    const int row_block = first / 32 + block, last = (rows - 1) / 32;
+    return static_cast<unsigned>((row_block < last ? row_block : last) * ksteps + step) * 3072u;
+}
+
 struct SplitGemmArgs {
     const unsigned char *blocks;  // A's blocks, then B's at b_base
     unsigned b_base, bytes;
@@ -220,15 +230,14 @@ __device__ __forceinline__ void gemm_f32_split_body(const SplitGemmArgs &p)
 
     const __amdgpu_buffer_rsrc_t rsrc =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char *>(p.blocks), 0, static_cast<int>(p.bytes), 0x00020000);
-    // Piece q of a stage: fragment q % 3 of row block q / 3 of the tile (A's blocks first).  Row blocks past the end of A
-    // read B's, those past the end of B read zeros; neither reaches a stored value.
+    // Piece q of a stage: fragment q % 3 of row block q / 3 of the tile (A's blocks first).
     unsigned piece_off[LOADS];
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
         const int q = min(wave * LOADS + i, PIECES - 1);
         const int block = q / 3, plane = q % 3;
-        const unsigned row_block = block < BM / 32 ? m0 / 32 + block : n0 / 32 + block - BM / 32;
-        piece_off[i] = (block < BM / 32 ? 0u : p.b_base) + (row_block * p.ksteps + step0) * 3072u + plane * 1024u;
+        piece_off[i] = plane * 1024u + (block < BM / 32 ? split_block_offset(m0, block, p.M, p.ksteps, step0)
+                                                        : p.b_base + split_block_offset(n0, block - BM / 32, p.N, p.ksteps, step0));
     }
     const unsigned lane_off = lane * 16;
     struct Where {
@@ -382,6 +391,28 @@ bool gemm_f32_split_applies(size_t m, size_t n, size_t k, double other_us, bool 
     const double bytes = (static_cast<double>(m) + n + 64) * (static_cast<double>(k) + 32) * 6.0;
     if (bytes >= static_cast<double>(1ull << 31)) return false;
     return plan_split(m, n, k, may_split_k).us < 0.9 * other_us;  // a tenth for the error of both estimates
+}
+
+GemmSplitPlanReport gemm_f32_split_plan_report(size_t m, size_t n, size_t k)
+{
+    const SplitPlan plan = plan_split(m, n, k, true);
+    const SplitConfig &config = *plan.config;
+    const int ksteps = static_cast<int>((k + 31) / 32 * 2);
+    const int rows[2] = {static_cast<int>(m), static_cast<int>(n)}, tile[2] = {config.bm, config.bn};
+    GemmSplitPlanReport report{};
+    report.tile_rows = config.bm;
+    report.tile_cols = config.bn;
+    report.k_splits = plan.splits;
+    report.steps_per_split = plan.steps_per_split;
+    for (int side = 0; side < 2; ++side) {
+        const int tiles = (rows[side] + tile[side] - 1) / tile[side];
+        (side == 0 ? report.tiles_m : report.tiles_n) = tiles;
+        report.bytes[side] = static_cast<uint64_t>((rows[side] + 31) / 32) * ksteps * 3072;
+        for (int t = 0; t < tiles; ++t)
+            for (int block = 0; block < tile[side] / 32; ++block)  // the last fragment of the last step
+                report.reach[side] = std::max<uint64_t>(report.reach[side], split_block_offset(t * tile[side], block, rows[side], ksteps, ksteps - 1) + 3072ull);
+    }
+    return report;
 }
 
 hipError_t launch_gemm_f32_split(size_t m, size_t n, size_t k, bool lhs_transposed, const float *lhs, bool rhs_packed, const float *rhs,

@@ -538,6 +538,27 @@ int st_hip_gemm_bf16_tile_plan(size_t m, size_t n, size_t k, st_hip_gemm_tile_pl
     return ST_HIP_OK;
 }
 
+int st_hip_gemm_f32_split_plan(size_t m, size_t n, size_t k, int lhs_transposed, int rhs_packed, st_hip_gemm_split_plan *plan)
+{
+    if (!plan) return fail(ST_HIP_ERR_INVALID, "gemm split_plan received a null out-pointer");
+    if (m > kMaxDim || n > kMaxDim || k > kMaxDim) return fail(ST_HIP_ERR_INVALID, "gemm dimensions exceed i32");
+    *plan = st_hip_gemm_split_plan{};
+    if (!gemm_f32_split_served(m, n, k, lhs_transposed != 0, rhs_packed != 0)) return ST_HIP_OK;
+    const GemmSplitPlanReport report = gemm_f32_split_plan_report(m, n, k);
+    plan->served = 1;
+    plan->tile_rows = report.tile_rows;
+    plan->tile_cols = report.tile_cols;
+    plan->tiles_m = report.tiles_m;
+    plan->tiles_n = report.tiles_n;
+    plan->k_splits = report.k_splits;
+    plan->steps_per_split = report.steps_per_split;
+    plan->a_bytes = report.bytes[0];
+    plan->a_reach = report.reach[0];
+    plan->b_bytes = report.bytes[1];
+    plan->b_reach = report.reach[1];
+    return ST_HIP_OK;
+}
+
 size_t st_hip_gemm_row_block(size_t k, size_t element_bytes)
 {
     size_t row_bytes = 0;

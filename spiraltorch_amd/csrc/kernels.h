@@ -49,6 +49,14 @@ hipError_t launch_gemm_f32_packed(size_t m, size_t n, size_t k, const float *lhs
 bool gemm_f32_split_applies(size_t m, size_t n, size_t k, double other_us, bool may_split_k);
 hipError_t launch_gemm_f32_split(size_t m, size_t n, size_t k, bool lhs_transposed, const float *lhs, bool rhs_packed, const float *rhs,
                                  float *out, const GemmEpilogue &epilogue, hipStream_t stream, bool may_split_k);
+// Whether launch_gemm_f32 (launch_gemm_f32_packed if `rhs_packed`) runs a product of 16-byte aligned operands that way, and how
+// it is then cut: see st_hip_gemm_split_plan.
+bool gemm_f32_split_served(size_t m, size_t n, size_t k, bool lhs_transposed, bool rhs_packed);
+struct GemmSplitPlanReport {
+    int tile_rows, tile_cols, tiles_m, tiles_n, k_splits, steps_per_split;
+    uint64_t bytes[2], reach[2];  // of A's and of B's blocks
+};
+GemmSplitPlanReport gemm_f32_split_plan_report(size_t m, size_t n, size_t k);
 // out = epilogue(sum of `slices` partial planes of m×n values, added in slice order).
 hipError_t launch_f32_slice_reduce(size_t m, size_t n, size_t slices, const float *partial, float *out, const GemmEpilogue &epilogue,
                                    hipStream_t stream);

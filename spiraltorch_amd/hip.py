@@ -245,6 +245,13 @@ def gemm_bf16_tile_plan(m: int, n: int, k: int) -> dict:
     return {name: int(getattr(plan, name)) for name, _ in _lib.GemmTilePlan._fields_}
 
 
+def gemm_f32_split_plan(m: int, n: int, k: int, lhs_transposed: bool = False, rhs_packed: bool = False) -> dict:
+    """Whether and how the f32 GEMM runs a product as products of three exact bf16 pieces per value."""
+    plan = _lib.GemmSplitPlan()
+    _check(_lib.load().st_hip_gemm_f32_split_plan(m, n, k, int(bool(lhs_transposed)), int(bool(rhs_packed)), ctypes.byref(plan)))
+    return {name: int(getattr(plan, name)) for name, _ in _lib.GemmSplitPlan._fields_}
+
+
 def gemm_row_block(k: int, element_bytes: int) -> int:
     """Rows of A per launch when an A of 2 GiB or more is cut into row blocks (0: not even 256 rows fit)."""
     return int(_lib.load().st_hip_gemm_row_block(k, element_bytes))

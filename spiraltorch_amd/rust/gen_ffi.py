@@ -17,7 +17,7 @@ TARGET = os.path.join(HERE, "st-backend-hip", "src", "ffi.rs")
 SCALARS = {"size_t": "usize", "int": "c_int", "float": "f32", "uint64_t": "u64", "uint16_t": "u16", "char": "c_char",
            "void": "c_void", "st_hip_device_props": "StHipDeviceProps", "st_hip_probe_result": "StHipProbeResult",
            "st_hip_decoder_config": "StHipDecoderConfig", "st_hip_attention_plan": "StHipAttentionPlan",
-           "st_hip_gemm_tile_plan": "StHipGemmTilePlan"}
+           "st_hip_gemm_tile_plan": "StHipGemmTilePlan", "st_hip_gemm_split_plan": "StHipGemmSplitPlan"}
 RUST_KEYWORDS = {"in": "input", "type": "kind", "ref": "reference"}
 
 STRUCTS = '''/// `st_hip_device_props`.
@@ -88,6 +88,23 @@ pub struct StHipGemmTilePlan {
     pub items: u64,
     pub out_of_range: u64,
     pub duplicates: u64,
+}
+
+/// `st_hip_gemm_split_plan`.
+#[repr(C)]
+#[derive(Clone, Copy, Debug, Default, PartialEq)]
+pub struct StHipGemmSplitPlan {
+    pub served: c_int,
+    pub tile_rows: c_int,
+    pub tile_cols: c_int,
+    pub tiles_m: c_int,
+    pub tiles_n: c_int,
+    pub k_splits: c_int,
+    pub steps_per_split: c_int,
+    pub a_bytes: u64,
+    pub a_reach: u64,
+    pub b_bytes: u64,
+    pub b_reach: u64,
 }
 '''
 

@@ -75,6 +75,23 @@ pub struct StHipGemmTilePlan {
     pub duplicates: u64,
 }
 
+/// `st_hip_gemm_split_plan`.
+#[repr(C)]
+#[derive(Clone, Copy, Debug, Default, PartialEq)]
+pub struct StHipGemmSplitPlan {
+    pub served: c_int,
+    pub tile_rows: c_int,
+    pub tile_cols: c_int,
+    pub tiles_m: c_int,
+    pub tiles_n: c_int,
+    pub k_splits: c_int,
+    pub steps_per_split: c_int,
+    pub a_bytes: u64,
+    pub a_reach: u64,
+    pub b_bytes: u64,
+    pub b_reach: u64,
+}
+
 #[link(name = "sthip")]
 extern "C" {
     pub fn st_hip_init() -> c_int;
@@ -114,6 +131,7 @@ extern "C" {
     pub fn st_hip_attention_f32(contexts: usize, sequence: usize, head_dim: usize, scale: f32, causal: c_int, q: *const f32, q_len: usize, k: *const f32, k_len: usize, v: *const f32, v_len: usize, z_bias: *const f32, z_bias_len: usize, attn_bias: *const f32, attn_bias_len: usize, out: *mut f32, out_len: usize) -> c_int;
     pub fn st_hip_attention_f32_launch_plan(contexts: usize, sequence: usize, head_dim: usize, causal: c_int, biased: c_int, plan: *mut StHipAttentionPlan) -> c_int;
     pub fn st_hip_gemm_bf16_tile_plan(m: usize, n: usize, k: usize, plan: *mut StHipGemmTilePlan) -> c_int;
+    pub fn st_hip_gemm_f32_split_plan(m: usize, n: usize, k: usize, lhs_transposed: c_int, rhs_packed: c_int, plan: *mut StHipGemmSplitPlan) -> c_int;
     pub fn st_hip_gemm_row_block(k: usize, element_bytes: usize) -> usize;
     pub fn st_hip_gemm_f32_dev(m: usize, n: usize, k: usize, scale: f32, lhs_transposed: c_int, lhs: *const f32, rhs: *const f32, out: *mut f32, stream: *mut c_void) -> c_int;
     pub fn st_hip_gemm_bias_act_f32_dev(m: usize, n: usize, k: usize, activation: c_int, lhs: *const f32, rhs: *const f32, bias: *const f32, residual: *const f32, out: *mut f32, stream: *mut c_void) -> c_int;

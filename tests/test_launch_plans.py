@@ -75,3 +75,30 @@ def test_bf16_tile_grids_decode_to_every_split_and_tile_once():
     assert hip.gemm_bf16_tile_plan(4096, 4096, 4096)["k_splits"] == 1     # 256 tiles of 256×256
     with pytest.raises(hip.HipErr):
         hip.gemm_bf16_tile_plan(128, 128, 100)                            # k not a multiple of 64: another kernel family
+
+
+# Ragged sizes of every tile shape: rows and columns one short of, on and one past the tiles and the 32-row blocks, long and
+# short reductions; the last three are products whose tiles once read 27 MB, 2 MB and 126 KB past the split operands.
+SPLIT_SIZES = (33, 64, 65, 97, 129, 161, 257, 425, 770, 1000, 1024, 1121, 1399, 1601, 2049, 3841, 4097)
+SPLIT_KNOWN = [(1024, 800, 50257), (4096, 800, 4096), (65, 4097, 1001)]
+
+
+def test_split_products_stay_inside_their_operands():
+    tiles = set()
+    shapes = list(itertools.product(SPLIT_SIZES, SPLIT_SIZES, (97, 515, 769, 2100, 4099))) + SPLIT_KNOWN
+    for (m, n, k), (transposed, packed) in itertools.product(shapes, ((False, False), (True, False), (False, True))):
+        plan = hip.gemm_f32_split_plan(m, n, k, transposed, packed)
+        where = (m, n, k, transposed, packed, plan)
+        if not plan["served"]:
+            continue
+        tiles.add((plan["tile_rows"], plan["tile_cols"], plan["k_splits"] > 1))
+        steps = (k + 31) // 32 * 2
+        assert plan["a_bytes"] == (m + 31) // 32 * steps * 3072 and plan["b_bytes"] == (n + 31) // 32 * steps * 3072, where
+        assert plan["a_reach"] == plan["a_bytes"] and plan["b_reach"] == plan["b_bytes"], where
+        assert plan["a_bytes"] + plan["b_bytes"] < 1 << 31, where
+        assert plan["tiles_m"] * plan["tile_rows"] >= m and plan["tiles_n"] * plan["tile_cols"] >= n, where
+        assert plan["steps_per_split"] % 2 == 0, where
+        assert plan["k_splits"] * plan["steps_per_split"] >= steps > (plan["k_splits"] - 1) * plan["steps_per_split"], where
+    for shape in SPLIT_KNOWN:
+        assert hip.gemm_f32_split_plan(*shape)["served"], shape
+    assert {t[0] for t in tiles} == {64, 96, 128, 160, 256} and {t[2] for t in tiles} == {False, True}, tiles
