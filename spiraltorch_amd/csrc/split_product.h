@@ -169,6 +169,7 @@ __device__ __forceinline__ bool split_product_loop(unsigned char *lds_bytes, int
     for (int a = 0; a < TM; ++a)
 #pragma unroll
         for (int b = 0; b < TN; ++b) acc[a][b] += fine[a][b];
+    ST_SPLIT_WAIT_VMCNT(0);  // the loads past the last step have written their stages: the caller may use the LDS behind a barrier
     return bad;
 }
 
