@@ -16,9 +16,9 @@
 // matrix cores save.  Errors against float64 are 0.34 to 0.62 of those of the kernels that ran before (rms, six layers with
 // rectified N(0,1) images).
 //
-// Values the pieces cannot carry (non-finite, 2^127 and more, whole rows below 2^-110) are found by the pass; the rows of
-// a marked tile are looked at in the original operands, and tiles that do hold such rows are computed with f32
-// multiply-adds from them.
+// Values the pieces cannot carry (non-finite, 2^127 and more, whole rows below 2^-110) or whose sums could overflow are
+// found by the pass; tiles that see such magnitudes are computed with f32 multiply-adds from the original operands.  Where
+// only small values are marked, the tile's rows are looked at there first.
 #include <algorithm>
 
 #include "kernels.h"
@@ -30,7 +30,7 @@ namespace {
 
 typedef __attribute__((address_space(3))) void *lds_void_ptr;
 
-constexpr unsigned kWild = 1, kTiny = 2;  // status bits: a value no pieces can carry; a non-zero value below 2^-110
+constexpr unsigned kTiny = 0x80000000u;  // a status word: the largest magnitude (split_top), this bit if there is a non-zero value below 2^-110
 constexpr unsigned kOutside = 0x80000000u;
 
 struct ConvSplitArgs {
@@ -49,13 +49,10 @@ struct ConvSplitArgs {
 
 __device__ __forceinline__ unsigned split_status_of(const float (&x)[8])
 {
-    bool wild = false, tiny = false;
+    bool tiny = false;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        wild |= split_wild(x[e]);
-        tiny |= fabsf(x[e]) > 0.0f && fabsf(x[e]) < kSplitOrdinary;
-    }
-    return (__any(wild) ? kWild : 0u) | (__any(tiny) ? kTiny : 0u);
+    for (int e = 0; e < 8; ++e) tiny |= fabsf(x[e]) > 0.0f && fabsf(x[e]) < kSplitOrdinary;
+    return wave_top(split_top(x, 0u)) | (__any(tiny) ? kTiny : 0u);
 }
 
 // Images: a workgroup takes 128 padded pixels of one 16-channel block, two lanes a pixel, eight channels each: reads are
@@ -89,7 +86,9 @@ __global__ __launch_bounds__(256) void conv_split_pieces_kernel(ConvSplitArgs p)
         const unsigned flag = split_status_of(x);
         if (lane == 0) flags[wave] = flag;
         __syncthreads();
-        if (tid == 0) p.status[blockIdx.x] = flags[0] | flags[1] | flags[2] | flags[3];
+        if (tid == 0)
+            p.status[blockIdx.x] = max(max(flags[0] & ~kTiny, flags[1] & ~kTiny), max(flags[2] & ~kTiny, flags[3] & ~kTiny)) |
+                                   ((flags[0] | flags[1] | flags[2] | flags[3]) & kTiny);
         return;
     }
     const int unit = static_cast<int>(blockIdx.x - p.image_groups) * 4 + wave;  // row block · ksteps + step
@@ -122,20 +121,29 @@ __device__ __forceinline__ float conv_split_weight(const ConvSplitArgs &p, int o
     return p.weight[static_cast<size_t>(oc) * p.weight_row + static_cast<size_t>(ci) * p.weight_channel + (p.flip ? p.taps - 1 - tap : tap)];
 }
 
-// Whether pixel rows [row0, row0 + rows) or output channels [oc0, oc0 + cols) hold anything the pieces cannot carry: the
-// status words of the images and weight blocks they lie in, and only where one is marked the rows themselves.
+// Whether pixel rows [row0, row0 + rows) or output channels [oc0, oc0 + cols) hold anything the pieces cannot carry, by the
+// status words of the images and weight blocks they lie in; where those have seen small values only, by the rows themselves.
 __device__ __forceinline__ bool conv_split_bad(const ConvSplitArgs &p, int row0, int rows, int oc0, int cols, int lane)
 {
     const ConvShape &s = p.s;
     if (row0 >= p.M || oc0 >= s.c_out) return false;
     const int row_end = min(row0 + rows, p.M), oc_end = min(oc0 + cols, s.c_out);
     const unsigned per_image = static_cast<unsigned>(p.channel_blocks) * p.groups_px;
-    unsigned flag = 0;
+    unsigned top_image = 0, top_weight = 0, tiny = 0;
     const unsigned end = (static_cast<unsigned>((row_end - 1) / p.spatial) + 1) * per_image;
-    for (unsigned i = static_cast<unsigned>(row0 / p.spatial) * per_image + lane; i < end; i += 64) flag |= p.status[i];
+    for (unsigned i = static_cast<unsigned>(row0 / p.spatial) * per_image + lane; i < end; i += 64) {
+        const unsigned status = p.status[i];
+        top_image = max(top_image, status & ~kTiny);
+        tiny |= status & kTiny;
+    }
     const int unit_end = ((oc_end - 1) / 32 + 1) * p.ksteps;
-    for (int i = oc0 / 32 * p.ksteps + lane; i < unit_end; i += 64) flag |= p.status[p.weight_status + i];
-    if (!__any(flag != 0)) return false;
+    for (int i = oc0 / 32 * p.ksteps + lane; i < unit_end; i += 64) {
+        const unsigned status = p.status[p.weight_status + i];
+        top_weight = max(top_weight, status & ~kTiny);
+        tiny |= status & kTiny;
+    }
+    if (!split_in_range(wave_top(top_image), wave_top(top_weight), s.c_in * p.taps)) return true;
+    if (!__any(tiny != 0)) return false;
     bool bad = false;
     for (int r = lane; r < row_end - row0 + oc_end - oc0; r += 64) {
         const bool is_pixel = r < row_end - row0;
@@ -145,7 +153,6 @@ __device__ __forceinline__ bool conv_split_bad(const ConvSplitArgs &p, int row0,
         for (int ci = 0; ci < s.c_in; ++ci)
             for (int tap = 0; tap < p.taps; ++tap) {
                 const float v = is_pixel ? conv_split_input(p, image, px, ci, tap) : conv_split_weight(p, row, ci, tap);
-                bad |= split_wild(v);
                 nonzero |= fabsf(v) > 0.0f;
                 ordinary |= fabsf(v) >= kSplitOrdinary;
             }

@@ -15,8 +15,9 @@
 // (223 TFLOP/s), 1576×3072×768 70 -> 48, A stored k×m 3072×768×1576 100 -> 62, B prepacked 2384×1120×3708 243 -> 133,
 // and where rows are unaligned or k is no multiple of 16 853×1399×1747 114 -> 43, 182×425×2895 161 -> 20 µs.
 //
-// Values for which the three pieces are not exact (non-finite, 2^127 and more, whole operand rows below 2^-110) are found
-// by the splitting pass; the tiles they touch are computed with f32 multiply-adds from the original operands.
+// Values for which the three pieces are not exact (non-finite, 2^127 and more, whole operand rows below 2^-110) or whose sums
+// could overflow are found by the splitting pass; the tiles they touch are computed with f32 multiply-adds from the original
+// operands.
 #include <algorithm>
 #include <type_traits>
 
@@ -38,8 +39,7 @@ typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 // product kernel needs no edge cases, and any m, n, k and alignment of the operands is served alike.
 //
 // Beside every pair of blocks along k, 16 bytes of status: bit r of word 0 is set when row r holds a non-zero value
-// there, bit r of word 1 when it holds one of at least 2^-110, word 2 is non-zero when some value is 2^127 or more or not
-// finite.
+// there, bit r of word 1 when it holds one of at least 2^-110, word 2 is the largest magnitude (split_top).
 struct SplitJob {
     const float *src;
     unsigned char *blocks;
@@ -92,7 +92,7 @@ __global__ __launch_bounds__(256) void split_operands_kernel(SplitJob first, Spl
     const int rb = job.transposed ? gr * 4 + wave : gr;
     const int pair = job.transposed ? gk : gk * 4 + wave;
     if (rb * 32 >= job.rows || pair * 2 >= job.ksteps) return;
-    unsigned nonzero = 0, ordinary = 0, wild = 0;
+    unsigned nonzero = 0, ordinary = 0, top = 0;
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
         const int ks = pair * 2 + half;
@@ -113,8 +113,8 @@ __global__ __launch_bounds__(256) void split_operands_kernel(SplitJob first, Spl
             const float most = fmaxf(fabsf(x[e]), fabsf(x[e + 1]));
             nz |= most > 0.0f;
             ord |= most >= kSplitOrdinary;
-            wild |= split_wild(x[e]) | split_wild(x[e + 1]);
         }
+        top = split_top(x, top);
         const unsigned long long nz64 = __ballot(nz), ord64 = __ballot(ord);
         nonzero |= static_cast<unsigned>(nz64) | static_cast<unsigned>(nz64 >> 32);
         ordinary |= static_cast<unsigned>(ord64) | static_cast<unsigned>(ord64 >> 32);
@@ -123,8 +123,8 @@ __global__ __launch_bounds__(256) void split_operands_kernel(SplitJob first, Spl
         for (int plane = 0; plane < 3; ++plane)
             *reinterpret_cast<uint4 *>(dst + plane * 1024) = make_uint4(piece[plane][0], piece[plane][1], piece[plane][2], piece[plane][3]);
     }
-    const unsigned any_wild = __ballot(wild != 0) != 0 ? 1u : 0u;
-    if (lane == 0) job.status[static_cast<size_t>(rb) * (job.ksteps / 2) + pair] = make_uint4(nonzero, ordinary, any_wild, 0u);
+    top = wave_top(top);
+    if (lane == 0) job.status[static_cast<size_t>(rb) * (job.ksteps / 2) + pair] = make_uint4(nonzero, ordinary, top, 0u);
 }
 
 // ---- the product -------------------------------------------------------------------------------------------------
@@ -164,7 +164,7 @@ __device__ __forceinline__ bool split_status_bad(const SplitGemmArgs &p, int ra,
     for (int b = 0; b < COUNT; ++b)  // (blocks past the end repeat the last one)
         line[b] = b < TM ? p.status_a + static_cast<size_t>(min(ra + b, blocks_a - 1)) * pairs
                          : p.status_b + static_cast<size_t>(min(rb + b - TM, blocks_b - 1)) * pairs;
-    unsigned nonzero[COUNT], ordinary[COUNT], wild = 0;
+    unsigned nonzero[COUNT], ordinary[COUNT], top_a = 0, top_b = 0;
 #pragma unroll
     for (int b = 0; b < COUNT; ++b) nonzero[b] = ordinary[b] = 0;
     for (int i = pair0 + lane; i < pair1; i += 64) {
@@ -175,13 +175,14 @@ __device__ __forceinline__ bool split_status_bad(const SplitGemmArgs &p, int ra,
         for (int b = 0; b < COUNT; ++b) {
             nonzero[b] |= s[b].x;
             ordinary[b] |= s[b].y;
-            wild |= s[b].z;
+            if (b < TM) top_a = max(top_a, s[b].z);
+            else top_b = max(top_b, s[b].z);
         }
     }
     unsigned suspect = 0;
 #pragma unroll
     for (int b = 0; b < COUNT; ++b) suspect |= nonzero[b] & ~ordinary[b];
-    if (__any(wild != 0)) return true;
+    if (!split_in_range(wave_top(top_a), wave_top(top_b), p.K)) return true;
     if (!__any(suspect != 0)) return false;
     // A row may be small in one stretch and ordinary in another: only rows that are small throughout count.
     unsigned bad = 0;

@@ -11,8 +11,28 @@ namespace sthip {
 #define ST_SPLIT_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (7 << 4) | (15 << 8) | ((((n) >> 4) & 3) << 14))
 #define ST_SPLIT_FENCE() __builtin_amdgcn_sched_barrier(0)
 
-// What the three pieces cannot carry among the values seen: non-finite or 2^127 and more.
-__device__ __forceinline__ bool split_wild(float v) { return !(fabsf(v) < 0x1p127f); }  // (a NaN fails the comparison)
+// The largest magnitude among eight values and `so_far`, as f32 bits (ordered like the magnitudes, infinities and NaN above
+// everything else), and over a wavefront.
+__device__ __forceinline__ unsigned split_top(const float (&x)[8], unsigned so_far)
+{
+#pragma unroll
+    for (int e = 0; e < 8; ++e) so_far = max(so_far, __float_as_uint(x[e]) & 0x7fffffffu);
+    return so_far;
+}
+__device__ __forceinline__ unsigned wave_top(unsigned top)
+{
+#pragma unroll
+    for (int mask = 32; mask > 0; mask >>= 1) top = max(top, static_cast<unsigned>(__shfl_xor(static_cast<int>(top), mask)));
+    return top;
+}
+// Whether the piece products can stand for sums of `terms` products of values up to `top_a` and `top_b`: finite values below
+// 2^127, and no partial sum that could pass 2^127.  (Where one overflows, mid·hi overflows as well, with the sign of the mid
+// piece, and Inf - Inf comes out where f32 sums give an infinity.)
+__device__ __forceinline__ bool split_in_range(unsigned top_a, unsigned top_b, int terms)
+{
+    const int a = static_cast<int>(top_a >> 23), b = static_cast<int>(top_b >> 23);  // values below 2^(a - 126)
+    return a < 254 && b < 254 && a + b - 252 + (32 - __clz(terms)) <= 127;
+}
 // Values from here on have three exact pieces (their lowest bits stay within bf16's range).
 constexpr float kSplitOrdinary = 0x1p-110f;
 

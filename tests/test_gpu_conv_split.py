@@ -81,6 +81,23 @@ def test_grad_input_against_float64(hip, case):
     check(got[:n].reshape(batch, c_in, h, wd), want, want, c_out * kernel[0] * kernel[1])
 
 
+def test_finite_operands_whose_products_overflow(hip):
+    case = (32, 64, 28, 28, 128, (3, 3), (1, 1), (1, 1), (1, 1))
+    rng = np.random.default_rng(4)
+    x = rng.normal(size=(32, 64, 28, 28)).astype(np.float32)
+    w = np.full((128, 64, 3, 3), 1.3e25, np.float32)
+    w[::2] *= -1.0
+    x[3] = rng.uniform(1e25, 2e25, (64, 28, 28))
+    for activation in (0, 1):
+        got = forward(hip, case, x, w, None, activation)
+        assert (got[3, 1::2] == np.inf).all() and (got[3, ::2] == (0.0 if activation else -np.inf)).all()
+        others = np.arange(32) != 3
+        want = forward64(case, x[others], w)
+        want = np.maximum(want, 0.0) if activation else want
+        # f32 sums of 576 terms, their roundings in quadrature, eight standard deviations
+        assert np.abs(got[others] - want).max() <= 8 * 2.0 ** -24 * np.sqrt(576) * 24 * 1.3e25
+
+
 def test_values_the_pieces_cannot_carry(hip):
     case = (32, 64, 28, 28, 128, (3, 3), (1, 1), (1, 1), (1, 1))
     rng = np.random.default_rng(3)

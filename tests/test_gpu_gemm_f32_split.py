@@ -48,6 +48,26 @@ def test_against_float64(hip, m, n, k, layout):
     assert np.abs(got - want).max() <= 8 * bound  # eight standard deviations
 
 
+@pytest.mark.parametrize("layout", ["n", "t", "p"])
+@pytest.mark.parametrize("m,n,k", [(1233, 1000, 700), (300, 700, 2100)])
+def test_finite_operands_whose_products_overflow(hip, m, n, k, layout):
+    """Every product of 1e25 and more leaves f32: an infinity of its sign, as f32 sums give, which a fused ReLU keeps."""
+    rng = np.random.default_rng(8)
+    a, b = (rng.uniform(1e25, 2e25, shape).astype(np.float32) for shape in ((m, k), (k, n)))
+    b[:, ::3] *= -1.0
+    negative = np.broadcast_to(np.arange(n) % 3 == 0, (m, n))
+    assert (run(hip, m, n, k, layout, a, b) == np.where(negative, -np.inf, np.inf)).all()
+    if layout != "t":
+        bias = np.zeros(n, np.float32)
+        assert (run(hip, m, n, k, layout, a, b, bias, None, 1) == np.where(negative, 0.0, np.inf)).all()
+    # products that just fit, sums that do not, and sums that do
+    a[:] = np.float32(2.0 ** 64)
+    b[:] = np.float32(2.0 ** 63) * np.where(np.arange(n) % 3 == 0, -1, 1)
+    assert (run(hip, m, n, k, layout, a, b) == np.where(negative, -np.inf, np.inf)).all()
+    b *= np.float32(2.0 ** -12)
+    assert (run(hip, m, n, k, layout, a, b) == np.where(negative, -1.0, 1.0) * k * 2.0 ** 115).all()
+
+
 def test_values_the_pieces_cannot_carry(hip):
     """Infinities, NaN, values next to the largest f32 and rows small enough to lose their low pieces: the tiles they touch
     give what f32 arithmetic on the operands gives, the other tiles are not disturbed."""
