@@ -16,9 +16,8 @@
 // matrix cores save.  Errors against float64 are 0.34 to 0.62 of those of the kernels that ran before (rms, six layers with
 // rectified N(0,1) images).
 //
-// Values the pieces cannot carry (non-finite, 2^127 and more, whole rows below 2^-110) or whose sums could overflow are
-// found by the pass; tiles that see such magnitudes are computed with f32 multiply-adds from the original operands.  Where
-// only small values are marked, the tile's rows are looked at there first.
+// Values the scaled pieces cannot carry or whose sums could overflow (gemm_f32_split.hip) are found by the pass, by the image
+// and by the weight block; tiles that see such magnitudes are computed with f32 multiply-adds from the original operands.
 #include <algorithm>
 
 #include "kernels.h"
@@ -30,14 +29,13 @@ namespace {
 
 typedef __attribute__((address_space(3))) void *lds_void_ptr;
 
-constexpr unsigned kTiny = 0x80000000u;  // a status word: the largest magnitude (split_top), this bit if there is a non-zero value below 2^-110
 constexpr unsigned kOutside = 0x80000000u;
 
 struct ConvSplitArgs {
     const float *input, *weight, *bias;
     float *out;  // the result, or the planes of the partial sums
     unsigned char *pieces;  // the images' strips, then the weights' blocks at weight_base
-    unsigned *status;       // one word per workgroup of the image pass, then one per weight block and step at weight_status
+    unsigned *status;       // the largest magnitude (split_top): one word per workgroup of the image pass, then one per weight block and step at weight_status
     ConvShape s;
     int weight_row, weight_channel, flip;  // element strides of the weights; flip: taps from last to first
     int padded_w, padded_pixels, channel_blocks, taps, groups_px;
@@ -47,19 +45,11 @@ struct ConvSplitArgs {
     int activation;
 };
 
-__device__ __forceinline__ unsigned split_status_of(const float (&x)[8])
-{
-    bool tiny = false;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) tiny |= fabsf(x[e]) > 0.0f && fabsf(x[e]) < kSplitOrdinary;
-    return wave_top(split_top(x, 0u)) | (__any(tiny) ? kTiny : 0u);
-}
-
 // Images: a workgroup takes 128 padded pixels of one 16-channel block, two lanes a pixel, eight channels each: reads are
 // 128-byte runs of eight planes in flight, writes 1 KB a wavefront and piece.  Weights: a wavefront a block and step.
 __global__ __launch_bounds__(256) void conv_split_pieces_kernel(ConvSplitArgs p)
 {
-    __shared__ unsigned flags[4];
+    __shared__ unsigned tops[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const ConvShape &s = p.s;
     float x[8];
@@ -83,12 +73,10 @@ __global__ __launch_bounds__(256) void conv_split_pieces_kernel(ConvSplitArgs p)
             for (int i = 0; i < 3; ++i)
                 *reinterpret_cast<uint4 *>(dst + static_cast<size_t>(i) * p.plane_bytes) = make_uint4(piece[i][0], piece[i][1], piece[i][2], piece[i][3]);
         }
-        const unsigned flag = split_status_of(x);
-        if (lane == 0) flags[wave] = flag;
+        const unsigned top = wave_top(split_top(x, 0u));
+        if (lane == 0) tops[wave] = top;
         __syncthreads();
-        if (tid == 0)
-            p.status[blockIdx.x] = max(max(flags[0] & ~kTiny, flags[1] & ~kTiny), max(flags[2] & ~kTiny, flags[3] & ~kTiny)) |
-                                   ((flags[0] | flags[1] | flags[2] | flags[3]) & kTiny);
+        if (tid == 0) p.status[blockIdx.x] = max(max(tops[0], tops[1]), max(tops[2], tops[3]));
         return;
     }
     const int unit = static_cast<int>(blockIdx.x - p.image_groups) * 4 + wave;  // row block · ksteps + step
@@ -104,8 +92,8 @@ __global__ __launch_bounds__(256) void conv_split_pieces_kernel(ConvSplitArgs p)
     unsigned char *dst = p.pieces + p.weight_base + static_cast<size_t>(unit) * 3072 + lane * 16;
 #pragma unroll
     for (int i = 0; i < 3; ++i) *reinterpret_cast<uint4 *>(dst + i * 1024) = make_uint4(piece[i][0], piece[i][1], piece[i][2], piece[i][3]);
-    const unsigned flag = split_status_of(x);
-    if (lane == 0) p.status[p.weight_status + unit] = flag;
+    const unsigned top = wave_top(split_top(x, 0u));
+    if (lane == 0) p.status[p.weight_status + unit] = top;
 }
 
 // The value tap (ky, kx) of channel ci reads for an output pixel; zero in the padding.
@@ -121,44 +109,20 @@ __device__ __forceinline__ float conv_split_weight(const ConvSplitArgs &p, int o
     return p.weight[static_cast<size_t>(oc) * p.weight_row + static_cast<size_t>(ci) * p.weight_channel + (p.flip ? p.taps - 1 - tap : tap)];
 }
 
-// Whether pixel rows [row0, row0 + rows) or output channels [oc0, oc0 + cols) hold anything the pieces cannot carry, by the
-// status words of the images and weight blocks they lie in; where those have seen small values only, by the rows themselves.
+// Whether pixel rows [row0, row0 + rows) against output channels [oc0, oc0 + cols) hold anything the pieces cannot carry, by
+// the status words of the images and weight blocks they lie in.
 __device__ __forceinline__ bool conv_split_bad(const ConvSplitArgs &p, int row0, int rows, int oc0, int cols, int lane)
 {
     const ConvShape &s = p.s;
     if (row0 >= p.M || oc0 >= s.c_out) return false;
     const int row_end = min(row0 + rows, p.M), oc_end = min(oc0 + cols, s.c_out);
     const unsigned per_image = static_cast<unsigned>(p.channel_blocks) * p.groups_px;
-    unsigned top_image = 0, top_weight = 0, tiny = 0;
+    unsigned top_image = 0, top_weight = 0;
     const unsigned end = (static_cast<unsigned>((row_end - 1) / p.spatial) + 1) * per_image;
-    for (unsigned i = static_cast<unsigned>(row0 / p.spatial) * per_image + lane; i < end; i += 64) {
-        const unsigned status = p.status[i];
-        top_image = max(top_image, status & ~kTiny);
-        tiny |= status & kTiny;
-    }
+    for (unsigned i = static_cast<unsigned>(row0 / p.spatial) * per_image + lane; i < end; i += 64) top_image = max(top_image, p.status[i]);
     const int unit_end = ((oc_end - 1) / 32 + 1) * p.ksteps;
-    for (int i = oc0 / 32 * p.ksteps + lane; i < unit_end; i += 64) {
-        const unsigned status = p.status[p.weight_status + i];
-        top_weight = max(top_weight, status & ~kTiny);
-        tiny |= status & kTiny;
-    }
-    if (!split_in_range(wave_top(top_image), wave_top(top_weight), s.c_in * p.taps)) return true;
-    if (!__any(tiny != 0)) return false;
-    bool bad = false;
-    for (int r = lane; r < row_end - row0 + oc_end - oc0; r += 64) {
-        const bool is_pixel = r < row_end - row0;
-        const int row = is_pixel ? row0 + r : oc0 + r - (row_end - row0);
-        const int image = row / p.spatial, px = row - image * p.spatial;
-        bool nonzero = false, ordinary = false;
-        for (int ci = 0; ci < s.c_in; ++ci)
-            for (int tap = 0; tap < p.taps; ++tap) {
-                const float v = is_pixel ? conv_split_input(p, image, px, ci, tap) : conv_split_weight(p, row, ci, tap);
-                nonzero |= fabsf(v) > 0.0f;
-                ordinary |= fabsf(v) >= kSplitOrdinary;
-            }
-        bad |= nonzero && !ordinary;
-    }
-    return __any(bad);
+    for (int i = oc0 / 32 * p.ksteps + lane; i < unit_end; i += 64) top_weight = max(top_weight, p.status[p.weight_status + i]);
+    return !split_in_range(wave_top(top_image), wave_top(top_weight), s.c_in * p.taps);
 }
 
 template <int BM, int BN, int WM, int WN, int STAGES>
@@ -257,7 +221,7 @@ __device__ __forceinline__ void conv_split_body(const ConvSplitArgs &p)
                 for (int r = 0; r < 16; ++r) {
                     const int oc = col_first + tn * 32 + (r >> 2) * 8 + lh * 4 + (r & 3);
                     if (row >= p.M || oc >= s.c_out) continue;
-                    float value = acc[tm][tn][r];
+                    float value = acc[tm][tn][r] * kSplitUnscale;
                     if (bad) {
                         value = 0.0f;
                         for (int t = step0; t < min(step0 + steps, p.real_steps); ++t) {

@@ -15,9 +15,9 @@
 // (223 TFLOP/s), 1576×3072×768 70 -> 48, A stored k×m 3072×768×1576 100 -> 62, B prepacked 2384×1120×3708 243 -> 133,
 // and where rows are unaligned or k is no multiple of 16 853×1399×1747 114 -> 43, 182×425×2895 161 -> 20 µs.
 //
-// Values for which the three pieces are not exact (non-finite, 2^127 and more, whole operand rows below 2^-110) or whose sums
-// could overflow are found by the splitting pass; the tiles they touch are computed with f32 multiply-adds from the original
-// operands.
+// Both operands are scaled by a power of two first, so that the pieces are exact down to the smallest f32 value.  Values too
+// large for that or not finite, and pairs of magnitudes whose scaled sums could overflow (about 1e10 against 1e10), are
+// found by the splitting pass; the tiles they touch are computed with f32 multiply-adds from the original operands.
 #include <algorithm>
 #include <type_traits>
 
@@ -38,12 +38,11 @@ typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 // terms 8·(l / 32) .. + 7.  Block (rb, ks) starts at (rb·ksteps + ks)·3 KB; rows and terms past the end are zeros, so the
 // product kernel needs no edge cases, and any m, n, k and alignment of the operands is served alike.
 //
-// Beside every pair of blocks along k, 16 bytes of status: bit r of word 0 is set when row r holds a non-zero value
-// there, bit r of word 1 when it holds one of at least 2^-110, word 2 is the largest magnitude (split_top).
+// Beside every pair of blocks along k, a status word: the largest magnitude in it (split_top).
 struct SplitJob {
     const float *src;
     unsigned char *blocks;
-    uint4 *status;
+    unsigned *status;
     int rows, k, ld;
     int transposed;  // 0: src[row·ld + term], 1: src[term·ld + row]
     int ksteps;  // ceil(k / 16), rounded up to even
@@ -92,7 +91,7 @@ __global__ __launch_bounds__(256) void split_operands_kernel(SplitJob first, Spl
     const int rb = job.transposed ? gr * 4 + wave : gr;
     const int pair = job.transposed ? gk : gk * 4 + wave;
     if (rb * 32 >= job.rows || pair * 2 >= job.ksteps) return;
-    unsigned nonzero = 0, ordinary = 0, top = 0;
+    unsigned top = 0;
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
         const int ks = pair * 2 + half;
@@ -107,24 +106,14 @@ __global__ __launch_bounds__(256) void split_operands_kernel(SplitJob first, Spl
         }
         uint32_t piece[3][4];
         split_pieces(x, piece);
-        bool nz = false, ord = false;
-#pragma unroll
-        for (int e = 0; e < 8; e += 2) {
-            const float most = fmaxf(fabsf(x[e]), fabsf(x[e + 1]));
-            nz |= most > 0.0f;
-            ord |= most >= kSplitOrdinary;
-        }
         top = split_top(x, top);
-        const unsigned long long nz64 = __ballot(nz), ord64 = __ballot(ord);
-        nonzero |= static_cast<unsigned>(nz64) | static_cast<unsigned>(nz64 >> 32);
-        ordinary |= static_cast<unsigned>(ord64) | static_cast<unsigned>(ord64 >> 32);
         unsigned char *dst = job.blocks + (static_cast<size_t>(rb) * job.ksteps + ks) * 3072 + lane * 16;
 #pragma unroll
         for (int plane = 0; plane < 3; ++plane)
             *reinterpret_cast<uint4 *>(dst + plane * 1024) = make_uint4(piece[plane][0], piece[plane][1], piece[plane][2], piece[plane][3]);
     }
     top = wave_top(top);
-    if (lane == 0) job.status[static_cast<size_t>(rb) * (job.ksteps / 2) + pair] = make_uint4(nonzero, ordinary, top, 0u);
+    if (lane == 0) job.status[static_cast<size_t>(rb) * (job.ksteps / 2) + pair] = top;
 }
 
 // ---- the product -------------------------------------------------------------------------------------------------
@@ -141,7 +130,7 @@ __host__ __device__ inline unsigned split_block_offset(int first, int block, int
 struct SplitGemmArgs {
     const unsigned char *blocks;  // A's blocks, then B's at b_base
     unsigned b_base, bytes;
-    const uint4 *status_a, *status_b;
+    const unsigned *status_a, *status_b;
     float *C;  // the result, or plane `split` of the partial sums
     const float *bias, *residual;
     const float *A, *B;  // the original operands, for the tiles the splitting pass marked
@@ -152,51 +141,21 @@ struct SplitGemmArgs {
     int activation;
 };
 
-// Whether A's 32-row blocks [ra, ra + TM) or B's [rb, rb + TN) hold anything the three pieces cannot carry, over block
+// Whether A's 32-row blocks [ra, ra + TM) against B's [rb, rb + TN) hold anything the three pieces cannot carry, over block
 // pairs [pair0, pair1): wavefront-uniform.
 template <int TM, int TN>
 __device__ __forceinline__ bool split_status_bad(const SplitGemmArgs &p, int ra, int rb, int pair0, int pair1, int lane)
 {
-    constexpr int COUNT = TM + TN;
     const int pairs = p.ksteps / 2, blocks_a = (p.M + 31) / 32, blocks_b = (p.N + 31) / 32;
-    const uint4 *line[COUNT];
-#pragma unroll
-    for (int b = 0; b < COUNT; ++b)  // (blocks past the end repeat the last one)
-        line[b] = b < TM ? p.status_a + static_cast<size_t>(min(ra + b, blocks_a - 1)) * pairs
-                         : p.status_b + static_cast<size_t>(min(rb + b - TM, blocks_b - 1)) * pairs;
-    unsigned nonzero[COUNT], ordinary[COUNT], top_a = 0, top_b = 0;
-#pragma unroll
-    for (int b = 0; b < COUNT; ++b) nonzero[b] = ordinary[b] = 0;
+    unsigned top_a = 0, top_b = 0;
     for (int i = pair0 + lane; i < pair1; i += 64) {
-        uint4 s[COUNT];
 #pragma unroll
-        for (int b = 0; b < COUNT; ++b) s[b] = line[b][i];
+        for (int b = 0; b < TM; ++b)  // (blocks past the end repeat the last one)
+            top_a = max(top_a, p.status_a[static_cast<size_t>(min(ra + b, blocks_a - 1)) * pairs + i]);
 #pragma unroll
-        for (int b = 0; b < COUNT; ++b) {
-            nonzero[b] |= s[b].x;
-            ordinary[b] |= s[b].y;
-            if (b < TM) top_a = max(top_a, s[b].z);
-            else top_b = max(top_b, s[b].z);
-        }
+        for (int b = 0; b < TN; ++b) top_b = max(top_b, p.status_b[static_cast<size_t>(min(rb + b, blocks_b - 1)) * pairs + i]);
     }
-    unsigned suspect = 0;
-#pragma unroll
-    for (int b = 0; b < COUNT; ++b) suspect |= nonzero[b] & ~ordinary[b];
-    if (!split_in_range(wave_top(top_a), wave_top(top_b), p.K)) return true;
-    if (!__any(suspect != 0)) return false;
-    // A row may be small in one stretch and ordinary in another: only rows that are small throughout count.
-    unsigned bad = 0;
-#pragma unroll 1
-    for (int b = 0; b < COUNT; ++b) {
-        unsigned nz = 0, ord = 0;
-        for (int i = pair0; i < pair1; ++i) {
-            const uint4 s = line[b][i];
-            nz |= s.x;
-            ord |= s.y;
-        }
-        bad |= nz & ~ord;
-    }
-    return bad != 0;
+    return !split_in_range(wave_top(top_a), wave_top(top_b), p.K);
 }
 
 template <int BM, int BN, int WM, int WN, int STAGES>
@@ -279,7 +238,8 @@ __device__ __forceinline__ void gemm_f32_split_body(const SplitGemmArgs &p)
 #pragma unroll
                     for (int g = 0; g < 4; ++g)
                         *reinterpret_cast<float4 *>(&strip[li * C_STRIDE + tn * 32 + g * 8 + lh * 4]) = make_float4(
-                            acc[tm][tn][4 * g], acc[tm][tn][4 * g + 1], acc[tm][tn][4 * g + 2], acc[tm][tn][4 * g + 3]);
+                            acc[tm][tn][4 * g] * kSplitUnscale, acc[tm][tn][4 * g + 1] * kSplitUnscale,
+                            acc[tm][tn][4 * g + 2] * kSplitUnscale, acc[tm][tn][4 * g + 3] * kSplitUnscale);
             } else {
                 const int k_end = min(p.K, (step0 + steps) * 16);
                 for (int e = lane; e < 32 * WTN; e += 64) {
@@ -424,11 +384,11 @@ hipError_t launch_gemm_f32_split(size_t m, size_t n, size_t k, bool lhs_transpos
     const size_t ksteps = (k + 31) / 32 * 2, rows_a = (m + 31) / 32, rows_b = (n + 31) / 32;
     const size_t bytes_a = rows_a * ksteps * 3072, bytes_b = rows_b * ksteps * 3072;
     void *blocks = nullptr, *planes = nullptr;
-    hipError_t rc = stream_workspace_slot(stream, 1, bytes_a + bytes_b + (rows_a + rows_b) * (ksteps / 2) * sizeof(uint4), &blocks);
+    hipError_t rc = stream_workspace_slot(stream, 1, bytes_a + bytes_b + (rows_a + rows_b) * (ksteps / 2) * sizeof(unsigned), &blocks);
     if (rc == hipSuccess && plan.splits > 1) rc = stream_workspace(stream, plan.splits * m * n * sizeof(float), &planes);
     if (rc != hipSuccess) return rc;
     unsigned char *const base = static_cast<unsigned char *>(blocks);
-    uint4 *const status = reinterpret_cast<uint4 *>(base + bytes_a + bytes_b);
+    unsigned *const status = reinterpret_cast<unsigned *>(base + bytes_a + bytes_b);
 
     SplitJob job_a{lhs, base, status, static_cast<int>(m), static_cast<int>(k), static_cast<int>(lhs_transposed ? m : k),
                    lhs_transposed ? 1 : 0, static_cast<int>(ksteps), 0};

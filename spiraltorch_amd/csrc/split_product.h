@@ -25,23 +25,27 @@ __device__ __forceinline__ unsigned wave_top(unsigned top)
     for (int mask = 32; mask > 0; mask >>= 1) top = max(top, static_cast<unsigned>(__shfl_xor(static_cast<int>(top), mask)));
     return top;
 }
+
+// Operands are scaled by 2^24 before they are split, and sums by 2^-48 behind the products: the last bit any f32 value can
+// have, 2^-149, is then a normal bf16 number, and the three pieces are exact for every value, however small.
+constexpr int kSplitScaleBits = 24;
+constexpr float kSplitScale = 0x1p24f, kSplitUnscale = 0x1p-48f;
+
 // Whether the piece products can stand for sums of `terms` products of values up to `top_a` and `top_b`: finite values below
-// 2^127, and no partial sum that could pass 2^127.  (Where one overflows, mid·hi overflows as well, with the sign of the mid
-// piece, and Inf - Inf comes out where f32 sums give an infinity.)
+// 2^127 when scaled, and no partial sum that could pass 2^127.  (Where one overflows, mid·hi overflows as well, with the
+// sign of the mid piece, and Inf - Inf comes out where f32 sums give an infinity.)
 __device__ __forceinline__ bool split_in_range(unsigned top_a, unsigned top_b, int terms)
 {
     const int a = static_cast<int>(top_a >> 23), b = static_cast<int>(top_b >> 23);  // values below 2^(a - 126)
-    return a < 254 && b < 254 && a + b - 252 + (32 - __clz(terms)) <= 127;
+    return max(a, b) <= 253 - kSplitScaleBits && a + b - 252 + 2 * kSplitScaleBits + (32 - __clz(terms)) <= 127;
 }
-// Values from here on have three exact pieces (their lowest bits stay within bf16's range).
-constexpr float kSplitOrdinary = 0x1p-110f;
 
-// x = hi + mid + lo for eight values, packed in pairs: piece[0] hi, [1] mid, [2] lo.
+// 2^24·x = hi + mid + lo for eight values, packed in pairs: piece[0] hi, [1] mid, [2] lo.
 __device__ __forceinline__ void split_pieces(const float (&x)[8], uint32_t (&piece)[3][4])
 {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        const float a = x[2 * e], b = x[2 * e + 1];
+        const float a = x[2 * e] * kSplitScale, b = x[2 * e + 1] * kSplitScale;
         piece[0][e] = pack_bf16x2_rne(a, b);
         const float ra = a - __uint_as_float(piece[0][e] << 16), rb = b - __uint_as_float(piece[0][e] & 0xffff0000u);
         piece[1][e] = pack_bf16x2_rne(ra, rb);
@@ -60,7 +64,7 @@ struct SplitTile {
     static constexpr int STAGE = PIECES * 1024;
 };
 
-// acc[tm][tn] = the wavefront's sums over `steps` (even) steps.  `locate(t)` is called once for every step in order and
+// acc[tm][tn] = the wavefront's sums over `steps` (even) steps, not scaled back.  `locate(t)` is called once for every step in order and
 // says where step t's data lies; `load(stage, i, where)` requests this wavefront's i-th piece of it into a stage (past the
 // last step too: those loads read nothing that is used).  `check()` runs under the first loads; its result is returned.
 template <int BM, int BN, int WM, int WN, int STAGES, class Locate, class Load, class Check>

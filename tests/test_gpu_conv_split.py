@@ -98,6 +98,19 @@ def test_finite_operands_whose_products_overflow(hip):
         assert np.abs(got[others] - want).max() <= 8 * 2.0 ** -24 * np.sqrt(576) * 24 * 1.3e25
 
 
+def test_small_values_beside_ordinary_ones(hip):
+    case = (32, 64, 28, 28, 128, (3, 3), (1, 1), (1, 1), (1, 1))
+    rng = np.random.default_rng(5)
+    x = rng.normal(size=(32, 64, 28, 28)).astype(np.float32)
+    x[:, 5] = (rng.normal(size=(32, 28, 28)) * 1e-37).astype(np.float32)  # subnormal ones among them
+    w = np.zeros((128, 64, 3, 3), np.float32)
+    w[:, 5] = (rng.normal(size=(128, 3, 3)) * 1e20).astype(np.float32)
+    got, want = forward(hip, case, x, w, None), forward64(case, x, w)
+    magnitude = forward64(case, np.abs(x), np.abs(w))
+    # nine products: each exact to 2^-26 of itself, their sums rounded at most nine times
+    assert (np.abs(got - want) <= 10 * 2.0 ** -24 * magnitude).all()
+
+
 def test_values_the_pieces_cannot_carry(hip):
     case = (32, 64, 28, 28, 128, (3, 3), (1, 1), (1, 1), (1, 1))
     rng = np.random.default_rng(3)

@@ -68,6 +68,27 @@ def test_finite_operands_whose_products_overflow(hip, m, n, k, layout):
     assert (run(hip, m, n, k, layout, a, b) == np.where(negative, -1.0, 1.0) * k * 2.0 ** 115).all()
 
 
+@pytest.mark.parametrize("layout", ["n", "t", "p"])
+@pytest.mark.parametrize("m,n,k", [(1233, 1000, 700), (300, 700, 2100)])
+def test_small_values_beside_ordinary_ones(hip, m, n, k, layout):
+    """A value of 1e-36, or a subnormal one, keeps all its bits in a row of ordinary values: the sums below hang on it."""
+    rng = np.random.default_rng(12)
+    a, b = rng.normal(size=(m, k)).astype(np.float32), np.zeros((k, n), np.float32)
+    a[:, 5] = (rng.normal(size=m) * 1e-36).astype(np.float32)
+    a[:, k - 2] = (rng.normal(size=m) * 1e-38).astype(np.float32)  # subnormal ones among them
+    b[5, ::2] = np.float32(1e20)
+    b[k - 2, 1::2] = np.float32(-1.3e20)
+    got = run(hip, m, n, k, layout, a, b)
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    # one product each: rounded once at the end (2^-24), piece products of 2^-26 left out, five roundings of sums 2^-8 its size
+    assert (np.abs(got - want) <= 1.5 * 2.0 ** -24 * np.abs(want)).all()
+    b[7] = rng.normal(size=n)
+    a[:, 7] = (rng.normal(size=m) * 1e-16).astype(np.float32)
+    got, want = run(hip, m, n, k, layout, a, b), a.astype(np.float64) @ b.astype(np.float64)
+    magnitude = np.abs(a.astype(np.float64)) @ np.abs(b.astype(np.float64))
+    assert (np.abs(got - want) <= 4 * 2.0 ** -24 * magnitude).all()
+
+
 def test_values_the_pieces_cannot_carry(hip):
     """Infinities, NaN, values next to the largest f32 and rows small enough to lose their low pieces: the tiles they touch
     give what f32 arithmetic on the operands gives, the other tiles are not disturbed."""
