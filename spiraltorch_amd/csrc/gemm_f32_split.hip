@@ -158,6 +158,48 @@ __device__ __forceinline__ bool split_status_bad(const SplitGemmArgs &p, int ra,
     return !split_in_range(wave_top(top_a), wave_top(top_b), p.K);
 }
 
+// acc = a marked tile's sums over terms [k_begin, k_end), from the original operands on the f32 matrix cores: f32 arithmetic,
+// infinities and NaN included.  Eight terms at a time straight from memory, four in each half of the wavefront; rows past
+// the end repeat the last one.  Bound by those loads.  2048³ with one NaN in every tile row, and with NaN throughout, 380 µs (97 without; a
+// chain of multiply-adds per value took 30000), 1576×3072×768 200 (52; 7000 to 13000).
+template <int TM, int TN>
+__device__ __forceinline__ void split_f32_sums(const SplitGemmArgs &p, int row_first, int col_first, int k_begin, int k_end, int lane,
+                                               f32x16 (&acc)[TM][TN])
+{
+    const int li = lane & 31, lh = lane >> 5;
+    const float *a_row[TM], *b_row[TN];
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm) a_row[tm] = p.A + static_cast<size_t>(min(row_first + tm * 32 + li, p.M - 1)) * p.a_row;
+#pragma unroll
+    for (int tn = 0; tn < TN; ++tn) b_row[tn] = p.B + static_cast<size_t>(min(col_first + tn * 32 + li, p.N - 1)) * p.b_col;
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn)
+            acc[tm][tn] = f32x16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    auto load4 = [&](const float *row, int stride, int k, f32x4 &v) {
+        if (k + 4 <= k_end && stride == 1) {
+            v = *reinterpret_cast<const f32x4_a4 *>(row + k);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = k + e < k_end ? row[static_cast<size_t>(k + e) * stride] : 0.0f;
+        }
+    };
+    for (int k = k_begin + lh * 4; k - lh * 4 < k_end; k += 8) {
+        f32x4 a[TM], b[TN];
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm) load4(a_row[tm], p.a_k, k, a[tm]);
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn) load4(b_row[tn], p.b_k, k, b[tn]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+                for (int tn = 0; tn < TN; ++tn) acc[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x2f32(b[tn][e], a[tm][e], acc[tm][tn], 0, 0, 0);
+    }
+}
+
 template <int BM, int BN, int WM, int WN, int STAGES>
 __device__ __forceinline__ void gemm_f32_split_body(const SplitGemmArgs &p)
 {
@@ -221,6 +263,8 @@ __device__ __forceinline__ void gemm_f32_split_body(const SplitGemmArgs &p)
     float *strip = reinterpret_cast<float *>(lds_bytes) + wave * (32 * C_STRIDE);
     const int row_first = m0 + wm * WTM, col_first = n0 + wn * WTN;
     const int col0 = col_first + (lane & (LPR - 1)) * 4;
+    if (bad) split_f32_sums<TM, TN>(p, row_first, col_first, step0 * 16, min(p.K, (step0 + steps) * 16), lane, acc);
+    const float unscale = bad ? 1.0f : kSplitUnscale;
     float *const C = p.C + static_cast<size_t>(split) * p.M * p.N;
     float bias[4] = {-0.0f, -0.0f, -0.0f, -0.0f};  // x + -0.0f == x for every x
     if (p.bias) {
@@ -232,26 +276,13 @@ __device__ __forceinline__ void gemm_f32_split_body(const SplitGemmArgs &p)
 #pragma unroll
         for (int tm = 0; tm < TM; ++tm) {
             const int row_base = row_first + tm * 32;
-            if (!bad) {
 #pragma unroll
-                for (int tn = 0; tn < TN; ++tn)
+            for (int tn = 0; tn < TN; ++tn)
 #pragma unroll
-                    for (int g = 0; g < 4; ++g)
-                        *reinterpret_cast<float4 *>(&strip[li * C_STRIDE + tn * 32 + g * 8 + lh * 4]) = make_float4(
-                            acc[tm][tn][4 * g] * kSplitUnscale, acc[tm][tn][4 * g + 1] * kSplitUnscale,
-                            acc[tm][tn][4 * g + 2] * kSplitUnscale, acc[tm][tn][4 * g + 3] * kSplitUnscale);
-            } else {
-                const int k_end = min(p.K, (step0 + steps) * 16);
-                for (int e = lane; e < 32 * WTN; e += 64) {
-                    const int row = row_base + e / WTN, col = col_first + e % WTN;
-                    float sum = 0.0f;
-                    if (row < p.M && col < p.N)
-                        for (int k = step0 * 16; k < k_end; ++k)
-                            sum = fmaf(p.A[static_cast<size_t>(row) * p.a_row + static_cast<size_t>(k) * p.a_k],
-                                       p.B[static_cast<size_t>(col) * p.b_col + static_cast<size_t>(k) * p.b_k], sum);
-                    strip[e / WTN * C_STRIDE + e % WTN] = sum;
-                }
-            }
+                for (int g = 0; g < 4; ++g)
+                    *reinterpret_cast<float4 *>(&strip[li * C_STRIDE + tn * 32 + g * 8 + lh * 4]) =
+                        make_float4(acc[tm][tn][4 * g] * unscale, acc[tm][tn][4 * g + 1] * unscale,
+                                    acc[tm][tn][4 * g + 2] * unscale, acc[tm][tn][4 * g + 3] * unscale);
 #pragma unroll
             for (int j = 0; j < PASSES; ++j) {
                 const int local_row = j * ROWS_PER_PASS + lane / LPR;

@@ -1,4 +1,6 @@
 """f32 convolutions that run on the bf16 matrix cores as sums of three exact bf16 pieces, against float64."""
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -141,3 +143,22 @@ def test_values_the_pieces_cannot_carry(hip):
     # tiles beside channel 9 are now summed in f32: both sums keep to the bound above, the results' rms is 24
     untouched, keep = np.arange(32) >= 8, np.arange(128) != 9
     assert np.abs(got[untouched][:, keep] - plain[untouched][:, keep]).max() <= 8 * 2.0 ** -24 * np.sqrt(576) * 24
+
+
+def test_marked_tiles_run_on_the_matrix_cores(hip):
+    """NaN throughout takes every tile to the f32 sums: four to five times the ordinary time (a chain of multiply-adds per
+    value took 65 to 100 times)."""
+    case = (32, 256, 14, 14, 256, (3, 3), (1, 1), (1, 1), (1, 1))
+    d_w, d_out = hip.DeviceBuffer.from_array(np.ones((256, 256, 3, 3), np.float32)), hip.DeviceBuffer.from_array(np.zeros(32 * 256 * 196, np.float32))
+
+    def best(value):
+        d_x = hip.DeviceBuffer.from_array(np.full((32, 256, 14, 14), value, np.float32))
+        times = []
+        for _ in range(5):
+            start = time.perf_counter()
+            hip.conv2d_bias_act_f32_dev(*case, 0, d_x, d_w, None, d_out)
+            hip.device_synchronize()
+            times.append(time.perf_counter() - start)
+        return min(times)
+
+    assert best(np.nan) <= 15 * best(1.0)

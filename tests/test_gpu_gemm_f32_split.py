@@ -1,4 +1,6 @@
 """f32 products that run on the bf16 matrix cores as sums of three exact bf16 pieces, against float64."""
+import time
+
 import numpy as np
 import pytest
 
@@ -115,3 +117,29 @@ def test_values_the_pieces_cannot_carry(hip):
     # sequential f32 sums: k roundings at most; below 2^-126 an f32 result is a multiple of 2^-149
     assert (np.abs(got[finite] - want[finite]) <= 2.0 ** -24 * k * magnitude[finite] + 2.0 ** -149 * k).all()
     assert (got[256:640, 256:900] == clean[256:640, 256:900]).all()
+
+
+@pytest.mark.parametrize("layout", ["n", "t", "p"])
+def test_marked_tiles_run_on_the_matrix_cores(hip, layout):
+    """NaN throughout takes every tile to the f32 sums: about four times the ordinary time (a chain of multiply-adds per value
+    took 130 to 300 times)."""
+    m = n = k = 2048
+    d_b, d_c = hip.DeviceBuffer.from_array(np.ones((k, n), np.float32)), hip.DeviceBuffer.from_array(np.zeros(m * n, np.float32))
+
+    def best(value):
+        d_a = hip.DeviceBuffer.from_array(np.full((m, k), value, np.float32))
+        times = []
+        for _ in range(5):
+            start = time.perf_counter()
+            if layout == "t":
+                hip.gemm_f32_dev(m, n, k, 1.0, True, d_a, d_b, d_c)
+            elif layout == "p":
+                hip.gemm_prepacked_bias_act_f32_dev(m, n, k, 0, d_a, d_b, None, None, d_c)
+            else:
+                hip.gemm_bias_act_f32_dev(m, n, k, 0, d_a, d_b, None, None, d_c)
+            hip.device_synchronize()
+            times.append(time.perf_counter() - start)
+        return min(times)
+
+    assert hip.gemm_f32_split_plan(m, n, k, layout == "t", layout == "p")["served"]
+    assert best(np.nan) <= 15 * best(1.0)
