@@ -655,12 +655,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DPAD <= 64 
 //
 // What bounds it: a 64-key stage of 32 queries is 96 matrix instructions (2.0 µs of a SIMD at the rate random operands allow,
 // 21 ns each) beside some 450 vector ones (softmax, the pieces of the probabilities and of the staged values), two
-// wavefronts per SIMD take 5.2 µs for theirs.  Measured, f32 matrix cores -> here: 128 × 2048 × 64 causal 615 -> 382 µs,
-// non-causal 1070 -> 665, 128 × 1024 causal 163 -> 106; biased 1 × 1000 26 -> 16 µs, 16 × 1024 60 -> 51, biases on rows of
+// wavefronts per SIMD take 5.2 µs for theirs.  Measured, f32 matrix cores -> here: 128 × 2048 × 64 causal 591 -> 359 µs,
+// non-causal 1070 -> 652, 128 × 1024 causal 163 -> 112; biased 1 × 1000 26 -> 16 µs, 16 × 1024 60 -> 51, biases on rows of
 // 777 (no 16-byte alignment: the general kernel) 162 -> 16.  Errors against float64 are 0.7 to 0.85 of the f32 kernel's.
 //
-// Values the pieces cannot carry — 2^40 and more in Q or K (2^127 in V), or a column of V below 2^-110 throughout — make
-// the workgroup redo its rows with f32 multiply-adds (redo_rows below).
+// V and the probabilities are scaled by 2^24 before they are split, and the output by 2^-48: the last bit of either is then a
+// normal bf16 number, and the pieces are exact however small a value is (a probability of 2^-124 may meet the only non-zero
+// entry of a column of V).  Q and K are not: what their pieces lose is below 2^-90 of a logit's unit.  Values the pieces
+// cannot carry — 2^40 and more in Q or K, 2^70 / S and more in V, where scaled sums could overflow — make the workgroup redo
+// its rows with f32 multiply-adds (redo_rows below): 12 times the time of an ordinary call for 1 × 1000, 20 to 45 times where every
+// unit is busy.  The scaling costs 2 to 4 % of a call: 128 × 2048 × 64 causal 352 -> 359 µs, 128 × 1024 108 -> 112.
 // -------------------------------------------------------------------------------------------------
 __device__ __forceinline__ void split_pair(float a, float b, uint32_t &hi, uint32_t &mid, uint32_t &lo)
 {
@@ -670,12 +674,12 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t &hi, uint3
     lo = pack_bf16x2_rne(ra - __uint_as_float(mid << 16), rb - __uint_as_float(mid & 0xffff0000u));
 }
 
-__device__ __forceinline__ void split8(const float (&x)[8], u32x4_t (&piece)[3])
+__device__ __forceinline__ void split8(const float (&x)[8], u32x4_t (&piece)[3], float scale = 1.0f)
 {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         uint32_t hi, mid, lo;
-        split_pair(x[2 * e], x[2 * e + 1], hi, mid, lo);
+        split_pair(x[2 * e] * scale, x[2 * e + 1] * scale, hi, mid, lo);
         piece[0][e] = hi;
         piece[1][e] = mid;
         piece[2][e] = lo;
@@ -761,9 +765,8 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_split_kernel(AttnArg
     constexpr int PER = ITEMS > THREADS ? ITEMS / THREADS : 1;
     // Eight wavefronts (one workgroup per compute unit): two stages.  Four: one, so that two workgroups fit a compute unit.
     constexpr int BUFFERS = WAVES == 8 ? 2 : 1;
-    constexpr float kWild = 0x1p40f, kWildV = 0x1p127f, kTiny = 0x1p-110f;
+    constexpr float kWild = 0x1p40f, kScale = 0x1p24f, kUnscale = 0x1p-48f;
     extern __shared__ __attribute__((aligned(16))) unsigned char split_lds[];
-    __shared__ unsigned column_top[DPAD];
     __shared__ int any_wild;
 
     const int tid = threadIdx.x;
@@ -804,9 +807,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_split_kernel(AttnArg
     const int q0 = q_tile * BQ;
     const int wq0 = q0 + wave * 32;
     const int my_q = wq0 + li;
-    float top_qk = 0.0f, top_v[PER];  // largest magnitudes this thread has split
-#pragma unroll
-    for (int r = 0; r < PER; ++r) top_v[r] = 0.0f;
+    float top_qk = 0.0f, top_v = 0.0f;  // largest magnitudes this thread has split
     // Q pieces: fragment c holds Q[my_q][16c + 8·lh .. + 7]; rows past the end read as zero.  A negative scale is moved
     // into Q, as in the kernel above.
     bf16x8 qf[QSTEPS][3];
@@ -865,8 +866,8 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_split_kernel(AttnArg
             unsigned char *dst = ks + ((key >> 5) * QSTEPS + (chunk >> 1)) * 3072 + ((chunk & 1) * 32 + (key & 31)) * 16;
 #pragma unroll
             for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x4_t *>(dst + i * 1024) = piece[i];
-            split8(rv[r], piece);
-            top_v[r] = largest8(rv[r], top_v[r]);
+            split8(rv[r], piece, kScale);
+            top_v = largest8(rv[r], top_v);
             const int d = f % DPAD, group = f / DPAD;
             dst = vs + ((d >> 5) * 4 + (group >> 1)) * 3072 + ((group & 1) * 32 + (d & 31)) * 16;
 #pragma unroll
@@ -979,7 +980,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_split_kernel(AttnArg
                     tile_sum += pr[e];
                 }
                 u32x4_t piece[3];
-                split8(pr, piece);
+                split8(pr, piece, kScale);
                 bf16x8 pf[3];
 #pragma unroll
                 for (int i = 0; i < 3; ++i) pf[i] = __builtin_bit_cast(bf16x8, piece[i]);
@@ -1000,7 +1001,6 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_split_kernel(AttnArg
         run_sum += tile_sum;
     };
 
-    if (tid < DPAD) column_top[tid] = 0u;
     if (tid == 0) any_wild = 0;
     if (stages > 0) {
         load_global(key_first);
@@ -1031,18 +1031,9 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_split_kernel(AttnArg
         __syncthreads();
     }
 
-    bool wild = top_qk >= kWild;
-    if (stages_items) {
-#pragma unroll
-        for (int r = 0; r < PER; ++r) {
-            wild |= top_v[r] >= kWildV;
-            atomicMax(&column_top[(tid + THREADS * r) % DPAD], __float_as_uint(top_v[r]));
-        }
-    }
-    if (wild) any_wild = 1;
+    if (top_qk >= kWild || top_v * S >= 0x1p70f) any_wild = 1;
     __syncthreads();
-    const float column = lane < DPAD ? __uint_as_float(column_top[lane % DPAD]) : 0.0f;
-    const bool redo = any_wild != 0 || __any(column > 0.0f && column < kTiny);
+    const bool redo = any_wild != 0;
 
     const float total = run_sum + __shfl_xor(run_sum, 32);
     if constexpr (CHAINS == 2) oacc[0] += oacc[1];
@@ -1052,7 +1043,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_split_kernel(AttnArg
         const bool partial = p.key_splits > 1;
         const size_t row = (static_cast<size_t>(split) * p.contexts + ctx) * S + my_q;
         float *orow = partial ? p.part_o + row * D : p.out + ctx_elem0 + static_cast<size_t>(my_q) * D;
-        const float inv = partial ? 1.0f : total > 0.0f ? 1.0f / total : 0.0f;
+        const float inv = partial ? kUnscale : total > 0.0f ? kUnscale / total : 0.0f;
 #pragma unroll
         for (int t = 0; t < DT; ++t)
 #pragma unroll
@@ -1064,7 +1055,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_split_kernel(AttnArg
             }
         if (partial && lh == 0) *reinterpret_cast<float2 *>(p.part_ml + row * 2) = make_float2(run_max, total);
     }
-    if (pass + 1 < passes) __syncthreads();  // column_top and the stages are written again
+    if (pass + 1 < passes) __syncthreads();  // any_wild and the stages are written again
     }  // pass
 }
 

@@ -72,3 +72,26 @@ def test_values_the_pieces_cannot_carry(hip):
     assert np.abs(got[2] - want).max() <= 2.0 ** -15
     want = exact(q2[3], k2[3], v2[3], 0.125, True)
     assert np.abs(got[3] - want).max() <= 2.0 ** -15
+
+
+@pytest.mark.parametrize("contexts,seq", [(4, 300), (128, 513)])  # 128 and 256 query rows a workgroup
+@pytest.mark.parametrize("dim", [32, 64])
+def test_small_probabilities_and_values_keep_their_bits(hip, contexts, seq, dim):
+    """A key of probability 2^-124 / (seq - 1) holds the only non-zero entry of a column of V; another column is subnormal
+    beside large entries of negligible weight."""
+    rng = np.random.default_rng(13)
+    q, k, v = (np.zeros((contexts, seq, dim), np.float32) for _ in range(3))
+    q[..., 0] = 2.0
+    k[:, 7, 0] = -86.0  # logit -86, all others 0: every product and sum of them is exact
+    v[:, 7, 3] = rng.uniform(1e15, 1e17, contexts)
+    v[..., 5] = rng.uniform(1e-39, 1e-38, (contexts, seq))
+    v[:, 7, 5] = 1.0
+    v[..., 9] = rng.normal(size=(contexts, seq))
+    got = run(hip, q, k, v, 0.5, False)
+    for c in (0, contexts // 2, contexts - 1):
+        want = exact(q[c], k[c], v[c], 0.5, False)
+        # the logit in log2 units is rounded at 124 (twice) and log2(e) before it: 3 · 2^-18 · ln 2, and sums of seq terms
+        assert np.abs(got[c, :, 3] / want[:, 3] - 1.0).max() <= 1e-5
+        # an f32 result of 1e-39 is a multiple of 2^-149; weighted sums of the entries round no more than seq times 2^-24
+        assert np.abs(got[c, :, 5] - want[:, 5]).max() <= 2.0 ** -149 + seq * 2.0 ** -24 * 1e-38
+        assert np.abs(got[c, :, 9] - want[:, 9]).max() <= 2.0 ** -20
