@@ -93,7 +93,11 @@ int st_hip_stream_destroy(void *stream);
 int st_hip_device_synchronize(void);
 /* Scratch memory (split-k partial sums, re-laid weights, padded operand copies) is kept per (stream, host thread) and
  * grows on demand; a buffer whose host thread has exited is re-used by the next thread that launches on that stream,
- * and st_hip_stream_destroy frees its stream's buffers.  st_hip_release_scratch waits for `stream` (NULL = the default
+ * and st_hip_stream_destroy frees its stream's buffers.  A call recorded into a graph keeps the buffers it was handed, which
+ * later calls on the stream and thread use as well: replay the graph on that stream, or ordered with its work.  A buffer
+ * that a graph may hold is not freed when the stream's scratch grows past it, only with the stream or by
+ * st_hip_release_scratch; the graph must not be replayed after that.  What is kept is what the largest call on a stream
+ * needed, up to 2 GiB of re-laid operands for f32 products and convolutions beside the partial sums.  st_hip_release_scratch waits for `stream` (NULL = the default
  * stream, which is never destroyed) and frees every scratch buffer kept for it; no other thread may be launching on
  * that stream meanwhile.  st_hip_scratch_buffer_count reports how many buffers are held in all.  No reference
  * counterpart: the reference allocates and frees per call (crates/st-backend-hip/src/real.rs:718-756). */
@@ -162,8 +166,8 @@ int st_hip_conv2d_bias_act_f32(size_t batch, size_t c_in, size_t h, size_t w, si
  * alignment of the weight and output pointers, assumed here); st_hip_conv2d_planned_kernel reports it for the forward
  * pass (direction 0) or for grad_input of that forward shape (direction 1) as one of ST_HIP_CONV_KERNEL_*.  Large layers
  * run on the bf16 matrix cores instead, as products of three exact bf16 pieces per value, while no family is forced and
- * the stream's scratch memory can hold the pieces; the query then names the kernel that serves them where it cannot (under
- * capture before a first call, or out of memory).
+ * the stream's scratch memory can hold the pieces; the query then names the kernel that serves them where it cannot
+ * (out of memory).
  * st_hip_conv2d_force_family is a process-wide diagnostic switch (the parity tests use it to run every family on
  * small shapes): with a family forced, a convolution whose shape that family cannot serve fails with
  * ST_HIP_ERR_UNSUPPORTED instead of silently running another kernel, and the query reports 0 for it.  No reference

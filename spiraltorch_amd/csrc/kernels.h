@@ -203,7 +203,7 @@ hipError_t stream_workspace(hipStream_t stream, size_t bytes, void **out);
 // A second buffer of the same kind (slot 1) for re-laid copies of a call's operands, which must stay where they are
 // while the kernels that read them take scratch from slot 0.
 hipError_t stream_workspace_slot(hipStream_t stream, int slot, size_t bytes, void **out);
-// Whether a launcher failed only because scratch memory could not grow (out of memory, or the stream is being captured):
+// Whether a launcher failed only because scratch memory could not grow (out of memory, or an allocation refused during capture):
 // nothing has been launched then, and a route that needs no scratch may still run.
 inline bool scratch_unavailable(hipError_t rc) { return rc == hipErrorOutOfMemory || rc == hipErrorStreamCaptureUnsupported; }
 void release_stream_workspace(hipStream_t stream);

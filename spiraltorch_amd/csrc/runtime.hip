@@ -106,6 +106,9 @@ namespace {
 // orphaned, and the next thread that asks for scratch on that stream and slot adopts it: work on one stream is
 // ordered and the former owner can no longer be between receiving the pointer and launching, so a pool of short-lived
 // threads keeps re-using the same few buffers instead of leaking one per thread.
+//
+// Capture: a launch recorded into a graph keeps the buffer it was handed.  Such a buffer is never freed by growing past it
+// (the graph may be replayed later): it is kept beside the entries, and freed with them.
 struct WorkspaceEntry {
     hipStream_t stream;
     std::thread::id owner;  // std::thread::id() once the owning thread has exited
@@ -113,6 +116,11 @@ struct WorkspaceEntry {
     size_t capacity;
     int slot;
     bool growing;  // its owner is replacing the buffer outside the lock
+    bool captured;  // handed out while the stream was being captured
+};
+struct RetiredBuffer {
+    hipStream_t stream;
+    void *ptr;
 };
 // Never destroyed: threads may exit (and orphan their entries) while the process is shutting down.
 std::mutex &workspace_mutex()
@@ -124,6 +132,11 @@ std::vector<WorkspaceEntry> &workspace_entries()
 {
     static std::vector<WorkspaceEntry> *entries = new std::vector<WorkspaceEntry>;
     return *entries;
+}
+std::vector<RetiredBuffer> &retired_buffers()
+{
+    static std::vector<RetiredBuffer> *buffers = new std::vector<RetiredBuffer>;
+    return *buffers;
 }
 
 struct ThreadScratchGuard {
@@ -139,11 +152,22 @@ struct ThreadScratchGuard {
 };
 thread_local ThreadScratchGuard thread_scratch_guard;
 
-// A stream under capture can neither be waited for nor followed by an allocation.
 bool being_captured(hipStream_t stream)
 {
+    if (stream == nullptr) return false;  // the legacy stream cannot be captured
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     return hipStreamIsCapturing(stream, &status) == hipSuccess && status != hipStreamCaptureStatusNone;
+}
+
+// An allocation is no part of a graph, and allowed during a capture of any mode only where the thread says that it means it.
+hipError_t scratch_malloc(void **out, size_t bytes, bool capturing)
+{
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (capturing && hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return hipErrorStreamCaptureUnsupported;
+    const hipError_t rc = hipMalloc(out, bytes);
+    if (rc != hipSuccess) (void)hipGetLastError();  // the caller may go on without scratch
+    if (capturing) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return rc;
 }
 
 WorkspaceEntry *find_entry(hipStream_t stream, std::thread::id owner, int slot)
@@ -160,8 +184,8 @@ hipError_t stream_workspace_slot(hipStream_t stream, int slot, size_t bytes, voi
 {
     const std::thread::id me = std::this_thread::get_id();
     const size_t wanted = bytes ? bytes : 256;
+    const bool capturing = being_captured(stream);
     void *old = nullptr;
-    bool adopted_or_own = false;
     {
         std::lock_guard<std::mutex> lock(workspace_mutex());
         thread_scratch_guard.armed = true;
@@ -172,20 +196,25 @@ hipError_t stream_workspace_slot(hipStream_t stream, int slot, size_t bytes, voi
         }
         if (e) {
             if (e->ptr != nullptr && e->capacity >= wanted) {
+                e->captured |= capturing;
                 *out = e->ptr;
                 return hipSuccess;
             }
-            if (being_captured(stream)) return hipErrorStreamCaptureUnsupported;
+            // (launches recorded earlier in this capture may hold the buffer as well)
+            if (e->ptr != nullptr && (e->captured || capturing)) {
+                retired_buffers().push_back(RetiredBuffer{stream, e->ptr});
+                e->ptr = nullptr;
+            }
             // Grow: outside the lock (the wait for the stream must not stall other threads' launches).  The entry stays
             // in the table, owned by this thread and empty, so nobody else touches it meanwhile.
             old = e->ptr;
             e->ptr = nullptr;
             e->capacity = 0;
+            e->captured = false;
             e->growing = true;
-            adopted_or_own = true;
         }
     }
-    if (adopted_or_own && old) {
+    if (old) {
         // earlier launches on this stream may still be using the old buffer
         hipError_t rc = hipStreamSynchronize(stream);
         if (rc == hipSuccess) rc = hipFree(old);
@@ -195,10 +224,8 @@ hipError_t stream_workspace_slot(hipStream_t stream, int slot, size_t bytes, voi
             return rc;
         }
     }
-    if (!adopted_or_own && being_captured(stream)) return hipErrorStreamCaptureUnsupported;
     void *fresh = nullptr;
-    const hipError_t rc = hipMalloc(&fresh, wanted);
-    if (rc != hipSuccess) (void)hipGetLastError();  // the caller may go on without scratch
+    const hipError_t rc = scratch_malloc(&fresh, wanted, capturing);
     std::lock_guard<std::mutex> lock(workspace_mutex());
     WorkspaceEntry *e = find_entry(stream, me, slot);
     if (rc != hipSuccess) {
@@ -209,8 +236,9 @@ hipError_t stream_workspace_slot(hipStream_t stream, int slot, size_t bytes, voi
         e->ptr = fresh;
         e->capacity = wanted;
         e->growing = false;
+        e->captured = capturing;
     } else {
-        workspace_entries().push_back(WorkspaceEntry{stream, me, fresh, wanted, slot, false});
+        workspace_entries().push_back(WorkspaceEntry{stream, me, fresh, wanted, slot, false, capturing});
     }
     *out = fresh;
     return hipSuccess;
@@ -228,6 +256,12 @@ void release_stream_workspace(hipStream_t stream)
             if (entries[i].ptr) doomed.push_back(entries[i].ptr);
             entries.erase(entries.begin() + static_cast<long>(i));
         }
+        std::vector<RetiredBuffer> &retired = retired_buffers();
+        for (size_t i = retired.size(); i-- > 0;) {
+            if (retired[i].stream != stream) continue;
+            doomed.push_back(retired[i].ptr);
+            retired.erase(retired.begin() + static_cast<long>(i));
+        }
     }
     for (void *ptr : doomed) (void)hipFree(ptr);
 }
@@ -235,7 +269,7 @@ void release_stream_workspace(hipStream_t stream)
 size_t stream_workspace_entry_count()
 {
     std::lock_guard<std::mutex> lock(workspace_mutex());
-    return workspace_entries().size();
+    return workspace_entries().size() + retired_buffers().size();
 }
 
 }  // namespace sthip
