@@ -1306,14 +1306,20 @@ __global__ __launch_bounds__(256) void attention_merge_splits_kernel(AttnArgs p,
     *reinterpret_cast<float4 *>(p.out + row * D + d) = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
 }
 
+// The plan in which a workgroup takes all keys of its query tile (causal: of a pair of tiles).
+size_t plan_unsplit(AttnArgs &args, const bool causal)
+{
+    args.key_splits = 1;
+    args.keys_per_split = args.S;
+    args.causal_items = 0;
+    return static_cast<size_t>(args.contexts) * (causal ? (args.q_tiles + 1) / 2 : args.q_tiles);
+}
+
 // Launch plan of the fast kernel: fills the split fields of `args` and returns the number of workgroups; `causal_r` is
 // the r of the causal key split (0 when the launch is not split that way).  Pure host arithmetic.
 size_t plan_fast(AttnArgs &args, const bool causal, int *causal_r)
 {
-    size_t blocks = static_cast<size_t>(args.contexts) * (causal ? (args.q_tiles + 1) / 2 : args.q_tiles);
-    args.key_splits = 1;
-    args.keys_per_split = args.S;
-    args.causal_items = 0;
+    size_t blocks = plan_unsplit(args, causal);
     *causal_r = 0;
     constexpr size_t kTargetBlocks = 512;
     if (blocks * 2 > kTargetBlocks || args.S < 256 || args.bq != kBQ) return blocks;
@@ -1446,8 +1452,8 @@ hipError_t launch_planned(void (*kernel)(AttnArgs), unsigned threads, size_t lds
 {
     args.part_o = args.part_ml = nullptr;
     int causal_r = 0;
-    const size_t blocks = plan_fast(args, causal, &causal_r);
-    if (!fast_plan_consistent(args, causal, blocks)) return hipErrorInvalidConfiguration;
+    const AttnArgs unplanned = args;
+    size_t blocks = plan_fast(args, causal, &causal_r);
     hipError_t rc = hipSuccess;
     if (args.key_splits > 1) {
         const size_t rows = static_cast<size_t>(args.contexts) * args.S;
@@ -1455,10 +1461,17 @@ hipError_t launch_planned(void (*kernel)(AttnArgs), unsigned threads, size_t lds
         const size_t ml_bytes = static_cast<size_t>(args.key_splits) * rows * 2 * sizeof(float);
         void *workspace = nullptr;
         rc = stream_workspace(stream, o_bytes + ml_bytes, &workspace);
-        if (rc != hipSuccess) return rc;
-        args.part_o = static_cast<float *>(workspace);
-        args.part_ml = reinterpret_cast<float *>(static_cast<unsigned char *>(workspace) + o_bytes);
+        if (scratch_unavailable(rc)) {  // every workgroup takes all keys, slower and without scratch
+            args = unplanned;
+            blocks = plan_unsplit(args, causal);
+        } else if (rc != hipSuccess) {
+            return rc;
+        } else {
+            args.part_o = static_cast<float *>(workspace);
+            args.part_ml = reinterpret_cast<float *>(static_cast<unsigned char *>(workspace) + o_bytes);
+        }
     }
+    if (!fast_plan_consistent(args, causal, blocks)) return hipErrorInvalidConfiguration;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(threads), lds_bytes, stream, args);
     rc = hipGetLastError();
     if (rc != hipSuccess || args.key_splits == 1) return rc;
