@@ -1315,32 +1315,35 @@ size_t plan_unsplit(AttnArgs &args, const bool causal)
     return static_cast<size_t>(args.contexts) * (causal ? (args.q_tiles + 1) / 2 : args.q_tiles);
 }
 
-// Launch plan of the fast kernel: fills the split fields of `args` and returns the number of workgroups; `causal_r` is
-// the r of the causal key split (0 when the launch is not split that way).  Pure host arithmetic.
+// Launch plan of the fast and split kernels: fills the split fields of `args` and returns the number of workgroups; `causal_r`
+// is the r of the causal key split (0 when the launch is not split that way).  Pure host arithmetic.
 size_t plan_fast(AttnArgs &args, const bool causal, int *causal_r)
 {
     size_t blocks = plan_unsplit(args, causal);
     *causal_r = 0;
     constexpr size_t kTargetBlocks = 512;
     if (blocks * 2 > kTargetBlocks || args.S < 256 || args.bq != kBQ) return blocks;
-    // The split kernel (head sizes up to 64): a stage of 64 keys costs a workgroup about 2 µs, its start and end 3, merging
-    // 2 and a quarter per chunk, and what counts is the fullest of the 256 compute units.  3 contexts of 1180 (30 query
-    // tiles): 7 chunks of 192 keys are 210 workgroups, 14.8 µs; 10 of 128 are 300, two on some units, 17.7.
+    const size_t tiles = static_cast<size_t>(args.q_tiles), contexts = static_cast<size_t>(args.contexts);
+    // causal, chunks of 128·r keys: sum of j / r + 1 over the query tiles j
+    auto items = [&](size_t r) {
+        const size_t full = tiles / r, rest = tiles % r;
+        return r * (full * (full + 1) / 2) + rest * (full + 1);
+    };
+    // Head sizes up to 64: a stage of 64 keys costs a workgroup of the split kernel about 2 µs, its start and end 3, merging 2
+    // and a quarter per chunk, and what counts is the fullest of the 256 compute units.  3 contexts of 1180 (30 query tiles):
+    // 7 chunks of 192 keys are 210 workgroups, 14.8 µs; 10 of 128 are 300, two on some units, 17.7.  The fast kernel (large
+    // logits) takes the same plan: against chunks for two workgroups a unit, as below, 1 × 300 15.9 instead of 20.5 µs,
+    // 8 × 777 29 instead of 36, 3 × 2000 44 instead of 50; 8 × 2000 89 instead of 82.
     if (args.D <= 64) {
-        const size_t tiles = static_cast<size_t>(args.q_tiles), contexts = static_cast<size_t>(args.contexts);
         auto cost = [](size_t workgroups, double stages, size_t chunks) {
             return static_cast<double>((workgroups + 255) / 256) * (2.0 * stages + 3.0) + (chunks > 1 ? 2.0 + 0.25 * chunks : 0.0);
         };
         if (causal) {
-            auto items = [&](size_t r) {
-                size_t total = 0;
-                for (size_t j = 0; j < tiles; ++j) total += j / r + 1;
-                return total;
-            };
             double best = cost(blocks, 2.0 * (tiles + 1), 1);
             for (size_t r = 1; r < tiles; ++r) {
-                const double us = cost(contexts * items(r), 2.0 * r, (tiles - 1) / r + 1);
-                if (contexts * items(r) <= blocks || us >= best) continue;
+                const size_t workgroups = contexts * items(r);
+                const double us = cost(workgroups, 2.0 * r, (tiles - 1) / r + 1);
+                if (workgroups <= blocks || us >= best) continue;
                 best = us;
                 *causal_r = static_cast<int>(r);
             }
@@ -1370,23 +1373,17 @@ size_t plan_fast(AttnArgs &args, const bool causal, int *causal_r)
         // Few contexts: pairs of query tiles leave most of the chip idle (8 contexts of 2048: 64 workgroups, slower than
         // the non-causal call that does twice the work).  Split every tile's keys into chunks of 128·r instead, with the
         // largest r that still gives about two workgroups per compute unit; all (tile, chunk) items then cost the same.
-        const size_t tiles = static_cast<size_t>(args.q_tiles);
-        auto items = [&](size_t r) {
-            size_t total = 0;
-            for (size_t j = 0; j < tiles; ++j) total += j / r + 1;
-            return total;
-        };
         size_t r = tiles;
-        while (r > 1 && static_cast<size_t>(args.contexts) * items(r) < kTargetBlocks) --r;
+        while (r > 1 && contexts * items(r) < kTargetBlocks) --r;
         const size_t per_context = items(r);
         // (r == tiles would be one chunk per tile: nothing to merge, and the kernel tells the two forms apart by
         // key_splits > 1 — such launches keep the pairing.)
-        if (r < tiles && static_cast<size_t>(args.contexts) * per_context > blocks) {
+        if (r < tiles && contexts * per_context > blocks) {
             *causal_r = static_cast<int>(r);
             args.keys_per_split = static_cast<int>(r) * kBQ;
             args.key_splits = static_cast<int>((tiles - 1) / r + 1);
             args.causal_items = static_cast<int>(per_context);
-            blocks = static_cast<size_t>(args.contexts) * per_context;
+            blocks = contexts * per_context;
         }
     } else {
         // Few query tiles (the reference's own caller attends within one context: crates/st-nn/src/z_rba/attention.rs:586):

@@ -1,6 +1,7 @@
 """Launch arithmetic checked on the CPU: the grid a launcher asks for must be exactly what its kernel's decode of the
 workgroup index assumes.  libsthip.so computes both with the same functions the GPU path uses (no device is touched)."""
 import itertools
+import time
 
 import pytest
 
@@ -56,6 +57,16 @@ def test_the_shape_that_once_read_past_its_operands_keeps_the_pairing():
     # the reference's caller: one context with a bias matrix, keys split over workgroups
     plan = hip.attention_f32_launch_plan(1, 2048, 64, False, True)
     assert plan["kernel"] == "fast_biased" and plan["key_splits"] > 1 and plan["workgroups"] == 16 * plan["key_splits"]
+
+
+def test_long_causal_sequences_are_planned_quickly():
+    # 508 query tiles: the number of (tile, chunk) items was once counted tile by tile for every chunk size, 1 to 2 ms a call
+    times = []
+    for _ in range(20):
+        start = time.perf_counter()
+        hip.attention_f32_launch_plan(1, 65000, 64, True, False)
+        times.append(time.perf_counter() - start)
+    assert min(times) < 3e-4
 
 
 def test_bf16_tile_grids_decode_to_every_split_and_tile_once():
