@@ -1388,11 +1388,14 @@ size_t plan_fast(AttnArgs &args, const bool causal, int *causal_r)
     } else {
         // Few query tiles (the reference's own caller attends within one context: crates/st-nn/src/z_rba/attention.rs:586):
         // split the keys over workgroups until the launch offers about two workgroups per compute unit, 128 keys at least
-        // per split, and merge the partial rows in a second kernel.
+        // per split, and merge the partial rows in a second kernel.  The last split may be shorter than 128 keys where every
+        // workgroup then has a unit to itself (head size 128: 1 × 300 27 instead of 35.5 µs, 3 × 777 32 instead of 40), not
+        // where that makes a second round (3 × 1180 58 instead of 42, 8 × 777 59 instead of 54).
         const size_t want = (kTargetBlocks + blocks - 1) / blocks;
-        const size_t most = (static_cast<size_t>(args.S) + 127) / 128;
-        const size_t splits = std::min(want, most);
-        const size_t per = std::max<size_t>(128, ((static_cast<size_t>(args.S) + splits - 1) / splits + 63) / 64 * 64);
+        const size_t keys = static_cast<size_t>(args.S), chunks = std::min(want, (keys + 127) / 128);
+        const bool one_round = blocks * chunks <= 256;
+        const size_t splits = one_round ? chunks : std::min(want, keys / 128);
+        const size_t per = std::max<size_t>(128, ((keys + splits - 1) / splits + 63) / 64 * 64);
         args.keys_per_split = static_cast<int>(per);
         args.key_splits = static_cast<int>((static_cast<size_t>(args.S) + per - 1) / per);
         blocks *= static_cast<size_t>(args.key_splits);

@@ -59,6 +59,14 @@ def test_the_shape_that_once_read_past_its_operands_keeps_the_pairing():
     assert plan["kernel"] == "fast_biased" and plan["key_splits"] > 1 and plan["workgroups"] == 16 * plan["key_splits"]
 
 
+def test_key_chunks_of_large_heads():
+    # chunks of 128 keys, the last one shorter, where every workgroup has a compute unit to itself; otherwise as many keys as
+    # two workgroups a unit leave each, 128 and more
+    cut = lambda contexts, seq: [hip.attention_f32_launch_plan(contexts, seq, 128)[name] for name in ("key_splits", "keys_per_split")]
+    assert cut(1, 300) == [3, 128] and cut(3, 777) == [7, 128] and cut(8, 500) == [4, 128]
+    assert cut(3, 1180) == [7, 192] and cut(8, 777) == [5, 192] and cut(8, 2000) == [4, 512]
+
+
 def test_long_causal_sequences_are_planned_quickly():
     # 508 query tiles: the number of (tile, chunk) items was once counted tile by tile for every chunk size, 1 to 2 ms a call
     times = []
