@@ -222,9 +222,14 @@ int st_hip_attention_f32(size_t contexts, size_t sequence, size_t head_dim, floa
  * ST_HIP_ERR_RUNTIME and nothing is launched).  st_hip_attention_f32_launch_plan reports that plan for a shape and
  * additionally walks the whole grid: `items` distinct work items decoded, `items_expected` what the shape calls for,
  * `out_of_range` workgroups that would read outside the operands and `duplicates` items decoded twice (both must be
- * 0), `consistent` the launcher's own check.  No reference counterpart (the reference's CPU loop,
- * crates/st-tensor/src/pure.rs:11845-11919, has no launch geometry). */
-enum { ST_HIP_ATTN_KERNEL_GENERAL = 1, ST_HIP_ATTN_KERNEL_FAST = 2, ST_HIP_ATTN_KERNEL_FAST_BIASED = 3, ST_HIP_ATTN_KERNEL_TINY = 4 };
+ * 0), `consistent` the launcher's own check.  Operands are taken to be 16-byte aligned.  The scale decides as well: head
+ * sizes up to 64 run as products of three exact bf16 pieces per value (ST_HIP_ATTN_KERNEL_SPLIT) while
+ * |scale|·sqrt(head_dim) is at most 4, on the f32 matrix cores above.  st_hip_attention_f32_launch_plan assumes the usual
+ * 1/sqrt(head_dim) and names both FAST (FAST_BIASED); st_hip_attention_f32_scaled_launch_plan takes the scale and tells
+ * them apart.  No reference counterpart (the reference's CPU loop, crates/st-tensor/src/pure.rs:11845-11919, has no launch
+ * geometry). */
+enum { ST_HIP_ATTN_KERNEL_GENERAL = 1, ST_HIP_ATTN_KERNEL_FAST = 2, ST_HIP_ATTN_KERNEL_FAST_BIASED = 3, ST_HIP_ATTN_KERNEL_TINY = 4,
+       ST_HIP_ATTN_KERNEL_SPLIT = 5 };
 typedef struct {
     int kernel;         /* ST_HIP_ATTN_KERNEL_* */
     int key_splits;     /* most key chunks a query tile is cut into (1: keys not split over workgroups) */
@@ -234,6 +239,8 @@ typedef struct {
 } st_hip_attention_plan;
 int st_hip_attention_f32_launch_plan(size_t contexts, size_t sequence, size_t head_dim, int causal, int biased,
                                      st_hip_attention_plan *plan);
+int st_hip_attention_f32_scaled_launch_plan(size_t contexts, size_t sequence, size_t head_dim, float scale, int causal, int biased,
+                                            st_hip_attention_plan *plan);
 /* The same for the 256-row bf16 GEMM kernels, whose workgroups decode their index into (k-split, tile): the tiling and
  * k-split launch_gemm would use for an m×n×k product (k a multiple of 64), the launcher's own check (`consistent`) and a
  * walk over the whole grid (`items` must equal `workgroups`, `out_of_range` and `duplicates` must be 0). */

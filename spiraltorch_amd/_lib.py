@@ -103,6 +103,7 @@ SIGNATURES = {
     "st_hip_conv2d_force_family": (c_int, [c_int]),
     "st_hip_conv2d_planned_kernel": (c_int, [c_size_t] * 13 + [c_int, POINTER(c_int)]),
     "st_hip_attention_f32_launch_plan": (c_int, [c_size_t, c_size_t, c_size_t, c_int, c_int, POINTER(AttentionPlan)]),
+    "st_hip_attention_f32_scaled_launch_plan": (c_int, [c_size_t, c_size_t, c_size_t, c_float, c_int, c_int, POINTER(AttentionPlan)]),
     "st_hip_gemm_row_block": (c_size_t, [c_size_t, c_size_t]),
     "st_hip_gemm_f32_split_plan": (c_int, [c_size_t, c_size_t, c_size_t, c_int, c_int, POINTER(GemmSplitPlan)]),
     "st_hip_probe_mfma_bf16_dev": (c_int, [c_size_t, c_size_t, c_void_p, c_void_p, c_void_p]),

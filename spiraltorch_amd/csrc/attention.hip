@@ -1437,6 +1437,21 @@ bool fast_plan_consistent(const AttnArgs &args, const bool causal, const size_t 
 // instruction adds the products of a logit in the reference's order.
 bool sums_in_reference_order(size_t head_dim, float scale) { return !(fabsf(scale) * sqrtf(static_cast<float>(head_dim)) <= 4.0f); }
 
+// Which kernel serves a call.  `vec`: head size a multiple of 4 and 16-byte aligned operands; `bias_aligned`: 16-byte aligned
+// bias tensors.
+int attention_route(size_t contexts, size_t sequence, size_t head_dim, float scale, bool bias, bool vec, bool bias_aligned)
+{
+    // The kernels below address one context through a 32-bit buffer range.
+    if (!vec || head_dim > 128 || sequence * head_dim * sizeof(float) >= (1ull << 31)) return ST_HIP_ATTN_KERNEL_GENERAL;
+    // Many contexts of at most 64 positions: a wavefront per context.
+    if (!bias && sequence <= 64 && contexts >= 256) return ST_HIP_ATTN_KERNEL_TINY;
+    const bool bias_fits = sequence * (sequence + 256) * sizeof(float) < (1ull << 31);  // rows past the end included
+    if (head_dim <= 64 && !sums_in_reference_order(head_dim, scale) && (!bias || bias_fits)) return ST_HIP_ATTN_KERNEL_SPLIT;
+    if (!bias) return ST_HIP_ATTN_KERNEL_FAST;
+    // The biases where their rows can be read 128 bits at a time.
+    return head_dim <= 64 && sequence % 4 == 0 && bias_aligned ? ST_HIP_ATTN_KERNEL_FAST_BIASED : ST_HIP_ATTN_KERNEL_GENERAL;
+}
+
 // Query rows per workgroup: the split kernel (head sizes up to 64) takes 256 where such tiles still give every compute
 // unit one, 128 otherwise and on every other kernel.
 int query_rows(size_t contexts, size_t sequence, size_t head_dim, bool causal)
@@ -1541,7 +1556,7 @@ hipError_t launch_dpad(const AttnArgs &args, bool causal, bool bias, bool vec, h
 
 }  // namespace
 
-AttentionPlanReport attention_f32_plan_report(size_t contexts, size_t sequence, size_t head_dim, bool causal, bool biased)
+AttentionPlanReport attention_f32_plan_report(size_t contexts, size_t sequence, size_t head_dim, float scale, bool causal, bool biased)
 {
     AttentionPlanReport report{};
     if (contexts == 0 || sequence == 0 || head_dim == 0 || head_dim > static_cast<size_t>(kAttentionMaxHeadDim)) return report;
@@ -1549,30 +1564,24 @@ AttentionPlanReport attention_f32_plan_report(size_t contexts, size_t sequence, 
     args.contexts = static_cast<int>(contexts);
     args.S = static_cast<int>(sequence);
     args.D = static_cast<int>(head_dim);
-    args.bq = query_rows(contexts, sequence, head_dim, causal);
+    report.kernel = attention_route(contexts, sequence, head_dim, scale, biased, head_dim % 4 == 0, true);
+    args.bq = report.kernel == ST_HIP_ATTN_KERNEL_SPLIT ? query_rows(contexts, sequence, head_dim, causal) : kBQ;
     args.q_tiles = static_cast<int>((sequence + args.bq - 1) / args.bq);
     args.swizzle = (contexts % 8 == 0) ? 1 : 0;
     args.key_splits = 1;
     args.keys_per_split = args.S;
-    const bool vec = head_dim % 4 == 0;
-    const bool fits_buffer = sequence * head_dim * sizeof(float) < (1ull << 31);
     report.key_splits = 1;
     report.keys_per_split = args.S;
-    if (!biased && vec && fits_buffer && head_dim <= 128 && sequence <= 64 && contexts >= 256) {
-        report.kernel = ST_HIP_ATTN_KERNEL_TINY;  // a wavefront per context, four (or two) contexts a workgroup
+    if (report.kernel == ST_HIP_ATTN_KERNEL_TINY) {  // a wavefront per context, four (or two) contexts a workgroup
         report.workgroups = (contexts + 3) / 4;
         report.items = report.items_expected = contexts;
         return report;
     }
-    const bool bias_fits = sequence * (sequence + 256) * sizeof(float) < (1ull << 31);
-    const bool fast = vec && fits_buffer && (biased ? head_dim <= 64 && bias_fits : head_dim <= 128);
-    if (!fast) {
-        report.kernel = ST_HIP_ATTN_KERNEL_GENERAL;  // one workgroup per (context, query tile), decoded by division
+    if (report.kernel == ST_HIP_ATTN_KERNEL_GENERAL) {  // one workgroup per (context, query tile), decoded by division
         report.workgroups = contexts * static_cast<size_t>(args.q_tiles);
         report.items = report.items_expected = report.workgroups;
         return report;
     }
-    report.kernel = biased ? ST_HIP_ATTN_KERNEL_FAST_BIASED : ST_HIP_ATTN_KERNEL_FAST;
     int causal_r = 0;
     const size_t blocks = plan_fast(args, causal, &causal_r);
     report.workgroups = blocks;
@@ -1644,17 +1653,13 @@ hipError_t launch_attention_f32(size_t contexts, size_t sequence, size_t head_di
     const bool bias = z_bias != nullptr || attn_bias != nullptr;
     auto aligned = [](const void *ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; };
     const bool vec = (head_dim % 4 == 0) && aligned(q) && aligned(k) && aligned(v) && aligned(out);
-    // The fast kernel addresses one context through a 32-bit buffer range.
-    const bool fits_buffer = sequence * head_dim * sizeof(float) < (1ull << 31);
-    const bool bias_fits = sequence * (sequence + 256) * sizeof(float) < (1ull << 31);  // rows past the end included
-    // Many contexts of at most 64 positions: a wavefront per context.
-    if (!bias && vec && fits_buffer && head_dim <= 128 && sequence <= 64 && contexts >= 256) {
+    const int route = attention_route(contexts, sequence, head_dim, scale, bias, vec, aligned(z_bias) && aligned(attn_bias));
+    if (route == ST_HIP_ATTN_KERNEL_TINY) {
         if (head_dim <= 32) return causal ? launch_tiny<32, true>(args, stream) : launch_tiny<32, false>(args, stream);
         if (head_dim <= 64) return causal ? launch_tiny<64, true>(args, stream) : launch_tiny<64, false>(args, stream);
         return causal ? launch_tiny<128, true>(args, stream) : launch_tiny<128, false>(args, stream);
     }
-    // Head sizes up to 64 on the bf16 matrix cores.
-    if (vec && fits_buffer && head_dim <= 64 && !sums_in_reference_order(head_dim, scale) && (!bias || bias_fits)) {
+    if (route == ST_HIP_ATTN_KERNEL_SPLIT) {
         args.bq = query_rows(contexts, sequence, head_dim, causal);
         args.q_tiles = static_cast<int>((sequence + args.bq - 1) / args.bq);
         if (head_dim <= 32) {
@@ -1664,14 +1669,12 @@ hipError_t launch_attention_f32(size_t contexts, size_t sequence, size_t head_di
         if (bias) return causal ? launch_split<64, true, true>(args, stream) : launch_split<64, false, true>(args, stream);
         return causal ? launch_split<64, true, false>(args, stream) : launch_split<64, false, false>(args, stream);
     }
-    if (!bias && vec && fits_buffer && head_dim <= 128) {
+    if (route == ST_HIP_ATTN_KERNEL_FAST) {
         if (head_dim <= 32) return causal ? launch_fast<32, true>(args, stream) : launch_fast<32, false>(args, stream);
         if (head_dim <= 64) return causal ? launch_fast<64, true>(args, stream) : launch_fast<64, false>(args, stream);
         return causal ? launch_fast<128, true>(args, stream) : launch_fast<128, false>(args, stream);
     }
-    // The same with the additive biases folded in, where their rows can be read 128 bits at a time.
-    const bool bias_vec = sequence % 4 == 0 && aligned(z_bias) && aligned(attn_bias);
-    if (bias && bias_vec && vec && fits_buffer && head_dim <= 64) {
+    if (route == ST_HIP_ATTN_KERNEL_FAST_BIASED) {
         if (head_dim <= 32) return causal ? launch_fast<32, true, true>(args, stream) : launch_fast<32, false, true>(args, stream);
         return causal ? launch_fast<64, true, true>(args, stream) : launch_fast<64, false, true>(args, stream);
     }

@@ -471,8 +471,8 @@ int st_hip_conv2d_planned_kernel(size_t batch, size_t c_in, size_t h, size_t w, 
     return ST_HIP_OK;
 }
 
-int st_hip_attention_f32_launch_plan(size_t contexts, size_t sequence, size_t head_dim, int causal, int biased,
-                                     st_hip_attention_plan *plan)
+int st_hip_attention_f32_scaled_launch_plan(size_t contexts, size_t sequence, size_t head_dim, float scale, int causal, int biased,
+                                            st_hip_attention_plan *plan)
 {
     if (!plan) return fail(ST_HIP_ERR_INVALID, "attention launch_plan received a null out-pointer");
     size_t rows = 0, volume = 0;
@@ -481,17 +481,27 @@ int st_hip_attention_f32_launch_plan(size_t contexts, size_t sequence, size_t he
         return fail(ST_HIP_ERR_INVALID, "attention dimensions overflow");
     if (head_dim > static_cast<size_t>(kAttentionMaxHeadDim))
         return fail(ST_HIP_ERR_UNSUPPORTED, "attention head_dim %zu exceeds %d", head_dim, kAttentionMaxHeadDim);
-    const AttentionPlanReport report = attention_f32_plan_report(contexts, sequence, head_dim, causal != 0, biased != 0);
+    const AttentionPlanReport report = attention_f32_plan_report(contexts, sequence, head_dim, scale, causal != 0, biased != 0);
     plan->kernel = report.kernel;
     plan->key_splits = report.key_splits;
     plan->keys_per_split = report.keys_per_split;
-    plan->consistent = report.kernel == ST_HIP_ATTN_KERNEL_FAST || report.kernel == ST_HIP_ATTN_KERNEL_FAST_BIASED ? report.consistent : 1;
+    plan->consistent = report.kernel == ST_HIP_ATTN_KERNEL_GENERAL || report.kernel == ST_HIP_ATTN_KERNEL_TINY || report.kernel == 0 ? 1 : report.consistent;
     plan->workgroups = report.workgroups;
     plan->items = report.items;
     plan->items_expected = report.items_expected;
     plan->out_of_range = report.out_of_range;
     plan->duplicates = report.duplicates;
     return ST_HIP_OK;
+}
+
+int st_hip_attention_f32_launch_plan(size_t contexts, size_t sequence, size_t head_dim, int causal, int biased,
+                                     st_hip_attention_plan *plan)
+{
+    const float usual = head_dim ? 1.0f / std::sqrt(static_cast<float>(head_dim)) : 1.0f;
+    const int rc = st_hip_attention_f32_scaled_launch_plan(contexts, sequence, head_dim, usual, causal, biased, plan);
+    if (rc == ST_HIP_OK && plan->kernel == ST_HIP_ATTN_KERNEL_SPLIT)
+        plan->kernel = biased ? ST_HIP_ATTN_KERNEL_FAST_BIASED : ST_HIP_ATTN_KERNEL_FAST;
+    return rc;
 }
 
 int st_hip_probe_mfma_bf16_dev(size_t workgroups, size_t iterations, const uint16_t *operands, float *sink, void *stream)

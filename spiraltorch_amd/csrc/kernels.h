@@ -154,7 +154,7 @@ struct AttentionPlanReport {
     int kernel, key_splits, keys_per_split, consistent;
     uint64_t workgroups, items, items_expected, out_of_range, duplicates;
 };
-AttentionPlanReport attention_f32_plan_report(size_t contexts, size_t sequence, size_t head_dim, bool causal, bool biased);
+AttentionPlanReport attention_f32_plan_report(size_t contexts, size_t sequence, size_t head_dim, float scale, bool causal, bool biased);
 
 // bf16 attention over heads stored as column slices of (batch·sequence, ld) matrices; head_dim 64 or 128.
 bool attention_bf16_supported(size_t sequence, size_t head_dim, size_t ld_in, size_t ld_out, const void *q,

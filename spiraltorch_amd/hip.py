@@ -224,15 +224,19 @@ def conv2d_backward_f32(batch, c_in, h, w, c_out, kernel, stride, padding, dilat
         _ptr(gb), gb.size))
 
 
-ATTENTION_KERNELS = {1: "general", 2: "fast", 3: "fast_biased", 4: "tiny"}
+ATTENTION_KERNELS = {1: "general", 2: "fast", 3: "fast_biased", 4: "tiny", 5: "split"}
 
 
-def attention_f32_launch_plan(contexts, sequence, head_dim, causal=False, biased=False) -> dict:
+def attention_f32_launch_plan(contexts, sequence, head_dim, causal=False, biased=False, scale=None) -> dict:
     """The launch arithmetic of the f32 attention for a shape, with the whole grid decoded on the host the way the
-    kernel decodes it (no device is touched)."""
+    kernel decodes it (no device is touched).  Without a scale, for the usual 1/sqrt(head_dim), and "fast" or "fast_biased"
+    stands for "split" as well."""
     plan = _lib.AttentionPlan()
-    _check(_lib.load().st_hip_attention_f32_launch_plan(contexts, sequence, head_dim, int(bool(causal)), int(bool(biased)),
-                                                         ctypes.byref(plan)))
+    masks = (int(bool(causal)), int(bool(biased)), ctypes.byref(plan))
+    if scale is None:
+        _check(_lib.load().st_hip_attention_f32_launch_plan(contexts, sequence, head_dim, *masks))
+    else:
+        _check(_lib.load().st_hip_attention_f32_scaled_launch_plan(contexts, sequence, head_dim, scale, *masks))
     out = {name: int(getattr(plan, name)) for name, _ in _lib.AttentionPlan._fields_}
     out["kernel"] = ATTENTION_KERNELS.get(out["kernel"], "none")
     return out

@@ -130,6 +130,7 @@ extern "C" {
     pub fn st_hip_conv2d_backward_f32(batch: usize, c_in: usize, h: usize, w: usize, c_out: usize, kh: usize, kw: usize, stride_h: usize, stride_w: usize, pad_h: usize, pad_w: usize, dil_h: usize, dil_w: usize, input: *const f32, input_len: usize, weight: *const f32, weight_len: usize, grad_output: *const f32, grad_output_len: usize, grad_input: *mut f32, grad_input_len: usize, grad_weight: *mut f32, grad_weight_len: usize, grad_bias: *mut f32, grad_bias_len: usize) -> c_int;
     pub fn st_hip_attention_f32(contexts: usize, sequence: usize, head_dim: usize, scale: f32, causal: c_int, q: *const f32, q_len: usize, k: *const f32, k_len: usize, v: *const f32, v_len: usize, z_bias: *const f32, z_bias_len: usize, attn_bias: *const f32, attn_bias_len: usize, out: *mut f32, out_len: usize) -> c_int;
     pub fn st_hip_attention_f32_launch_plan(contexts: usize, sequence: usize, head_dim: usize, causal: c_int, biased: c_int, plan: *mut StHipAttentionPlan) -> c_int;
+    pub fn st_hip_attention_f32_scaled_launch_plan(contexts: usize, sequence: usize, head_dim: usize, scale: f32, causal: c_int, biased: c_int, plan: *mut StHipAttentionPlan) -> c_int;
     pub fn st_hip_gemm_bf16_tile_plan(m: usize, n: usize, k: usize, plan: *mut StHipGemmTilePlan) -> c_int;
     pub fn st_hip_gemm_f32_split_plan(m: usize, n: usize, k: usize, lhs_transposed: c_int, rhs_packed: c_int, plan: *mut StHipGemmSplitPlan) -> c_int;
     pub fn st_hip_gemm_row_block(k: usize, element_bytes: usize) -> usize;

@@ -59,6 +59,22 @@ def test_the_shape_that_once_read_past_its_operands_keeps_the_pairing():
     assert plan["kernel"] == "fast_biased" and plan["key_splits"] > 1 and plan["workgroups"] == 16 * plan["key_splits"]
 
 
+def test_the_attention_plan_knows_the_scale():
+    plan = lambda *shape, **options: hip.attention_f32_launch_plan(*shape, **options)
+    # 256-row tiles belong to the split kernel alone
+    assert plan(128, 2048, 64, True, scale=0.125)["kernel"] == "split" and plan(128, 2048, 64, True, scale=0.125)["workgroups"] == 128 * 4
+    assert plan(128, 2048, 64, True, scale=0.6)["kernel"] == "fast" and plan(128, 2048, 64, True, scale=0.6)["workgroups"] == 128 * 8
+    assert plan(128, 2048, 62, True)["kernel"] == "general" and plan(128, 2048, 62, True)["workgroups"] == 128 * 16
+    # biases: rows the f32 kernel cannot read 16 bytes at a time, larger heads
+    assert plan(2, 777, 64, False, True, scale=0.6)["kernel"] == "general" and plan(2, 776, 64, False, True, scale=0.6)["kernel"] == "fast_biased"
+    assert plan(2, 777, 64, False, True, scale=-0.5)["kernel"] == "split" and plan(2, 776, 80, False, True, scale=0.1)["kernel"] == "general"
+    assert plan(300, 64, 64, True, scale=0.6)["kernel"] == "tiny" and plan(300, 64, 64, True, scale=0.125)["kernel"] == "tiny"
+    for contexts, seq, dim, causal, biased in itertools.product(CONTEXTS, SEQUENCES, (32, 64, 128), (False, True), (False, True)):
+        got = plan(contexts, seq, dim, causal, biased, scale=0.9)
+        assert got["consistent"] == 1 and got["out_of_range"] == 0 and got["duplicates"] == 0, (contexts, seq, dim, causal, biased, got)
+        assert got["items"] == got["items_expected"], (contexts, seq, dim, causal, biased, got)
+
+
 def test_key_chunks_of_large_heads():
     # chunks of 128 keys, the last one shorter, where every workgroup has a compute unit to itself; otherwise as many keys as
     # two workgroups a unit leave each, 128 and more
