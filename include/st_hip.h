@@ -167,7 +167,7 @@ int st_hip_conv2d_bias_act_f32(size_t batch, size_t c_in, size_t h, size_t w, si
  * pass (direction 0) or for grad_input of that forward shape (direction 1) as one of ST_HIP_CONV_KERNEL_*.  Large layers
  * run on the bf16 matrix cores instead, as products of three exact bf16 pieces per value, while no family is forced and
  * the stream's scratch memory can hold the pieces; the query then names the kernel that serves them where it cannot
- * (out of memory).
+ * (out of memory); st_hip_conv2d_f32_split_plan reports them.
  * st_hip_conv2d_force_family is a process-wide diagnostic switch (the parity tests use it to run every family on
  * small shapes): with a family forced, a convolution whose shape that family cannot serve fails with
  * ST_HIP_ERR_UNSUPPORTED instead of silently running another kernel, and the query reports 0 for it.  No reference
@@ -188,6 +188,20 @@ int st_hip_conv2d_force_family(int family);
 int st_hip_conv2d_planned_kernel(size_t batch, size_t c_in, size_t h, size_t w, size_t c_out, size_t kh,
                                  size_t kw, size_t stride_h, size_t stride_w, size_t pad_h, size_t pad_w,
                                  size_t dil_h, size_t dil_w, int direction, int *kernel);
+
+/* Whether a convolution of 16-byte aligned operands runs on the bf16 matrix cores, as products of three exact bf16 pieces per
+ * value (`served`; the rest is 0 if not), forward (direction 0) or as grad_input of that forward shape (direction 1), and
+ * how it is cut: pixels and output channels per tile, workgroups along the reduction, 16-term steps each of them walks, the
+ * size of the split operands in the stream's scratch memory and how far into each the kernel's loads reach. */
+typedef struct {
+    int served;
+    int tile_pixels, tile_channels;
+    int k_splits, steps_per_split;
+    uint64_t image_bytes, image_reach, weight_bytes, weight_reach;
+} st_hip_conv2d_split_plan;
+int st_hip_conv2d_f32_split_plan(size_t batch, size_t c_in, size_t h, size_t w, size_t c_out, size_t kh, size_t kw, size_t stride_h,
+                                 size_t stride_w, size_t pad_h, size_t pad_w, size_t dil_h, size_t dil_w, int direction,
+                                 st_hip_conv2d_split_plan *split);
 
 /* Conv2d::backward, crates/st-nn/src/layers/conv.rs:780-813 with col2im :860-916: from the forward input
  * (N, C_in, H, W), the OIHW weight and grad_output (N, C_out, OH, OW) computes

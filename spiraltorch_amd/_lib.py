@@ -53,6 +53,11 @@ class GemmSplitPlan(ctypes.Structure):
         [(name, c_uint64) for name in ("a_bytes", "a_reach", "b_bytes", "b_reach")]
 
 
+class ConvSplitPlan(ctypes.Structure):
+    _fields_ = [(name, c_int) for name in ("served", "tile_pixels", "tile_channels", "k_splits", "steps_per_split")] + \
+        [(name, c_uint64) for name in ("image_bytes", "image_reach", "weight_bytes", "weight_reach")]
+
+
 class DecoderConfig(ctypes.Structure):
     _fields_ = [
         ("vocab", c_size_t),
@@ -102,6 +107,7 @@ SIGNATURES = {
     "st_hip_conv2d_output_hw": (c_int, [c_size_t] * 10 + [POINTER(c_size_t), POINTER(c_size_t)]),
     "st_hip_conv2d_force_family": (c_int, [c_int]),
     "st_hip_conv2d_planned_kernel": (c_int, [c_size_t] * 13 + [c_int, POINTER(c_int)]),
+    "st_hip_conv2d_f32_split_plan": (c_int, [c_size_t] * 13 + [c_int, POINTER(ConvSplitPlan)]),
     "st_hip_attention_f32_launch_plan": (c_int, [c_size_t, c_size_t, c_size_t, c_int, c_int, POINTER(AttentionPlan)]),
     "st_hip_attention_f32_scaled_launch_plan": (c_int, [c_size_t, c_size_t, c_size_t, c_float, c_int, c_int, POINTER(AttentionPlan)]),
     "st_hip_gemm_row_block": (c_size_t, [c_size_t, c_size_t]),

@@ -576,6 +576,13 @@ int planned_conv_grad_input_kernel(const ConvShape &shape)
     return planned_conv_kernel(t, true, true);
 }
 
+bool conv2d_split_served(const ConvShape &shape, bool grad_input, ConvShape *computed)
+{
+    *computed = shape;
+    if (grad_input && !grad_input_as_forward(shape, *computed)) return false;
+    return conv2d_f32_split_preferred(*computed, true, true, grad_input);
+}
+
 hipError_t launch_conv2d_grad_input_f32(const ConvShape &shape, const float *grad_output, const float *weight,
                                         float *grad_input, hipStream_t stream, float *weight_scratch)
 {

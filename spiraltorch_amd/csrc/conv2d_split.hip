@@ -166,6 +166,18 @@ __device__ __forceinline__ void conv_split_f32_sums(const ConvSplitArgs &p, int 
     }
 }
 
+// Where the first tap of output pixel px lies among an image's padded pixels, and how far behind it tap `tap`.
+__host__ __device__ inline int conv_split_pixel(const ConvShape &s, int padded_w, int px)
+{
+    const int oy = px / s.ow, ox = px - oy * s.ow;
+    return oy * s.stride_h * padded_w + ox * s.stride_w;
+}
+__host__ __device__ inline int conv_split_tap(const ConvShape &s, int padded_w, int tap)
+{
+    const int ky = tap / s.kw, kx = tap - ky * s.kw;
+    return ky * s.dil_h * padded_w + kx * s.dil_w;
+}
+
 template <int BM, int BN, int WM, int WN, int STAGES>
 __device__ __forceinline__ void conv_split_body(const ConvSplitArgs &p)
 {
@@ -199,9 +211,9 @@ __device__ __forceinline__ void conv_split_body(const ConvSplitArgs &p)
         const int block = q / 3, plane = q % 3;
         if (block < BM / 32) {
             const int row = m0 + block * 32 + li;
-            const int image = row / p.spatial, px = row - image * p.spatial, oy = px / s.ow, ox = px - oy * s.ow;
+            const int image = row / p.spatial, px = row - image * p.spatial;
             vector_off[i] = row < p.M ? static_cast<unsigned>(image) * p.image_bytes +
-                                            static_cast<unsigned>(lh * p.padded_pixels + oy * s.stride_h * p.padded_w + ox * s.stride_w) * 16u
+                                            static_cast<unsigned>(lh * p.padded_pixels + conv_split_pixel(s, p.padded_w, px)) * 16u
                                       : kOutside;
             scalar_off[i] = plane * p.plane_bytes;
         } else {
@@ -222,7 +234,7 @@ __device__ __forceinline__ void conv_split_body(const ConvSplitArgs &p)
         const int first = min(step0, p.real_steps - 1), channel_block = first / p.taps, tap = first - channel_block * p.taps;
         ky = tap / s.kw;
         kx = tap - ky * s.kw;
-        image_off = channel_block * p.block_bytes + static_cast<unsigned>(ky * s.dil_h * p.padded_w + kx * s.dil_w) * 16u;
+        image_off = channel_block * p.block_bytes + static_cast<unsigned>(conv_split_tap(s, p.padded_w, tap)) * 16u;
     }
     const unsigned next_row = static_cast<unsigned>(s.dil_h * p.padded_w - (s.kw - 1) * s.dil_w) * 16u;
     const unsigned next_block = p.block_bytes - static_cast<unsigned>((s.kh - 1) * s.dil_h * p.padded_w + (s.kw - 1) * s.dil_w) * 16u;
@@ -362,6 +374,25 @@ bool conv2d_f32_split_applies(const ConvShape &s, double other_us)
     if (image_bytes + weight_bytes >= static_cast<double>(1ull << 31) - 65536.0) return false;
     if (static_cast<double>(s.c_in) * s.c_out * s.kh * s.kw >= static_cast<double>(1ull << 31) || m * s.c_out >= 4e9) return false;
     return plan.us < 0.95 * other_us;  // a margin for the error of both estimates
+}
+
+ConvSplitPlanReport conv2d_f32_split_plan_report(const ConvShape &s)
+{
+    const ConvSplitPlan plan = plan_conv_split(s);
+    const int taps = s.kh * s.kw, padded_w = static_cast<int>(plan.padded_w), padded_pixels = static_cast<int>(plan.padded_h * plan.padded_w);
+    ConvSplitPlanReport report{};
+    report.tile_pixels = plan.config->bm;
+    report.tile_channels = plan.config->bn;
+    report.k_splits = plan.splits;
+    report.steps_per_split = plan.steps_per_split;
+    const uint64_t block_bytes = static_cast<uint64_t>(padded_pixels) * 96;
+    report.image_bytes = static_cast<uint64_t>(s.batch) * plan.channel_blocks * block_bytes;
+    report.weight_bytes = (static_cast<uint64_t>(s.c_out) + 31) / 32 * plan.ksteps * 3072;
+    // the last lane, piece, tap and channel block of the last pixel's loads
+    report.image_reach = (static_cast<uint64_t>(s.batch) * plan.channel_blocks - 1) * block_bytes + static_cast<uint64_t>(padded_pixels) * 64 +
+                         (static_cast<uint64_t>(padded_pixels) + conv_split_pixel(s, padded_w, s.oh * s.ow - 1) + conv_split_tap(s, padded_w, taps - 1)) * 16 + 16;
+    report.weight_reach = ((static_cast<uint64_t>(s.c_out) - 1) / 32 * plan.ksteps + plan.ksteps - 1) * 3072 + 3072;
+    return report;
 }
 
 hipError_t launch_conv2d_f32_split(const ConvShape &shape, int activation, const float *input, const float *weight, bool adjoint_weight,

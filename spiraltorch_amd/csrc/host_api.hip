@@ -471,6 +471,30 @@ int st_hip_conv2d_planned_kernel(size_t batch, size_t c_in, size_t h, size_t w, 
     return ST_HIP_OK;
 }
 
+int st_hip_conv2d_f32_split_plan(size_t batch, size_t c_in, size_t h, size_t w, size_t c_out, size_t kh, size_t kw, size_t stride_h,
+                                 size_t stride_w, size_t pad_h, size_t pad_w, size_t dil_h, size_t dil_w, int direction,
+                                 st_hip_conv2d_split_plan *split)
+{
+    if (!split) return fail(ST_HIP_ERR_INVALID, "conv2d split_plan received a null out-pointer");
+    if (direction != 0 && direction != 1) return fail(ST_HIP_ERR_INVALID, "unknown conv2d direction %d", direction);
+    *split = st_hip_conv2d_split_plan{};
+    ConvPlan plan;
+    ST_HIP_CHECK(plan_conv(batch, c_in, h, w, c_out, kh, kw, stride_h, stride_w, pad_h, pad_w, dil_h, dil_w, &plan));
+    ConvShape computed;
+    if (!conv2d_split_served(plan.shape, direction == 1, &computed)) return ST_HIP_OK;
+    const ConvSplitPlanReport report = conv2d_f32_split_plan_report(computed);
+    split->served = 1;
+    split->tile_pixels = report.tile_pixels;
+    split->tile_channels = report.tile_channels;
+    split->k_splits = report.k_splits;
+    split->steps_per_split = report.steps_per_split;
+    split->image_bytes = report.image_bytes;
+    split->image_reach = report.image_reach;
+    split->weight_bytes = report.weight_bytes;
+    split->weight_reach = report.weight_reach;
+    return ST_HIP_OK;
+}
+
 int st_hip_attention_f32_scaled_launch_plan(size_t contexts, size_t sequence, size_t head_dim, float scale, int causal, int biased,
                                             st_hip_attention_plan *plan)
 {

@@ -113,6 +113,15 @@ hipError_t launch_conv2d_f32_split(const ConvShape &shape, int activation, const
 // same bits whatever the batch).
 bool conv2d_f32_split_preferred(const ConvShape &shape, bool weight_aligned, bool out_aligned, bool keep_strip);
 
+// Whether launch_conv2d_f32 (launch_conv2d_grad_input_f32 of that forward shape) runs a layer that way, for 16-byte aligned
+// operands, and the layer it then computes; how that is cut: see st_hip_conv2d_split_plan.
+bool conv2d_split_served(const ConvShape &shape, bool grad_input, ConvShape *computed);
+struct ConvSplitPlanReport {
+    int tile_pixels, tile_channels, k_splits, steps_per_split;
+    uint64_t image_bytes, image_reach, weight_bytes, weight_reach;
+};
+ConvSplitPlanReport conv2d_f32_split_plan_report(const ConvShape &shape);
+
 // Which of its kernels launch_conv2d_f32 would run for `shape` when the split product does not serve it (one of ST_HIP_CONV_KERNEL_*; 0 when the family forced with
 // set_conv_forced_family cannot serve it), and the same for launch_conv2d_grad_input_f32 on the forward `shape`.
 int planned_conv_kernel(const ConvShape &shape, bool weight_aligned, bool out_aligned);

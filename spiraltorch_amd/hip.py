@@ -203,6 +203,15 @@ def conv2d_planned_kernel(batch, c_in, h, w, c_out, kernel, stride, padding, dil
     return CONV_KERNELS[which.value]
 
 
+def conv2d_f32_split_plan(batch, c_in, h, w, c_out, kernel, stride, padding, dilation, direction="forward") -> dict:
+    """Whether and how a convolution runs as products of three exact bf16 pieces per value ("forward" or "grad_input")."""
+    plan = _lib.ConvSplitPlan()
+    _check(_lib.load().st_hip_conv2d_f32_split_plan(
+        batch, c_in, h, w, c_out, kernel[0], kernel[1], stride[0], stride[1], padding[0], padding[1], dilation[0],
+        dilation[1], {"forward": 0, "grad_input": 1}[direction], ctypes.byref(plan)))
+    return {name: int(getattr(plan, name)) for name, _ in _lib.ConvSplitPlan._fields_}
+
+
 def conv2d_bias_activation_f32(batch, c_in, h, w, c_out, kernel, stride, padding, dilation, activation,
                                input, weight, bias, out) -> None:
     x, wgt, out = _f32(input, "input"), _f32(weight, "weight"), _out(out, "out")

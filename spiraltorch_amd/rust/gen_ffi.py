@@ -17,7 +17,8 @@ TARGET = os.path.join(HERE, "st-backend-hip", "src", "ffi.rs")
 SCALARS = {"size_t": "usize", "int": "c_int", "float": "f32", "uint64_t": "u64", "uint16_t": "u16", "char": "c_char",
            "void": "c_void", "st_hip_device_props": "StHipDeviceProps", "st_hip_probe_result": "StHipProbeResult",
            "st_hip_decoder_config": "StHipDecoderConfig", "st_hip_attention_plan": "StHipAttentionPlan",
-           "st_hip_gemm_tile_plan": "StHipGemmTilePlan", "st_hip_gemm_split_plan": "StHipGemmSplitPlan"}
+           "st_hip_gemm_tile_plan": "StHipGemmTilePlan", "st_hip_gemm_split_plan": "StHipGemmSplitPlan",
+           "st_hip_conv2d_split_plan": "StHipConv2dSplitPlan"}
 RUST_KEYWORDS = {"in": "input", "type": "kind", "ref": "reference"}
 
 STRUCTS = '''/// `st_hip_device_props`.
@@ -105,6 +106,21 @@ pub struct StHipGemmSplitPlan {
     pub a_reach: u64,
     pub b_bytes: u64,
     pub b_reach: u64,
+}
+
+/// `st_hip_conv2d_split_plan`.
+#[repr(C)]
+#[derive(Clone, Copy, Debug, Default, PartialEq)]
+pub struct StHipConv2dSplitPlan {
+    pub served: c_int,
+    pub tile_pixels: c_int,
+    pub tile_channels: c_int,
+    pub k_splits: c_int,
+    pub steps_per_split: c_int,
+    pub image_bytes: u64,
+    pub image_reach: u64,
+    pub weight_bytes: u64,
+    pub weight_reach: u64,
 }
 '''
 

@@ -162,3 +162,15 @@ def test_marked_tiles_run_on_the_matrix_cores(hip):
         return min(times)
 
     assert best(np.nan) <= 15 * best(1.0)
+
+
+def test_the_shapes_above_run_on_the_split_kernels(hip):
+    plans = [hip.conv2d_f32_split_plan(*case) for case in SHAPES]
+    assert all(plan["served"] for plan in plans)
+    assert {plan["tile_channels"] for plan in plans} == {32, 64, 128} and {plan["k_splits"] > 1 for plan in plans} == {False, True}
+    assert sum(hip.conv2d_f32_split_plan(*case, direction="grad_input")["served"] for case in SHAPES) >= 7
+    hip.conv2d_force_family("tile")
+    try:
+        assert not any(hip.conv2d_f32_split_plan(*case)["served"] for case in SHAPES)
+    finally:
+        hip.conv2d_force_family("auto")

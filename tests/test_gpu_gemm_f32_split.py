@@ -143,3 +143,10 @@ def test_marked_tiles_run_on_the_matrix_cores(hip, layout):
 
     assert hip.gemm_f32_split_plan(m, n, k, layout == "t", layout == "p")["served"]
     assert best(np.nan) <= 15 * best(1.0)
+
+
+def test_the_shapes_above_run_on_the_split_kernels(hip):
+    layouts = {"n": (False, False), "t": (True, False), "p": (False, True)}
+    plans = [hip.gemm_f32_split_plan(m, n, k, *layouts[layout]) for m, n, k in SHAPES for layout in layouts]
+    assert all(plan["served"] for plan in plans)
+    assert {plan["k_splits"] > 1 for plan in plans} == {False, True}

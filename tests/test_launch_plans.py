@@ -137,3 +137,34 @@ def test_split_products_stay_inside_their_operands():
     for shape in SPLIT_KNOWN:
         assert hip.gemm_f32_split_plan(*shape)["served"], shape
     assert {t[0] for t in tiles} == {64, 96, 128, 160, 256} and {t[2] for t in tiles} == {False, True}, tiles
+
+
+def test_split_convolutions_stay_inside_their_operands():
+    served = 0
+    geometries = [((1, 1), (1, 1), (0, 0), (1, 1)), ((3, 3), (1, 1), (1, 1), (1, 1)), ((3, 3), (2, 2), (1, 1), (1, 1)), ((5, 3), (2, 1), (2, 0), (1, 1)),
+                  ((3, 3), (1, 1), (2, 2), (2, 2)), ((3, 3), (1, 1), (4, 3), (1, 1)), ((7, 7), (1, 1), (3, 3), (1, 1))]
+    for batch, c_in, side, c_out in itertools.product((1, 2, 31, 32), (16, 33, 64, 250, 512), (7, 14, 29, 56), (31, 64, 129, 512)):
+        for kernel, stride, padding, dilation in geometries:
+            for direction in ("forward", "grad_input"):
+                if side + 2 * padding[0] < (kernel[0] - 1) * dilation[0] + 1:
+                    continue
+                shape = (batch, c_in, side, side + 1, c_out, kernel, stride, padding, dilation)
+                plan = hip.conv2d_f32_split_plan(*shape, direction=direction)
+                where = (shape, direction, plan)
+                if not plan["served"]:
+                    continue
+                served += 1
+                channels, rows = (c_in, c_out) if direction == "forward" else (c_out, c_in)
+                steps = ((channels + 15) // 16 * kernel[0] * kernel[1] + 1) // 2 * 2
+                assert plan["weight_bytes"] == (rows + 31) // 32 * steps * 3072, where
+                assert plan["image_reach"] <= plan["image_bytes"] and plan["weight_reach"] == plan["weight_bytes"], where
+                assert plan["image_bytes"] + plan["weight_bytes"] < 1 << 31, where
+                assert plan["steps_per_split"] % 2 == 0, where
+                assert plan["k_splits"] * plan["steps_per_split"] >= steps > (plan["k_splits"] - 1) * plan["steps_per_split"], where
+    assert served > 100
+    # a strip kernel's grad_input for an image is the same bits whatever the batch: such layers stay on it
+    layer = (32, 64, 56, 56, 128, (3, 3), (1, 1), (1, 1), (1, 1))
+    assert hip.conv2d_f32_split_plan(*layer)["served"] == 1
+    assert hip.conv2d_planned_kernel(*layer, direction="grad_input") == "strip9"
+    assert hip.conv2d_f32_split_plan(*layer, direction="grad_input")["served"] == 0
+    assert hip.conv2d_f32_split_plan(2, 8, 9, 9, 4, (3, 3), (1, 1), (1, 1), (1, 1))["served"] == 0
