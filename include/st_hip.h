@@ -168,6 +168,10 @@ int st_hip_conv2d_bias_act_f32(size_t batch, size_t c_in, size_t h, size_t w, si
  * run on the bf16 matrix cores instead, as products of three exact bf16 pieces per value, while no family is forced and
  * the stream's scratch memory can hold the pieces; the query then names the kernel that serves them where it cannot
  * (out of memory); st_hip_conv2d_f32_split_plan reports them.
+ * The bits of an image's result may depend on the batch around it, forward and grad_input alike: the kernel and the cut of
+ * the reduction are chosen from the whole call, and every choice keeps to the f32 tolerance.  The one exception is grad_input
+ * where this query says STRIP12, STRIP12_WIDE or STRIP9 (such layers never run as bf16 pieces): the same bits for an image
+ * in every batch that gets that answer.
  * st_hip_conv2d_force_family is a process-wide diagnostic switch (the parity tests use it to run every family on
  * small shapes): with a family forced, a convolution whose shape that family cannot serve fails with
  * ST_HIP_ERR_UNSUPPORTED instead of silently running another kernel, and the query reports 0 for it.  No reference
