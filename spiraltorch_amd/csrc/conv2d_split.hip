@@ -35,7 +35,7 @@ struct ConvSplitArgs {
     const float *input, *weight, *bias;
     float *out;  // the result, or the planes of the partial sums
     unsigned char *pieces;  // the images' strips, then the weights' blocks at weight_base
-    unsigned *status;       // the largest magnitude (split_top): one word per workgroup of the image pass, then one per weight block and step at weight_status
+    unsigned *status;  // the largest magnitude (split_top): a word per workgroup of the image pass, then per weight block and step
     ConvShape s;
     int weight_row, weight_channel, flip;  // element strides of the weights; flip: taps from last to first
     int padded_w, padded_pixels, channel_blocks, taps, groups_px;

@@ -962,10 +962,11 @@ namespace {
 hipError_t launch_gemm_f32_native(size_t m, size_t n, size_t k, bool lhs_transposed, const float *lhs, const float *rhs, float *out,
                                   const GemmEpilogue &epilogue, hipStream_t stream, bool scratch_free)
 {
-    // A k that is not a multiple of 4 in a product too large for the split kernels: the rows of A start at odd addresses, which the direct-to-LDS kernels do not take, and the general kernel runs at about 0.6 of their
-    // speed (1024×1024×4099: 140 µs against 80 µs at 4096).  Where the product is large against its operands, copies
-    // of A and B zero-padded along k to a multiple of 16 (exact: the new terms are 0·0) go into the stream's second
-    // scratch buffer, one launch for both, and the product runs on them.
+    // A k that is not a multiple of 4 in a product too large for the split kernels: the rows of A start at odd addresses, which
+    // the direct-to-LDS kernels do not take, and the general kernel runs at about 0.6 of their speed (1024×1024×4099: 140 µs
+    // against 80 µs at 4096).  Where the product is large against its operands, copies of A and B zero-padded along k to a
+    // multiple of 16 (exact: the new terms are 0·0) go into the stream's second scratch buffer, one launch for both, and the
+    // product runs on them.
     // (Only where the copies then take the fast kernels: B's rows, and A's when it is stored k×m, must be 16-byte aligned.)
     if (k % 4 != 0 && k > 64 && m >= 128 && n >= 128 && n % 4 == 0 && (!lhs_transposed || m % 4 == 0) && scratch_free &&
         2.0 * m * n * k >= 2e9 &&

@@ -122,8 +122,9 @@ struct ConvSplitPlanReport {
 };
 ConvSplitPlanReport conv2d_f32_split_plan_report(const ConvShape &shape);
 
-// Which of its kernels launch_conv2d_f32 would run for `shape` when the split product does not serve it (one of ST_HIP_CONV_KERNEL_*; 0 when the family forced with
-// set_conv_forced_family cannot serve it), and the same for launch_conv2d_grad_input_f32 on the forward `shape`.
+// Which of its kernels launch_conv2d_f32 would run for `shape` when the split product does not serve it (one of
+// ST_HIP_CONV_KERNEL_*; 0 when the family forced with set_conv_forced_family cannot serve it), and the same for
+// launch_conv2d_grad_input_f32 on the forward `shape`.
 int planned_conv_kernel(const ConvShape &shape, bool weight_aligned, bool out_aligned);
 int planned_conv_grad_input_kernel(const ConvShape &shape);
 void set_conv_forced_family(int family);

@@ -717,7 +717,9 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 // (128 registers a wavefront, four wavefronts per SIMD); with 1024 threads and the row padded to 65536 values one row
 // filled the unit.  The index a row without a usable sum needs is found by reading the row again: no row of ordinary
 // values pays for it.
-// 1024 × 50257 115 -> 102 µs, × 40000 78 -> 63, × 32000 53 -> 39 (6.7 TB/s), 2048 × 5001 20.5 -> 14.3, 4 × 50257 14 -> 9.7.
+// 1024 × 50257 114 -> 104 µs, × 40000 80 -> 67, × 32000 61 -> 52 (5 TB/s), 2048 × 5001 23 -> 19, 4 × 50257 14 -> 9.7 on tensors
+// that come from memory (53 -> 39 and 20.5 -> 14.1 for × 32000 and × 5001 where they stay in the memory-side cache); 2048 × 50257
+// 204 either way.  Rows that start on 16 bytes take the same time: 1024 × 50304 112 -> 100.
 template <int CH, int THREADS>
 __device__ __forceinline__ void row_softmax_block_body(int cols, const float *in, float *out)
 {

@@ -64,9 +64,10 @@ struct SplitTile {
     static constexpr int STAGE = PIECES * 1024;
 };
 
-// acc[tm][tn] = the wavefront's sums over `steps` (even) steps, not scaled back.  `locate(t)` is called once for every step in order and
-// says where step t's data lies; `load(stage, i, where)` requests this wavefront's i-th piece of it into a stage (past the
-// last step too: those loads read nothing that is used).  `check()` runs under the first loads; its result is returned.
+// acc[tm][tn] = the wavefront's sums over `steps` (even) steps, not scaled back.  `locate(t)` is called once for every step in
+// order and says where step t's data lies; `load(stage, i, where)` requests this wavefront's i-th piece of it into a stage
+// (past the last step too: those loads read nothing that is used).  `check()` runs under the first loads; its result is
+// returned.
 template <int BM, int BN, int WM, int WN, int STAGES, class Locate, class Load, class Check>
 __device__ __forceinline__ bool split_product_loop(unsigned char *lds_bytes, int wave, int lane, int steps,
                                                    f32x16 (&acc)[BM / WM / 32][BN / WN / 32], Locate &&locate, Load &&load,
