@@ -643,7 +643,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DPAD <= 64 
 // Head sizes up to 64, with or without biases: both products on the bf16 matrix cores, every f32 value (Q, K, V and the
 // probabilities) as the exact sum of three bf16 values, x = hi + mid + lo, and a product as the six piece products
 //     lo·hi, mid·hi, mid·mid, hi·mid, hi·lo, hi·hi
-// accumulated in f32; what is left out is below 2^-26 of the product.  (gemm_f32_split.hip does the same for matrix
+// accumulated in f32; what is left out is at most 2^-24 of the product, 2^-27.4 in the rms.  (gemm_f32_split.hip does the same for matrix
 // products, with its error measurements.)  Six bf16 instructions replace eight f32 ones of twice their duration.
 //
 // Same transposed formulation, masks and running maximum as the kernel above.  A stage of 64 keys is split into its pieces

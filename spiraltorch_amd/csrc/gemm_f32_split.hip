@@ -2,7 +2,8 @@
 // x = hi + mid + lo (hi = bf16(x), mid = bf16(x - hi), lo = x - hi - mid, each difference exact: 3 × 8 mantissa bits hold
 // all 24 of an f32), and a product a·b is accumulated in f32 from six of the nine piece products,
 //     lo·hi, mid·hi, mid·mid, hi·mid, hi·lo, hi·hi.
-// What is left out (mid·lo, lo·mid, lo·lo) is below 2^-26 of |a·b|, a quarter of what rounding one f32 product costs.
+// What is left out (mid·lo, lo·mid, lo·lo) is at most 2^-24 of |a·b|, as much as rounding one f32 product can cost, and 2^-27.4 in
+// the rms over N(0,1) operands (|mid| <= 2^-8 |x|, |lo| <= 2^-17 |x|).
 // v_mfma_f32_32x32x16_bf16 multiplies exactly and adds into f32 accumulators, and the result carries one rounding of the
 // large sum per sixteen terms where the f32 instruction rounds after every term, so it is closer to the exact sum than the
 // f32 matrix cores' (rms error against float64, N(0,1) operands, of the result's rms: k = 768 1.6e-7 against 5.0e-7,

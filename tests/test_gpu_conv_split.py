@@ -109,7 +109,7 @@ def test_small_values_beside_ordinary_ones(hip):
     w[:, 5] = (rng.normal(size=(128, 3, 3)) * 1e20).astype(np.float32)
     got, want = forward(hip, case, x, w, None), forward64(case, x, w)
     magnitude = forward64(case, np.abs(x), np.abs(w))
-    # nine products: each exact to 2^-26 of itself, their sums rounded at most nine times
+    # nine products, of each at most 2^-24 left out, their sums rounded at most nine times
     assert (np.abs(got - want) <= 10 * 2.0 ** -24 * magnitude).all()
 
 

@@ -82,8 +82,8 @@ def test_small_values_beside_ordinary_ones(hip, m, n, k, layout):
     b[k - 2, 1::2] = np.float32(-1.3e20)
     got = run(hip, m, n, k, layout, a, b)
     want = a.astype(np.float64) @ b.astype(np.float64)
-    # one product each: rounded once at the end (2^-24), piece products of 2^-26 left out, five roundings of sums 2^-8 its size
-    assert (np.abs(got - want) <= 1.5 * 2.0 ** -24 * np.abs(want)).all()
+    # one product each: rounded once at the end (2^-24), piece products of 2^-24 left out, five roundings of sums 2^-8 its size
+    assert (np.abs(got - want) <= 2.02 * 2.0 ** -24 * np.abs(want)).all()
     b[7] = rng.normal(size=n)
     a[:, 7] = (rng.normal(size=m) * 1e-16).astype(np.float32)
     got, want = run(hip, m, n, k, layout, a, b), a.astype(np.float64) @ b.astype(np.float64)
