@@ -37,7 +37,9 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 # Published MI355X peaks the roofline fractions are priced against.
-PEAK_TFLOPS = {"f32": 157.3, "bf16": 2500.0}
+# f32 work that runs as six bf16 products of exact pieces per product (the library's plan queries say which) is priced
+# against a sixth of the bf16 peak, the most that route can reach.
+PEAK_TFLOPS = {"f32": 157.3, "bf16": 2500.0, "f32_pieces": 2500.0 / 6}
 PEAK_HBM_GBS = 8000.0
 
 # HBM bytes per launch measured with rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE (KiB per dispatch; FETCH_SIZE
@@ -52,12 +54,7 @@ MEASURED_TRAFFIC_BYTES = {
     "gemm_bf16_f32acc_4096x4096x4096_prepacked_rhs": (98406 * 2 + 65536) * 1024,
     "gemm_bf16_f32acc_16x4096x4096": ((16927 + 1045) * 2 + 2048 + 256) * 1024,
     "gemm_bf16_f32acc_16x4096x4096_prepacked_rhs": (16924 * 2 + 256) * 1024,
-    "attention_f32_b8_h16_s2048_d64_noncausal": (98379 * 2 + 65536) * 1024,
-    "attention_f32_b8_h16_s2048_d64_causal": (134572 * 2 + 65547) * 1024,
-    "attention_f32_attn_bias_c1_s2048_d64": ((10840 + 4260) * 2 + 8448 + 512) * 1024,
-    "attention_f32_attn_bias_c16_s1024_d64": ((49240 + 8484) * 2 + 16896 + 4096) * 1024,
     "gemm_f32_100352x128x576_conv_equivalent": (136982 * 2 + 50176) * 1024,
-    "gemm_f32_4096x4096x4096": (196708 * 2 + 65536) * 1024,
     "gemm_f32_512x512x512": (4646 * 2 + 1024) * 1024,
     "attention_bf16_b16_h8_s1024_d64_causal": (25124 * 2 + 16384) * 1024,
     "layer_norm_f32_to_bf16_16384x512": (16432 * 2 + 16384) * 1024,
@@ -65,6 +62,15 @@ MEASURED_TRAFFIC_BYTES = {
     "gelu_backward_f32_16384x512": (32788 * 2 + 32768) * 1024,
     "scale_f32_16384x512": (16394 * 2 + 32768) * 1024,
     "sum_axis0_f32_16384x512": ((16401 + 527) * 2 + 512 + 2) * 1024,
+}
+# The same for workloads that run as products of bf16 pieces: the pass that writes the pieces (6 bytes a value) included.
+PIECES_TRAFFIC_BYTES = {
+    "conv2d_bias_relu_f32_n32_c64to128_56x56_k3s1p1": ((16250 + 22269) * 2 + 40924 + 50176) * 1024,
+    "attention_f32_b8_h16_s2048_d64_noncausal": (98416 * 2 + 65536) * 1024,
+    "attention_f32_b8_h16_s2048_d64_causal": (160096 * 2 + 65536) * 1024,
+    "attention_f32_attn_bias_c1_s2048_d64": ((10898 + 4260) * 2 + 8448 + 512) * 1024,
+    "attention_f32_attn_bias_c16_s1024_d64": ((53394 + 4260) * 2 + 8448 + 4096) * 1024,
+    "gemm_f32_4096x4096x4096": ((65571 + 393587) * 2 + 197308 + 65536) * 1024,
 }
 
 
@@ -128,7 +134,7 @@ class Timer:
 def roofline(bound, dtype, flops, bytes_, ms):
     if bound == "mfma":
         achieved = flops / (ms * 1e-3) / 1e12
-        peak = PEAK_TFLOPS[dtype]
+        peak = round(PEAK_TFLOPS[dtype], 1)
         return {"bound": "mfma", "achieved": round(achieved, 3), "peak": peak, "unit": "TFLOP/s",
                 "frac": round(achieved / peak, 4), "traffic": None}
     achieved = bytes_ / (ms * 1e-3) / 1e9
@@ -136,13 +142,14 @@ def roofline(bound, dtype, flops, bytes_, ms):
             "frac": round(achieved / PEAK_HBM_GBS, 4), "traffic": None}
 
 
-def entry(name, dtype, flops, bytes_, bound, wall_ms, event_ms, extra=None, sustained=None):
-    kind = "bf16" if dtype == "bf16" else "f32"
+def entry(name, dtype, flops, bytes_, bound, wall_ms, event_ms, extra=None, sustained=None, pieces=False):
+    """`pieces`: an f32 workload that the library runs as products of bf16 pieces."""
+    kind = "bf16" if dtype == "bf16" else "f32_pieces" if pieces else "f32"
     out = {"workload": name, "dtype": dtype, "flops_per_step": flops, "min_bytes_per_step": bytes_,
            "ms_per_step": round(wall_ms, 5), "kernel_ms_per_step": round(event_ms, 5),
            "gflops": round(flops / (wall_ms * 1e-3) / 1e9, 1),
            "roofline": roofline(bound, kind, flops, bytes_, event_ms)}
-    out["roofline"]["traffic"] = MEASURED_TRAFFIC_BYTES.get(name)
+    out["roofline"]["traffic"] = (PIECES_TRAFFIC_BYTES if pieces else MEASURED_TRAFFIC_BYTES).get(name)
     if sustained:
         again = roofline(bound, kind, flops, bytes_, sustained["kernel_ms_per_step"])
         out["sustained"] = dict(sustained, achieved=again["achieved"], frac=again["frac"])
@@ -181,7 +188,8 @@ def wl_conv2d(hip, inputs, timer):
     wall, ev, sus = timer.measure(step, headline=True)
     flops = 2 * batch * c_out * h * w * c_in * 9
     bytes_ = 4 * (x.size + wt.size + b.size + batch * c_out * h * w)
-    return entry("conv2d_bias_relu_f32_n32_c64to128_56x56_k3s1p1", "f32", flops, bytes_, "mfma", wall, ev, sustained=sus), \
+    pieces = bool(hip.conv2d_f32_split_plan(batch, c_in, h, w, c_out, *geom)["served"])
+    return entry("conv2d_bias_relu_f32_n32_c64to128_56x56_k3s1p1", "f32", flops, bytes_, "mfma", wall, ev, sustained=sus, pieces=pieces), \
         (x, wt, b, geom, (batch, c_in, h, w, c_out))
 
 
@@ -226,7 +234,8 @@ def wl_conv2d_backward(hip, inputs, timer, which):
         bytes_ = 4 * (g.size + wt.size + x.size)
     wall, ev, sus = timer.measure(step)
     flops = 2 * batch * c_out * h * w * c_in * 9
-    return entry(f"conv2d_{which}_f32_n32_c64to128_56x56_k3s1p1", "f32", flops, bytes_, "mfma", wall, ev, sustained=sus)
+    pieces = which == "grad_input" and bool(hip.conv2d_f32_split_plan(batch, c_in, h, w, c_out, *geom, direction="grad_input")["served"])
+    return entry(f"conv2d_{which}_f32_n32_c64to128_56x56_k3s1p1", "f32", flops, bytes_, "mfma", wall, ev, sustained=sus, pieces=pieces)
 
 
 def wl_gemm_f32(hip, inputs, timer, m, n, k, name, long=False):
@@ -239,7 +248,8 @@ def wl_gemm_f32(hip, inputs, timer, m, n, k, name, long=False):
         hip.gemm_f32_dev(m, n, k, 1.0, False, d_a, d_b, d_c, stream)
 
     wall, ev, sus = timer.measure(step, long=long)
-    return entry(name, "f32", 2 * m * n * k, 4 * (m * k + k * n + m * n), "mfma", wall, ev, sustained=sus)
+    return entry(name, "f32", 2 * m * n * k, 4 * (m * k + k * n + m * n), "mfma", wall, ev, sustained=sus,
+                 pieces=bool(hip.gemm_f32_split_plan(m, n, k)["served"]))
 
 
 def wl_gemm_bf16(hip, inputs, timer, m, n, k, name, bound, packed=False):
@@ -294,12 +304,13 @@ def wl_attention(hip, inputs, timer, causal):
     wall, ev, sus = timer.measure(step, long=True)
     flops = 4 * dim * contexts * (seq * (seq + 1) // 2 if causal else seq * seq)
     name = "attention_f32_b8_h16_s2048_d64_" + ("causal" if causal else "noncausal")
-    return entry(name, "f32", flops, 4 * 4 * count, "mfma", wall, ev, sustained=sus)
+    return entry(name, "f32", flops, 4 * 4 * count, "mfma", wall, ev, sustained=sus,
+                 pieces=hip.attention_f32_launch_plan(contexts, seq, dim, causal, scale=0.125)["kernel"] == "split")
 
 
 def wl_attention_bias(hip, inputs, timer, contexts, seq):
     """Attention with a per-query bias matrix, the form the reference's only in-tree Rust caller uses (one context
-    per head with an attn_bias kernel matrix, crates/st-nn/src/z_rba/attention.rs:586-595): general kernel."""
+    per head with an attn_bias kernel matrix, crates/st-nn/src/z_rba/attention.rs:586-595)."""
     dim = 64
     count = contexts * seq * dim
     q, k, v = (inputs.normal(inputs.seed_for(3, i), count) for i in range(3))
@@ -313,7 +324,8 @@ def wl_attention_bias(hip, inputs, timer, contexts, seq):
     wall, ev, sus = timer.measure(step)
     flops = 4 * dim * contexts * seq * seq
     return entry(f"attention_f32_attn_bias_c{contexts}_s{seq}_d64", "f32", flops, 4 * (4 * count + bias.size), "mfma",
-                 wall, ev, sustained=sus)
+                 wall, ev, sustained=sus,
+                 pieces=hip.attention_f32_launch_plan(contexts, seq, dim, False, True, scale=0.125)["kernel"] == "split")
 
 
 def wl_attention_bf16(hip, inputs, timer):
