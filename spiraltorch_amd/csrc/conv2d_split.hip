@@ -9,7 +9,7 @@
 // bounds checks along x and y.  The weights become blocks of 32 rows × 16 terms in the same step order.
 //
 // What bounds it is the matrix cores on random operands, as in the GEMM (21 ns per 32×32×16 instruction and SIMD).
-// Of the whole call, f32 kernels -> here, batch 32 unless given, 3×3: 64 -> 128 on 56×56 146 -> 121 µs (of which 14 are the
+// Of the whole call, f32 kernels -> here, batch 32 unless given, 3×3: 64 -> 128 on 56×56 146 -> 115 µs (of which 15 are the
 // pass), 128 -> 128 on 28×28 93 -> 65, 256 -> 256 on 14×14 99 -> 64, 512 -> 512 on 7×7 119 -> 72,
 // 250 -> 250 on 14×15, batch 31, 189 -> 64, 24 -> 96 5×5 on 112×112, batch 4, 105 -> 67, 256 -> 256 on 28×28, batch 2, 41 -> 30.
 // 64 -> 64 on 56×56 and one-tap layers stay on the f32 kernels (70 against 69 µs, 46 against 51): the pass costs what the
