@@ -655,16 +655,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DPAD <= 64 
 //
 // What bounds it: a 64-key stage of 32 queries is 96 matrix instructions (2.0 µs of a SIMD at the rate random operands allow,
 // 21 ns each) beside some 450 vector ones (softmax, the pieces of the probabilities and of the staged values), two
-// wavefronts per SIMD take 5.2 µs for theirs.  Measured, f32 matrix cores -> here: 128 × 2048 × 64 causal 591 -> 359 µs,
-// non-causal 1070 -> 652, 128 × 1024 causal 163 -> 112; biased 1 × 1000 26 -> 16 µs, 16 × 1024 60 -> 51, biases on rows of
+// wavefronts per SIMD take 5.2 µs for theirs.  Measured, f32 matrix cores -> here: 128 × 2048 × 64 causal 591 -> 360 µs,
+// non-causal 1070 -> 643, 128 × 1024 causal 163 -> 102; biased 1 × 1000 26 -> 16 µs, 16 × 1024 60 -> 51, biases on rows of
 // 777 (no 16-byte alignment: the general kernel) 162 -> 16.  Errors against float64 are 0.7 to 0.85 of the f32 kernel's.
 //
 // V and the probabilities are scaled by 2^24 before they are split, and the output by 2^-48: the last bit of either is then a
 // normal bf16 number, and the pieces are exact however small a value is (a probability of 2^-124 may meet the only non-zero
 // entry of a column of V).  Q and K are not: what their pieces lose is below 2^-90 of a logit's unit.  Values the pieces
 // cannot carry — 2^40 and more in Q or K, 2^70 / S and more in V, where scaled sums could overflow — make the workgroup redo
-// its rows with f32 multiply-adds (redo_rows below): 12 times the time of an ordinary call for 1 × 1000, 20 to 45 times where every
-// unit is busy.  The scaling costs 2 to 4 % of a call: 128 × 2048 × 64 causal 352 -> 359 µs, 128 × 1024 108 -> 112.
+// its rows on the f32 matrix cores (redo_rows below), straight from memory: 3 times the time of an ordinary call for 1 × 1000, 5
+// times where every unit is busy (128 × 2048 × 64 causal 1710 µs; a chain of multiply-adds per row took 8960).  The scaling
+// costs 1 to 2 %.
 // -------------------------------------------------------------------------------------------------
 __device__ __forceinline__ void split_pair(float a, float b, uint32_t &hi, uint32_t &mid, uint32_t &lo)
 {
@@ -693,65 +694,108 @@ __device__ __forceinline__ float largest8(const float (&x)[8], float so_far)
     return so_far;
 }
 
-// One thread per query row, f32 multiply-adds throughout: what the split kernel's workgroups fall back to for operands its
-// pieces cannot carry.  Rows q0 .. q0 + count - 1 over keys [key_first, key_end), in the units of the split kernel.
+// What the split kernel's workgroups fall back to for operands its pieces cannot carry: a wavefront's 32 query rows over keys
+// [key_first, key_end) on the f32 matrix cores, operands straight from memory, in the units of the split kernel.  Keys that
+// some of the rows do not see, and the last ones short of 32, are taken one by one, so that a value behind a row's mask never
+// meets it (zero times infinity).
 template <int DPAD, bool CAUSAL, bool BIAS>
-__device__ void redo_rows(const AttnArgs &p, int ctx, int q0, int count, int threads, int tid, int split, int key_first, int key_end,
-                          float scale_log2e, float exp_scale)
+__device__ void redo_rows(const AttnArgs &p, int ctx, int wq0, int lane, int split, int key_first, int key_end, float scale_log2e,
+                          float exp_scale)
 {
-    const int S = p.S, D = p.D;
+    constexpr int CHUNKS = DPAD / 8, DT = DPAD / 32;
+    const int S = p.S, D = p.D, li = lane & 31, lh = lane >> 5, my_q = wq0 + li;
+    if (wq0 >= S) return;
     const size_t first = static_cast<size_t>(ctx) * S * D;
-    for (int i = tid; i < count; i += threads) {
-        const int row = q0 + i;
-        if (row >= S) continue;
-        // (four dimensions at a time: D is a multiple of 4 here)
-        float4 q[DPAD / 4], o[DPAD / 4];
-        const float *q_row = p.q + first + static_cast<size_t>(row) * D;
+    const float *const keys = p.k + first, *const values = p.v + first;
+    auto load4 = [&](const float *row, int chunk) {  // this half's four of eight dimensions (D is a multiple of 4 here)
+        const int d = chunk * 8 + lh * 4;
+        return d < D ? *reinterpret_cast<const f32x4 *>(row + d) : f32x4{0.f, 0.f, 0.f, 0.f};
+    };
+    const size_t row = static_cast<size_t>(ctx) * S + min(my_q, S - 1);
+    auto with_bias = [&](float logit, int key) {
+        if constexpr (!BIAS) return logit;
+        float bias = p.attn_bias ? p.attn_bias[row * S + key] : 0.0f;
+        if (p.z_bias) bias += p.z_bias[static_cast<size_t>(ctx) * S + key];
+        return fmaf(logit, scale_log2e, bias * kLog2e);
+    };
+    f32x4 q[CHUNKS];
+    f32x16 o[DT];
 #pragma unroll
-        for (int g = 0; g < DPAD / 4; ++g) {
-            q[g] = o[g] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (g * 4 < D) q[g] = *reinterpret_cast<const float4 *>(q_row + g * 4);
-            if (p.scale < 0.0f) q[g] = make_float4(-q[g].x, -q[g].y, -q[g].z, -q[g].w);
-        }
-        float top = -INFINITY, sum = 0.0f;
-        const int end = CAUSAL ? min(key_end, row + 1) : key_end;
-        for (int key = key_first; key < end; ++key) {
-            const float *k = p.k + first + static_cast<size_t>(key) * D, *v = p.v + first + static_cast<size_t>(key) * D;
-            float logit = 0.0f;
-#pragma unroll
-            for (int g = 0; g < DPAD / 4; ++g) {
-                if (g * 4 >= D) break;
-                const float4 k4 = *reinterpret_cast<const float4 *>(k + g * 4);
-                logit = fmaf(k4.w, q[g].w, fmaf(k4.z, q[g].z, fmaf(k4.y, q[g].y, fmaf(k4.x, q[g].x, logit))));
-            }
-            if constexpr (BIAS) {
-                float bias = p.attn_bias ? p.attn_bias[(static_cast<size_t>(ctx) * S + row) * S + key] : 0.0f;
-                if (p.z_bias) bias += p.z_bias[static_cast<size_t>(ctx) * S + key];
-                logit = fmaf(logit, scale_log2e, bias * kLog2e);
-            }
-            const float new_top = fmaxf(top, logit);
-            const float safe = new_top == -INFINITY ? 0.0f : new_top;
-            const float alpha = __builtin_amdgcn_exp2f((top - safe) * exp_scale);
-            const float w = __builtin_amdgcn_exp2f(fmaf(logit, exp_scale, -safe * exp_scale));
-            sum = fmaf(sum, alpha, w);
-#pragma unroll
-            for (int g = 0; g < DPAD / 4; ++g) {
-                if (g * 4 >= D) break;
-                const float4 v4 = *reinterpret_cast<const float4 *>(v + g * 4);
-                o[g] = make_float4(fmaf(w, v4.x, o[g].x * alpha), fmaf(w, v4.y, o[g].y * alpha), fmaf(w, v4.z, o[g].z * alpha),
-                                   fmaf(w, v4.w, o[g].w * alpha));
-            }
-            top = new_top;
-        }
-        const bool partial = p.key_splits > 1;
-        const size_t at = (static_cast<size_t>(split) * p.contexts + ctx) * S + row;
-        float *out = partial ? p.part_o + at * D : p.out + first + static_cast<size_t>(row) * D;
-        const float inv = partial ? 1.0f : sum > 0.0f ? 1.0f / sum : 0.0f;
-#pragma unroll
-        for (int g = 0; g < DPAD / 4; ++g)
-            if (g * 4 < D) *reinterpret_cast<float4 *>(out + g * 4) = make_float4(o[g].x * inv, o[g].y * inv, o[g].z * inv, o[g].w * inv);
-        if (partial) *reinterpret_cast<float2 *>(p.part_ml + at * 2) = make_float2(top, sum);
+    for (int c = 0; c < CHUNKS; ++c) {
+        q[c] = load4(p.q + row * D, c);
+        if (p.scale < 0.0f) q[c] = -q[c];
     }
+#pragma unroll
+    for (int t = 0; t < DT; ++t) o[t] = f32x16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float top = -INFINITY, sum = 0.0f;
+    auto rescale = [&](float logit) {  // to the running maximum with `logit` in it; returns what an exponent is shifted by
+        const float new_top = fmaxf(top, logit), safe = new_top == -INFINITY ? 0.0f : new_top;
+        const float alpha = __builtin_amdgcn_exp2f((top - safe) * exp_scale);
+        sum *= alpha;
+#pragma unroll
+        for (int t = 0; t < DT; ++t) o[t] *= alpha;
+        top = new_top;
+        return -safe * exp_scale;
+    };
+    const int plain_end = min(key_end, CAUSAL ? min(S, wq0 + 1) : S), end = min(key_end, CAUSAL ? min(S, wq0 + 32) : S);
+    int key = key_first;
+    for (; key + 32 <= plain_end; key += 32) {
+        // register 4g + j of lane (li, lh): key 8g + 4·lh + j, query li
+        f32x16 score = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < CHUNKS; ++c) {
+            const f32x4 k4 = load4(keys + static_cast<size_t>(key + li) * D, c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) score = __builtin_amdgcn_mfma_f32_32x32x2f32(k4[e], q[c][e], score, 0, 0, 0);
+        }
+        float most = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            score[r] = with_bias(score[r], key + (r >> 2) * 8 + lh * 4 + (r & 3));
+            most = fmaxf(most, score[r]);
+        }
+        const float shift = rescale(fmaxf(most, __shfl_xor(most, 32)));
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            score[r] = __builtin_amdgcn_exp2f(fmaf(score[r], exp_scale, shift));
+            sum += score[r];
+            const float *const value = values + static_cast<size_t>(key + (r >> 2) * 8 + lh * 4 + (r & 3)) * D;
+#pragma unroll
+            for (int t = 0; t < DT; ++t)
+                o[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(t * 32 + li < D ? value[t * 32 + li] : 0.0f, score[r], o[t], 0, 0, 0);
+        }
+    }
+    sum += __shfl_xor(sum, 32);  // both halves go on with the row's whole sum
+    for (; key < end; ++key) {
+        float logit = 0.0f;
+#pragma unroll
+        for (int c = 0; c < CHUNKS; ++c) {
+            const f32x4 k4 = load4(keys + static_cast<size_t>(key) * D, c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) logit = fmaf(k4[e], q[c][e], logit);
+        }
+        logit = with_bias(logit + __shfl_xor(logit, 32), key);
+        if (CAUSAL && key > my_q) continue;
+        const float weight = __builtin_amdgcn_exp2f(fmaf(logit, exp_scale, rescale(logit)));
+        sum += weight;
+#pragma unroll
+        for (int c = 0; c < CHUNKS; ++c) {
+            const f32x4 v4 = load4(values + static_cast<size_t>(key) * D, c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[c / 4][c % 4 * 4 + e] = fmaf(weight, v4[e], o[c / 4][c % 4 * 4 + e]);
+        }
+    }
+    if (my_q >= S) return;
+    const bool partial = p.key_splits > 1;
+    const size_t at = (static_cast<size_t>(split) * p.contexts + ctx) * S + my_q;
+    float *const out = partial ? p.part_o + at * D : p.out + first + static_cast<size_t>(my_q) * D;
+    const float inv = partial ? 1.0f : sum > 0.0f ? 1.0f / sum : 0.0f;
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c)
+        if (c * 8 + lh * 4 < D)
+            *reinterpret_cast<float4 *>(out + c * 8 + lh * 4) = make_float4(o[c / 4][c % 4 * 4] * inv, o[c / 4][c % 4 * 4 + 1] * inv,
+                                                                           o[c / 4][c % 4 * 4 + 2] * inv, o[c / 4][c % 4 * 4 + 3] * inv);
+    if (partial && lh == 0) *reinterpret_cast<float2 *>(p.part_ml + at * 2) = make_float2(top, sum);
 }
 
 template <int DPAD, bool CAUSAL, bool BIAS, int WAVES>
@@ -1038,7 +1082,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_split_kernel(AttnArg
     const float total = run_sum + __shfl_xor(run_sum, 32);
     if constexpr (CHAINS == 2) oacc[0] += oacc[1];
     if (redo) {
-        redo_rows<DPAD, CAUSAL, BIAS>(p, ctx, q0, BQ, THREADS, tid, split, key_first, key_end, scale_log2e, exp_scale);
+        redo_rows<DPAD, CAUSAL, BIAS>(p, ctx, wq0, lane, split, key_first, key_end, scale_log2e, exp_scale);
     } else if (my_q < S) {
         const bool partial = p.key_splits > 1;
         const size_t row = (static_cast<size_t>(split) * p.contexts + ctx) * S + my_q;

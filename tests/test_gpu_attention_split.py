@@ -1,4 +1,6 @@
 """f32 attention on the bf16 matrix cores (head sizes up to 64), every value as three exact bf16 pieces, against float64."""
+import time
+
 import numpy as np
 import pytest
 
@@ -95,3 +97,43 @@ def test_small_probabilities_and_values_keep_their_bits(hip, contexts, seq, dim)
         # an f32 result of 1e-39 is a multiple of 2^-149; weighted sums of the entries round no more than seq times 2^-24
         assert np.abs(got[c, :, 5] - want[:, 5]).max() <= 2.0 ** -149 + seq * 2.0 ** -24 * 1e-38
         assert np.abs(got[c, :, 9] - want[:, 9]).max() <= 2.0 ** -20
+
+
+@pytest.mark.parametrize("contexts,seq,dim,causal,biased", [
+    (1, 1, 64, False, True), (2, 65, 64, True, False), (3, 129, 60, False, True), (2, 191, 36, True, True), (1, 777, 64, False, True),
+    (5, 333, 32, False, False), (4, 1001, 64, True, True), (2, 1025, 20, False, True), (128, 513, 64, True, False), (90, 641, 64, False, False)])
+def test_redone_rows_against_float64(hip, contexts, seq, dim, causal, biased):
+    """Every query holds a value of 2^41 that meets zeros in K: no logit depends on it, but every workgroup sums in f32."""
+    rng = np.random.default_rng(seq + dim)
+    q, k, v = (rng.normal(size=(contexts, seq, dim)).astype(np.float32) for _ in range(3))
+    q[..., 1] = 2.0 ** 41
+    k[..., 1] = 0.0
+    zb = rng.normal(0, 0.5, (contexts, seq)).astype(np.float32) if biased else None
+    ab = rng.normal(0, 0.5, (contexts, seq, seq)).astype(np.float32) if biased else None
+    for scale in (1.0 / np.sqrt(dim), -0.3):
+        got = run(hip, q, k, v, scale, causal, zb, ab)
+        for c in sorted({0, contexts // 2, contexts - 1}):
+            want = exact(q[c], k[c], v[c], float(np.float32(scale)), causal, None if zb is None else zb[c], None if ab is None else ab[c])
+            error = got[c] - want  # the bounds of the test above; f32 sums of `dim` and `seq` terms stay within them
+            assert np.sqrt(np.mean(error ** 2)) <= 2.0 ** -20 * np.sqrt(np.mean(want ** 2))
+            assert np.abs(error).max() <= 2.0 ** -15
+
+
+def test_redone_rows_take_the_matrix_cores(hip):
+    """About five times the ordinary time where every workgroup redoes its rows (a chain of multiply-adds per row: 20 to 45)."""
+    n = 128 * 1024 * 64
+    data = np.random.default_rng(1).normal(size=n).astype(np.float32)
+    wild = data.copy()
+    wild[::64] = 2.0 ** 41
+    d_q, d_wild, d_out = (hip.DeviceBuffer.from_array(a) for a in (data, wild, data))
+    for causal in (False, True):
+        def best(d_k):
+            times = []
+            for _ in range(5):
+                start = time.perf_counter()
+                hip.attention_f32_dev(128, 1024, 64, 0.125, causal, d_q, d_k, d_q, None, None, d_out)
+                hip.device_synchronize()
+                times.append(time.perf_counter() - start)
+            return min(times)
+
+        assert best(d_wild) <= 15 * best(d_q)
