@@ -661,7 +661,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DPAD <= 64 
 //
 // V and the probabilities are scaled by 2^24 before they are split, and the output by 2^-48: the last bit of either is then a
 // normal bf16 number, and the pieces are exact however small a value is (a probability of 2^-124 may meet the only non-zero
-// entry of a column of V).  Q and K are not: what their pieces lose is below 2^-90 of a logit's unit.  Values the pieces
+// entry of a column of V).  Q and K are not: what their pieces lose is below 2^-80, against the 1 a logit is compared with.  Values the pieces
 // cannot carry — 2^40 and more in Q or K, 2^70 / S and more in V, where scaled sums could overflow — make the workgroup redo
 // its rows on the f32 matrix cores (redo_rows below), straight from memory: 3 times the time of an ordinary call for 1 × 1000, 5
 // times where every unit is busy (128 × 2048 × 64 causal 1710 µs; a chain of multiply-adds per row took 8960).  The scaling

@@ -17,7 +17,8 @@
 // rectified N(0,1) images).
 //
 // Values the scaled pieces cannot carry or whose sums could overflow (gemm_f32_split.hip) are found by the pass, by the image
-// and by the weight block; tiles that see such magnitudes are computed with f32 multiply-adds from the original operands.
+// and by the weight block; tiles that see such magnitudes are summed on the f32 matrix cores from the original operands.  Small
+// values, subnormal ones included, cost nothing.
 #include <algorithm>
 
 #include "kernels.h"

@@ -18,7 +18,7 @@
 //
 // Both operands are scaled by a power of two first, so that the pieces are exact down to the smallest f32 value.  Values too
 // large for that or not finite, and pairs of magnitudes whose scaled sums could overflow (about 1e10 against 1e10), are
-// found by the splitting pass; the tiles they touch are computed with f32 multiply-adds from the original operands.
+// found by the splitting pass; the tiles they touch are summed on the f32 matrix cores from the original operands.
 #include <algorithm>
 #include <type_traits>
 
