@@ -140,7 +140,7 @@ def test_values_the_pieces_cannot_carry(hip):
             bound = 8 * 2.0 ** -24 * np.sqrt(576) * scale + 576 * 2.0 ** -149
             diff = np.abs(got[image, channels][ok] - want[image, channels][ok])
             assert (diff <= np.maximum(bound, 2.0 ** -20 * np.abs(want[image, channels][ok]))).all(), image
-    # tiles beside channel 9 are now summed in f32: both sums keep to the bound above, the results' rms is 24
+    # images and channels without such values: both runs keep to the bound above, the results' rms is 24
     untouched, keep = np.arange(32) >= 8, np.arange(128) != 9
     assert np.abs(got[untouched][:, keep] - plain[untouched][:, keep]).max() <= 8 * 2.0 ** -24 * np.sqrt(576) * 24
 

@@ -92,8 +92,8 @@ def test_small_values_beside_ordinary_ones(hip, m, n, k, layout):
 
 
 def test_values_the_pieces_cannot_carry(hip):
-    """Infinities, NaN, values next to the largest f32 and rows small enough to lose their low pieces: the tiles they touch
-    give what f32 arithmetic on the operands gives, the other tiles are not disturbed."""
+    """Infinities, NaN and values next to the largest f32: the tiles they touch give what f32 arithmetic on the operands
+    gives, the other tiles are not disturbed.  Rows below 2^-110 are carried like any other."""
     m, n, k = 1233, 1000, 700
     rng = np.random.default_rng(3)
     a, b = rng.normal(size=(m, k)).astype(np.float32), rng.normal(size=(k, n)).astype(np.float32)
