@@ -78,6 +78,54 @@ __device__ __forceinline__ float layer_norm_scale_shift(float normalised, float 
     return scaled + beta;
 }
 
+// Sum over a wavefront, the same in every lane: v += the value 32, 16, ... 1 lanes away (lane ^ offset), without a trip
+// through LDS.  The exchanges over 32 and 16 lanes swap halves and rows; within a row of sixteen the sum so far repeats every
+// 2·offset lanes, so that a rotation by `offset` reaches the value of lane ^ offset.
+__device__ __forceinline__ float wave_sum(float v)
+{
+    const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(halves[0]) + __uint_as_float(halves[1]);
+    const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(rows[0]) + __uint_as_float(rows[1]);
+    auto rotated = [](float x, auto control) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(control)::value, 0xf, 0xf, true));
+    };
+    v += rotated(v, std::integral_constant<int, 0x128>{});  // row_ror:8
+    v += rotated(v, std::integral_constant<int, 0x124>{});
+    v += rotated(v, std::integral_constant<int, 0x122>{});
+    v += rotated(v, std::integral_constant<int, 0x121>{});
+    return v;
+}
+
+// The normalisation of a row whose sum and sum of squares are known.
+struct LayerNormRow {
+    float mean, denom, inv;
+    __device__ __forceinline__ LayerNormRow(float sum, float sumsq, float cols_f, float epsilon)
+    {
+        mean = sum / cols_f;
+        denom = layer_norm_denominator(layer_norm_variance(sumsq, mean, cols_f), epsilon);
+        inv = 1.0f / denom;
+    }
+    // (v - mean) / denom for every element, with one real division per row: the product with the correctly rounded
+    // reciprocal, corrected once by its exact remainder (two fused multiply-adds), is the correctly rounded quotient
+    // again, i.e. bit for bit what the division gives; only the last bit matters here, because it decides some of
+    // the bf16 roundings downstream and the decoder is compared with a CPU stack that divides.
+    __device__ __forceinline__ float quotient(float a) const
+    {
+        const float q = a * inv;
+        return fmaf(fmaf(-q, denom, a), inv, q);
+    }
+    __device__ __forceinline__ float4 apply(const float4 &v, const float4 &gamma, const float4 &beta) const
+    {
+        float4 o;
+        o.x = layer_norm_scale_shift(quotient(v.x - mean), gamma.x, beta.x);
+        o.y = layer_norm_scale_shift(quotient(v.y - mean), gamma.y, beta.y);
+        o.z = layer_norm_scale_shift(quotient(v.z - mean), gamma.z, beta.z);
+        o.w = layer_norm_scale_shift(quotient(v.w - mean), gamma.w, beta.w);
+        return o;
+    }
+};
+
 // Runs `body(act, has_residual)` with the activation as a callable and the presence of a residual as a compile-time
 // constant, chosen once from the (wavefront-uniform) launch arguments: an epilogue that decides them per element
 // compiles to a chain of scalar branches around every store.

@@ -2333,6 +2333,22 @@ TilePlan plan_tiles(size_t m, size_t n, size_t k)
     return plan;
 }
 
+// Whether the small tiles of gemm_bf16_small.hip take an m×n×k product (operands on 16-byte boundaries), by the estimated time
+// of the kernels here: both tilings, k split or not, in rounds of what the chip holds; the general kernel where those do not
+// take the shape.  The constants are those of the split's estimate and about 4 µs a launch (measured 6.5 to 8 µs at k = 512
+// from 128 to 2048 rows).
+bool small_tiles_apply(size_t m, size_t n, size_t k)
+{
+    if (k < 64 || k % 64 != 0) return false;
+    const size_t cols = (n + 127) / 128, tiles_128 = (m + 127) / 128 * cols, tiles_256 = (m + 255) / 256 * cols;
+    auto rounds = [](size_t tiles, size_t most) { return static_cast<double>((tiles + most - 1) / most); };
+    const double us = n % 128 != 0 && (m <= 64 || n <= 128)
+                          ? 6.0 + 0.01 * static_cast<double>(k)
+                          : 4.0 + std::min(rounds(tiles_128, 512) * estimate_k_splits(m, n, k, tiles_128, 512, 0.42).cost_us,
+                                           rounds(tiles_256, 256) * estimate_k_splits(m, n, k, tiles_256, 256, 0.5).cost_us);
+    return gemm_bf16_small_applies(m, n, k, us);
+}
+
 // The launch arithmetic of the tiled kernels whose workgroups decode their index into (k-split, tile), checked on the
 // host before every launch: the grid is tiles × k-splits and fits the 32-bit ids the kernels compute with, the tiles
 // cover the matrix without an empty row or column of tiles, every split has k-tiles to walk and together they cover K,
@@ -2706,6 +2722,18 @@ hipError_t launch_gemm_bf16(size_t m, size_t n, size_t k, const uint16_t *lhs, c
         fits_buffer)
         return launch_skinny_packed(args, stream);
     size_t workspace_offset = 0;
+    // Few rows or few columns: small tiles with k split inside the workgroup.  (A row-major B of up to 64 rows and a long k
+    // stays with the skinny kernel, which reads it in longer pieces: 64×768×3072 8.6 µs against 9.9.)
+    if (aligned16(lhs) && aligned16(rhs) && fits_buffer && small_tiles_apply(m, n, k) && !(skinny && k > 1024)) {
+        if (rhs_packed || n % 8 == 0) return launch_gemm_bf16_small(m, n, k, lhs, rhs, rhs_packed, out_f32, out_bf16, epilogue, stream);
+        // rows of B that start at any 2-byte boundary: packed first, one pass
+        void *workspace = nullptr;
+        hipError_t rc = stream_workspace(stream, k * n * sizeof(uint16_t), &workspace);
+        if (rc != hipSuccess) return rc;
+        rc = launch_transpose_u16(k, n, rhs, static_cast<uint16_t *>(workspace), stream);
+        if (rc != hipSuccess) return rc;
+        return launch_gemm_bf16_small(m, n, k, lhs, static_cast<const uint16_t *>(workspace), true, out_f32, out_bf16, epilogue, stream);
+    }
     // An n that is not a multiple of 128 (a vocabulary of 50257, 1000 classes) with a k the 256-row kernels take: the
     // packed kernels run it as it is — rows of Bᵀ past n read as zero through the buffer range check, and the epilogue
     // for a ragged n stores at any alignment.  A row-major B is packed into the stream's workspace first (one pass
@@ -2952,8 +2980,9 @@ hipError_t launch_gemm_bf16_residual_layer_norm(size_t m, size_t n, size_t k, co
     // k = 512, 51.2 against 37.9 + 10.1 µs at k = 2048 — a 64-row tile streams the whole of B through every compute unit,
     // which costs more than the saved pass over the rows once k is long.
     // (m <= 64 stays with the GEMM dispatcher, which splits k over the chip for such shapes, and so does every shape of
-    // few row tiles and a long k that the dispatcher would split: the split sums add up in another order.)
-    if (n == 512 && m > 64 && k >= 64 && k % 64 == 0 && k <= 1024 && fits_buffer && aligned && plan_tiles(m, n, k).k_splits == 1) {
+    // few row tiles and a long k that the dispatcher would split or give to the small tiles: those sums add up in another order.)
+    if (n == 512 && m > 64 && k >= 64 && k % 64 == 0 && k <= 1024 && fits_buffer && aligned && plan_tiles(m, n, k).k_splits == 1 &&
+        !small_tiles_apply(m, n, k)) {
         RowLnArgs row;
         row.g.A = lhs;
         row.g.B = packed_rhs;

@@ -36,14 +36,6 @@ constexpr int kUnroll = 4;  // 16-byte loads of A in flight per lane
 __device__ __forceinline__ float bf16_lo(uint32_t pair) { return __builtin_bit_cast(float, pair << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t pair) { return __builtin_bit_cast(float, pair & 0xffff0000u); }
 
-// Sum over the 64 lanes, the same tree in every wavefront.
-__device__ __forceinline__ float wave_sum(float v)
-{
-#pragma unroll
-    for (int offset = 32; offset > 0; offset >>= 1) v += __shfl_xor(v, offset, 64);
-    return v;
-}
-
 // Finishes a row: the cross-wavefront sum when the workgroup shares the row (WIDE), then the epilogue, written by lane 0.
 template <int NC, bool WIDE>
 __device__ __forceinline__ void finish_row(const GemvArgs &p, int row, bool active, float (&acc)[NC])

@@ -20,13 +20,6 @@ __device__ __forceinline__ int token_to_index(float value, int vocab)
     return index;
 }
 
-__device__ __forceinline__ float wave_sum(float v)
-{
-#pragma unroll
-    for (int offset = 32; offset > 0; offset >>= 1) v += __shfl_xor(v, offset);
-    return v;
-}
-
 // One wavefront per row.  layer_norm_cpu, crates/st-tensor/src/pure.rs:4008-4058:
 // mean = Σv/cols; var = max(Σv²/cols − mean², 0); out = ((v − mean)/sqrt(var + eps))·γ + β.
 __global__ __launch_bounds__(256) void layer_norm_kernel(int rows, int cols, const float *x, const float *residual,
@@ -125,27 +118,12 @@ __global__ __launch_bounds__(256) void layer_norm_vec_kernel(int rows, int cols,
         }
         sum = wave_sum(sum);
         sumsq = wave_sum(sumsq);
-        const float mean = sum / cols_f;
-        const float var = layer_norm_variance(sumsq, mean, cols_f);
-        const float denom = layer_norm_denominator(var, epsilon);
-        // (v - mean) / denom for every element, with one real division per row: the product with the correctly rounded
-        // reciprocal, corrected once by its exact remainder (two fused multiply-adds), is the correctly rounded quotient
-        // again, i.e. bit for bit what the division gives; only the last bit matters here, because it decides some of
-        // the bf16 roundings downstream and the decoder is compared with a CPU stack that divides.
-        const float inv = 1.0f / denom;
-        auto quotient = [&](float a) {
-            const float q = a * inv;
-            return fmaf(fmaf(-q, denom, a), inv, q);
-        };
+        const LayerNormRow norm(sum, sumsq, cols_f, epsilon);
 #pragma unroll
         for (int i = 0; i < CHUNKS; ++i) {
             const int c = (lane + 64 * i) * 4;
             if (c >= cols) continue;
-            float4 o;
-            o.x = layer_norm_scale_shift(quotient(v[r][i].x - mean), g[i].x, b[i].x);
-            o.y = layer_norm_scale_shift(quotient(v[r][i].y - mean), g[i].y, b[i].y);
-            o.z = layer_norm_scale_shift(quotient(v[r][i].z - mean), g[i].z, b[i].z);
-            o.w = layer_norm_scale_shift(quotient(v[r][i].w - mean), g[i].w, b[i].w);
+            const float4 o = norm.apply(v[r][i], g[i], b[i]);
             if (out_f32) *reinterpret_cast<float4 *>(out_f32 + offset + c) = o;
             if (out_bf16) {
                 uint2 packed;
