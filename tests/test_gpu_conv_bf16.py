@@ -142,3 +142,53 @@ def test_unsupported_and_invalid_arguments(hip):
     assert info.value.kind == "Unsupported" or "aligned" in info.value.message
     # an empty batch is a no-op
     hip.conv2d_bias_act_bf16_dev(0, 3, 8, 8, 4, (3, 3), (1, 1), (1, 1), (1, 1), 0, d, d, None, d, None)
+
+
+@pytest.mark.parametrize("shape", [
+    (1, 64, 9, 9, 64, (3, 3), (1, 1), (1, 1), (1, 1)),       # 81 pixels: two 64-wide tiles, k cut over workgroups
+    (2, 72, 12, 11, 40, (5, 5), (1, 1), (2, 2), (1, 1)),     # 225 chunks: the last k-tile one eighth full; planes of 132
+    (1, 512, 5, 5, 96, (7, 7), (2, 2), (3, 3), (1, 1)),      # 392 k-tiles for nine pixels: many cuts, odd planes
+    (4, 20, 33, 47, 100, (1, 1), (2, 3), (0, 0), (1, 1)),    # one tap, strides: only the pixels it is put on are copied
+    (2, 9, 20, 21, 33, (1, 5), (3, 2), (1, 2), (2, 1)),      # one row of taps with stride and padding
+    (2, 9, 21, 20, 33, (5, 1), (2, 3), (2, 1), (1, 2)),      # one column
+    (1, 5, 30, 30, 17, (9, 9), (1, 1), (4, 4), (1, 1)),      # 81 taps: more than a pass of the weights takes
+    (1, 16, 30, 30, 17, (9, 9), (2, 2), (4, 4), (1, 1)),
+    (6, 128, 40, 40, 128, (3, 3), (1, 1), (1, 1), (1, 1)),   # 128-row tiles
+    (16, 24, 56, 56, 128, (3, 3), (1, 1), (1, 1), (1, 1)),   # wide tiles, ragged k
+    (9, 256, 47, 46, 288, (3, 3), (1, 1), (1, 1), (1, 1)),   # 256-row tiles, 288 channels
+])
+def test_tiles_chunks_and_cuts_of_k(hip, shape):
+    """Every tile and route of conv2d_bf16.hip against float64: exact products, so a sum of k of them is off by at most k f32
+    roundings of the sum of magnitudes.  Both outputs, bias and ReLU; the same bits from call to call."""
+    import torch
+    import torch.nn.functional as F
+    from spiraltorch_amd import inputs
+    batch, c_in, h, w, c_out, kernel, stride, padding, dilation = shape
+    rng = np.random.default_rng(sum(shape[:5]) + kernel[0])
+    x16, w16, bias = operands(rng, shape)
+    x = torch.from_numpy(inputs.from_bf16(x16).reshape(batch, c_in, h, w).astype(np.float64))
+    wt = torch.from_numpy(inputs.from_bf16(w16).reshape(c_out, c_in, *kernel).astype(np.float64))
+    conv = lambda a, b: F.conv2d(a, b, None, stride, padding, dilation).numpy()
+    plain, magnitude = conv(x, wt), conv(x.abs(), wt.abs())
+    bound = c_in * kernel[0] * kernel[1] * 2.0 ** -24 * (magnitude + np.abs(bias)[None, :, None, None])
+    got, got16 = run(hip, shape, 1, x16, w16, bias, True, True)
+    want = np.maximum(plain + bias[None, :, None, None], 0.0)
+    assert (np.abs(got.reshape(want.shape) - want) <= bound).all()
+    assert (got16 == inputs.to_bf16(got)).all()
+    again, _ = run(hip, shape, 1, x16, w16, bias, True, False)
+    assert (again.view(np.uint32) == got.view(np.uint32)).all()
+
+
+def test_non_finite_pixels_stay_where_they_belong(hip):
+    """Infinity and NaN reach exactly the outputs whose window holds them: nothing of the padding of channels, of k or of the
+    image multiplies a neighbouring value by zero."""
+    from spiraltorch_amd import inputs
+    shape = (2, 11, 14, 18, 10, (3, 3), (1, 1), (1, 1), (1, 1))
+    x16, w16, _ = operands(np.random.default_rng(8), shape)
+    x = inputs.from_bf16(x16).reshape(2, 11, 14, 18).copy()
+    x[0, 10, 13, 17], x[1, 0, 0, 0] = np.inf, np.nan
+    got, _ = run(hip, shape, 0, inputs.to_bf16(x.ravel()), w16, None)
+    bad = ~np.isfinite(got.reshape(2, 10, 14, 18))
+    want = np.zeros_like(bad)
+    want[0, :, 12:, 16:] = want[1, :, :2, :2] = True
+    assert (bad == want).all()
