@@ -931,6 +931,23 @@ bool f32_split_preferred(size_t m, size_t n, size_t k, bool lhs_transposed, bool
     return gemm_f32_split_applies(m, n, k, f32_kernels_us(m, n, k, lhs_transposed, rhs_packed, lhs, rhs, scratch_free), scratch_free);
 }
 
+// The same for products of few tiles, µs (within a fifth of some hundred from 8 rows up), and whether the small tiles of
+// gemm_f32_small.hip beat it.  What the kernels here take grows with the k-tiles a workgroup walks, up to where k is sliced; the
+// ring kernel that splits k inside a workgroup is the least of them.  (Asked after the split products: those keep the shapes they
+// take, with fewer roundings.)
+bool f32_small_preferred(size_t m, size_t n, size_t k, bool lhs_transposed, bool rhs_packed, const float *lhs, const float *rhs)
+{
+    const double flops = 2.0 * m * n * k, k_tiles = static_cast<double>((k + 15) / 16);
+    const bool rows = aligned16(lhs) && aligned16(rhs) && (lhs_transposed ? m : k) % 4 == 0 && (rhs_packed ? k : n) % 4 == 0;
+    const bool ring = rows && k % 16 == 0;
+    double us;
+    if (lhs_transposed) us = 4.1 + (ring ? 0.30 : rows ? 0.40 : 0.48) * std::min(k_tiles, 25.0) + flops / 100.0e6;
+    else if (rhs_packed) us = (ring ? 4.0 + 0.30 * std::min(k_tiles, 23.0) : 6.8 + 0.60 * k_tiles) + flops / 100.0e6;
+    else if (ring) us = (k >= 128 ? 3.2 + 0.05 * k_tiles : 5.2) + flops / 90.0e6;
+    else us = 4.2 + 0.55 * std::min(k_tiles, 24.0) + flops / 100.0e6;
+    return gemm_f32_small_applies(m, n, k, lhs_transposed, rhs_packed, lhs, rhs, us);
+}
+
 hipError_t launch_gemm_f32_native(size_t m, size_t n, size_t k, bool lhs_transposed, const float *lhs, const float *rhs, float *out,
                                   const GemmEpilogue &epilogue, hipStream_t stream, bool scratch_free);
 
@@ -954,6 +971,8 @@ hipError_t launch_gemm_f32(size_t m, size_t n, size_t k, bool lhs_transposed, co
         const hipError_t rc = launch_gemm_f32_split(m, n, k, lhs_transposed, lhs, false, rhs, out, epilogue, stream, scratch_free);
         if (!scratch_unavailable(rc)) return rc;
     }
+    if (f32_small_preferred(m, n, k, lhs_transposed, false, lhs, rhs))
+        return launch_gemm_f32_small(m, n, k, lhs_transposed, lhs, false, rhs, out, epilogue, stream);
     return launch_gemm_f32_native(m, n, k, lhs_transposed, lhs, rhs, out, epilogue, stream, scratch_free);
 }
 
@@ -1104,6 +1123,8 @@ hipError_t launch_gemm_f32_packed(size_t m, size_t n, size_t k, const float *lhs
         const hipError_t rc = launch_gemm_f32_split(m, n, k, false, lhs, true, packed_rhs, out, epilogue, stream, true);
         if (!scratch_unavailable(rc)) return rc;
     }
+    if (f32_small_preferred(m, n, k, false, true, lhs, packed_rhs))
+        return launch_gemm_f32_small(m, n, k, false, lhs, true, packed_rhs, out, epilogue, stream);
     const bool ring_ok = k >= 16 && k % 16 == 0 && aligned16(lhs) && aligned16(packed_rhs) && m * k * 4 < (1ull << 31) &&
                          k * n * 4 < (1ull << 31);
     if (!ring_ok) {

@@ -49,7 +49,12 @@ hipError_t launch_gemm_f32_packed(size_t m, size_t n, size_t k, const float *lhs
 bool gemm_f32_split_applies(size_t m, size_t n, size_t k, double other_us, bool may_split_k);
 hipError_t launch_gemm_f32_split(size_t m, size_t n, size_t k, bool lhs_transposed, const float *lhs, bool rhs_packed, const float *rhs,
                                  float *out, const GemmEpilogue &epilogue, hipStream_t stream, bool may_split_k);
-// Whether launch_gemm_f32 (launch_gemm_f32_packed if `rhs_packed`) runs a product of 16-byte aligned operands that way, and how
+// The same products on small tiles with k split inside the workgroup (gemm_f32_small.hip): any layout, size and alignment, no
+// scratch memory.  `applies`: operands that fit 32-bit offsets and an estimated time below `other_us`.
+bool gemm_f32_small_applies(size_t m, size_t n, size_t k, bool lhs_transposed, bool rhs_packed, const float *lhs, const float *rhs, double other_us);
+hipError_t launch_gemm_f32_small(size_t m, size_t n, size_t k, bool lhs_transposed, const float *lhs, bool rhs_packed, const float *rhs,
+                                 float *out, const GemmEpilogue &epilogue, hipStream_t stream);
+// Whether launch_gemm_f32 (launch_gemm_f32_packed if `rhs_packed`) runs a product of 16-byte aligned operands on the split kernels, and how
 // it is then cut: see st_hip_gemm_split_plan.
 bool gemm_f32_split_served(size_t m, size_t n, size_t k, bool lhs_transposed, bool rhs_packed);
 struct GemmSplitPlanReport {
