@@ -6,6 +6,8 @@
 // stream has drained — also on error paths (StreamCompletionGuard, real.rs:669-697).  Instead of the
 // reference's per-call hipMalloc/hipStreamCreate, buffers and streams come from a pool of workspaces;
 // a workspace is used by one call at a time, so concurrent callers never share device memory.
+#include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -73,7 +75,8 @@ class Lease {
     ~Lease()
     {
         if (ws_) {
-            (void)hipStreamSynchronize(ws_->stream);
+            if (!drained_) (void)hipStreamSynchronize(ws_->stream);
+            for (const PinnedBuffer &stage : stages_) pinned_release(stage);
             pool().release(ws_);
         }
     }
@@ -103,8 +106,23 @@ class Lease {
         ST_HIP_CHECK(buffer(slot, bytes, device));
         if (bytes) {
             count_transfer(true, bytes);
-            ST_HIP_TRY(hipMemcpyAsync(*device, host, bytes, hipMemcpyHostToDevice, ws_->stream),
-                       "hipMemcpyAsync(H2D)");
+            drained_ = false;
+            // Ordinary memory is copied into pinned memory piece by piece, and each piece sent by a kernel beside the copying of the
+            // next: the runtime's own copy holds the caller as long and then waits between the engines.
+            constexpr size_t kPiece = 256u << 10;
+            PinnedBuffer stage;
+            if (bytes > kStageMost || (bytes >= kPiece && is_pinned(host)) || !pinned_acquire(bytes, &stage)) {
+                ST_HIP_TRY(hipMemcpyAsync(*device, host, bytes, hipMemcpyHostToDevice, ws_->stream),
+                           "hipMemcpyAsync(H2D)");
+                return ST_HIP_OK;
+            }
+            stages_.push_back(stage);
+            for (size_t at = 0; at < bytes; at += kPiece) {
+                const size_t piece = std::min(kPiece, bytes - at);
+                unsigned char *const pinned = static_cast<unsigned char *>(stage.ptr) + at;
+                std::memcpy(pinned, static_cast<const unsigned char *>(host) + at, piece);
+                ST_HIP_TRY(launch_copy_from_pinned(static_cast<unsigned char *>(*device) + at, pinned, piece, ws_->stream), "copy launch");
+            }
         }
         return ST_HIP_OK;
     }
@@ -112,8 +130,34 @@ class Lease {
     {
         if (bytes) {
             count_transfer(false, bytes);
-            ST_HIP_TRY(hipMemcpyAsync(host, device, bytes, hipMemcpyDeviceToHost, ws_->stream),
-                       "hipMemcpyAsync(D2H)");
+            const size_t pieces = (bytes + kCopyPiece - 1) / kCopyPiece, flags = (bytes + 63) / 64 * 64;
+            PinnedBuffer stage;
+            if (bytes > kStageMost || is_pinned(host) || !pinned_acquire(flags + pieces * sizeof(unsigned), &stage)) {
+                ST_HIP_TRY(hipMemcpyAsync(host, device, bytes, hipMemcpyDeviceToHost, ws_->stream),
+                           "hipMemcpyAsync(D2H)");
+            } else {
+                stages_.push_back(stage);
+                unsigned char *const pinned = static_cast<unsigned char *>(stage.ptr);
+                unsigned *const arrived = reinterpret_cast<unsigned *>(pinned + flags);
+                std::memset(arrived, 0, pieces * sizeof(unsigned));
+                drained_ = false;
+                ST_HIP_TRY(launch_copy_to_pinned(pinned, device, bytes, arrived, ws_->stream), "copy launch");
+                // Pieces are taken as they arrive.  Where none does for a while the stream is waited for, which also reports
+                // what went wrong on it.
+                auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
+                for (size_t p = 0; p < pieces;) {
+                    if (__atomic_load_n(&arrived[p], __ATOMIC_ACQUIRE) != 0) {
+                        const size_t at = p * kCopyPiece;
+                        std::memcpy(static_cast<unsigned char *>(host) + at, pinned + at, std::min(kCopyPiece, bytes - at));
+                        ++p;
+                    } else if (std::chrono::steady_clock::now() > until) {
+                        ST_HIP_TRY(hipStreamSynchronize(ws_->stream), "hipStreamSynchronize");
+                        if (__atomic_load_n(&arrived[p], __ATOMIC_ACQUIRE) == 0) return fail(ST_HIP_ERR_RUNTIME, "a copy to the host did not arrive");
+                    }
+                }
+                drained_ = true;  // the last kernel of the stream has said so
+                return ST_HIP_OK;
+            }
         }
         ST_HIP_TRY(hipStreamSynchronize(ws_->stream), "hipStreamSynchronize");
         return ST_HIP_OK;
@@ -121,6 +165,8 @@ class Lease {
 
   private:
     Workspace *ws_ = nullptr;
+    std::vector<PinnedBuffer> stages_;  // in use until the stream has drained
+    bool drained_ = false;              // nothing is left on the stream
     int status_ = ST_HIP_OK;
 };
 
@@ -1088,20 +1134,43 @@ int st_hip_count_nonfinite_f32_dev(size_t count, const float *data, uint64_t *no
     if (count == 0) return ST_HIP_OK;
     if (!data) return fail(ST_HIP_ERR_INVALID, "count_nonfinite received a null pointer");
     hipStream_t s = as_stream(stream);
-    void *workspace = nullptr;
-    ST_HIP_TRY(stream_workspace(s, 16, &workspace), "hipMalloc");
-    unsigned long long *status = static_cast<unsigned long long *>(workspace);
-    const unsigned long long init[2] = {0ull, ~0ull};
-    ST_HIP_TRY(hipMemcpyAsync(status, init, sizeof init, hipMemcpyHostToDevice, s), "hipMemcpyAsync(H2D)");
-    ST_HIP_CHECK(launch_status(launch_nonfinite_probe_f32(count, data, status, s), "count_nonfinite launch"));
-    unsigned long long result[2] = {0, 0};
-    ST_HIP_TRY(hipMemcpyAsync(result, status, sizeof result, hipMemcpyDeviceToHost, s), "hipMemcpyAsync(D2H)");
-    ST_HIP_TRY(hipStreamSynchronize(s), "hipStreamSynchronize");
-    *nonfinite = result[0];
-    if (result[0] != 0) {
-        if (first_index) *first_index = result[1];
+    const size_t groups = nonfinite_probe_groups(count);
+    PinnedBuffer memory;
+    if (!pinned_acquire(groups * 2 * sizeof(uint64_t), &memory)) return hip_fail(hipErrorOutOfMemory, "hipHostMalloc");
+    unsigned long long *const slots = static_cast<unsigned long long *>(memory.ptr);
+    std::memset(slots, 0, groups * 2 * sizeof(uint64_t));
+    hipError_t rc = launch_nonfinite_probe_f32(count, data, slots, s);
+    // The words are watched for a while (6 µs from the launch, where waiting for the stream takes 11 and a copy behind the kernel
+    // 20), then the stream is waited for, which also reports what went wrong on it.
+    auto arrived = [&](size_t i) { return (__atomic_load_n(&slots[i], __ATOMIC_ACQUIRE) >> 63) != 0; };
+    size_t seen = 0;
+    if (rc == hipSuccess) {
+        const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+        while (seen < 2 * groups) {
+            if (arrived(seen)) ++seen;
+            else if (std::chrono::steady_clock::now() > until) break;
+        }
+    }
+    if (seen < 2 * groups) {
+        const hipError_t drained = hipStreamSynchronize(s);
+        if (rc == hipSuccess) rc = drained;
+        while (rc == hipSuccess && seen < 2 * groups) {
+            if (!arrived(seen)) rc = hipErrorUnknown;
+            ++seen;
+        }
+    }
+    uint64_t found = 0, first = ~0ull >> 1;
+    for (size_t g = 0; rc == hipSuccess && g < groups; ++g) {
+        found += slots[2 * g] & (~0ull >> 1);
+        first = std::min<uint64_t>(first, slots[2 * g + 1] & (~0ull >> 1));
+    }
+    pinned_release(memory);
+    if (rc != hipSuccess) return hip_fail(rc, "count_nonfinite launch");
+    *nonfinite = found;
+    if (found != 0) {
+        if (first_index) *first_index = first;
         if (first_value) {
-            ST_HIP_TRY(hipMemcpyAsync(first_value, data + result[1], sizeof(float), hipMemcpyDeviceToHost, s), "hipMemcpyAsync(D2H)");
+            ST_HIP_TRY(hipMemcpyAsync(first_value, data + first, sizeof(float), hipMemcpyDeviceToHost, s), "hipMemcpyAsync(D2H)");
             ST_HIP_TRY(hipStreamSynchronize(s), "hipStreamSynchronize");
         }
     }

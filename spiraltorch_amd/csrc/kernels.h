@@ -203,8 +203,10 @@ hipError_t launch_merge_heads_f32(size_t batch, size_t seq, size_t heads, size_t
 // Element-wise and row-wise tensor utilities (all f32, row-major).
 hipError_t launch_row_softmax_f32(size_t rows, size_t cols, const float *in, float *out, hipStream_t stream);
 hipError_t launch_gelu_f32(size_t count, const float *in, float *out, hipStream_t stream);
-// status[0] += number of non-finite values of data, status[1] = min(status[1], index of one).
-hipError_t launch_nonfinite_probe_f32(size_t count, const float *data, unsigned long long *status, hipStream_t stream);
+// Workgroup g of the probe's nonfinite_probe_groups(count) writes slots[2g] = 2^63 + the number of non-finite values among its
+// own and slots[2g + 1] = 2^63 + the smallest index of one (2^63 - 1 + 2^63 if none): host memory the GPU can write, cleared before.
+size_t nonfinite_probe_groups(size_t count);
+hipError_t launch_nonfinite_probe_f32(size_t count, const float *data, unsigned long long *slots, hipStream_t stream);
 hipError_t launch_gelu_backward_f32(size_t count, const float *z, const float *grad, float *out, hipStream_t stream);
 hipError_t launch_scale_f32(size_t count, const float *in, float scale, float *out, hipStream_t stream);
 hipError_t launch_add_row_f32(size_t rows, size_t cols, float *data, const float *bias, hipStream_t stream);
@@ -229,6 +231,24 @@ hipError_t stream_workspace_slot(hipStream_t stream, int slot, size_t bytes, voi
 inline bool scratch_unavailable(hipError_t rc) { return rc == hipErrorOutOfMemory || rc == hipErrorStreamCaptureUnsupported; }
 void release_stream_workspace(hipStream_t stream);
 size_t stream_workspace_entry_count();
+// Pinned host memory for a call's copies and results, from a pool that keeps up to kPinnedIdleBytes between calls and is safe with
+// several threads; false where the host has none to give (the caller then copies without it).  A buffer is handed back when
+// nothing on the GPU uses it any more.
+struct PinnedBuffer {
+    void *ptr = nullptr;
+    size_t capacity = 0;
+};
+constexpr size_t kPinnedIdleBytes = 64u << 20;
+bool pinned_acquire(size_t bytes, PinnedBuffer *out);
+void pinned_release(const PinnedBuffer &buffer);
+bool is_pinned(const void *host);
+// The most a copy goes through pinned memory with.
+constexpr size_t kStageMost = 16u << 20;
+// device[0, bytes) = pinned[0, bytes) by a kernel (device on a 16-byte boundary), and back: the piece of kCopyPiece bytes with
+// number p is in host memory when word p of `arrived` (host memory, cleared before) is not zero.
+constexpr size_t kCopyPiece = 16u << 10;
+hipError_t launch_copy_from_pinned(void *device, const void *pinned, size_t bytes, hipStream_t stream);
+hipError_t launch_copy_to_pinned(void *pinned, const void *device, size_t bytes, unsigned *arrived, hipStream_t stream);
 // Host<->device copies made by the library, for tests that check where tensors live.
 void count_transfer(bool to_device, size_t bytes);
 

@@ -1,5 +1,7 @@
 // Row-wise, HBM-bound helpers of the decoder stack: layer-norm, embedding gather, f32->bf16 rounding
 // and the (tokens, heads*dim) <-> (contexts*seq, dim) re-layouts around attention.
+#include <algorithm>
+
 #include "device_math.h"
 #include "kernels.h"
 
@@ -799,22 +801,80 @@ __global__ __launch_bounds__(256) void gelu_forward_vec_kernel(size_t count4, co
     }
 }
 
-// status[0] = number of non-finite values, status[1] = smallest index of one (status[1] must start at ~0).
-// The first workgroup resets nothing: the caller clears the two words before the launch.
-__global__ __launch_bounds__(256) void nonfinite_probe_kernel(size_t count, const float *data, unsigned long long *status)
+// The number of non-finite values and the smallest index of one, by workgroup, written where the host waits for them: every word
+// carries bit 63, so that one that has arrived is known by itself, and nothing is copied, cleared or added up on the GPU.
+__global__ __launch_bounds__(256) void nonfinite_probe_kernel(size_t count, const float *data, unsigned long long *slots)
 {
-    const size_t stride = static_cast<size_t>(gridDim.x) * 256;
-    unsigned long long found = 0, first = ~0ull;
-    for (size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x; i < count; i += stride) {
-        if (!isfinite(data[i])) {
-            ++found;
-            if (i < first) first = i;
-        }
+    __shared__ unsigned long long counts[4], firsts[4];
+    typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+    const unsigned long long kNone = ~0ull >> 1, kArrived = 1ull << 63;
+    const size_t quads = count / 4, stride = static_cast<size_t>(gridDim.x) * 256;
+    unsigned long long found = 0, first = kNone;
+    auto look = [&](float v, size_t i) {
+        if (isfinite(v)) return;
+        ++found;
+        if (i < first) first = i;
+    };
+    for (size_t q = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x; q < quads; q += stride) {
+        const f32x4_a4 v = *reinterpret_cast<const f32x4_a4 *>(data + q * 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) look(v[e], q * 4 + e);
     }
-    if (found) {
-        atomicAdd(&status[0], found);
-        atomicMin(&status[1], first);
+    if (blockIdx.x == 0 && threadIdx.x < count - quads * 4) look(data[quads * 4 + threadIdx.x], quads * 4 + threadIdx.x);
+#pragma unroll
+    for (int offset = 32; offset > 0; offset >>= 1) {
+        found += __shfl_xor(found, offset);
+        first = min(first, static_cast<unsigned long long>(__shfl_xor(first, offset)));
     }
+    if ((threadIdx.x & 63) == 0) {
+        counts[threadIdx.x >> 6] = found;
+        firsts[threadIdx.x >> 6] = first;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    found = counts[0] + counts[1] + counts[2] + counts[3];
+    first = min(min(firsts[0], firsts[1]), min(firsts[2], firsts[3]));
+    __hip_atomic_store(&slots[2 * blockIdx.x], found | kArrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&slots[2 * blockIdx.x + 1], first | kArrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// A workgroup a piece of kCopyPiece bytes, 16 bytes a lane and four in flight; the last bytes one by one.
+__global__ __launch_bounds__(256) void copy_from_pinned_kernel(size_t bytes, const unsigned char *pinned, unsigned char *device)
+{
+    const size_t base = static_cast<size_t>(blockIdx.x) * kCopyPiece + threadIdx.x * 16;
+    uint4 v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (base + i * 4096 + 16 <= bytes) v[i] = *reinterpret_cast<const uint4 *>(pinned + base + i * 4096);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const size_t at = base + i * 4096;
+        if (at + 16 <= bytes) *reinterpret_cast<uint4 *>(device + at) = v[i];
+        else
+            for (size_t e = at; e < bytes; ++e) device[e] = pinned[e];
+    }
+}
+
+// The other way.  The stores go to host memory past the caches (system scope); each wavefront waits for its own to be
+// acknowledged before the workgroup's word says that the piece is there.
+__global__ __launch_bounds__(256) void copy_to_pinned_kernel(size_t bytes, const unsigned char *device, unsigned char *pinned, unsigned *arrived)
+{
+    const size_t base = static_cast<size_t>(blockIdx.x) * kCopyPiece + threadIdx.x * 8;
+    unsigned long long v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        if (base + i * 2048 + 8 <= bytes) v[i] = *reinterpret_cast<const unsigned long long *>(device + base + i * 2048);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const size_t at = base + i * 2048;
+        if (at + 8 <= bytes)
+            __hip_atomic_store(reinterpret_cast<unsigned long long *>(pinned + at), v[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        else
+            for (size_t e = at; e < bytes; ++e) __hip_atomic_store(pinned + e, device[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(&arrived[blockIdx.x], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // gelu_prime(z)·g, crates/st-tensor/src/pure.rs:12033-12040 and :6549-6552.
@@ -1238,9 +1298,26 @@ hipError_t launch_gelu_f32(size_t count, const float *in, float *out, hipStream_
     return hipGetLastError();
 }
 
-hipError_t launch_nonfinite_probe_f32(size_t count, const float *data, unsigned long long *status, hipStream_t stream)
+size_t nonfinite_probe_groups(size_t count) { return std::min<size_t>(std::max<size_t>((count + 2047) / 2048, 1), 512); }
+
+hipError_t launch_nonfinite_probe_f32(size_t count, const float *data, unsigned long long *slots, hipStream_t stream)
 {
-    hipLaunchKernelGGL(nonfinite_probe_kernel, dim3(count ? grid_for(count) : 1), dim3(256), 0, stream, count, data, status);
+    hipLaunchKernelGGL(nonfinite_probe_kernel, dim3(static_cast<unsigned>(nonfinite_probe_groups(count))), dim3(256), 0, stream, count, data,
+                       slots);
+    return hipGetLastError();
+}
+
+hipError_t launch_copy_from_pinned(void *device, const void *pinned, size_t bytes, hipStream_t stream)
+{
+    hipLaunchKernelGGL(copy_from_pinned_kernel, dim3(static_cast<unsigned>((bytes + kCopyPiece - 1) / kCopyPiece)), dim3(256), 0, stream, bytes,
+                       static_cast<const unsigned char *>(pinned), static_cast<unsigned char *>(device));
+    return hipGetLastError();
+}
+
+hipError_t launch_copy_to_pinned(void *pinned, const void *device, size_t bytes, unsigned *arrived, hipStream_t stream)
+{
+    hipLaunchKernelGGL(copy_to_pinned_kernel, dim3(static_cast<unsigned>((bytes + kCopyPiece - 1) / kCopyPiece)), dim3(256), 0, stream, bytes,
+                       static_cast<const unsigned char *>(device), static_cast<unsigned char *>(pinned), arrived);
     return hipGetLastError();
 }
 

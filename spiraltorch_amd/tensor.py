@@ -195,9 +195,10 @@ class Tensor:
         remembered, so an operator's validated result is not examined again when it feeds the next operator."""
         if self._finite is None:
             if self._host is not None:
-                bad = self._host[~np.isfinite(self._host)]
-                self._finite = bad.size == 0
+                finite = np.isfinite(self._host)
+                self._finite = bool(finite.all())
                 if not self._finite:
+                    bad = self._host[~finite]
                     raise TensorError("NonFiniteValue", f"non-finite value encountered in {label}: {bad[0]}", label=label)
             else:
                 self._validate_result(label)

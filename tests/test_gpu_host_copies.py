@@ -1,0 +1,84 @@
+"""What the host-slice calls move through pinned memory, and the finite check's words: every byte, at the edges of pieces, from
+several threads at once."""
+import ctypes
+import threading
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def outer(hip, column, row):
+    """column · row as a host-slice product of one term: exact, every operand and result byte moved."""
+    out = np.full(column.size * row.size, 7.5, np.float32)
+    hip.gemm_f32(column.size, row.size, 1, column, row, out)
+    return out.reshape(column.size, row.size)
+
+
+# around a 16 KiB piece of the result, a 256 KiB piece of an operand, and what is no multiple of sixteen bytes
+@pytest.mark.parametrize("m,n", [(1, 1), (3, 1), (1, 4095), (1, 4096), (1, 4097), (5, 819), (65536, 1), (65537, 1), (70001, 1), (131, 1021),
+                                 (1024, 1024), (2049, 2051)])
+def test_every_byte_arrives(hip, m, n):
+    rng = np.random.default_rng(m + n)
+    column, row = rng.integers(-999, 999, m).astype(np.float32), rng.integers(-999, 999, n).astype(np.float32)
+    assert (outer(hip, column, row) == column[:, None] * row[None, :]).all()
+
+
+def test_pinned_operands_and_results(hip):
+    """Host memory that is pinned already is copied from and to directly."""
+    runtime = ctypes.CDLL("libamdhip64.so.7")  # the one the library is linked with
+    m, n = 600, 700
+    rng = np.random.default_rng(1)
+    blocks, arrays = [], []
+    for size in (m, n, m * n):
+        block = ctypes.c_void_p()
+        assert runtime.hipHostMalloc(ctypes.byref(block), ctypes.c_size_t(size * 4), ctypes.c_uint(0)) == 0
+        blocks.append(block)
+        arrays.append(np.ctypeslib.as_array(ctypes.cast(block, ctypes.POINTER(ctypes.c_float)), (size,)))
+    arrays[0][:], arrays[1][:] = rng.integers(-99, 99, m), rng.integers(-99, 99, n)
+    hip.gemm_f32(m, n, 1, *arrays)
+    assert (arrays[2].reshape(m, n) == arrays[0][:, None] * arrays[1][None, :]).all()
+    del arrays
+    for block in blocks:
+        assert runtime.hipHostFree(block) == 0
+
+
+def test_calls_from_several_threads_keep_their_bytes(hip):
+    wrong = []
+
+    def work(seed):
+        rng = np.random.default_rng(seed)
+        for _ in range(20):
+            m, n = int(rng.integers(1, 700)), int(rng.integers(1, 700))
+            column, row = rng.integers(-999, 999, m).astype(np.float32), rng.integers(-999, 999, n).astype(np.float32)
+            if not (outer(hip, column, row) == column[:, None] * row[None, :]).all():
+                wrong.append((seed, m, n))
+            data = rng.normal(size=m * n).astype(np.float32)
+            data[m * n // 2] = np.nan
+            d_data = hip.DeviceBuffer.from_array(data)
+            if hip.count_nonfinite_f32_dev(m * n, d_data)[:2] != (1, m * n // 2):
+                wrong.append((seed, m, n, "count"))
+
+    threads = [threading.Thread(target=work, args=(seed,)) for seed in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert wrong == []
+
+
+@pytest.mark.parametrize("count", [1, 3, 4, 5, 255, 2047, 2048, 2049, 8193, (1 << 20) + 3, 512 * 2048 * 3 + 1])
+def test_count_nonfinite(hip, count):
+    """Counts and first indices at both ends, at any alignment, with infinities and NaN."""
+    data = np.ones(count + 1, np.float32)
+    d = hip.DeviceBuffer.from_array(data)
+    for shift in (0, 1):
+        assert hip.count_nonfinite_f32_dev(count, d.at(4 * shift)) == (0, 0, 0.0)
+    for places in ({0}, {count - 1}, {0, count // 2, count - 1}):  # (fewer where they coincide)
+        bad = data.copy()
+        for i, place in enumerate(sorted(places)):
+            bad[1 + place] = (np.inf, -np.inf, np.nan)[i]
+        d_bad = hip.DeviceBuffer.from_array(bad)
+        found, first, value = hip.count_nonfinite_f32_dev(count, d_bad.at(4))
+        assert (found, first) == (len(places), min(places)) and value == np.inf
