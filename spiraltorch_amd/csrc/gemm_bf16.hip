@@ -33,6 +33,7 @@ struct GemmBf16Args {
     const float *residual;
     int M, N, K;
     int tiles_m, tiles_n;
+    int first_col = 0, columns = 0;  // a launch of whole tiles that covers only `columns` of C's columns, from first_col on (0: all)
     int swizzle;  // 1: remap workgroup ids so each XCD (id % 8) works on a compact block of tiles
     float scale;
     int activation;
@@ -596,7 +597,7 @@ __device__ __forceinline__ void gemm_bf16_packed_body(const GemmBf16Args &p)
     const int group_size = min(p.tiles_m - first_m, GROUP_M);
     const int tile_m = first_m + (logical % width) % group_size;
     const int tile_n = (logical % width) / group_size;
-    const int m0 = tile_m * BM, n0 = tile_n * BN;
+    const int m0 = tile_m * BM, n0 = p.first_col + tile_n * BN;
     const int tile0 = split * p.tiles_per_split;  // first k-tile of this workgroup
 
     const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(
@@ -1035,7 +1036,7 @@ __device__ __forceinline__ void gemm_bf16_rowmajor_body(const GemmBf16Args &p)
     const int group_size = min(p.tiles_m - first_m, GROUP_M);
     const int tile_m = first_m + (logical % width) % group_size;
     const int tile_n = (logical % width) / group_size;
-    const int m0 = tile_m * BM, n0 = tile_n * BN;
+    const int m0 = tile_m * BM, n0 = p.first_col + tile_n * BN;
     const int tile0 = split * p.tiles_per_split;  // first k-tile of this workgroup
 
     const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(
@@ -2156,7 +2157,9 @@ bool tile_launch_consistent(const GemmBf16Args &a, size_t grid, int bm, int bn)
     const size_t tiles = static_cast<size_t>(a.tiles_m) * static_cast<size_t>(a.tiles_n), k_tiles = static_cast<size_t>(a.K) / 64;
     if (grid == 0 || grid > 0x7fffffffu || a.k_splits < 1 || grid != tiles * static_cast<size_t>(a.k_splits)) return false;
     if (static_cast<size_t>(a.tiles_m) * bm < static_cast<size_t>(a.M) || static_cast<size_t>(a.tiles_m - 1) * bm >= static_cast<size_t>(a.M)) return false;
-    if (static_cast<size_t>(a.tiles_n) * bn < static_cast<size_t>(a.N) || static_cast<size_t>(a.tiles_n - 1) * bn >= static_cast<size_t>(a.N)) return false;
+    const size_t col = static_cast<size_t>(a.first_col), last_col = a.columns ? col + a.columns : static_cast<size_t>(a.N);
+    if (a.first_col < 0 || last_col > static_cast<size_t>(a.N) || last_col <= col) return false;
+    if (col + static_cast<size_t>(a.tiles_n) * bn < last_col || col + static_cast<size_t>(a.tiles_n - 1) * bn >= last_col) return false;
     if (a.k_splits > 1) {
         const size_t per = static_cast<size_t>(a.tiles_per_split);
         if (a.tiles_per_split < 1 || a.partial == nullptr) return false;
@@ -2169,10 +2172,10 @@ bool tile_launch_consistent(const GemmBf16Args &a, size_t grid, int bm, int bn)
 size_t plan_256(GemmBf16Args &args, int bn)
 {
     args.tiles_m = (args.M + 255) / 256;
-    args.tiles_n = (args.N + bn - 1) / bn;  // the packed kernels take a ragged N: rows of Bᵀ past it read as zero
+    args.tiles_n = ((args.columns ? args.columns : args.N) + bn - 1) / bn;  // the packed kernels take a ragged N: rows of Bᵀ past it read as zero
     size_t tiles = static_cast<size_t>(args.tiles_m) * static_cast<size_t>(args.tiles_n);
     const size_t k_tiles = static_cast<size_t>(args.K) / 64;
-    const size_t splits = choose_k_splits(args.M, args.N, args.K, tiles);
+    const size_t splits = args.columns ? 1 : choose_k_splits(args.M, args.N, args.K, tiles);
     args.k_splits = 1;
     if (splits > 1) {
         args.tiles_per_split = static_cast<int>((k_tiles + splits - 1) / splits);
@@ -2227,7 +2230,7 @@ hipError_t launch_256(GemmBf16Args args, bool packed, hipStream_t stream, size_t
 hipError_t launch_128(GemmBf16Args args, bool packed, hipStream_t stream, size_t splits = 1, size_t workspace_offset = 0)
 {
     args.tiles_m = (args.M + 127) / 128;
-    args.tiles_n = (args.N + 127) / 128;
+    args.tiles_n = ((args.columns ? args.columns : args.N) + 127) / 128;
     size_t tiles = static_cast<size_t>(args.tiles_m) * static_cast<size_t>(args.tiles_n);
     if (tiles > 0x7fffffffu) return hipErrorInvalidConfiguration;
     SkinnyArgs reduce{};
@@ -2268,6 +2271,25 @@ hipError_t launch_128(GemmBf16Args args, bool packed, hipStream_t stream, size_t
     hipLaunchKernelGGL(gemm_bf16_skinny_reduce_kernel, dim3(static_cast<unsigned>((plane + 255) / 256)), dim3(256), 0, stream,
                        reduce);
     return hipGetLastError();
+}
+
+// 256×256 tiles in rounds of 256.  A last round for a few of the compute units (1024×50257 is 788 tiles, three rounds and 20)
+// takes as long as a full one: where the columns behind the full rounds are at most 256 tiles of 128×128, those run them, two
+// workgroups a unit, in a launch of their own.  Same sums in the same order.  1024×50257×768: 154 -> 131 µs, 1500×33333×384
+// 112 -> 96.
+hipError_t launch_256_rounds(GemmBf16Args args, bool packed, const TilePlan &plan, hipStream_t stream, size_t workspace_offset)
+{
+    const size_t m = static_cast<size_t>(args.M), n = static_cast<size_t>(args.N), row_tiles = (m + 255) / 256;
+    const size_t whole = plan.tiles / 256 * 256 / row_tiles * 256;  // columns of the full rounds
+    if (plan.k_splits == 1 && plan.tiles > 256 && whole > 0 && whole < n && (m + 127) / 128 * ((n - whole + 127) / 128) <= 256) {
+        GemmBf16Args rest = args;
+        args.columns = static_cast<int>(whole);
+        rest.first_col = static_cast<int>(whole);
+        rest.columns = static_cast<int>(n - whole);
+        const hipError_t rc = launch_256<256>(args, packed, stream, workspace_offset);
+        return rc == hipSuccess ? launch_128(rest, packed, stream) : rc;
+    }
+    return launch_256<256>(args, packed, stream, workspace_offset);
 }
 
 // The persistent kernel: one workgroup per compute unit (fewer when there are fewer tiles), twelve wavefronts each.
@@ -2552,7 +2574,7 @@ hipError_t launch_gemm_bf16(size_t m, size_t n, size_t k, const uint16_t *lhs, c
         const size_t tiles_128 = ((m + 127) / 128) * ((n + 127) / 128);
         if (plan.tiles < 192 && tiles_128 >= 2 * plan.tiles && plan.k_splits == 1) return launch_128(args, true, stream);
         if (plan.narrow) return launch_256<128>(args, true, stream, workspace_offset);
-        return launch_256<256>(args, true, stream, workspace_offset);
+        return launch_256_rounds(args, true, plan, stream, workspace_offset);
     }
     if (rhs_packed && (!fits_256 || skinny) && k > 0) {
         // Shapes the packed 256-row kernels do not take: unpack B into the front of the stream's workspace (sized for
@@ -2600,7 +2622,7 @@ hipError_t launch_gemm_bf16(size_t m, size_t n, size_t k, const uint16_t *lhs, c
             k <= 512 && (m / 256) * (n / 128) >= 1024 && m * n * 4 < (1ull << 32))
             return launch_persistent_256x128(args, stream);
         if (narrow) return launch_256<128>(args, rhs_packed, stream, workspace_offset);
-        return launch_256<256>(args, rhs_packed, stream, workspace_offset);
+        return launch_256_rounds(args, rhs_packed, plan, stream, workspace_offset);
     }
     return launch_tile<128, 128, 32>(args, vec, stream, workspace_offset);
 }

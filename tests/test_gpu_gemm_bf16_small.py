@@ -62,3 +62,34 @@ def test_small_tiles_of_non_finite_operands(hip):
     got = out.to_array(np.float32, m * n).reshape(m, n)
     assert np.isinf(got[7]).all() and np.isnan(got[44]).all()
     assert np.isfinite(np.delete(got, (7, 44), axis=0)).all()
+
+
+@pytest.mark.parametrize("m,n,k,layouts", [
+    (1024, 16600, 64, "p"), (1024, 16641, 192, "pr"),  # 260 and 264 tiles of 256×256; columns off every boundary
+    (1000, 16640, 128, "pr"), (2049, 8064, 64, "pr"),  # a multiple of 128; ragged rows
+    (300, 33024, 64, "p"),                             # 258 tiles: one column of tiles behind the full round
+])
+def test_columns_behind_the_full_rounds(hip, m, n, k, layouts):
+    """A last round of a few 256×256 tiles runs as 128×128 tiles in a launch of its own: every column against float64 (the bound
+    as above), and the columns of the first round bit for bit what a product of those alone gives."""
+    from spiraltorch_amd import inputs
+    rng = np.random.default_rng(m + n + k)
+    a, b = inputs.to_bf16(rng.normal(size=m * k).astype(np.float32)), inputs.to_bf16(rng.normal(size=n * k).astype(np.float32))
+    bias = rng.normal(size=n).astype(np.float32)
+    a64, b64 = inputs.from_bf16(a).reshape(m, k).astype(np.float64), inputs.from_bf16(b).reshape(n, k).astype(np.float64)
+    want, bound = a64 @ b64.T + bias, k * 2.0 ** -24 * (np.abs(a64) @ np.abs(b64).T + np.abs(bias))
+    d_a, d_bias, d_p = hip.DeviceBuffer.from_array(a), hip.DeviceBuffer.from_array(bias), hip.DeviceBuffer.from_array(b)
+    d_r = hip.DeviceBuffer.from_array(np.ascontiguousarray(b.reshape(n, k).T))
+    d32, d16 = hip.DeviceBuffer((m * n + 64) * 4), hip.DeviceBuffer(m * n * 2)
+    bits = []
+    for layout in layouts:
+        d32.zero()
+        call, operand = (hip.gemm_bf16_prepacked_bias_act_dev, d_p) if layout == "p" else (hip.gemm_bf16_bias_act_dev, d_r)
+        call(m, n, k, 0, d_a, operand, d_bias, None, d32, d16)
+        hip.device_synchronize()
+        got = d32.to_array(np.float32, m * n + 64)
+        assert (got[m * n:] == 0).all()
+        bits.append(got[:m * n].reshape(m, n))
+        assert (np.abs(bits[-1] - want) <= bound).all(), layout
+        assert (d16.to_array(np.uint16, m * n) == inputs.to_bf16(got[:m * n])).all()
+    assert all((x == bits[0]).all() for x in bits)
