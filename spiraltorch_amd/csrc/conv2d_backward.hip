@@ -15,6 +15,7 @@
 //   * grad_bias is a per-channel sum over NCHW planes.
 #include "device_math.h"
 #include "kernels.h"
+#include "split_product.h"
 
 #include <algorithm>
 #include <cmath>
@@ -230,18 +231,33 @@ struct GradWeightArgs {
 };
 
 // One workgroup: a (64·TM output channels) × (64·TN reduction columns s) tile of grad_weight, summed over the pixels
-// of its images; four wavefronts in a 2×2 arrangement, each owning TM×TN 32×32 accumulators.  Per 16-pixel step the G
-// tile (pixel-contiguous in NCHW) and the patch tile (gathered: a thread owns TN columns s, whose channel/tap offsets
-// are fixed for the whole kernel) are fetched into registers while the MFMAs of the previous step run, then written to
-// the other LDS stage.  The big tile (TM = 2, TN = 3: 128 × 192, three of which span a 3×3 layer's 576 columns exactly
-// for 64 input channels) reads 5 fragments per 24 MFMAs instead of 2 per 4.
+// of its images; four wavefronts in a 2×2 arrangement, each owning TM×TN 32×32 accumulators.  The f32 operands are held as
+// three exact bf16 pieces (split_product.h), cut here: per 16-pixel step the G tile (pixel-contiguous in NCHW) and the patch
+// tile (gathered: a thread owns TN columns s, whose channel/tap offsets are fixed for the whole kernel) are fetched into
+// registers two steps ahead, and cut and written to the other LDS stage among the matrix instructions of the step before.
 //
-// SETS > 1: the workgroup is SETS such groups of four wavefronts working on the same tile.  Each takes its own run of
-// steps (chunk·SETS + set) through LDS stages of its own; at the end the sets' accumulators are added through LDS in
-// the order ((0 + 1) + 2) and set 0 stores the one partial tile — a third of the partial tiles, of the bytes the
-// chunk reduction reads back, and of the store burst at the end of the launch, for the same wavefronts per SIMD.
-template <bool VEC, int TM, int TN, int SETS = 1>
-__device__ __forceinline__ void conv_grad_weight_body(const GradWeightArgs &p, float *As, float *Bs)
+// On the f32 matrix instruction the step was bound by it (94 of 150 µs for 32 images, 64 -> 128 channels, 56×56, 3×3); the six
+// piece products take 36 µs, and the kernel now 104: one wavefront a SIMD, whose 36 matrix instructions a step cover the 190
+// vector instructions of cutting and addressing (written into their gaps: 2.2 instead of 2.7 thousand cycles), and which then
+// waits for its first LDS reads behind the barrier.  The whole call, two launches, old / new µs (and the error against float64,
+// 3.6e-7 / 2.1e-7 and the like): that layer 158 / 113, 128 -> 128 at 28×28 90 / 63, 256 -> 256 at 14×14 176 / 75, 512 -> 512 at
+// 7×7 235 / 106, 8 × 64 -> 64 at 56×56 (the small tile) 39.5 / 31, 4 × 24 -> 96 at 28×28 20 / 14.4, 14 × 64 -> 16 at 46×47 41 / 35.
+//
+// The big tile (TM = 2, TN = 3: 128 × 192, three of which span a 3×3 layer's 576 columns exactly for 64 input channels)
+// cuts 20 values a thread for 36 matrix instructions of a wavefront, 8 for 6 in the small one.
+template <int TM, int TN>
+constexpr int kGradWeightStages = 2 * 3 * (64 * (TM + TN) * 32 + 256);  // two stages of three pieces (or of f32 rows)
+
+// How a thread gets its four pixels of a row or column: one 16-byte load of the window under them (buffer loads need four-byte
+// alignment only), or four loads.
+enum class Gather {
+    kValues,   // G and patches value by value: a G below four values an image
+    kTaps,     // patches value by value
+    kWindows,  // patches by windows: no stride and rows that are a multiple of four pixels
+};
+
+template <Gather GATHER, int TM, int TN>
+__device__ __forceinline__ void conv_grad_weight_body(const GradWeightArgs &p, unsigned char *lds)
 {
     constexpr int BM = 64 * TM, BN = 64 * TN, BK = 16;
     // Both tiles are kept pixel-contiguous (row = channel or patch column, 16 pixels + 4 words of padding), so that a
@@ -249,13 +265,17 @@ __device__ __forceinline__ void conv_grad_weight_body(const GradWeightArgs &p, f
     constexpr int A_STRIDE = BK + 4, B_STRIDE = BK + 4;
     constexpr int A_STAGE = BM * A_STRIDE, B_STAGE = BN * B_STRIDE;
 
-    const int set = SETS > 1 ? __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 8)) : 0;
-    float *const lds_all = As;  // (SETS > 1: As is the start of the workgroup's LDS, [set][A stages | B stages])
-    if constexpr (SETS > 1) {
-        As = lds_all + set * (2 * A_STAGE + 2 * B_STAGE);
-        Bs = As + 2 * A_STAGE;
-    }
-    const int tid = threadIdx.x & 255;
+    // A stage as pieces: [piece][half][row][8 pixels]: a lane's operand is sixteen bytes, those of 32 rows side by side.  (32 bytes
+    // a row cost four cycles of bank conflicts a read and twelve a write of the gathered columns.)  The 64 bytes between the halves
+    // keep the two that a quad of lanes of the G tile writes on different banks.
+    constexpr int A_HALF = BM * 16 + 64, B_HALF = BN * 16 + 64;
+    constexpr int A_PIECE = 2 * A_HALF, B_PIECE = 2 * B_HALF, PIECES_STAGE = 3 * (A_PIECE + B_PIECE);
+    constexpr int STAGES_BYTES = kGradWeightStages<TM, TN>;
+    static_assert(2 * PIECES_STAGE <= STAGES_BYTES && (2 * A_STAGE + 2 * B_STAGE) * 4 <= STAGES_BYTES, "two stages of either kind");
+    __shared__ int beyond;
+
+    float *const As = reinterpret_cast<float *>(lds), *const Bs = As + 2 * A_STAGE;
+    const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // scalar: the pixel bookkeeping below stays off the VALU
     const int wm = wave >> 1, wn = wave & 1;
@@ -272,7 +292,7 @@ __device__ __forceinline__ void conv_grad_weight_body(const GradWeightArgs &p, f
     bid /= p.tiles_s;
     const int tiles_oc = (s.c_out + BM - 1) / BM;
     const int tile_oc = bid % tiles_oc;
-    const int chunk = (bid / tiles_oc) * SETS + set;
+    const int chunk = bid / tiles_oc;
     const int oc0 = tile_oc * BM, s0 = tile_s * BN;
 
     // This thread's patch columns (lane + 64·j) and their fixed taps.
@@ -288,21 +308,16 @@ __device__ __forceinline__ void conv_grad_weight_body(const GradWeightArgs &p, f
         const int ky = rem / s.kw, kx = rem - ky * s.kw;
         dy[j] = ky * s.dil_h - s.pad_h;
         dx[j] = kx * s.dil_w - s.pad_w;
-        tap_offset[j] = ic * H * W;
+        tap_offset[j] = GATHER == Gather::kWindows ? ic * H * W + dy[j] * W + dx[j] : ic * H * W;
+        if (GATHER == Gather::kWindows && !col_valid[j]) dy[j] = -(1 << 30);  // no row of the image
     }
     const int prow0 = wave * 4;  // patch rows prow0 .. prow0+3 of a step: four consecutive pixels, the same for all lanes
 
     // G tile: a thread loads 4 consecutive pixels of the channel rows a_row + 64·i.
     const int a_row = tid >> 2, a_c4 = (tid & 3) * 4;
 
-    f32x16 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
+    // hi·hi and the five small products accumulate apart: one rounding against the large sum every sixteen terms.
+    f32x16 acc[TM][TN], fine[TM][TN];
     const int steps_per_image = (p.spatial + BK - 1) / BK;
     const int first_step = chunk * p.steps_per_chunk;
     const int total_steps = max(0, min(s.batch * steps_per_image, first_step + p.steps_per_chunk) - first_step);
@@ -310,81 +325,104 @@ __device__ __forceinline__ void conv_grad_weight_body(const GradWeightArgs &p, f
     // (oy, ox) of this wavefront's first pixel of the step being loaded, advanced by 16 pixels per step without
     // divisions.  Memory is addressed through per-image buffer descriptors with 32-bit offsets; anything outside
     // (padding, pixels past the end, channels past C_out) gets an out-of-range offset and reads as zero.
-    int load_image = first_step / steps_per_image, load_step = first_step - load_image * steps_per_image;
-    int oy, ox;
-    {
+    int load_image, load_step, oy, ox;
+    auto start = [&]() {
+        load_image = first_step / steps_per_image;
+        load_step = first_step - load_image * steps_per_image;
         const int first_pixel = load_step * BK + prow0;
         oy = first_pixel / s.ow;
         ox = first_pixel - oy * s.ow;
-    }
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+                acc[i][j] = fine[i][j] = f32x16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    };
     const unsigned image_bytes = static_cast<unsigned>(s.c_in) * H * W * 4u;
     const unsigned grad_bytes = static_cast<unsigned>(s.c_out) * p.spatial * 4u;
     constexpr unsigned kOutside = 0x80000000u;
-    unsigned a_base[TM];
+    const int last_window = s.c_in * H * W - 4;
+    const unsigned edge_from = max(W - 3, 0);
+    const int last_g_window = s.c_out * p.spatial - 4;
+    const bool a_valid[2] = {oc0 + a_row < s.c_out, oc0 + a_row + 64 < s.c_out};
+    int a_base[TM];
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
-        a_base[i] = oc0 + a_row + 64 * i < s.c_out ? (static_cast<unsigned>(oc0 + a_row + 64 * i) * p.spatial + a_c4) * 4u : kOutside;
+    for (int i = 0; i < TM; ++i) a_base[i] = (oc0 + a_row + 64 * i) * p.spatial + a_c4;
 
-    u32x4_t ra[TM];
-    float rb[TN][4];
-    auto load_global = [&]() {
+    // This thread's values of a step.  A window may reach over the left or right border (edge: some lane's does) or over an end
+    // of the image, and is then loaded from inside it (clamped: some lane's was moved, by moved floats).  ox: the window's first output
+    // column.  pixel: the step's first one in the image.
+    struct Raw {
+        u32x4_t a[TM], b[TN];
+        int pixel, ox, a_moved[TM], moved[TN];
+        bool edge, clamped;
+    };
+    // The offset of the four floats under a lane's window, whether any of them is wanted, and the floats that the load is moved by to
+    // stay inside the image (0 but at its two ends).
+    auto window = [&](int j, int row, int col, int &off, int &moved) {
+        const int at = tap_offset[j] + (row * W + col);
+        off = min(max(at, 0), last_window);
+        moved = off - at;
+        return (static_cast<unsigned>(row + dy[j]) < static_cast<unsigned>(H)) & (static_cast<unsigned>(col + dx[j] + 3) < static_cast<unsigned>(W + 3));
+    };
+    // No branch and the same number of loads whatever the step is, also behind the last one (descriptors of no bytes): a load
+    // that only some paths make has every later wait count for the path without it, and the values of two steps ahead were
+    // waited for in each step (1.75 µs a step against 0.5 µs of matrix instructions).
+    auto load_global = [&](Raw &raw, bool live) {
         const int p0 = load_step * BK;
         const __amdgpu_buffer_rsrc_t rsrc_g = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<float *>(p.grad_output + static_cast<size_t>(load_image) * s.c_out * p.spatial), 0,
-            static_cast<int>(grad_bytes), 0x00020000);
+            live ? static_cast<int>(grad_bytes) : 0, 0x00020000);
         const __amdgpu_buffer_rsrc_t rsrc_x = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<float *>(p.input + static_cast<size_t>(load_image) * s.c_in * H * W), 0, static_cast<int>(image_bytes),
-            0x00020000);
+            const_cast<float *>(p.input + static_cast<size_t>(load_image) * s.c_in * H * W), 0,
+            live ? static_cast<int>(image_bytes) : 0, 0x00020000);
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
-            if (VEC) {  // spatial % 4 == 0: a 16-byte chunk is entirely inside its channel row or entirely past it
-                const unsigned off = (p0 + a_c4 < p.spatial) ? a_base[i] + static_cast<unsigned>(p0) * 4u : kOutside;
-                ra[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_g, off, 0, 0);
+            if (GATHER != Gather::kValues) {
+                const int at = a_base[i] + p0, off = min(at, last_g_window);
+                raw.a_moved[i] = off - at;
+                raw.a[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_g, a_valid[i] ? static_cast<unsigned>(off) * 4u : kOutside, 0, 0);
             } else {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const unsigned off = (p0 + a_c4 + e < p.spatial) ? a_base[i] + static_cast<unsigned>(p0 + e) * 4u : kOutside;
-                    ra[i][e] = __builtin_amdgcn_raw_buffer_load_b32(rsrc_g, off, 0, 0);
+                    const bool inside = a_valid[i] & (p0 + a_c4 + e < p.spatial);
+                    raw.a[i][e] = __builtin_amdgcn_raw_buffer_load_b32(rsrc_g, inside ? static_cast<unsigned>(a_base[i] + p0 + e) * 4u : kOutside, 0, 0);
                 }
             }
         }
-        // The four pixels are the same for every lane of the wavefront (lanes differ in their taps), so whether they
-        // sit in one image row is a scalar question.  If they do, and no lane's tap straddles the left or right
-        // border, the four values are one 128-bit load (dword-aligned is enough for buffer loads).
-        const bool one_row = s.stride_w == 1 && ox + 3 < s.ow && p0 + prow0 + 3 < p.spatial;
+        raw.pixel = p0;
+        // The four pixels are the same for every lane of the wavefront (lanes differ in their taps).
+        if (GATHER == Gather::kWindows) {
+            raw.ox = ox;
+            raw.edge = raw.clamped = false;
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            bool vector_done = false;
-            if (one_row) {
-                const int iy = oy * s.stride_h + dy[j], ix0 = ox + dx[j];
-                const bool row_ok = col_valid[j] && static_cast<unsigned>(iy) < static_cast<unsigned>(H);
-                const bool full = row_ok && ix0 >= 0 && ix0 + 3 < W;
-                if (__builtin_amdgcn_ballot_w64(row_ok && !full) == 0) {
-                    const unsigned off = full ? static_cast<unsigned>(tap_offset[j] + iy * W + ix0) * 4u : kOutside;
-                    const u32x4_t raw = __builtin_amdgcn_raw_buffer_load_b128(rsrc_x, off, 0, 0);
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) rb[j][r] = __uint_as_float(raw[r]);
-                    vector_done = true;
-                }
+            for (int j = 0; j < TN; ++j) {
+                int off;
+                const bool wanted = window(j, oy, ox, off, raw.moved[j]) & (p0 + prow0 < p.spatial);
+                raw.b[j] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_x, wanted ? static_cast<unsigned>(off) * 4u : kOutside, 0, 0);
+                raw.edge |= __builtin_amdgcn_ballot_w64(wanted & (static_cast<unsigned>(ox + dx[j]) >= edge_from)) != 0;
+                raw.clamped |= __builtin_amdgcn_ballot_w64(wanted & (raw.moved[j] != 0)) != 0;
             }
-            if (!vector_done) {
-                int py = oy, px = ox;
+        } else {
+            int py = oy, px = ox;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
+            for (int r = 0; r < 4; ++r) {
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
                     const int iy = py * s.stride_h + dy[j], ix = px * s.stride_w + dx[j];
-                    const bool inside = col_valid[j] && p0 + prow0 + r < p.spatial &&
-                                        static_cast<unsigned>(iy) < static_cast<unsigned>(H) &&
-                                        static_cast<unsigned>(ix) < static_cast<unsigned>(W);
+                    const bool inside = col_valid[j] & (p0 + prow0 + r < p.spatial) &
+                                        (static_cast<unsigned>(iy) < static_cast<unsigned>(H)) &
+                                        (static_cast<unsigned>(ix) < static_cast<unsigned>(W));
                     const unsigned off = inside ? static_cast<unsigned>(tap_offset[j] + iy * W + ix) * 4u : kOutside;
-                    rb[j][r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc_x, off, 0, 0));
-                    if (++px == s.ow) {
-                        px = 0;
-                        ++py;
-                    }
+                    raw.b[j][r] = __builtin_amdgcn_raw_buffer_load_b32(rsrc_x, off, 0, 0);
                 }
+                const bool wrap = ++px == s.ow;
+                px = wrap ? 0 : px;
+                py += wrap ? 1 : 0;
             }
         }
-        // advance to the next step (possibly the next image)
+    };
+    auto advance = [&]() {  // to the next step, possibly the next image's first
         if (++load_step == steps_per_image) {
             load_step = 0;
             ++load_image;
@@ -398,18 +436,97 @@ __device__ __forceinline__ void conv_grad_weight_body(const GradWeightArgs &p, f
             }
         }
     };
-    auto store_lds = [&](int stage) {
+    // Values in their places where a load was moved, zeros for what lies outside the row of the image or behind the last pixel.
+    auto put_back = [](u32x4_t &values, int moved) {
+        const u32x4_t got = values;
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
-            *reinterpret_cast<u32x4_t *>(&As[stage * A_STAGE + (a_row + 64 * i) * A_STRIDE + a_c4]) = ra[i];
+        for (int r = 0; r < 4; ++r) {
+            unsigned value = got[r];
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            f32x4 packed;
-            packed[0] = rb[j][0]; packed[1] = rb[j][1]; packed[2] = rb[j][2]; packed[3] = rb[j][3];
-            *reinterpret_cast<f32x4 *>(&Bs[stage * B_STAGE + (j * 64 + lane) * B_STRIDE + prow0]) = packed;
+            for (int from = 0; from < 4; ++from) value = from + moved == r ? got[from] : value;
+            values[r] = value;
         }
     };
-    auto compute = [&](int stage) {
+    auto settle = [&](Raw &raw) {
+        if (GATHER != Gather::kValues && raw.pixel + BK > p.spatial) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                put_back(raw.a[i], raw.a_moved[i]);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) raw.a[i][r] = raw.pixel + a_c4 + r < p.spatial ? raw.a[i][r] : 0u;
+            }
+        }
+        if (GATHER != Gather::kWindows) return;
+        if (raw.clamped) {
+#pragma unroll
+            for (int j = 0; j < TN; ++j) put_back(raw.b[j], raw.moved[j]);
+        }
+        if (raw.edge) {
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    raw.b[j][r] = static_cast<unsigned>(raw.ox + dx[j] + r) < static_cast<unsigned>(W) ? raw.b[j][r] : 0u;
+        }
+    };
+    // Four neighbouring pixels of a row in pieces.
+    auto split4 = [](unsigned char *dst, int piece_bytes, const u32x4_t &bits) {
+        const f32x4 x = __builtin_bit_cast(f32x4, bits);
+        uint32_t piece[3][2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const float a = x[2 * e] * kSplitScale, b = x[2 * e + 1] * kSplitScale;
+            piece[0][e] = pack_bf16x2_rne(a, b);
+            const float ra = a - __uint_as_float(piece[0][e] << 16), rb = b - __uint_as_float(piece[0][e] & 0xffff0000u);
+            piece[1][e] = pack_bf16x2_rne(ra, rb);
+            const float la = ra - __uint_as_float(piece[1][e] << 16), lb = rb - __uint_as_float(piece[1][e] & 0xffff0000u);
+            piece[2][e] = pack_bf16x2_rne(la, lb);
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i) *reinterpret_cast<uint2 *>(dst + i * piece_bytes) = make_uint2(piece[i][0], piece[i][1]);
+    };
+    auto store_pieces = [&](int stage, const Raw &raw) {
+        unsigned char *const as = lds + stage * PIECES_STAGE, *const bs = as + 3 * A_PIECE;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+            split4(as + (a_c4 >> 3) * A_HALF + (a_row + 64 * i) * 16 + (a_c4 & 4) * 2, A_PIECE, raw.a[i]);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) split4(bs + (prow0 >> 3) * B_HALF + (j * 64 + lane) * 16 + (prow0 & 4) * 2, B_PIECE, raw.b[j]);
+    };
+    // the six piece products, smallest first: (piece of G, piece of the patches)
+    auto compute_pieces = [&](int stage, auto &&between) {
+        constexpr int kFirst[6] = {2, 0, 1, 1, 0, 0}, kSecond[6] = {0, 2, 1, 0, 1, 0};  // (the first three name all pieces)
+        const unsigned char *const as = lds + stage * PIECES_STAGE + (wm * 32 * TM + li) * 16 + lh * A_HALF;
+        const unsigned char *const bs = lds + stage * PIECES_STAGE + 3 * A_PIECE + (wn * 32 * TN + li) * 16 + lh * B_HALF;
+        bf16x8 fa[TM][3], fb[TN][3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {  // in the order of their first use
+#pragma unroll
+            for (int j = 0; j < TN; ++j) fb[j][kSecond[q]] = *reinterpret_cast<const bf16x8 *>(bs + kSecond[q] * B_PIECE + j * 512);
+#pragma unroll
+            for (int i = 0; i < TM; ++i) fa[i][kFirst[q]] = *reinterpret_cast<const bf16x8 *>(as + kFirst[q] * A_PIECE + i * 512);
+        }
+        between();
+#pragma unroll
+        for (int q = 0; q < 6; ++q)
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    f32x16 &sum = q < 5 ? fine[i][j] : acc[i][j];
+                    sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i][kFirst[q]], fb[j][kSecond[q]], sum, 0, 0, 0);
+                }
+    };
+    auto store_lds = [&](int stage, const Raw &raw) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+            *reinterpret_cast<u32x4_t *>(&As[stage * A_STAGE + (a_row + 64 * i) * A_STRIDE + a_c4]) = raw.a[i];
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+            *reinterpret_cast<u32x4_t *>(&Bs[stage * B_STAGE + (j * 64 + lane) * B_STRIDE + prow0]) = raw.b[j];
+    };
+    auto compute = [&](int stage, auto &&between) {
+        between();
         const float *as = As + stage * A_STAGE;
         const float *bs = Bs + stage * B_STAGE;
 #pragma unroll
@@ -431,58 +548,73 @@ __device__ __forceinline__ void conv_grad_weight_body(const GradWeightArgs &p, f
         }
     };
 
-    if (total_steps > 0) {
-        load_global();
-        store_lds(0);
-    }
-    __syncthreads();
-    // (SETS > 1: every set goes through the barriers of the longest run; a set whose run is shorter idles.)
-    const int barrier_steps = SETS > 1 ? p.steps_per_chunk : total_steps;
-    for (int t = 0; t < barrier_steps; ++t) {
-        const bool more = t + 1 < total_steps;
-        if (more) load_global();
-        if (t < total_steps) compute(t & 1);
-        if (more) store_lds((t + 1) & 1);
-        __syncthreads();
-    }
-
-    if constexpr (SETS > 1) {
-        // Thread t's 16·TM·TN accumulator values as 128-bit pieces e at (e·256 + t)·16 bytes: conflict-free both ways.
-        static_assert(TM * TN * 16 * 256 * 4 <= SETS * (2 * A_STAGE + 2 * B_STAGE) * 4, "the tile fits the workgroup's LDS");
-        f32x4 *exchange = reinterpret_cast<f32x4 *>(lds_all);
-#pragma unroll
-        for (int other = 1; other < SETS; ++other) {
-            if (set == other) {
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int j = 0; j < TN; ++j)
-#pragma unroll
-                        for (int q = 0; q < 4; ++q)
-                            exchange[((i * TN + j) * 4 + q) * 256 + tid] =
-                                f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-            }
+    // Step t is computed from LDS while the values of step t + 1 wait in registers and those of t + 2 are on their way.
+    auto sum_steps = [&](auto &&store, auto &&compute_step) {
+        start();
+        Raw raw[2];
+        load_global(raw[0], total_steps > 0);
+        if (total_steps <= 1) {  // nothing to run ahead of (0.4 µs of the smallest layers' 8)
+            settle(raw[0]);
+            store(0, raw[0]);
             __syncthreads();
-            if (set == 0) {
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int j = 0; j < TN; ++j)
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            const f32x4 v = exchange[((i * TN + j) * 4 + q) * 256 + tid];
-                            acc[i][j][4 * q] += v[0];
-                            acc[i][j][4 * q + 1] += v[1];
-                            acc[i][j][4 * q + 2] += v[2];
-                            acc[i][j][4 * q + 3] += v[3];
-                        }
-            }
-            __syncthreads();
+            compute_step(0, [] {});
+            return;
         }
-        if (set != 0) return;
-    }
+        advance();
+        load_global(raw[1], true);
+        advance();
+        settle(raw[0]);
+        store(0, raw[0]);
+        load_global(raw[0], total_steps > 2);
+        __syncthreads();
+        auto step = [&](int t, Raw &next) {
+            compute_step(t & 1, [&] {
+                settle(next);
+                advance();
+                store((t + 1) & 1, next);
+                load_global(next, t + 3 < total_steps);
+            });
+            // The cutting and addressing of the two steps ahead into the gaps between the matrix instructions.  (The small tile has
+            // four wavefronts a SIMD for that.)
+            if constexpr (TM * TN > 1) {
+#pragma unroll
+                for (int g = 0; g < 6 * TM * TN; ++g) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+                }
+            }
+            __syncthreads();
+        };
+        // the last step has none to prepare
+        int t = 0;
+        for (; t + 2 < total_steps; t += 2) {
+            step(t, raw[1]);
+            step(t + 1, raw[0]);
+        }
+        if (t + 1 < total_steps) step(t++, raw[1]);
+        if (t < total_steps) compute_step(t & 1, [] {});
+    };
+    if (threadIdx.x == 0) beyond = 0;
+    sum_steps(store_pieces, compute_pieces);
+    // A value the scaled pieces cannot carry, or a sum that overflows, leaves an infinity or NaN behind, which no later term takes
+    // away: the tile is then summed again on the f32 matrix instruction, from the original values.
+    bool finite = true;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                acc[i][j][r] += fine[i][j][r];
+                finite = finite && fabsf(acc[i][j][r]) < INFINITY;
+                acc[i][j][r] *= kSplitUnscale;
+            }
+    if (!finite) beyond = 1;
+    __syncthreads();
+    if (beyond) sum_steps(store_lds, compute);
 
-    float *dst = p.partial + static_cast<size_t>(SETS > 1 ? chunk / SETS : chunk) * s.c_out * p.S;
+    float *dst = p.partial + static_cast<size_t>(chunk) * s.c_out * p.S;
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
         const int out_col = s0 + wn * 32 * TN + j * 32 + li;
@@ -497,31 +629,18 @@ __device__ __forceinline__ void conv_grad_weight_body(const GradWeightArgs &p, f
     }
 }
 
-template <bool VEC>
-__global__ __launch_bounds__(256) void conv_grad_weight_kernel(GradWeightArgs p)
+template <Gather GATHER>
+__global__ __launch_bounds__(256, 4) void conv_grad_weight_kernel(GradWeightArgs p)
 {
-    __shared__ __attribute__((aligned(16))) float As[2 * 64 * 20];
-    __shared__ __attribute__((aligned(16))) float Bs[2 * 64 * 20];
-    conv_grad_weight_body<VEC, 1, 1>(p, As, Bs);
+    extern __shared__ __attribute__((aligned(16))) unsigned char grad_weight_lds[];
+    conv_grad_weight_body<GATHER, 1, 1>(p, grad_weight_lds);
 }
 
-// Three workgroups per compute unit (3 × 51,200 B of LDS, three wavefronts per SIMD): the occupancy attribute makes
-// the compiler fit 170 registers (it does, 160 without spilling) instead of spreading the accumulators over the
-// accumulation registers at two wavefronts per SIMD.
-template <bool VEC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void conv_grad_weight_big_kernel(GradWeightArgs p)
+template <Gather GATHER>
+__global__ __launch_bounds__(256, 1) void conv_grad_weight_big_kernel(GradWeightArgs p)
 {
-    __shared__ __attribute__((aligned(16))) float As[2 * 128 * 20];
-    __shared__ __attribute__((aligned(16))) float Bs[2 * 192 * 20];
-    conv_grad_weight_body<VEC, 2, 3>(p, As, Bs);
-}
-
-// The same tile with three sets of four wavefronts in one workgroup (one workgroup per compute unit, 153,600 B of LDS).
-template <bool VEC>
-__global__ __launch_bounds__(768) __attribute__((amdgpu_waves_per_eu(3, 3))) void conv_grad_weight_big3_kernel(GradWeightArgs p)
-{
-    extern __shared__ __attribute__((aligned(16))) float grad_weight_lds[];
-    conv_grad_weight_body<VEC, 2, 3, 3>(p, grad_weight_lds, nullptr);
+    extern __shared__ __attribute__((aligned(16))) unsigned char grad_weight_lds[];
+    conv_grad_weight_body<GATHER, 2, 3>(p, grad_weight_lds);
 }
 
 }  // namespace
@@ -669,8 +788,8 @@ hipError_t launch_conv2d_grad_weight_f32(const ConvShape &shape, const float *in
     const size_t count = static_cast<size_t>(shape.c_out) * S;
     if (count == 0) return hipSuccess;
     // One image of the input and of grad_output is addressed through 32-bit byte offsets.
-    if (static_cast<size_t>(shape.c_in) * shape.h * shape.w * 4 >= (1ull << 31) ||
-        static_cast<size_t>(shape.c_out) * shape.oh * shape.ow * 4 >= (1ull << 31))
+    const size_t image_floats = static_cast<size_t>(shape.c_in) * shape.h * shape.w;
+    if (image_floats * 4 >= (1ull << 31) || static_cast<size_t>(shape.c_out) * shape.oh * shape.ow * 4 >= (1ull << 31))
         return hipErrorInvalidValue;
     GradWeightArgs args;
     args.input = input;
@@ -681,47 +800,42 @@ hipError_t launch_conv2d_grad_weight_f32(const ConvShape &shape, const float *in
     // 128 × 192 tiles when they waste little (every output channel and column a tile covers beyond the matrix is
     // arithmetic thrown away), 64 × 64 tiles otherwise.
     const long long big_cover = static_cast<long long>((shape.c_out + 127) / 128 * 128) * ((S + 191) / 192 * 192);
-    const bool big = big_cover * 10 <= static_cast<long long>(count) * 12;
+    const bool big = big_cover * 10 <= static_cast<long long>(count) * 12;  // (of 107 channels at least: never kValues)
     const int bm = big ? 128 : 64, bn = big ? 192 : 64;
     args.tiles_s = (S + bn - 1) / bn;
     const int tiles = args.tiles_s * ((shape.c_out + bm - 1) / bm);
     // The reduction (all 16-pixel steps of all images, numbered image by image) is cut into chunks so that the
-    // launch is about one round of resident workgroups (8 small or 3 big tiles per compute unit).
+    // launch is about one round of resident workgroups (four small tiles or one big tile per compute unit).
     const long long steps_per_image = (args.spatial + 15) / 16;
     const long long total_steps = steps_per_image * shape.batch;
-    const long long slots = big ? 768 : 2048;
+    const long long slots = big ? 256 : 1024;
     long long chunks = slots / tiles;  // rounded down: one workgroup too many would run as a round of its own
     if (chunks > total_steps) chunks = total_steps;
     if (chunks < 1) chunks = 1;
     args.steps_per_chunk = static_cast<int>(total_steps > 0 ? (total_steps + chunks - 1) / chunks : 1);
     chunks = total_steps > 0 ? (total_steps + args.steps_per_chunk - 1) / args.steps_per_chunk : 1;
-    // Big tiles with at least three runs of steps per tile: three runs share a workgroup (and a partial tile).
-    const bool three_sets = big && chunks >= 3;
-    if (three_sets) chunks = (chunks + 2) / 3;
     void *workspace = nullptr;
     hipError_t rc = stream_workspace(stream, static_cast<size_t>(chunks) * count * sizeof(float), &workspace);
     if (rc != hipSuccess) return rc;
     args.partial = static_cast<float *>(workspace);
-    const bool vec = args.spatial % 4 == 0 && (reinterpret_cast<uintptr_t>(grad_output) & 15u) == 0;
     const size_t workgroups = static_cast<size_t>(tiles) * static_cast<size_t>(chunks);
     if (workgroups > 0x7ffffff0u) return hipErrorInvalidConfiguration;
     args.workgroups = static_cast<int>(workgroups);
     const dim3 grid(static_cast<unsigned>((workgroups + 7) / 8 * 8));
-    if (three_sets) {
-        constexpr size_t lds_bytes = 3 * (2 * 128 * 20 + 2 * 192 * 20) * sizeof(float);
-        auto kernel = vec ? conv_grad_weight_big3_kernel<true> : conv_grad_weight_big3_kernel<false>;
-        rc = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                 static_cast<int>(lds_bytes));
+    // Windows need the four pixels of a thread in one output row and neighbouring columns of the input, and an image that holds one.
+    // (Rows of other widths as two windows, the second for the pixels in the next row: 111 instead of 75 µs for 256 -> 256 channels at
+    // 14×14, and between 4 % less and 10 % more in the small tile.)
+    const bool windows = shape.stride_h == 1 && shape.stride_w == 1 && shape.ow % 4 == 0 && image_floats >= 4;
+    const Gather gather = static_cast<size_t>(shape.c_out) * args.spatial < 4 ? Gather::kValues : windows ? Gather::kWindows : Gather::kTaps;
+    auto kernel = gather == Gather::kValues    ? conv_grad_weight_kernel<Gather::kValues>
+                  : gather == Gather::kWindows ? (big ? conv_grad_weight_big_kernel<Gather::kWindows> : conv_grad_weight_kernel<Gather::kWindows>)
+                                               : (big ? conv_grad_weight_big_kernel<Gather::kTaps> : conv_grad_weight_kernel<Gather::kTaps>);
+    const size_t lds_bytes = big ? kGradWeightStages<2, 3> : kGradWeightStages<1, 1>;
+    if (big) {  // (beyond what a launch may take unasked)
+        rc = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes));
         if (rc != hipSuccess) return rc;
-        hipLaunchKernelGGL(kernel, grid, dim3(768), lds_bytes, stream, args);
-    } else if (big && vec)
-        hipLaunchKernelGGL(conv_grad_weight_big_kernel<true>, grid, dim3(256), 0, stream, args);
-    else if (big)
-        hipLaunchKernelGGL(conv_grad_weight_big_kernel<false>, grid, dim3(256), 0, stream, args);
-    else if (vec)
-        hipLaunchKernelGGL(conv_grad_weight_kernel<true>, grid, dim3(256), 0, stream, args);
-    else
-        hipLaunchKernelGGL(conv_grad_weight_kernel<false>, grid, dim3(256), 0, stream, args);
+    }
+    hipLaunchKernelGGL(kernel, grid, dim3(256), lds_bytes, stream, args);
     rc = hipGetLastError();
     if (rc != hipSuccess) return rc;
     if (count % 4 == 0 && ((reinterpret_cast<uintptr_t>(args.partial) | reinterpret_cast<uintptr_t>(grad_weight)) & 15u) == 0)

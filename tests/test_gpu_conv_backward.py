@@ -319,3 +319,101 @@ def test_conv2d_layer_backward_accumulates(hip, oracle):
     with pytest.raises(st.TensorError, match="ShapeMismatch"):
         conv.backward(x, st.Tensor.zeros(batch, 7))
     assert conv.backward(st.Tensor.zeros(0, 90), st.Tensor.zeros(0, 120)).shape() == (0, 90)
+
+
+def grad_weight_f64(case, x, g):
+    """grad_weight · batch from its definition in float64, and the same sum over magnitudes."""
+    batch, c_in, h, w, c_out, kernel, stride, padding, dilation = case
+    x = np.pad(x.astype(np.float64).reshape(batch, c_in, h, w), ((0, 0), (0, 0), (padding[0],) * 2, (padding[1],) * 2))
+    oh = (h + 2 * padding[0] - dilation[0] * (kernel[0] - 1) - 1) // stride[0] + 1
+    ow = (w + 2 * padding[1] - dilation[1] * (kernel[1] - 1) - 1) // stride[1] + 1
+    g = g.astype(np.float64).reshape(batch, c_out, oh * ow).transpose(1, 0, 2).reshape(c_out, -1)
+    out = np.zeros((2, c_out, c_in, *kernel))
+    for ky in range(kernel[0]):
+        for kx in range(kernel[1]):
+            seen = x[:, :, ky * dilation[0]:, kx * dilation[1]:][:, :, :oh * stride[0]:stride[0], :ow * stride[1]:stride[1]]
+            seen = seen.transpose(0, 2, 3, 1).reshape(-1, c_in)
+            with np.errstate(invalid="ignore"):
+                out[:, :, :, ky, kx] = g @ seen, np.abs(g) @ np.abs(seen)
+    return out.reshape(2, -1)
+
+
+def run_grad_weight(hip, case, x, g, n):
+    d_x, d_g, d_w = hip.DeviceBuffer.from_array(x), hip.DeviceBuffer.from_array(g), hip.DeviceBuffer(4 * n)
+    hip.conv2d_grad_weight_f32_dev(*case, d_x, d_g, 1.0, d_w)
+    hip.device_synchronize()
+    return d_w.to_array(np.float32, n)
+
+
+def grad_weight_inputs(hip, case, seed):
+    batch, c_in, h, w, c_out, kernel, stride, padding, dilation = case
+    oh = (h + 2 * padding[0] - dilation[0] * (kernel[0] - 1) - 1) // stride[0] + 1
+    ow = (w + 2 * padding[1] - dilation[1] * (kernel[1] - 1) - 1) // stride[1] + 1
+    rng = np.random.default_rng(seed)
+    return (rng.normal(size=batch * c_in * h * w).astype(np.float32), rng.normal(size=batch * c_out * oh * ow).astype(np.float32),
+            c_out * c_in * kernel[0] * kernel[1])
+
+
+GRAD_WEIGHT_CASES = [
+    # windows over the borders: rows of one window, both ends of the image, more padding than the image is wide
+    (3, 1, 2, 2, 5, (3, 3), (1, 1), (2, 2), (1, 1)),
+    (2, 3, 1, 4, 70, (1, 7), (1, 1), (0, 3), (1, 1)),
+    (1, 2, 5, 1, 3, (3, 2), (1, 1), (1, 2), (1, 1)),
+    (2, 5, 6, 8, 66, (5, 9), (1, 1), (2, 4), (1, 1)),
+    (2, 9, 8, 10, 33, (3, 3), (1, 1), (2, 3), (2, 2)),
+    # one step and no full step; columns and channels just past a tile, of either tile
+    (1, 64, 4, 4, 64, (1, 1), (1, 1), (0, 0), (1, 1)),
+    (1, 65, 3, 4, 65, (1, 1), (1, 1), (0, 0), (1, 1)),
+    (5, 64, 12, 12, 128, (3, 3), (1, 1), (1, 1), (1, 1)),
+    (2, 43, 20, 20, 255, (3, 3), (1, 1), (1, 1), (1, 1)),
+    (40, 64, 28, 28, 128, (3, 3), (1, 1), (1, 1), (1, 1)),
+    # four loads of one value: widths that are no multiple of four, strides, planes of odd sizes
+    (3, 64, 7, 7, 128, (3, 3), (1, 1), (1, 1), (1, 1)),
+    (2, 64, 14, 14, 128, (3, 3), (1, 1), (1, 1), (1, 1)),
+    (2, 64, 15, 16, 128, (3, 3), (2, 1), (1, 1), (1, 1)),
+    # a gradient below one window of four, and one that is exactly one
+    (5, 3, 2, 5, 1, (2, 3), (1, 1), (0, 0), (1, 1)),
+    (5, 3, 2, 6, 1, (2, 3), (1, 1), (0, 0), (1, 1)),
+]
+
+
+@pytest.mark.parametrize("case", GRAD_WEIGHT_CASES)
+def test_grad_weight_against_float64(hip, case):
+    """Sums of products of pieces: every product is exact to 2^-24, the large ones take a rounding each sixteen terms, the
+    partial sums of the workgroups one each.  2^-22 of the summed magnitudes holds 4 roundings of a sum as large as all of them;
+    the roundings are of running sums, which are smaller."""
+    x, g, n = grad_weight_inputs(hip, case, 5)
+    want, magnitudes = grad_weight_f64(case, x, g)
+    got = run_grad_weight(hip, case, x, g, n)
+    assert np.all(np.abs(got - want) <= 2.0 ** -22 * magnitudes + 1e-30)
+
+
+@pytest.mark.parametrize("case", [GRAD_WEIGHT_CASES[3], GRAD_WEIGHT_CASES[7], GRAD_WEIGHT_CASES[11]])
+@pytest.mark.parametrize("x_scale, g_scale", [(2.0 ** 110, 2.0 ** -60), (2.0 ** -100, 2.0 ** -20), (2.0 ** 57, 2.0 ** 60)])
+def test_grad_weight_of_any_magnitude(hip, case, x_scale, g_scale):
+    """Values too large for scaled pieces and sums beyond them are summed again in f32: a rounding a term, half the terms'
+    square root of them in the same direction (observed; the bound takes 32 of the largest).  The largest products here are of
+    2^122, so that their sums of up to 720 terms (2^9.5 of them by magnitude, 27 of their size in the mean) stay below 2^128."""
+    x, g, n = grad_weight_inputs(hip, case, 6)
+    x, g = x * np.float32(x_scale), g * np.float32(g_scale)
+    want, magnitudes = grad_weight_f64(case, x, g)
+    got = run_grad_weight(hip, case, x, g, n)
+    assert np.all(np.isfinite(got))
+    assert np.all(np.abs(got - want) <= 2.0 ** -19 * magnitudes + 2.0 ** -149)
+
+
+@pytest.mark.parametrize("case", [GRAD_WEIGHT_CASES[3], GRAD_WEIGHT_CASES[7], GRAD_WEIGHT_CASES[10]])
+def test_grad_weight_keeps_infinities_and_nan_to_their_terms(hip, case):
+    """A value at the end of an image row reaches the columns whose taps read it and no others, although the loads do."""
+    batch, c_in, h, w, c_out, kernel, stride, padding, dilation = case
+    x, g, n = grad_weight_inputs(hip, case, 7)
+    x = x.reshape(batch, c_in, h, w)
+    g = np.abs(g) + np.float32(0.5)
+    x[0, 1, 2, w - 1], x[batch - 1, 0, 0, 0], x[0, c_in - 1, h - 1, w - 1], x[0, 3, h - 1, 0] = np.inf, np.nan, -np.inf, np.inf
+    want, magnitudes = grad_weight_f64(case, x.reshape(-1), g)
+    got = run_grad_weight(hip, case, x.reshape(-1), g, n)
+    finite = np.isfinite(want)
+    # a kernel of f32 products adds zeros for what lies outside the image, so a border tap's sums stay as the float64 ones
+    assert np.array_equal(np.isfinite(got), finite)
+    assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
+    assert np.all(np.abs(got[finite] - want[finite]) <= 2.0 ** -19 * magnitudes[finite])
