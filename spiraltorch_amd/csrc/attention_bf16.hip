@@ -582,6 +582,221 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     }
 }
 
+// -------------------------------------------------------------------------------------------------
+// Few queries for the chip: 32 of them a workgroup instead of 128, and the keys dealt out to its four wavefronts in tiles of 32
+// (wavefront w takes tiles w, w + 4, ...), each with its own maximum, sum and accumulators, which are put together through LDS at the
+// end.  What bounds a launch of a few workgroups is the chain of one wavefront, a tile after the other: a quarter of the tiles,
+// in four times the workgroups.  K comes as fragments straight from memory and V through a piece of LDS of the wavefront's own, both
+// two tiles ahead, so that nothing waits for another wavefront before the end.
+// -------------------------------------------------------------------------------------------------
+constexpr int kBQSplit = 32;
+// One workgroup of it a compute unit: a quarter of the chain in the place of idle units.  µs before / after, causal, 8 contexts of 64
+// values a head: 117 queries 5.5 / 4.4, 500 10.7 / 6.7, 1000 (256 workgroups) 17.7 / 9.3; 128 values: 117 8.0 / 6.5, 1000 26.2 / 15.6.
+// Two a unit pay only for 64 values a head and some length (2048 queries 31.4 / 20.7, 32 contexts of 500 10.8 / 9.0; 64 contexts of 256
+// 7.5 / 7.1 causal, 7.7 / 7.8 not; 128 values: 32 of 500 16.1 / 17.0), where the kernels above read K and V a quarter as often: at
+// 1024 workgroups 18.5 / 20.2.  Below 65 queries the wide heads' putting together costs what the split gains (40 queries 5.5 / 5.5).
+bool split_keys(size_t contexts, size_t sequence, size_t head_dim)
+{
+    const size_t workgroups = contexts * ((sequence + kBQSplit - 1) / kBQSplit);
+    if (head_dim == 64) return workgroups <= (sequence > 384 ? 512 : 256);
+    return sequence > 64 && workgroups <= 256;
+}
+template <int D>
+constexpr int kSplitLdsFloats = 4 * (32 * (D + 4) + 64);  // four partial outputs and their maxima and sums; V fits below
+
+template <int D, bool CAUSAL>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void attention_bf16_keys_kernel(AttnBf16Args p)
+{
+    constexpr int VS = D + 8;      // V row stride (elements), as in the kernel above
+    constexpr int OS = D + 4;      // row stride of the partial outputs (floats)
+    constexpr int KC = D / 16, DT = D / 32, LOADS = 32 * D / 8 / 64;
+    __shared__ __attribute__((aligned(16))) float lds[kSplitLdsFloats<D>];
+    static_assert(4 * 32 * VS * 2 <= 4 * 32 * OS * 4, "V tiles where the partial outputs will be");
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 31, lh = lane >> 5;
+    const int S = p.S;
+    const int contexts = p.batch * p.heads;
+    // a context's tiles on one XCD where the contexts divide evenly; the longest rows first
+    int ctx, q_tile;
+    if (p.swizzle) {
+        const int per_xcd = contexts >> 3, i = blockIdx.x >> 3;
+        q_tile = p.q_tiles - 1 - i / per_xcd;
+        ctx = (blockIdx.x & 7) * per_xcd + i % per_xcd;
+    } else {
+        q_tile = p.q_tiles - 1 - blockIdx.x / contexts;
+        ctx = blockIdx.x % contexts;
+    }
+    const int q0 = q_tile * kBQSplit;
+    const int my_q = q0 + li;
+    const int b = ctx / p.heads, h = ctx % p.heads;
+    const size_t in_base = static_cast<size_t>(b) * S * p.ld_in + static_cast<size_t>(h) * D;
+    const unsigned in_bytes = (static_cast<unsigned>(S - 1) * static_cast<unsigned>(p.ld_in) + D) * 2u;
+    const __amdgpu_buffer_rsrc_t rsrc_q =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(p.q + in_base), 0, static_cast<int>(in_bytes), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc_k =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(p.k + in_base), 0, static_cast<int>(in_bytes), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc_v =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(p.v + in_base), 0, static_cast<int>(in_bytes), 0x00020000);
+    auto fetch8 = [&](const __amdgpu_buffer_rsrc_t &rsrc, int row, int d) -> u32x4_t {  // zeros for rows past the end
+        const unsigned off = (static_cast<unsigned>(row) * static_cast<unsigned>(p.ld_in) + d) * 2u;
+        return __builtin_amdgcn_raw_buffer_load_b128(rsrc, row < S ? off : 0x80000000u, 0, 0);
+    };
+
+    struct Tile {  // a lane's share of 32 keys: K fragments, and V rows to be stored
+        u32x4_t k[KC], v[LOADS];
+    };
+    auto load = [&](Tile &tile, int key0) {
+#pragma unroll
+        for (int c = 0; c < KC; ++c) tile.k[c] = fetch8(rsrc_k, key0 + li, c * 16 + lh * 8);
+#pragma unroll
+        for (int r = 0; r < LOADS; ++r) {
+            const int f = lane + 64 * r;
+            tile.v[r] = fetch8(rsrc_v, key0 + f / (D / 8), (f % (D / 8)) * 8);
+        }
+    };
+    bf16x8 qf[KC];
+    Tile tiles[2];
+    {
+        u32x4_t raw[KC];
+#pragma unroll
+        for (int c = 0; c < KC; ++c) raw[c] = fetch8(rsrc_q, my_q, c * 16 + lh * 8);
+        load(tiles[0], wave * 32);
+        load(tiles[1], wave * 32 + 128);
+#pragma unroll
+        for (int c = 0; c < KC; ++c) {
+            if (p.scale < 0.0f) raw[c] ^= 0x80008000u;  // (the scale applied below is never negative)
+            qf[c] = __builtin_bit_cast(bf16x8, raw[c]);
+        }
+    }
+    f32x16 oacc[DT];
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+        oacc[t] = f32x16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float run_max = -INFINITY, run_sum = 0.0f;
+    const float scale_log2e = fmaxf(fabsf(p.scale) * kLog2e16, 1e-30f);
+    const float lag = 8.0f / scale_log2e;
+    const int last_key = CAUSAL ? min(my_q, S - 1) : S - 1;
+    uint16_t *const vs = reinterpret_cast<uint16_t *>(lds) + wave * 32 * VS;
+    const int i16 = lane & 15, c16 = (lane >> 4) & 1;
+    const int v_read = (lh * 4 + (i16 >> 2)) * VS + c16 * 16 + (i16 & 3) * 4;
+
+    auto compute = [&](Tile &tile, int key0) {
+        f32x16 sacc = f32x16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < KC; ++c)
+            sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, tile.k[c]), qf[c], sacc, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < LOADS; ++r) {
+            const int f = lane + 64 * r;
+            *reinterpret_cast<u32x4_t *>(&vs[f / (D / 8) * VS + (f % (D / 8)) * 8]) = tile.v[r];
+        }
+        load(tile, key0 + 256);
+        float tile_max = -INFINITY;
+        if (key0 + 32 > S || (CAUSAL && key0 + 31 > q0)) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (key0 + (r >> 2) * 8 + lh * 4 + (r & 3) > last_key) sacc[r] = -INFINITY;
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) tile_max = fmaxf(tile_max, sacc[r]);
+        tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32));
+        if (__any(tile_max > run_max + lag)) {  // the reference maximum may lag, as in the kernel above
+            const float new_max = fmaxf(run_max, tile_max);
+            const float alpha = __builtin_amdgcn_exp2f((run_max - (new_max == -INFINITY ? 0.0f : new_max)) * scale_log2e);
+            run_sum *= alpha;
+#pragma unroll
+            for (int t = 0; t < DT; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) oacc[t][r] *= alpha;
+            run_max = new_max;
+        }
+        const float shift = -(run_max == -INFINITY ? 0.0f : run_max) * scale_log2e;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            sacc[r] = __builtin_amdgcn_exp2f(fmaf(sacc[r], scale_log2e, shift));
+            run_sum += sacc[r];
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wavefront's V rows are in LDS
+        // Oᵀ += Vᵀ·Pᵀ, 16 keys per MFMA, with V gathered to the keys' order in the accumulators as in the kernel above
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            u32x4_t packed;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) packed[e] = pack_bf16x2(sacc[8 * j + 2 * e], sacc[8 * j + 2 * e + 1]);
+            const bf16x8 pf = __builtin_bit_cast(bf16x8, packed);
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) {
+                const uint16_t *src = &vs[j * 16 * VS + v_read + dt * 32];
+                const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(src));
+                const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(src + 8 * VS));
+                const bf16x8 vf = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf, oacc[dt], 0, 0, 0);
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // and read, before the next tile's take their place
+    };
+    const int key_end = CAUSAL ? min(S, q0 + kBQSplit) : S;
+    for (int key0 = wave * 32; key0 < key_end; key0 += 256) {
+        compute(tiles[0], key0);
+        if (key0 + 128 < key_end) compute(tiles[1], key0 + 128);
+    }
+
+    // The four parts of each query: everything on the scale of the largest maximum, added in the order of the wavefronts.
+    run_sum += __shfl_xor(run_sum, 32);
+    float *const maxima = lds + 4 * 32 * OS, *const sums = maxima + 128;
+    if (lh == 0) {
+        maxima[wave * 32 + li] = run_max;
+        sums[wave * 32 + li] = run_sum;
+    }
+    __syncthreads();
+    float top = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) top = fmaxf(top, maxima[w * 32 + li]);
+    const float safe_top = top == -INFINITY ? 0.0f : top;
+    const float mine = __builtin_amdgcn_exp2f((run_max - safe_top) * scale_log2e);  // nothing seen: exp2(-inf) = 0
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            f32x4 part;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) part[e] = oacc[t][g * 4 + e] * mine;
+            *reinterpret_cast<f32x4 *>(&lds[(wave * 32 + li) * OS + t * 32 + g * 8 + lh * 4]) = part;
+        }
+    __syncthreads();
+    const int row = tid >> 3, query = q0 + row;
+    if (query >= S) return;
+    float row_top = -INFINITY, total = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) row_top = fmaxf(row_top, maxima[w * 32 + row]);
+    row_top = row_top == -INFINITY ? 0.0f : row_top;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) total += sums[w * 32 + row] * __builtin_amdgcn_exp2f((maxima[w * 32 + row] - row_top) * scale_log2e);
+    const float inv = total > 0.0f ? 1.0f / total : 0.0f;
+    uint16_t *const orow = p.out + (static_cast<size_t>(b) * S + query) * p.ld_out + static_cast<size_t>(h) * D;
+#pragma unroll
+    for (int i = 0; i < D / 32; ++i) {  // eight lanes write 32 neighbouring values
+        const int d = i * 32 + (tid & 7) * 4;
+        f32x4 sum = *reinterpret_cast<const f32x4 *>(&lds[row * OS + d]);
+#pragma unroll
+        for (int w = 1; w < 4; ++w) sum += *reinterpret_cast<const f32x4 *>(&lds[(w * 32 + row) * OS + d]);
+        const u32x2_t packed = {pack_bf16x2(sum[0] * inv, sum[1] * inv), pack_bf16x2(sum[2] * inv, sum[3] * inv)};
+        *reinterpret_cast<u32x2_t *>(orow + d) = packed;
+    }
+}
+
+template <int D, bool CAUSAL>
+hipError_t launch_keys(AttnBf16Args args, hipStream_t stream)
+{
+    args.q_tiles = (args.S + kBQSplit - 1) / kBQSplit;
+    const unsigned blocks = static_cast<unsigned>(args.batch * args.heads * args.q_tiles);
+    hipLaunchKernelGGL((attention_bf16_keys_kernel<D, CAUSAL>), dim3(blocks), dim3(256), 0, stream, args);
+    return hipGetLastError();
+}
+
 template <bool CAUSAL>
 hipError_t launch_d64(const AttnBf16Args &args, hipStream_t stream)
 {
@@ -642,6 +857,10 @@ hipError_t launch_attention_bf16(size_t batch, size_t heads, size_t sequence, si
     if (contexts * static_cast<size_t>(args.q_tiles) > 0x7fffffffu) return hipErrorInvalidConfiguration;
     args.swizzle = (contexts % 8 == 0) ? 1 : 0;
     args.scale = scale;
+    if (split_keys(contexts, sequence, head_dim)) {
+        if (head_dim == 64) return causal ? launch_keys<64, true>(args, stream) : launch_keys<64, false>(args, stream);
+        return causal ? launch_keys<128, true>(args, stream) : launch_keys<128, false>(args, stream);
+    }
     if (head_dim == 64) return causal ? launch_d64<true>(args, stream) : launch_d64<false>(args, stream);
     return causal ? launch_variant<128, true>(args, stream) : launch_variant<128, false>(args, stream);
 }

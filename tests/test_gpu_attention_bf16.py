@@ -110,3 +110,28 @@ def test_unsupported_shapes_are_rejected(hip):
         hip.attention_bf16_dev(1, 2, 8, 64, 0.1, False, buf, buf, buf, 64, buf, 128)     # ld_in < heads*head_dim
     with pytest.raises(hip.HipErr):
         hip.attention_bf16_dev(1, 1, 8, 64, float("inf"), False, buf, buf, buf, 64, buf, 64)
+
+
+# 32-query workgroups whose wavefronts share the keys: below, at and past their limits in workgroups and sequence, tiles of
+# 32 keys that leave wavefronts without any, one and two rounds of eight tiles, and the first shapes of the 128-query kernels.
+KEYS_CASES = [
+    (1, 1, 2, 64, True), (1, 3, 32, 64, False), (3, 1, 95, 64, True), (1, 2, 128, 64, True), (1, 1, 161, 64, False),
+    (1, 1, 290, 64, True), (1, 2, 545, 64, False), (2, 8, 512, 64, True), (3, 11, 511, 64, True), (1, 64, 129, 64, False),
+    (4, 13, 130, 64, True), (1, 1, 64, 128, True), (1, 1, 65, 128, True), (2, 3, 300, 128, False), (2, 16, 256, 128, True),
+    (3, 11, 255, 128, False),
+]
+
+
+@pytest.mark.parametrize("batch,heads,seq,dim,causal", KEYS_CASES)
+def test_keys_shared_by_the_wavefronts(hip, oracle, batch, heads, seq, dim, causal):
+    rng = np.random.default_rng(seq + dim)
+    qkv = rng.normal(size=(batch * seq, 3, heads * dim)).astype(np.float32)
+    qkv[:, 0] *= 4  # weights that differ by more than the lag of the maximum allows
+    qkv[1 % (batch * seq), 0, :dim] = np.nan  # one query of the first head: nothing of the others
+    bits = inputs.to_bf16(qkv.ravel())
+    got = run_fused(hip, batch, heads, seq, dim, float(1.0 / np.sqrt(dim)), bits, causal)
+    qkv[1 % (batch * seq), 0, :dim] = 0
+    want = oracle_fused(oracle, batch, heads, seq, dim, float(1.0 / np.sqrt(dim)), inputs.to_bf16(qkv.ravel()), causal)
+    assert np.all(np.isnan(got[1 % (batch * seq), :dim]))
+    got[1 % (batch * seq), :dim] = want[1 % (batch * seq), :dim]
+    assert_close(got, want, BF16_REL, ABS, f"bf16 attention b{batch} h{heads} s{seq} d{dim} causal={causal}")
