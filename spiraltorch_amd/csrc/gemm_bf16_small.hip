@@ -8,8 +8,8 @@
 // results do not depend on scheduling, and are the same for both layouts of B.
 //
 // What bounds it is latency: a launch (2.0 µs for an empty kernel), one trip to memory, the sums' trip through LDS.  Of a
-// launch among others, before -> here: 117×1536×512 10.4 -> 4.1 µs, 117×512×512 10.1 -> 3.1, 117×2048×512 10.0 -> 4.4,
-// 117×512×2048 11.4 -> 4.9, 512×1536×512 8.3 -> 7.3, 1024×512×2048 14.4 -> 9.6, 256×1000×512 11.0 -> 4.3.  Larger launches are
+// launch among others, before -> here: 117×1536×512 10.4 -> 4.1 µs, 117×512×512 10.1 -> 3.1, 117×2048×512 10.0 -> 4.0,
+// 117×512×2048 11.4 -> 4.5, 512×1536×512 8.3 -> 7.0, 1024×512×2048 14.4 -> 9.6, 256×1000×512 11.0 -> 4.3.  Larger launches are
 // bound by LDS and L2 traffic (16 to 32 flops a byte) and belong to the large tiles.  Layer normalisation of the rows on their
 // way in was tried: 3.2 µs more a launch, where the kernel of its own takes 2.4.
 #include <algorithm>
@@ -59,7 +59,18 @@ __device__ __forceinline__ void gemm_bf16_small_body(const SmallArgs &p)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lj = lane & 15, lg = lane >> 4;
     const int M = p.M, N = p.N, K = p.K;
-    const int tile_n = static_cast<int>(blockIdx.x) / p.tiles_m, tile_m = static_cast<int>(blockIdx.x) - tile_n * p.tiles_m;
+    // Workgroup ids go round-robin over the 8 XCDs: each takes a contiguous run of tiles, down the rows of up to eight row tiles
+    // first, so that the tiles that share columns of B or rows of A find them in its L2.  Before / after: 117×512×2048 4.7 / 4.3 µs,
+    // 64×4096×4096 12.3 / 9.0, 6272×256×2304 25.6 / 20.7.  (Without the groups of eight, 4096×512×2048 went from 18.7 to 26.6.)
+    const int grid = static_cast<int>(gridDim.x), xcd = static_cast<int>(blockIdx.x) & 7;
+    int run = xcd * (grid >> 3) + min(xcd, grid & 7) + (static_cast<int>(blockIdx.x) >> 3), first_m = 0, rows = p.tiles_m;
+    if (p.tiles_m > 8) {
+        const int group_tiles = 8 * (grid / p.tiles_m), group = run / group_tiles;
+        run -= group * group_tiles;
+        first_m = group * 8;
+        rows = min(p.tiles_m - first_m, 8);
+    }
+    const int tile_n = run / rows, tile_m = first_m + run - tile_n * rows;
     const int m0 = tile_m * BM, n0 = tile_n * BN;
     const int k_tiles = K / 64, per_wave = (k_tiles + WAVES - 1) / WAVES;
     const int first = wave * per_wave, count = max(0, min(k_tiles, first + per_wave) - first);

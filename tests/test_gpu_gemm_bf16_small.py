@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
     (117, 512, 512), (117, 1536, 512), (65, 504, 576),  # a stage a wavefront; nine k-tiles over eight wavefronts
     (40, 500, 512), (40, 257, 1024),                  # rows of B off 16-byte boundaries (packed first); an odd width
     (117, 512, 2048), (64, 768, 3136),                # several stages a wavefront, an uneven last share
-    (1024, 512, 2048), (600, 1000, 448), (2048, 300, 640),  # 64×64 tiles
+    (1024, 512, 2048), (600, 1000, 448), (2048, 300, 640),  # 64×64 tiles; groups of eight row tiles, a ragged last one
+    (545, 72, 256),                                   # a grid that eight does not divide, a group of one or two row tiles
 ])
 def test_small_tiles(hip, m, n, k):
     """Both layouts of B, plain and with scale-free bias + residual + GELU into both outputs, against float64.  The bound: the
