@@ -698,13 +698,13 @@ __device__ __forceinline__ float largest8(const float (&x)[8], float so_far)
 // [key_first, key_end) on the f32 matrix cores, operands straight from memory, in the units of the split kernel.  Keys that
 // some of the rows do not see, and the last ones short of 32, are taken one by one, so that a value behind a row's mask never
 // meets it (zero times infinity).
+// Leaves this lane's outputs of its row before the division, and the row's reference maximum and sum.
 template <int DPAD, bool CAUSAL, bool BIAS>
-__device__ void redo_rows(const AttnArgs &p, int ctx, int wq0, int lane, int split, int key_first, int key_end, float scale_log2e,
-                          float exp_scale)
+__device__ void redo_sums(const AttnArgs &p, int ctx, int wq0, int lane, int key_first, int key_end, float scale_log2e, float exp_scale,
+                          f32x16 (&o)[DPAD / 32], float &top, float &sum)
 {
     constexpr int CHUNKS = DPAD / 8, DT = DPAD / 32;
     const int S = p.S, D = p.D, li = lane & 31, lh = lane >> 5, my_q = wq0 + li;
-    if (wq0 >= S) return;
     const size_t first = static_cast<size_t>(ctx) * S * D;
     const float *const keys = p.k + first, *const values = p.v + first;
     auto load4 = [&](const float *row, int chunk) {  // this half's four of eight dimensions (D is a multiple of 4 here)
@@ -719,7 +719,6 @@ __device__ void redo_rows(const AttnArgs &p, int ctx, int wq0, int lane, int spl
         return fmaf(logit, scale_log2e, bias * kLog2e);
     };
     f32x4 q[CHUNKS];
-    f32x16 o[DT];
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) {
         q[c] = load4(p.q + row * D, c);
@@ -727,7 +726,8 @@ __device__ void redo_rows(const AttnArgs &p, int ctx, int wq0, int lane, int spl
     }
 #pragma unroll
     for (int t = 0; t < DT; ++t) o[t] = f32x16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    float top = -INFINITY, sum = 0.0f;
+    top = -INFINITY;
+    sum = 0.0f;
     auto rescale = [&](float logit) {  // to the running maximum with `logit` in it; returns what an exponent is shifted by
         const float new_top = fmaxf(top, logit), safe = new_top == -INFINITY ? 0.0f : new_top;
         const float alpha = __builtin_amdgcn_exp2f((top - safe) * exp_scale);
@@ -785,6 +785,19 @@ __device__ void redo_rows(const AttnArgs &p, int ctx, int wq0, int lane, int spl
             for (int e = 0; e < 4; ++e) o[c / 4][c % 4 * 4 + e] = fmaf(weight, v4[e], o[c / 4][c % 4 * 4 + e]);
         }
     }
+}
+
+template <int DPAD, bool CAUSAL, bool BIAS>
+__device__ void redo_rows(const AttnArgs &p, int ctx, int wq0, int lane, int split, int key_first, int key_end, float scale_log2e,
+                          float exp_scale)
+{
+    constexpr int CHUNKS = DPAD / 8, DT = DPAD / 32;
+    const int S = p.S, D = p.D, li = lane & 31, lh = lane >> 5, my_q = wq0 + li;
+    if (wq0 >= S) return;
+    const size_t first = static_cast<size_t>(ctx) * S * D;
+    f32x16 o[DT];
+    float top, sum;
+    redo_sums<DPAD, CAUSAL, BIAS>(p, ctx, wq0, lane, key_first, key_end, scale_log2e, exp_scale, o, top, sum);
     if (my_q >= S) return;
     const bool partial = p.key_splits > 1;
     const size_t at = (static_cast<size_t>(split) * p.contexts + ctx) * S + my_q;
@@ -1101,6 +1114,225 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_split_kernel(AttnArg
     }
     if (pass + 1 < passes) __syncthreads();  // any_wild and the stages are written again
     }  // pass
+}
+
+// -------------------------------------------------------------------------------------------------
+// The split kernel's arithmetic for few queries: 32 of them a workgroup, and the keys dealt out to its eight wavefronts in tiles
+// of 32 (wavefront w takes tiles w, w + 8, ...), whose maxima, sums and outputs are put together through LDS.  One launch, no scratch,
+// and an eighth of the chain of a wavefront that takes all keys; K and V come straight from memory in the order of the matrix
+// instructions' operands and are cut in registers, so that nothing waits for another wavefront before the end.  The next tile's
+// K is requested behind this one's logits, its V behind the outputs.
+// -------------------------------------------------------------------------------------------------
+constexpr int kKeysWaves = 8, kKeysRows = 32;
+
+template <int DPAD, bool CAUSAL, bool BIAS>
+__global__ __launch_bounds__(64 * kKeysWaves) void attention_f32_keys_kernel(AttnArgs p)
+{
+    constexpr int QSTEPS = DPAD / 16, DT = DPAD / 32, OS = DPAD + 4, STRIDE = 32 * kKeysWaves;
+    constexpr float kWild = 0x1p40f, kScale = 0x1p24f, kUnscale = 0x1p-48f;
+    extern __shared__ __attribute__((aligned(16))) float keys_lds[];  // [wave][32 rows][OS], maxima and sums [wave][32]
+    float *const maxima = keys_lds + kKeysWaves * 32 * OS, *const sums = maxima + kKeysWaves * 32;
+    __shared__ int any_wild;
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 31, lh = lane >> 5;
+    const int S = p.S, D = p.D;
+    // the longest rows of all contexts first
+    const int item = static_cast<int>(blockIdx.x) / p.key_splits, split = static_cast<int>(blockIdx.x) - item * p.key_splits;
+    const int q_tile = p.q_tiles - 1 - item / p.contexts, ctx = item % p.contexts;
+    const int q0 = q_tile * kKeysRows, my_q = q0 + li;
+    const int key_first = split * p.keys_per_split, key_end = min(CAUSAL ? min(S, q0 + kKeysRows) : S, key_first + p.keys_per_split);
+    const size_t ctx_elem0 = static_cast<size_t>(ctx) * S * D;
+    const unsigned ctx_bytes = static_cast<unsigned>(S) * static_cast<unsigned>(D) * 4u;
+    const __amdgpu_buffer_rsrc_t rsrc_q =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.q + ctx_elem0), 0, static_cast<int>(ctx_bytes), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc_k =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.k + ctx_elem0), 0, static_cast<int>(ctx_bytes), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc_v =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.v + ctx_elem0), 0, static_cast<int>(ctx_bytes), 0x00020000);
+    const unsigned long long bias_values = static_cast<unsigned long long>(S) * S;
+    const __amdgpu_buffer_rsrc_t rsrc_ab = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(p.attn_bias + (BIAS && p.attn_bias ? ctx * bias_values : 0)), 0,
+        BIAS && p.attn_bias ? static_cast<int>(bias_values * 4) : 0, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc_zb = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(p.z_bias + (BIAS && p.z_bias ? static_cast<size_t>(ctx) * S : 0)), 0, BIAS && p.z_bias ? S * 4 : 0, 0x00020000);
+    constexpr unsigned kOutside = 0x80000000u;  // beyond every context: reads as zero
+    auto load8 = [&](const __amdgpu_buffer_rsrc_t &rsrc, int row, int d, u32x4_t (&x)[2]) {
+        const unsigned at = (static_cast<unsigned>(row) * D + d) * 4u;
+        x[0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, d < D ? at : kOutside, 0, 0);  // (rows past the end: outside as well)
+        x[1] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, d + 4 < D ? at + 16u : kOutside, 0, 0);
+    };
+    auto cut = [](const u32x4_t (&raw)[2], float sign, float scale, float &top, bf16x8 (&pieces)[3]) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = __uint_as_float(raw[e >> 2][e & 3]);
+        top = largest8(x, top);
+        u32x4_t piece[3];
+        split8(x, piece, sign * scale);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) pieces[i] = __builtin_bit_cast(bf16x8, piece[i]);
+    };
+
+    u32x4_t rk[QSTEPS][2], rv[DT][2][2];
+    auto load_k = [&](int key0) {  // lane (li, lh): K[key0 + li][16c + 8·lh .. + 7]
+#pragma unroll
+        for (int c = 0; c < QSTEPS; ++c) load8(rsrc_k, key0 + li, c * 16 + lh * 8, rk[c]);
+    };
+    auto load_v = [&](int key0) {  // V[the eight keys of this half in a step of sixteen][32·dt + li]
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+            const int d = dt * 32 + li;
+            const unsigned at = d < D ? (static_cast<unsigned>(key0 + lh * 4) * D + d) * 4u : kOutside;
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    rv[dt][j][e >> 2][e & 3] =
+                        __builtin_amdgcn_raw_buffer_load_b32(rsrc_v, at + (j * 16 + (e >> 2) * 8 + (e & 3)) * (D * 4u), 0, 0);
+        }
+    };
+
+    float top_qk = 0.0f, top_v = 0.0f;  // largest magnitudes this lane has cut
+    bf16x8 qf[QSTEPS][3];
+    {
+        u32x4_t rq[QSTEPS][2];
+#pragma unroll
+        for (int c = 0; c < QSTEPS; ++c) load8(rsrc_q, my_q, c * 16 + lh * 8, rq[c]);
+        load_k(key_first + wave * 32);
+        load_v(key_first + wave * 32);
+#pragma unroll
+        for (int c = 0; c < QSTEPS; ++c) cut(rq[c], p.scale < 0.0f ? -1.0f : 1.0f, 1.0f, top_qk, qf[c]);
+    }
+    f32x16 oacc[DT];
+#pragma unroll
+    for (int t = 0; t < DT; ++t) oacc[t] = f32x16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float run_max = -INFINITY, run_sum = 0.0f;
+    const float scale_log2e = fmaxf(fabsf(p.scale) * kLog2e, 1e-30f);
+    const float exp_scale = BIAS ? 1.0f : scale_log2e;
+    const float lag = 8.0f / exp_scale;
+    const int last_key = CAUSAL ? min(my_q, S - 1) : S - 1;
+    constexpr int kFirst[6] = {2, 1, 1, 0, 0, 0}, kSecond[6] = {0, 0, 1, 1, 2, 0};  // as in the kernel above, smallest first
+    if (tid == 0) any_wild = 0;
+    for (int key0 = key_first + wave * 32; key0 < key_end; key0 += STRIDE) {
+        u32x4_t ab4[BIAS ? 4 : 1], zb4[BIAS ? 4 : 1];
+        if constexpr (BIAS) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {  // (past the end of a row whatever is there: those keys are masked)
+                const unsigned key = key0 + g * 8 + lh * 4;
+                ab4[g] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_ab, (static_cast<unsigned>(my_q) * S + key) * 4u, 0, 0);
+                zb4[g] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_zb, key * 4u, 0, 0);
+            }
+        }
+        f32x16 score = f32x16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < QSTEPS; ++c) {
+            bf16x8 kf[3];
+            cut(rk[c], 1.0f, 1.0f, top_qk, kf);
+#pragma unroll
+            for (int i = 0; i < 6; ++i) score = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kFirst[i]], qf[c][kSecond[i]], score, 0, 0, 0);
+        }
+        if constexpr (BIAS) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                score[r] = fmaf(score[r], scale_log2e, (__uint_as_float(ab4[r >> 2][r & 3]) + __uint_as_float(zb4[r >> 2][r & 3])) * kLog2e);
+        }
+        load_k(key0 + STRIDE);
+        if (key0 + 32 > S || (CAUSAL && key0 + 31 > q0)) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (key0 + (r >> 2) * 8 + lh * 4 + (r & 3) > last_key) score[r] = -INFINITY;
+        }
+        float tile_max = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) tile_max = fmaxf(tile_max, score[r]);
+        tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32));
+        if (__any(tile_max > run_max + lag)) {
+            const float new_max = fmaxf(run_max, tile_max);
+            const float alpha = __builtin_amdgcn_exp2f((run_max - (new_max == -INFINITY ? 0.0f : new_max)) * exp_scale);
+            run_sum *= alpha;
+#pragma unroll
+            for (int t = 0; t < DT; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) oacc[t][r] *= alpha;
+            run_max = new_max;
+        }
+        const float shift = -(run_max == -INFINITY ? 0.0f : run_max) * exp_scale;
+        float tile_sum = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            float pr[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                pr[e] = __builtin_amdgcn_exp2f(fmaf(score[8 * j + e], exp_scale, shift));
+                tile_sum += pr[e];
+            }
+            u32x4_t piece[3];
+            split8(pr, piece, kScale);
+            bf16x8 pf[3], vf[DT][3];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) pf[i] = __builtin_bit_cast(bf16x8, piece[i]);
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) cut(rv[dt][j], 1.0f, kScale, top_v, vf[dt]);
+#pragma unroll
+            for (int i = 0; i < 6; ++i)
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+                    oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[dt][kFirst[i]], pf[kSecond[i]], oacc[dt], 0, 0, 0);
+        }
+        run_sum += tile_sum;
+        load_v(key0 + STRIDE);
+    }
+    __syncthreads();
+    if (top_qk >= kWild || top_v * S >= 0x1p70f) any_wild = 1;
+    __syncthreads();
+    run_sum += __shfl_xor(run_sum, 32);
+    float unscale = kUnscale;
+    if (any_wild != 0) {  // a run of keys each, in f32
+        const int per = max(key_end - key_first + kKeysWaves - 1, 0) / kKeysWaves, first = min(key_first + wave * per, key_end);
+        redo_sums<DPAD, CAUSAL, BIAS>(p, ctx, q0, lane, first, min(first + per, key_end), scale_log2e, exp_scale, oacc, run_max, run_sum);
+        unscale = 1.0f;
+    }
+
+    // The eight parts of each row: everything on the scale of the largest maximum, added in the order of the wavefronts.
+    if (lh == 0) {
+        maxima[wave * 32 + li] = run_max;
+        sums[wave * 32 + li] = run_sum;
+    }
+    __syncthreads();
+    float top = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < kKeysWaves; ++w) top = fmaxf(top, maxima[w * 32 + li]);
+    const float mine = unscale * __builtin_amdgcn_exp2f((run_max - (top == -INFINITY ? 0.0f : top)) * exp_scale);  // no keys: 0
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            f32x4 part;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) part[e] = oacc[t][g * 4 + e] * mine;
+            *reinterpret_cast<f32x4 *>(&keys_lds[(wave * 32 + li) * OS + t * 32 + g * 8 + lh * 4]) = part;
+        }
+    __syncthreads();
+    const int row = tid >> 4, d = (tid & 15) * 4;
+    if (q0 + row >= S || d >= D) return;
+    float row_top = -INFINITY, total = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kKeysWaves; ++w) row_top = fmaxf(row_top, maxima[w * 32 + row]);
+    row_top = row_top == -INFINITY ? 0.0f : row_top;
+    f32x4 out = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < kKeysWaves; ++w) {
+        total += sums[w * 32 + row] * __builtin_amdgcn_exp2f((maxima[w * 32 + row] - row_top) * exp_scale);
+        out += *reinterpret_cast<const f32x4 *>(&keys_lds[(w * 32 + row) * OS + d]);
+    }
+    const bool partial = p.key_splits > 1;
+    const size_t at = (static_cast<size_t>(split) * p.contexts + ctx) * S + q0 + row;
+    const float inv = partial ? 1.0f : total > 0.0f ? 1.0f / total : 0.0f;
+    float *const dst = partial ? p.part_o + at * D : p.out + ctx_elem0 + static_cast<size_t>(q0 + row) * D;
+    *reinterpret_cast<float4 *>(dst + d) = make_float4(out[0] * inv, out[1] * inv, out[2] * inv, out[3] * inv);
+    if (partial && d == 0) *reinterpret_cast<float2 *>(p.part_ml + at * 2) = make_float2(total > 0.0f ? row_top : -INFINITY, total);
 }
 
 // -------------------------------------------------------------------------------------------------
@@ -1505,6 +1737,29 @@ int query_rows(size_t contexts, size_t sequence, size_t head_dim, bool causal)
     return contexts * (causal ? (tiles + 1) / 2 : tiles) >= 256 ? 256 : kBQ;
 }
 
+// Room in the stream's scratch for the outputs, maxima and sums of every run of keys.
+hipError_t parts_scratch(AttnArgs &args, hipStream_t stream)
+{
+    const size_t rows = static_cast<size_t>(args.contexts) * args.S;
+    const size_t o_bytes = static_cast<size_t>(args.key_splits) * rows * args.D * sizeof(float);
+    const size_t ml_bytes = static_cast<size_t>(args.key_splits) * rows * 2 * sizeof(float);
+    void *workspace = nullptr;
+    const hipError_t rc = stream_workspace(stream, o_bytes + ml_bytes, &workspace);
+    if (rc != hipSuccess) return rc;
+    args.part_o = static_cast<float *>(workspace);
+    args.part_ml = reinterpret_cast<float *>(static_cast<unsigned char *>(workspace) + o_bytes);
+    return hipSuccess;
+}
+
+hipError_t merge_parts(const AttnArgs &args, bool bias, int causal_r, hipStream_t stream)
+{
+    const float scale_log2e = fmaxf(fabsf(args.scale) * kLog2e, 1e-30f);
+    const size_t work = static_cast<size_t>(args.contexts) * args.S * (args.D / 4);
+    hipLaunchKernelGGL(attention_merge_splits_kernel, dim3(static_cast<unsigned>((work + 255) / 256)), dim3(256), 0, stream, args,
+                       bias ? 1.0f : scale_log2e, causal_r);
+    return hipGetLastError();
+}
+
 // Plans, checks and launches a kernel whose workgroups decode their items with decode_fast_block, and merges the key splits.
 hipError_t launch_planned(void (*kernel)(AttnArgs), unsigned threads, size_t lds_bytes, AttnArgs args, bool causal, bool bias,
                           hipStream_t stream)
@@ -1515,30 +1770,18 @@ hipError_t launch_planned(void (*kernel)(AttnArgs), unsigned threads, size_t lds
     size_t blocks = plan_fast(args, causal, &causal_r);
     hipError_t rc = hipSuccess;
     if (args.key_splits > 1) {
-        const size_t rows = static_cast<size_t>(args.contexts) * args.S;
-        const size_t o_bytes = static_cast<size_t>(args.key_splits) * rows * args.D * sizeof(float);
-        const size_t ml_bytes = static_cast<size_t>(args.key_splits) * rows * 2 * sizeof(float);
-        void *workspace = nullptr;
-        rc = stream_workspace(stream, o_bytes + ml_bytes, &workspace);
+        rc = parts_scratch(args, stream);
         if (scratch_unavailable(rc)) {  // every workgroup takes all keys, slower and without scratch
             args = unplanned;
             blocks = plan_unsplit(args, causal);
         } else if (rc != hipSuccess) {
             return rc;
-        } else {
-            args.part_o = static_cast<float *>(workspace);
-            args.part_ml = reinterpret_cast<float *>(static_cast<unsigned char *>(workspace) + o_bytes);
         }
     }
     if (!fast_plan_consistent(args, causal, blocks)) return hipErrorInvalidConfiguration;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(threads), lds_bytes, stream, args);
     rc = hipGetLastError();
-    if (rc != hipSuccess || args.key_splits == 1) return rc;
-    const float scale_log2e = fmaxf(fabsf(args.scale) * kLog2e, 1e-30f);
-    const size_t work = static_cast<size_t>(args.contexts) * args.S * (args.D / 4);
-    hipLaunchKernelGGL(attention_merge_splits_kernel, dim3(static_cast<unsigned>((work + 255) / 256)), dim3(256), 0, stream, args,
-                       bias ? 1.0f : scale_log2e, causal_r);
-    return hipGetLastError();
+    return rc != hipSuccess || args.key_splits == 1 ? rc : merge_parts(args, bias, causal_r, stream);
 }
 
 template <int DPAD, bool CAUSAL, bool BIAS = false>
@@ -1563,9 +1806,60 @@ hipError_t launch_split_rows(AttnArgs args, hipStream_t stream)
     return launch_planned(kernel, 64 * WAVES, lds_bytes, args, CAUSAL, BIAS, stream);
 }
 
+// How many runs of keys a call of the split kernel's arithmetic is cut into when the wavefronts of 32-row workgroups share them; 0
+// where the wider tiles are the better ones.  A launch of them is one round of a workgroup a compute unit: about 5.5 µs and 1.9 for
+// 128 keys (64 values a head), and 4.5 for the second launch that puts runs together.  Before / after, 64 values: 1 × 250 17.6 / 10.0 µs
+// (causal 27.7 / 9.8), 1 × 1000 15.4 / 12.6 (biased 16.8 / 13.3), 4 × 500 15.4 / 12.8, 8 × 1000 27.4 / 24.8, 32 × 250 18.0 / 10.8; the error
+// against float64 3.2e-7 / 2.4e-7.  Beyond a round or some length the 128-row tiles, which read K and V a quarter as often and cut
+// them once for four wavefronts, are level or ahead: 32 × 500 26.2 / 27.6, 4 × 1000 in one run each 20.3 / 22.7, 1 × 2048 20.8 / 34.8;
+// up to 32 queries, where one wavefront has all keys, they have less to put together: 8 × 16 5.8 / 6.7.
+size_t keys_shared(size_t contexts, size_t sequence, size_t *keys_per_split)
+{
+    const size_t workgroups = contexts * ((sequence + kKeysRows - 1) / kKeysRows);
+    if (sequence <= 32 || workgroups > 256) return 0;
+    auto us = [&](size_t splits, size_t keys) { return 5.5 + 1.9 * static_cast<double>((keys + 127) / 128) + (splits > 1 ? 4.5 : 0.0); };
+    size_t best = 1, best_keys = sequence;
+    for (size_t splits = 2; splits * workgroups <= 256 && splits * 128 < sequence + 128; ++splits) {
+        const size_t keys = std::max<size_t>(128, ((sequence + splits - 1) / splits + 63) / 64 * 64);
+        if (keys <= 256 && (splits - 1) * keys < sequence && us(splits, keys) < us(best, best_keys)) best = splits, best_keys = keys;
+    }
+    *keys_per_split = best_keys;
+    return best_keys <= 512 || (workgroups > 128 && sequence <= 1024) ? best : 0;
+}
+
+template <int DPAD, bool CAUSAL, bool BIAS>
+hipError_t launch_keys(AttnArgs args, hipStream_t stream)
+{
+    constexpr size_t lds_bytes = kKeysWaves * 32 * (DPAD + 4 + 2) * sizeof(float);
+    auto kernel = attention_f32_keys_kernel<DPAD, CAUSAL, BIAS>;
+    hipError_t rc = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                              static_cast<int>(lds_bytes));
+    if (rc != hipSuccess) return rc;
+    args.q_tiles = (args.S + kKeysRows - 1) / kKeysRows;
+    if (args.key_splits > 1) {
+        const hipError_t scratch = parts_scratch(args, stream);
+        if (scratch_unavailable(scratch)) {  // every workgroup takes all keys, slower and without scratch
+            args.key_splits = 1;
+            args.keys_per_split = args.S;
+        } else if (scratch != hipSuccess) {
+            return scratch;
+        }
+    }
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(args.contexts) * args.q_tiles * args.key_splits), dim3(64 * kKeysWaves), lds_bytes,
+                       stream, args);
+    rc = hipGetLastError();
+    return rc != hipSuccess || args.key_splits == 1 ? rc : merge_parts(args, BIAS, 0, stream);
+}
+
 template <int DPAD, bool CAUSAL, bool BIAS>
 hipError_t launch_split(AttnArgs args, hipStream_t stream)
 {
+    size_t keys = 0;
+    if (const size_t splits = keys_shared(args.contexts, args.S, &keys)) {
+        args.key_splits = static_cast<int>(splits);
+        args.keys_per_split = static_cast<int>(keys);
+        return launch_keys<DPAD, CAUSAL, BIAS>(args, stream);
+    }
     if (args.bq == 256) return launch_split_rows<DPAD, CAUSAL, BIAS, 8>(args, stream);
     return launch_split_rows<DPAD, CAUSAL, BIAS, 4>(args, stream);
 }
@@ -1624,6 +1918,15 @@ AttentionPlanReport attention_f32_plan_report(size_t contexts, size_t sequence, 
     if (report.kernel == ST_HIP_ATTN_KERNEL_GENERAL) {  // one workgroup per (context, query tile), decoded by division
         report.workgroups = contexts * static_cast<size_t>(args.q_tiles);
         report.items = report.items_expected = report.workgroups;
+        return report;
+    }
+    size_t keys = 0, runs = 0;
+    if (report.kernel == ST_HIP_ATTN_KERNEL_SPLIT && (runs = keys_shared(contexts, sequence, &keys)) > 0) {  // decoded by division
+        report.workgroups = contexts * ((sequence + kKeysRows - 1) / kKeysRows) * runs;
+        report.key_splits = static_cast<int>(runs);
+        report.keys_per_split = static_cast<int>(keys);
+        report.items = report.items_expected = report.workgroups;
+        report.consistent = 1;
         return report;
     }
     int causal_r = 0;

@@ -137,3 +137,13 @@ def test_redone_rows_take_the_matrix_cores(hip):
             return min(times)
 
         assert best(d_wild) <= 15 * best(d_q)
+
+
+# Keys shared by eight wavefronts of 32-row workgroups: its first and last sequences, wavefronts without keys, a run short of a tile,
+# runs of keys put together by a second launch (rows that see none of a run), a grid of exactly one round and the first beyond it.
+@pytest.mark.parametrize("contexts,seq,dim,causal,biased", [
+    (1, 32, 64, True, False), (1, 33, 64, True, True), (3, 63, 20, False, True), (2, 97, 64, True, False), (1, 255, 64, False, True),
+    (4, 256, 32, True, False), (1, 289, 60, True, True), (3, 385, 64, True, False), (1, 1000, 32, True, True), (2, 999, 64, False, True),
+    (32, 256, 64, True, False), (33, 256, 64, True, False), (7, 1024, 64, False, False)])
+def test_keys_shared_by_the_wavefronts(hip, contexts, seq, dim, causal, biased):
+    test_against_float64(hip, contexts, seq, dim, causal, biased)
