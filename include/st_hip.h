@@ -98,8 +98,8 @@ int st_hip_device_synchronize(void);
  * that a graph may hold is not freed when the stream's scratch grows past it, only with the stream or by
  * st_hip_release_scratch; the graph must not be replayed after that.  What is kept is what the largest call on a stream
  * needed, up to 2 GiB of re-laid operands for f32 products and convolutions beside the partial sums.  st_hip_release_scratch waits for `stream` (NULL = the default
- * stream, which is never destroyed) and frees every scratch buffer kept for it; no other thread may be launching on
- * that stream meanwhile.  st_hip_scratch_buffer_count reports how many buffers are held in all.  No reference
+ * stream, which is never destroyed) and frees every scratch buffer kept for it, and the pinned host memory (up to 64 MiB) that
+ * is kept for copies between calls; no other thread may be launching on that stream meanwhile.  st_hip_scratch_buffer_count reports how many buffers are held in all.  No reference
  * counterpart: the reference allocates and frees per call (crates/st-backend-hip/src/real.rs:718-756). */
 int st_hip_release_scratch(void *stream);
 size_t st_hip_scratch_buffer_count(void);
@@ -261,7 +261,8 @@ int st_hip_attention_f32_scaled_launch_plan(size_t contexts, size_t sequence, si
                                             st_hip_attention_plan *plan);
 /* The same for the 256-row bf16 GEMM kernels, whose workgroups decode their index into (k-split, tile): the tiling and
  * k-split launch_gemm would use for an m×n×k product (k a multiple of 64), the launcher's own check (`consistent`) and a
- * walk over the whole grid (`items` must equal `workgroups`, `out_of_range` and `duplicates` must be 0). */
+ * walk over the whole grid (`items` must equal `workgroups`, `out_of_range` and `duplicates` must be 0).  Small products that
+ * other kernels take, and the columns behind the last full round that a second launch takes, are described as if they were not. */
 typedef struct {
     int tile_cols;          /* 256 or 128 columns per tile (256 rows) */
     int tiles_m, tiles_n;

@@ -241,6 +241,7 @@ struct PinnedBuffer {
 constexpr size_t kPinnedIdleBytes = 64u << 20;
 bool pinned_acquire(size_t bytes, PinnedBuffer *out);
 void pinned_release(const PinnedBuffer &buffer);
+void pinned_release_idle();  // frees what no call holds
 bool is_pinned(const void *host);
 // The most a copy goes through pinned memory with.
 constexpr size_t kStageMost = 16u << 20;

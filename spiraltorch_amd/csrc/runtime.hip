@@ -162,6 +162,18 @@ void pinned_release(const PinnedBuffer &buffer)
     (void)hipHostFree(buffer.ptr);
 }
 
+void pinned_release_idle()
+{
+    PinnedPool &pool = pinned_pool();
+    std::vector<PinnedBuffer> doomed;
+    {
+        std::lock_guard<std::mutex> lock(pool.mutex);
+        doomed.swap(pool.idle);
+        pool.idle_bytes = 0;
+    }
+    for (const PinnedBuffer &buffer : doomed) (void)hipHostFree(buffer.ptr);
+}
+
 namespace {
 // Scratch is keyed by (stream, host thread, slot): launches on one stream from one thread are ordered, so they never
 // use the buffer at the same time; two host threads that share a stream (every caller that passes none shares the
@@ -495,6 +507,7 @@ int st_hip_release_scratch(void *stream)
     ST_HIP_CHECK(ensure_init());
     ST_HIP_TRY(hipStreamSynchronize(as_stream(stream)), "hipStreamSynchronize");
     release_stream_workspace(as_stream(stream));
+    pinned_release_idle();
     return ST_HIP_OK;
 }
 

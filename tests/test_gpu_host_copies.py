@@ -82,3 +82,10 @@ def test_count_nonfinite(hip, count):
         d_bad = hip.DeviceBuffer.from_array(bad)
         found, first, value = hip.count_nonfinite_f32_dev(count, d_bad.at(4))
         assert (found, first) == (len(places), min(places)) and value == np.inf
+
+
+def test_copies_after_the_kept_memory_was_freed(hip):
+    column, row = np.arange(1, 300, dtype=np.float32), np.arange(1, 200, dtype=np.float32)
+    for _ in range(3):
+        assert (outer(hip, column, row) == column[:, None] * row[None, :]).all()
+        hip.release_scratch()
