@@ -48,8 +48,7 @@ PEAK_HBM_GBS = 8000.0
 MEASURED_TRAFFIC_BYTES = {
     "conv2d_bias_relu_f32_n32_c64to128_56x56_k3s1p1": (14291 * 2 + 50176) * 1024,
     "conv2d_grad_input_f32_n32_c64to128_56x56_k3s1p1": ((32964 + 660) * 2 + 25088 + 288) * 1024,
-    "conv2d_grad_weight_f32_n32_c64to128_56x56_k3s1p1": ((44801 + 12109) * 2 + 24192 + 288) * 1024,
-    "conv2d_bias_relu_bf16_f32acc_n32_c64to128_56x56_k3s1p1": ((12703 + 8123) * 2 + 13600 + 50176) * 1024,
+    "conv2d_bias_relu_bf16_f32acc_n32_c64to128_56x56_k3s1p1": ((7921 + 8022) * 2 + 13600 + 50176) * 1024,
     "gemm_bf16_f32acc_4096x4096x4096": (98511 * 2 + 65536) * 1024,
     "gemm_bf16_f32acc_4096x4096x4096_prepacked_rhs": (98406 * 2 + 65536) * 1024,
     "gemm_bf16_f32acc_16x4096x4096": ((16927 + 1045) * 2 + 2048 + 256) * 1024,
@@ -66,6 +65,7 @@ MEASURED_TRAFFIC_BYTES = {
 # The same for workloads that run as products of bf16 pieces: the pass that writes the pieces (6 bytes a value) included.
 PIECES_TRAFFIC_BYTES = {
     "conv2d_bias_relu_f32_n32_c64to128_56x56_k3s1p1": ((16250 + 22269) * 2 + 40924 + 50176) * 1024,
+    "conv2d_grad_weight_f32_n32_c64to128_56x56_k3s1p1": ((40920 + 12257) * 2 + 24480 + 288) * 1024,
     "attention_f32_b8_h16_s2048_d64_noncausal": (98416 * 2 + 65536) * 1024,
     "attention_f32_b8_h16_s2048_d64_causal": (160096 * 2 + 65536) * 1024,
     "attention_f32_attn_bias_c1_s2048_d64": ((10898 + 4260) * 2 + 8448 + 512) * 1024,
@@ -234,7 +234,7 @@ def wl_conv2d_backward(hip, inputs, timer, which):
         bytes_ = 4 * (g.size + wt.size + x.size)
     wall, ev, sus = timer.measure(step)
     flops = 2 * batch * c_out * h * w * c_in * 9
-    pieces = which == "grad_input" and bool(hip.conv2d_f32_split_plan(batch, c_in, h, w, c_out, *geom, direction="grad_input")["served"])
+    pieces = which == "grad_weight" or bool(hip.conv2d_f32_split_plan(batch, c_in, h, w, c_out, *geom, direction="grad_input")["served"])
     return entry(f"conv2d_{which}_f32_n32_c64to128_56x56_k3s1p1", "f32", flops, bytes_, "mfma", wall, ev, sustained=sus, pieces=pieces)
 
 
