@@ -2543,9 +2543,14 @@ hipError_t launch_gemm_bf16(size_t m, size_t n, size_t k, const uint16_t *lhs, c
     size_t workspace_offset = 0;
     // Few rows or few columns: small tiles with k split inside the workgroup.  (A row-major B of up to 64 rows and a long k
     // stays with the skinny kernel, which reads it in longer pieces: 64×768×3072 8.6 µs against 9.9.)
-    if (aligned16(lhs) && aligned16(rhs) && fits_buffer && small_tiles_apply(m, n, k) && !(skinny && k > 1024)) {
-        if (rhs_packed || n % 8 == 0) return launch_gemm_bf16_small(m, n, k, lhs, rhs, rhs_packed, out_f32, out_bf16, epilogue, stream);
-        // rows of B that start at any 2-byte boundary: packed first, one pass
+    // Rows of B that start at any 2-byte boundary are packed first, a pass of about 1.9 µs for a million values: up to 64 rows, the general
+    // kernel, which reads B once as it is, is ahead beyond ten million (seven up to 16 rows), and in a single k-tile.  Packed / general:
+    // 1×6853×6144 84.7 / 46.6 µs, 8×4001×2048 23.9 / 22.3, 33×6853×2048 41.7 / 38.5, 1×1953×64 7.9 / 6.5; 3×4001×1024 15.7 / 21.2,
+    // 33×4001×2048 24.2 / 27.5, 8×1001×256 7.7 / 12.4.
+    const size_t packing_most = m > 64 ? SIZE_MAX : m > 16 ? 10'000'000 : 7'000'000;
+    const bool as_it_is = rhs_packed || n % 8 == 0, packing_pays = n * k <= packing_most && (k > 64 || (m > 16 && m * n <= 1'000'000));
+    if (aligned16(lhs) && aligned16(rhs) && fits_buffer && small_tiles_apply(m, n, k) && !(skinny && k > 1024) && (as_it_is || packing_pays)) {
+        if (as_it_is) return launch_gemm_bf16_small(m, n, k, lhs, rhs, rhs_packed, out_f32, out_bf16, epilogue, stream);
         void *workspace = nullptr;
         hipError_t rc = stream_workspace(stream, k * n * sizeof(uint16_t), &workspace);
         if (rc != hipSuccess) return rc;
