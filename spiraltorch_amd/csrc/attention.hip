@@ -1812,11 +1812,12 @@ hipError_t launch_split_rows(AttnArgs args, hipStream_t stream)
 // (causal 27.7 / 9.8), 1 × 1000 15.4 / 12.6 (biased 16.8 / 13.3), 4 × 500 15.4 / 12.8, 8 × 1000 27.4 / 24.8, 32 × 250 18.0 / 10.8; the error
 // against float64 3.2e-7 / 2.4e-7.  Beyond a round or some length the 128-row tiles, which read K and V a quarter as often and cut
 // them once for four wavefronts, are level or ahead: 32 × 500 26.2 / 27.6, 4 × 1000 in one run each 20.3 / 22.7, 1 × 2048 20.8 / 34.8;
-// up to 32 queries, where one wavefront has all keys, they have less to put together: 8 × 16 5.8 / 6.7.
-size_t keys_shared(size_t contexts, size_t sequence, size_t *keys_per_split)
+// up to 32 queries (64 with biases), where one or two wavefronts have all keys, they have less to put together: 8 × 16 5.8 / 6.7,
+// 6 × 40 biased 7.2 / 7.6.
+size_t keys_shared(size_t contexts, size_t sequence, bool biased, size_t *keys_per_split)
 {
     const size_t workgroups = contexts * ((sequence + kKeysRows - 1) / kKeysRows);
-    if (sequence <= 32 || workgroups > 256) return 0;
+    if (sequence <= (biased ? 64 : 32) || workgroups > 256) return 0;
     auto us = [&](size_t splits, size_t keys) { return 5.5 + 1.9 * static_cast<double>((keys + 127) / 128) + (splits > 1 ? 4.5 : 0.0); };
     size_t best = 1, best_keys = sequence;
     for (size_t splits = 2; splits * workgroups <= 256 && splits * 128 < sequence + 128; ++splits) {
@@ -1855,7 +1856,7 @@ template <int DPAD, bool CAUSAL, bool BIAS>
 hipError_t launch_split(AttnArgs args, hipStream_t stream)
 {
     size_t keys = 0;
-    if (const size_t splits = keys_shared(args.contexts, args.S, &keys)) {
+    if (const size_t splits = keys_shared(args.contexts, args.S, BIAS, &keys)) {
         args.key_splits = static_cast<int>(splits);
         args.keys_per_split = static_cast<int>(keys);
         return launch_keys<DPAD, CAUSAL, BIAS>(args, stream);
@@ -1921,7 +1922,7 @@ AttentionPlanReport attention_f32_plan_report(size_t contexts, size_t sequence, 
         return report;
     }
     size_t keys = 0, runs = 0;
-    if (report.kernel == ST_HIP_ATTN_KERNEL_SPLIT && (runs = keys_shared(contexts, sequence, &keys)) > 0) {  // decoded by division
+    if (report.kernel == ST_HIP_ATTN_KERNEL_SPLIT && (runs = keys_shared(contexts, sequence, biased, &keys)) > 0) {  // decoded by division
         report.workgroups = contexts * ((sequence + kKeysRows - 1) / kKeysRows) * runs;
         report.key_splits = static_cast<int>(runs);
         report.keys_per_split = static_cast<int>(keys);
