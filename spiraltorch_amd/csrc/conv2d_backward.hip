@@ -253,7 +253,7 @@ constexpr int kGradWeightStages = 2 * 3 * (64 * (TM + TN) * 32 + 256);  // two s
 enum class Gather {
     kValues,   // G and patches value by value: a G below four values an image
     kTaps,     // patches value by value
-    kWindows,  // patches by windows: no stride and rows that are a multiple of four pixels
+    kWindows,  // patches by windows: no stride, and rows that are a multiple of four pixels or the whole image
 };
 
 template <Gather GATHER, int TM, int TN>
@@ -797,6 +797,13 @@ hipError_t launch_conv2d_grad_weight_f32(const ConvShape &shape, const float *in
     args.s = shape;
     args.S = S;
     args.spatial = shape.oh * shape.ow;
+    const bool unit = shape.stride_h == 1 && shape.stride_w == 1;
+    // A kernel of one tap that reads every pixel: the image is one long row, whose end is its only border.
+    const bool one_row = unit && shape.kh == 1 && shape.kw == 1 && shape.pad_h == 0 && shape.pad_w == 0;
+    if (one_row) {
+        args.s.h = args.s.oh = 1;
+        args.s.w = args.s.ow = args.spatial;
+    }
     // 128 × 192 tiles when they waste little (every output channel and column a tile covers beyond the matrix is
     // arithmetic thrown away), 64 × 64 tiles otherwise.
     const long long big_cover = static_cast<long long>((shape.c_out + 127) / 128 * 128) * ((S + 191) / 192 * 192);
@@ -822,10 +829,11 @@ hipError_t launch_conv2d_grad_weight_f32(const ConvShape &shape, const float *in
     if (workgroups > 0x7ffffff0u) return hipErrorInvalidConfiguration;
     args.workgroups = static_cast<int>(workgroups);
     const dim3 grid(static_cast<unsigned>((workgroups + 7) / 8 * 8));
-    // Windows need the four pixels of a thread in one output row and neighbouring columns of the input, and an image that holds one.
+    // Windows need the four pixels of a thread in one output row (of one row, the last ones may lie beyond it: the input's column is then
+    // beyond its row as well) and neighbouring columns of the input, and an image that holds one.
     // (Rows of other widths as two windows, the second for the pixels in the next row: 111 instead of 75 µs for 256 -> 256 channels at
     // 14×14, and between 4 % less and 10 % more in the small tile.)
-    const bool windows = shape.stride_h == 1 && shape.stride_w == 1 && shape.ow % 4 == 0 && image_floats >= 4;
+    const bool windows = unit && (one_row || shape.ow % 4 == 0) && image_floats >= 4;
     const Gather gather = static_cast<size_t>(shape.c_out) * args.spatial < 4 ? Gather::kValues : windows ? Gather::kWindows : Gather::kTaps;
     auto kernel = gather == Gather::kValues    ? conv_grad_weight_kernel<Gather::kValues>
                   : gather == Gather::kWindows ? (big ? conv_grad_weight_big_kernel<Gather::kWindows> : conv_grad_weight_kernel<Gather::kWindows>)

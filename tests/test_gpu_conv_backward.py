@@ -371,6 +371,11 @@ GRAD_WEIGHT_CASES = [
     (3, 64, 7, 7, 128, (3, 3), (1, 1), (1, 1), (1, 1)),
     (2, 64, 14, 14, 128, (3, 3), (1, 1), (1, 1), (1, 1)),
     (2, 64, 15, 16, 128, (3, 3), (2, 1), (1, 1), (1, 1)),
+    # one tap over every pixel: an image as one row, of a length that is no multiple of four and of one below a window
+    (3, 64, 13, 13, 64, (1, 1), (1, 1), (0, 0), (1, 1)),
+    (2, 200, 7, 11, 130, (1, 1), (1, 1), (0, 0), (1, 1)),
+    (2, 1, 3, 1, 5, (1, 1), (1, 1), (0, 0), (1, 1)),
+    (2, 2, 3, 1, 5, (1, 1), (1, 1), (0, 0), (1, 1)),
     # a gradient below one window of four, and one that is exactly one
     (5, 3, 2, 5, 1, (2, 3), (1, 1), (0, 0), (1, 1)),
     (5, 3, 2, 6, 1, (2, 3), (1, 1), (0, 0), (1, 1)),
