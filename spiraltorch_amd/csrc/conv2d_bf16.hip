@@ -507,9 +507,11 @@ hipError_t launch_conv2d_bf16(const ConvShape &c, int activation, const uint16_t
     hipLaunchKernelGGL(conv_bf16_chunks_kernel, dim3(static_cast<unsigned>(image_groups + weight_groups + 1)), dim3(256), 0, stream, args);
     rc = hipGetLastError();
     if (rc != hipSuccess) return rc;
-    rc = hipFuncSetAttribute(reinterpret_cast<const void *>(config.kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                             static_cast<int>(config.lds_bytes()));
-    if (rc != hipSuccess) return rc;
+    if (config.lds_bytes() > 64 * 1024) {  // more than a launch may take unasked
+        rc = hipFuncSetAttribute(reinterpret_cast<const void *>(config.kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 static_cast<int>(config.lds_bytes()));
+        if (rc != hipSuccess) return rc;
+    }
     hipLaunchKernelGGL(config.kernel, dim3(static_cast<unsigned>(workgroups)), dim3(static_cast<unsigned>(config.waves) * 64),
                        config.lds_bytes(), stream, args);
     rc = hipGetLastError();

@@ -308,8 +308,10 @@ hipError_t launch_gemm_bf16_small(size_t m, size_t n, size_t k, const uint16_t *
     const size_t lds = config.waves * config.ring_bytes(k), tiles = config.tiles(m, n);
     if (tiles > 0x7fffffffu || lds > 160 * 1024) return hipErrorInvalidConfiguration;
     auto kernel = rhs_packed ? config.packed : config.rowmajor;
-    const hipError_t rc = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-    if (rc != hipSuccess) return rc;
+    if (lds > 64 * 1024) {  // more than a launch may take unasked; the most any k needs, whatever other threads ask for meanwhile
+        const hipError_t rc = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        if (rc != hipSuccess) return rc;
+    }
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles)), dim3(static_cast<unsigned>(config.waves) * 64), lds, stream, args);
     return hipGetLastError();
 }
