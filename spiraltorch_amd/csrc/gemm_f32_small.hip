@@ -292,9 +292,9 @@ bool gemm_f32_small_applies(size_t m, size_t n, size_t k, bool lhs_transposed, b
     const int layout = lhs_transposed ? 2 : rhs_packed ? 1 : 0;
     const bool any = any_alignment(m, n, k, layout, lhs, rhs);
     const SmallF32Config &c = choose_small(m, n, k, layout, any);
-    // Beyond two rounds the estimates of both sides are a fifth off, and the gain is small where there is one: 635×832×2496 as
-    // A·Bᵀ 43.7 µs against 34.7.
-    return c.us(m, n, k, layout, any) < (c.tiles(m, n) > 512 ? 0.75 : 0.95) * other_us;
+    // Beyond two rounds, and as A·Bᵀ beyond one, the estimates of both sides are a fifth off and the gain is small where there is one:
+    // as A·Bᵀ 635×832×2496 took 43.7 µs against 34.7, 468×640×1920 25.6 against 23.0.
+    return c.us(m, n, k, layout, any) < (c.tiles(m, n) > (layout == 1 ? 256 : 512) ? 0.75 : 0.95) * other_us;
 }
 
 hipError_t launch_gemm_f32_small(size_t m, size_t n, size_t k, bool lhs_transposed, const float *lhs, bool rhs_packed, const float *rhs,
