@@ -103,6 +103,8 @@ int st_hip_device_synchronize(void);
  * counterpart: the reference allocates and frees per call (crates/st-backend-hip/src/real.rs:718-756). */
 int st_hip_release_scratch(void *stream);
 size_t st_hip_scratch_buffer_count(void);
+/* counters[0]: bytes of pinned host memory held for copies, in use or kept; counters[1]: how often such memory has been allocated. */
+int st_hip_pinned_memory_counters(uint64_t *counters);
 /* Timing events recorded on the stream the kernels run on. */
 int st_hip_event_create(void **event);
 int st_hip_event_record(void *event, void *stream);

@@ -91,6 +91,7 @@ SIGNATURES = {
     "st_hip_stream_destroy": (c_int, [c_void_p]),
     "st_hip_release_scratch": (c_int, [c_void_p]),
     "st_hip_scratch_buffer_count": (c_size_t, []),
+    "st_hip_pinned_memory_counters": (c_int, [POINTER(c_uint64)]),
     "st_hip_device_synchronize": (c_int, []),
     "st_hip_event_create": (c_int, [POINTER(c_void_p)]),
     "st_hip_event_record": (c_int, [c_void_p, c_void_p]),

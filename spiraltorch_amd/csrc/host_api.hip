@@ -76,7 +76,7 @@ class Lease {
     {
         if (ws_) {
             if (!drained_) (void)hipStreamSynchronize(ws_->stream);
-            for (const PinnedBuffer &stage : stages_) pinned_release(stage);
+            for (size_t i = 0; i < stage_count_; ++i) pinned_release(stages_[i]);
             pool().release(ws_);
         }
     }
@@ -111,12 +111,11 @@ class Lease {
             // next: the runtime's own copy holds the caller as long and then waits between the engines.
             constexpr size_t kPiece = 256u << 10;
             PinnedBuffer stage;
-            if (bytes > kStageMost || (bytes >= kPiece && is_pinned(host)) || !pinned_acquire(bytes, &stage)) {
+            if (bytes > kUploadMost || (bytes >= kPiece && is_pinned(host)) || !hold(bytes, &stage)) {
                 ST_HIP_TRY(hipMemcpyAsync(*device, host, bytes, hipMemcpyHostToDevice, ws_->stream),
                            "hipMemcpyAsync(H2D)");
                 return ST_HIP_OK;
             }
-            stages_.push_back(stage);
             for (size_t at = 0; at < bytes; at += kPiece) {
                 const size_t piece = std::min(kPiece, bytes - at);
                 unsigned char *const pinned = static_cast<unsigned char *>(stage.ptr) + at;
@@ -130,33 +129,12 @@ class Lease {
     {
         if (bytes) {
             count_transfer(false, bytes);
-            const size_t pieces = (bytes + kCopyPiece - 1) / kCopyPiece, flags = (bytes + 63) / 64 * 64;
             PinnedBuffer stage;
-            if (bytes > kStageMost || is_pinned(host) || !pinned_acquire(flags + pieces * sizeof(unsigned), &stage)) {
+            if (bytes > kDownloadMost || is_pinned(host) || !hold(std::min(bytes, kDownloadRing), &stage)) {
                 ST_HIP_TRY(hipMemcpyAsync(host, device, bytes, hipMemcpyDeviceToHost, ws_->stream),
                            "hipMemcpyAsync(D2H)");
             } else {
-                stages_.push_back(stage);
-                unsigned char *const pinned = static_cast<unsigned char *>(stage.ptr);
-                unsigned *const arrived = reinterpret_cast<unsigned *>(pinned + flags);
-                std::memset(arrived, 0, pieces * sizeof(unsigned));
-                drained_ = false;
-                ST_HIP_TRY(launch_copy_to_pinned(pinned, device, bytes, arrived, ws_->stream), "copy launch");
-                // Pieces are taken as they arrive.  Where none does for a while the stream is waited for, which also reports
-                // what went wrong on it.
-                auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
-                for (size_t p = 0; p < pieces;) {
-                    if (__atomic_load_n(&arrived[p], __ATOMIC_ACQUIRE) != 0) {
-                        const size_t at = p * kCopyPiece;
-                        std::memcpy(static_cast<unsigned char *>(host) + at, pinned + at, std::min(kCopyPiece, bytes - at));
-                        ++p;
-                    } else if (std::chrono::steady_clock::now() > until) {
-                        ST_HIP_TRY(hipStreamSynchronize(ws_->stream), "hipStreamSynchronize");
-                        if (__atomic_load_n(&arrived[p], __ATOMIC_ACQUIRE) == 0) return fail(ST_HIP_ERR_RUNTIME, "a copy to the host did not arrive");
-                    }
-                }
-                drained_ = true;  // the last kernel of the stream has said so
-                return ST_HIP_OK;
+                return download_staged(host, device, bytes, stage);
             }
         }
         ST_HIP_TRY(hipStreamSynchronize(ws_->stream), "hipStreamSynchronize");
@@ -164,8 +142,56 @@ class Lease {
     }
 
   private:
+    // The result goes through a ring of pinned memory in pieces, which are taken out of it as they arrive.  A result larger than the
+    // ring comes in quarters of it, each sent by a launch of its own once the quarter before it in the same place has been
+    // taken.  Where no piece arrives for a while the stream is waited for, which also reports what went wrong on it.
+    int download_staged(void *host, const void *device, size_t bytes, const PinnedBuffer &stage)
+    {
+        constexpr size_t kRingPieces = kDownloadRing / kCopyPiece, kQuarterPieces = kRingPieces / 4;
+        static_assert(kDownloadRing % (4 * kCopyPiece) == 0, "quarters of whole pieces");
+        const size_t pieces = (bytes + kCopyPiece - 1) / kCopyPiece, batch = pieces <= kRingPieces ? pieces : kQuarterPieces;
+        unsigned char *const pinned = static_cast<unsigned char *>(stage.ptr);
+        unsigned *const arrived = stage.words();
+        drained_ = false;
+        auto send = [&](size_t first) {  // up to `batch` pieces from this one on
+            const size_t slot = first % kRingPieces, count = std::min(batch, pieces - first), at = first * kCopyPiece;
+            std::memset(arrived + slot, 0, count * sizeof(unsigned));
+            return launch_copy_to_pinned(pinned + slot * kCopyPiece, static_cast<const unsigned char *>(device) + at,
+                                         std::min(count * kCopyPiece, bytes - at), arrived + slot, ws_->stream);
+        };
+        size_t sent = 0;
+        for (; sent < std::min(pieces, kRingPieces); sent += batch) ST_HIP_TRY(send(sent), "copy launch");
+        auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
+        for (size_t p = 0; p < pieces;) {
+            const size_t slot = p % kRingPieces;
+            if (__atomic_load_n(&arrived[slot], __ATOMIC_ACQUIRE) != 0) {
+                const size_t at = p * kCopyPiece;
+                std::memcpy(static_cast<unsigned char *>(host) + at, pinned + slot * kCopyPiece, std::min(kCopyPiece, bytes - at));
+                if (++p % batch == 0 && sent < pieces) {
+                    ST_HIP_TRY(send(sent), "copy launch");
+                    sent += batch;
+                    until = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
+                }
+            } else if (std::chrono::steady_clock::now() > until) {
+                ST_HIP_TRY(hipStreamSynchronize(ws_->stream), "hipStreamSynchronize");
+                if (__atomic_load_n(&arrived[slot], __ATOMIC_ACQUIRE) == 0) return fail(ST_HIP_ERR_RUNTIME, "a copy to the host did not arrive");
+            }
+        }
+        drained_ = true;  // the last kernel of the stream has said so
+        return ST_HIP_OK;
+    }
+    // Pinned memory in use until the stream has drained.
+    bool hold(size_t bytes, PinnedBuffer *stage)
+    {
+        if (stage_count_ == kMostStages || !pinned_acquire(bytes, stage)) return false;
+        stages_[stage_count_++] = *stage;
+        return true;
+    }
+
+    static constexpr size_t kMostStages = 2 * kWorkspaceBuffers;  // an operand or a result each
     Workspace *ws_ = nullptr;
-    std::vector<PinnedBuffer> stages_;  // in use until the stream has drained
+    PinnedBuffer stages_[kMostStages];
+    size_t stage_count_ = 0;
     bool drained_ = false;              // nothing is left on the stream
     int status_ = ST_HIP_OK;
 };

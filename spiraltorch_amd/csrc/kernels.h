@@ -231,20 +231,25 @@ hipError_t stream_workspace_slot(hipStream_t stream, int slot, size_t bytes, voi
 inline bool scratch_unavailable(hipError_t rc) { return rc == hipErrorOutOfMemory || rc == hipErrorStreamCaptureUnsupported; }
 void release_stream_workspace(hipStream_t stream);
 size_t stream_workspace_entry_count();
-// Pinned host memory for a call's copies and results, from a pool that keeps up to kPinnedIdleBytes between calls and is safe with
-// several threads; false where the host has none to give (the caller then copies without it).  A buffer is handed back when
-// nothing on the GPU uses it any more.
+// Pinned host memory for a call's copies and results, from a pool that is safe with several threads and holds kPinnedMost bytes at
+// the most, in use or kept for the next call; false where it has none to give (the caller then copies without it).  A buffer is
+// handed back when nothing on the GPU uses it any more.  Behind its `capacity` bytes lies a word for every piece of them.
 struct PinnedBuffer {
     void *ptr = nullptr;
     size_t capacity = 0;
+    unsigned *words() const { return reinterpret_cast<unsigned *>(static_cast<unsigned char *>(ptr) + capacity); }
 };
-constexpr size_t kPinnedIdleBytes = 64u << 20;
+constexpr size_t kPinnedMost = 64u << 20;
 bool pinned_acquire(size_t bytes, PinnedBuffer *out);
 void pinned_release(const PinnedBuffer &buffer);
 void pinned_release_idle();  // frees what no call holds
 bool is_pinned(const void *host);
-// The most a copy goes through pinned memory with.
-constexpr size_t kStageMost = 16u << 20;
+// The most that copies go through pinned memory with, where that is faster than the runtime's copy: operands of a host call (µs of
+// relu(A·B + bias) with square operands of 0.34, 0.67, 1, 4 and 16 MiB and a result of the same size, staged up to 0.5 / 1 / 3 MiB: 85 / 85 / 85,
+// 114 / 123 / 122, 135 / 148 / 147, 408 / 413 / 421, 2019 / 2027 / 2043; 88, 121, 154, 538, 2142 without staging), its results (2048×2048
+// of one term 585 against 1002), and st_hip_memcpy_d2h (1 KiB 13 against 21, 16 KiB 13 against 27, 64 KiB and more level).  A result
+// goes through a ring: pinned memory takes 0.25 to 0.5 ms a MiB to allocate, and is then held.
+constexpr size_t kUploadMost = 512u << 10, kDownloadMost = 16u << 20, kDownloadRing = 2u << 20, kReadMost = 64u << 10;
 // device[0, bytes) = pinned[0, bytes) by a kernel (device on a 16-byte boundary), and back: the piece of kCopyPiece bytes with
 // number p is in host memory when word p of `arrived` (host memory, cleared before) is not zero.
 constexpr size_t kCopyPiece = 16u << 10;

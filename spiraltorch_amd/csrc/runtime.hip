@@ -96,18 +96,48 @@ void count_transfer(bool to_device, size_t bytes)
 }
 
 namespace {
+// Allocating and freeing are no part of a graph, and allowed while some stream of the process is being captured only where the thread
+// says that it means it.
+class RelaxedCapture {
+  public:
+    RelaxedCapture() { exchanged_ = hipThreadExchangeStreamCaptureMode(&mode_) == hipSuccess; }
+    ~RelaxedCapture()
+    {
+        if (exchanged_) (void)hipThreadExchangeStreamCaptureMode(&mode_);
+    }
+    RelaxedCapture(const RelaxedCapture &) = delete;
+    RelaxedCapture &operator=(const RelaxedCapture &) = delete;
+
+  private:
+    hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+    bool exchanged_ = false;
+};
+
 // Never destroyed: threads may hand buffers back while the process is shutting down.
+constexpr size_t kPinnedSmallest = 64u << 10;
 struct PinnedPool {
     std::mutex mutex;
-    std::vector<PinnedBuffer> idle;
-    size_t idle_bytes = 0;
+    PinnedBuffer idle[kPinnedMost / kPinnedSmallest];  // as many as there can be
+    size_t idle_count = 0;
+    size_t held = 0;  // bytes, in use or idle
+    uint64_t allocations = 0;
+
+    void take(size_t i, PinnedBuffer *out)
+    {
+        *out = idle[i];
+        idle[i] = idle[--idle_count];
+    }
 };
 PinnedPool &pinned_pool()
 {
     static PinnedPool *pool = new PinnedPool;
     return *pool;
 }
-
+void pinned_free(const PinnedBuffer &buffer)
+{
+    const RelaxedCapture relaxed;
+    if (hipHostFree(buffer.ptr) != hipSuccess) (void)hipGetLastError();
+}
 }  // namespace
 
 bool is_pinned(const void *host)
@@ -121,26 +151,47 @@ bool is_pinned(const void *host)
     return attributes.type == hipMemoryTypeHost || attributes.type == hipMemoryTypeManaged || attributes.type == hipMemoryTypeDevice;
 }
 
+// The smallest idle buffer that fits and is not far too large; a new one where the pool may grow; any that fits; a new one in the
+// place of smaller ones.  Nothing is freed only because a call has ended: calls that need all there is would pin their memory
+// anew each time.
 bool pinned_acquire(size_t bytes, PinnedBuffer *out)
 {
-    PinnedPool &pool = pinned_pool();
-    {
-        std::lock_guard<std::mutex> lock(pool.mutex);
-        size_t best = pool.idle.size();
-        for (size_t i = 0; i < pool.idle.size(); ++i)
-            if (pool.idle[i].capacity >= bytes && (best == pool.idle.size() || pool.idle[i].capacity < pool.idle[best].capacity)) best = i;
-        if (best < pool.idle.size()) {
-            *out = pool.idle[best];
-            pool.idle_bytes -= out->capacity;
-            pool.idle.erase(pool.idle.begin() + static_cast<std::ptrdiff_t>(best));
-            return true;
-        }
-    }
-    size_t capacity = 64u << 10;
+    if (bytes > kPinnedMost) return false;
+    size_t capacity = kPinnedSmallest;
     while (capacity < bytes) capacity *= 2;
+    PinnedPool &pool = pinned_pool();
+    for (;;) {
+        PinnedBuffer doomed;
+        {
+            std::lock_guard<std::mutex> lock(pool.mutex);
+            size_t best = pool.idle_count, smallest = pool.idle_count;
+            for (size_t i = 0; i < pool.idle_count; ++i) {
+                const size_t has = pool.idle[i].capacity;
+                if (has >= bytes && (best == pool.idle_count || has < pool.idle[best].capacity)) best = i;
+                if (smallest == pool.idle_count || has < pool.idle[smallest].capacity) smallest = i;
+            }
+            const bool room = pool.held + capacity <= kPinnedMost;
+            if (best < pool.idle_count && (pool.idle[best].capacity <= 4 * capacity || !room)) {
+                pool.take(best, out);
+                return true;
+            }
+            if (room) {
+                pool.held += capacity;
+                ++pool.allocations;
+                break;
+            }
+            if (smallest == pool.idle_count) return false;
+            pool.take(smallest, &doomed);
+            pool.held -= doomed.capacity;
+        }
+        pinned_free(doomed);
+    }
     void *ptr = nullptr;
-    if (hipHostMalloc(&ptr, capacity, hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
+    const RelaxedCapture relaxed;
+    if (hipHostMalloc(&ptr, capacity + capacity / kCopyPiece * sizeof(unsigned), hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
         (void)hipGetLastError();
+        std::lock_guard<std::mutex> lock(pool.mutex);
+        pool.held -= capacity;
         return false;
     }
     *out = PinnedBuffer{ptr, capacity};
@@ -151,27 +202,23 @@ void pinned_release(const PinnedBuffer &buffer)
 {
     if (buffer.ptr == nullptr) return;
     PinnedPool &pool = pinned_pool();
-    {
-        std::lock_guard<std::mutex> lock(pool.mutex);
-        if (pool.idle_bytes + buffer.capacity <= kPinnedIdleBytes) {
-            pool.idle.push_back(buffer);
-            pool.idle_bytes += buffer.capacity;
-            return;
-        }
-    }
-    (void)hipHostFree(buffer.ptr);
+    std::lock_guard<std::mutex> lock(pool.mutex);
+    pool.idle[pool.idle_count++] = buffer;
 }
 
 void pinned_release_idle()
 {
     PinnedPool &pool = pinned_pool();
-    std::vector<PinnedBuffer> doomed;
-    {
-        std::lock_guard<std::mutex> lock(pool.mutex);
-        doomed.swap(pool.idle);
-        pool.idle_bytes = 0;
+    for (;;) {
+        PinnedBuffer doomed;
+        {
+            std::lock_guard<std::mutex> lock(pool.mutex);
+            if (pool.idle_count == 0) return;
+            pool.take(pool.idle_count - 1, &doomed);
+            pool.held -= doomed.capacity;
+        }
+        pinned_free(doomed);
     }
-    for (const PinnedBuffer &buffer : doomed) (void)hipHostFree(buffer.ptr);
 }
 
 namespace {
@@ -449,9 +496,8 @@ int st_hip_memcpy_d2h(void *host_dst, const void *device_src, size_t bytes, void
 {
     if (bytes == 0) return ST_HIP_OK;
     count_transfer(false, bytes);
-    // Through pinned memory: 256 KiB in 14 µs, 1 MiB in 38, where the runtime's copy into ordinary memory takes 20 and 63.
     PinnedBuffer stage;
-    const bool staged = bytes <= kStageMost && !is_pinned(host_dst) && pinned_acquire(bytes, &stage);
+    const bool staged = bytes <= kReadMost && !is_pinned(host_dst) && pinned_acquire(bytes, &stage);
     const hipError_t rc = hipMemcpyAsync(staged ? stage.ptr : host_dst, device_src, bytes, hipMemcpyDeviceToHost, as_stream(stream));
     const hipError_t drained = hipStreamSynchronize(as_stream(stream));  // before the pinned memory is handed back
     if (staged && rc == hipSuccess && drained == hipSuccess) std::memcpy(host_dst, stage.ptr, bytes);
@@ -512,6 +558,16 @@ int st_hip_release_scratch(void *stream)
 }
 
 size_t st_hip_scratch_buffer_count(void) { return stream_workspace_entry_count(); }
+
+int st_hip_pinned_memory_counters(uint64_t *counters)
+{
+    if (!counters) return fail(ST_HIP_ERR_INVALID, "pinned_memory_counters received a null out-pointer");
+    PinnedPool &pool = pinned_pool();
+    std::lock_guard<std::mutex> lock(pool.mutex);
+    counters[0] = pool.held;
+    counters[1] = pool.allocations;
+    return ST_HIP_OK;
+}
 
 int st_hip_device_synchronize(void)
 {

@@ -404,6 +404,13 @@ def scratch_buffer_count() -> int:
     return int(_lib.load().st_hip_scratch_buffer_count())
 
 
+def pinned_memory_counters() -> tuple:
+    """(bytes of pinned host memory held for copies, how often such memory has been allocated)."""
+    counters = (ctypes.c_uint64 * 2)()
+    _check(_lib.load().st_hip_pinned_memory_counters(counters))
+    return int(counters[0]), int(counters[1])
+
+
 def device_synchronize() -> None:
     _check(_lib.load().st_hip_device_synchronize())
 
