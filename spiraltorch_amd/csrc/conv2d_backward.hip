@@ -241,7 +241,7 @@ struct GradWeightArgs {
 // vector instructions of cutting and addressing (written into their gaps: 2.2 instead of 2.7 thousand cycles), and which then
 // waits for its first LDS reads behind the barrier.  The whole call, two launches, old / new µs (and the error against float64,
 // 3.6e-7 / 2.1e-7 and the like): that layer 158 / 113, 128 -> 128 at 28×28 90 / 63, 256 -> 256 at 14×14 176 / 75, 512 -> 512 at
-// 7×7 235 / 106, 8 × 64 -> 64 at 56×56 (the small tile) 39.5 / 31, 4 × 24 -> 96 at 28×28 20 / 14.4, 14 × 64 -> 16 at 46×47 41 / 35.
+// 7×7 235 / 106, 8 × 64 -> 64 at 56×56 (the small tile) 39.5 / 31, 4 × 24 -> 96 at 28×28 20 / 14.4, 14 × 64 -> 16 at 46×47 41 / 28.
 //
 // The big tile (TM = 2, TN = 3: 128 × 192, three of which span a 3×3 layer's 576 columns exactly for 64 input channels)
 // cuts 20 values a thread for 36 matrix instructions of a wavefront, 8 for 6 in the small one.
@@ -254,12 +254,14 @@ enum class Gather {
     kValues,   // G and patches value by value: a G below four values an image
     kTaps,     // patches value by value
     kWindows,  // patches by windows: no stride, and rows that are a multiple of four pixels or the whole image
+    kRows,     // by a window where the four pixels lie in one row, else value by value: no stride
 };
 
 template <Gather GATHER, int TM, int TN>
 __device__ __forceinline__ void conv_grad_weight_body(const GradWeightArgs &p, unsigned char *lds)
 {
     constexpr int BM = 64 * TM, BN = 64 * TN, BK = 16;
+    constexpr bool kByWindow = GATHER == Gather::kWindows || GATHER == Gather::kRows;
     // Both tiles are kept pixel-contiguous (row = channel or patch column, 16 pixels + 4 words of padding), so that a
     // lane's four k-values of either operand are one conflict-free 128-bit LDS read.
     constexpr int A_STRIDE = BK + 4, B_STRIDE = BK + 4;
@@ -308,8 +310,8 @@ __device__ __forceinline__ void conv_grad_weight_body(const GradWeightArgs &p, u
         const int ky = rem / s.kw, kx = rem - ky * s.kw;
         dy[j] = ky * s.dil_h - s.pad_h;
         dx[j] = kx * s.dil_w - s.pad_w;
-        tap_offset[j] = GATHER == Gather::kWindows ? ic * H * W + dy[j] * W + dx[j] : ic * H * W;
-        if (GATHER == Gather::kWindows && !col_valid[j]) dy[j] = -(1 << 30);  // no row of the image
+        tap_offset[j] = kByWindow ? ic * H * W + dy[j] * W + dx[j] : ic * H * W;
+        if (kByWindow && !col_valid[j]) dy[j] = -(1 << 30);  // no row of the image
     }
     const int prow0 = wave * 4;  // patch rows prow0 .. prow0+3 of a step: four consecutive pixels, the same for all lanes
 
@@ -392,9 +394,11 @@ __device__ __forceinline__ void conv_grad_weight_body(const GradWeightArgs &p, u
         }
         raw.pixel = p0;
         // The four pixels are the same for every lane of the wavefront (lanes differ in their taps).
-        if (GATHER == Gather::kWindows) {
+        if (kByWindow) {
             raw.ox = ox;
             raw.edge = raw.clamped = false;
+        }
+        if (GATHER == Gather::kWindows || (GATHER == Gather::kRows && ox + 3 < s.ow && p0 + prow0 + 3 < p.spatial)) {
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
                 int off;
@@ -409,11 +413,13 @@ __device__ __forceinline__ void conv_grad_weight_body(const GradWeightArgs &p, u
             for (int r = 0; r < 4; ++r) {
 #pragma unroll
                 for (int j = 0; j < TN; ++j) {
-                    const int iy = py * s.stride_h + dy[j], ix = px * s.stride_w + dx[j];
+                    const int sy = GATHER == Gather::kRows ? py : py * s.stride_h, sx = GATHER == Gather::kRows ? px : px * s.stride_w;
+                    const int iy = sy + dy[j], ix = sx + dx[j];
                     const bool inside = col_valid[j] & (p0 + prow0 + r < p.spatial) &
                                         (static_cast<unsigned>(iy) < static_cast<unsigned>(H)) &
                                         (static_cast<unsigned>(ix) < static_cast<unsigned>(W));
-                    const unsigned off = inside ? static_cast<unsigned>(tap_offset[j] + iy * W + ix) * 4u : kOutside;
+                    const int at = GATHER == Gather::kRows ? tap_offset[j] + (sy * W + sx) : tap_offset[j] + iy * W + ix;
+                    const unsigned off = inside ? static_cast<unsigned>(at) * 4u : kOutside;
                     raw.b[j][r] = __builtin_amdgcn_raw_buffer_load_b32(rsrc_x, off, 0, 0);
                 }
                 const bool wrap = ++px == s.ow;
@@ -456,7 +462,7 @@ __device__ __forceinline__ void conv_grad_weight_body(const GradWeightArgs &p, u
                 for (int r = 0; r < 4; ++r) raw.a[i][r] = raw.pixel + a_c4 + r < p.spatial ? raw.a[i][r] : 0u;
             }
         }
-        if (GATHER != Gather::kWindows) return;
+        if (!kByWindow) return;
         if (raw.clamped) {
 #pragma unroll
             for (int j = 0; j < TN; ++j) put_back(raw.b[j], raw.moved[j]);
@@ -834,8 +840,17 @@ hipError_t launch_conv2d_grad_weight_f32(const ConvShape &shape, const float *in
     // (Rows of other widths as two windows, the second for the pixels in the next row: 111 instead of 75 µs for 256 -> 256 channels at
     // 14×14, and between 4 % less and 10 % more in the small tile.)
     const bool windows = unit && (one_row || shape.ow % 4 == 0) && image_floats >= 4;
-    const Gather gather = static_cast<size_t>(shape.c_out) * args.spatial < 4 ? Gather::kValues : windows ? Gather::kWindows : Gather::kTaps;
+    // In the small tile each four pixels of such layers take a window where they lie in one row, by a branch of the whole wavefront: value by
+    // value a wavefront asks for four times as many cache lines.  Value by value / this, over 330 layers: of launches above 50 µs
+    // with rows of 40 and more 1 / 0.83 (30×256 -> 64 at 74×74, 3×1, 235 / 168 µs),
+    // 20 to 40 1 / 0.86, below 12 level.  In the big tile, one wavefront a SIMD, the branch's waits are not covered.
+    const bool rows = unit && !big && !windows && shape.ow > 4 && image_floats >= 4;
+    const Gather gather = static_cast<size_t>(shape.c_out) * args.spatial < 4 ? Gather::kValues
+                          : windows                                          ? Gather::kWindows
+                          : rows                                             ? Gather::kRows
+                                                                             : Gather::kTaps;
     auto kernel = gather == Gather::kValues    ? conv_grad_weight_kernel<Gather::kValues>
+                  : gather == Gather::kRows    ? conv_grad_weight_kernel<Gather::kRows>
                   : gather == Gather::kWindows ? (big ? conv_grad_weight_big_kernel<Gather::kWindows> : conv_grad_weight_kernel<Gather::kWindows>)
                                                : (big ? conv_grad_weight_big_kernel<Gather::kTaps> : conv_grad_weight_kernel<Gather::kTaps>);
     const size_t lds_bytes = big ? kGradWeightStages<2, 3> : kGradWeightStages<1, 1>;

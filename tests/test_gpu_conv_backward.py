@@ -379,6 +379,13 @@ GRAD_WEIGHT_CASES = [
     # a gradient below one window of four, and one that is exactly one
     (5, 3, 2, 5, 1, (2, 3), (1, 1), (0, 0), (1, 1)),
     (5, 3, 2, 6, 1, (2, 3), (1, 1), (0, 0), (1, 1)),
+    # rows of odd widths, four pixels in one row and over the end of it, with and without borders
+    (3, 5, 6, 5, 20, (3, 3), (1, 1), (1, 1), (1, 1)),
+    (2, 3, 9, 13, 33, (5, 3), (1, 1), (2, 1), (1, 1)),
+    (2, 4, 15, 23, 40, (7, 1), (1, 1), (0, 0), (2, 1)),
+    (2, 6, 7, 18, 20, (3, 5), (1, 1), (1, 4), (1, 2)),
+    (1, 1, 3, 6, 5, (1, 3), (1, 1), (0, 1), (1, 1)),
+    (3, 70, 5, 9, 65, (3, 3), (1, 1), (0, 0), (1, 1)),
 ]
 
 
@@ -407,7 +414,7 @@ def test_grad_weight_of_any_magnitude(hip, case, x_scale, g_scale):
     assert np.all(np.abs(got - want) <= 2.0 ** -19 * magnitudes + 2.0 ** -149)
 
 
-@pytest.mark.parametrize("case", [GRAD_WEIGHT_CASES[3], GRAD_WEIGHT_CASES[7], GRAD_WEIGHT_CASES[10]])
+@pytest.mark.parametrize("case", [GRAD_WEIGHT_CASES[3], GRAD_WEIGHT_CASES[7], GRAD_WEIGHT_CASES[10], GRAD_WEIGHT_CASES[22]])
 def test_grad_weight_keeps_infinities_and_nan_to_their_terms(hip, case):
     """A value at the end of an image row reaches the columns whose taps read it and no others, although the loads do."""
     batch, c_in, h, w, c_out, kernel, stride, padding, dilation = case
