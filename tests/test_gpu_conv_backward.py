@@ -379,6 +379,11 @@ GRAD_WEIGHT_CASES = [
     # a gradient below one window of four, and one that is exactly one
     (5, 3, 2, 5, 1, (2, 3), (1, 1), (0, 0), (1, 1)),
     (5, 3, 2, 6, 1, (2, 3), (1, 1), (0, 0), (1, 1)),
+    # a stride in the large tile; sixteen steps and seventeen (the small tile and the large one); 268 large tiles, a mostly empty second round
+    (3, 64, 15, 16, 128, (3, 3), (2, 1), (1, 1), (1, 1)),
+    (16, 64, 4, 4, 128, (3, 3), (1, 1), (1, 1), (1, 1)),
+    (17, 64, 4, 4, 128, (3, 3), (1, 1), (1, 1), (1, 1)),
+    (1, 512, 7, 17, 512, (5, 5), (1, 1), (2, 2), (1, 1)),
     # rows of odd widths, four pixels in one row and over the end of it, with and without borders
     (3, 5, 6, 5, 20, (3, 3), (1, 1), (1, 1), (1, 1)),
     (2, 3, 9, 13, 33, (5, 3), (1, 1), (2, 1), (1, 1)),
@@ -414,7 +419,7 @@ def test_grad_weight_of_any_magnitude(hip, case, x_scale, g_scale):
     assert np.all(np.abs(got - want) <= 2.0 ** -19 * magnitudes + 2.0 ** -149)
 
 
-@pytest.mark.parametrize("case", [GRAD_WEIGHT_CASES[3], GRAD_WEIGHT_CASES[7], GRAD_WEIGHT_CASES[10], GRAD_WEIGHT_CASES[22]])
+@pytest.mark.parametrize("case", [GRAD_WEIGHT_CASES[3], GRAD_WEIGHT_CASES[7], GRAD_WEIGHT_CASES[10], GRAD_WEIGHT_CASES[26]])
 def test_grad_weight_keeps_infinities_and_nan_to_their_terms(hip, case):
     """A value at the end of an image row reaches the columns whose taps read it and no others, although the loads do."""
     batch, c_in, h, w, c_out, kernel, stride, padding, dilation = case
