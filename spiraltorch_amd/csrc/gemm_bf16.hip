@@ -2553,10 +2553,12 @@ hipError_t launch_gemm_bf16(size_t m, size_t n, size_t k, const uint16_t *lhs, c
         if (as_it_is) return launch_gemm_bf16_small(m, n, k, lhs, rhs, rhs_packed, out_f32, out_bf16, epilogue, stream);
         void *workspace = nullptr;
         hipError_t rc = stream_workspace(stream, k * n * sizeof(uint16_t), &workspace);
-        if (rc != hipSuccess) return rc;
-        rc = launch_transpose_u16(k, n, rhs, static_cast<uint16_t *>(workspace), stream);
-        if (rc != hipSuccess) return rc;
-        return launch_gemm_bf16_small(m, n, k, lhs, static_cast<const uint16_t *>(workspace), true, out_f32, out_bf16, epilogue, stream);
+        if (rc == hipSuccess) {
+            rc = launch_transpose_u16(k, n, rhs, static_cast<uint16_t *>(workspace), stream);
+            if (rc != hipSuccess) return rc;
+            return launch_gemm_bf16_small(m, n, k, lhs, static_cast<const uint16_t *>(workspace), true, out_f32, out_bf16, epilogue, stream);
+        }
+        if (!scratch_unavailable(rc)) return rc;  // else the kernels below, of which the general one reads B as it is
     }
     // An n that is not a multiple of 128 (a vocabulary of 50257, 1000 classes) with a k the 256-row kernels take: the
     // packed kernels run it as it is — rows of Bᵀ past n read as zero through the buffer range check, and the epilogue

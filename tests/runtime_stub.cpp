@@ -1,0 +1,82 @@
+// A HIP runtime without a GPU, for tests of what the library's host code asks of the real one: launches are counted and not run,
+// device memory is host memory, of which there may be none (stub_no_memory), and addresses within [stub_device_first,
+// stub_device_end) are reported as device memory.  Loaded before libsthip.so with its symbols global.
+#include <hip/hip_runtime_api.h>
+
+#include <cstdlib>
+#include <cstring>
+
+extern "C" {
+int stub_no_memory = 0;
+unsigned long long stub_launches = 0, stub_copies = 0, stub_last_grid = 0;
+const char *stub_device_first = nullptr, *stub_device_end = nullptr;
+const void *stub_copied_from = nullptr;
+int stub_copy_kind = -1;
+
+hipError_t hipGetDeviceCount(int *count) { *count = 1; return hipSuccess; }
+hipError_t hipGetDevice(int *device) { *device = 0; return hipSuccess; }
+hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600 *props, int)
+{
+    std::memset(props, 0, sizeof *props);
+    std::strcpy(props->gcnArchName, "gfx950");
+    props->multiProcessorCount = 256;
+    return hipSuccess;
+}
+hipError_t hipGetSymbolAddress(void **address, const void *symbol) { *address = const_cast<void *>(symbol); return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipMalloc(void **ptr, size_t bytes)
+{
+    if (stub_no_memory) return hipErrorOutOfMemory;
+    *ptr = std::aligned_alloc(4096, (bytes + 4095) / 4096 * 4096);
+    return *ptr ? hipSuccess : hipErrorOutOfMemory;
+}
+hipError_t hipFree(void *ptr) { std::free(ptr); return hipSuccess; }
+hipError_t hipHostMalloc(void **ptr, size_t bytes, unsigned)
+{
+    *ptr = std::aligned_alloc(4096, (bytes + 4095) / 4096 * 4096);
+    return hipSuccess;
+}
+hipError_t hipHostFree(void *ptr) { std::free(ptr); return hipSuccess; }
+hipError_t hipStreamCreate(hipStream_t *stream) { *stream = reinterpret_cast<hipStream_t>(std::malloc(1)); return hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t stream) { std::free(stream); return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *status) { *status = hipStreamCaptureStatusNone; return hipSuccess; }
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode *) { return hipSuccess; }
+hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
+static dim3 pushed_grid, pushed_block;
+hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t, hipStream_t)
+{
+    pushed_grid = grid;
+    pushed_block = block;
+    return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *lds, hipStream_t *stream)
+{
+    *grid = pushed_grid;
+    *block = pushed_block;
+    *lds = 0;
+    *stream = nullptr;
+    return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void *, dim3 grid, dim3, void **, size_t, hipStream_t)
+{
+    ++stub_launches;
+    stub_last_grid = static_cast<unsigned long long>(grid.x) * grid.y * grid.z;
+    return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void *, const void *src, size_t, hipMemcpyKind kind, hipStream_t)
+{
+    ++stub_copies;
+    stub_copied_from = src;
+    stub_copy_kind = static_cast<int>(kind);
+    return hipSuccess;
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t *attributes, const void *ptr)
+{
+    const char *const at = static_cast<const char *>(ptr);
+    if (at < stub_device_first || at >= stub_device_end) return hipErrorInvalidValue;
+    std::memset(attributes, 0, sizeof *attributes);
+    attributes->type = hipMemoryTypeDevice;
+    return hipSuccess;
+}
+}
