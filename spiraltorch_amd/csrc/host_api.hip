@@ -111,7 +111,9 @@ class Lease {
             // next: the runtime's own copy holds the caller as long and then waits between the engines.
             constexpr size_t kPiece = 256u << 10;
             PinnedBuffer stage;
-            if (bytes > kUploadMost || (bytes >= kPiece && is_pinned(host)) || !hold(bytes, &stage)) {
+            const HostMemory memory = host_memory(host);
+            if (bytes > kUploadMost || memory == HostMemory::kRuntime || (memory == HostMemory::kPinned && bytes >= kPiece) ||
+                !hold(bytes, &stage)) {
                 ST_HIP_TRY(hipMemcpyAsync(*device, host, bytes, hipMemcpyHostToDevice, ws_->stream),
                            "hipMemcpyAsync(H2D)");
                 return ST_HIP_OK;
@@ -130,7 +132,7 @@ class Lease {
         if (bytes) {
             count_transfer(false, bytes);
             PinnedBuffer stage;
-            if (bytes > kDownloadMost || is_pinned(host) || !hold(std::min(bytes, kDownloadRing), &stage)) {
+            if (bytes > kDownloadMost || host_memory(host) != HostMemory::kOrdinary || !hold(std::min(bytes, kDownloadRing), &stage)) {
                 ST_HIP_TRY(hipMemcpyAsync(host, device, bytes, hipMemcpyDeviceToHost, ws_->stream),
                            "hipMemcpyAsync(D2H)");
             } else {

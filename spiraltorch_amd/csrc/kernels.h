@@ -243,7 +243,10 @@ constexpr size_t kPinnedMost = 64u << 20;
 bool pinned_acquire(size_t bytes, PinnedBuffer *out);
 void pinned_release(const PinnedBuffer &buffer);
 void pinned_release_idle();  // frees what no call holds
-bool is_pinned(const void *host);
+// What a caller's "host" pointer is: memory of the host, pinned or not, or what only the runtime's copies may touch (managed memory, and
+// device memory, which they have always taken).
+enum class HostMemory { kOrdinary, kPinned, kRuntime };
+HostMemory host_memory(const void *host);
 // The most that copies go through pinned memory with, where that is faster than the runtime's copy: operands of a host call (µs of
 // relu(A·B + bias) with square operands of 0.34, 0.67, 1, 4 and 16 MiB and a result of the same size, staged up to 0.5 / 1 / 3 MiB: 85 / 85 / 85,
 // 114 / 123 / 122, 135 / 148 / 147, 408 / 413 / 421, 2019 / 2027 / 2043; 88, 121, 154, 538, 2142 without staging), its results (2048×2048

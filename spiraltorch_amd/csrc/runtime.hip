@@ -140,15 +140,15 @@ void pinned_free(const PinnedBuffer &buffer)
 }
 }  // namespace
 
-bool is_pinned(const void *host)
+HostMemory host_memory(const void *host)
 {
     hipPointerAttribute_t attributes;
-    const hipError_t rc = hipPointerGetAttributes(&attributes, host);
-    if (rc != hipSuccess) {
+    if (hipPointerGetAttributes(&attributes, host) != hipSuccess) {
         (void)hipGetLastError();
-        return false;
+        return HostMemory::kOrdinary;
     }
-    return attributes.type == hipMemoryTypeHost || attributes.type == hipMemoryTypeManaged || attributes.type == hipMemoryTypeDevice;
+    if (attributes.type == hipMemoryTypeHost) return HostMemory::kPinned;
+    return attributes.type == hipMemoryTypeManaged || attributes.type == hipMemoryTypeDevice ? HostMemory::kRuntime : HostMemory::kOrdinary;
 }
 
 // The smallest idle buffer that fits and is not far too large; a new one where the pool may grow; any that fits; a new one in the
@@ -497,7 +497,7 @@ int st_hip_memcpy_d2h(void *host_dst, const void *device_src, size_t bytes, void
     if (bytes == 0) return ST_HIP_OK;
     count_transfer(false, bytes);
     PinnedBuffer stage;
-    const bool staged = bytes <= kReadMost && !is_pinned(host_dst) && pinned_acquire(bytes, &stage);
+    const bool staged = bytes <= kReadMost && host_memory(host_dst) == HostMemory::kOrdinary && pinned_acquire(bytes, &stage);
     const hipError_t rc = hipMemcpyAsync(staged ? stage.ptr : host_dst, device_src, bytes, hipMemcpyDeviceToHost, as_stream(stream));
     const hipError_t drained = hipStreamSynchronize(as_stream(stream));  // before the pinned memory is handed back
     if (staged && rc == hipSuccess && drained == hipSuccess) std::memcpy(host_dst, stage.ptr, bytes);

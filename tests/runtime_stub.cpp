@@ -8,10 +8,9 @@
 
 extern "C" {
 int stub_no_memory = 0;
-unsigned long long stub_launches = 0, stub_copies = 0, stub_last_grid = 0;
+unsigned long long stub_launches = 0;
 const char *stub_device_first = nullptr, *stub_device_end = nullptr;
-const void *stub_copied_from = nullptr;
-int stub_copy_kind = -1;
+const void *stub_first_source = nullptr;  // of the runtime's copies
 
 hipError_t hipGetDeviceCount(int *count) { *count = 1; return hipSuccess; }
 hipError_t hipGetDevice(int *device) { *device = 0; return hipSuccess; }
@@ -58,17 +57,14 @@ hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *lds, hipSt
     *stream = nullptr;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *, dim3 grid, dim3, void **, size_t, hipStream_t)
+hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t)
 {
     ++stub_launches;
-    stub_last_grid = static_cast<unsigned long long>(grid.x) * grid.y * grid.z;
     return hipSuccess;
 }
-hipError_t hipMemcpyAsync(void *, const void *src, size_t, hipMemcpyKind kind, hipStream_t)
+hipError_t hipMemcpyAsync(void *, const void *src, size_t, hipMemcpyKind, hipStream_t)
 {
-    ++stub_copies;
-    stub_copied_from = src;
-    stub_copy_kind = static_cast<int>(kind);
+    if (stub_first_source == nullptr) stub_first_source = src;
     return hipSuccess;
 }
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t *attributes, const void *ptr)

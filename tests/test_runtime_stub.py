@@ -42,3 +42,23 @@ for fail in (1, 0):
     print(launches.value - before)
 """)
     assert out == ["1", "2"]
+
+
+@pytest.mark.parametrize("rows", [1, 64, 300])  # one value, and either side of the 256 KiB from which the pointer was looked at
+def test_operands_in_device_memory_are_left_to_the_runtime(stub, rows):
+    """A host call whose operand lies in device or managed memory (here: pages nobody may read) copies it with the runtime's copy."""
+    out = run(stub, f"""
+import mmap, numpy as np
+libc = ctypes.CDLL(None)
+libc.mmap.restype = ctypes.c_void_p
+libc.mmap.argtypes = [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_long]
+count = {rows} * 256
+closed = libc.mmap(None, 1 << 20, 0, mmap.MAP_PRIVATE | mmap.MAP_ANONYMOUS, -1, 0)
+for name, value in (("stub_device_first", closed), ("stub_device_end", closed + (1 << 20))):
+    ctypes.c_void_p.in_dll(stub, name).value = value
+n = (1 << 22) // count + 1  # (a result that is not staged: no kernel writes one here)
+rhs, out = np.ones(n, np.float32), np.zeros(count * n, np.float32)
+status = lib.st_hip_gemm_f32(count, n, 1, 1.0, 0, closed, count, rhs.ctypes.data, n, out.ctypes.data, count * n)
+print(status, ctypes.c_void_p.in_dll(stub, "stub_first_source").value == closed)
+""")
+    assert out == ["0", "True"]
