@@ -1125,6 +1125,16 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_split_kernel(AttnArg
 // -------------------------------------------------------------------------------------------------
 constexpr int kKeysWaves = 8, kKeysRows = 32;
 
+struct KeysItem {
+    int q_tile, ctx, split;
+};
+// Workgroup -> (query tile, context, run of keys): the longest rows of all contexts first.
+__host__ __device__ inline KeysItem decode_keys_block(int contexts, int q_tiles, int key_splits, int block)
+{
+    const int item = block / key_splits;
+    return KeysItem{q_tiles - 1 - item / contexts, item % contexts, block - item * key_splits};
+}
+
 template <int DPAD, bool CAUSAL, bool BIAS>
 __global__ __launch_bounds__(64 * kKeysWaves) void attention_f32_keys_kernel(AttnArgs p)
 {
@@ -1139,10 +1149,9 @@ __global__ __launch_bounds__(64 * kKeysWaves) void attention_f32_keys_kernel(Att
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 31, lh = lane >> 5;
     const int S = p.S, D = p.D;
-    // the longest rows of all contexts first
-    const int item = static_cast<int>(blockIdx.x) / p.key_splits, split = static_cast<int>(blockIdx.x) - item * p.key_splits;
-    const int q_tile = p.q_tiles - 1 - item / p.contexts, ctx = item % p.contexts;
-    const int q0 = q_tile * kKeysRows, my_q = q0 + li;
+    const KeysItem item = decode_keys_block(p.contexts, p.q_tiles, p.key_splits, static_cast<int>(blockIdx.x));
+    const int ctx = item.ctx, split = item.split;
+    const int q0 = item.q_tile * kKeysRows, my_q = q0 + li;
     const int key_first = split * p.keys_per_split, key_end = min(CAUSAL ? min(S, q0 + kKeysRows) : S, key_first + p.keys_per_split);
     const size_t ctx_elem0 = static_cast<size_t>(ctx) * S * D;
     const unsigned ctx_bytes = static_cast<unsigned>(S) * static_cast<unsigned>(D) * 4u;
@@ -1828,6 +1837,23 @@ size_t keys_shared(size_t contexts, size_t sequence, bool biased, size_t *keys_p
     return best_keys <= 512 || (workgroups > 128 && sequence <= 1024) ? best : 0;
 }
 
+bool keys_block_in_range(const AttnArgs &args, size_t block)
+{
+    const KeysItem item = decode_keys_block(args.contexts, args.q_tiles, args.key_splits, static_cast<int>(block));
+    return item.ctx >= 0 && item.ctx < args.contexts && item.q_tile >= 0 && item.q_tile < args.q_tiles && item.split >= 0 &&
+           item.split < args.key_splits && item.split * args.keys_per_split < args.S;
+}
+
+// The check before a launch: the grid is what the decode assumes, tiles and runs cover queries and keys and none of them is empty.
+bool keys_plan_consistent(const AttnArgs &args, size_t blocks)
+{
+    const long long rows = static_cast<long long>(args.q_tiles) * kKeysRows, keys = static_cast<long long>(args.key_splits) * args.keys_per_split;
+    if (args.q_tiles <= 0 || args.key_splits <= 0 || args.keys_per_split <= 0 || blocks > 0x7fffffffu) return false;
+    if (blocks != static_cast<size_t>(args.contexts) * args.q_tiles * args.key_splits) return false;
+    if (rows < args.S || rows - kKeysRows >= args.S || keys < args.S || keys - args.keys_per_split >= args.S) return false;
+    return keys_block_in_range(args, 0) && keys_block_in_range(args, blocks - 1);
+}
+
 template <int DPAD, bool CAUSAL, bool BIAS>
 hipError_t launch_keys(AttnArgs args, hipStream_t stream)
 {
@@ -1846,8 +1872,9 @@ hipError_t launch_keys(AttnArgs args, hipStream_t stream)
             return scratch;
         }
     }
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(args.contexts) * args.q_tiles * args.key_splits), dim3(64 * kKeysWaves), lds_bytes,
-                       stream, args);
+    const size_t blocks = static_cast<size_t>(args.contexts) * args.q_tiles * args.key_splits;
+    if (!keys_plan_consistent(args, blocks)) return hipErrorInvalidConfiguration;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(64 * kKeysWaves), lds_bytes, stream, args);
     rc = hipGetLastError();
     return rc != hipSuccess || args.key_splits == 1 ? rc : merge_parts(args, BIAS, 0, stream);
 }
@@ -1922,12 +1949,23 @@ AttentionPlanReport attention_f32_plan_report(size_t contexts, size_t sequence, 
         return report;
     }
     size_t keys = 0, runs = 0;
-    if (report.kernel == ST_HIP_ATTN_KERNEL_SPLIT && (runs = keys_shared(contexts, sequence, biased, &keys)) > 0) {  // decoded by division
-        report.workgroups = contexts * ((sequence + kKeysRows - 1) / kKeysRows) * runs;
-        report.key_splits = static_cast<int>(runs);
-        report.keys_per_split = static_cast<int>(keys);
-        report.items = report.items_expected = report.workgroups;
-        report.consistent = 1;
+    if (report.kernel == ST_HIP_ATTN_KERNEL_SPLIT && (runs = keys_shared(contexts, sequence, biased, &keys)) > 0) {
+        args.q_tiles = (args.S + kKeysRows - 1) / kKeysRows;
+        report.key_splits = args.key_splits = static_cast<int>(runs);
+        report.keys_per_split = args.keys_per_split = static_cast<int>(keys);
+        report.workgroups = report.items_expected = contexts * static_cast<size_t>(args.q_tiles) * runs;
+        report.consistent = keys_plan_consistent(args, report.workgroups) ? 1 : 0;
+        std::vector<unsigned char> seen(report.workgroups, 0);
+        for (size_t block = 0; block < report.workgroups; ++block) {
+            if (!keys_block_in_range(args, block)) {
+                ++report.out_of_range;
+                continue;
+            }
+            const KeysItem item = decode_keys_block(args.contexts, args.q_tiles, args.key_splits, static_cast<int>(block));
+            unsigned char &cell = seen[(static_cast<size_t>(item.ctx) * args.q_tiles + item.q_tile) * runs + item.split];
+            if (cell) ++report.duplicates; else ++report.items;
+            cell = 1;
+        }
         return report;
     }
     int causal_r = 0;

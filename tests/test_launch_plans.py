@@ -75,6 +75,22 @@ def test_the_attention_plan_knows_the_scale():
         assert got["items"] == got["items_expected"], (contexts, seq, dim, causal, biased, got)
 
 
+@pytest.mark.parametrize("causal,biased", [(False, False), (True, False), (False, True), (True, True)])
+def test_shared_keys_are_dealt_out_completely(causal, biased):
+    # a workgroup 32 queries of a context and one run of keys: at most one for each of the 256 compute units, every one its own item
+    cut = set()
+    for contexts, seq, dim in itertools.product((1, 2, 3, 7, 8, 31, 32, 64, 128), SEQUENCES + (33, 96, 250, 333, 777), (32, 48, 64)):
+        plan = hip.attention_f32_launch_plan(contexts, seq, dim, causal, biased, scale=dim ** -0.5)
+        where = (contexts, seq, dim, causal, biased, plan)
+        assert plan["consistent"] == 1 and plan["out_of_range"] == 0 and plan["duplicates"] == 0, where
+        assert plan["items"] == plan["items_expected"], where
+        if plan["kernel"] == "split" and plan["workgroups"] == contexts * -(-seq // 32) * plan["key_splits"]:
+            assert plan["workgroups"] <= 256, where
+            assert plan["key_splits"] * plan["keys_per_split"] >= seq > (plan["key_splits"] - 1) * plan["keys_per_split"], where
+            cut.add(plan["key_splits"])
+    assert {1, 4, 8} <= cut, cut
+
+
 def test_key_chunks_of_large_heads():
     # chunks of 128 keys, the last one shorter, where every workgroup has a compute unit to itself; otherwise as many keys as
     # two workgroups a unit leave each, 128 and more
