@@ -53,6 +53,33 @@ __device__ __forceinline__ unsigned pack_bf16x2(float lo, float hi)
     return __builtin_bit_cast(unsigned, v);
 }
 
+struct Bf16Item {
+    int ctx, q_tile;
+};
+// Workgroup -> (context, query tile): each XCD (workgroup id mod 8) keeps whole contexts, where they divide evenly, so their K/V stay in
+// its L2; causal tiles, and those of few queries, run longest-first across all contexts (of the XCD).
+__host__ __device__ inline Bf16Item decode_bf16_block(bool longest_first, int contexts, int q_tiles, int swizzle, unsigned block)
+{
+    const unsigned of_xcd = swizzle ? contexts >> 3 : contexts, first = swizzle ? (block & 7) * of_xcd : 0, i = swizzle ? block >> 3 : block;
+    const unsigned tiles = static_cast<unsigned>(q_tiles), tile = longest_first ? tiles - 1 - i / of_xcd : i % tiles;
+    return Bf16Item{static_cast<int>(first + (longest_first ? i % of_xcd : i / tiles)), static_cast<int>(tile)};
+}
+
+// The check before a launch: the grid is what the decode assumes, its tiles of `rows` queries cover them without an empty one, and
+// the first and last workgroups lie inside.
+bool bf16_grid_consistent(const AttnBf16Args &a, int rows, bool longest_first, size_t blocks)
+{
+    const int contexts = a.batch * a.heads;
+    const long long covered = static_cast<long long>(a.q_tiles) * rows;
+    if (contexts <= 0 || a.q_tiles <= 0 || blocks > 0x7fffffffu || blocks != static_cast<size_t>(contexts) * a.q_tiles) return false;
+    if (covered < a.S || covered - rows >= a.S || (a.swizzle && contexts % 8 != 0)) return false;
+    for (const size_t block : {static_cast<size_t>(0), blocks - 1}) {
+        const Bf16Item item = decode_bf16_block(longest_first, contexts, a.q_tiles, a.swizzle, static_cast<unsigned>(block));
+        if (item.ctx < 0 || item.ctx >= contexts || item.q_tile < 0 || item.q_tile >= a.q_tiles) return false;
+    }
+    return true;
+}
+
 template <int D, bool CAUSAL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? (CAUSAL ? 4 : 3) : 2, D == 64 ? (CAUSAL ? 4 : 3) : 2))) void attention_bf16_kernel(AttnBf16Args p)
 {
@@ -74,28 +101,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? (
     const int S = p.S;
     const int contexts = p.batch * p.heads;
 
-    // Workgroup -> (context, query tile): each XCD (workgroup id mod 8) keeps whole contexts so their K/V
-    // stay in its L2; causal tiles run longest-first across all contexts of the XCD.
-    int ctx, q_tile;
-    if (p.swizzle) {
-        const int per_xcd = contexts >> 3;
-        const int xcd = blockIdx.x & 7, i = blockIdx.x >> 3;
-        if (CAUSAL) {
-            q_tile = p.q_tiles - 1 - i / per_xcd;
-            ctx = xcd * per_xcd + i % per_xcd;
-        } else {
-            ctx = xcd * per_xcd + i / p.q_tiles;
-            q_tile = i % p.q_tiles;
-        }
-    } else {
-        if (CAUSAL) {
-            q_tile = p.q_tiles - 1 - blockIdx.x / contexts;
-            ctx = blockIdx.x % contexts;
-        } else {
-            ctx = blockIdx.x / p.q_tiles;
-            q_tile = blockIdx.x % p.q_tiles;
-        }
-    }
+    const Bf16Item item = decode_bf16_block(CAUSAL, contexts, p.q_tiles, p.swizzle, blockIdx.x);
+    const int ctx = item.ctx, q_tile = item.q_tile;
     const int q0 = q_tile * kBQ16;
     const int wq0 = q0 + wave * 32;
     const int my_q = wq0 + li;
@@ -338,27 +345,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     const int S = p.S;
     const int contexts = p.batch * p.heads;
 
-    // Workgroup -> (context, query tile) as in the kernel above.
-    int ctx, q_tile;
-    if (p.swizzle) {
-        const int per_xcd = contexts >> 3;
-        const int xcd = blockIdx.x & 7, i = blockIdx.x >> 3;
-        if (CAUSAL) {
-            q_tile = p.q_tiles - 1 - i / per_xcd;
-            ctx = xcd * per_xcd + i % per_xcd;
-        } else {
-            ctx = xcd * per_xcd + i / p.q_tiles;
-            q_tile = i % p.q_tiles;
-        }
-    } else {
-        if (CAUSAL) {
-            q_tile = p.q_tiles - 1 - blockIdx.x / contexts;
-            ctx = blockIdx.x % contexts;
-        } else {
-            ctx = blockIdx.x / p.q_tiles;
-            q_tile = blockIdx.x % p.q_tiles;
-        }
-    }
+    const Bf16Item item = decode_bf16_block(CAUSAL, contexts, p.q_tiles, p.swizzle, blockIdx.x);
+    const int ctx = item.ctx, q_tile = item.q_tile;
     const int q0 = q_tile * kBQ16;
     const int wq0 = q0 + wave * 32;
     const int my_q = wq0 + li;
@@ -619,16 +607,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     const int li = lane & 31, lh = lane >> 5;
     const int S = p.S;
     const int contexts = p.batch * p.heads;
-    // a context's tiles on one XCD where the contexts divide evenly; the longest rows first
-    int ctx, q_tile;
-    if (p.swizzle) {
-        const int per_xcd = contexts >> 3, i = blockIdx.x >> 3;
-        q_tile = p.q_tiles - 1 - i / per_xcd;
-        ctx = (blockIdx.x & 7) * per_xcd + i % per_xcd;
-    } else {
-        q_tile = p.q_tiles - 1 - blockIdx.x / contexts;
-        ctx = blockIdx.x % contexts;
-    }
+    const Bf16Item item = decode_bf16_block(true, contexts, p.q_tiles, p.swizzle, blockIdx.x);
+    const int ctx = item.ctx, q_tile = item.q_tile;
     const int q0 = q_tile * kBQSplit;
     const int my_q = q0 + li;
     const int b = ctx / p.heads, h = ctx % p.heads;
@@ -792,8 +772,9 @@ template <int D, bool CAUSAL>
 hipError_t launch_keys(AttnBf16Args args, hipStream_t stream)
 {
     args.q_tiles = (args.S + kBQSplit - 1) / kBQSplit;
-    const unsigned blocks = static_cast<unsigned>(args.batch * args.heads * args.q_tiles);
-    hipLaunchKernelGGL((attention_bf16_keys_kernel<D, CAUSAL>), dim3(blocks), dim3(256), 0, stream, args);
+    const size_t blocks = static_cast<size_t>(args.batch) * args.heads * args.q_tiles;
+    if (!bf16_grid_consistent(args, kBQSplit, true, blocks)) return hipErrorInvalidConfiguration;
+    hipLaunchKernelGGL((attention_bf16_keys_kernel<D, CAUSAL>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, args);
     return hipGetLastError();
 }
 
@@ -806,6 +787,7 @@ hipError_t launch_d64(const AttnBf16Args &args, hipStream_t stream)
                                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes));
     if (rc != hipSuccess) return rc;
     const size_t blocks = static_cast<size_t>(args.batch) * args.heads * args.q_tiles;
+    if (!bf16_grid_consistent(args, kBQ16, CAUSAL, blocks)) return hipErrorInvalidConfiguration;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), lds_bytes, stream, args);
     return hipGetLastError();
 }
@@ -819,6 +801,7 @@ hipError_t launch_variant(const AttnBf16Args &args, hipStream_t stream)
                                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes));
     if (rc != hipSuccess) return rc;
     const size_t blocks = static_cast<size_t>(args.batch) * args.heads * args.q_tiles;
+    if (!bf16_grid_consistent(args, kBQ16, CAUSAL, blocks)) return hipErrorInvalidConfiguration;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), lds_bytes, stream, args);
     return hipGetLastError();
 }

@@ -62,3 +62,16 @@ status = lib.st_hip_gemm_f32(count, n, 1, 1.0, 0, closed, count, rhs.ctypes.data
 print(status, ctypes.c_void_p.in_dll(stub, "stub_first_source").value == closed)
 """)
     assert out == ["0", "True"]
+
+
+def test_bf16_attention_launches_pass_their_check(stub):
+    """Every grid the launchers of bf16 attention ask for passes the check made of it with the kernels' own decode."""
+    out = run(stub, """
+import itertools
+calls = 0
+for batch, heads, seq, dim, causal in itertools.product((1, 2, 3, 8), (1, 4, 7, 8), (1, 31, 32, 33, 64, 65, 128, 129, 500, 1000, 2048), (64, 128), (False, True)):
+    hip.attention_bf16_dev(batch, heads, seq, dim, 0.125, causal, 1 << 20, 2 << 20, 3 << 20, 3 * heads * dim, 4 << 20, heads * dim)
+    calls += 1
+print(calls == launches.value)
+""")
+    assert out == ["True"]
