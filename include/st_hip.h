@@ -208,6 +208,18 @@ typedef struct {
 int st_hip_conv2d_f32_split_plan(size_t batch, size_t c_in, size_t h, size_t w, size_t c_out, size_t kh, size_t kw, size_t stride_h,
                                  size_t stride_w, size_t pad_h, size_t pad_w, size_t dil_h, size_t dil_w, int direction,
                                  st_hip_conv2d_split_plan *split);
+/* How the bf16 convolution is cut (all 0 where it is refused): output channels and pixels per tile, workgroups along the reduction
+ * and the 64-term k-tiles each of them walks, the launcher's own check (`consistent`) and a walk over the whole grid (`items`
+ * must equal `workgroups`, `out_of_range` and `duplicates` must be 0). */
+typedef struct {
+    int tile_channels, tile_pixels;
+    int k_splits, k_tiles_per_split;
+    int consistent;
+    uint64_t workgroups, items, out_of_range, duplicates;
+} st_hip_conv2d_bf16_plan;
+int st_hip_conv2d_bf16_launch_plan(size_t batch, size_t c_in, size_t h, size_t w, size_t c_out, size_t kh, size_t kw, size_t stride_h,
+                                   size_t stride_w, size_t pad_h, size_t pad_w, size_t dil_h, size_t dil_w,
+                                   st_hip_conv2d_bf16_plan *plan);
 
 /* Conv2d::backward, crates/st-nn/src/layers/conv.rs:780-813 with col2im :860-916: from the forward input
  * (N, C_in, H, W), the OIHW weight and grad_output (N, C_out, OH, OW) computes

@@ -58,6 +58,11 @@ class ConvSplitPlan(ctypes.Structure):
         [(name, c_uint64) for name in ("image_bytes", "image_reach", "weight_bytes", "weight_reach")]
 
 
+class ConvBf16Plan(ctypes.Structure):
+    _fields_ = [(name, c_int) for name in ("tile_channels", "tile_pixels", "k_splits", "k_tiles_per_split", "consistent")] + \
+        [(name, c_uint64) for name in ("workgroups", "items", "out_of_range", "duplicates")]
+
+
 class DecoderConfig(ctypes.Structure):
     _fields_ = [
         ("vocab", c_size_t),
@@ -109,6 +114,7 @@ SIGNATURES = {
     "st_hip_conv2d_force_family": (c_int, [c_int]),
     "st_hip_conv2d_planned_kernel": (c_int, [c_size_t] * 13 + [c_int, POINTER(c_int)]),
     "st_hip_conv2d_f32_split_plan": (c_int, [c_size_t] * 13 + [c_int, POINTER(ConvSplitPlan)]),
+    "st_hip_conv2d_bf16_launch_plan": (c_int, [c_size_t] * 13 + [POINTER(ConvBf16Plan)]),
     "st_hip_attention_f32_launch_plan": (c_int, [c_size_t, c_size_t, c_size_t, c_int, c_int, POINTER(AttentionPlan)]),
     "st_hip_attention_f32_scaled_launch_plan": (c_int, [c_size_t, c_size_t, c_size_t, c_float, c_int, c_int, POINTER(AttentionPlan)]),
     "st_hip_gemm_row_block": (c_size_t, [c_size_t, c_size_t]),

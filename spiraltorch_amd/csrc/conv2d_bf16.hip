@@ -17,6 +17,7 @@
 // none slower.  More stages in flight (six and eight, one workgroup a unit) gain nothing, and 128×128 with four wavefronts
 // of one 64×64 each is slower than with eight that halve k (20.8 against 17.9 µs on the first).
 #include <algorithm>
+#include <vector>
 
 #include "device_math.h"
 #include "kernels.h"
@@ -126,6 +127,18 @@ __global__ __launch_bounds__(256) void conv_bf16_chunks_kernel(ConvBf16Args p)
     }
 }
 
+struct ConvBf16Item {
+    int split, tile_m, tile_n;
+};
+// Workgroup -> (run of k-tiles, tile): every XCD takes one contiguous run of tiles, those of the same pixels next to each other: they
+// share an L2.
+__host__ __device__ inline ConvBf16Item decode_conv_bf16_block(int grid, int k_splits, int tiles_m, int block)
+{
+    const int xcd = block & 7, more = grid & 7;
+    const int logical = xcd * (grid >> 3) + (xcd < more ? xcd : more) + (block >> 3), tile = logical / k_splits;
+    return ConvBf16Item{logical - tile * k_splits, tile % tiles_m, tile / tiles_m};
+}
+
 // Output channels 64·WM × pixels 64·WN by a workgroup of WM·WN·KS wavefronts, each 64×64 of it over a KS-th of every 64-wide
 // k-tile (a wavefront tile of 64×64 reads four fragments for four products, the least LDS traffic its accumulators allow).
 template <int WM, int WN, int KS, int STAGES>
@@ -141,13 +154,10 @@ __device__ __forceinline__ void conv_bf16_body(const ConvBf16Args &p)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ks = wave / (WM * WN), wm = wave / WN % WM, wn = wave % WN;
     const int li = lane & 31, lh = lane >> 5;
-    // Every XCD takes one contiguous run of tiles, those of the same pixels next to each other: they share an L2.
-    const int grid = static_cast<int>(gridDim.x), xcd = static_cast<int>(blockIdx.x) & 7;
-    int logical = xcd * (grid >> 3) + min(xcd, grid & 7) + (static_cast<int>(blockIdx.x) >> 3);
-    const int split = logical % p.k_splits;
-    logical /= p.k_splits;
+    const ConvBf16Item item = decode_conv_bf16_block(static_cast<int>(gridDim.x), p.k_splits, p.tiles_m, static_cast<int>(blockIdx.x));
+    const int split = item.split;
     const int tile0 = split * p.tiles_per_split, tiles = min(p.tiles_per_split, p.k_tiles - tile0);
-    const int m0 = logical % p.tiles_m * BM, n0 = logical / p.tiles_m * BN;
+    const int m0 = item.tile_m * BM, n0 = item.tile_n * BN;
 
     const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(p.weights, 0, static_cast<int>(p.weight_bytes), 0x00020000);
     const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc(p.images, 0, static_cast<int>(p.image_bytes), 0x00020000);
@@ -426,6 +436,56 @@ ConvBf16Plan plan_conv_bf16(const ConvShape &c, size_t k_tiles, bool may_split)
 
 size_t round_256(size_t bytes) { return (bytes + 255) & ~static_cast<size_t>(255); }
 
+// What the shape alone decides.
+void set_geometry(ConvBf16Args &args, const ConvShape &c)
+{
+    args.s = c;
+    // The copy holds the rows and columns the taps reach; of a kernel one row high (or one column wide) only those it is put on.
+    args.step_h = c.kh == 1 ? c.stride_h : 1;
+    args.step_w = c.kw == 1 ? c.stride_w : 1;
+    args.stride_h = c.kh == 1 ? 1 : c.stride_h;
+    args.stride_w = c.kw == 1 ? 1 : c.stride_w;
+    const size_t hp = static_cast<size_t>(c.oh - 1) * args.stride_h + static_cast<size_t>(c.kh - 1) * c.dil_h + 1;
+    const size_t wp = static_cast<size_t>(c.ow - 1) * args.stride_w + static_cast<size_t>(c.kw - 1) * c.dil_w + 1;
+    args.padded_w = static_cast<int>(wp);
+    args.padded_pixels = static_cast<int>(hp * wp);
+    args.channel_chunks = (c.c_in + 7) / 8;
+    args.taps = c.kh * c.kw;
+    args.chunks = args.channel_chunks * args.taps;
+    args.k_tiles = (args.chunks + 7) / 8;
+    args.spatial = c.oh * c.ow;
+    args.pixels = c.batch * args.spatial;
+    args.image_bytes = static_cast<unsigned>(static_cast<size_t>(c.batch) * args.channel_chunks * args.padded_pixels * 16);
+    args.weight_bytes = static_cast<unsigned>(static_cast<size_t>(args.chunks) * c.c_out * 16);
+}
+
+// How the plan cuts it; the number of workgroups.
+size_t set_tiles(ConvBf16Args &args, const ConvBf16Plan &plan)
+{
+    args.tiles_per_split = static_cast<int>((args.k_tiles + plan.k_splits - 1) / plan.k_splits);
+    args.k_splits = (args.k_tiles + args.tiles_per_split - 1) / args.tiles_per_split;
+    args.tiles_m = (args.s.c_out + plan.config->bm - 1) / plan.config->bm;
+    return plan.config->tiles(args.s) * args.k_splits;
+}
+
+bool conv_bf16_block_in_range(const ConvBf16Args &a, const ConvBf16Config &config, size_t grid, size_t block)
+{
+    const ConvBf16Item item = decode_conv_bf16_block(static_cast<int>(grid), a.k_splits, a.tiles_m, static_cast<int>(block));
+    return item.split >= 0 && item.split * static_cast<long long>(a.tiles_per_split) < a.k_tiles && item.split < a.k_splits && item.tile_m >= 0 &&
+           item.tile_m < a.tiles_m && item.tile_n >= 0 && item.tile_n * static_cast<long long>(config.bn) < a.pixels;
+}
+
+// The check before a launch: the grid is tiles × runs of k-tiles, tiles and runs cover the layer and none of them is empty.
+bool conv_bf16_consistent(const ConvBf16Args &a, const ConvBf16Config &config, size_t grid)
+{
+    if (a.k_splits < 1 || a.tiles_per_split < 1 || a.tiles_m < 1 || grid == 0 || grid > 0x7fffffffu) return false;
+    const size_t tiles_n = (static_cast<size_t>(a.pixels) + config.bn - 1) / config.bn;
+    if (grid != static_cast<size_t>(a.tiles_m) * tiles_n * a.k_splits) return false;
+    const long long rows = static_cast<long long>(a.tiles_m) * config.bm, k = static_cast<long long>(a.k_splits) * a.tiles_per_split;
+    if (rows < a.s.c_out || rows - config.bm >= a.s.c_out || k < a.k_tiles || k - a.tiles_per_split >= a.k_tiles) return false;
+    return conv_bf16_block_in_range(a, config, grid, 0) && conv_bf16_block_in_range(a, config, grid, grid - 1);
+}
+
 }  // namespace
 
 bool conv2d_bf16_supported(const ConvShape &c)
@@ -447,33 +507,15 @@ hipError_t launch_conv2d_bf16(const ConvShape &c, int activation, const uint16_t
     if (c.batch <= 0 || c.c_out <= 0 || c.oh <= 0 || c.ow <= 0) return hipSuccess;
     if (!conv2d_bf16_supported(c)) return hipErrorInvalidValue;
     ConvBf16Args args{};
+    set_geometry(args, c);
     args.input = input;
     args.weight = weight;
-    args.s = c;
-    // The copy holds the rows and columns the taps reach; of a kernel one row high (or one column wide) only those it is put on.
-    args.step_h = c.kh == 1 ? c.stride_h : 1;
-    args.step_w = c.kw == 1 ? c.stride_w : 1;
-    args.stride_h = c.kh == 1 ? 1 : c.stride_h;
-    args.stride_w = c.kw == 1 ? 1 : c.stride_w;
-    const size_t hp = static_cast<size_t>(c.oh - 1) * args.stride_h + static_cast<size_t>(c.kh - 1) * c.dil_h + 1;
-    const size_t wp = static_cast<size_t>(c.ow - 1) * args.stride_w + static_cast<size_t>(c.kw - 1) * c.dil_w + 1;
-    args.padded_w = static_cast<int>(wp);
-    args.padded_pixels = static_cast<int>(hp * wp);
-    args.channel_chunks = (c.c_in + 7) / 8;
-    args.taps = c.kh * c.kw;
-    args.chunks = args.channel_chunks * args.taps;
-    args.k_tiles = (args.chunks + 7) / 8;
     args.whole_chunks = c.c_in % 8 == 0 && args.taps <= kTapsPerPass && (reinterpret_cast<uintptr_t>(weight) & 15u) == 0;
-    args.spatial = c.oh * c.ow;
-    args.pixels = c.batch * args.spatial;
-    const size_t image_bytes = static_cast<size_t>(c.batch) * args.channel_chunks * hp * wp * 16;
-    const size_t weight_bytes = static_cast<size_t>(args.chunks) * c.c_out * 16, outputs = static_cast<size_t>(args.pixels) * c.c_out;
-    args.image_bytes = static_cast<unsigned>(image_bytes);
-    args.weight_bytes = static_cast<unsigned>(weight_bytes);
+    const size_t outputs = static_cast<size_t>(args.pixels) * c.c_out;
 
     ConvBf16Plan plan = plan_conv_bf16(c, static_cast<size_t>(args.k_tiles), true);
     args.offsets = (args.k_tiles + kMostStages + 1) * 8;
-    const size_t weights_at = round_256(image_bytes), offsets_at = weights_at + round_256(weight_bytes);
+    const size_t weights_at = round_256(args.image_bytes), offsets_at = weights_at + round_256(args.weight_bytes);
     const size_t partial_at = offsets_at + round_256(args.offsets * sizeof(unsigned));
     void *scratch = nullptr;
     hipError_t rc = stream_workspace(stream, partial_at + (plan.k_splits > 1 ? plan.k_splits * outputs * sizeof(float) : 0), &scratch);
@@ -488,18 +530,16 @@ hipError_t launch_conv2d_bf16(const ConvShape &c, int activation, const uint16_t
     args.weights = reinterpret_cast<uint16_t *>(base + weights_at);
     args.image_offsets = reinterpret_cast<unsigned *>(base + offsets_at);
     args.partial = reinterpret_cast<float *>(base + partial_at);
-    args.tiles_per_split = static_cast<int>((args.k_tiles + plan.k_splits - 1) / plan.k_splits);
-    args.k_splits = (args.k_tiles + args.tiles_per_split - 1) / args.tiles_per_split;
-    args.tiles_m = (c.c_out + config.bm - 1) / config.bm;
+    const size_t workgroups = set_tiles(args, plan);
+    if (!conv_bf16_consistent(args, config, workgroups)) return hipErrorInvalidConfiguration;
     const bool split = args.k_splits > 1;
     args.bias = split ? nullptr : bias;
     args.C32 = split ? nullptr : out_f32;
     args.C16 = split ? nullptr : out_bf16;
     args.activation = split ? ST_HIP_ACT_NONE : activation;
-    const size_t groups_px = (hp * wp + 255) / 256, image_groups = static_cast<size_t>(c.batch) * args.channel_chunks * groups_px;
+    const size_t groups_px = (static_cast<size_t>(args.padded_pixels) + 255) / 256, image_groups = static_cast<size_t>(c.batch) * args.channel_chunks * groups_px;
     const size_t weight_groups = static_cast<size_t>(args.channel_chunks) * ((c.c_out + 15) / 16);
-    const size_t workgroups = config.tiles(c) * args.k_splits;
-    if (image_groups + weight_groups + 1 > 0x7fffffffu || workgroups > 0x7fffffffu) return hipErrorInvalidConfiguration;
+    if (image_groups + weight_groups + 1 > 0x7fffffffu) return hipErrorInvalidConfiguration;
     args.groups_px = static_cast<unsigned>(groups_px);
     args.image_groups = static_cast<unsigned>(image_groups);
     args.weight_groups = static_cast<unsigned>(weight_groups);
@@ -521,6 +561,35 @@ hipError_t launch_conv2d_bf16(const ConvShape &c, int activation, const uint16_t
                        dim3(static_cast<unsigned>((outputs / (quads ? 4 : 1) + 255) / 256)), dim3(256), 0, stream, args, bias, activation, out_f32,
                        out_bf16);
     return hipGetLastError();
+}
+
+ConvBf16PlanReport conv2d_bf16_plan_report(const ConvShape &c)
+{
+    ConvBf16PlanReport report{};
+    if (c.batch <= 0 || c.c_out <= 0 || c.oh <= 0 || c.ow <= 0 || !conv2d_bf16_supported(c)) return report;
+    ConvBf16Args args{};
+    set_geometry(args, c);
+    const ConvBf16Plan plan = plan_conv_bf16(c, static_cast<size_t>(args.k_tiles), true);
+    const size_t grid = set_tiles(args, plan);
+    report.tile_channels = plan.config->bm;
+    report.tile_pixels = plan.config->bn;
+    report.k_splits = args.k_splits;
+    report.k_tiles_per_split = args.tiles_per_split;
+    report.consistent = conv_bf16_consistent(args, *plan.config, grid) ? 1 : 0;
+    report.workgroups = grid;
+    if (grid > (1u << 24)) return report;  // the walk is for tests
+    std::vector<unsigned char> seen(grid, 0);
+    for (size_t block = 0; block < grid; ++block) {
+        if (!conv_bf16_block_in_range(args, *plan.config, grid, block)) {
+            ++report.out_of_range;
+            continue;
+        }
+        const ConvBf16Item item = decode_conv_bf16_block(static_cast<int>(grid), args.k_splits, args.tiles_m, static_cast<int>(block));
+        unsigned char &cell = seen[(static_cast<size_t>(item.tile_n) * args.tiles_m + item.tile_m) * args.k_splits + item.split];
+        if (cell) ++report.duplicates; else ++report.items;
+        cell = 1;
+    }
+    return report;
 }
 
 }  // namespace sthip

@@ -569,6 +569,26 @@ int st_hip_conv2d_f32_split_plan(size_t batch, size_t c_in, size_t h, size_t w, 
     return ST_HIP_OK;
 }
 
+int st_hip_conv2d_bf16_launch_plan(size_t batch, size_t c_in, size_t h, size_t w, size_t c_out, size_t kh, size_t kw, size_t stride_h,
+                                   size_t stride_w, size_t pad_h, size_t pad_w, size_t dil_h, size_t dil_w, st_hip_conv2d_bf16_plan *plan)
+{
+    if (!plan) return fail(ST_HIP_ERR_INVALID, "conv2d launch_plan received a null out-pointer");
+    *plan = st_hip_conv2d_bf16_plan{};
+    ConvPlan conv;
+    ST_HIP_CHECK(plan_conv(batch, c_in, h, w, c_out, kh, kw, stride_h, stride_w, pad_h, pad_w, dil_h, dil_w, &conv));
+    const ConvBf16PlanReport report = conv2d_bf16_plan_report(conv.shape);
+    plan->tile_channels = report.tile_channels;
+    plan->tile_pixels = report.tile_pixels;
+    plan->k_splits = report.k_splits;
+    plan->k_tiles_per_split = report.k_tiles_per_split;
+    plan->consistent = report.consistent;
+    plan->workgroups = report.workgroups;
+    plan->items = report.items;
+    plan->out_of_range = report.out_of_range;
+    plan->duplicates = report.duplicates;
+    return ST_HIP_OK;
+}
+
 int st_hip_attention_f32_scaled_launch_plan(size_t contexts, size_t sequence, size_t head_dim, float scale, int causal, int biased,
                                             st_hip_attention_plan *plan)
 {

@@ -143,6 +143,12 @@ void set_conv_forced_family(int family);
 // The same convolution on bf16 images and weights (NCHW / OIHW bit patterns), f32 accumulation, f32 bias, f32 and/or bf16
 // output (either may be null).  Uses the stream's scratch buffer for the re-laid operands.
 bool conv2d_bf16_supported(const ConvShape &shape);
+// See st_hip_conv2d_bf16_launch_plan.
+struct ConvBf16PlanReport {
+    int tile_channels = 0, tile_pixels = 0, k_splits = 0, k_tiles_per_split = 0, consistent = 0;
+    unsigned long long workgroups = 0, items = 0, out_of_range = 0, duplicates = 0;
+};
+ConvBf16PlanReport conv2d_bf16_plan_report(const ConvShape &shape);
 hipError_t launch_conv2d_bf16(const ConvShape &shape, int activation, const uint16_t *input, const uint16_t *weight,
                               const float *bias, float *out_f32, uint16_t *out_bf16, hipStream_t stream);
 

@@ -212,6 +212,14 @@ def conv2d_f32_split_plan(batch, c_in, h, w, c_out, kernel, stride, padding, dil
     return {name: int(getattr(plan, name)) for name, _ in _lib.ConvSplitPlan._fields_}
 
 
+def conv2d_bf16_launch_plan(batch, c_in, h, w, c_out, kernel, stride, padding, dilation) -> dict:
+    """Tiling and split of the reduction of the bf16 convolution for a layer, with the whole grid decoded on the host."""
+    plan = _lib.ConvBf16Plan()
+    _check(_lib.load().st_hip_conv2d_bf16_launch_plan(batch, c_in, h, w, c_out, kernel[0], kernel[1], stride[0], stride[1], padding[0],
+                                                      padding[1], dilation[0], dilation[1], ctypes.byref(plan)))
+    return {name: int(getattr(plan, name)) for name, _ in _lib.ConvBf16Plan._fields_}
+
+
 def conv2d_bias_activation_f32(batch, c_in, h, w, c_out, kernel, stride, padding, dilation, activation,
                                input, weight, bias, out) -> None:
     x, wgt, out = _f32(input, "input"), _f32(weight, "weight"), _out(out, "out")

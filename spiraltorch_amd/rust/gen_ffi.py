@@ -18,7 +18,7 @@ SCALARS = {"size_t": "usize", "int": "c_int", "float": "f32", "uint64_t": "u64",
            "void": "c_void", "st_hip_device_props": "StHipDeviceProps", "st_hip_probe_result": "StHipProbeResult",
            "st_hip_decoder_config": "StHipDecoderConfig", "st_hip_attention_plan": "StHipAttentionPlan",
            "st_hip_gemm_tile_plan": "StHipGemmTilePlan", "st_hip_gemm_split_plan": "StHipGemmSplitPlan",
-           "st_hip_conv2d_split_plan": "StHipConv2dSplitPlan"}
+           "st_hip_conv2d_split_plan": "StHipConv2dSplitPlan", "st_hip_conv2d_bf16_plan": "StHipConv2dBf16Plan"}
 RUST_KEYWORDS = {"in": "input", "type": "kind", "ref": "reference"}
 
 STRUCTS = '''/// `st_hip_device_props`.
@@ -121,6 +121,21 @@ pub struct StHipConv2dSplitPlan {
     pub image_reach: u64,
     pub weight_bytes: u64,
     pub weight_reach: u64,
+}
+
+/// `st_hip_conv2d_bf16_plan`.
+#[repr(C)]
+#[derive(Clone, Copy, Debug, Default, PartialEq)]
+pub struct StHipConv2dBf16Plan {
+    pub tile_channels: c_int,
+    pub tile_pixels: c_int,
+    pub k_splits: c_int,
+    pub k_tiles_per_split: c_int,
+    pub consistent: c_int,
+    pub workgroups: u64,
+    pub items: u64,
+    pub out_of_range: u64,
+    pub duplicates: u64,
 }
 '''
 

@@ -107,6 +107,21 @@ pub struct StHipConv2dSplitPlan {
     pub weight_reach: u64,
 }
 
+/// `st_hip_conv2d_bf16_plan`.
+#[repr(C)]
+#[derive(Clone, Copy, Debug, Default, PartialEq)]
+pub struct StHipConv2dBf16Plan {
+    pub tile_channels: c_int,
+    pub tile_pixels: c_int,
+    pub k_splits: c_int,
+    pub k_tiles_per_split: c_int,
+    pub consistent: c_int,
+    pub workgroups: u64,
+    pub items: u64,
+    pub out_of_range: u64,
+    pub duplicates: u64,
+}
+
 #[link(name = "sthip")]
 extern "C" {
     pub fn st_hip_init() -> c_int;
@@ -144,6 +159,7 @@ extern "C" {
     pub fn st_hip_conv2d_force_family(family: c_int) -> c_int;
     pub fn st_hip_conv2d_planned_kernel(batch: usize, c_in: usize, h: usize, w: usize, c_out: usize, kh: usize, kw: usize, stride_h: usize, stride_w: usize, pad_h: usize, pad_w: usize, dil_h: usize, dil_w: usize, direction: c_int, kernel: *mut c_int) -> c_int;
     pub fn st_hip_conv2d_f32_split_plan(batch: usize, c_in: usize, h: usize, w: usize, c_out: usize, kh: usize, kw: usize, stride_h: usize, stride_w: usize, pad_h: usize, pad_w: usize, dil_h: usize, dil_w: usize, direction: c_int, split: *mut StHipConv2dSplitPlan) -> c_int;
+    pub fn st_hip_conv2d_bf16_launch_plan(batch: usize, c_in: usize, h: usize, w: usize, c_out: usize, kh: usize, kw: usize, stride_h: usize, stride_w: usize, pad_h: usize, pad_w: usize, dil_h: usize, dil_w: usize, plan: *mut StHipConv2dBf16Plan) -> c_int;
     pub fn st_hip_conv2d_backward_f32(batch: usize, c_in: usize, h: usize, w: usize, c_out: usize, kh: usize, kw: usize, stride_h: usize, stride_w: usize, pad_h: usize, pad_w: usize, dil_h: usize, dil_w: usize, input: *const f32, input_len: usize, weight: *const f32, weight_len: usize, grad_output: *const f32, grad_output_len: usize, grad_input: *mut f32, grad_input_len: usize, grad_weight: *mut f32, grad_weight_len: usize, grad_bias: *mut f32, grad_bias_len: usize) -> c_int;
     pub fn st_hip_attention_f32(contexts: usize, sequence: usize, head_dim: usize, scale: f32, causal: c_int, q: *const f32, q_len: usize, k: *const f32, k_len: usize, v: *const f32, v_len: usize, z_bias: *const f32, z_bias_len: usize, attn_bias: *const f32, attn_bias_len: usize, out: *mut f32, out_len: usize) -> c_int;
     pub fn st_hip_attention_f32_launch_plan(contexts: usize, sequence: usize, head_dim: usize, causal: c_int, biased: c_int, plan: *mut StHipAttentionPlan) -> c_int;

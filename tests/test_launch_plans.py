@@ -184,3 +184,20 @@ def test_split_convolutions_stay_inside_their_operands():
     assert hip.conv2d_planned_kernel(*layer, direction="grad_input") == "strip9"
     assert hip.conv2d_f32_split_plan(*layer, direction="grad_input")["served"] == 0
     assert hip.conv2d_f32_split_plan(2, 8, 9, 9, 4, (3, 3), (1, 1), (1, 1), (1, 1))["served"] == 0
+
+
+def test_bf16_convolution_grids_decode_to_every_run_and_tile_once():
+    tiles, cut = set(), set()
+    geometries = [((1, 1), (1, 1), (0, 0), (1, 1)), ((3, 3), (1, 1), (1, 1), (1, 1)), ((3, 3), (2, 2), (1, 1), (1, 1)), ((7, 7), (2, 2), (3, 3), (1, 1))]
+    for batch, c_in, side, c_out, geometry in itertools.product((1, 2, 13, 32), (3, 16, 65, 512), (7, 14, 29, 56), (1, 33, 64, 129, 288, 512), geometries):
+        plan = hip.conv2d_bf16_launch_plan(batch, c_in, side, side + 1, c_out, *geometry)
+        where = (batch, c_in, side, c_out, geometry, plan)
+        assert plan["consistent"] == 1 and plan["out_of_range"] == 0 and plan["duplicates"] == 0, where
+        assert plan["items"] == plan["workgroups"], where
+        k_tiles = -(-(-(-c_in // 8) * geometry[0][0] * geometry[0][1]) // 8)
+        assert plan["k_splits"] * plan["k_tiles_per_split"] >= k_tiles > (plan["k_splits"] - 1) * plan["k_tiles_per_split"], where
+        tiles.add((plan["tile_channels"], plan["tile_pixels"]))
+        cut.add(plan["k_splits"])
+    assert tiles == {(64, 64), (128, 64), (64, 128), (128, 128), (256, 128), (128, 256)} and len(cut) > 3, (tiles, cut)
+    # a layer whose operands' copies are too large for the kernels' offsets
+    assert hip.conv2d_bf16_launch_plan(64, 2048, 128, 128, 64, (1, 1), (1, 1), (0, 0), (1, 1))["workgroups"] == 0
