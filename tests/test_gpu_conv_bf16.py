@@ -43,21 +43,21 @@ def check(got, want, what):
 
 
 SHAPES = [
-    (2, 3, 9, 7, 4, (3, 3), (1, 1), (1, 1), (1, 1)),        # three channels padded to 64; a plane of 63 pixels (not a multiple of 4)
+    (2, 3, 9, 7, 4, (3, 3), (1, 1), (1, 1), (1, 1)),        # three channels padded to eight; a plane of 63 pixels (not a multiple of 4)
     (1, 2, 9, 9, 3, (3, 3), (1, 1), (0, 0), (2, 2)),        # dilation, no padding
     (3, 5, 6, 11, 7, (2, 4), (2, 3), (1, 2), (1, 1)),       # ragged kernel, strides and padding
     (2, 4, 5, 5, 6, (1, 1), (1, 1), (0, 0), (1, 1)),        # 1×1
     (1, 1, 4, 4, 1, (4, 4), (1, 1), (0, 0), (1, 1)),        # a single output value
-    (2, 64, 20, 20, 70, (3, 3), (1, 1), (1, 1), (1, 1)),    # one channel block, 800 pixels: several pixel tiles
-    (1, 70, 33, 17, 130, (5, 3), (2, 1), (2, 1), (1, 2)),   # two channel blocks (70 -> 128), 130 output channels (256-row tiles)
+    (2, 64, 20, 20, 70, (3, 3), (1, 1), (1, 1), (1, 1)),    # 800 pixels: several pixel tiles
+    (1, 70, 33, 17, 130, (5, 3), (2, 1), (2, 1), (1, 2)),   # 70 channels padded to 72, 130 output channels: three row tiles of 64
     (5, 128, 12, 12, 64, (3, 3), (2, 2), (0, 0), (1, 1)),   # planes of 25 pixels: a tile spans several images
-    (3, 192, 14, 14, 300, (3, 3), (1, 1), (1, 1), (1, 1)),  # three channel blocks, two row tiles of 256 channels
-    (40, 64, 28, 28, 256, (3, 3), (1, 1), (1, 1), (1, 1)),  # 31360 pixels × 256 channels: the 256×256 tiles
+    (3, 192, 14, 14, 300, (3, 3), (1, 1), (1, 1), (1, 1)),  # 27 k-tiles, five row tiles of 64 channels, the last ragged
+    (40, 64, 28, 28, 256, (3, 3), (1, 1), (1, 1), (1, 1)),  # 31360 pixels × 256 channels: 256×128 tiles
     (2, 16, 7, 7, 8, (7, 7), (1, 1), (3, 3), (1, 1)),       # 49 taps
-    (17, 8, 55, 53, 70, (3, 3), (1, 1), (1, 1), (1, 1)),    # 49555 pixels (odd planes) × 70 channels: pixels on the 256-row side
-    (16, 128, 64, 64, 128, (1, 1), (1, 1), (0, 0), (1, 1)), # the same tiling, two channel blocks, one tap
-    (2, 3, 3, 1000, 4, (1, 3), (1, 1), (0, 1), (1, 1)),     # rows wider than the re-layout tile: copied in pieces
-    (1, 5, 40, 225, 6, (3, 3), (1, 2), (2, 2), (1, 1)),     # one row per re-layout group, several rows of padding
+    (17, 8, 55, 53, 70, (3, 3), (1, 1), (1, 1), (1, 1)),    # 49555 pixels (odd planes) × 70 channels: 128×256 tiles
+    (16, 128, 64, 64, 128, (1, 1), (1, 1), (0, 0), (1, 1)), # the same tiles, one tap
+    (2, 3, 3, 1000, 4, (1, 3), (1, 1), (0, 1), (1, 1)),     # planes of a few long rows
+    (1, 5, 40, 225, 6, (3, 3), (1, 2), (2, 2), (1, 1)),     # rows that no group of 256 pixels holds, several rows of padding
 ]
 
 
@@ -144,22 +144,46 @@ def test_unsupported_and_invalid_arguments(hip):
     hip.conv2d_bias_act_bf16_dev(0, 3, 8, 8, 4, (3, 3), (1, 1), (1, 1), (1, 1), 0, d, d, None, d, None)
 
 
-@pytest.mark.parametrize("shape", [
-    (1, 64, 9, 9, 64, (3, 3), (1, 1), (1, 1), (1, 1)),       # 81 pixels: two 64-wide tiles, k cut over workgroups
-    (2, 72, 12, 11, 40, (5, 5), (1, 1), (2, 2), (1, 1)),     # 225 chunks: the last k-tile one eighth full; planes of 132
-    (1, 512, 5, 5, 96, (7, 7), (2, 2), (3, 3), (1, 1)),      # 392 k-tiles for nine pixels: many cuts, odd planes
-    (4, 20, 33, 47, 100, (1, 1), (2, 3), (0, 0), (1, 1)),    # one tap, strides: only the pixels it is put on are copied
-    (2, 9, 20, 21, 33, (1, 5), (3, 2), (1, 2), (2, 1)),      # one row of taps with stride and padding
-    (2, 9, 21, 20, 33, (5, 1), (2, 3), (2, 1), (1, 2)),      # one column
-    (1, 5, 30, 30, 17, (9, 9), (1, 1), (4, 4), (1, 1)),      # 81 taps: more than a pass of the weights takes
-    (1, 16, 30, 30, 17, (9, 9), (2, 2), (4, 4), (1, 1)),
-    (6, 128, 40, 40, 128, (3, 3), (1, 1), (1, 1), (1, 1)),   # 128-row tiles
-    (16, 24, 56, 56, 128, (3, 3), (1, 1), (1, 1), (1, 1)),   # wide tiles, ragged k
-    (9, 256, 47, 46, 288, (3, 3), (1, 1), (1, 1), (1, 1)),   # 256-row tiles, 288 channels
+G33 = ((3, 3), (1, 1), (1, 1), (1, 1))
+
+
+@pytest.mark.parametrize("shape,tile,cut", [
+    ((1, 64, 9, 9, 64, *G33), (64, 64), False),                               # 81 pixels: two tiles
+    ((2, 72, 12, 11, 40, (5, 5), (1, 1), (2, 2), (1, 1)), (64, 64), True),    # 225 chunks: the last k-tile one eighth full; planes of 132
+    ((1, 512, 5, 5, 96, (7, 7), (2, 2), (3, 3), (1, 1)), (64, 64), True),     # 392 k-tiles for nine pixels: many cuts, odd planes
+    ((4, 20, 33, 47, 100, (1, 1), (2, 3), (0, 0), (1, 1)), (64, 64), False),  # one tap, strides: only the pixels it is put on are copied
+    ((2, 9, 20, 21, 33, (1, 5), (3, 2), (1, 2), (2, 1)), (64, 64), False),    # one row of taps with stride and padding
+    ((2, 9, 21, 20, 33, (5, 1), (2, 3), (2, 1), (1, 2)), (64, 64), False),    # one column
+    ((1, 5, 30, 30, 17, (9, 9), (1, 1), (4, 4), (1, 1)), (64, 64), False),    # 81 taps: more than a pass of the weights takes
+    ((1, 16, 30, 30, 17, (9, 9), (2, 2), (4, 4), (1, 1)), (64, 64), True),
+    ((6, 128, 40, 40, 128, *G33), (64, 64), False),                           # more tiles than compute units
+    # every other tile: a single k-tile with a ragged channel block and odd planes, and even and odd numbers of k-tiles
+    ((20, 3, 38, 39, 17, (1, 1), (1, 1), (0, 0), (1, 1)), (64, 128), False),
+    ((32, 30, 33, 34, 40, *G33), (64, 128), False),
+    ((32, 96, 13, 14, 257, *G33), (64, 128), False),
+    ((13, 100, 23, 24, 17, (7, 7), (1, 1), (3, 3), (1, 1)), (64, 128), True),
+    ((9, 3, 37, 37, 72, (1, 1), (1, 1), (0, 0), (1, 1)), (128, 64), False),
+    ((7, 30, 56, 56, 72, *G33), (128, 64), False),
+    ((9, 40, 25, 28, 200, *G33), (128, 64), False),
+    ((2, 96, 37, 40, 72, (7, 7), (1, 1), (3, 3), (1, 1)), (128, 64), True),
+    ((7, 512, 41, 42, 72, (3, 3), (2, 2), (1, 1), (1, 1)), (128, 64), True),
+    ((7, 3, 59, 59, 72, (1, 1), (1, 1), (0, 0), (1, 1)), (128, 128), False),
+    ((20, 30, 25, 28, 150, (5, 5), (1, 1), (2, 2), (1, 1)), (128, 128), False),
+    ((13, 24, 33, 34, 200, (5, 5), (1, 1), (2, 2), (1, 1)), (128, 128), False),
+    ((13, 3, 41, 41, 130, (1, 1), (1, 1), (0, 0), (1, 1)), (256, 128), False),
+    ((13, 30, 44, 47, 150, *G33), (256, 128), False),
+    ((9, 96, 52, 52, 130, *G33), (256, 128), False),
+    ((20, 3, 50, 53, 72, (1, 1), (1, 1), (0, 0), (1, 1)), (128, 256), False),
+    ((20, 30, 53, 56, 72, *G33), (128, 256), False),
+    ((20, 24, 51, 54, 72, (5, 5), (1, 1), (2, 2), (1, 1)), (128, 256), False),
+    ((16, 24, 56, 56, 128, *G33), (128, 256), False),                         # three and a half k-tiles
+    ((9, 256, 47, 46, 288, *G33), (128, 256), False),                         # 36 k-tiles, a ragged row tile
 ])
-def test_tiles_chunks_and_cuts_of_k(hip, shape):
+def test_tiles_chunks_and_cuts_of_k(hip, shape, tile, cut):
     """Every tile and route of conv2d_bf16.hip against float64: exact products, so a sum of k of them is off by at most k f32
     roundings of the sum of magnitudes.  Both outputs, bias and ReLU; the same bits from call to call."""
+    plan = hip.conv2d_bf16_launch_plan(*shape)
+    assert (plan["tile_channels"], plan["tile_pixels"], plan["k_splits"] > 1) == (*tile, cut), plan
     import torch
     import torch.nn.functional as F
     from spiraltorch_amd import inputs
