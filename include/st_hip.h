@@ -286,6 +286,12 @@ typedef struct {
     uint64_t workgroups, items, out_of_range, duplicates;
 } st_hip_gemm_tile_plan;
 int st_hip_gemm_bf16_tile_plan(size_t m, size_t n, size_t k, st_hip_gemm_tile_plan *plan);
+/* Which of these an m×n×k product (k a multiple of 64, a prepacked B, 16-byte aligned operands) meets: the small tiles for products of
+ * few tiles, the second launch for the columns behind the last full round of 256×256 tiles, and the single kernel of
+ * st_hip_gemm_bf16_prepacked_residual_layer_norm_dev.  0 where none.  (Rows that the kernel for at most 32 of them takes, and
+ * what the persistent kernel takes, is described as if it were not.) */
+enum { ST_HIP_GEMM_BF16_SMALL_TILES = 1, ST_HIP_GEMM_BF16_COLUMNS_BEHIND = 2, ST_HIP_GEMM_BF16_RESIDUAL_LAYER_NORM = 4 };
+int st_hip_gemm_bf16_routes(size_t m, size_t n, size_t k);
 /* Whether the f32 GEMM entry points run an m×n×k product of 16-byte aligned operands on the bf16 matrix cores, as products of
  * three exact bf16 pieces per value (`served`; the rest is 0 if not), and how it is cut: tiles, workgroups along k, 16-term
  * steps each of them walks, the size of the split operands in the stream's scratch memory and how far into each the

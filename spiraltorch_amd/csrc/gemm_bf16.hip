@@ -2277,15 +2277,21 @@ hipError_t launch_128(GemmBf16Args args, bool packed, hipStream_t stream, size_t
 // takes as long as a full one: where the columns behind the full rounds are at most 256 tiles of 128×128, those run them, two
 // workgroups a unit, in a launch of their own.  Same sums in the same order.  1024×50257×768: 154 -> 131 µs, 1500×33333×384
 // 112 -> 96.
+size_t columns_behind_rounds(size_t m, size_t n, const TilePlan &plan)
+{
+    if (plan.narrow || plan.k_splits != 1 || plan.tiles <= 256) return 0;
+    const size_t whole = plan.tiles / 256 * 256 / ((m + 255) / 256) * 256;  // columns of the full rounds
+    return whole > 0 && whole < n && (m + 127) / 128 * ((n - whole + 127) / 128) <= 256 ? n - whole : 0;
+}
+
 hipError_t launch_256_rounds(GemmBf16Args args, bool packed, const TilePlan &plan, hipStream_t stream, size_t workspace_offset)
 {
-    const size_t m = static_cast<size_t>(args.M), n = static_cast<size_t>(args.N), row_tiles = (m + 255) / 256;
-    const size_t whole = plan.tiles / 256 * 256 / row_tiles * 256;  // columns of the full rounds
-    if (plan.k_splits == 1 && plan.tiles > 256 && whole > 0 && whole < n && (m + 127) / 128 * ((n - whole + 127) / 128) <= 256) {
+    const size_t behind = columns_behind_rounds(static_cast<size_t>(args.M), static_cast<size_t>(args.N), plan);
+    if (behind > 0) {
         GemmBf16Args rest = args;
-        args.columns = static_cast<int>(whole);
-        rest.first_col = static_cast<int>(whole);
-        rest.columns = static_cast<int>(n - whole);
+        args.columns = args.N - static_cast<int>(behind);
+        rest.first_col = args.columns;
+        rest.columns = static_cast<int>(behind);
         const hipError_t rc = launch_256<256>(args, packed, stream, workspace_offset);
         return rc == hipSuccess ? launch_128(rest, packed, stream) : rc;
     }
@@ -2682,6 +2688,24 @@ GemmTilePlanReport gemm_bf16_tile_plan_report(size_t m, size_t n, size_t k)
     return report;
 }
 
+// Measured at m = 16384 (one 64-row workgroup per compute unit): 27.3 µs against 18.2 + 10.2 µs for the two kernels at
+// k = 512, 51.2 against 37.9 + 10.1 µs at k = 2048 — a 64-row tile streams the whole of B through every compute unit,
+// which costs more than the saved pass over the rows once k is long.
+// (m <= 64 stays with the GEMM dispatcher, which splits k over the chip for such shapes, and so does every shape of
+// few row tiles and a long k that the dispatcher would split or give to the small tiles: those sums add up in another order.)
+bool residual_layer_norm_single(size_t m, size_t n, size_t k)
+{
+    return n == 512 && m > 64 && k >= 64 && k % 64 == 0 && k <= 1024 && m * k * 2 < (1ull << 31) && plan_tiles(m, n, k).k_splits == 1 &&
+           !small_tiles_apply(m, n, k);
+}
+
+int gemm_bf16_routes(size_t m, size_t n, size_t k)
+{
+    if (m == 0 || n == 0 || k < 64 || k % 64 != 0 || m * k * 2 >= (1ull << 31) || k * n * 2 >= (1ull << 31)) return 0;
+    return (small_tiles_apply(m, n, k) ? ST_HIP_GEMM_BF16_SMALL_TILES : columns_behind_rounds(m, n, plan_tiles(m, n, k)) > 0 ? ST_HIP_GEMM_BF16_COLUMNS_BEHIND : 0) |
+           (residual_layer_norm_single(m, n, k) ? ST_HIP_GEMM_BF16_RESIDUAL_LAYER_NORM : 0);
+}
+
 // out_f32 = (lhs·rhs + bias) + residual, out_ln = layer_norm(out_f32; gamma, beta, epsilon) rounded to bf16; rhs packed n×k.
 // n = 512 with k a multiple of 64 up to 1024 and 16-byte aligned operands runs as ONE kernel (the row-complete GEMM above with the
 // normalisation in its epilogue); every other shape as the GEMM followed by the layer-norm kernel.
@@ -2690,16 +2714,9 @@ hipError_t launch_gemm_bf16_residual_layer_norm(size_t m, size_t n, size_t k, co
                                                 float epsilon, float *out_f32, uint16_t *out_ln, hipStream_t stream)
 {
     if (m == 0 || n == 0) return hipSuccess;
-    const bool fits_buffer = m * k * 2 < (1ull << 31) && k * n * 2 < (1ull << 31);
     const bool aligned = aligned16(lhs) && aligned16(packed_rhs) && aligned16(bias) && aligned16(residual) && aligned16(gamma) &&
                          aligned16(beta) && aligned16(out_f32) && (reinterpret_cast<uintptr_t>(out_ln) & 7u) == 0;
-    // Measured at m = 16384 (one 64-row workgroup per compute unit): 27.3 µs against 18.2 + 10.2 µs for the two kernels at
-    // k = 512, 51.2 against 37.9 + 10.1 µs at k = 2048 — a 64-row tile streams the whole of B through every compute unit,
-    // which costs more than the saved pass over the rows once k is long.
-    // (m <= 64 stays with the GEMM dispatcher, which splits k over the chip for such shapes, and so does every shape of
-    // few row tiles and a long k that the dispatcher would split or give to the small tiles: those sums add up in another order.)
-    if (n == 512 && m > 64 && k >= 64 && k % 64 == 0 && k <= 1024 && fits_buffer && aligned && plan_tiles(m, n, k).k_splits == 1 &&
-        !small_tiles_apply(m, n, k)) {
+    if (aligned && residual_layer_norm_single(m, n, k)) {
         RowLnArgs row;
         row.g.A = lhs;
         row.g.B = packed_rhs;

@@ -666,6 +666,11 @@ int st_hip_gemm_bf16_tile_plan(size_t m, size_t n, size_t k, st_hip_gemm_tile_pl
     return ST_HIP_OK;
 }
 
+int st_hip_gemm_bf16_routes(size_t m, size_t n, size_t k)
+{
+    return m > kMaxDim || n > kMaxDim || k > kMaxDim ? 0 : gemm_bf16_routes(m, n, k);
+}
+
 int st_hip_gemm_f32_split_plan(size_t m, size_t n, size_t k, int lhs_transposed, int rhs_packed, st_hip_gemm_split_plan *plan)
 {
     if (!plan) return fail(ST_HIP_ERR_INVALID, "gemm split_plan received a null out-pointer");

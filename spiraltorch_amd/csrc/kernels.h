@@ -86,6 +86,7 @@ struct GemmTilePlanReport {
     uint64_t workgroups, items, out_of_range, duplicates;
 };
 GemmTilePlanReport gemm_bf16_tile_plan_report(size_t m, size_t n, size_t k);
+int gemm_bf16_routes(size_t m, size_t n, size_t k);  // see st_hip_gemm_bf16_routes
 
 // out_f32 = (lhs·rhs + bias) + residual and out_ln = layer_norm(out_f32) rounded to bf16, rhs packed n×k: Linear + residual +
 // LayerNorm of a transformer block (crates/st-vision/src/models/vit.rs:256-265) in one launch where the shape allows.

@@ -266,6 +266,15 @@ def gemm_bf16_tile_plan(m: int, n: int, k: int) -> dict:
     return {name: int(getattr(plan, name)) for name, _ in _lib.GemmTilePlan._fields_}
 
 
+GEMM_BF16_ROUTES = {1: "small_tiles", 2: "columns_behind", 4: "residual_layer_norm"}
+
+
+def gemm_bf16_routes(m: int, n: int, k: int) -> set:
+    """Which of the special kernels a bf16 product of these sizes meets."""
+    bits = int(_lib.load().st_hip_gemm_bf16_routes(m, n, k))
+    return {name for bit, name in GEMM_BF16_ROUTES.items() if bits & bit}
+
+
 def gemm_f32_split_plan(m: int, n: int, k: int, lhs_transposed: bool = False, rhs_packed: bool = False) -> dict:
     """Whether and how the f32 GEMM runs a product as products of three exact bf16 pieces per value."""
     plan = _lib.GemmSplitPlan()

@@ -165,6 +165,7 @@ extern "C" {
     pub fn st_hip_attention_f32_launch_plan(contexts: usize, sequence: usize, head_dim: usize, causal: c_int, biased: c_int, plan: *mut StHipAttentionPlan) -> c_int;
     pub fn st_hip_attention_f32_scaled_launch_plan(contexts: usize, sequence: usize, head_dim: usize, scale: f32, causal: c_int, biased: c_int, plan: *mut StHipAttentionPlan) -> c_int;
     pub fn st_hip_gemm_bf16_tile_plan(m: usize, n: usize, k: usize, plan: *mut StHipGemmTilePlan) -> c_int;
+    pub fn st_hip_gemm_bf16_routes(m: usize, n: usize, k: usize) -> c_int;
     pub fn st_hip_gemm_f32_split_plan(m: usize, n: usize, k: usize, lhs_transposed: c_int, rhs_packed: c_int, plan: *mut StHipGemmSplitPlan) -> c_int;
     pub fn st_hip_gemm_row_block(k: usize, element_bytes: usize) -> usize;
     pub fn st_hip_gemm_f32_dev(m: usize, n: usize, k: usize, scale: f32, lhs_transposed: c_int, lhs: *const f32, rhs: *const f32, out: *mut f32, stream: *mut c_void) -> c_int;

@@ -240,16 +240,23 @@ def test_skinny_prepacked_single_launch(hip, oracle, m, n, k):
         assert (d16.to_array(np.uint16, m * n) == inputs.to_bf16(got32)).all()
 
 
-@pytest.mark.parametrize("m,n,k", [(65, 512, 64), (1000, 512, 512), (16384, 512, 192), (130, 512, 2048), (1, 512, 128), (65, 512, 1024), (300, 512, 1024),
-                                   (64, 512, 512), (256, 512, 1024),
-                                   # other widths: the GEMM and the layer-norm kernel one after the other
-                                   (300, 384, 128), (33, 512, 96), (70, 1024, 256)])
+# one kernel: whole and ragged row tiles of 64, one k-tile, few and the most
+SINGLE_KERNEL = [(16384, 512, 192), (1601, 512, 64), (2049, 512, 512), (3007, 512, 576), (2240, 512, 1024)]
+
+
+@pytest.mark.parametrize("m,n,k", SINGLE_KERNEL +
+                         # few rows: the small tiles, or k split, and the layer-norm kernel behind them
+                         [(65, 512, 64), (1000, 512, 512), (130, 512, 2048), (1, 512, 128), (65, 512, 1024), (300, 512, 1024),
+                          (64, 512, 512), (256, 512, 1024),
+                          # other widths
+                          (300, 384, 128), (33, 512, 96), (70, 1024, 256)])
 def test_gemm_residual_layer_norm(hip, oracle, m, n, k):
     """Linear + residual + LayerNorm in one call: the rows before normalisation against the oracle's GEMM (+ bias +
     residual), the normalised bf16 rows against the oracle's layer-norm of those rows (within one bf16 step: the
     row statistics are summed in another order), and against the separate GEMM and layer-norm kernels (the same
     arithmetic in the same order: equal bits)."""
     from spiraltorch_amd import inputs
+    assert ("residual_layer_norm" in hip.gemm_bf16_routes(m, n, k)) == ((m, n, k) in SINGLE_KERNEL)
     rng = np.random.default_rng(m + 3 * n + 5 * k)
     a, b = bf16_pair(rng, m, n, k, std=0.5)
     bias = rng.normal(size=n).astype(np.float32)

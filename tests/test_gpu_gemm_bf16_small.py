@@ -66,15 +66,18 @@ def test_small_tiles_of_non_finite_operands(hip):
     assert np.isfinite(np.delete(got, (7, 44), axis=0)).all()
 
 
-@pytest.mark.parametrize("m,n,k,layouts", [
-    (1024, 16600, 64, "p"), (1024, 16641, 192, "pr"),  # 260 and 264 tiles of 256×256; columns off every boundary
-    (1000, 16640, 128, "pr"), (2049, 8064, 64, "pr"),  # a multiple of 128; ragged rows
-    (300, 33024, 64, "p"),                             # 258 tiles: one column of tiles behind the full round
+@pytest.mark.parametrize("m,n,k,layouts,behind", [
+    (1024, 49408, 64, "pr", 256), (2048, 24832, 128, "r", 256),   # 772 and 776 tiles of 256×256, B as it is
+    (1024, 50257, 64, "p", 1105), (2047, 24700, 192, "pr", 124),  # columns off every boundary, ragged rows; a row-major B packed first
+    # a last round of a few tiles as well, but in tiles of 256×128 throughout
+    (1024, 16600, 64, "p", 0), (1024, 16641, 192, "pr", 0), (1000, 16640, 128, "pr", 0), (2049, 8064, 64, "pr", 0), (300, 33024, 64, "p", 0),
 ])
-def test_columns_behind_the_full_rounds(hip, m, n, k, layouts):
+def test_columns_behind_the_full_rounds(hip, m, n, k, layouts, behind):
     """A last round of a few 256×256 tiles runs as 128×128 tiles in a launch of its own: every column against float64 (the bound
-    as above), and the columns of the first round bit for bit what a product of those alone gives."""
+    as above), and the columns of the full rounds bit for bit what a product of those alone gives."""
     from spiraltorch_amd import inputs
+    assert ("columns_behind" in hip.gemm_bf16_routes(m, n, k)) == (behind > 0)
+    whole = n - behind
     rng = np.random.default_rng(m + n + k)
     a, b = inputs.to_bf16(rng.normal(size=m * k).astype(np.float32)), inputs.to_bf16(rng.normal(size=n * k).astype(np.float32))
     bias = rng.normal(size=n).astype(np.float32)
@@ -84,6 +87,11 @@ def test_columns_behind_the_full_rounds(hip, m, n, k, layouts):
     d_r = hip.DeviceBuffer.from_array(np.ascontiguousarray(b.reshape(n, k).T))
     d32, d16 = hip.DeviceBuffer((m * n + 64) * 4), hip.DeviceBuffer(m * n * 2)
     bits = []
+    if behind:
+        assert not hip.gemm_bf16_routes(m, whole, k) and hip.gemm_bf16_tile_plan(m, whole, k)["tile_cols"] == 256
+        hip.gemm_bf16_prepacked_bias_act_dev(m, whole, k, 0, d_a, d_p, d_bias, None, d32, d16)
+        hip.device_synchronize()
+        first = d32.to_array(np.float32, m * whole).reshape(m, whole)
     for layout in layouts:
         d32.zero()
         call, operand = (hip.gemm_bf16_prepacked_bias_act_dev, d_p) if layout == "p" else (hip.gemm_bf16_bias_act_dev, d_r)
@@ -94,4 +102,6 @@ def test_columns_behind_the_full_rounds(hip, m, n, k, layouts):
         bits.append(got[:m * n].reshape(m, n))
         assert (np.abs(bits[-1] - want) <= bound).all(), layout
         assert (d16.to_array(np.uint16, m * n) == inputs.to_bf16(got[:m * n])).all()
+        if behind:
+            assert (bits[-1][:, :whole] == first).all(), layout
     assert all((x == bits[0]).all() for x in bits)
