@@ -1821,12 +1821,17 @@ hipError_t launch_split_rows(AttnArgs args, hipStream_t stream)
 // (causal 27.7 / 9.8), 1 × 1000 15.4 / 12.6 (biased 16.8 / 13.3), 4 × 500 15.4 / 12.8, 8 × 1000 27.4 / 24.8, 32 × 250 18.0 / 10.8; the error
 // against float64 3.2e-7 / 2.4e-7.  Beyond a round or some length the 128-row tiles, which read K and V a quarter as often and cut
 // them once for four wavefronts, are level or ahead: 32 × 500 26.2 / 27.6, 4 × 1000 in one run each 20.3 / 22.7, 1 × 2048 20.8 / 34.8;
-// up to 32 queries (64 with biases), where one or two wavefronts have all keys, they have less to put together: 8 × 16 5.8 / 6.7,
-// 6 × 40 biased 7.2 / 7.6.
-size_t keys_shared(size_t contexts, size_t sequence, bool biased, size_t *keys_per_split)
+// up to 32 queries (64 with biases, or in a head padded to 64 values without the causal mask), where one or two wavefronts have all
+// keys, they have less to put together: 8 × 16 5.8 / 6.7, 6 × 40 biased 7.2 / 7.6, 4 × 64 of 56 values 6.3 / 6.6.
+// More than 512 keys in one run, over 500 calls: heads of up to 32 values gain up to 1024 keys (0.73 to 0.98 of the time); the wider
+// ones only while the round is full enough that the 128-row tiles, in a quarter of the workgroups, leave units idle.  With 129 to 160
+// workgroups 5 × 680 keys 0.98 of the time, 5 × 830 1.03, 5 × 1000 causal 1.11 to 1.17; 161 to 224 not causal 0.83 to 0.95 throughout,
+// causal 1.00 at 6 × 890, 1.08 to 1.16 beyond; 225 to 256 0.80 to 0.90.
+size_t keys_shared(size_t contexts, size_t sequence, size_t head_dim, bool causal, bool biased, size_t *keys_per_split)
 {
     const size_t workgroups = contexts * ((sequence + kKeysRows - 1) / kKeysRows);
-    if (sequence <= (biased ? 64 : 32) || workgroups > 256) return 0;
+    const bool padded = head_dim > 32 && head_dim < 64;
+    if (sequence <= (biased || (padded && !causal) ? 64 : 32) || workgroups > 256) return 0;
     auto us = [&](size_t splits, size_t keys) { return 5.5 + 1.9 * static_cast<double>((keys + 127) / 128) + (splits > 1 ? 4.5 : 0.0); };
     size_t best = 1, best_keys = sequence;
     for (size_t splits = 2; splits * workgroups <= 256 && splits * 128 < sequence + 128; ++splits) {
@@ -1834,7 +1839,8 @@ size_t keys_shared(size_t contexts, size_t sequence, bool biased, size_t *keys_p
         if (keys <= 256 && (splits - 1) * keys < sequence && us(splits, keys) < us(best, best_keys)) best = splits, best_keys = keys;
     }
     *keys_per_split = best_keys;
-    return best_keys <= 512 || (workgroups > 128 && sequence <= 1024) ? best : 0;
+    const size_t longest = head_dim <= 32 || workgroups > 224 ? 1024 : workgroups > 160 ? (causal ? 896 : 1024) : 768;
+    return best_keys <= 512 || (workgroups > 128 && best_keys <= longest) ? best : 0;
 }
 
 bool keys_block_in_range(const AttnArgs &args, size_t block)
@@ -1883,7 +1889,7 @@ template <int DPAD, bool CAUSAL, bool BIAS>
 hipError_t launch_split(AttnArgs args, hipStream_t stream)
 {
     size_t keys = 0;
-    if (const size_t splits = keys_shared(args.contexts, args.S, BIAS, &keys)) {
+    if (const size_t splits = keys_shared(args.contexts, args.S, args.D, CAUSAL, BIAS, &keys)) {
         args.key_splits = static_cast<int>(splits);
         args.keys_per_split = static_cast<int>(keys);
         return launch_keys<DPAD, CAUSAL, BIAS>(args, stream);
@@ -1949,7 +1955,7 @@ AttentionPlanReport attention_f32_plan_report(size_t contexts, size_t sequence, 
         return report;
     }
     size_t keys = 0, runs = 0;
-    if (report.kernel == ST_HIP_ATTN_KERNEL_SPLIT && (runs = keys_shared(contexts, sequence, biased, &keys)) > 0) {
+    if (report.kernel == ST_HIP_ATTN_KERNEL_SPLIT && (runs = keys_shared(contexts, sequence, head_dim, causal, biased, &keys)) > 0) {
         args.q_tiles = (args.S + kKeysRows - 1) / kKeysRows;
         report.key_splits = args.key_splits = static_cast<int>(runs);
         report.keys_per_split = args.keys_per_split = static_cast<int>(keys);
