@@ -815,12 +815,15 @@ hipError_t launch_conv2d_grad_weight_f32(const ConvShape &shape, const float *in
     const long long big_cover = static_cast<long long>((shape.c_out + 127) / 128 * 128) * ((S + 191) / 192 * 192);
     // Nor where they have little to sum, or run in rounds of 256 workgroups of which the last is mostly empty (the small ones, four a
     // unit, take a third more time a value).  Big / small, µs, batch × channels, side: 1×64 -> 128, 4, 3×3 11.0 / 7.5; 4×512 -> 256, 4, 3×3
-    // 21.3 / 15.5; 16×512 -> 512, 7, 3×3 (64 steps) 65.8 / 80.0; with 268 tiles 2×512 -> 512, 7, 5×5 61 / 49 and 32 images 365 / 289; with 524
+    // 21.3 / 15.5; 16×512 -> 512, 7, 3×3 (64 steps) 65.8 / 80.0.  With a step or less for each of 256 workgroups 20.8 / 14.0 (1×64 -> 512, 18, 3×3
+    // and 92 other layers of 17 to 128 steps), with two to four 25 / 20, four to six 28.6 / 24.6, six to ten 32.6 / 29.6, ten to twenty
+    // 41 / 42, beyond 69 / 76.  With 268 tiles 2×512 -> 512, 7, 5×5 61 / 49 and 32 images 365 / 289; with 524
     // 2×512 -> 512, 2×7, 7×7 72 / 61 and 32 images of 7 554 / 510.
     const long long steps_per_image = (args.spatial + 15) / 16, total_steps = steps_per_image * shape.batch;
     const long long big_tiles = static_cast<long long>((shape.c_out + 127) / 128) * ((S + 191) / 192);
     const bool full_rounds = big_tiles <= 256 || (big_tiles + 255) / 256 * 256 * 5 <= big_tiles * 6;
-    const bool big = big_cover * 10 <= static_cast<long long>(count) * 12 && total_steps > 16 && full_rounds;  // (of 107 channels at least: never kValues)
+    const bool big = big_cover * 10 <= static_cast<long long>(count) * 12 && total_steps > 16 && total_steps * big_tiles >= 6 * 256 &&
+                     full_rounds;  // (of 107 channels at least: never kValues)
     const int bm = big ? 128 : 64, bn = big ? 192 : 64;
     args.tiles_s = (S + bn - 1) / bn;
     const int tiles = args.tiles_s * ((shape.c_out + bm - 1) / bm);
