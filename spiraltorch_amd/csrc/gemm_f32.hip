@@ -931,10 +931,12 @@ bool f32_split_preferred(size_t m, size_t n, size_t k, bool lhs_transposed, bool
     return gemm_f32_split_applies(m, n, k, f32_kernels_us(m, n, k, lhs_transposed, rhs_packed, lhs, rhs, scratch_free), scratch_free);
 }
 
-// The same for products of few tiles, µs (within a fifth of some hundred from 8 rows up), and whether the small tiles of
+// The same for products of few tiles, µs (nine in ten of some thousand from one row up within a third), and whether the small tiles of
 // gemm_f32_small.hip beat it.  What the kernels here take grows with the k-tiles a workgroup walks, up to where k is sliced; the
-// ring kernel that splits k inside a workgroup is the least of them.  (Asked after the split products: those keep the shapes they
-// take, with fewer roundings.)
+// ring kernel that splits k inside a workgroup is the least of them: from k = 2048 on it also slices k over workgroups, 3 µs for the
+// launch that adds them (few tiles: k = 2000 9.8 µs, 2100 8.9, 3000 10.6, 3200 8.9; counted as one slice, 3392 terms were
+// estimated at 13.8 µs, and 37×896×3520 went to the small tiles, 14.1 µs instead of 10.2).  (Asked after the split products: those
+// keep the shapes they take, with fewer roundings.)
 bool f32_small_preferred(size_t m, size_t n, size_t k, bool lhs_transposed, bool rhs_packed, const float *lhs, const float *rhs)
 {
     const double flops = 2.0 * m * n * k, k_tiles = static_cast<double>((k + 15) / 16);
@@ -943,8 +945,11 @@ bool f32_small_preferred(size_t m, size_t n, size_t k, bool lhs_transposed, bool
     double us;
     if (lhs_transposed) us = 4.1 + (ring ? 0.30 : rows ? 0.40 : 0.48) * std::min(k_tiles, 25.0) + flops / 100.0e6;
     else if (rhs_packed) us = (ring ? 4.0 + 0.30 * std::min(k_tiles, 23.0) : 6.8 + 0.60 * k_tiles) + flops / 100.0e6;
-    else if (ring) us = (k >= 128 ? 3.2 + 0.05 * k_tiles : 5.2) + flops / 90.0e6;
-    else us = 4.2 + 0.55 * std::min(k_tiles, 24.0) + flops / 100.0e6;
+    else if (ring && k >= 128) {
+        const size_t slices = choose_k_slices(m, n, k, (m + 31) / 32 * ((n + 31) / 32), k / 16, 64);
+        us = 3.2 + 0.05 * k_tiles / static_cast<double>(slices) + (slices > 1 ? 3.0 : 0.0) + flops / 130.0e6;
+    } else if (ring) us = 5.2 + flops / 90.0e6;
+    else us = (4.2 + 0.55 * std::min(k_tiles, 24.0) + flops / 100.0e6) / (rows ? 1.15 : 1.0);
     return gemm_f32_small_applies(m, n, k, lhs_transposed, rhs_packed, lhs, rhs, us);
 }
 

@@ -294,7 +294,12 @@ bool gemm_f32_small_applies(size_t m, size_t n, size_t k, bool lhs_transposed, b
     const SmallF32Config &c = choose_small(m, n, k, layout, any);
     // Beyond two rounds, and as A·Bᵀ beyond one, the estimates of both sides are a fifth off and the gain is small where there is one:
     // as A·Bᵀ 635×832×2496 took 43.7 µs against 34.7, 468×640×1920 25.6 against 23.0.
-    return c.us(m, n, k, layout, any) < (c.tiles(m, n) > (layout == 1 ? 256 : 512) ? 0.75 : 0.95) * other_us;
+    // The A stored k×m is read in rows of 128 bytes whatever the tile: 208×3584×384 in 784 tiles 17.2 µs against 11.8.
+    // Beyond 1024 tiles of one or two k-tiles each, where a tile is little but its turn on a unit and its stores, the estimate is up to half
+    // too low: as A·Bᵀ 3520×513×13 11.4 µs against 8.5, 2493×1002×27 13.6 against 10.5; 192×3129×29 7.0 against 5.4.
+    const size_t tiles = c.tiles(m, n);
+    const double margin = tiles > 1024 && k <= 64 ? 0.6 : tiles > (layout == 1 ? 256 : 512) ? (layout == 2 && !any ? 0.7 : 0.75) : 0.95;
+    return c.us(m, n, k, layout, any) < margin * other_us;
 }
 
 hipError_t launch_gemm_f32_small(size_t m, size_t n, size_t k, bool lhs_transposed, const float *lhs, bool rhs_packed, const float *rhs,
