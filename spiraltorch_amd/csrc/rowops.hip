@@ -700,7 +700,9 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 // 1024 × 50257 114 -> 104 µs, × 40000 80 -> 67, × 32000 61 -> 52 (5 TB/s), 2048 × 5001 23 -> 19, 4 × 50257 14 -> 9.7 on tensors
 // that come from memory (53 -> 39 and 20.5 -> 14.1 for × 32000 and × 5001 where they stay in the memory-side cache); 2048 × 50257
 // 204 either way.  Rows that start on 16 bytes take the same time: 1024 × 50304 112 -> 100.
-template <int CH, int THREADS, bool BYPASS>
+// What of a launch passes the memory-side cache by.
+enum class Bypass { kNone, kStores, kAll };
+template <int CH, int THREADS, Bypass BYPASS>
 __device__ __forceinline__ void row_softmax_block_body(int cols, const float *in, float *out)
 {
     __shared__ float scratch_f[THREADS / 64];
@@ -711,17 +713,16 @@ __device__ __forceinline__ void row_softmax_block_body(int cols, const float *in
     // (Buffer accesses: an offset register each instead of a 64-bit address, of which the compiler keeps one per piece.)
     const __amdgpu_buffer_rsrc_t rsrc_x = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(x), 0, cols * 4, 0x00020000);
     const __amdgpu_buffer_rsrc_t rsrc_y = __builtin_amdgcn_make_buffer_rsrc(y, 0, cols * 4, 0x00020000);
-    // BYPASS: every value passes once, and is marked so: what a product has just left in the memory-side cache then stays there until it
-    // is read, and the probabilities do not push it out.  (1024 rows of 50257 behind the head's product: 101 -> 76 µs; from
-    // memory 103 -> 95; loads or stores alone 96 and 101.)
-    constexpr int kPolicy = BYPASS ? 2 : 0;  // non-temporal
+    // Marked so, what a product has just left in the memory-side cache stays there until it is read, and the probabilities do not push
+    // it out.
+    constexpr int kNonTemporal = 2, kLoadPolicy = BYPASS == Bypass::kAll ? kNonTemporal : 0, kStorePolicy = BYPASS != Bypass::kNone ? kNonTemporal : 0;
     // A piece that would pass the end of the row is read from the row's last four values instead; the ones before the
     // piece's own start are another thread's and count as -inf here, as NaN entries do (skipped: a weight of zero).
     float v[CH][4];
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
         const f32x4 t = __builtin_bit_cast(
-            f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_x, min((tid + THREADS * i) * 4, cols - 4) * 4, 0, kPolicy));
+            f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_x, min((tid + THREADS * i) * 4, cols - 4) * 4, 0, kLoadPolicy));
         v[i][0] = t[0]; v[i][1] = t[1]; v[i][2] = t[2]; v[i][3] = t[3];
     }
     // The piece offsets of each phase are computed anew from a copy of the thread index the compiler takes for another
@@ -769,7 +770,7 @@ __device__ __forceinline__ void row_softmax_block_body(int cols, const float *in
         const int c = (tid_store + THREADS * i) * 4;
         if (c + 4 <= cols) {
             const f32x4 o = {v[i][0] * inv, v[i][1] * inv, v[i][2] * inv, v[i][3] * inv};
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), rsrc_y, c * 4, 0, kPolicy);
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), rsrc_y, c * 4, 0, kStorePolicy);
         } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
@@ -777,13 +778,13 @@ __device__ __forceinline__ void row_softmax_block_body(int cols, const float *in
         }
     }
 }
-template <int CH, bool BYPASS>
+template <int CH, Bypass BYPASS>
 __global__ __launch_bounds__(512, 4) void row_softmax_block_kernel(int cols, const float *in, float *out)
 {
     row_softmax_block_body<CH, 512, BYPASS>(cols, in, out);
 }
 // Up to 65536 values: more than 25 pieces a thread do not leave room for a second row.
-template <bool BYPASS>
+template <Bypass BYPASS>
 __global__ __launch_bounds__(1024) void row_softmax_block_wide_kernel(int cols, const float *in, float *out)
 {
     row_softmax_block_body<16, 1024, BYPASS>(cols, in, out);
@@ -1237,7 +1238,7 @@ hipError_t launch_merge_heads_f32(size_t batch, size_t seq, size_t heads, size_t
 }
 
 namespace {
-template <bool BYPASS>
+template <Bypass BYPASS>
 void launch_softmax_block(size_t pieces, dim3 grid, hipStream_t stream, int cols, const float *in, float *out)
 {
     if (pieces > 25) {
@@ -1284,10 +1285,17 @@ hipError_t launch_row_softmax_f32(size_t rows, size_t cols, const float *in, flo
         // The row in the registers of a workgroup: 4 to 25 pieces of 16 bytes per thread, 16 in the wide kernel.
         const dim3 rows_grid(static_cast<unsigned>(rows));
         const size_t pieces = (cols + 2047) / 2048;
-        // Values and results that the 256 MB memory-side cache cannot both hold pass it by: behind the product that wrote them, 1024×50257
-        // 222 / 181 µs for the two, 2048×20000 170 / 146; below that they are better left to it (1311×14966 24 / 29 µs, 512×50257 39 / 48).
-        if (rows * cols * sizeof(float) > (128u << 20)) launch_softmax_block<true>(pieces, rows_grid, stream, c, in, out);
-        else launch_softmax_block<false>(pieces, rows_grid, stream, c, in, out);
+        // Values and results that the 256 MiB memory-side cache cannot both hold: the results pass it by; where the values alone take three
+        // quarters of it, they do as well.  µs of the product and the softmax behind it in one run, nothing / stores / both: on the same buffers again
+        // 1329×26295 (133 MiB) 129 / 121 / 128, 1024×34000 153 / 126 / 137, 2048×20000 142 / 121 / 124, 1500×33333 (190) 173 / 147 / 168;
+        // 1024×50257 (196) 235 / 226 / 202, 2048×25088 160 / 126 / 130, 1200×50257 255 / 237 / 221, 4096×16384 (256) 211 / 191 / 160, 2048×50257
+        // 377 / 378 / 329.  The first pass on new buffers: 138 / 140 / 157, 162 / 165 / 179, 139 / 142 / 150, 174 / 183 / 196; 245 / 237 / 240,
+        // 142 / 144 / 160, 271 / 280 / 274, 187 / 186 / 209, 383 / 401 / 378.  Below 128 MiB they are better left to it (1311×14966 24 / 29 µs for
+        // nothing and both, 512×50257 39 / 48).
+        const size_t bytes = rows * cols * sizeof(float);
+        if (bytes > (192u << 20)) launch_softmax_block<Bypass::kAll>(pieces, rows_grid, stream, c, in, out);
+        else if (bytes > (128u << 20)) launch_softmax_block<Bypass::kStores>(pieces, rows_grid, stream, c, in, out);
+        else launch_softmax_block<Bypass::kNone>(pieces, rows_grid, stream, c, in, out);
     } else if (cols > 2048) {
         // A workgroup per row: 1024 threads while the rows are few, 256 once the rows alone fill the chip.
         const bool vec_long = cols % 4 == 0 && ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0;

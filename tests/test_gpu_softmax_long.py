@@ -34,3 +34,18 @@ def test_against_float64(hip, cols, in_place):
     assert (np.abs(got[:3] - want) <= 2.0 ** -17 * want + 2.0 ** -120).all()
     assert got[3].sum() == 1.0 and got[3, cols - 2] == 1.0
     assert got[4].sum() == 1.0 and got[4, cols // 2] == 1.0
+
+
+@pytest.mark.parametrize("rows,cols", [(800, 50257), (8200, 5001), (1024, 65536)])  # beyond 128 MiB, 128 MiB, and 192 MiB of values
+@pytest.mark.parametrize("in_place", [False, True])
+def test_what_passes_the_cache_by_gives_the_same_bits(hip, rows, cols, in_place):
+    few = np.random.default_rng(cols).normal(size=(7, cols)).astype(np.float32) * 3
+    d_few, d_want = hip.DeviceBuffer.from_array(few), hip.DeviceBuffer(few.nbytes)
+    hip.row_softmax_f32_dev(7, cols, d_few, d_want)
+    order = np.arange(rows) % 7
+    d_x = hip.DeviceBuffer.from_array(few[order])
+    d_y = d_x if in_place else hip.DeviceBuffer(rows * cols * 4)
+    hip.row_softmax_f32_dev(rows, cols, d_x, d_y)
+    hip.device_synchronize()
+    want = d_want.to_array(np.uint32, few.size).reshape(7, cols)
+    assert (d_y.to_array(np.uint32, rows * cols).reshape(rows, cols) == want[order]).all()
