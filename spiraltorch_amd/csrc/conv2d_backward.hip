@@ -862,10 +862,7 @@ hipError_t launch_conv2d_grad_weight_f32(const ConvShape &shape, const float *in
                   : gather == Gather::kWindows ? (big ? conv_grad_weight_big_kernel<Gather::kWindows> : conv_grad_weight_kernel<Gather::kWindows>)
                                                : (big ? conv_grad_weight_big_kernel<Gather::kTaps> : conv_grad_weight_kernel<Gather::kTaps>);
     const size_t lds_bytes = big ? kGradWeightStages<2, 3> : kGradWeightStages<1, 1>;
-    if (big) {  // (beyond what a launch may take unasked)
-        rc = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes));
-        if (rc != hipSuccess) return rc;
-    }
+    static_assert(kGradWeightStages<2, 3> <= 64 * 1024, "what a launch may take unasked");
     hipLaunchKernelGGL(kernel, grid, dim3(256), lds_bytes, stream, args);
     rc = hipGetLastError();
     if (rc != hipSuccess) return rc;
