@@ -196,7 +196,7 @@ def wl_conv2d(hip, inputs, timer):
 def wl_conv2d_bf16(hip, inputs, timer):
     """Config 2's layer on bf16-rounded operands (bf16 NCHW images and OIHW weights, f32 accumulation, f32 output): the
     implicit GEMM on the bf16 matrix cores, priced against the bf16 peak.  The timed step includes the copy of the images
-    into the padded channels-last layout the kernel works on and the re-layout of the weights."""
+    and weights into the blocks of eight channels the kernel works on."""
     batch, c_in, h, w, c_out = 32, 64, 56, 56, 128
     x = inputs.to_bf16(inputs.normal(inputs.seed_for(2, 0), batch * c_in * h * w))
     wt = inputs.to_bf16(inputs.normal(inputs.seed_for(2, 1), c_out * c_in * 9, 0.0, math.sqrt(2.0 / (c_in * 9))))

@@ -1031,7 +1031,7 @@ int st_hip_conv2d_bias_act_bf16_dev(size_t batch, size_t c_in, size_t h, size_t 
     if (misaligned(out_f32, 16) || misaligned(out_bf16, 8))
         return fail(ST_HIP_ERR_UNSUPPORTED, "bf16 conv2d needs a 16-byte aligned f32 output and an 8-byte aligned bf16 output");
     if (!conv2d_bf16_supported(plan.shape))
-        return fail(ST_HIP_ERR_UNSUPPORTED, "bf16 conv2d: the padded channels-last copy of the input or the re-laid weights exceed 2 GiB");
+        return fail(ST_HIP_ERR_UNSUPPORTED, "bf16 conv2d: the padded images or the weights, counted with the channels in blocks of 64, exceed 2 GiB");
     return launch_status(launch_conv2d_bf16(plan.shape, activation, input, weight, bias, out_f32, out_bf16, as_stream(stream)),
                          "conv2d bf16 launch");
 }
