@@ -2550,11 +2550,15 @@ hipError_t launch_gemm_bf16(size_t m, size_t n, size_t k, const uint16_t *lhs, c
     // Few rows or few columns: small tiles with k split inside the workgroup.  (A row-major B of up to 64 rows and a long k
     // stays with the skinny kernel, which reads it in longer pieces: 64×768×3072 8.6 µs against 9.9.)
     // Rows of B that start at any 2-byte boundary are packed first, a pass of about 1.9 µs for a million values: up to 64 rows, the general
-    // kernel, which reads B once as it is, is ahead beyond ten million (seven up to 16 rows), and in a single k-tile.  Packed / general:
-    // 1×6853×6144 84.7 / 46.6 µs, 8×4001×2048 23.9 / 22.3, 33×6853×2048 41.7 / 38.5, 1×1953×64 7.9 / 6.5; 3×4001×1024 15.7 / 21.2,
-    // 33×4001×2048 24.2 / 27.5, 8×1001×256 7.7 / 12.4.
+    // kernel, which reads B once as it is, is ahead beyond ten million (seven up to 16 rows), beyond some columns, the more the more
+    // rows there are, and in a single k-tile of few rows or more columns still.  Packed / general: 1×6853×6144 84.7 / 46.6 µs,
+    // 8×4001×2048 23.9 / 22.3, 33×6853×2048 41.7 / 38.5; 1×39723×128 19.2 / 7.8, 58×15819×128 11.8 / 16.2,
+    // 5×6199×256 8.9 / 12.6; 1×1953×64 7.9 / 6.5, 22×24591×64 11.2 / 8.5, 53×15221×64 9.8 / 13.7; 3×4001×1024 15.7 / 21.2, 33×4001×2048
+    // 24.2 / 27.5, 8×1001×256 7.7 / 12.4.  (Of 2397 products packed, k from 64 to 512, 7 are more than 3 % slower for it.)
     const size_t packing_most = m > 64 ? SIZE_MAX : m > 16 ? 10'000'000 : 7'000'000;
-    const bool as_it_is = rhs_packed || n % 8 == 0, packing_pays = n * k <= packing_most && (k > 64 || (m > 16 && m * n <= 1'000'000));
+    const size_t columns_most = m > 64 ? SIZE_MAX : (6500 + 200 * m) * (k >= 512 ? 5 : 4) / 4;
+    const bool as_it_is = rhs_packed || n % 8 == 0;
+    const bool packing_pays = n * k <= packing_most && n <= columns_most && (k > 64 || (m > 16 && n <= 450 * m));
     if (aligned16(lhs) && aligned16(rhs) && fits_buffer && small_tiles_apply(m, n, k) && !(skinny && k > 1024) && (as_it_is || packing_pays)) {
         if (as_it_is) return launch_gemm_bf16_small(m, n, k, lhs, rhs, rhs_packed, out_f32, out_bf16, epilogue, stream);
         void *workspace = nullptr;

@@ -10,6 +10,7 @@ pytestmark = pytest.mark.gpu
     (117, 512, 512), (117, 1536, 512), (65, 504, 576),  # a stage a wavefront; nine k-tiles over eight wavefronts
     (40, 500, 512), (40, 257, 1024),                  # rows of B off 16-byte boundaries (packed first); an odd width
     (9, 3500, 2048), (9, 3412, 2048), (33, 4884, 2048),  # row-major: just beyond and within what is packed, of few and more rows
+    (3, 7099, 128), (17, 7649, 64), (40, 18125, 512),  # the most columns that are packed
     (117, 512, 2048), (64, 768, 3136),                # several stages a wavefront, an uneven last share
     (1024, 512, 2048), (600, 1000, 448), (2048, 300, 640),  # 64×64 tiles; groups of eight row tiles, a ragged last one
     (545, 72, 256),                                   # a grid that eight does not divide, a group of one or two row tiles

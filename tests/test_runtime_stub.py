@@ -75,3 +75,15 @@ for batch, heads, seq, dim, causal in itertools.product((1, 2, 3, 8), (1, 4, 7, 
 print(calls == launches.value)
 """)
     assert out == ["True"]
+
+
+@pytest.mark.parametrize("m,k,columns", [(3, 128, 7099), (16, 192, 9699), (17, 64, 7649), (40, 512, 18125), (16, 960, 7291), (40, 960, 10415)])
+def test_how_many_columns_are_packed(stub, m, k, columns):
+    """Few rows against a row-major bf16 B at odd boundaries: packed (two launches) up to so many columns, the general kernel beyond."""
+    out = run(stub, f"""
+for n in ({columns}, {columns} + 2):
+    before = launches.value
+    hip.gemm_bf16_bias_act_dev({m}, n, {k}, 0, 1 << 20, 2 << 20, None, None, 3 << 20, None)
+    print(launches.value - before)
+""")
+    assert out[0] == "2" and out[1] == "1"
