@@ -1322,7 +1322,7 @@ hipError_t launch_gelu_f32(size_t count, const float *in, float *out, hipStream_
 }
 
 // Few enough words for the host to wait for; a tensor from memory wants more bytes in flight than 512 workgroups ask for, one load a lane
-// (512 / 2048 of them, µs: 256 million values 322 / 187, 70 million 72 / 66).
+// (512 / 2048 of them, µs: 256 million values 322 / 187).
 size_t nonfinite_probe_groups(size_t count) { return std::min<size_t>(std::max<size_t>((count + 2047) / 2048, 1), count > (size_t(1) << 26) ? 2048 : 512); }
 
 hipError_t launch_nonfinite_probe_f32(size_t count, const float *data, unsigned long long *slots, hipStream_t stream)
