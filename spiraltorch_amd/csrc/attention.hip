@@ -1817,7 +1817,8 @@ hipError_t launch_split_rows(AttnArgs args, hipStream_t stream)
 
 // How many runs of keys a call of the split kernel's arithmetic is cut into when the wavefronts of 32-row workgroups share them; 0
 // where the wider tiles are the better ones.  A launch of them is one round of a workgroup a compute unit: about 5.5 µs and 1.9 for
-// 128 keys (64 values a head), and 4.5 for the second launch that puts runs together.  Before / after, 64 values: 1 × 250 17.6 / 10.0 µs
+// 128 keys (64 values a head; smaller heads take less, and of 1450 drawn calls of 16 to 56 values that it may cut the slowest takes 0.93
+// of the time before), and 4.5 for the second launch that puts runs together.  Before / after, 64 values: 1 × 250 17.6 / 10.0 µs
 // (causal 27.7 / 9.8), 1 × 1000 15.4 / 12.6 (biased 16.8 / 13.3), 4 × 500 15.4 / 12.8, 8 × 1000 27.4 / 24.8, 32 × 250 18.0 / 10.8; the error
 // against float64 3.2e-7 / 2.4e-7.  Beyond a round or some length the 128-row tiles, which read K and V a quarter as often and cut
 // them once for four wavefronts, are level or ahead: 32 × 500 26.2 / 27.6, 4 × 1000 in one run each 20.3 / 22.7, 1 × 2048 20.8 / 34.8;
