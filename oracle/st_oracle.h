@@ -1,7 +1,7 @@
 /*
  * st_oracle.h — CPU restatement of SpiralTorch's dense CPU path (TEST INFRASTRUCTURE ONLY).
  *
- * This library is the checker for the HIP backend: it restates, loop for loop, what the reference's
+ * The HIP backend is tested against this library: it restates, loop for loop, what the reference's
  * Rust CPU kernels compute (sequential-k f32 sums with separately rounded multiply and add, the
  * normalised online-softmax attention recurrence, im2col convolution, layer-norm).  It must never be
  * linked into, imported by, or called from the product path; only tests, the smoke check and the
