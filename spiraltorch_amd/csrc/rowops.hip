@@ -397,54 +397,27 @@ __device__ __forceinline__ float wave_max(float v)
     return v;
 }
 
-// One wavefront per row.  cpu_row_softmax_hardmax, crates/st-tensor/src/pure.rs:11930-11980: the maximum is
-// taken over the non-NaN entries (first occurrence wins), base = max if finite else 0, weights exp(v - base)
-// (0 for NaN), divided by their sum when that is finite and above f32 epsilon; otherwise the row becomes the
-// one-hot of the maximum.  A row of only NaNs gives zeros.
-__global__ __launch_bounds__(256) void row_softmax_kernel(int rows, int cols, const float *in, float *out)
+// Four adjacent values of a row at any 4-byte alignment; past `end` they read as NaN, which every phase skips.
+__device__ __forceinline__ void load_quad_or_nan(const float *x, int c, int end, float (&v)[4])
 {
-    const int lane = threadIdx.x & 63;
-    const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (row >= rows) return;
-    const float *x = in + static_cast<size_t>(row) * cols;
-    float *y = out + static_cast<size_t>(row) * cols;
-    float best = -INFINITY;
-    int best_index = 0x7fffffff;
-    for (int c = lane; c < cols; c += 64) {
-        const float v = x[c];
-        if (v != v) continue;
-        if (best_index == 0x7fffffff || v > best) {
-            best = v;
-            best_index = c;
-        }
-    }
-    // first occurrence of the largest value across the wavefront
-    const float row_max = wave_max(best_index == 0x7fffffff ? -INFINITY : best);
-    int candidate = (best_index != 0x7fffffff && best == row_max) ? best_index : 0x7fffffff;
+    if (c + 4 <= end) {
+        const f32x4_a4 t = *reinterpret_cast<const f32x4_a4 *>(x + c);
+        v[0] = t[0]; v[1] = t[1]; v[2] = t[2]; v[3] = t[3];
+    } else {
 #pragma unroll
-    for (int offset = 32; offset > 0; offset >>= 1) candidate = min(candidate, __shfl_xor(candidate, offset));
-    const bool found = candidate != 0x7fffffff;
-    const float base = (found && isfinite(row_max)) ? row_max : 0.0f;
-    float denom = 0.0f;
-    for (int c = lane; c < cols; c += 64) {
-        const float v = x[c];
-        denom += (!found || v != v) ? 0.0f : expf(v - base);
-    }
-    denom = wave_sum(denom);
-    const bool normal = isfinite(denom) && denom > 1.1920929e-7f;
-    const float inv = normal ? 1.0f / denom : 0.0f;
-    for (int c = lane; c < cols; c += 64) {
-        const float v = x[c];
-        const float weight = (!found || v != v) ? 0.0f : expf(v - base);
-        float value = weight * inv;
-        if (found && !normal) value = c == candidate ? 1.0f : 0.0f;
-        y[c] = value;
+        for (int e = 0; e < 4; ++e) v[e] = (c + e < end) ? x[c + e] : __builtin_nanf("");
     }
 }
 
-// Same for rows of at most 2048 values with 16-byte aligned rows: one 128-bit read per lane and chunk, the row stays
-// in registers for all three phases.
-template <int CHUNKS>
+// One wavefront per row of at most 2048 values, which stays in registers for all three phases, 16 bytes a lane and piece.
+// cpu_row_softmax_hardmax, crates/st-tensor/src/pure.rs:11930-11980: the maximum is taken over the non-NaN entries (first
+// occurrence wins), base = max if finite else 0, weights exp(v - base) (0 for NaN), divided by their sum when that is finite
+// and above f32 epsilon; otherwise the row becomes the one-hot of the maximum.  A row of only NaNs gives zeros.
+// ANY: rows of any length at any 4-byte boundary (global memory takes 16-byte accesses there), the last piece of a row value by
+// value; W = 1, a value a lane, for rows that pieces of four would leave most lanes without.  Bound by one trip to memory and back:
+// a row read three times, value by value, took 18.9 µs for 697×2027 (here 6.1), 13.6 for 4×1635 (5.0), 11.4 for 2048×1023 (5.4), 54.6
+// for 20000×901 (25.7), 5.7 for 1478×414 (4.0), 27.6 for 100000×63 (20.6; 41 for 100000×10 in pieces of four, 18.0 by values).
+template <int CHUNKS, bool ANY, int W = 4>
 __global__ __launch_bounds__(256) void row_softmax_vec_kernel(int rows, int cols, const float *in, float *out)
 {
     const int lane = threadIdx.x & 63;
@@ -452,20 +425,24 @@ __global__ __launch_bounds__(256) void row_softmax_vec_kernel(int rows, int cols
     if (row >= rows) return;
     const float *x = in + static_cast<size_t>(row) * cols;
     float *y = out + static_cast<size_t>(row) * cols;
-    float v[CHUNKS][4];
+    float v[CHUNKS][W];
     float best = -INFINITY;
     int best_index = 0x7fffffff;
 #pragma unroll
     for (int i = 0; i < CHUNKS; ++i) {
-        const int c = (lane + 64 * i) * 4;
-        if (c < cols) {
+        const int c = (lane + 64 * i) * W;
+        if constexpr (W == 1) {
+            v[i][0] = c < cols ? x[c] : __builtin_nanf("");
+        } else if constexpr (ANY) {
+            load_quad_or_nan(x, c, cols, v[i]);
+        } else if (c < cols) {
             const float4 t = *reinterpret_cast<const float4 *>(x + c);
             v[i][0] = t.x; v[i][1] = t.y; v[i][2] = t.z; v[i][3] = t.w;
         } else {
             v[i][0] = v[i][1] = v[i][2] = v[i][3] = __builtin_nanf("");  // skipped like NaN entries, never stored
         }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
+        for (int e = 0; e < W; ++e) {
             const float value = v[i][e];
             if (value != value) continue;
             if (best_index == 0x7fffffff || value > best) {  // columns visited in ascending order per lane
@@ -484,9 +461,10 @@ __global__ __launch_bounds__(256) void row_softmax_vec_kernel(int rows, int cols
 #pragma unroll
     for (int i = 0; i < CHUNKS; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
+        for (int e = 0; e < W; ++e) {
             const float value = v[i][e];
-            const float weight = (!found || value != value) ? 0.0f : __expf(value - base);  // exp2 of a scaled argument
+            // (__expf: exp2 of a scaled argument)
+            const float weight = (!found || value != value) ? 0.0f : ANY ? expf(value - base) : __expf(value - base);
             v[i][e] = weight;
             denom += weight;
         }
@@ -495,15 +473,25 @@ __global__ __launch_bounds__(256) void row_softmax_vec_kernel(int rows, int cols
     const float inv = normal ? 1.0f / denom : 0.0f;
 #pragma unroll
     for (int i = 0; i < CHUNKS; ++i) {
-        const int c = (lane + 64 * i) * 4;
+        const int c = (lane + 64 * i) * W;
         if (c >= cols) continue;
-        float o[4];
+        float o[W];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
+        for (int e = 0; e < W; ++e) {
             o[e] = v[i][e] * inv;
             if (found && !normal) o[e] = (c + e == candidate) ? 1.0f : 0.0f;
         }
-        *reinterpret_cast<float4 *>(y + c) = make_float4(o[0], o[1], o[2], o[3]);
+        if constexpr (W == 1) {
+            y[c] = o[0];
+        } else if constexpr (!ANY) {
+            *reinterpret_cast<float4 *>(y + c) = make_float4(o[0], o[1], o[2], o[3]);
+        } else if (c + 4 <= cols) {
+            *reinterpret_cast<f32x4_a4 *>(y + c) = f32x4_a4{o[0], o[1], o[2], o[3]};
+        } else {
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+                if (c + e < cols) y[c + e] = o[e];
+        }
     }
 }
 
@@ -583,18 +571,6 @@ struct SoftmaxSegment {
     int index;    // its first column, 0x7fffffff when the segment has none
     float sum;    // sum of exp(v - base), base = best if finite else 0
 };
-
-// Four adjacent values of a row at any 4-byte alignment; past `end` they read as NaN, which every phase skips.
-__device__ __forceinline__ void load_quad_or_nan(const float *x, int c, int end, float (&v)[4])
-{
-    if (c + 4 <= end) {
-        const f32x4_a4 t = *reinterpret_cast<const f32x4_a4 *>(x + c);
-        v[0] = t[0]; v[1] = t[1]; v[2] = t[2]; v[3] = t[3];
-    } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = (c + e < end) ? x[c + e] : __builtin_nanf("");
-    }
-}
 
 __global__ __launch_bounds__(256) void row_softmax_split_partial_kernel(int cols, int segment, const float *in, SoftmaxSegment *parts)
 {
@@ -697,7 +673,8 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 // (128 registers a wavefront, four wavefronts per SIMD); with 1024 threads and the row padded to 65536 values one row
 // filled the unit.  The index a row without a usable sum needs is found by reading the row again: no row of ordinary
 // values pays for it.
-// 1024 × 50257 114 -> 104 µs, × 40000 80 -> 67, × 32000 61 -> 52 (5 TB/s), 2048 × 5001 23 -> 19, 4 × 50257 14 -> 9.7 on tensors
+// Against three sweeps by workgroups of 1024 or 256 threads, rows of 2049 to 4096 values: 1519 × 3008 14.5 -> 7.3 µs, 2048 × 4095 19.8 ->
+// 11.6, 8000 × 2500 34.1 -> 24.5, 4 × 3007 4.3 -> 3.8.  1024 × 50257 114 -> 104 µs, × 40000 80 -> 67, × 32000 61 -> 52 (5 TB/s), 2048 × 5001 23 -> 19, 4 × 50257 14 -> 9.7 on tensors
 // that come from memory (53 -> 39 and 20.5 -> 14.1 for × 32000 and × 5001 where they stay in the memory-side cache); 2048 × 50257
 // 204 either way.  Rows that start on 16 bytes take the same time: 1024 × 50304 112 -> 100.
 // What of a launch passes the memory-side cache by.
@@ -1240,7 +1217,8 @@ void launch_softmax_block(size_t pieces, dim3 grid, hipStream_t stream, int cols
         hipLaunchKernelGGL(row_softmax_block_wide_kernel<BYPASS>, grid, dim3(1024), 0, stream, cols, in, out);
         return;
     }
-    auto kernel = pieces <= 4    ? row_softmax_block_kernel<4, BYPASS>
+    auto kernel = pieces <= 2    ? row_softmax_block_kernel<2, BYPASS>
+                  : pieces <= 4  ? row_softmax_block_kernel<4, BYPASS>
                   : pieces <= 8  ? row_softmax_block_kernel<8, BYPASS>
                   : pieces <= 16 ? row_softmax_block_kernel<16, BYPASS>
                   : pieces <= 20 ? row_softmax_block_kernel<20, BYPASS>
@@ -1254,14 +1232,15 @@ hipError_t launch_row_softmax_f32(size_t rows, size_t cols, const float *in, flo
     if (rows == 0 || cols == 0) return hipSuccess;
     const dim3 grid(static_cast<unsigned>((rows + 3) / 4)), block(256);
     const int r = static_cast<int>(rows), c = static_cast<int>(cols);
-    const bool vec = cols % 4 == 0 && cols <= 2048 && ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0;
-    if (vec && cols <= 512)
-        hipLaunchKernelGGL(row_softmax_vec_kernel<2>, grid, block, 0, stream, r, c, in, out);
-    else if (vec && cols <= 1024)
-        hipLaunchKernelGGL(row_softmax_vec_kernel<4>, grid, block, 0, stream, r, c, in, out);
-    else if (vec)
-        hipLaunchKernelGGL(row_softmax_vec_kernel<8>, grid, block, 0, stream, r, c, in, out);
-    else if (cols > 65536 && rows <= 128) {
+    if (cols <= 2048) {
+        const bool vec = cols % 4 == 0 && aligned16(in) && aligned16(out);
+        auto kernel = !vec && cols <= 64    ? row_softmax_vec_kernel<1, true, 1>
+                      : !vec && cols <= 128 ? row_softmax_vec_kernel<2, true, 1>
+                      : cols <= 512  ? (vec ? row_softmax_vec_kernel<2, false> : row_softmax_vec_kernel<2, true>)
+                      : cols <= 1024 ? (vec ? row_softmax_vec_kernel<4, false> : row_softmax_vec_kernel<4, true>)
+                                     : (vec ? row_softmax_vec_kernel<8, false> : row_softmax_vec_kernel<8, true>);
+        hipLaunchKernelGGL(kernel, grid, block, 0, stream, r, c, in, out);
+    } else if (cols > 65536 && rows <= 128) {
         // Few rows too long for a workgroup's registers: segments of at least 8192 values, up to about 1024 workgroups,
         // at most 64 segments a row (4 × 1000000: 34 µs; 16 × 128256: 20 µs; 100 × 100000: 35 → 30 µs.  Up to 65536
         // values the register kernel below is as fast or faster from a handful of rows on: 128 × 50257 19 against 23 µs).
@@ -1276,8 +1255,8 @@ hipError_t launch_row_softmax_f32(size_t rows, size_t cols, const float *in, flo
         const int seg = static_cast<int>(segment);
         hipLaunchKernelGGL(row_softmax_split_partial_kernel, split_grid, dim3(256), 0, stream, c, seg, in, parts);
         hipLaunchKernelGGL(row_softmax_split_write_kernel, split_grid, dim3(256), 0, stream, c, seg, in, parts, out);
-    } else if (cols > 4096 && cols <= 65536) {
-        // The row in the registers of a workgroup: 4 to 25 pieces of 16 bytes per thread, 16 in the wide kernel.
+    } else if (cols <= 65536) {
+        // The row in the registers of a workgroup: 2 to 25 pieces of 16 bytes per thread, 16 in the wide kernel.
         const dim3 rows_grid(static_cast<unsigned>(rows));
         const size_t pieces = (cols + 2047) / 2048;
         // Values and results that the 256 MiB memory-side cache cannot both hold: the results pass it by; where the values alone take three
@@ -1291,7 +1270,7 @@ hipError_t launch_row_softmax_f32(size_t rows, size_t cols, const float *in, flo
         if (bytes > (192u << 20)) launch_softmax_block<Bypass::kAll>(pieces, rows_grid, stream, c, in, out);
         else if (bytes > (128u << 20)) launch_softmax_block<Bypass::kStores>(pieces, rows_grid, stream, c, in, out);
         else launch_softmax_block<Bypass::kNone>(pieces, rows_grid, stream, c, in, out);
-    } else if (cols > 2048) {
+    } else {
         // A workgroup per row: 1024 threads while the rows are few, 256 once the rows alone fill the chip.
         const bool vec_long = cols % 4 == 0 && ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0;
         const dim3 rows_grid(static_cast<unsigned>(rows));
@@ -1302,8 +1281,7 @@ hipError_t launch_row_softmax_f32(size_t rows, size_t cols, const float *in, flo
             if (vec_long) hipLaunchKernelGGL((row_softmax_long_kernel<256, true>), rows_grid, dim3(256), 0, stream, c, in, out);
             else hipLaunchKernelGGL((row_softmax_long_kernel<256, false>), rows_grid, dim3(256), 0, stream, c, in, out);
         }
-    } else
-        hipLaunchKernelGGL(row_softmax_kernel, grid, block, 0, stream, r, c, in, out);
+    }
     return hipGetLastError();
 }
 
