@@ -143,6 +143,14 @@ def test_elementwise_kernels_on_unaligned_pointers(hip, oracle):
     assert (d_x.to_array(np.float32, n + 1)[1:] == oracle.add_row_f32(rows, cols, x[1:], bias[1:])).all()
 
 
+# one launch: a group of lanes with one row and with none, the 64 and 256 groups' remainders, strips of 16 columns cut short, more than one strip
+# an XCD; and the first sizes of two launches
+@pytest.mark.parametrize("rows,cols", [(1, 15), (63, 16), (64, 17), (255, 130), (256, 33), (257, 4), (1023, 48), (1025, 5), (2048, 35), (2049, 35),
+                                       (2049, 36), (4095, 52), (4096, 52), (40, 16384), (40, 16388), (2048, 4096), (2049, 4096)])
+def test_sum_axis0_of_few_rows(hip, oracle, rows, cols):
+    test_sum_axis0(hip, oracle, rows, cols)
+
+
 @pytest.mark.parametrize("rows,cols", [(1, 1), (3, 2), (64, 256), (65, 257), (1000, 19), (16384, 512), (100000, 8), (37, 260), (131, 1028), (5, 4),
                                        # rows that do not start on 16-byte boundaries: 16-byte loads all the same
                                        (300, 1001), (4097, 67), (70, 50257), (129, 66)])
@@ -497,3 +505,32 @@ def test_scratch_of_exited_threads_is_reused_not_leaked(hip, oracle):
         assert_close(got, want, F32_REL, 1e-3, "column sums from concurrent threads")
     hip.release_scratch(None)
     assert hip.scratch_buffer_count() == before
+
+
+def test_column_sums_from_threads_sharing_the_null_stream(hip):
+    """Column sums in two launches keep partial sums in scratch memory: each thread's stay right while its scratch grows."""
+    import threading
+    failures = []
+
+    def work(index):
+        try:
+            rng = np.random.default_rng(index)
+            for round_ in range(6):
+                rows, cols = 4200 + 700 * round_, 64 * (index + 1)
+                x = rng.normal(size=rows * cols).astype(np.float32)
+                d_x, d_s = hip.DeviceBuffer.from_array(x), hip.DeviceBuffer(cols * 4)
+                hip.sum_axis0_f32_dev(rows, cols, d_x, 1.0, d_s)
+                hip.device_synchronize()
+                want = x.astype(np.float64).reshape(rows, cols).sum(axis=0)
+                # f32 sums in any order: at most rows roundings of half an ulp of the sum of magnitudes each
+                if np.abs(d_s.to_array(np.float32, cols) - want).max() > 2.0 ** -24 * rows * np.abs(x).reshape(rows, cols).sum(axis=0).max():
+                    failures.append((index, round_))
+        except Exception as err:  # surfaced below
+            failures.append(err)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failures, failures
