@@ -434,3 +434,19 @@ def test_grad_weight_keeps_infinities_and_nan_to_their_terms(hip, case):
     assert np.array_equal(np.isfinite(got), finite)
     assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
     assert np.all(np.abs(got[finite] - want[finite]) <= 2.0 ** -19 * magnitudes[finite])
+
+
+# one launch: fewer images than wavefronts (planes cut in parts, some of them empty), as many, more; and the first size of two launches
+@pytest.mark.parametrize("batch,c_out,oh,ow", [(1, 3, 1, 1), (1, 5, 7, 9), (3, 2, 5, 13), (5, 17, 33, 31), (15, 4, 9, 9), (16, 3, 56, 56), (17, 3, 31, 33),
+                                               (33, 2, 1, 3), (1, 2, 256, 512), (2, 2, 257, 256), (32, 1, 64, 64), (32, 1, 64, 65)])
+def test_grad_bias_of_a_channel(hip, batch, c_out, oh, ow):
+    g = np.random.default_rng(batch * oh + ow).normal(size=batch * c_out * oh * ow).astype(np.float32)
+    d_g, d_gb = hip.DeviceBuffer.from_array(g), hip.DeviceBuffer.from_array(np.full(c_out + 8, 7.5, np.float32))
+    hip.conv2d_grad_bias_f32_dev(batch, 1, oh, ow, c_out, (1, 1), (1, 1), (0, 0), (1, 1), d_g, 0.5, d_gb)
+    hip.device_synchronize()
+    got = d_gb.to_array(np.float32, c_out + 8)
+    assert (got[c_out:] == 7.5).all()
+    terms = g.astype(np.float64).reshape(batch, c_out, oh * ow)
+    # any order of f32 additions: at most one rounding a term of half an ulp of the sum of magnitudes
+    bound = 2.0 ** -24 * batch * oh * ow * np.abs(terms).sum(axis=(0, 2)) + 1e-30
+    assert (np.abs(got[:c_out] - 0.5 * terms.sum(axis=(0, 2))) <= bound).all()
