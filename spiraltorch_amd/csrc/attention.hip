@@ -640,7 +640,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DPAD <= 64 
 }
 
 // -------------------------------------------------------------------------------------------------
-// Head sizes up to 64, with or without biases: both products on the bf16 matrix cores, every f32 value (Q, K, V and the
+// Head sizes up to 128, with or without biases: both products on the bf16 matrix cores, every f32 value (Q, K, V and the
 // probabilities) as the exact sum of three bf16 values, x = hi + mid + lo, and a product as the six piece products
 //     lo·hi, mid·hi, mid·mid, hi·mid, hi·lo, hi·hi
 // accumulated in f32; what is left out is at most 2^-24 of the product, 2^-27.4 in the rms.  (gemm_f32_split.hip does the same for matrix
@@ -658,6 +658,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DPAD <= 64 
 // wavefronts per SIMD take 5.2 µs for theirs.  Measured, f32 matrix cores -> here: 128 × 2048 × 64 causal 591 -> 360 µs,
 // non-causal 1070 -> 643, 128 × 1024 causal 163 -> 102; biased 1 × 1000 26 -> 16 µs, 16 × 1024 60 -> 51, biases on rows of
 // 777 (no 16-byte alignment: the general kernel) 162 -> 16.  Errors against float64 are 0.7 to 0.85 of the f32 kernel's.
+//
+// Heads above 64 are padded to 96 or 128 values and staged 32 keys at a time by four wavefronts, two workgroups a unit: the pieces of Q and
+// the outputs alone are 120 or 160 registers.  f32 matrix cores -> here, heads of 80 / 128: 128 × 1024 594 -> 263 / 607 -> 369 µs, causal
+// 353 -> 172 / 361 -> 274, 32 × 500 73 -> 37 / 79 -> 50, 16 × 500 causal 32 -> 24 / 34 -> 32, biased 16 × 500 127 -> 26 / 130 -> 38.
+// Errors against float64 0.7 to 0.85 of the f32 kernels'.
 //
 // V and the probabilities are scaled by 2^24 before they are split, and the output by 2^-48: the last bit of either is then a
 // normal bf16 number, and the pieces are exact however small a value is (a probability of 2^-124 may meet the only non-zero
@@ -812,14 +817,14 @@ __device__ void redo_rows(const AttnArgs &p, int ctx, int wq0, int lane, int spl
 }
 
 template <int DPAD, bool CAUSAL, bool BIAS, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void attention_f32_split_kernel(AttnArgs p)
+__global__ __launch_bounds__(64 * WAVES, DPAD > 64 ? 2 : 1) void attention_f32_split_kernel(AttnArgs p)
 {
-    constexpr int BKV = 64, THREADS = 64 * WAVES, BQ = 32 * WAVES;
+    constexpr int KT = DPAD > 64 ? 1 : 2, BKV = 32 * KT, THREADS = 64 * WAVES, BQ = 32 * WAVES;
     constexpr int QSTEPS = DPAD / 16, DT = DPAD / 32;
     constexpr int CHAINS = DT == 1 ? 2 : 1;  // a single chain of dependent matrix instructions would wait for each
-    constexpr int K_BYTES = 2 * QSTEPS * 3072, V_BYTES = DT * 4 * 3072, STAGE = K_BYTES + V_BYTES;
-    constexpr int ITEMS = 64 * DPAD / 8;  // groups of eight values of K (and of V) in a stage
-    constexpr int PER = ITEMS > THREADS ? ITEMS / THREADS : 1;
+    constexpr int K_BYTES = KT * QSTEPS * 3072, V_BYTES = DT * 2 * KT * 3072, STAGE = K_BYTES + V_BYTES;
+    constexpr int ITEMS = BKV * DPAD / 8;  // groups of eight values of K (and of V) in a stage
+    constexpr int PER = (ITEMS + THREADS - 1) / THREADS;
     // Eight wavefronts (one workgroup per compute unit): two stages.  Four: one, so that two workgroups fit a compute unit.
     constexpr int BUFFERS = WAVES == 8 ? 2 : 1;
     constexpr float kWild = 0x1p40f, kScale = 0x1p24f, kUnscale = 0x1p-48f;
@@ -831,7 +836,8 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_split_kernel(AttnArg
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 31, lh = lane >> 5;
     const int S = p.S, D = p.D;
-    const bool stages_items = ITEMS >= THREADS || tid < ITEMS;  // (head size 32 leaves half of eight wavefronts without any)
+    // (Head size 32 leaves half of eight wavefronts without any, 96 half of four without a second one.)
+    auto stages_item = [&](int r) { return ITEMS % THREADS == 0 || tid + THREADS * r < ITEMS; };
 
     const FastItem item = decode_fast_block<CAUSAL>(p.contexts, p.q_tiles, p.swizzle, p.key_splits, p.keys_per_split,
                                                     p.causal_items, static_cast<int>(blockIdx.x));
@@ -896,37 +902,46 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_split_kernel(AttnArg
     const int stages = (key_end - key_first + BKV - 1) / BKV;
 
     float rk[PER][8], rv[PER][8];
+    // The staging's addresses are computed anew for every stage of a wide head, from copies of the thread's index and the row length
+    // that the compiler takes for other values: it would keep them all in registers, and spill others.
     auto load_global = [&](int key0) {
-        if (!stages_items) return;
+        int tid_now = tid, d_now = D;
+        if constexpr (DPAD > 64) {
+            asm volatile("" : "+v"(tid_now));
+            asm volatile("" : "+s"(d_now));
+        }
 #pragma unroll
         for (int r = 0; r < PER; ++r) {
-            const int f = tid + THREADS * r;
-            load8(rsrc_k, key0 + (f & 63), (f >> 6) * 8, rk[r]);
+            if (!stages_item(r)) continue;
+            const int f = tid_now + THREADS * r;
+            load8(rsrc_k, key0 + f % BKV, f / BKV * 8, rk[r]);
             const int d = f % DPAD, group = f / DPAD;  // group: 16-key step group / 2, accumulator half group % 2
             const int key = key0 + (group >> 1) * 16 + (group & 1) * 4;
-            const unsigned at = d < D ? (static_cast<unsigned>(key) * D + d) * 4u : kOutside;
+            const unsigned at = d < D ? (static_cast<unsigned>(key) * d_now + d) * 4u : kOutside;
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-                rv[r][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc_v, at + ((e >> 2) * 8 + (e & 3)) * (D * 4u), 0, 0));
+                rv[r][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc_v, at + ((e >> 2) * 8 + (e & 3)) * (d_now * 4u), 0, 0));
         }
     };
     auto store_lds = [&](int stage) {
-        if (!stages_items) return;
         unsigned char *ks = split_lds + stage * STAGE, *vs = ks + K_BYTES;
+        int tid_now = tid;
+        if constexpr (DPAD > 64) asm volatile("" : "+v"(tid_now));
 #pragma unroll
         for (int r = 0; r < PER; ++r) {
-            const int f = tid + THREADS * r;
+            if (!stages_item(r)) continue;
+            const int f = tid_now + THREADS * r;
             u32x4_t piece[3];
             split8(rk[r], piece);
             top_qk = largest8(rk[r], top_qk);
-            const int key = f & 63, chunk = f >> 6;
+            const int key = f % BKV, chunk = f / BKV;
             unsigned char *dst = ks + ((key >> 5) * QSTEPS + (chunk >> 1)) * 3072 + ((chunk & 1) * 32 + (key & 31)) * 16;
 #pragma unroll
             for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x4_t *>(dst + i * 1024) = piece[i];
             split8(rv[r], piece, kScale);
             top_v = largest8(rv[r], top_v);
             const int d = f % DPAD, group = f / DPAD;
-            dst = vs + ((d >> 5) * 4 + (group >> 1)) * 3072 + ((group & 1) * 32 + (d & 31)) * 16;
+            dst = vs + ((d >> 5) * (2 * KT) + (group >> 1)) * 3072 + ((group & 1) * 32 + (d & 31)) * 16;
 #pragma unroll
             for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x4_t *>(dst + i * 1024) = piece[i];
         }
@@ -1041,19 +1056,24 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_split_kernel(AttnArg
                 bf16x8 pf[3];
 #pragma unroll
                 for (int i = 0; i < 3; ++i) pf[i] = __builtin_bit_cast(bf16x8, piece[i]);
-                bf16x8 vf[DT][3];
+                // (Two tiles of V at a time: with all four of a wide head, registers spill.)
+                constexpr int VT = DT == 4 ? 2 : DT;
 #pragma unroll
-                for (int dt = 0; dt < DT; ++dt)
+                for (int d0 = 0; d0 < DT; d0 += VT) {
+                    bf16x8 vf[VT][3];
 #pragma unroll
-                    for (int i = 0; i < 3; ++i)
-                        vf[dt][i] = *reinterpret_cast<const bf16x8 *>(vs + (dt * 4 + t * 2 + j) * 3072 + i * 1024);
+                    for (int dt = 0; dt < VT; ++dt)
 #pragma unroll
-                for (int i = 0; i < 6; ++i)
+                        for (int i = 0; i < 3; ++i)
+                            vf[dt][i] = *reinterpret_cast<const bf16x8 *>(vs + ((d0 + dt) * (2 * KT) + t * 2 + j) * 3072 + i * 1024);
 #pragma unroll
-                    for (int dt = 0; dt < DT; ++dt) {
-                        const int at = CHAINS == 1 ? dt : i & 1;
-                        oacc[at] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[dt][kFirst[i]], pf[kSecond[i]], oacc[at], 0, 0, 0);
-                    }
+                    for (int i = 0; i < 6; ++i)
+#pragma unroll
+                        for (int dt = 0; dt < VT; ++dt) {
+                            const int at = CHAINS == 1 ? d0 + dt : i & 1;
+                            oacc[at] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[dt][kFirst[i]], pf[kSecond[i]], oacc[at], 0, 0, 0);
+                        }
+                }
             }
         run_sum += tile_sum;
     };
@@ -1072,7 +1092,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_split_kernel(AttnArg
     for (; t < plain_stages; ++t) {
         const bool more = t + 1 < stages;
         if (more) load_global(key_first + (t + 1) * BKV);
-        compute(std::integral_constant<int, 2>{}, std::false_type{}, t % BUFFERS, key_first + t * BKV);
+        compute(std::integral_constant<int, KT>{}, std::false_type{}, t % BUFFERS, key_first + t * BKV);
         if (BUFFERS == 1) __syncthreads();
         if (more) store_lds((t + 1) % BUFFERS);
         __syncthreads();
@@ -1081,7 +1101,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_split_kernel(AttnArg
         const bool more = t + 1 < stages;
         if (more) load_global(key_first + (t + 1) * BKV);
         const int key0 = key_first + t * BKV;
-        if (key0 + 32 < limit) compute(std::integral_constant<int, 2>{}, std::true_type{}, t % BUFFERS, key0);
+        if (KT == 2 && key0 + 32 < limit) compute(std::integral_constant<int, KT>{}, std::true_type{}, t % BUFFERS, key0);
         else if (key0 < limit) compute(std::integral_constant<int, 1>{}, std::true_type{}, t % BUFFERS, key0);
         if (BUFFERS == 1) __syncthreads();
         if (more) store_lds((t + 1) % BUFFERS);
@@ -1123,7 +1143,9 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_split_kernel(AttnArg
 // instructions' operands and are cut in registers, so that nothing waits for another wavefront before the end.  The next tile's
 // K is requested behind this one's logits, its V behind the outputs.
 // -------------------------------------------------------------------------------------------------
-constexpr int kKeysWaves = 8, kKeysRows = 32;
+constexpr int kKeysRows = 32;
+// Head sizes above 64 need the registers of a whole SIMD: four wavefronts a workgroup.
+constexpr int keys_waves(size_t head_dim) { return head_dim > 64 ? 4 : 8; }
 
 struct KeysItem {
     int q_tile, ctx, split;
@@ -1136,12 +1158,12 @@ __host__ __device__ inline KeysItem decode_keys_block(int contexts, int q_tiles,
 }
 
 template <int DPAD, bool CAUSAL, bool BIAS>
-__global__ __launch_bounds__(64 * kKeysWaves) void attention_f32_keys_kernel(AttnArgs p)
+__global__ __launch_bounds__(64 * keys_waves(DPAD)) void attention_f32_keys_kernel(AttnArgs p)
 {
-    constexpr int QSTEPS = DPAD / 16, DT = DPAD / 32, OS = DPAD + 4, STRIDE = 32 * kKeysWaves;
+    constexpr int WAVES = keys_waves(DPAD), QSTEPS = DPAD / 16, DT = DPAD / 32, OS = DPAD + 4, STRIDE = 32 * WAVES;
     constexpr float kWild = 0x1p40f, kScale = 0x1p24f, kUnscale = 0x1p-48f;
     extern __shared__ __attribute__((aligned(16))) float keys_lds[];  // [wave][32 rows][OS], maxima and sums [wave][32]
-    float *const maxima = keys_lds + kKeysWaves * 32 * OS, *const sums = maxima + kKeysWaves * 32;
+    float *const maxima = keys_lds + WAVES * 32 * OS, *const sums = maxima + WAVES * 32;
     __shared__ int any_wild;
 
     const int tid = threadIdx.x;
@@ -1299,7 +1321,7 @@ __global__ __launch_bounds__(64 * kKeysWaves) void attention_f32_keys_kernel(Att
     run_sum += __shfl_xor(run_sum, 32);
     float unscale = kUnscale;
     if (any_wild != 0) {  // a run of keys each, in f32
-        const int per = max(key_end - key_first + kKeysWaves - 1, 0) / kKeysWaves, first = min(key_first + wave * per, key_end);
+        const int per = max(key_end - key_first + WAVES - 1, 0) / WAVES, first = min(key_first + wave * per, key_end);
         redo_sums<DPAD, CAUSAL, BIAS>(p, ctx, q0, lane, first, min(first + per, key_end), scale_log2e, exp_scale, oacc, run_max, run_sum);
         unscale = 1.0f;
     }
@@ -1312,7 +1334,7 @@ __global__ __launch_bounds__(64 * kKeysWaves) void attention_f32_keys_kernel(Att
     __syncthreads();
     float top = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < kKeysWaves; ++w) top = fmaxf(top, maxima[w * 32 + li]);
+    for (int w = 0; w < WAVES; ++w) top = fmaxf(top, maxima[w * 32 + li]);
     const float mine = unscale * __builtin_amdgcn_exp2f((run_max - (top == -INFINITY ? 0.0f : top)) * exp_scale);  // no keys: 0
 #pragma unroll
     for (int t = 0; t < DT; ++t)
@@ -1324,24 +1346,28 @@ __global__ __launch_bounds__(64 * kKeysWaves) void attention_f32_keys_kernel(Att
             *reinterpret_cast<f32x4 *>(&keys_lds[(wave * 32 + li) * OS + t * 32 + g * 8 + lh * 4]) = part;
         }
     __syncthreads();
-    const int row = tid >> 4, d = (tid & 15) * 4;
-    if (q0 + row >= S || d >= D) return;
-    float row_top = -INFINITY, total = 0.0f;
-#pragma unroll
-    for (int w = 0; w < kKeysWaves; ++w) row_top = fmaxf(row_top, maxima[w * 32 + row]);
-    row_top = row_top == -INFINITY ? 0.0f : row_top;
-    f32x4 out = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int w = 0; w < kKeysWaves; ++w) {
-        total += sums[w * 32 + row] * __builtin_amdgcn_exp2f((maxima[w * 32 + row] - row_top) * exp_scale);
-        out += *reinterpret_cast<const f32x4 *>(&keys_lds[(w * 32 + row) * OS + d]);
-    }
+    constexpr int QUADS = DPAD / 4;
     const bool partial = p.key_splits > 1;
-    const size_t at = (static_cast<size_t>(split) * p.contexts + ctx) * S + q0 + row;
-    const float inv = partial ? 1.0f : total > 0.0f ? 1.0f / total : 0.0f;
-    float *const dst = partial ? p.part_o + at * D : p.out + ctx_elem0 + static_cast<size_t>(q0 + row) * D;
-    *reinterpret_cast<float4 *>(dst + d) = make_float4(out[0] * inv, out[1] * inv, out[2] * inv, out[3] * inv);
-    if (partial && d == 0) *reinterpret_cast<float2 *>(p.part_ml + at * 2) = make_float2(total > 0.0f ? row_top : -INFINITY, total);
+#pragma unroll
+    for (int e = tid; e < 32 * QUADS; e += 64 * WAVES) {
+        const int row = e / QUADS, d = e % QUADS * 4;
+        if (q0 + row >= S || d >= D) continue;
+        float row_top = -INFINITY, total = 0.0f;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) row_top = fmaxf(row_top, maxima[w * 32 + row]);
+        row_top = row_top == -INFINITY ? 0.0f : row_top;
+        f32x4 out = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            total += sums[w * 32 + row] * __builtin_amdgcn_exp2f((maxima[w * 32 + row] - row_top) * exp_scale);
+            out += *reinterpret_cast<const f32x4 *>(&keys_lds[(w * 32 + row) * OS + d]);
+        }
+        const size_t at = (static_cast<size_t>(split) * p.contexts + ctx) * S + q0 + row;
+        const float inv = partial ? 1.0f : total > 0.0f ? 1.0f / total : 0.0f;
+        float *const dst = partial ? p.part_o + at * D : p.out + ctx_elem0 + static_cast<size_t>(q0 + row) * D;
+        *reinterpret_cast<float4 *>(dst + d) = make_float4(out[0] * inv, out[1] * inv, out[2] * inv, out[3] * inv);
+        if (partial && d == 0) *reinterpret_cast<float2 *>(p.part_ml + at * 2) = make_float2(total > 0.0f ? row_top : -INFINITY, total);
+    }
 }
 
 // -------------------------------------------------------------------------------------------------
@@ -1730,8 +1756,10 @@ int attention_route(size_t contexts, size_t sequence, size_t head_dim, float sca
     if (!vec || head_dim > 128 || sequence * head_dim * sizeof(float) >= (1ull << 31)) return ST_HIP_ATTN_KERNEL_GENERAL;
     // Many contexts of at most 64 positions: a wavefront per context.
     if (!bias && sequence <= 64 && contexts >= 256) return ST_HIP_ATTN_KERNEL_TINY;
+    // Wide heads with biases: up to 768 keys, and what one tile of keys holds only while the head's registers are few (1 × 16 × 128 biased
+    // 9.9 µs here, 10.3 by one wavefront of the split kernels).
     const bool bias_fits = sequence * (sequence + 256) * sizeof(float) < (1ull << 31);  // rows past the end included
-    if (head_dim <= 64 && !sums_in_reference_order(head_dim, scale) && (!bias || bias_fits)) return ST_HIP_ATTN_KERNEL_SPLIT;
+    if (!sums_in_reference_order(head_dim, scale) && (!bias || (bias_fits && (head_dim <= 64 || (sequence <= 768 && (head_dim <= 96 || sequence > 32)))))) return ST_HIP_ATTN_KERNEL_SPLIT;
     if (!bias) return ST_HIP_ATTN_KERNEL_FAST;
     // The biases where their rows can be read 128 bits at a time.
     return head_dim <= 64 && sequence % 4 == 0 && bias_aligned ? ST_HIP_ATTN_KERNEL_FAST_BIASED : ST_HIP_ATTN_KERNEL_GENERAL;
@@ -1807,7 +1835,7 @@ hipError_t launch_fast(AttnArgs args, hipStream_t stream)
 template <int DPAD, bool CAUSAL, bool BIAS, int WAVES>
 hipError_t launch_split_rows(AttnArgs args, hipStream_t stream)
 {
-    constexpr size_t lds_bytes = (WAVES == 8 ? 2 : 1) * static_cast<size_t>(2 * (DPAD / 16) + 4 * (DPAD / 32)) * 3072;
+    constexpr size_t lds_bytes = (WAVES == 8 ? 2 : 1) * (DPAD > 64 ? 1 : 2) * static_cast<size_t>(DPAD / 16 + 2 * (DPAD / 32)) * 3072;
     auto kernel = attention_f32_split_kernel<DPAD, CAUSAL, BIAS, WAVES>;
     const hipError_t rc = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                               static_cast<int>(lds_bytes));
@@ -1832,6 +1860,18 @@ size_t keys_shared(size_t contexts, size_t sequence, size_t head_dim, bool causa
 {
     const size_t workgroups = contexts * ((sequence + kKeysRows - 1) / kKeysRows);
     const bool padded = head_dim > 32 && head_dim < 64;
+    // Wide heads: a wavefront has a SIMD to itself and four of them 128 keys, runs of which are cut as far as one round of workgroups
+    // takes them; up to 256 keys in one run.  128-row tiles on the f32 matrix cores / here, µs, heads of 80 and 128: 1 × 128 22.4 / 9.0 and 23.6 /
+    // 13.0, 1 × 250 causal 62 / 12.3 and 64 / 17.4, 16 × 200 37 / 12.3 and 38 / 17.5, 1 × 1000 27 / 14.0 and 28.7 / 19.0, biased 1 × 700 172 / 13.4
+    // and 174 / 18.2.
+    if (head_dim > 64) {
+        if (workgroups > 256) return 0;
+        const size_t runs = (sequence + 127) / 128;
+        const bool one = sequence <= 256, cut = runs > 1 && runs * workgroups <= 256;
+        if (!one && !cut) return 0;
+        *keys_per_split = one ? sequence : 128;
+        return one ? 1 : runs;
+    }
     if (sequence <= (biased || (padded && !causal) ? 64 : 32) || workgroups > 256) return 0;
     auto us = [&](size_t splits, size_t keys) { return 5.5 + 1.9 * static_cast<double>((keys + 127) / 128) + (splits > 1 ? 4.5 : 0.0); };
     size_t best = 1, best_keys = sequence;
@@ -1864,7 +1904,7 @@ bool keys_plan_consistent(const AttnArgs &args, size_t blocks)
 template <int DPAD, bool CAUSAL, bool BIAS>
 hipError_t launch_keys(AttnArgs args, hipStream_t stream)
 {
-    constexpr size_t lds_bytes = kKeysWaves * 32 * (DPAD + 4 + 2) * sizeof(float);
+    constexpr size_t lds_bytes = keys_waves(DPAD) * 32 * (DPAD + 4 + 2) * sizeof(float);
     auto kernel = attention_f32_keys_kernel<DPAD, CAUSAL, BIAS>;
     hipError_t rc = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                               static_cast<int>(lds_bytes));
@@ -1881,7 +1921,7 @@ hipError_t launch_keys(AttnArgs args, hipStream_t stream)
     }
     const size_t blocks = static_cast<size_t>(args.contexts) * args.q_tiles * args.key_splits;
     if (!keys_plan_consistent(args, blocks)) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(64 * kKeysWaves), lds_bytes, stream, args);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(64 * keys_waves(DPAD)), lds_bytes, stream, args);
     rc = hipGetLastError();
     return rc != hipSuccess || args.key_splits == 1 ? rc : merge_parts(args, BIAS, 0, stream);
 }
@@ -1895,7 +1935,9 @@ hipError_t launch_split(AttnArgs args, hipStream_t stream)
         args.keys_per_split = static_cast<int>(keys);
         return launch_keys<DPAD, CAUSAL, BIAS>(args, stream);
     }
-    if (args.bq == 256) return launch_split_rows<DPAD, CAUSAL, BIAS, 8>(args, stream);
+    if constexpr (DPAD <= 64) {
+        if (args.bq == 256) return launch_split_rows<DPAD, CAUSAL, BIAS, 8>(args, stream);
+    }
     return launch_split_rows<DPAD, CAUSAL, BIAS, 4>(args, stream);
 }
 
@@ -2059,8 +2101,16 @@ hipError_t launch_attention_f32(size_t contexts, size_t sequence, size_t head_di
             if (bias) return causal ? launch_split<32, true, true>(args, stream) : launch_split<32, false, true>(args, stream);
             return causal ? launch_split<32, true, false>(args, stream) : launch_split<32, false, false>(args, stream);
         }
-        if (bias) return causal ? launch_split<64, true, true>(args, stream) : launch_split<64, false, true>(args, stream);
-        return causal ? launch_split<64, true, false>(args, stream) : launch_split<64, false, false>(args, stream);
+        if (head_dim <= 64) {
+            if (bias) return causal ? launch_split<64, true, true>(args, stream) : launch_split<64, false, true>(args, stream);
+            return causal ? launch_split<64, true, false>(args, stream) : launch_split<64, false, false>(args, stream);
+        }
+        if (head_dim <= 96) {
+            if (bias) return causal ? launch_split<96, true, true>(args, stream) : launch_split<96, false, true>(args, stream);
+            return causal ? launch_split<96, true, false>(args, stream) : launch_split<96, false, false>(args, stream);
+        }
+        if (bias) return causal ? launch_split<128, true, true>(args, stream) : launch_split<128, false, true>(args, stream);
+        return causal ? launch_split<128, true, false>(args, stream) : launch_split<128, false, false>(args, stream);
     }
     if (route == ST_HIP_ATTN_KERNEL_FAST) {
         if (head_dim <= 32) return causal ? launch_fast<32, true>(args, stream) : launch_fast<32, false>(args, stream);

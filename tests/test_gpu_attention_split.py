@@ -1,4 +1,4 @@
-"""f32 attention on the bf16 matrix cores (head sizes up to 64), every value as three exact bf16 pieces, against float64."""
+"""f32 attention on the bf16 matrix cores (head sizes up to 128), every value as three exact bf16 pieces, against float64."""
 import time
 
 import numpy as np
@@ -51,6 +51,30 @@ def test_against_float64(hip, contexts, seq, dim, causal, biased):
             error = got[c] - want
             assert np.sqrt(np.mean(error ** 2)) <= 2.0 ** -20 * np.sqrt(np.mean(want ** 2))
             assert np.abs(error).max() <= 2.0 ** -15
+
+
+# Heads padded to 96 and 128 values: shared keys in one run (one tile a wavefront, two, wavefronts without any) and in runs, 128-row tiles
+# unsplit, in pairs and with their keys cut, 32-key stages cut short; biases up to the longest that are served.
+@pytest.mark.parametrize("contexts,seq,causal,biased", [
+    (1, 1, False, False), (2, 31, True, False), (3, 33, False, True), (1, 128, True, True), (5, 129, False, False), (2, 255, True, False), (7, 257, False, True),
+    (1, 300, True, False), (1, 768, False, True), (16, 500, True, False), (40, 225, False, False), (70, 289, True, False), (33, 290, True, True)])
+@pytest.mark.parametrize("dim", [68, 80, 96, 100, 128])
+def test_wide_heads_against_float64(hip, contexts, seq, dim, causal, biased):
+    assert hip.attention_f32_launch_plan(contexts, seq, dim, causal, biased, scale=dim ** -0.5)["kernel"] == "split" or (dim > 96 and biased and seq <= 32)
+    test_against_float64(hip, contexts, seq, dim, causal, biased)
+
+
+@pytest.mark.parametrize("contexts,seq", [(2, 150), (2, 400), (80, 260)])  # shared keys in one run and in several, 128-row tiles
+@pytest.mark.parametrize("dim", [80, 128])
+def test_wide_heads_the_pieces_cannot_carry(hip, contexts, seq, dim):
+    rng = np.random.default_rng(dim + seq)
+    q, k, v = (rng.normal(size=(contexts, seq, dim)).astype(np.float32) for _ in range(3))
+    q[0, 5] *= np.float32(2.0 ** 45)
+    k[0, :6] *= np.float32(2.0 ** -45)
+    v[1, 40, dim - 1] = np.inf
+    got = run(hip, q, k, v, dim ** -0.5, True)
+    assert np.abs(got[0] - exact(q[0], k[0], v[0], float(np.float32(dim ** -0.5)), True)).max() <= 2.0 ** -15
+    assert not np.isfinite(got[1, 40:, dim - 1]).any() and np.isfinite(got[1, :40]).all() and np.isfinite(got[1, :, :dim - 1]).all()
 
 
 def test_values_the_pieces_cannot_carry(hip):

@@ -91,6 +91,18 @@ def test_shared_keys_are_dealt_out_completely(causal, biased):
     assert {1, 4, 8} <= cut, cut
 
 
+@pytest.mark.parametrize("causal,biased", [(False, False), (True, False), (False, True), (True, True)])
+def test_wide_heads_are_dealt_out_completely(causal, biased):
+    kernels = set()
+    for contexts, seq, dim in itertools.product((1, 2, 7, 8, 31, 64, 128), SEQUENCES + (33, 96, 250, 333, 768, 769), (68, 96, 100, 128)):
+        plan = hip.attention_f32_launch_plan(contexts, seq, dim, causal, biased, scale=dim ** -0.5)
+        where = (contexts, seq, dim, causal, biased, plan)
+        assert plan["out_of_range"] == 0 and plan["duplicates"] == 0 and plan["items"] == plan["items_expected"], where
+        assert plan["kernel"] != "split" or plan["consistent"] == 1, where
+        kernels.add(plan["kernel"])
+    assert "split" in kernels
+
+
 def test_key_chunks_of_large_heads():
     # chunks of 128 keys, the last one shorter, where every workgroup has a compute unit to itself; otherwise as many keys as
     # two workgroups a unit leave each, 128 and more
