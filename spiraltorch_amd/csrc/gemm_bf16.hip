@@ -2131,20 +2131,33 @@ TilePlan plan_tiles(size_t m, size_t n, size_t k)
     return plan;
 }
 
-// Whether the small tiles of gemm_bf16_small.hip take an m×n×k product (operands on 16-byte boundaries), by the estimated time
-// of the kernels here: both tilings, k split or not, in rounds of what the chip holds; the general kernel where those do not
-// take the shape.  The constants are those of the split's estimate and about 4 µs a launch (measured 6.5 to 8 µs at k = 512
-// from 128 to 2048 rows).
-bool small_tiles_apply(size_t m, size_t n, size_t k)
+// The least estimated time of 128×128 tiles over k-splits: up to 256 workgroups, one a compute unit, are bound by the latency of their
+// k-tiles (0.41 µs each); beyond, two share a unit.
+double tiles_128_us(size_t m, size_t n, size_t k)
 {
-    if (k < 64 || k % 64 != 0) return false;
-    const size_t cols = (n + 127) / 128, tiles_128 = (m + 127) / 128 * cols, tiles_256 = (m + 255) / 256 * cols;
-    auto rounds = [](size_t tiles, size_t most) { return static_cast<double>((tiles + most - 1) / most); };
-    const double us = n % 128 != 0 && (m <= 64 || n <= 128)
-                          ? 6.0 + 0.01 * static_cast<double>(k)
-                          : 4.0 + std::min(rounds(tiles_128, 512) * estimate_k_splits(m, n, k, tiles_128, 512, 0.42).cost_us,
-                                           rounds(tiles_256, 256) * estimate_k_splits(m, n, k, tiles_256, 256, 0.5).cost_us);
-    return gemm_bf16_small_applies(m, n, k, us);
+    const size_t tiles = ((m + 127) / 128) * ((n + 127) / 128), k_tiles = k / 64;
+    double best = 1e30;
+    for (size_t splits = 1; splits == 1 || (splits * tiles <= 512 && splits * 2 <= k_tiles); ++splits) {
+        const double per = static_cast<double>((k_tiles + splits - 1) / splits), units = static_cast<double>(tiles * splits) / 256;
+        const double sums = splits > 1 ? 3.5 + static_cast<double>(splits * m * n) * 8.0 / 4.0e6 : 0.0;
+        best = std::min(best, 3.6 + 0.41 * per + std::min(units, 1.0) * (1.06 + 0.064 * per) + std::max(std::ceil(units) - 1, 0.0) * (2.0 + 0.35 * per) + sums);
+    }
+    return best;
+}
+
+// Which of the small tiles of gemm_bf16_small.hip takes an m×n×k product (operands on 16-byte boundaries), -1 for none, by the
+// estimated time of the kernels here: both tilings, k split or not, with the epilogue of a ragged n (4.5 µs); the general kernel where
+// those do not take the shape.
+int small_tile(size_t m, size_t n, size_t k)
+{
+    const GemmSmallChoice small = gemm_bf16_small_choice(m, n, k);
+    if (small.tile < 0) return -1;
+    const double k_tiles = static_cast<double>(k / 64);
+    if (n % 128 != 0 && (m <= 64 || n <= 128)) return small.pays(6.0 + 0.64 * k_tiles) ? small.tile : -1;
+    if (small.pays(std::min(3.6 + 0.41 * k_tiles, 6.9))) return small.tile;  // (less than what the tilings below take unsplit, and split)
+    const size_t tiles_256 = (m + 255) / 256 * ((n + 127) / 128);
+    const double us = std::min(tiles_128_us(m, n, k), 4.0 + static_cast<double>((tiles_256 + 255) / 256) * estimate_k_splits(m, n, k, tiles_256, 256, 0.5).cost_us);
+    return small.pays(us + (n % 128 != 0 ? 4.5 : 0.0)) ? small.tile : -1;
 }
 
 // The launch arithmetic of the tiled kernels whose workgroups decode their index into (k-split, tile), checked on the
@@ -2559,14 +2572,15 @@ hipError_t launch_gemm_bf16(size_t m, size_t n, size_t k, const uint16_t *lhs, c
     const size_t columns_most = m > 64 ? SIZE_MAX : (6500 + 200 * m) * (k >= 512 ? 5 : 4) / 4;
     const bool as_it_is = rhs_packed || n % 8 == 0;
     const bool packing_pays = n * k <= packing_most && n <= columns_most && (k > 64 || (m > 16 && n <= 450 * m));
-    if (aligned16(lhs) && aligned16(rhs) && fits_buffer && small_tiles_apply(m, n, k) && !(skinny && k > 1024) && (as_it_is || packing_pays)) {
-        if (as_it_is) return launch_gemm_bf16_small(m, n, k, lhs, rhs, rhs_packed, out_f32, out_bf16, epilogue, stream);
+    const int small = aligned16(lhs) && aligned16(rhs) && fits_buffer && !(skinny && k > 1024) && (as_it_is || packing_pays) ? small_tile(m, n, k) : -1;
+    if (small >= 0) {
+        if (as_it_is) return launch_gemm_bf16_small(small, m, n, k, lhs, rhs, rhs_packed, out_f32, out_bf16, epilogue, stream);
         void *workspace = nullptr;
         hipError_t rc = stream_workspace(stream, k * n * sizeof(uint16_t), &workspace);
         if (rc == hipSuccess) {
             rc = launch_transpose_u16(k, n, rhs, static_cast<uint16_t *>(workspace), stream);
             if (rc != hipSuccess) return rc;
-            return launch_gemm_bf16_small(m, n, k, lhs, static_cast<const uint16_t *>(workspace), true, out_f32, out_bf16, epilogue, stream);
+            return launch_gemm_bf16_small(small, m, n, k, lhs, static_cast<const uint16_t *>(workspace), true, out_f32, out_bf16, epilogue, stream);
         }
         if (!scratch_unavailable(rc)) return rc;  // else the kernels below, of which the general one reads B as it is
     }
@@ -2589,7 +2603,7 @@ hipError_t launch_gemm_bf16(size_t m, size_t n, size_t k, const uint16_t *lhs, c
             args.B = static_cast<const uint16_t *>(workspace);
         }
         const size_t tiles_128 = ((m + 127) / 128) * ((n + 127) / 128);
-        if (plan.tiles < 192 && tiles_128 >= 2 * plan.tiles && plan.k_splits == 1) return launch_128(args, true, stream);
+        if (plan.tiles < 192 && (tiles_128 <= 256 || tiles_128 >= 2 * plan.tiles) && plan.k_splits == 1) return launch_128(args, true, stream);
         if (plan.narrow) return launch_256<128>(args, true, stream, workspace_offset);
         return launch_256_rounds(args, true, plan, stream, workspace_offset);
     }
@@ -2613,11 +2627,13 @@ hipError_t launch_gemm_bf16(size_t m, size_t n, size_t k, const uint16_t *lhs, c
     if (fits_256) {
         const TilePlan plan = plan_tiles(m, n, k);
         const bool narrow = plan.narrow;
+        // (As 128×128 tiles they are at most a workgroup a unit: 840×1536×512 8.9 -> 7.5 µs, 600×3072×768 11.0 -> 9.4, 1575×768×768 11.2 -> 9.0,
+        // 840×1024×256 6.6 -> 5.2; B row-major 600×2304×768 15.2 -> 11.4.)
         // A 256-row tiling that would leave most compute units without a tile, and a k not worth splitting: 128×128
         // tiles, two workgroups per compute unit (1024³: 16 tiles of 256×256, 64 of 128×128).
         const size_t tiles_256 = plan.tiles;
         const size_t tiles_128 = ((m + 127) / 128) * (n / 128);
-        if (tiles_256 < 192 && tiles_128 >= 2 * tiles_256) {
+        if (tiles_256 < 192 && (tiles_128 <= 256 || tiles_128 >= 2 * tiles_256)) {
             // Either tiling may split k; the smaller tiles need fewer splits (less partial-sum traffic) for the same
             // number of workgroups, and two of their workgroups share a compute unit.
             const SplitChoice big = estimate_k_splits(m, n, k, tiles_256, 256, 0.5);
@@ -2700,13 +2716,13 @@ GemmTilePlanReport gemm_bf16_tile_plan_report(size_t m, size_t n, size_t k)
 bool residual_layer_norm_single(size_t m, size_t n, size_t k)
 {
     return n == 512 && m > 64 && k >= 64 && k % 64 == 0 && k <= 1024 && m * k * 2 < (1ull << 31) && plan_tiles(m, n, k).k_splits == 1 &&
-           !small_tiles_apply(m, n, k);
+           small_tile(m, n, k) < 0;
 }
 
 int gemm_bf16_routes(size_t m, size_t n, size_t k)
 {
     if (m == 0 || n == 0 || k < 64 || k % 64 != 0 || m * k * 2 >= (1ull << 31) || k * n * 2 >= (1ull << 31)) return 0;
-    return (small_tiles_apply(m, n, k) ? ST_HIP_GEMM_BF16_SMALL_TILES : columns_behind_rounds(m, n, plan_tiles(m, n, k)) > 0 ? ST_HIP_GEMM_BF16_COLUMNS_BEHIND : 0) |
+    return (small_tile(m, n, k) >= 0 ? ST_HIP_GEMM_BF16_SMALL_TILES : columns_behind_rounds(m, n, plan_tiles(m, n, k)) > 0 ? ST_HIP_GEMM_BF16_COLUMNS_BEHIND : 0) |
            (residual_layer_norm_single(m, n, k) ? ST_HIP_GEMM_BF16_RESIDUAL_LAYER_NORM : 0);
 }
 

@@ -8,11 +8,12 @@
 // results do not depend on scheduling, and are the same for both layouts of B.
 //
 // What bounds it is latency: a launch (2.0 µs for an empty kernel), one trip to memory, the sums' trip through LDS.  Of a
-// launch among others, before -> here: 117×1536×512 10.4 -> 4.1 µs, 117×512×512 10.1 -> 3.1, 117×2048×512 10.0 -> 4.0,
+// launch among others, before -> here: 117×1536×512 10.4 -> 3.6 µs, 117×512×512 10.1 -> 3.1, 117×2048×512 10.0 -> 3.6,
 // 117×512×2048 11.4 -> 4.5, 512×1536×512 8.3 -> 7.0, 1024×512×2048 14.4 -> 9.6, 256×1000×512 11.0 -> 4.3.  Larger launches are
 // bound by LDS and L2 traffic (16 to 32 flops a byte) and belong to the large tiles.  Layer normalisation of the rows on their
 // way in was tried: 3.2 µs more a launch, where the kernel of its own takes 2.4.
 #include <algorithm>
+#include <cmath>
 
 #include "device_math.h"
 #include "kernels.h"
@@ -231,64 +232,70 @@ __global__ __launch_bounds__(512) void gemm_bf16_small_32x16_rm_kernel(SmallArgs
 __global__ __launch_bounds__(512) void gemm_bf16_small_32x32_rm_kernel(SmallArgs p) { gemm_bf16_small_body<2, 2, 8, true>(p); }
 __global__ __launch_bounds__(256) void gemm_bf16_small_64x64_rm_kernel(SmallArgs p) { gemm_bf16_small_body<4, 4, 4, true>(p); }
 
-// Estimated time with `tiles` workgroups on the chip: a tile alone, and what each further round of 256 adds (µs; the first
-// of a pair is constant, the second per 64 of k), fitted to some two hundred products of 16 to 4096 rows, k = 256 to 4096, each
-// timed with every tile: 5 % of the estimates are more than a fifth too high, 5 % more than a fourth too low.
+// Estimated time (µs; of a pair the first is constant, the second per 64 of k): a launch alone, what 256 workgroups add, what having more
+// than 256 adds, and each further round, a round being what the compute units hold at a time.  Fitted to some 200 products a tile of 33 to 4096 rows, 14 shapes of n and
+// k from 256 to 4096, the small ones timed without the host between them, operands that the L2 does not hold from the launch before:
+// within 15 % of each, 5 % in the rms.
 struct SmallTimes {
-    double alone, alone_k, round, round_k;
+    double alone, alone_k, units, units_k, second, round, round_k;
 };
 struct SmallConfig {
     void (*packed)(SmallArgs);
     void (*rowmajor)(SmallArgs);
-    int bm, bn, waves;
+    int bm, bn, waves;  // powers of two
     SmallTimes packed_us, rowmajor_us;
 
     size_t tiles(size_t m, size_t n) const { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); }
-    double us(size_t m, size_t n, size_t k, const SmallTimes &t) const
-    {
-        const double k_tiles = static_cast<double>(k) / 64, rounds = static_cast<double>(tiles(m, n)) / 256;
-        return t.alone + t.alone_k * k_tiles + std::max(rounds - 0.5, 0.0) * (t.round + t.round_k * k_tiles);
-    }
     // A wavefront's stages (one is enough where it has one k-tile), and its sums in the same place.
     size_t ring_bytes(size_t k) const
     {
-        const size_t stages = (k / 64 + waves - 1) / waves > 1 ? kSmallStages : 1;
+        const size_t stages = k / 64 > static_cast<size_t>(waves) ? kSmallStages : 1;
         return std::max<size_t>(stages * (bm + bn) * 128, static_cast<size_t>(bm) * (bn + 4) * sizeof(float));
     }
 };
 const SmallConfig kSmallConfigs[] = {
-    {gemm_bf16_small_32x16_kernel, gemm_bf16_small_32x16_rm_kernel, 32, 16, 8, {2.53, 0.060, 0.26, 0.092}, {2.55, 0.134, 0.14, 0.127}},
-    {gemm_bf16_small_32x32_kernel, gemm_bf16_small_32x32_rm_kernel, 32, 32, 8, {2.86, 0.081, 0.49, 0.140}, {2.55, 0.149, 0.48, 0.150}},
-    {gemm_bf16_small_64x64_kernel, gemm_bf16_small_64x64_rm_kernel, 64, 64, 4, {4.12, 0.163, 1.38, 0.258}, {3.98, 0.227, 1.29, 0.325}},
+    {gemm_bf16_small_32x16_kernel, gemm_bf16_small_32x16_rm_kernel, 32, 16, 8,
+     {2.42, 0.051, 0.22, 0.034, 0.40, 1.03, 0.028}, {2.42, 0.094, 0.39, 0.025, 0.40, 0.77, 0.090}},
+    {gemm_bf16_small_32x32_kernel, gemm_bf16_small_32x32_rm_kernel, 32, 32, 8,
+     {2.44, 0.089, 0.57, 0.005, 0.00, 1.09, 0.069}, {2.44, 0.124, 0.47, 0.008, 0.00, 1.30, 0.097}},
+    {gemm_bf16_small_64x64_kernel, gemm_bf16_small_64x64_rm_kernel, 64, 64, 4,
+     {3.89, 0.174, 1.03, 0.000, 0.00, 2.33, 0.159}, {3.89, 0.227, 1.08, 0.000, 0.00, 3.62, 0.135}},
 };
-
-// The same tile for both layouts of B, so that they give the same bits.
-const SmallConfig &choose_small(size_t m, size_t n, size_t k)
-{
-    const SmallConfig *best = nullptr;
-    double best_us = 0.0;
-    for (const SmallConfig &c : kSmallConfigs) {
-        const double us = c.us(m, n, k, c.packed_us) + 0.3 * c.us(m, n, k, c.rowmajor_us);
-        if (best == nullptr || us < best_us) best = &c, best_us = us;
-    }
-    return *best;
-}
 
 }  // namespace
 
-bool gemm_bf16_small_applies(size_t m, size_t n, size_t k, double other_us)
+// The same tile for both layouts of B, so that they give the same bits.  (Asked for every launch, of which a short decoder makes forty: no
+// 64-bit divisions.)
+GemmSmallChoice gemm_bf16_small_choice(size_t m, size_t n, size_t k)
 {
+    GemmSmallChoice best;
     // 32-bit byte offsets up to a tile past the operands' ends
-    if (m == 0 || n == 0 || k < 64 || k % 64 != 0 || k > 65536 || (m + 64) * k * 2 >= (1ull << 31) || (n + 64) * k * 2 >= (1ull << 31))
-        return false;
-    const SmallConfig &c = choose_small(m, n, k);
-    return c.us(m, n, k, c.packed_us) < 0.9 * other_us && c.us(m, n, k, c.rowmajor_us) < 1.1 * other_us;
+    if (m == 0 || n == 0 || k < 64 || k % 64 != 0 || k > 65536 || (m + 64) * k * 2 >= (1ull << 31) || (n + 64) * k * 2 >= (1ull << 31)) return best;
+    const double k_tiles = static_cast<double>(k / 64);
+    double best_us = 0.0;
+    for (int i = 0; i < 3; ++i) {
+        const SmallConfig &c = kSmallConfigs[i];
+        const unsigned bm = static_cast<unsigned>(c.bm), bn = static_cast<unsigned>(c.bn);
+        const double units = static_cast<double>((static_cast<unsigned>(m) + bm - 1) >> __builtin_ctz(bm)) *
+                             static_cast<double>((static_cast<unsigned>(n) + bn - 1) >> __builtin_ctz(bn)) / 256;
+        const unsigned resident = std::min(160u * 1024 / (static_cast<unsigned>(c.ring_bytes(k)) * c.waves), 32u / c.waves);
+        const double rounds = units > resident ? std::ceil(units / resident) - 1 : 0.0;
+        auto us = [&](const SmallTimes &t) {
+            return t.alone + t.alone_k * k_tiles + units * (t.units + t.units_k * k_tiles) + (units > 1.0 ? t.second : 0.0) + rounds * (t.round + t.round_k * k_tiles);
+        };
+        const double packed = us(c.packed_us), rowmajor = us(c.rowmajor_us);
+        if (best.tile < 0 || packed + 0.3 * rowmajor < best_us) {
+            best = GemmSmallChoice{i, packed, rowmajor};
+            best_us = packed + 0.3 * rowmajor;
+        }
+    }
+    return best;
 }
 
-hipError_t launch_gemm_bf16_small(size_t m, size_t n, size_t k, const uint16_t *lhs, const uint16_t *rhs, bool rhs_packed, float *out_f32,
+hipError_t launch_gemm_bf16_small(int tile, size_t m, size_t n, size_t k, const uint16_t *lhs, const uint16_t *rhs, bool rhs_packed, float *out_f32,
                                   uint16_t *out_bf16, const GemmEpilogue &epilogue, hipStream_t stream)
 {
-    const SmallConfig &config = choose_small(m, n, k);
+    const SmallConfig &config = kSmallConfigs[tile];
     auto aligned = [](const void *ptr, uintptr_t bytes) { return (reinterpret_cast<uintptr_t>(ptr) & (bytes - 1)) == 0; };
     SmallArgs args;
     args.A = lhs;

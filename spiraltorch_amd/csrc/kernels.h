@@ -74,10 +74,15 @@ hipError_t launch_gemm_bf16(size_t m, size_t n, size_t k, const uint16_t *lhs, c
                             float *out_f32, uint16_t *out_bf16, const GemmEpilogue &epilogue,
                             hipStream_t stream, bool rhs_packed = false);
 // The same products on small tiles with k split inside the workgroup (gemm_bf16_small.hip), operands on 16-byte boundaries, a
-// row-major rhs of a multiple of eight columns.  `applies`: k a multiple of 64, operands that fit 32-bit offsets and an
-// estimated time below `other_us`.
-bool gemm_bf16_small_applies(size_t m, size_t n, size_t k, double other_us);
-hipError_t launch_gemm_bf16_small(size_t m, size_t n, size_t k, const uint16_t *lhs, const uint16_t *rhs, bool rhs_packed, float *out_f32,
+// row-major rhs of a multiple of eight columns.  The tile that suits a product best and its estimated times; none (-1) where k is no
+// multiple of 64 or operands do not fit 32-bit offsets.
+struct GemmSmallChoice {
+    int tile = -1;
+    double packed_us = 0.0, rowmajor_us = 0.0;
+    bool pays(double other_us) const { return tile >= 0 && packed_us < 0.97 * other_us && rowmajor_us < 1.15 * other_us; }
+};
+GemmSmallChoice gemm_bf16_small_choice(size_t m, size_t n, size_t k);
+hipError_t launch_gemm_bf16_small(int tile, size_t m, size_t n, size_t k, const uint16_t *lhs, const uint16_t *rhs, bool rhs_packed, float *out_f32,
                                   uint16_t *out_bf16, const GemmEpilogue &epilogue, hipStream_t stream);
 // The launch arithmetic of the 256-row bf16 kernels for a shape, every workgroup decoded on the host: see
 // st_hip_gemm_tile_plan.
