@@ -87,6 +87,9 @@ SIGNATURES = {
     "st_hip_last_error_message": (c_size_t, [c_char_p, c_size_t]),
     "st_hip_malloc": (c_int, [POINTER(c_void_p), c_size_t]),
     "st_hip_free": (c_int, [c_void_p]),
+    "st_hip_tensor_malloc": (c_int, [POINTER(c_void_p), c_size_t]),
+    "st_hip_tensor_free": (c_int, [c_void_p, c_size_t]),
+    "st_hip_tensor_upload": (c_int, [c_void_p, c_void_p, c_size_t]),
     "st_hip_memcpy_h2d": (c_int, [c_void_p, c_void_p, c_size_t, c_void_p]),
     "st_hip_memcpy_d2h": (c_int, [c_void_p, c_void_p, c_size_t, c_void_p]),
     "st_hip_memset_zero": (c_int, [c_void_p, c_size_t, c_void_p]),

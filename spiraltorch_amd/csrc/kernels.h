@@ -254,6 +254,8 @@ struct PinnedBuffer {
 constexpr size_t kPinnedMost = 64u << 20;
 bool pinned_acquire(size_t bytes, PinnedBuffer *out);
 void pinned_release(const PinnedBuffer &buffer);
+// The same for a buffer that a kernel may still be reading: until all `count` words are set.  They lie in the buffer.
+void pinned_release_when_read(const PinnedBuffer &buffer, const unsigned *words, size_t count);
 void pinned_release_idle();  // frees what no call holds
 // What a caller's "host" pointer is: memory of the host, pinned or not, or what only the runtime's copies may touch (managed memory, and
 // device memory, which they have always taken).
@@ -263,13 +265,15 @@ HostMemory host_memory(const void *host);
 // relu(A·B + bias) with square operands of 0.34, 0.67, 1, 2, 4 and 16 MiB and a result of the same size, staged up to 0.5 / 1 / 4 MiB: 73 / 73 / 72,
 // 114 / 111 / 111, 135 / 136 / 136, 252 / 252 / 269, 415 / 411 / 443, 2035 / 2043 / 2040; 88, 121, 156, 291, 539, 2330 without staging), its results
 // (2048×2048 of one term 585 against 1002), and st_hip_memcpy_d2h (1 KiB 13 against 21, 16 KiB 13 against 27, 256 KiB 19.5 against 20.4, 512 KiB
-// 29.5 against 30.9, 2 MiB 110 against 119; a read is staged whole, so that more than the ring's size would be held for it alone).  A
+// 29.5 against 30.9, 2 MiB 110 against 119; by a kernel that says what has arrived, without waiting for the stream; a read is staged whole, so that more than the ring's size would be held for it alone).  A
 // result goes through a ring: pinned memory takes 0.25 to 0.5 ms a MiB to allocate, and is then held.
 constexpr size_t kUploadMost = 512u << 10, kDownloadMost = 16u << 20, kDownloadRing = 2u << 20, kReadMost = kDownloadRing;
 // device[0, bytes) = pinned[0, bytes) by a kernel (device on a 16-byte boundary), and back: the piece of kCopyPiece bytes with
 // number p is in host memory when word p of `arrived` (host memory, cleared before) is not zero.
 constexpr size_t kCopyPiece = 16u << 10;
-hipError_t launch_copy_from_pinned(void *device, const void *pinned, size_t bytes, hipStream_t stream);
+// `read`: host memory, a word for every kUploadGroup bytes, set (from 0) when the kernel has read them.
+constexpr size_t kUploadGroup = 4096;
+hipError_t launch_copy_from_pinned(void *device, const void *pinned, size_t bytes, hipStream_t stream, unsigned *read = nullptr);
 hipError_t launch_copy_to_pinned(void *pinned, const void *device, size_t bytes, unsigned *arrived, hipStream_t stream);
 // Host<->device copies made by the library, for tests that check where tensors live.
 void count_transfer(bool to_device, size_t bytes);

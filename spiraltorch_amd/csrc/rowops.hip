@@ -824,13 +824,17 @@ __global__ __launch_bounds__(256) void nonfinite_probe_kernel(size_t count, cons
 // 16 bytes a lane, and as many workgroups as that makes: what one compute unit has in flight to the host bounds it otherwise (three
 // operands of 16 KiB in one workgroup each, four loads a lane: a call of 50 µs instead of 35, of 32 KiB 54 and 40).  The last bytes one
 // by one.
-constexpr size_t kUploadGroup = 256 * 16;
-__global__ __launch_bounds__(256) void copy_from_pinned_kernel(size_t bytes, const unsigned char *pinned, unsigned char *device)
+static_assert(kUploadGroup == 256 * 16, "a load a lane");
+// `read`, if given: a word a workgroup, set when it has read its part.
+__global__ __launch_bounds__(256) void copy_from_pinned_kernel(size_t bytes, const unsigned char *pinned, unsigned char *device, unsigned *read)
 {
     const size_t at = blockIdx.x * kUploadGroup + threadIdx.x * 16;
     if (at + 16 <= bytes) *reinterpret_cast<uint4 *>(device + at) = *reinterpret_cast<const uint4 *>(pinned + at);
     else
         for (size_t e = at; e < bytes; ++e) device[e] = pinned[e];
+    if (read == nullptr) return;
+    __syncthreads();  // (waits for this workgroup's memory accesses)
+    if (threadIdx.x == 0) __hip_atomic_store(&read[blockIdx.x], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // The other way.  The stores go to host memory past the caches (system scope); each wavefront waits for its own to be
@@ -1359,10 +1363,10 @@ hipError_t launch_nonfinite_probe_f32(size_t count, const float *data, unsigned 
     return hipGetLastError();
 }
 
-hipError_t launch_copy_from_pinned(void *device, const void *pinned, size_t bytes, hipStream_t stream)
+hipError_t launch_copy_from_pinned(void *device, const void *pinned, size_t bytes, hipStream_t stream, unsigned *read)
 {
     hipLaunchKernelGGL(copy_from_pinned_kernel, dim3(static_cast<unsigned>((bytes + kUploadGroup - 1) / kUploadGroup)), dim3(256), 0, stream, bytes,
-                       static_cast<const unsigned char *>(pinned), static_cast<unsigned char *>(device));
+                       static_cast<const unsigned char *>(pinned), static_cast<unsigned char *>(device), read);
     return hipGetLastError();
 }
 

@@ -351,6 +351,28 @@ class DeviceBuffer:
             pass
 
 
+class TensorBuffer(DeviceBuffer):
+    """Device memory that is used on the default stream alone: kept by the library for the next one when freed."""
+
+    def __init__(self, nbytes: int):
+        self.nbytes = int(nbytes)
+        ptr = ctypes.c_void_p()
+        _check(_lib.load().st_hip_tensor_malloc(ctypes.byref(ptr), self.nbytes))
+        self.ptr = ptr
+
+    @classmethod
+    def from_array(cls, array: np.ndarray) -> "TensorBuffer":
+        a = np.ascontiguousarray(array)
+        buf = cls(a.nbytes)
+        _check(_lib.load().st_hip_tensor_upload(buf.ptr, ctypes.c_void_p(a.ctypes.data), a.nbytes))
+        return buf
+
+    def free(self) -> None:
+        if self.ptr is not None and self.ptr.value:
+            _lib.load().st_hip_tensor_free(self.ptr, self.nbytes)
+            self.ptr = None
+
+
 class Stream:
     """Owning stream handle (HipStream of real.rs:190-214); default priority."""
 

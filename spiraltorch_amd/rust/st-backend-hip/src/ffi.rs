@@ -133,6 +133,9 @@ extern "C" {
     pub fn st_hip_last_error_message(buf: *mut c_char, len: usize) -> usize;
     pub fn st_hip_malloc(device_ptr: *mut *mut c_void, bytes: usize) -> c_int;
     pub fn st_hip_free(device_ptr: *mut c_void) -> c_int;
+    pub fn st_hip_tensor_malloc(device_ptr: *mut *mut c_void, bytes: usize) -> c_int;
+    pub fn st_hip_tensor_free(device_ptr: *mut c_void, bytes: usize) -> c_int;
+    pub fn st_hip_tensor_upload(device_ptr: *mut c_void, host_src: *const c_void, bytes: usize) -> c_int;
     pub fn st_hip_memcpy_h2d(device_dst: *mut c_void, host_src: *const c_void, bytes: usize, stream: *mut c_void) -> c_int;
     pub fn st_hip_memcpy_d2h(host_dst: *mut c_void, device_src: *const c_void, bytes: usize, stream: *mut c_void) -> c_int;
     pub fn st_hip_memset_zero(device_dst: *mut c_void, bytes: usize, stream: *mut c_void) -> c_int;

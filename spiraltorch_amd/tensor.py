@@ -65,7 +65,7 @@ class PackedB:
         the bus for a weight that already lives on the device.  The host copy is fetched only if `as_slice` asks."""
         pack = cls(tensor.rows, tensor.cols, None)
         try:
-            pack._dev = hip.DeviceBuffer(max(len(tensor), 1) * 4)
+            pack._dev = hip.TensorBuffer(max(len(tensor), 1) * 4)
             if len(tensor):
                 hip.pack_rhs_f32_dev(tensor.rows, tensor.cols, tensor._device(), pack._dev)
         except hip.HipErr as err:
@@ -98,7 +98,7 @@ class PackedB:
     def _device(self) -> hip.DeviceBuffer:
         if self._dev is None:
             source = getattr(self, "_source", None)
-            self._dev = source._device() if source is not None else hip.DeviceBuffer.from_array(self._buf)
+            self._dev = source._device() if source is not None else hip.TensorBuffer.from_array(self._buf)
         return self._dev
 
 
@@ -143,7 +143,7 @@ class Tensor:
         out.rows, out.cols = int(rows), int(cols)
         out._host = None
         try:
-            out._dev = hip.DeviceBuffer(max(out.rows * out.cols, 1) * 4)
+            out._dev = hip.TensorBuffer(max(out.rows * out.cols, 1) * 4)
         except hip.HipErr as err:
             raise _backend_failure(err) from err
         out._finite = None
@@ -185,7 +185,7 @@ class Tensor:
     def _device(self) -> hip.DeviceBuffer:
         if self._dev is None:
             try:
-                self._dev = hip.DeviceBuffer.from_array(self._host)
+                self._dev = hip.TensorBuffer.from_array(self._host)
             except hip.HipErr as err:
                 raise _backend_failure(err) from err
         return self._dev

@@ -127,3 +127,63 @@ def test_copies_after_the_kept_memory_was_freed(hip):
     for _ in range(3):
         assert (outer(hip, column, row) == column[:, None] * row[None, :]).all()
         hip.release_scratch()
+
+
+@pytest.mark.parametrize("size", [1, 7, 8, 9, 4095, 4096, 4097, 16383, 16384, 16385, 100003, (1 << 19) - 1, 1 << 19, (1 << 19) + 1, (1 << 21) - 3, 1 << 21, (1 << 21) + 5])
+def test_every_byte_of_a_tensor_up_and_down(hip, size):
+    """Around a workgroup's part of an upload, a piece of a read, what is staged up and down, and what is no multiple of eight bytes."""
+    data = np.random.default_rng(size).integers(0, 256, size).astype(np.uint8)
+    for kind in (hip.TensorBuffer, hip.DeviceBuffer):
+        d = kind.from_array(data)
+        assert (d.to_array(np.uint8, size) == data).all()
+        if size > 5000:  # from the middle, on a 16-byte boundary and off it
+            for first in (4096, 4099):
+                out = np.empty(size - first, np.uint8)
+                status = __import__("spiraltorch_amd._lib", fromlist=["load"]).load().st_hip_memcpy_d2h(
+                    ctypes.c_void_p(out.ctypes.data), ctypes.c_void_p(d.at(first)), out.nbytes, None)
+                assert status == 0 and (out == data[first:]).all()
+
+
+def test_tensor_memory_taken_over_while_its_last_use_is_queued(hip):
+    """A tensor is freed with kernels on it still queued, and its memory goes to the next one, whose values are uploaded at once."""
+    n = 128 * 1024  # half a MiB: staged
+    before = hip.DeviceBuffer.from_array(np.arange(n, dtype=np.float32))
+    outs = [hip.DeviceBuffer(n * 4) for _ in range(8)]
+    busy = hip.DeviceBuffer.from_array(np.zeros((2048, 2048), np.float32))
+    result = hip.DeviceBuffer(2048 * 2048 * 4)
+    addresses, source = set(), np.empty(n, np.float32)
+    for i, out in enumerate(outs):
+        source[:] = i + 1.0
+        tensor = hip.TensorBuffer.from_array(source)
+        source[:] = -77.0  # the call has taken its copy
+        addresses.add(tensor.ptr.value)
+        hip.gemm_f32_dev(2048, 2048, 2048, 1.0, False, busy, busy, result)  # the reads below are queued behind this
+        hip.scale_f32_dev(n, tensor, 2.0, out)
+        tensor.free()
+    assert len(addresses) < len(outs)
+    for i, out in enumerate(outs):
+        assert (out.to_array(np.float32, n) == 2.0 * (i + 1.0)).all(), i
+    assert (before.to_array(np.float32, n) == np.arange(n)).all()
+
+
+def test_tensors_from_several_threads_keep_their_values(hip):
+    import spiraltorch_amd as st
+    wrong = []
+
+    def work(seed):
+        rng = np.random.default_rng(seed)
+        for _ in range(40):
+            rows, cols = int(rng.integers(1, 300)), int(rng.integers(1, 300))
+            x = rng.integers(-99, 99, (rows, cols)).astype(np.float32)
+            y = st.Tensor.from_numpy(x).scale(2.0).scale(0.25)
+            if not (y.numpy() == x * 0.5).all():
+                wrong.append((seed, rows, cols))
+
+    threads = [threading.Thread(target=work, args=(seed,)) for seed in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert wrong == []
+    hip.release_scratch()
+    assert hip.pinned_memory_counters()[0] == 0
