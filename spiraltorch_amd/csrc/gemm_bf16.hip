@@ -462,55 +462,57 @@ __device__ __forceinline__ void gemm_bf16_epilogue_ragged(const GemmBf16Args &p,
         for (int e = 0; e < 4; ++e)
             if (col0 + e < N) bias[e] = p.bias[col0 + e];
     }
+    // (Activation, residual and outputs are decided once per wavefront here as well.  Decided per element, as they were, they cost a
+    // 128×128 tile 4 µs and a 256×256 tile 8.)
+    auto run = [&](auto &&act, auto residual_tag, auto out32_tag, auto out16_tag) {
+        constexpr bool RES = decltype(residual_tag)::value, OUT32 = decltype(out32_tag)::value, OUT16 = decltype(out16_tag)::value;
 #pragma unroll
-    for (int tm = 0; tm < TM; ++tm) {
-        const int row_base = row_first + tm * 32;
+        for (int tm = 0; tm < TM; ++tm) {
+            const int row_base = row_first + tm * 32;
 #pragma unroll
-        for (int tn = 0; tn < TN; ++tn) {
-            const f32x16 tile = acc[tm][tn];
+            for (int tn = 0; tn < TN; ++tn) {
+                const f32x16 tile = acc[tm][tn];
 #pragma unroll
-            for (int g = 0; g < 4; ++g)
-                *reinterpret_cast<float4 *>(&strip[li * C_STRIDE + tn * 32 + g * 8 + lh * 4]) =
-                    make_float4(tile[4 * g], tile[4 * g + 1], tile[4 * g + 2], tile[4 * g + 3]);
-        }
+                for (int g = 0; g < 4; ++g)
+                    *reinterpret_cast<float4 *>(&strip[li * C_STRIDE + tn * 32 + g * 8 + lh * 4]) =
+                        make_float4(tile[4 * g], tile[4 * g + 1], tile[4 * g + 2], tile[4 * g + 3]);
+            }
 #pragma unroll
-        for (int j = 0; j < PASSES; ++j) {
-            const int local_row = j * ROWS_PER_PASS + lane / LPR;
-            const int row = row_base + local_row;
-            const float4 s4 = *reinterpret_cast<const float4 *>(&strip[local_row * C_STRIDE + (lane & (LPR - 1)) * 4]);
-            if (row >= M || col0 >= N) continue;
-            const size_t idx = static_cast<size_t>(row) * N + col0;
-            float v[4] = {s4.x, s4.y, s4.z, s4.w};
-            float res[4] = {0.f, 0.f, 0.f, 0.f};
-            if (p.residual) {
+            for (int j = 0; j < PASSES; ++j) {
+                const int local_row = j * ROWS_PER_PASS + lane / LPR;
+                const int row = row_base + local_row;
+                const float4 s4 = *reinterpret_cast<const float4 *>(&strip[local_row * C_STRIDE + (lane & (LPR - 1)) * 4]);
+                if (row >= M || col0 >= N) continue;
+                const size_t idx = static_cast<size_t>(row) * N + col0;
+                float v[4] = {s4.x * scale + bias[0], s4.y * scale + bias[1], s4.z * scale + bias[2], s4.w * scale + bias[3]};
                 if (whole) {
-                    const f32x4_a4 r4 = *reinterpret_cast<const f32x4_a4 *>(p.residual + idx);
-                    res[0] = r4[0]; res[1] = r4[1]; res[2] = r4[2]; res[3] = r4[3];
+                    if constexpr (RES) {
+                        const f32x4_a4 r4 = *reinterpret_cast<const f32x4_a4 *>(p.residual + idx);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) v[e] += r4[e];
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = act(v[e]);
+                    if constexpr (OUT32) *reinterpret_cast<f32x4_a4 *>(p.C32 + idx) = f32x4_a4{v[0], v[1], v[2], v[3]};
+                    if constexpr (OUT16) *reinterpret_cast<u32x2_a2 *>(p.C16 + idx) = u32x2_a2{pack_bf16x2_rne(v[0], v[1]), pack_bf16x2_rne(v[2], v[3])};
                 } else {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (col0 + e < N) res[e] = p.residual[idx + e];
-                }
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                float value = v[e] * scale + bias[e];
-                if (p.residual) value += res[e];
-                v[e] = apply_activation(value, p.activation);
-            }
-            if (whole) {
-                if (p.C32) *reinterpret_cast<f32x4_a4 *>(p.C32 + idx) = f32x4_a4{v[0], v[1], v[2], v[3]};
-                if (p.C16) *reinterpret_cast<u32x2_a2 *>(p.C16 + idx) = u32x2_a2{pack_bf16x2_rne(v[0], v[1]), pack_bf16x2_rne(v[2], v[3])};
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    if (col0 + e >= N) continue;
-                    if (p.C32) p.C32[idx + e] = v[e];
-                    if (p.C16) p.C16[idx + e] = f32_to_bf16_rne(v[e]);
+                    for (int e = 0; e < 3; ++e) {
+                        if (col0 + e >= N) continue;
+                        if constexpr (RES) v[e] += p.residual[idx + e];
+                        v[e] = act(v[e]);
+                        if constexpr (OUT32) p.C32[idx + e] = v[e];
+                        if constexpr (OUT16) p.C16[idx + e] = f32_to_bf16_rne(v[e]);
+                    }
                 }
             }
         }
-    }
+    };
+    with_epilogue_ops(p.activation, p.residual != nullptr, [&](auto &&act, auto has_residual) {
+        if (p.C32 && p.C16) run(act, has_residual, std::true_type{}, std::true_type{});
+        else if (p.C32) run(act, has_residual, std::true_type{}, std::false_type{});
+        else run(act, has_residual, std::false_type{}, std::true_type{});
+    });
 }
 
 template <int WTN, int TM = 2>
@@ -2146,7 +2148,7 @@ double tiles_128_us(size_t m, size_t n, size_t k)
 }
 
 // Which of the small tiles of gemm_bf16_small.hip takes an m×n×k product (operands on 16-byte boundaries), -1 for none, by the
-// estimated time of the kernels here: both tilings, k split or not, with the epilogue of a ragged n (4.5 µs); the general kernel where
+// estimated time of the kernels here: both tilings, k split or not, with the epilogue of a ragged n (2.3 µs); the general kernel where
 // those do not take the shape.
 int small_tile(size_t m, size_t n, size_t k)
 {
@@ -2157,7 +2159,7 @@ int small_tile(size_t m, size_t n, size_t k)
     if (small.pays(std::min(3.6 + 0.41 * k_tiles, 6.9))) return small.tile;  // (less than what the tilings below take unsplit, and split)
     const size_t tiles_256 = (m + 255) / 256 * ((n + 127) / 128);
     const double us = std::min(tiles_128_us(m, n, k), 4.0 + static_cast<double>((tiles_256 + 255) / 256) * estimate_k_splits(m, n, k, tiles_256, 256, 0.5).cost_us);
-    return small.pays(us + (n % 128 != 0 ? 4.5 : 0.0)) ? small.tile : -1;
+    return small.pays(us + (n % 128 != 0 ? 2.3 : 0.0)) ? small.tile : -1;
 }
 
 // The launch arithmetic of the tiled kernels whose workgroups decode their index into (k-split, tile), checked on the

@@ -24,6 +24,8 @@ namespace {
 
 typedef float f32x4_acc __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void *lds_void_ptr;
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
 typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 
@@ -39,7 +41,6 @@ struct SmallArgs {
     int ring_bytes;  // LDS of a wavefront: its one or two stages, later its sums
     float scale;
     int activation;
-    int vector_stores;  // rows of C32, C16 and residual start at multiples of four values and the pointers are aligned for them
 };
 
 // Where 16-byte chunk q of row r stands in a 128-byte LDS row: the sixteen rows of a fragment read spread over all banks.
@@ -197,22 +198,24 @@ __device__ __forceinline__ void gemm_bf16_small_body(const SmallArgs &p)
                 v.x += q.x; v.y += q.y; v.z += q.z; v.w += q.w;
             }
             float value[4] = {v.x * p.scale, v.y * p.scale, v.z * p.scale, v.w * p.scale};
-            if (p.vector_stores) {
+            if (col + 4 <= N) {  // (16-byte accesses at whatever boundary the rows have)
                 if (p.bias) {
-                    const float4 b = *reinterpret_cast<const float4 *>(p.bias + col);
-                    value[0] += b.x; value[1] += b.y; value[2] += b.z; value[3] += b.w;
+                    const f32x4_a4 b = *reinterpret_cast<const f32x4_a4 *>(p.bias + col);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) value[i] += b[i];
                 }
                 if constexpr (decltype(has_residual)::value) {
-                    const float4 r = *reinterpret_cast<const float4 *>(p.residual + idx);
-                    value[0] += r.x; value[1] += r.y; value[2] += r.z; value[3] += r.w;
+                    const f32x4_a4 r = *reinterpret_cast<const f32x4_a4 *>(p.residual + idx);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) value[i] += r[i];
                 }
 #pragma unroll
                 for (int i = 0; i < 4; ++i) value[i] = act(value[i]);
-                if (p.C32) *reinterpret_cast<float4 *>(p.C32 + idx) = make_float4(value[0], value[1], value[2], value[3]);
-                if (p.C16) *reinterpret_cast<uint2 *>(p.C16 + idx) = make_uint2(pack_bf16x2_rne(value[0], value[1]), pack_bf16x2_rne(value[2], value[3]));
+                if (p.C32) *reinterpret_cast<f32x4_a4 *>(p.C32 + idx) = f32x4_a4{value[0], value[1], value[2], value[3]};
+                if (p.C16) *reinterpret_cast<u32x2_a2 *>(p.C16 + idx) = u32x2_a2{pack_bf16x2_rne(value[0], value[1]), pack_bf16x2_rne(value[2], value[3])};
             } else {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
+                for (int i = 0; i < 3; ++i) {
                     if (col + i >= N) continue;
                     if (p.bias) value[i] += p.bias[col + i];
                     if constexpr (decltype(has_residual)::value) value[i] += p.residual[idx + i];
@@ -296,7 +299,6 @@ hipError_t launch_gemm_bf16_small(int tile, size_t m, size_t n, size_t k, const 
                                   uint16_t *out_bf16, const GemmEpilogue &epilogue, hipStream_t stream)
 {
     const SmallConfig &config = kSmallConfigs[tile];
-    auto aligned = [](const void *ptr, uintptr_t bytes) { return (reinterpret_cast<uintptr_t>(ptr) & (bytes - 1)) == 0; };
     SmallArgs args;
     args.A = lhs;
     args.B = rhs;
@@ -310,7 +312,6 @@ hipError_t launch_gemm_bf16_small(int tile, size_t m, size_t n, size_t k, const 
     args.tiles_m = static_cast<int>((m + config.bm - 1) / config.bm);
     args.scale = epilogue.scale;
     args.activation = epilogue.activation;
-    args.vector_stores = n % 4 == 0 && aligned(out_f32, 16) && aligned(out_bf16, 8) && aligned(epilogue.bias, 16) && aligned(epilogue.residual, 16);
     args.ring_bytes = static_cast<int>(config.ring_bytes(k));
     const size_t lds = config.waves * config.ring_bytes(k), tiles = config.tiles(m, n);
     if (tiles > 0x7fffffffu || lds > 160 * 1024) return hipErrorInvalidConfiguration;
