@@ -2035,45 +2035,59 @@ hipError_t launch_skinny_packed(const GemmBf16Args &args, hipStream_t stream)
 
 // out(cols×rows) = in(rows×cols)ᵀ for 16-bit elements, 64×64 tiles through LDS, 128-bit global accesses when the
 // shape allows (PackedB::from_row_major, crates/st-tensor/src/pure.rs:1299-1316, for bf16 storage).
-__global__ __launch_bounds__(256) void transpose_u16_kernel(int rows, int cols, int vec, const uint16_t *in, uint16_t *out)
+struct TransposeJob {
+    const uint16_t *in;  // rows × cols
+    uint16_t *out;       // cols × pitch, columns rows .. pitch - 1 zeros
+    unsigned rows, cols, pitch, col_blocks;
+};
+// Reads and writes of 16 bytes at any 2-byte boundary, element by element only at the ends of rows.
+__device__ __forceinline__ void transpose_u16_tile(const TransposeJob &job, unsigned block)
 {
-    __shared__ uint16_t tile[64][66];
+    typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+    __shared__ __attribute__((aligned(16))) uint16_t tile[64][66];
     const int t = threadIdx.x;
-    const int c0 = blockIdx.x * 64, r0 = blockIdx.y * 64;
+    const unsigned c0 = block % job.col_blocks * 64, r0 = block / job.col_blocks * 64;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        const int r = (t >> 3) + 32 * i, c8 = (t & 7) * 8;
-        uint16_t e[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        if (r0 + r < rows) {
-            const uint16_t *src = in + static_cast<size_t>(r0 + r) * cols + c0 + c8;
-            if (vec && c0 + c8 + 8 <= cols) {
-                *reinterpret_cast<uint4 *>(e) = *reinterpret_cast<const uint4 *>(src);
+        const unsigned r = (t >> 3) + 32 * i, c8 = (t & 7) * 8;
+        u32x4_a2 e = {0, 0, 0, 0};
+        if (r0 + r < job.rows) {
+            const uint16_t *src = job.in + static_cast<size_t>(r0 + r) * job.cols + c0 + c8;
+            if (c0 + c8 + 8 <= job.cols) {
+                e = *reinterpret_cast<const u32x4_a2 *>(src);
             } else {
 #pragma unroll
                 for (int j = 0; j < 8; ++j)
-                    if (c0 + c8 + j < cols) e[j] = src[j];
+                    if (c0 + c8 + j < job.cols) e[j >> 1] |= static_cast<uint32_t>(src[j]) << (16 * (j & 1));
             }
         }
 #pragma unroll
-        for (int j = 0; j < 8; ++j) tile[r][c8 + j] = e[j];
+        for (int j = 0; j < 4; ++j) *reinterpret_cast<uint32_t *>(&tile[r][c8 + 2 * j]) = e[j];
     }
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        const int c = (t >> 3) + 32 * i, r8 = (t & 7) * 8;
-        if (c0 + c >= cols) continue;
-        uint16_t e[8];
+        const unsigned c = (t >> 3) + 32 * i, r8 = (t & 7) * 8;
+        if (c0 + c >= job.cols) continue;
+        uint32_t e[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) e[j] = tile[r8 + j][c];
-        uint16_t *dst = out + static_cast<size_t>(c0 + c) * rows + r0 + r8;
-        if (vec && r0 + r8 + 8 <= rows) {
-            *reinterpret_cast<uint4 *>(dst) = *reinterpret_cast<const uint4 *>(e);
+        uint16_t *dst = job.out + static_cast<size_t>(c0 + c) * job.pitch + r0 + r8;
+        if (r0 + r8 + 8 <= job.pitch) {
+            *reinterpret_cast<u32x4_a2 *>(dst) = u32x4_a2{e[0] | e[1] << 16, e[2] | e[3] << 16, e[4] | e[5] << 16, e[6] | e[7] << 16};
         } else {
 #pragma unroll
             for (int j = 0; j < 8; ++j)
-                if (r0 + r8 + j < rows) dst[j] = e[j];
+                if (r0 + r8 + j < job.pitch) dst[j] = static_cast<uint16_t>(e[j]);
         }
     }
+}
+__global__ __launch_bounds__(256) void transpose_u16_kernel(TransposeJob job) { transpose_u16_tile(job, blockIdx.x); }
+
+unsigned transpose_blocks(TransposeJob &job)
+{
+    job.col_blocks = (job.cols + 63) / 64;
+    return job.col_blocks * ((job.pitch + 63) / 64);
 }
 
 // Few tiles and a long k (a batch of a hundred rows against a 4096² weight is 32 tiles of 64 k-tiles each): split k
@@ -2442,13 +2456,11 @@ struct PadJob {
     unsigned rows, cols, rows_pad, cols_pad;
 };
 
-__global__ __launch_bounds__(256) void pad_u16_pair_kernel(PadJob first, PadJob second, unsigned first_blocks)
+__device__ __forceinline__ void pad_u16_piece(const PadJob &job, unsigned block)
 {
     typedef uint32_t pad_u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
-    const bool is_first = blockIdx.x < first_blocks;
-    const PadJob &job = is_first ? first : second;
     const unsigned chunks = (job.cols_pad + 7) / 8;
-    const unsigned idx = (blockIdx.x - (is_first ? 0u : first_blocks)) * 256u + threadIdx.x;  // below 2^28: the copies are below 2 GiB
+    const unsigned idx = block * 256u + threadIdx.x;  // below 2^28: the copies are below 2 GiB
     const unsigned r = idx / chunks;
     const unsigned c0 = (idx - r * chunks) * 8;
     if (r >= job.rows_pad) return;
@@ -2464,6 +2476,17 @@ __global__ __launch_bounds__(256) void pad_u16_pair_kernel(PadJob first, PadJob 
         if (c < job.cols_pad) dst[e] = (r < job.rows && c < job.cols) ? src[e] : static_cast<uint16_t>(0);
     }
 }
+// A and a packed B padded along k, or A padded and a row-major B packed and padded: one launch.
+__global__ __launch_bounds__(256) void pad_u16_pair_kernel(PadJob first, PadJob second, unsigned first_blocks)
+{
+    if (blockIdx.x < first_blocks) pad_u16_piece(first, blockIdx.x);
+    else pad_u16_piece(second, blockIdx.x - first_blocks);
+}
+__global__ __launch_bounds__(256) void pad_and_pack_u16_kernel(PadJob first, TransposeJob second, unsigned first_blocks)
+{
+    if (blockIdx.x < first_blocks) pad_u16_piece(first, blockIdx.x);
+    else transpose_u16_tile(second, blockIdx.x - first_blocks);
+}
 
 PadJob pad_job(size_t rows, size_t cols, size_t rows_pad, size_t cols_pad, const uint16_t *in, uint16_t *out)
 {
@@ -2471,14 +2494,22 @@ PadJob pad_job(size_t rows, size_t cols, size_t rows_pad, size_t cols_pad, const
                   static_cast<unsigned>(cols_pad)};
 }
 
-hipError_t launch_pad_u16_pair(const PadJob &first, const PadJob &second, hipStream_t stream)
+unsigned pad_blocks(const PadJob &job) { return static_cast<unsigned>((static_cast<size_t>(job.rows_pad) * ((job.cols_pad + 7) / 8) + 255) / 256); }
+
+// a_pad (m × k_pad) and b_pad (n × k_pad) from A and B as k×n or n×k.
+hipError_t launch_pad_operands(size_t m, size_t n, size_t k, size_t k_pad, const uint16_t *lhs, const uint16_t *rhs, bool rhs_packed,
+                               uint16_t *a_pad, uint16_t *b_pad, hipStream_t stream)
 {
-    auto blocks = [](const PadJob &job) {
-        return static_cast<unsigned>((static_cast<size_t>(job.rows_pad) * ((job.cols_pad + 7) / 8) + 255) / 256);
-    };
-    const unsigned first_blocks = blocks(first), all = first_blocks + blocks(second);
-    if (all == 0) return hipSuccess;
-    hipLaunchKernelGGL(pad_u16_pair_kernel, dim3(all), dim3(256), 0, stream, first, second, first_blocks);
+    const PadJob a = pad_job(m, k, m, k_pad, lhs, a_pad);
+    const unsigned first = pad_blocks(a);
+    if (rhs_packed) {
+        const PadJob b = pad_job(n, k, n, k_pad, rhs, b_pad);
+        hipLaunchKernelGGL(pad_u16_pair_kernel, dim3(first + pad_blocks(b)), dim3(256), 0, stream, a, b, first);
+    } else {
+        TransposeJob b{rhs, b_pad, static_cast<unsigned>(k), static_cast<unsigned>(n), static_cast<unsigned>(k_pad), 0};
+        const unsigned second = transpose_blocks(b);
+        hipLaunchKernelGGL(pad_and_pack_u16_kernel, dim3(first + second), dim3(256), 0, stream, a, b, first);
+    }
     return hipGetLastError();
 }
 
@@ -2487,11 +2518,24 @@ hipError_t launch_pad_u16_pair(const PadJob &first, const PadJob &second, hipStr
 hipError_t launch_transpose_u16(size_t rows, size_t cols, const uint16_t *in, uint16_t *out, hipStream_t stream)
 {
     if (rows == 0 || cols == 0) return hipSuccess;
-    const int vec = rows % 8 == 0 && cols % 8 == 0 && aligned16(in) && aligned16(out) ? 1 : 0;
-    const dim3 grid(static_cast<unsigned>((cols + 63) / 64), static_cast<unsigned>((rows + 63) / 64));
-    hipLaunchKernelGGL(transpose_u16_kernel, grid, dim3(256), 0, stream, static_cast<int>(rows), static_cast<int>(cols), vec,
-                       in, out);
+    TransposeJob job{in, out, static_cast<unsigned>(rows), static_cast<unsigned>(cols), static_cast<unsigned>(rows), 0};
+    const size_t blocks = (cols + 63) / 64 * ((rows + 63) / 64);
+    if (blocks > 0x7fffffffu) return hipErrorInvalidConfiguration;
+    hipLaunchKernelGGL(transpose_u16_kernel, dim3(transpose_blocks(job)), dim3(256), 0, stream, job);
     return hipGetLastError();
+}
+
+// Whether a product with a k that is no multiple of 64 runs on zero-padded copies of A and B.  The general kernel takes any k, but walks it
+// in k-tiles of 32 with one 128×128 tile a workgroup: of 200 products drawn from 1 to 4096 rows, 32 to 8192 columns and k from 70 to 8192
+// (up to 60 GFLOP, B of up to 50 million values) the copies, their pass included, take 0.31 of its time with B packed and 0.40 with B
+// row-major, none more (448×383×2566 56 -> 12 µs, 16×663×329 16 -> 6.1).  It stays where a pass over B is most of the work: a row-major B
+// of more than 14 million values or 16384 columns for up to 64 rows (16×8192×8190 39 / 68 µs general / copies, 1×8191×8191 65 / 82,
+// 4×50257×100 11 / 26; at 16×4096×4097 they are level), and k beyond 16384, which it cuts over the chip (33×100×50257 34 / 59, packed 49 / 59).
+static bool padding_pays(size_t m, size_t n, size_t k, bool rhs_packed)
+{
+    if (k <= 64) return false;
+    if (m >= 128 && n >= 128 && 2.0 * m * n * k >= 2e9) return true;
+    return k <= 16384 && (rhs_packed || m > 64 || (n <= 16384 && n * k <= 14'000'000));
 }
 
 hipError_t launch_gemm_bf16(size_t m, size_t n, size_t k, const uint16_t *lhs, const uint16_t *rhs,
@@ -2515,23 +2559,22 @@ hipError_t launch_gemm_bf16(size_t m, size_t n, size_t k, const uint16_t *lhs, c
         }
         return hipSuccess;
     }
-    // A k that is not a multiple of 64 (784 inputs, 1000 features): the direct-to-LDS kernels take whole 64-wide k-tiles
-    // only, and the general kernel runs such a product at half their speed (8192×4096×1000: 141 µs against 65 µs at
-    // k = 1024).  Where the product is large against its operands, zero-padded copies of A and B along k (exact: the
-    // new terms are 0·0) go into the stream's second scratch buffer, one launch for both, and the product runs on them.
-    if (k % 64 != 0 && k > 64 && m >= 128 && n >= 128 && 2.0 * m * n * k >= 2e9 && m * (k + 64) * sizeof(uint16_t) < (1ull << 31) &&
-        (k + 64) * n * sizeof(uint16_t) < (1ull << 31)) {
+    // A k that is not a multiple of 64 (784 inputs, 1000 features): the direct-to-LDS kernels take whole 64-wide k-tiles only.  Copies of
+    // A and B padded with zeros along k (exact: the new terms are 0·0), B as n×k, go into the stream's second scratch buffer, one launch for
+    // both, and the product runs on them.
+    if (k % 64 != 0 && padding_pays(m, n, k, rhs_packed) && m * (k + 64) * sizeof(uint16_t) < (1ull << 31) && (k + 64) * n * sizeof(uint16_t) < (1ull << 31)) {
         const size_t k_pad = (k + 63) / 64 * 64;
         const size_t a_bytes = (m * k_pad * sizeof(uint16_t) + 255) & ~static_cast<size_t>(255);
         void *copies = nullptr;
         hipError_t rc = stream_workspace_slot(stream, 1, a_bytes + k_pad * n * sizeof(uint16_t), &copies);
-        if (rc != hipSuccess) return rc;
-        uint16_t *a_pad = static_cast<uint16_t *>(copies);
-        uint16_t *b_pad = reinterpret_cast<uint16_t *>(static_cast<unsigned char *>(copies) + a_bytes);
-        rc = launch_pad_u16_pair(pad_job(m, k, m, k_pad, lhs, a_pad),
-                                 rhs_packed ? pad_job(n, k, n, k_pad, rhs, b_pad) : pad_job(k, n, k_pad, n, rhs, b_pad), stream);
-        if (rc != hipSuccess) return rc;
-        return launch_gemm_bf16(m, n, k_pad, a_pad, b_pad, out_f32, out_bf16, epilogue, stream, rhs_packed);
+        if (rc == hipSuccess) {
+            uint16_t *a_pad = static_cast<uint16_t *>(copies);
+            uint16_t *b_pad = reinterpret_cast<uint16_t *>(static_cast<unsigned char *>(copies) + a_bytes);
+            rc = launch_pad_operands(m, n, k, k_pad, lhs, rhs, rhs_packed, a_pad, b_pad, stream);
+            if (rc != hipSuccess) return rc;
+            return launch_gemm_bf16(m, n, k_pad, a_pad, b_pad, out_f32, out_bf16, epilogue, stream, true);
+        }
+        if (!scratch_unavailable(rc)) return rc;  // else the kernels below, of which the general one takes any k
     }
     GemmBf16Args args;
     args.A = lhs;

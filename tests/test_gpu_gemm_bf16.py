@@ -378,6 +378,24 @@ def test_k_that_is_not_a_multiple_of_64(hip, oracle, m, n, k):
         assert (d16.to_array(np.uint16, m * n) == inputs.to_bf16(got32)).all()
 
 
+# few rows, few columns, the first k that is padded and one past a k-tile, transposed blocks of 64 cut short both ways, odd everything
+@pytest.mark.parametrize("m,n,k", [(1, 40, 65), (16, 663, 329), (3, 8, 1001), (33, 257, 70), (64, 100, 129), (70, 33, 4097), (65, 64, 127), (200, 1000, 72),
+                                   (448, 383, 2566), (129, 65, 16383)])
+def test_small_products_of_any_k(hip, oracle, m, n, k):
+    test_k_that_is_not_a_multiple_of_64(hip, oracle, m, n, k)
+
+
+# B packed by the transposing kernel at any size
+@pytest.mark.parametrize("rows,cols", [(1, 1), (63, 65), (64, 64), (65, 63), (7, 200), (200, 7), (129, 1001), (1000, 72)])
+def test_packing_any_size(hip, rows, cols):
+    b = np.random.default_rng(rows + cols).integers(0, 65536, rows * cols).astype(np.uint16)
+    d_b, d_out = hip.DeviceBuffer.from_array(b), hip.DeviceBuffer.from_array(np.full(rows * cols + 64, 7, np.uint16))
+    hip.pack_rhs_bf16_dev(rows, cols, d_b, d_out)
+    hip.device_synchronize()
+    got = d_out.to_array(np.uint16, rows * cols + 64)
+    assert (got[:rows * cols].reshape(cols, rows) == b.reshape(rows, cols).T).all() and (got[rows * cols:] == 7).all()
+
+
 @pytest.mark.parametrize("m,n,k", [(1024, 1024, 1024), (300, 1024, 512), (130, 2048, 256), (1000, 1280, 192), (2048, 2048, 64),
                                    (513, 384, 448)])
 def test_mid_size_128_row_tiles(hip, oracle, m, n, k):

@@ -44,6 +44,25 @@ for fail in (1, 0):
     assert out == ["1", "2"]
 
 
+# around the bounds on what is copied for up to 64 rows, and on k
+@pytest.mark.parametrize("m,n,k,launched", [(16, 663, 329, 2), (100, 1001, 300, 2), (64, 16384, 850, 2), (64, 16392, 65, 1), (64, 16384, 855, 1), (65, 40, 16383, 2),
+                                            (3000, 40, 16385, 1), (20, 40, 63, 1)])
+def test_products_of_any_k_go_on_without_room_for_padded_copies(stub, m, n, k, launched):
+    """A k that is no multiple of 64 is padded in scratch memory where that pays; without any to be had, the general kernel takes it as it
+    is (a k it would cut over the chip needs scratch there too, as ever)."""
+    out = run(stub, f"""
+for fail in (1, 0) if {k} < 1024 else (0,):
+    no_memory.value, before = fail, launches.value
+    hip.gemm_bf16_bias_act_dev({m}, {n}, {k}, 0, 1 << 20, 2 << 20, None, None, 1 << 40, None)
+    print(launches.value - before)
+""")
+    counts = [int(c) for c in out]
+    if k < 1024:
+        assert counts == [1, launched]
+    else:  # padded: the pass and a product; not: slices of k and their sum
+        assert counts[0] >= 2
+
+
 @pytest.mark.parametrize("rows", [1, 64, 300])  # one value, and either side of the 256 KiB from which the pointer was looked at
 def test_operands_in_device_memory_are_left_to_the_runtime(stub, rows):
     """A host call whose operand lies in device or managed memory (here: pages nobody may read) copies it with the runtime's copy."""
