@@ -935,22 +935,29 @@ __global__ __launch_bounds__(256) void conv2d_f32_direct_kernel(ConvArgs p)
 
 // The same for unit stride and dilation along x and a kernel width known at compile time: a thread owns four adjacent
 // pixels of an output row, so that a row segment of KW + 3 input values (one 16-byte load at any alignment plus KW - 1
-// single ones) feeds 4·KW·CO multiply-adds, and the weights (at most 64 KB) are read from LDS, every lane the same word.
+// single ones) feeds 4·KW·CO multiply-adds, and the weights (at most 144 KB) are read from LDS, every lane the same word.
 // KH: the kernel height when it equals KW and is at most 5 (the loop over its rows is then unrolled, so that the loads of all rows of
 // a channel are in flight together: a thread's chain of load → multiply-add steps is what bounds this kernel), else 0.
-template <int CO, int KW, int KH>
-__global__ __launch_bounds__(256) void conv2d_f32_direct_rows_kernel(ConvArgs p)
+// GROUPS: wavefronts that share the input channels of 64 threads' worth of pixels and add their sums through LDS in a fixed order (the
+// wavefronts of a workgroup), 1: each of four wavefronts takes all channels of its own pixels.
+// All channels / shared by four, 3×3, images × channels, side -> channels: 17×512, 66×67 -> 3 700 / 195 µs, 32×256, 50 -> 3 355 / 100,
+// 32×64, 64 -> 3 78 / 28, 6×64, 112 -> 3 75 / 28, 32×512, 46 -> 1 493 / 120 (16 wavefronts a workgroup, each with one of sixteen
+// groups: 340, 185, 66, 60, 136).
+template <int CO, int KW, int KH, int GROUPS>
+__global__ __launch_bounds__(GROUPS == 1 ? 256 : 64 * GROUPS) void conv2d_f32_direct_rows_kernel(ConvArgs p)
 {
+    constexpr int THREADS = GROUPS == 1 ? 256 : 64 * GROUPS, ITEMS = GROUPS == 1 ? 256 : 64;
     typedef float direct_f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
-    extern __shared__ float direct_weights[];  // CO × K, as stored
+    extern __shared__ float direct_weights[];  // CO × K, as stored; the groups' sums behind them
     const ConvShape &s = p.s;
     const int K = p.K;
-    for (int i = static_cast<int>(threadIdx.x); i < CO * K; i += 256) direct_weights[i] = p.weight[i];
+    for (int i = static_cast<int>(threadIdx.x); i < CO * K; i += THREADS) direct_weights[i] = p.weight[i];
     __syncthreads();
     const int quads = (s.ow + 3) / 4;  // threads per output row
-    const int item = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
-    if (item >= s.oh * quads) return;
-    const int oy = item / quads, ox0 = (item - oy * quads) * 4;
+    const int item = static_cast<int>(blockIdx.x) * ITEMS + static_cast<int>(threadIdx.x) % ITEMS;
+    const bool live = item < s.oh * quads;
+    if (GROUPS == 1 && !live) return;
+    const int oy = live ? item / quads : 0, ox0 = live ? (item - oy * quads) * 4 : 0;
     const int image = static_cast<int>(blockIdx.y);
     const int iy0 = oy * s.stride_h - s.pad_h, ix0 = ox0 - s.pad_w;
     constexpr int SEG = KW + 3;
@@ -964,7 +971,7 @@ __global__ __launch_bounds__(256) void conv2d_f32_direct_rows_kernel(ConvArgs p)
         for (int j = 0; j < 4; ++j) acc[co][j] = 0.0f;
     const int kh = KH > 0 ? KH : s.kh;
 #pragma unroll 2
-    for (int ci = 0; ci < s.c_in; ++ci) {
+    for (int ci = GROUPS == 1 ? 0 : static_cast<int>(threadIdx.x) / ITEMS; ci < s.c_in; ci += GROUPS) {
         const float *plane = in + static_cast<size_t>(ci) * plane_elems;
 #pragma unroll
         for (int ky = 0; ky < kh; ++ky) {
@@ -997,6 +1004,25 @@ __global__ __launch_bounds__(256) void conv2d_f32_direct_rows_kernel(ConvArgs p)
                 }
         }
     }
+    if constexpr (GROUPS > 1) {
+        float *const sums = direct_weights + CO * K;  // [group][result][64]
+        const int group = static_cast<int>(threadIdx.x) / ITEMS, lane = static_cast<int>(threadIdx.x) % ITEMS;
+#pragma unroll
+        for (int co = 0; co < CO; ++co)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) sums[(group * CO * 4 + co * 4 + j) * 64 + lane] = acc[co][j];
+        __syncthreads();
+        for (int result = group; result < CO * 4; result += GROUPS) {
+            const int co = result / 4, j = result % 4;
+            if (!live || ox0 + j >= s.ow) continue;
+            float total = 0.0f;
+#pragma unroll
+            for (int g = 0; g < GROUPS; ++g) total += sums[(g * CO * 4 + result) * 64 + lane];
+            p.out[(static_cast<size_t>(image) * CO + co) * p.spatial + static_cast<size_t>(oy) * s.ow + ox0 + j] =
+                apply_activation(total + (p.bias ? p.bias[co] : -0.0f), p.activation);
+        }
+        return;
+    }
 #pragma unroll
     for (int co = 0; co < CO; ++co) {
         const float b = p.bias ? p.bias[co] : -0.0f;
@@ -1007,15 +1033,33 @@ __global__ __launch_bounds__(256) void conv2d_f32_direct_rows_kernel(ConvArgs p)
     }
 }
 
+constexpr size_t kDirectWeightBytes = 144 * 1024;  // the LDS, less the groups' sums (4 · 16 · 64 floats)
+
+template <int CO, int KW, int KH, int GROUPS>
+hipError_t launch_direct_groups(const ConvArgs &args, hipStream_t stream)
+{
+    constexpr size_t kItems = GROUPS == 1 ? 256 : 64;
+    const size_t items = static_cast<size_t>(args.s.oh) * ((args.s.ow + 3) / 4);
+    const dim3 grid(static_cast<unsigned>((items + kItems - 1) / kItems), static_cast<unsigned>(args.s.batch));
+    const size_t lds_bytes = (static_cast<size_t>(CO) * args.K + (GROUPS == 1 ? 0 : GROUPS * CO * 4 * 64)) * sizeof(float);
+    auto kernel = conv2d_f32_direct_rows_kernel<CO, KW, KH, GROUPS>;
+    if (lds_bytes > 64 * 1024) {  // more than a launch may take unasked
+        const hipError_t rc = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        if (rc != hipSuccess) return rc;
+    }
+    hipLaunchKernelGGL(kernel, grid, dim3(GROUPS == 1 ? 256 : 64 * GROUPS), lds_bytes, stream, args);
+    return hipGetLastError();
+}
+
 template <int CO, int KW>
 hipError_t launch_direct_rows(const ConvArgs &args, hipStream_t stream)
 {
-    const size_t items = static_cast<size_t>(args.s.oh) * ((args.s.ow + 3) / 4);
-    const dim3 grid(static_cast<unsigned>((items + 255) / 256), static_cast<unsigned>(args.s.batch));
-    const size_t lds_bytes = static_cast<size_t>(CO) * args.K * sizeof(float);
-    if (args.s.kh == KW && KW <= 5) hipLaunchKernelGGL((conv2d_f32_direct_rows_kernel<CO, KW, KW>), grid, dim3(256), lds_bytes, stream, args);
-    else hipLaunchKernelGGL((conv2d_f32_direct_rows_kernel<CO, KW, 0>), grid, dim3(256), lds_bytes, stream, args);
-    return hipGetLastError();
+    const size_t workgroups = (static_cast<size_t>(args.s.oh) * ((args.s.ow + 3) / 4) + 255) / 256 * args.s.batch;
+    // (Whole / shared are level once whole ones give the chip two workgroups a unit, 8×64, 256×256, 3×3 104 / 107, later where a channel is
+    // more work, the same with 7×7 taps 460 / 393; of 32 channels there is too little to share: 16×32, 128×128, 5×5 79 / 86.)
+    const bool shared = (args.s.c_in >= 48 || args.s.c_in * args.s.kh > 160) && workgroups < (KW > 3 ? 2048 : 512);
+    if (args.s.kh == KW && KW <= 5) return shared ? launch_direct_groups<CO, KW, KW, 4>(args, stream) : launch_direct_groups<CO, KW, KW, 1>(args, stream);
+    return shared ? launch_direct_groups<CO, KW, 0, 4>(args, stream) : launch_direct_groups<CO, KW, 0, 1>(args, stream);
 }
 
 template <int CO>
@@ -1034,7 +1078,7 @@ hipError_t launch_direct(const ConvArgs &args, hipStream_t stream)
 {
     const ConvShape &s = args.s;
     if (s.stride_w == 1 && s.dil_w == 1 && (s.kw == 1 || s.kw == 3 || s.kw == 5 || s.kw == 7) &&
-        static_cast<size_t>(CO) * args.K * sizeof(float) <= 64 * 1024)
+        static_cast<size_t>(CO) * args.K * sizeof(float) <= kDirectWeightBytes)
         return launch_direct_rows_for<CO>(args, stream);
     const dim3 grid(static_cast<unsigned>((args.spatial + 255) / 256), static_cast<unsigned>(args.s.batch));
     hipLaunchKernelGGL(conv2d_f32_direct_kernel<CO>, grid, dim3(256), 0, stream, args);

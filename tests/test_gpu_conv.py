@@ -154,6 +154,32 @@ def test_few_output_channels_over_many_pixels(hip, oracle, shape):
     assert float(np.abs(got).max()) > 0.1
 
 
+# channels shared by four wavefronts: as many as they are and not, the first counts that are shared, every width of kernel and number of
+# results, rows of no multiple of four pixels, weights beyond 64 KiB and the last that fit, and (whole channels) just past them
+@pytest.mark.parametrize("shape", [
+    (16, 48, 64, 65, 3, (3, 3), (1, 1), (1, 1), (1, 1)), (16, 49, 64, 67, 1, (3, 3), (1, 1), (1, 1), (1, 1)), (5, 33, 115, 117, 2, (5, 5), (1, 1), (2, 2), (1, 1)),
+    (3, 24, 150, 150, 4, (7, 7), (1, 1), (3, 3), (1, 1)), (4, 50, 130, 127, 2, (2, 1), (1, 1), (1, 0), (1, 1)), (16, 512, 64, 64, 4, (3, 3), (1, 1), (1, 1), (1, 1)),
+    (16, 250, 64, 64, 3, (7, 7), (1, 1), (3, 3), (1, 1)), (16, 251, 64, 64, 3, (7, 7), (1, 1), (3, 3), (1, 1)), (8, 70, 100, 101, 3, (3, 5), (2, 1), (1, 2), (1, 1)),
+])
+def test_few_output_channels_of_many_input_channels(hip, shape):
+    import torch
+    batch, c_in, h, w, c_out, kernel, stride, padding, dilation = shape
+    if batch * np.prod(hip.conv2d_output_hw(h, w, kernel, stride, padding, dilation)) >= 65536:
+        assert hip.conv2d_planned_kernel(*shape) == "direct"
+    rng = np.random.default_rng(c_in + h)
+    x = rng.normal(size=batch * c_in * h * w).astype(np.float32)
+    wt = rng.normal(0, 0.1, c_out * c_in * kernel[0] * kernel[1]).astype(np.float32)
+    b = rng.uniform(-0.5, 0.5, c_out).astype(np.float32)
+    X, W = torch.from_numpy(x).double().view(batch, c_in, h, w), torch.from_numpy(wt).double().view(c_out, c_in, *kernel)
+    exact = torch.nn.functional.conv2d(X, W, torch.from_numpy(b).double(), stride, padding, dilation).numpy().ravel()
+    terms = torch.nn.functional.conv2d(X.abs(), W.abs(), torch.from_numpy(b).double().abs(), stride, padding, dilation).numpy().ravel()
+    bound = 2.0 ** -24 * (c_in * kernel[0] * kernel[1] + 2) * terms  # any order of f32 sums of products
+    got = run(hip, *shape, 0, x, wt, b)
+    assert (np.abs(got - exact) <= bound).all()
+    got = run(hip, *shape, 1, x, wt, b)
+    assert (np.abs(got - np.maximum(exact, 0.0)) <= bound).all()
+
+
 G33 = ((3, 3), (1, 1), (1, 1), (1, 1))
 FAMILY_SHAPES = {
     # name: (batch, c_in, h, w, c_out, kernel, stride, padding, dilation)
