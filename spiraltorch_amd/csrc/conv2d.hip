@@ -538,6 +538,7 @@ struct StripArgs {
     int total;             // workgroups
     int xcd_swizzle;
     int activation;
+    int adjoint = 0;  // `weight` is [c_in][c_out][taps] and its taps run backwards: the forward layer's, whose input gradient this layer is
 };
 
 constexpr int kStripTaps = 9, kStripThreads = 1024;
@@ -572,7 +573,40 @@ __device__ __forceinline__ void conv2d_f32_strip_body(const StripArgs &p)
 
     // Weights of the strip: LDS index of (oc, ic, tap) is (ic*32 + oc)*PITCH + tap, so that a lane's nine taps of a
     // channel are consecutive and the 32 lanes of a half-wavefront sit PITCH words apart (no bank conflicts for 9 or 12).
-    if (K % 4 == 0 && (reinterpret_cast<uintptr_t>(p.weight) & 15u) == 0) {
+    if (p.adjoint) {
+        // The strip's part of a channel is one run of 32 × 9 values at any 4-byte boundary.  (A pass that re-lays the weights is a launch of
+        // its own before this one: 32×64 -> 128, 56×56 143.4 -> 142.1 µs, 32×64 -> 64 78.2 -> 77.0.)
+        typedef float strip_f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+        constexpr int BATCH = 5, PER_CHANNEL = 32 * kStripTaps / 4;
+        const int values = min(32, s.c_out - oc0) * kStripTaps, total = s.c_in * PER_CHANNEL;
+        for (int base = 0; base < total; base += kStripThreads * BATCH) {
+            strip_f32x4_a4 held[BATCH];
+#pragma unroll
+            for (int j = 0; j < BATCH; ++j) {
+                const int v = base + j * kStripThreads + tid, ic = v / PER_CHANNEL, r = (v - ic * PER_CHANNEL) * 4;
+                const float *const src = p.weight + (static_cast<size_t>(ic) * s.c_out + oc0) * kStripTaps + r;
+                held[j] = strip_f32x4_a4{0.0f, 0.0f, 0.0f, 0.0f};
+                if (v >= total) continue;
+                if (r + 4 <= values) {
+                    held[j] = *reinterpret_cast<const strip_f32x4_a4 *>(src);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 3; ++e)
+                        if (r + e < values) held[j][e] = src[e];
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < BATCH; ++j) {
+                const int v = base + j * kStripThreads + tid, ic = v / PER_CHANNEL, r0 = (v - ic * PER_CHANNEL) * 4;
+                if (v >= total) continue;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int r = r0 + e, oc = r / kStripTaps, tap = kStripTaps - 1 - (r - oc * kStripTaps);
+                    lds_w[(ic * 32 + oc) * PITCH + tap] = held[j][e];
+                }
+            }
+        }
+    } else if (K % 4 == 0 && (reinterpret_cast<uintptr_t>(p.weight) & 15u) == 0) {
         constexpr int BATCH = 5;  // 128-bit reads in flight per lane before the first is scattered into LDS
         const int per_row = K >> 2, total = 32 * per_row;
         for (int base = 0; base < total; base += kStripThreads * BATCH) {
@@ -1179,6 +1213,25 @@ size_t conv2d_scratch_bytes(const ConvShape &shape, bool weight_aligned, bool ou
         ST_HIP_CONV_KERNEL_TILE_KSLICED)
         return 0;
     return static_cast<size_t>(conv_k_slices(shape)) * shape.batch * shape.c_out * shape.oh * shape.ow * sizeof(float);
+}
+
+bool launch_conv2d_strip_adjoint(const ConvShape &shape, const float *input, const float *forward_weight, float *out, hipStream_t stream,
+                                 bool allow_slices, hipError_t *rc)
+{
+    if (shape.batch == 0 || shape.c_out == 0 || shape.oh == 0 || shape.ow == 0) return false;
+    StripArgs strip;
+    const bool out_aligned = (reinterpret_cast<uintptr_t>(out) & 15u) == 0;
+    const int kernel = choose_conv_kernel(shape, true, out_aligned, g_forced_family.load(std::memory_order_relaxed), strip, allow_slices);
+    if (kernel != ST_HIP_CONV_KERNEL_STRIP12 && kernel != ST_HIP_CONV_KERNEL_STRIP12_WIDE && kernel != ST_HIP_CONV_KERNEL_STRIP9) return false;
+    strip.input = input;
+    strip.weight = forward_weight;
+    strip.bias = nullptr;
+    strip.out = out;
+    strip.s = shape;
+    strip.activation = ST_HIP_ACT_NONE;
+    strip.adjoint = 1;
+    *rc = launch_strip(strip, kernel, stream);
+    return true;
 }
 
 hipError_t launch_conv2d_f32(const ConvShape &shape, int activation, const float *input, const float *weight,

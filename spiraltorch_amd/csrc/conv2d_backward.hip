@@ -787,6 +787,7 @@ hipError_t launch_conv2d_grad_input_f32(const ConvShape &shape, const float *gra
         }
         return hipSuccess;
     }
+    if (as_forward && launch_conv2d_strip_adjoint(t, grad_output, weight, grad_input, stream, weight_scratch == nullptr, &rc)) return rc;
     float *adjoint_weight = weight_scratch;  // room for weight_count values, owned by the caller
     // The re-laid weights sit at the front of the stream's scratch buffer; a forward launch that cuts its reduction
     // into slices keeps its partial sums behind them (sized here, so the buffer does not move in between).

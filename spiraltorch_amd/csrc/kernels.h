@@ -115,6 +115,10 @@ constexpr int kConvScratchStream = 0, kConvScratchNone = 1;
 hipError_t launch_conv2d_f32(const ConvShape &shape, int activation, const float *input,
                              const float *weight, const float *bias, float *out, hipStream_t stream,
                              int scratch = kConvScratchStream, size_t scratch_offset = 0);
+// grad_input of a layer as the forward layer `shape` (see launch_conv2d_grad_input_f32) where a strip kernel serves that: straight from the
+// layer's own weights, the bits that weights re-laid for launch_conv2d_f32 would give.  False, and nothing launched, elsewhere.
+bool launch_conv2d_strip_adjoint(const ConvShape &shape, const float *input, const float *forward_weight, float *out, hipStream_t stream,
+                                 bool allow_slices, hipError_t *rc);
 // Bytes of the stream's scratch buffer launch_conv2d_f32 uses for `shape` (0 for most shapes).
 size_t conv2d_scratch_bytes(const ConvShape &shape, bool weight_aligned, bool out_aligned);
 
