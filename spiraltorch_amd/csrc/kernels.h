@@ -278,6 +278,16 @@ constexpr size_t kCopyPiece = 16u << 10;
 // `read`: host memory, a word for every kUploadGroup bytes, set (from 0) when the kernel has read them.
 constexpr size_t kUploadGroup = 4096;
 hipError_t launch_copy_from_pinned(void *device, const void *pinned, size_t bytes, hipStream_t stream, unsigned *read = nullptr);
+// Up to kMostCopies of them, none empty, in one launch (which counts their workgroups).
+constexpr int kMostCopies = 8;
+struct PinnedCopies {
+    int count = 0;
+    unsigned groups[kMostCopies];
+    size_t bytes[kMostCopies];
+    const unsigned char *pinned[kMostCopies];
+    unsigned char *device[kMostCopies];
+};
+hipError_t launch_copies_from_pinned(PinnedCopies &copies, hipStream_t stream);
 hipError_t launch_copy_to_pinned(void *pinned, const void *device, size_t bytes, unsigned *arrived, hipStream_t stream);
 // Host<->device copies made by the library, for tests that check where tensors live.
 void count_transfer(bool to_device, size_t bytes);

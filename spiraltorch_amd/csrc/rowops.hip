@@ -837,6 +837,20 @@ __global__ __launch_bounds__(256) void copy_from_pinned_kernel(size_t bytes, con
     if (threadIdx.x == 0) __hip_atomic_store(&read[blockIdx.x], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// Several such copies, a workgroup for every kUploadGroup bytes of each.
+__global__ __launch_bounds__(256) void copy_several_from_pinned_kernel(PinnedCopies copies)
+{
+    unsigned block = blockIdx.x;
+    int i = 0;
+    while (i + 1 < copies.count && block >= copies.groups[i]) block -= copies.groups[i++];
+    const size_t bytes = copies.bytes[i], at = block * kUploadGroup + threadIdx.x * 16;
+    const unsigned char *const pinned = copies.pinned[i];
+    unsigned char *const device = copies.device[i];
+    if (at + 16 <= bytes) *reinterpret_cast<uint4 *>(device + at) = *reinterpret_cast<const uint4 *>(pinned + at);
+    else
+        for (size_t e = at; e < bytes; ++e) device[e] = pinned[e];
+}
+
 // The other way.  The stores go to host memory past the caches (system scope); each wavefront waits for its own to be
 // acknowledged before the workgroup's word says that the piece is there.
 __global__ __launch_bounds__(256) void copy_to_pinned_kernel(size_t bytes, const unsigned char *device, unsigned char *pinned, unsigned *arrived)
@@ -1367,6 +1381,15 @@ hipError_t launch_copy_from_pinned(void *device, const void *pinned, size_t byte
 {
     hipLaunchKernelGGL(copy_from_pinned_kernel, dim3(static_cast<unsigned>((bytes + kUploadGroup - 1) / kUploadGroup)), dim3(256), 0, stream, bytes,
                        static_cast<const unsigned char *>(pinned), static_cast<unsigned char *>(device), read);
+    return hipGetLastError();
+}
+
+hipError_t launch_copies_from_pinned(PinnedCopies &copies, hipStream_t stream)
+{
+    unsigned groups = 0;
+    for (int i = 0; i < copies.count; ++i) groups += copies.groups[i] = static_cast<unsigned>((copies.bytes[i] + kUploadGroup - 1) / kUploadGroup);
+    if (groups == 0) return hipSuccess;
+    hipLaunchKernelGGL(copy_several_from_pinned_kernel, dim3(groups), dim3(256), 0, stream, copies);
     return hipGetLastError();
 }
 

@@ -187,3 +187,16 @@ def test_tensors_from_several_threads_keep_their_values(hip):
     assert wrong == []
     hip.release_scratch()
     assert hip.pinned_memory_counters()[0] == 0
+
+
+# operands that go up together, and one value past what does, first, last and both; parts of 4 KiB cut short
+@pytest.mark.parametrize("m,n", [(1023, 1025), (32767, 3), (32768, 5), (32769, 5), (3, 32768), (5, 32769), (32768, 32), (32769, 33)])
+def test_operands_that_go_up_together(hip, m, n):
+    rng = np.random.default_rng(m + n)
+    column, row = rng.integers(-999, 999, m).astype(np.float32), rng.integers(-999, 999, n).astype(np.float32)
+    bias = rng.integers(-999, 999, n).astype(np.float32)
+    residual = rng.integers(-999, 999, m * n).astype(np.float32)
+    out = np.full(m * n, 7.5, np.float32)
+    hip.gemm_bias_activation_f32(m, n, 1, hip.GemmActivation.Relu, column, row, bias, residual, out)
+    want = column[:, None] * row[None, :] + bias + residual.reshape(m, n)
+    assert (out.reshape(m, n) == np.maximum(want, 0.0)).all()
