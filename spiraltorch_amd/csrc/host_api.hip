@@ -117,6 +117,10 @@ class Lease {
             constexpr size_t kPiece = 256u << 10;
             PinnedBuffer stage;
             const HostMemory memory = host_memory(host);
+            if (bytes > kTogether) {
+                send();
+                together_ = false;
+            }
             if (bytes > kUploadMost || memory == HostMemory::kRuntime || (memory == HostMemory::kPinned && bytes >= kPiece) ||
                 !hold(bytes, &stage)) {
                 ST_HIP_TRY(hipMemcpyAsync(*device, host, bytes, hipMemcpyHostToDevice, ws_->stream),
@@ -126,7 +130,7 @@ class Lease {
             // Small operands wait for each other and go up in one launch.  A call with operands of that size is launches and their gaps: µs of relu(A·B
             // + bias) with a launch an operand / one for all, square: 16 22.1 / 17.9, 64 28.1 / 23.1, 128 30.9 / 26.3, 180 36.2 / 33.1.  Above, the first
             // operand's way up is worth more beside the copying of the next: 200 39.0 / 39.4.
-            if (bytes <= kTogether && copies_.count < kMostCopies) {
+            if (together_ && bytes <= kTogether && copies_.count < kMostCopies) {
                 std::memcpy(stage.ptr, host, bytes);
                 copies_.bytes[copies_.count] = bytes;
                 copies_.pinned[copies_.count] = static_cast<const unsigned char *>(stage.ptr);
@@ -216,6 +220,7 @@ class Lease {
 
     static constexpr size_t kTogether = 128u << 10;
     PinnedCopies copies_;            // operands that are not sent yet
+    bool together_ = true;           // all operands so far are small ones
     hipError_t sent_ = hipSuccess;   // what became of those that were
     static constexpr size_t kMostStages = 2 * kWorkspaceBuffers;  // an operand or a result each
     Workspace *ws_ = nullptr;

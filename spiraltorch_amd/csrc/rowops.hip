@@ -841,11 +841,20 @@ __global__ __launch_bounds__(256) void copy_from_pinned_kernel(size_t bytes, con
 __global__ __launch_bounds__(256) void copy_several_from_pinned_kernel(PinnedCopies copies)
 {
     unsigned block = blockIdx.x;
-    int i = 0;
-    while (i + 1 < copies.count && block >= copies.groups[i]) block -= copies.groups[i++];
-    const size_t bytes = copies.bytes[i], at = block * kUploadGroup + threadIdx.x * 16;
-    const unsigned char *const pinned = copies.pinned[i];
-    unsigned char *const device = copies.device[i];
+    size_t bytes = copies.bytes[0];
+    const unsigned char *pinned = copies.pinned[0];
+    unsigned char *device = copies.device[0];
+    bool found = block < copies.groups[0];
+#pragma unroll
+    for (int i = 1; i < kMostCopies; ++i) {  // (all arguments at once, not one after the other)
+        if (found || i >= copies.count) continue;
+        block -= copies.groups[i - 1];
+        bytes = copies.bytes[i];
+        pinned = copies.pinned[i];
+        device = copies.device[i];
+        found = block < copies.groups[i];
+    }
+    const size_t at = block * kUploadGroup + threadIdx.x * 16;
     if (at + 16 <= bytes) *reinterpret_cast<uint4 *>(device + at) = *reinterpret_cast<const uint4 *>(pinned + at);
     else
         for (size_t e = at; e < bytes; ++e) device[e] = pinned[e];
@@ -1389,6 +1398,7 @@ hipError_t launch_copies_from_pinned(PinnedCopies &copies, hipStream_t stream)
     unsigned groups = 0;
     for (int i = 0; i < copies.count; ++i) groups += copies.groups[i] = static_cast<unsigned>((copies.bytes[i] + kUploadGroup - 1) / kUploadGroup);
     if (groups == 0) return hipSuccess;
+    if (copies.count == 1) return launch_copy_from_pinned(copies.device[0], copies.pinned[0], copies.bytes[0], stream);
     hipLaunchKernelGGL(copy_several_from_pinned_kernel, dim3(groups), dim3(256), 0, stream, copies);
     return hipGetLastError();
 }
