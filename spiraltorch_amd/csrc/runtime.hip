@@ -9,6 +9,7 @@
 #include <mutex>
 #include <string>
 #include <thread>
+#include <unordered_map>
 #include <vector>
 
 #include "common.h"
@@ -275,6 +276,7 @@ struct TensorBlock {
 struct TensorPool {
     std::mutex mutex;
     std::vector<TensorBlock> idle;
+    std::unordered_map<void *, TensorBlock> lent;  // a block may be freed by a thread whose device is another
     size_t held = 0;
 };
 TensorPool &tensor_pool()  // never destroyed: tensors may be freed while the process is shutting down
@@ -551,7 +553,13 @@ int st_hip_malloc(void **device_ptr, size_t bytes)
     ST_HIP_CHECK(ensure_init());
     if (!device_ptr) return fail(ST_HIP_ERR_INVALID, "st_hip_malloc received a null out-pointer");
     *device_ptr = nullptr;
-    ST_HIP_TRY(hipMalloc(device_ptr, bytes ? bytes : 1), "hipMalloc");  // real.rs:652 max(1)
+    hipError_t rc = hipMalloc(device_ptr, bytes ? bytes : 1);  // real.rs:652 max(1)
+    if (rc == hipErrorOutOfMemory) {  // what freed tensors left may make the room
+        (void)hipGetLastError();
+        tensor_release_idle();
+        rc = hipMalloc(device_ptr, bytes ? bytes : 1);
+    }
+    ST_HIP_TRY(rc, "hipMalloc");
     return ST_HIP_OK;
 }
 
@@ -578,6 +586,7 @@ int st_hip_tensor_malloc(void **device_ptr, size_t bytes)
             if (pool.idle[i].capacity != capacity || pool.idle[i].device != device) continue;
             *device_ptr = pool.idle[i].ptr;
             pool.held -= capacity;
+            pool.lent[*device_ptr] = pool.idle[i];
             pool.idle[i] = pool.idle.back();
             pool.idle.pop_back();
             return ST_HIP_OK;
@@ -590,21 +599,27 @@ int st_hip_tensor_malloc(void **device_ptr, size_t bytes)
         rc = hipMalloc(device_ptr, capacity);
     }
     if (rc != hipSuccess) return hip_fail(rc, "hipMalloc");
+    TensorPool &pool = tensor_pool();
+    std::lock_guard<std::mutex> lock(pool.mutex);
+    pool.lent[*device_ptr] = TensorBlock{*device_ptr, capacity, device};
     return ST_HIP_OK;
 }
 
 int st_hip_tensor_free(void *device_ptr, size_t bytes)
 {
     if (!device_ptr) return ST_HIP_OK;
-    int device = 0;
-    if (bytes <= kTensorLargest && hipGetDevice(&device) == hipSuccess) {
-        const size_t capacity = tensor_capacity(bytes);
+    if (bytes <= kTensorLargest) {
         TensorPool &pool = tensor_pool();
         std::lock_guard<std::mutex> lock(pool.mutex);
-        if (pool.held + capacity <= kTensorMost) {
-            pool.idle.push_back(TensorBlock{device_ptr, capacity, device});
-            pool.held += capacity;
-            return ST_HIP_OK;
+        const auto found = pool.lent.find(device_ptr);
+        if (found != pool.lent.end()) {
+            const TensorBlock block = found->second;
+            pool.lent.erase(found);
+            if (pool.held + block.capacity <= kTensorMost) {
+                pool.idle.push_back(block);
+                pool.held += block.capacity;
+                return ST_HIP_OK;
+            }
         }
     }
     return st_hip_free(device_ptr);
@@ -615,7 +630,7 @@ int st_hip_tensor_upload(void *device_ptr, const void *host_src, size_t bytes)
     PinnedBuffer stage;
     const size_t groups = (bytes + kUploadGroup - 1) / kUploadGroup, words_at = (bytes + 15) / 16 * 16;
     if (bytes == 0 || bytes > kUploadMost || reinterpret_cast<uintptr_t>(device_ptr) % 16 != 0 || host_memory(host_src) != HostMemory::kOrdinary ||
-        !pinned_acquire(words_at + groups * sizeof(unsigned), &stage))
+        !on_current_device(device_ptr) || !pinned_acquire(words_at + groups * sizeof(unsigned), &stage))
         return st_hip_memcpy_h2d(device_ptr, host_src, bytes, nullptr);
     count_transfer(true, bytes);
     unsigned *const read = reinterpret_cast<unsigned *>(static_cast<unsigned char *>(stage.ptr) + words_at);

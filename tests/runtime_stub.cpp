@@ -7,13 +7,13 @@
 #include <cstring>
 
 extern "C" {
-int stub_no_memory = 0;
+int stub_no_memory = 0, stub_device = 0;
 unsigned long long stub_launches = 0;
 const char *stub_device_first = nullptr, *stub_device_end = nullptr;
 const void *stub_first_source = nullptr;  // of the runtime's copies
 
 hipError_t hipGetDeviceCount(int *count) { *count = 1; return hipSuccess; }
-hipError_t hipGetDevice(int *device) { *device = 0; return hipSuccess; }
+hipError_t hipGetDevice(int *device) { *device = stub_device; return hipSuccess; }
 hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600 *props, int)
 {
     std::memset(props, 0, sizeof *props);

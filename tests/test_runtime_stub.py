@@ -83,6 +83,31 @@ print(status, ctypes.c_void_p.in_dll(stub, "stub_first_source").value == closed)
     assert out == ["0", "True"]
 
 
+def test_tensor_memory_goes_back_to_the_device_it_is_on(stub):
+    """A tensor freed where another device is current (by a collector's thread, say) is not handed out there, and memory that is not a
+    tensor's is not kept."""
+    out = run(stub, """
+device = ctypes.c_int.in_dll(stub, "stub_device")
+def take():
+    p = ctypes.c_void_p()
+    assert lib.st_hip_tensor_malloc(ctypes.byref(p), 5000) == 0
+    return p.value
+first = take()
+device.value = 1
+lib.st_hip_tensor_free(first, 5000)
+other = take()
+device.value = 0
+print(other != first, take() == first)
+plain = ctypes.c_void_p()
+lib.st_hip_malloc(ctypes.byref(plain), 5000)
+lib.st_hip_tensor_free(plain, 5000)
+second = take()
+lib.st_hip_tensor_free(second, 5000)
+print(take() == second)
+""")
+    assert out == ["True", "True", "True"]
+
+
 def test_bf16_attention_launches_pass_their_check(stub):
     """Every grid the launchers of bf16 attention ask for passes the check made of it with the kernels' own decode."""
     out = run(stub, """
