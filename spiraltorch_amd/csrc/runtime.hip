@@ -6,10 +6,10 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <map>
 #include <mutex>
 #include <string>
 #include <thread>
-#include <unordered_map>
 #include <vector>
 
 #include "common.h"
@@ -170,18 +170,6 @@ HostMemory host_memory(const void *host)
     return attributes.type == hipMemoryTypeManaged || attributes.type == hipMemoryTypeDevice ? HostMemory::kRuntime : HostMemory::kOrdinary;
 }
 
-// Whether a kernel on the current device may read `device`: memory of that device.
-static bool on_current_device(const void *device)
-{
-    hipPointerAttribute_t attributes;
-    int current = 0;
-    if (hipPointerGetAttributes(&attributes, device) != hipSuccess || hipGetDevice(&current) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
-    return attributes.type == hipMemoryTypeDevice && attributes.device == current;
-}
-
 // The smallest idle buffer that fits and is not far too large; a new one where the pool may grow; any that fits; a new one in the
 // place of smaller ones.  Nothing is freed only because a call has ended: calls that need all there is would pin their memory
 // anew each time.
@@ -271,13 +259,23 @@ constexpr size_t kTensorSmallest = 4u << 10, kTensorLargest = 8u << 20, kTensorM
 struct TensorBlock {
     void *ptr;
     size_t capacity;
+    size_t bytes;  // that were asked for
     int device;
 };
 struct TensorPool {
     std::mutex mutex;
     std::vector<TensorBlock> idle;
-    std::unordered_map<void *, TensorBlock> lent;  // a block may be freed by a thread whose device is another
+    std::map<const char *, TensorBlock> lent;  // a block may be freed by a thread whose device is another
     size_t held = 0;
+    // The tensor whose memory `ptr` lies in.
+    const TensorBlock *find(const void *ptr) const
+    {
+        const char *const at = static_cast<const char *>(ptr);
+        auto after = lent.upper_bound(at);
+        if (after == lent.begin()) return nullptr;
+        const TensorBlock &block = (--after)->second;
+        return at < after->first + block.capacity ? &block : nullptr;
+    }
 };
 TensorPool &tensor_pool()  // never destroyed: tensors may be freed while the process is shutting down
 {
@@ -300,6 +298,52 @@ void tensor_release_idle()
         pool.held = 0;
     }
     for (const TensorBlock &block : doomed) (void)hipFree(block.ptr);
+}
+
+// Where `bytes` from `ptr` on lie.  What is behind a tensor in its block is not the tensor's: a copy that passes the tensor's end is
+// refused as the runtime refuses one that passes an allocation's.
+enum class TensorRange { kElsewhere, kInside, kOutside };
+TensorRange tensor_range(const void *ptr, size_t bytes, int *device)
+{
+    TensorPool &pool = tensor_pool();
+    std::lock_guard<std::mutex> lock(pool.mutex);
+    const TensorBlock *block = pool.find(ptr);
+    if (block == nullptr) return TensorRange::kElsewhere;
+    *device = block->device;
+    const size_t offset = static_cast<size_t>(static_cast<const char *>(ptr) - static_cast<const char *>(block->ptr));
+    return offset <= block->bytes && bytes <= block->bytes - offset ? TensorRange::kInside : TensorRange::kOutside;
+}
+bool passes_tensor_end(const void *ptr, size_t bytes)
+{
+    int device;
+    return tensor_range(ptr, bytes, &device) == TensorRange::kOutside;
+}
+
+// Whether a kernel on the current device may access `bytes` from `ptr` on: memory of that device, all of it in one allocation.  Whatever
+// else is left to the runtime's copy, which judges it.
+bool kernel_may_access(const void *ptr, size_t bytes)
+{
+    int current = 0, device = 0;
+    if (hipGetDevice(&current) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    const TensorRange range = tensor_range(ptr, bytes, &device);
+    if (range != TensorRange::kElsewhere) return range == TensorRange::kInside && device == current;
+    hipPointerAttribute_t attributes;
+    if (hipPointerGetAttributes(&attributes, ptr) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (attributes.type != hipMemoryTypeDevice || attributes.device != current) return false;
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipMemGetAddressRange(&base, &size, const_cast<void *>(ptr)) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    const size_t offset = static_cast<size_t>(static_cast<const char *>(ptr) - static_cast<const char *>(base));
+    return offset <= size && bytes <= size - offset;
 }
 }  // namespace
 
@@ -566,6 +610,11 @@ int st_hip_malloc(void **device_ptr, size_t bytes)
 int st_hip_free(void *device_ptr)
 {
     if (!device_ptr) return ST_HIP_OK;
+    {
+        TensorPool &pool = tensor_pool();
+        std::lock_guard<std::mutex> lock(pool.mutex);
+        pool.lent.erase(static_cast<const char *>(device_ptr));  // (the address may come back as something else)
+    }
     ST_HIP_TRY(hipFree(device_ptr), "hipFree");
     return ST_HIP_OK;
 }
@@ -586,7 +635,8 @@ int st_hip_tensor_malloc(void **device_ptr, size_t bytes)
             if (pool.idle[i].capacity != capacity || pool.idle[i].device != device) continue;
             *device_ptr = pool.idle[i].ptr;
             pool.held -= capacity;
-            pool.lent[*device_ptr] = pool.idle[i];
+            pool.idle[i].bytes = bytes;
+            pool.lent[static_cast<const char *>(*device_ptr)] = pool.idle[i];
             pool.idle[i] = pool.idle.back();
             pool.idle.pop_back();
             return ST_HIP_OK;
@@ -601,7 +651,7 @@ int st_hip_tensor_malloc(void **device_ptr, size_t bytes)
     if (rc != hipSuccess) return hip_fail(rc, "hipMalloc");
     TensorPool &pool = tensor_pool();
     std::lock_guard<std::mutex> lock(pool.mutex);
-    pool.lent[*device_ptr] = TensorBlock{*device_ptr, capacity, device};
+    pool.lent[static_cast<const char *>(*device_ptr)] = TensorBlock{*device_ptr, capacity, bytes, device};
     return ST_HIP_OK;
 }
 
@@ -611,7 +661,7 @@ int st_hip_tensor_free(void *device_ptr, size_t bytes)
     if (bytes <= kTensorLargest) {
         TensorPool &pool = tensor_pool();
         std::lock_guard<std::mutex> lock(pool.mutex);
-        const auto found = pool.lent.find(device_ptr);
+        const auto found = pool.lent.find(static_cast<const char *>(device_ptr));
         if (found != pool.lent.end()) {
             const TensorBlock block = found->second;
             pool.lent.erase(found);
@@ -630,7 +680,7 @@ int st_hip_tensor_upload(void *device_ptr, const void *host_src, size_t bytes)
     PinnedBuffer stage;
     const size_t groups = (bytes + kUploadGroup - 1) / kUploadGroup, words_at = (bytes + 15) / 16 * 16;
     if (bytes == 0 || bytes > kUploadMost || reinterpret_cast<uintptr_t>(device_ptr) % 16 != 0 || host_memory(host_src) != HostMemory::kOrdinary ||
-        !on_current_device(device_ptr) || !pinned_acquire(words_at + groups * sizeof(unsigned), &stage))
+        !kernel_may_access(device_ptr, bytes) || !pinned_acquire(words_at + groups * sizeof(unsigned), &stage))
         return st_hip_memcpy_h2d(device_ptr, host_src, bytes, nullptr);
     count_transfer(true, bytes);
     unsigned *const read = reinterpret_cast<unsigned *>(static_cast<unsigned char *>(stage.ptr) + words_at);
@@ -648,6 +698,7 @@ int st_hip_tensor_upload(void *device_ptr, const void *host_src, size_t bytes)
 int st_hip_memcpy_h2d(void *device_dst, const void *host_src, size_t bytes, void *stream)
 {
     if (bytes == 0) return ST_HIP_OK;
+    if (passes_tensor_end(device_dst, bytes)) return hip_fail(hipErrorInvalidValue, "hipMemcpyAsync(H2D)");
     count_transfer(true, bytes);
     ST_HIP_TRY(hipMemcpyAsync(device_dst, host_src, bytes, hipMemcpyHostToDevice, as_stream(stream)),
                "hipMemcpyAsync(H2D)");
@@ -658,10 +709,11 @@ int st_hip_memcpy_h2d(void *device_dst, const void *host_src, size_t bytes, void
 int st_hip_memcpy_d2h(void *host_dst, const void *device_src, size_t bytes, void *stream)
 {
     if (bytes == 0) return ST_HIP_OK;
+    if (passes_tensor_end(device_src, bytes)) return hip_fail(hipErrorInvalidValue, "hipMemcpyAsync(D2H)");
     count_transfer(false, bytes);
     PinnedBuffer stage;
     const bool staged = bytes <= kReadMost && host_memory(host_dst) == HostMemory::kOrdinary && pinned_acquire(bytes, &stage);
-    if (staged && reinterpret_cast<uintptr_t>(device_src) % 16 == 0 && on_current_device(device_src)) {
+    if (staged && reinterpret_cast<uintptr_t>(device_src) % 16 == 0 && kernel_may_access(device_src, bytes)) {
         const size_t pieces = (bytes + kCopyPiece - 1) / kCopyPiece;
         unsigned *const words = stage.words();
         std::memset(words, 0, pieces * sizeof(unsigned));
@@ -696,6 +748,7 @@ int st_hip_memcpy_d2h(void *host_dst, const void *device_src, size_t bytes, void
 int st_hip_memset_zero(void *device_dst, size_t bytes, void *stream)
 {
     if (bytes == 0) return ST_HIP_OK;
+    if (passes_tensor_end(device_dst, bytes)) return hip_fail(hipErrorInvalidValue, "hipMemsetAsync");
     ST_HIP_TRY(hipMemsetAsync(device_dst, 0, bytes, as_stream(stream)), "hipMemsetAsync");
     return ST_HIP_OK;
 }

@@ -62,8 +62,14 @@ hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_
     ++stub_launches;
     return hipSuccess;
 }
-hipError_t hipMemcpyAsync(void *, const void *src, size_t, hipMemcpyKind, hipStream_t)
+static bool passes_device_end(const void *ptr, size_t bytes)
 {
+    const char *const at = static_cast<const char *>(ptr);
+    return at >= stub_device_first && at < stub_device_end && bytes > static_cast<size_t>(stub_device_end - at);
+}
+hipError_t hipMemcpyAsync(void *dst, const void *src, size_t bytes, hipMemcpyKind, hipStream_t)
+{
+    if (passes_device_end(src, bytes) || passes_device_end(dst, bytes)) return hipErrorInvalidValue;
     if (stub_first_source == nullptr) stub_first_source = src;
     return hipSuccess;
 }
@@ -75,4 +81,11 @@ hipError_t hipPointerGetAttributes(hipPointerAttribute_t *attributes, const void
     attributes->type = hipMemoryTypeDevice;
     return hipSuccess;
 }
+hipError_t hipMemGetAddressRange(hipDeviceptr_t *base, size_t *size, hipDeviceptr_t)  // (of what is device memory, asked before)
+{
+    *base = const_cast<char *>(stub_device_first);
+    *size = static_cast<size_t>(stub_device_end - stub_device_first);
+    return hipSuccess;
+}
+hipError_t hipMemsetAsync(void *, int, size_t, hipStream_t) { return hipSuccess; }
 }

@@ -108,6 +108,54 @@ print(take() == second)
     assert out == ["True", "True", "True"]
 
 
+def test_copies_past_the_end_of_device_memory_are_refused(stub):
+    """A read that a kernel makes, and a tensor's upload, are refused where the runtime's copy refuses: no kernel is launched."""
+    out = run(stub, """
+import numpy as np
+host, memory = np.zeros(9000, np.uint8), np.zeros(9000, np.uint8)
+first = (memory.ctypes.data + 15) // 16 * 16
+for name, value in (("stub_device_first", first), ("stub_device_end", first + 5000)):
+    ctypes.c_void_p.in_dll(stub, name).value = value
+def launched(call, *args):
+    before = launches.value
+    status = call(*args)
+    return launches.value - before, status != 0
+read = lambda at, bytes: launched(lib.st_hip_memcpy_d2h, host.ctypes.data, at, bytes, None)
+send = lambda at, bytes: launched(lib.st_hip_tensor_upload, at, host.ctypes.data, bytes)
+for at in (first, first + 4096):
+    room = first + 5000 - at
+    print(read(at, room)[0], read(at, room + 1) == (0, True), send(at, room)[0], send(at, room + 1) == (0, True))
+""")
+    assert out == ["1", "True", "1", "True"] * 2
+
+
+def test_copies_past_the_end_of_a_tensor_are_refused(stub):
+    """A tensor's block is larger than the tensor; what lies behind it is not the tensor's, now or when the block was another's."""
+    out = run(stub, """
+import numpy as np
+host = np.zeros(20000, np.uint8)
+p = ctypes.c_void_p()
+for size in (8000, 5000, 6000):
+    assert lib.st_hip_tensor_malloc(ctypes.byref(p), size) == 0
+    first = p.value
+    for at in (first, first + 4096, first + size - 1):
+        room = first + size - at
+        before = launches.value
+        kept = (lib.st_hip_memcpy_h2d(at, host.ctypes.data, room, None), lib.st_hip_memset_zero(at, room, None))
+        refused = [call != 0 for call in (
+            lib.st_hip_tensor_upload(at, host.ctypes.data, room + 1), lib.st_hip_memcpy_h2d(at, host.ctypes.data, room + 1, None),
+            lib.st_hip_memcpy_d2h(host.ctypes.data, at, room + 1, None), lib.st_hip_memset_zero(at, room + 1, None))]
+        print(kept == (0, 0), all(refused), launches.value == before)
+    before = launches.value
+    print(lib.st_hip_tensor_upload(first, host.ctypes.data, size) == 0, launches.value == before + 1)
+    lib.st_hip_tensor_free(first, size)
+lib.st_hip_tensor_malloc(ctypes.byref(p), 5000)
+lib.st_hip_free(p)
+print(lib.st_hip_memcpy_h2d(p, host.ctypes.data, 6000, None) == 0)  # whatever is there next
+""")
+    assert out == ["True"] * len(out) and len(out) == 34
+
+
 def test_bf16_attention_launches_pass_their_check(stub):
     """Every grid the launchers of bf16 attention ask for passes the check made of it with the kernels' own decode."""
     out = run(stub, """
