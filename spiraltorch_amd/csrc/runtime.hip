@@ -261,18 +261,19 @@ struct TensorBlock {
     size_t capacity;
     size_t bytes;  // that were asked for
     int device;
+    bool idle;
 };
 struct TensorPool {
     std::mutex mutex;
-    std::vector<TensorBlock> idle;
-    std::map<const char *, TensorBlock> lent;  // a block may be freed by a thread whose device is another
+    std::map<const char *, TensorBlock> blocks;  // in use or idle; a block may be freed by a thread whose device is another
+    std::vector<TensorBlock *> idle;
     size_t held = 0;
     // The tensor whose memory `ptr` lies in.
     const TensorBlock *find(const void *ptr) const
     {
         const char *const at = static_cast<const char *>(ptr);
-        auto after = lent.upper_bound(at);
-        if (after == lent.begin()) return nullptr;
+        auto after = blocks.upper_bound(at);
+        if (after == blocks.begin()) return nullptr;
         const TensorBlock &block = (--after)->second;
         return at < after->first + block.capacity ? &block : nullptr;
     }
@@ -290,18 +291,22 @@ size_t tensor_capacity(size_t bytes)
 }
 void tensor_release_idle()
 {
-    std::vector<TensorBlock> doomed;
+    std::vector<void *> doomed;
     {
         TensorPool &pool = tensor_pool();
         std::lock_guard<std::mutex> lock(pool.mutex);
-        doomed.swap(pool.idle);
+        for (const TensorBlock *block : pool.idle) {
+            doomed.push_back(block->ptr);
+            pool.blocks.erase(static_cast<const char *>(doomed.back()));
+        }
+        pool.idle.clear();
         pool.held = 0;
     }
-    for (const TensorBlock &block : doomed) (void)hipFree(block.ptr);
+    for (void *ptr : doomed) (void)hipFree(ptr);
 }
 
-// Where `bytes` from `ptr` on lie.  What is behind a tensor in its block is not the tensor's: a copy that passes the tensor's end is
-// refused as the runtime refuses one that passes an allocation's.
+// Where `bytes` from `ptr` on lie.  What is behind a tensor in its block is not the tensor's, and an idle block is nobody's: a copy there
+// is refused as the runtime refuses one that passes an allocation's end.
 enum class TensorRange { kElsewhere, kInside, kOutside };
 TensorRange tensor_range(const void *ptr, size_t bytes, int *device)
 {
@@ -311,7 +316,7 @@ TensorRange tensor_range(const void *ptr, size_t bytes, int *device)
     if (block == nullptr) return TensorRange::kElsewhere;
     *device = block->device;
     const size_t offset = static_cast<size_t>(static_cast<const char *>(ptr) - static_cast<const char *>(block->ptr));
-    return offset <= block->bytes && bytes <= block->bytes - offset ? TensorRange::kInside : TensorRange::kOutside;
+    return !block->idle && offset <= block->bytes && bytes <= block->bytes - offset ? TensorRange::kInside : TensorRange::kOutside;
 }
 bool passes_tensor_end(const void *ptr, size_t bytes)
 {
@@ -613,7 +618,11 @@ int st_hip_free(void *device_ptr)
     {
         TensorPool &pool = tensor_pool();
         std::lock_guard<std::mutex> lock(pool.mutex);
-        pool.lent.erase(static_cast<const char *>(device_ptr));  // (the address may come back as something else)
+        const auto found = pool.blocks.find(static_cast<const char *>(device_ptr));
+        if (found != pool.blocks.end()) {
+            if (found->second.idle) return hip_fail(hipErrorInvalidValue, "hipFree");  // freed before
+            pool.blocks.erase(found);  // (the address may come back as something else)
+        }
     }
     ST_HIP_TRY(hipFree(device_ptr), "hipFree");
     return ST_HIP_OK;
@@ -632,11 +641,12 @@ int st_hip_tensor_malloc(void **device_ptr, size_t bytes)
         TensorPool &pool = tensor_pool();
         std::lock_guard<std::mutex> lock(pool.mutex);
         for (size_t i = pool.idle.size(); i-- > 0;) {
-            if (pool.idle[i].capacity != capacity || pool.idle[i].device != device) continue;
-            *device_ptr = pool.idle[i].ptr;
+            TensorBlock &block = *pool.idle[i];
+            if (block.capacity != capacity || block.device != device) continue;
+            *device_ptr = block.ptr;
+            block.bytes = bytes;
+            block.idle = false;
             pool.held -= capacity;
-            pool.idle[i].bytes = bytes;
-            pool.lent[static_cast<const char *>(*device_ptr)] = pool.idle[i];
             pool.idle[i] = pool.idle.back();
             pool.idle.pop_back();
             return ST_HIP_OK;
@@ -651,25 +661,22 @@ int st_hip_tensor_malloc(void **device_ptr, size_t bytes)
     if (rc != hipSuccess) return hip_fail(rc, "hipMalloc");
     TensorPool &pool = tensor_pool();
     std::lock_guard<std::mutex> lock(pool.mutex);
-    pool.lent[static_cast<const char *>(*device_ptr)] = TensorBlock{*device_ptr, capacity, bytes, device};
+    pool.blocks[static_cast<const char *>(*device_ptr)] = TensorBlock{*device_ptr, capacity, bytes, device, false};
     return ST_HIP_OK;
 }
 
 int st_hip_tensor_free(void *device_ptr, size_t bytes)
 {
     if (!device_ptr) return ST_HIP_OK;
-    if (bytes <= kTensorLargest) {
+    {
         TensorPool &pool = tensor_pool();
         std::lock_guard<std::mutex> lock(pool.mutex);
-        const auto found = pool.lent.find(static_cast<const char *>(device_ptr));
-        if (found != pool.lent.end()) {
-            const TensorBlock block = found->second;
-            pool.lent.erase(found);
-            if (pool.held + block.capacity <= kTensorMost) {
-                pool.idle.push_back(block);
-                pool.held += block.capacity;
-                return ST_HIP_OK;
-            }
+        const auto found = pool.blocks.find(static_cast<const char *>(device_ptr));
+        if (found != pool.blocks.end() && !found->second.idle && bytes <= kTensorLargest && pool.held + found->second.capacity <= kTensorMost) {
+            found->second.idle = true;
+            pool.idle.push_back(&found->second);
+            pool.held += found->second.capacity;
+            return ST_HIP_OK;
         }
     }
     return st_hip_free(device_ptr);

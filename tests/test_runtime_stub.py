@@ -108,6 +108,24 @@ print(take() == second)
     assert out == ["True", "True", "True"]
 
 
+def test_tensor_memory_is_freed_once(stub):
+    """A second free of a tensor is an error, as the runtime's of any memory, and does not touch the block that is kept."""
+    out = run(stub, """
+import numpy as np
+def take():
+    p = ctypes.c_void_p()
+    assert lib.st_hip_tensor_malloc(ctypes.byref(p), 5000) == 0
+    return p.value
+first, other = take(), take()
+print(lib.st_hip_tensor_free(first, 5000) == 0, lib.st_hip_tensor_free(first, 5000) != 0, lib.st_hip_free(first) != 0)
+host = np.zeros(16, np.uint8)
+print(lib.st_hip_memcpy_h2d(first, host.ctypes.data, 16, None) != 0)
+print(take() == first, take() not in (first, other))
+print(lib.st_hip_tensor_free(first, 5000) == 0)
+""")
+    assert out == ["True"] * 7
+
+
 def test_copies_past_the_end_of_device_memory_are_refused(stub):
     """A read that a kernel makes, and a tensor's upload, are refused where the runtime's copy refuses: no kernel is launched."""
     out = run(stub, """
