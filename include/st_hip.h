@@ -79,9 +79,10 @@ size_t st_hip_last_error_message(char *buf, size_t len);
 /* DeviceBuffer / HipStream RAII pairs of real.rs:649-667 and :190-220, flattened to C. */
 int st_hip_malloc(void **device_ptr, size_t bytes);
 int st_hip_free(void *device_ptr);
-/* The same for memory whose every use is a call on the default stream (NULL): st_hip_tensor_free (with the size it was asked for) does
- * not wait for the device, and keeps up to 64 MiB of blocks of up to 8 MiB for the next st_hip_tensor_malloc on the current device, whose
- * work on that stream comes after what is queued.  st_hip_release_scratch(NULL) frees what is kept.  No reference counterpart. */
+/* The same for memory whose every use is a call on the default stream (NULL): st_hip_tensor_free (with the size it was asked for) keeps
+ * up to 64 MiB of blocks of up to 8 MiB for the next st_hip_tensor_malloc on the current device, whose work on that stream comes after
+ * what is queued.  It waits for the device only where blocks go back to the runtime: larger ones, and the longest idle where the room is
+ * used up.  st_hip_release_scratch(NULL) frees what is kept.  No reference counterpart. */
 int st_hip_tensor_malloc(void **device_ptr, size_t bytes);
 int st_hip_tensor_free(void *device_ptr, size_t bytes);
 /* Such memory's values from the host, ordered with the default stream's work: the source may be changed when the call returns, which

@@ -6,6 +6,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <deque>
 #include <map>
 #include <mutex>
 #include <string>
@@ -253,21 +254,23 @@ namespace {
 // Device memory of tensors that are used on the default stream alone: what one frees the next may take at once, for their work is
 // ordered, whatever threads they belong to.  hipFree waits for the whole device instead, 6.5 µs with nothing to wait for, and waiting for the
 // stream costs about two for every launch since the last wait: a call of a classifier on 64 rows, five tensors, takes 152 µs with hipFree, a
-// waiting upload and a waiting read, 149 with either of the three in their way, 116 with none (the read: st_hip_memcpy_d2h).  Blocks of powers of two, kept for the device they are on, kTensorMost
-// bytes at the most; larger ones and what finds no room go back to the runtime.
+// waiting upload and a waiting read, 149 with either of the three in their way, 116 with none (the read: st_hip_memcpy_d2h).  Blocks of
+// powers of two, kept for the device they are on, kTensorMost bytes at the most: the longest idle ones make room for the next, so that
+// sizes a program no longer uses do not keep out those it does.  Larger ones go back to the runtime.
 constexpr size_t kTensorSmallest = 4u << 10, kTensorLargest = 8u << 20, kTensorMost = 64u << 20;
 struct TensorBlock {
     void *ptr;
     size_t capacity;
     size_t bytes;  // that were asked for
     int device;
-    bool idle;
+    uint64_t idle_since;  // 0: in use
 };
 struct TensorPool {
     std::mutex mutex;
     std::map<const char *, TensorBlock> blocks;  // in use or idle; a block may be freed by a thread whose device is another
-    std::vector<TensorBlock *> idle;
+    std::deque<TensorBlock *> idle[__builtin_ctzll(kTensorLargest / kTensorSmallest) + 1];  // by size, the longest idle first
     size_t held = 0;
+    uint64_t frees = 0;
     // The tensor whose memory `ptr` lies in.
     const TensorBlock *find(const void *ptr) const
     {
@@ -276,6 +279,21 @@ struct TensorPool {
         if (after == blocks.begin()) return nullptr;
         const TensorBlock &block = (--after)->second;
         return at < after->first + block.capacity ? &block : nullptr;
+    }
+    std::deque<TensorBlock *> &idle_of(size_t capacity) { return idle[__builtin_ctzll(capacity / kTensorSmallest)]; }
+    // Makes `most` of what is held, of the longest idle blocks: the caller frees what it is given.
+    void shrink(size_t most, std::vector<void *> &doomed)
+    {
+        while (held > most) {
+            std::deque<TensorBlock *> *oldest = nullptr;
+            for (auto &blocks_of_size : idle)
+                if (!blocks_of_size.empty() && (oldest == nullptr || blocks_of_size.front()->idle_since < oldest->front()->idle_since)) oldest = &blocks_of_size;
+            const TensorBlock *const block = oldest->front();
+            oldest->pop_front();
+            held -= block->capacity;
+            doomed.push_back(block->ptr);
+            blocks.erase(static_cast<const char *>(doomed.back()));
+        }
     }
 };
 TensorPool &tensor_pool()  // never destroyed: tensors may be freed while the process is shutting down
@@ -295,12 +313,7 @@ void tensor_release_idle()
     {
         TensorPool &pool = tensor_pool();
         std::lock_guard<std::mutex> lock(pool.mutex);
-        for (const TensorBlock *block : pool.idle) {
-            doomed.push_back(block->ptr);
-            pool.blocks.erase(static_cast<const char *>(doomed.back()));
-        }
-        pool.idle.clear();
-        pool.held = 0;
+        pool.shrink(0, doomed);
     }
     for (void *ptr : doomed) (void)hipFree(ptr);
 }
@@ -316,7 +329,7 @@ TensorRange tensor_range(const void *ptr, size_t bytes, int *device)
     if (block == nullptr) return TensorRange::kElsewhere;
     *device = block->device;
     const size_t offset = static_cast<size_t>(static_cast<const char *>(ptr) - static_cast<const char *>(block->ptr));
-    return !block->idle && offset <= block->bytes && bytes <= block->bytes - offset ? TensorRange::kInside : TensorRange::kOutside;
+    return block->idle_since == 0 && offset <= block->bytes && bytes <= block->bytes - offset ? TensorRange::kInside : TensorRange::kOutside;
 }
 bool passes_tensor_end(const void *ptr, size_t bytes)
 {
@@ -620,7 +633,7 @@ int st_hip_free(void *device_ptr)
         std::lock_guard<std::mutex> lock(pool.mutex);
         const auto found = pool.blocks.find(static_cast<const char *>(device_ptr));
         if (found != pool.blocks.end()) {
-            if (found->second.idle) return hip_fail(hipErrorInvalidValue, "hipFree");  // freed before
+            if (found->second.idle_since != 0) return hip_fail(hipErrorInvalidValue, "hipFree");  // freed before
             pool.blocks.erase(found);  // (the address may come back as something else)
         }
     }
@@ -640,15 +653,15 @@ int st_hip_tensor_malloc(void **device_ptr, size_t bytes)
     {
         TensorPool &pool = tensor_pool();
         std::lock_guard<std::mutex> lock(pool.mutex);
-        for (size_t i = pool.idle.size(); i-- > 0;) {
-            TensorBlock &block = *pool.idle[i];
-            if (block.capacity != capacity || block.device != device) continue;
+        std::deque<TensorBlock *> &idle = pool.idle_of(capacity);
+        for (size_t i = idle.size(); i-- > 0;) {
+            TensorBlock &block = *idle[i];
+            if (block.device != device) continue;
+            idle.erase(idle.begin() + static_cast<long>(i));
             *device_ptr = block.ptr;
             block.bytes = bytes;
-            block.idle = false;
+            block.idle_since = 0;
             pool.held -= capacity;
-            pool.idle[i] = pool.idle.back();
-            pool.idle.pop_back();
             return ST_HIP_OK;
         }
     }
@@ -661,25 +674,29 @@ int st_hip_tensor_malloc(void **device_ptr, size_t bytes)
     if (rc != hipSuccess) return hip_fail(rc, "hipMalloc");
     TensorPool &pool = tensor_pool();
     std::lock_guard<std::mutex> lock(pool.mutex);
-    pool.blocks[static_cast<const char *>(*device_ptr)] = TensorBlock{*device_ptr, capacity, bytes, device, false};
+    pool.blocks[static_cast<const char *>(*device_ptr)] = TensorBlock{*device_ptr, capacity, bytes, device, 0};
     return ST_HIP_OK;
 }
 
 int st_hip_tensor_free(void *device_ptr, size_t bytes)
 {
     if (!device_ptr) return ST_HIP_OK;
-    {
+    std::vector<void *> doomed;
+    auto keep = [&] {
         TensorPool &pool = tensor_pool();
         std::lock_guard<std::mutex> lock(pool.mutex);
         const auto found = pool.blocks.find(static_cast<const char *>(device_ptr));
-        if (found != pool.blocks.end() && !found->second.idle && bytes <= kTensorLargest && pool.held + found->second.capacity <= kTensorMost) {
-            found->second.idle = true;
-            pool.idle.push_back(&found->second);
-            pool.held += found->second.capacity;
-            return ST_HIP_OK;
-        }
-    }
-    return st_hip_free(device_ptr);
+        if (found == pool.blocks.end() || found->second.idle_since != 0 || bytes > kTensorLargest) return false;
+        TensorBlock &block = found->second;
+        pool.held += block.capacity;
+        pool.shrink(kTensorMost, doomed);
+        block.idle_since = ++pool.frees;
+        pool.idle_of(block.capacity).push_back(&block);
+        return true;
+    };
+    if (!keep()) return st_hip_free(device_ptr);
+    for (void *ptr : doomed) (void)hipFree(ptr);
+    return ST_HIP_OK;
 }
 
 int st_hip_tensor_upload(void *device_ptr, const void *host_src, size_t bytes)

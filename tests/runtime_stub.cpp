@@ -8,7 +8,7 @@
 
 extern "C" {
 int stub_no_memory = 0, stub_device = 0;
-unsigned long long stub_launches = 0;
+unsigned long long stub_launches = 0, stub_frees = 0;
 const char *stub_device_first = nullptr, *stub_device_end = nullptr;
 const void *stub_first_source = nullptr;  // of the runtime's copies
 
@@ -29,7 +29,7 @@ hipError_t hipMalloc(void **ptr, size_t bytes)
     *ptr = std::aligned_alloc(4096, (bytes + 4095) / 4096 * 4096);
     return *ptr ? hipSuccess : hipErrorOutOfMemory;
 }
-hipError_t hipFree(void *ptr) { std::free(ptr); return hipSuccess; }
+hipError_t hipFree(void *ptr) { ++stub_frees; std::free(ptr); return hipSuccess; }
 hipError_t hipHostMalloc(void **ptr, size_t bytes, unsigned)
 {
     *ptr = std::aligned_alloc(4096, (bytes + 4095) / 4096 * 4096);

@@ -126,6 +126,32 @@ print(lib.st_hip_tensor_free(first, 5000) == 0)
     assert out == ["True"] * 7
 
 
+def test_tensors_no_longer_used_make_room_for_those_that_are(stub):
+    """All that is kept is of one size, and a program goes on with others: theirs are kept in its place, the longest idle go."""
+    out = run(stub, """
+frees = ctypes.c_ulonglong.in_dll(stub, "stub_frees")
+def take(size):
+    p = ctypes.c_void_p()
+    assert lib.st_hip_tensor_malloc(ctypes.byref(p), size) == 0
+    return p.value
+MIB = 1 << 20
+large = [take(8 * MIB) for _ in range(9)]
+for p in large: lib.st_hip_tensor_free(p, 8 * MIB)
+print(frees.value)  # the first of nine
+small = [take(size) for size in (5000, 70000, 3 * MIB)]
+for p, size in zip(small, (5000, 70000, 3 * MIB)): lib.st_hip_tensor_free(p, size)
+print(frees.value)  # and the second
+again = [take(size) for size in (5000, 70000, 3 * MIB)]
+print(again == small, frees.value)
+rest = [take(8 * MIB) for _ in range(7)]
+print(sorted(rest) == sorted(large[2:]))
+for p, size in zip(again, (5000, 70000, 3 * MIB)): lib.st_hip_tensor_free(p, size)
+lib.st_hip_release_scratch(None)
+print(frees.value)
+""")
+    assert out == ["1", "2", "True", "2", "True", "5"]
+
+
 def test_copies_past_the_end_of_device_memory_are_refused(stub):
     """A read that a kernel makes, and a tensor's upload, are refused where the runtime's copy refuses: no kernel is launched."""
     out = run(stub, """
