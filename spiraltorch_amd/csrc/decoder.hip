@@ -41,7 +41,7 @@ struct Decoder {
     int alloc(T **out, size_t count)
     {
         void *ptr = nullptr;
-        ST_HIP_TRY(hipMalloc(&ptr, (count ? count : 1) * sizeof(T)), "hipMalloc");
+        ST_HIP_TRY(device_malloc(&ptr, (count ? count : 1) * sizeof(T)), "hipMalloc");
         allocations.push_back(ptr);
         *out = static_cast<T *>(ptr);
         return ST_HIP_OK;
@@ -121,7 +121,7 @@ int st_hip_decoder_create(const st_hip_decoder_config *config, const float *host
         status = dec->alloc(dst, in * out);
         if (status != ST_HIP_OK) return;
         void *rounded = nullptr;
-        hipError_t rc = hipMalloc(&rounded, (in * out ? in * out : 1) * sizeof(uint16_t));
+        hipError_t rc = device_malloc(&rounded, (in * out ? in * out : 1) * sizeof(uint16_t));
         if (rc != hipSuccess) { status = hip_fail(rc, "hipMalloc"); return; }
         staging.push_back(rounded);
         rc = launch_f32_to_bf16(in * out, src, static_cast<uint16_t *>(rounded), nullptr);

@@ -100,7 +100,7 @@ class Lease {
                 ws_->capacity[slot] = 0;
             }
             const size_t rounded = ((bytes ? bytes : 1) + 255) & ~static_cast<size_t>(255);
-            ST_HIP_TRY(hipMalloc(&ws_->buffers[slot], rounded), "hipMalloc");
+            ST_HIP_TRY(device_malloc(&ws_->buffers[slot], rounded), "hipMalloc");
             ws_->capacity[slot] = rounded;
         }
         *out = ws_->buffers[slot];

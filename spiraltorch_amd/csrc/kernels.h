@@ -234,6 +234,8 @@ hipError_t launch_probe_mfma_bf16(size_t workgroups, size_t iterations, const ui
 hipError_t launch_probe_mfma_f32(size_t workgroups, size_t iterations, const float *operands, float *sink, hipStream_t stream);
 hipError_t launch_probe_stream_lds(size_t workgroups, size_t iterations, const void *region, size_t region_bytes, hipStream_t stream);
 
+// hipMalloc, which frees what freed tensors left (st_hip_tensor_free) before it gives up.
+hipError_t device_malloc(void **out, size_t bytes);
 // One grow-only device buffer per (stream, host thread) for kernels that need scratch memory (split-k partial sums,
 // column-sum partials).  A thread's work on a stream is ordered, so two of its launches never use the buffer at the
 // same time, and threads that share a stream (the NULL stream) do not share scratch.  A buffer whose thread has exited

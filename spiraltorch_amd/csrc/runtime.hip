@@ -365,6 +365,17 @@ bool kernel_may_access(const void *ptr, size_t bytes)
 }
 }  // namespace
 
+hipError_t device_malloc(void **out, size_t bytes)
+{
+    hipError_t rc = hipMalloc(out, bytes);
+    if (rc == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        tensor_release_idle();
+        rc = hipMalloc(out, bytes);
+    }
+    return rc;
+}
+
 namespace {
 // Scratch is keyed by (stream, host thread, slot): launches on one stream from one thread are ordered, so they never
 // use the buffer at the same time; two host threads that share a stream (every caller that passes none shares the
@@ -434,7 +445,7 @@ hipError_t scratch_malloc(void **out, size_t bytes, bool capturing)
 {
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
     if (capturing && hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return hipErrorStreamCaptureUnsupported;
-    const hipError_t rc = hipMalloc(out, bytes);
+    const hipError_t rc = capturing ? hipMalloc(out, bytes) : device_malloc(out, bytes);
     if (rc != hipSuccess) (void)hipGetLastError();  // the caller may go on without scratch
     if (capturing) (void)hipThreadExchangeStreamCaptureMode(&mode);
     return rc;
@@ -615,13 +626,7 @@ int st_hip_malloc(void **device_ptr, size_t bytes)
     ST_HIP_CHECK(ensure_init());
     if (!device_ptr) return fail(ST_HIP_ERR_INVALID, "st_hip_malloc received a null out-pointer");
     *device_ptr = nullptr;
-    hipError_t rc = hipMalloc(device_ptr, bytes ? bytes : 1);  // real.rs:652 max(1)
-    if (rc == hipErrorOutOfMemory) {  // what freed tensors left may make the room
-        (void)hipGetLastError();
-        tensor_release_idle();
-        rc = hipMalloc(device_ptr, bytes ? bytes : 1);
-    }
-    ST_HIP_TRY(rc, "hipMalloc");
+    ST_HIP_TRY(device_malloc(device_ptr, bytes ? bytes : 1), "hipMalloc");  // real.rs:652 max(1)
     return ST_HIP_OK;
 }
 
@@ -665,13 +670,7 @@ int st_hip_tensor_malloc(void **device_ptr, size_t bytes)
             return ST_HIP_OK;
         }
     }
-    hipError_t rc = hipMalloc(device_ptr, capacity);
-    if (rc == hipErrorOutOfMemory) {
-        (void)hipGetLastError();
-        tensor_release_idle();
-        rc = hipMalloc(device_ptr, capacity);
-    }
-    if (rc != hipSuccess) return hip_fail(rc, "hipMalloc");
+    ST_HIP_TRY(device_malloc(device_ptr, capacity), "hipMalloc");
     TensorPool &pool = tensor_pool();
     std::lock_guard<std::mutex> lock(pool.mutex);
     pool.blocks[static_cast<const char *>(*device_ptr)] = TensorBlock{*device_ptr, capacity, bytes, device, 0};

@@ -1,14 +1,15 @@
 // A HIP runtime without a GPU, for tests of what the library's host code asks of the real one: launches are counted and not run,
-// device memory is host memory, of which there may be none (stub_no_memory), and addresses within [stub_device_first,
+// device memory is host memory, of which there may be none (stub_no_memory) or so much (stub_memory_most), and addresses within [stub_device_first,
 // stub_device_end) are reported as device memory.  Loaded before libsthip.so with its symbols global.
 #include <hip/hip_runtime_api.h>
 
 #include <cstdlib>
 #include <cstring>
+#include <map>
 
 extern "C" {
 int stub_no_memory = 0, stub_device = 0;
-unsigned long long stub_launches = 0, stub_frees = 0;
+unsigned long long stub_launches = 0, stub_frees = 0, stub_memory_used = 0, stub_memory_most = ~0ull;
 const char *stub_device_first = nullptr, *stub_device_end = nullptr;
 const void *stub_first_source = nullptr;  // of the runtime's copies
 
@@ -23,13 +24,22 @@ hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600 *props, int)
 }
 hipError_t hipGetSymbolAddress(void **address, const void *symbol) { *address = const_cast<void *>(symbol); return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
+static std::map<void *, size_t> &allocations() { static auto *all = new std::map<void *, size_t>; return *all; }
 hipError_t hipMalloc(void **ptr, size_t bytes)
 {
-    if (stub_no_memory) return hipErrorOutOfMemory;
+    if (stub_no_memory || stub_memory_used + bytes > stub_memory_most) return hipErrorOutOfMemory;
     *ptr = std::aligned_alloc(4096, (bytes + 4095) / 4096 * 4096);
+    if (*ptr) stub_memory_used += allocations()[*ptr] = bytes;
     return *ptr ? hipSuccess : hipErrorOutOfMemory;
 }
-hipError_t hipFree(void *ptr) { ++stub_frees; std::free(ptr); return hipSuccess; }
+hipError_t hipFree(void *ptr)
+{
+    ++stub_frees;
+    stub_memory_used -= allocations()[ptr];
+    allocations().erase(ptr);
+    std::free(ptr);
+    return hipSuccess;
+}
 hipError_t hipHostMalloc(void **ptr, size_t bytes, unsigned)
 {
     *ptr = std::aligned_alloc(4096, (bytes + 4095) / 4096 * 4096);

@@ -152,6 +152,32 @@ print(frees.value)
     assert out == ["1", "2", "True", "2", "True", "5"]
 
 
+@pytest.mark.parametrize("call", ["hip.DeviceBuffer(20 << 20)", "hip.TensorBuffer(20 << 20)", "hip.TensorBuffer(3 << 20)",
+                                  # a host call's operands, scratch for slices of k, a decoder's memory
+                                  "hip.gemm_f32(2048, 8, 1024, np.ones(2 << 20, np.float32), np.ones(8 << 10, np.float32), np.ones(16 << 10, np.float32))",
+                                  "hip.gemm_bf16_bias_act_dev(3000, 1000, 1000, 0, 1 << 20, 2 << 20, None, None, 3 << 20, None)",
+                                  "hip.Decoder(256, 256, 4, 2, 1024, 1, 64, 1e-5, np.zeros(256 * 256 + 2 * (4 * 256 + 256 * 768 + 768 + 256 * 256 + 256 + 2 * (256 * 1024) + 1024 + 256) + 2 * 256 + 256 * 256 + 256, np.float32))"])
+def test_allocations_take_the_room_that_freed_tensors_left(stub, call):
+    out = run(stub, f"""
+import numpy as np
+frees = ctypes.c_ulonglong.in_dll(stub, "stub_frees")
+used, most = (ctypes.c_ulonglong.in_dll(stub, "stub_memory_" + name) for name in ("used", "most"))
+tensors = [hip.TensorBuffer(8 << 20) for _ in range(4)]
+for tensor in tensors: tensor.free()
+most.value = (32 << 20) + 1000
+before = launches.value
+try:
+    {call}
+    print("done")
+except hip.HipErr as err:
+    print("failed" if "hipMalloc" in str(err) or "OutOfMemory" in str(err) else "done")
+print(frees.value >= 4, launches.value - before)
+""")
+    assert out[:2] == ["done", "True"], out
+    if "bf16" in call:
+        assert out[2] == "2"  # the padded copies and the product on them
+
+
 def test_copies_past_the_end_of_device_memory_are_refused(stub):
     """A read that a kernel makes, and a tensor's upload, are refused where the runtime's copy refuses: no kernel is launched."""
     out = run(stub, """
