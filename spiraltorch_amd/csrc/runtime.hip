@@ -337,12 +337,12 @@ bool passes_tensor_end(const void *ptr, size_t bytes)
     return tensor_range(ptr, bytes, &device) == TensorRange::kOutside;
 }
 
-// Whether a kernel on the current device may access `bytes` from `ptr` on: memory of that device, all of it in one allocation.  Whatever
+// Whether a kernel on `stream` may access `bytes` from `ptr` on: memory of the stream's device, all of it in one allocation.  Whatever
 // else is left to the runtime's copy, which judges it.
-bool kernel_may_access(const void *ptr, size_t bytes)
+bool kernel_may_access(const void *ptr, size_t bytes, hipStream_t stream)
 {
     int current = 0, device = 0;
-    if (hipGetDevice(&current) != hipSuccess) {
+    if ((stream == nullptr ? hipGetDevice(&current) : hipStreamGetDevice(stream, &current)) != hipSuccess) {
         (void)hipGetLastError();
         return false;
     }
@@ -703,7 +703,7 @@ int st_hip_tensor_upload(void *device_ptr, const void *host_src, size_t bytes)
     PinnedBuffer stage;
     const size_t groups = (bytes + kUploadGroup - 1) / kUploadGroup, words_at = (bytes + 15) / 16 * 16;
     if (bytes == 0 || bytes > kUploadMost || reinterpret_cast<uintptr_t>(device_ptr) % 16 != 0 || host_memory(host_src) != HostMemory::kOrdinary ||
-        !kernel_may_access(device_ptr, bytes) || !pinned_acquire(words_at + groups * sizeof(unsigned), &stage))
+        !kernel_may_access(device_ptr, bytes, nullptr) || !pinned_acquire(words_at + groups * sizeof(unsigned), &stage))
         return st_hip_memcpy_h2d(device_ptr, host_src, bytes, nullptr);
     count_transfer(true, bytes);
     unsigned *const read = reinterpret_cast<unsigned *>(static_cast<unsigned char *>(stage.ptr) + words_at);
@@ -736,7 +736,7 @@ int st_hip_memcpy_d2h(void *host_dst, const void *device_src, size_t bytes, void
     count_transfer(false, bytes);
     PinnedBuffer stage;
     const bool staged = bytes <= kReadMost && host_memory(host_dst) == HostMemory::kOrdinary && pinned_acquire(bytes, &stage);
-    if (staged && reinterpret_cast<uintptr_t>(device_src) % 16 == 0 && kernel_may_access(device_src, bytes)) {
+    if (staged && reinterpret_cast<uintptr_t>(device_src) % 16 == 0 && kernel_may_access(device_src, bytes, as_stream(stream))) {
         const size_t pieces = (bytes + kCopyPiece - 1) / kCopyPiece;
         unsigned *const words = stage.words();
         std::memset(words, 0, pieces * sizeof(unsigned));

@@ -8,7 +8,7 @@
 #include <map>
 
 extern "C" {
-int stub_no_memory = 0, stub_device = 0;
+int stub_no_memory = 0, stub_device = 0, stub_stream_device = 0;
 unsigned long long stub_launches = 0, stub_frees = 0, stub_memory_used = 0, stub_memory_most = ~0ull;
 const char *stub_device_first = nullptr, *stub_device_end = nullptr;
 const void *stub_first_source = nullptr;  // of the runtime's copies
@@ -48,6 +48,7 @@ hipError_t hipHostMalloc(void **ptr, size_t bytes, unsigned)
 hipError_t hipHostFree(void *ptr) { std::free(ptr); return hipSuccess; }
 hipError_t hipStreamCreate(hipStream_t *stream) { *stream = reinterpret_cast<hipStream_t>(std::malloc(1)); return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t stream) { std::free(stream); return hipSuccess; }
+hipError_t hipStreamGetDevice(hipStream_t, hipDevice_t *device) { *device = stub_stream_device; return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *status) { *status = hipStreamCaptureStatusNone; return hipSuccess; }
 hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode *) { return hipSuccess; }

@@ -199,6 +199,21 @@ for at in (first, first + 4096):
     assert out == ["1", "True", "1", "True"] * 2
 
 
+def test_a_read_on_a_stream_of_another_device_is_left_to_the_runtime(stub):
+    """The kernel would run there and read memory of the current device."""
+    out = run(stub, """
+import numpy as np
+host, tensor, stream = np.zeros(4096, np.uint8), hip.TensorBuffer(4096), hip.Stream()
+device = ctypes.c_int.in_dll(stub, "stub_stream_device")
+for device.value in (0, 1):
+    before = launches.value
+    status = lib.st_hip_memcpy_d2h(host.ctypes.data, tensor.ptr, 4096, stream.ptr)
+    print(launches.value - before)
+print(status)
+""")
+    assert out == ["1", "0", "0"]
+
+
 def test_copies_past_the_end_of_a_tensor_are_refused(stub):
     """A tensor's block is larger than the tensor; what lies behind it is not the tensor's, now or when the block was another's."""
     out = run(stub, """
