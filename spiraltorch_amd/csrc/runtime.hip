@@ -337,15 +337,16 @@ bool passes_tensor_end(const void *ptr, size_t bytes)
     return tensor_range(ptr, bytes, &device) == TensorRange::kOutside;
 }
 
-// Whether a kernel on `stream` may access `bytes` from `ptr` on: memory of the stream's device, all of it in one allocation.  Whatever
-// else is left to the runtime's copy, which judges it.
+// Whether a kernel on `stream` may access `bytes` from `ptr` on: memory of the current device, which is the stream's as well, all of it in
+// one allocation.  Whatever else is left to the runtime's copy, which judges it.
 bool kernel_may_access(const void *ptr, size_t bytes, hipStream_t stream)
 {
-    int current = 0, device = 0;
-    if ((stream == nullptr ? hipGetDevice(&current) : hipStreamGetDevice(stream, &current)) != hipSuccess) {
+    int current = 0, device = 0, streams = 0;
+    if (hipGetDevice(&current) != hipSuccess || (stream != nullptr && hipStreamGetDevice(stream, &streams) != hipSuccess)) {
         (void)hipGetLastError();
         return false;
     }
+    if (stream != nullptr && streams != current) return false;
     const TensorRange range = tensor_range(ptr, bytes, &device);
     if (range != TensorRange::kElsewhere) return range == TensorRange::kInside && device == current;
     hipPointerAttribute_t attributes;

@@ -204,14 +204,14 @@ def test_a_read_on_a_stream_of_another_device_is_left_to_the_runtime(stub):
     out = run(stub, """
 import numpy as np
 host, tensor, stream = np.zeros(4096, np.uint8), hip.TensorBuffer(4096), hip.Stream()
-device = ctypes.c_int.in_dll(stub, "stub_stream_device")
-for device.value in (0, 1):
+current, device = (ctypes.c_int.in_dll(stub, name) for name in ("stub_device", "stub_stream_device"))
+for current.value, device.value in ((0, 0), (0, 1), (1, 0)):
     before = launches.value
     status = lib.st_hip_memcpy_d2h(host.ctypes.data, tensor.ptr, 4096, stream.ptr)
     print(launches.value - before)
 print(status)
 """)
-    assert out == ["1", "0", "0"]
+    assert out == ["1", "0", "0", "0"]
 
 
 def test_copies_past_the_end_of_a_tensor_are_refused(stub):
