@@ -1580,7 +1580,7 @@ __global__ __launch_bounds__(256) void attention_merge_splits_kernel(AttnArgs p,
     const size_t row = id / quads;
     const int d = static_cast<int>(id % quads) * 4;
     // Eight splits at a time, all their loads requested before the first is used (a plain loop over the splits is a
-    // chain of dependent memory round trips); splits past the end repeat the last one with weight zero.
+    // chain of dependent memory round trips); splits past the end load the last one again and are left out.
     // causal: the query tile of this row has (tile / r) + 1 chunks of keys; the planes beyond were never written
     const int splits = causal_r > 0 ? (static_cast<int>(row % static_cast<size_t>(p.S)) / kBQ) / causal_r + 1 : p.key_splits;
     const int last = splits - 1;
@@ -1606,8 +1606,8 @@ __global__ __launch_bounds__(256) void attention_merge_splits_kernel(AttnArgs p,
         }
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            // a split with no weight: 2^-inf = 0
-            const float w = s0 + j <= last ? __builtin_amdgcn_exp2f((ml[j].x - safe_top) * exp_scale) : 0.0f;
+            if (s0 + j > last) break;  // (a weight of zero would make NaN of an infinity)
+            const float w = __builtin_amdgcn_exp2f((ml[j].x - safe_top) * exp_scale);  // a split with no weight: 2^-inf = 0
             acc.x = fmaf(w, o[j].x, acc.x); acc.y = fmaf(w, o[j].y, acc.y);
             acc.z = fmaf(w, o[j].z, acc.z); acc.w = fmaf(w, o[j].w, acc.w);
             denom = fmaf(w, ml[j].y, denom);

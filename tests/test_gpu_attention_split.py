@@ -77,6 +77,27 @@ def test_wide_heads_the_pieces_cannot_carry(hip, contexts, seq, dim):
     assert not np.isfinite(got[1, 40:, dim - 1]).any() and np.isfinite(got[1, :40]).all() and np.isfinite(got[1, :, :dim - 1]).all()
 
 
+# keys in as many runs as are no multiple of eight (the merging loads eight at a time): shared keys and 128-row tiles, and on the f32
+# matrix cores (a large scale)
+@pytest.mark.parametrize("contexts,seq,dim,causal,biased,scale", [
+    (1, 700, 80, False, True, None), (1, 700, 128, True, True, None), (1, 890, 64, False, True, None), (2, 400, 96, False, False, None), (3, 1500, 64, True, False, None),
+    (4, 1700, 80, False, True, None), (1, 600, 64, False, True, 0.6), (1, 1200, 128, False, False, 0.5)])
+def test_infinite_values_in_the_last_run_of_keys(hip, contexts, seq, dim, causal, biased, scale):
+    scale = dim ** -0.5 if scale is None else scale
+    assert hip.attention_f32_launch_plan(contexts, seq, dim, causal, biased, scale=scale)["key_splits"] % 8 > 0
+    rng = np.random.default_rng(seq + dim)
+    q, k, v = (rng.normal(size=(contexts, seq, dim)).astype(np.float32) * 0.5 for _ in range(3))
+    z, a = (rng.normal(size=shape).astype(np.float32) * 0.5 if biased else None for shape in ((contexts, seq), (contexts, seq, seq)))
+    want = run(hip, q, k, v, scale, causal, z, a)
+    v[0, seq - 1, dim - 1], v[0, seq - 2, 0] = np.inf, -np.inf
+    got = run(hip, q, k, v, scale, causal, z, a)
+    assert np.abs(got[0, :, 1:dim - 1] - want[0, :, 1:dim - 1]).max() <= 2.0 ** -14  # either is within 2^-15 of the exact one (above)
+    sees = np.arange(seq) if causal else np.full(seq, seq)
+    assert (got[0, sees >= seq - 1, dim - 1] == np.inf).all() and np.isfinite(got[0, sees < seq - 1, dim - 1]).all()
+    assert (got[0, sees >= seq - 2, 0] == -np.inf).all() and np.isfinite(got[0, sees < seq - 2, 0]).all()
+    assert np.isfinite(got[1:]).all()
+
+
 def test_values_the_pieces_cannot_carry(hip):
     rng = np.random.default_rng(9)
     q, k, v = (rng.normal(size=(4, 300, 64)).astype(np.float32) for _ in range(3))
