@@ -1170,6 +1170,12 @@ int choose_conv_kernel(const ConvShape &shape, bool weight_aligned, bool out_ali
     return ST_HIP_CONV_KERNEL_RING;
 }
 
+// The tile kernels' offset table packs ky*dh and kx*dw into 16 bits each; a layer is refused or served whole, whichever kernel would take it.
+bool taps_fit(const ConvShape &shape)
+{
+    return (shape.kh - 1) * static_cast<long long>(shape.dil_h) <= 0x7fff && (shape.kw - 1) * static_cast<long long>(shape.dil_w) <= 0x7fff;
+}
+
 }  // namespace
 
 void set_conv_forced_family(int family) { g_forced_family.store(family, std::memory_order_relaxed); }
@@ -1218,7 +1224,7 @@ size_t conv2d_scratch_bytes(const ConvShape &shape, bool weight_aligned, bool ou
 bool launch_conv2d_strip_adjoint(const ConvShape &shape, const float *input, const float *forward_weight, float *out, hipStream_t stream,
                                  bool allow_slices, hipError_t *rc)
 {
-    if (shape.batch == 0 || shape.c_out == 0 || shape.oh == 0 || shape.ow == 0) return false;
+    if (shape.batch == 0 || shape.c_out == 0 || shape.oh == 0 || shape.ow == 0 || !taps_fit(shape)) return false;
     StripArgs strip;
     const bool out_aligned = (reinterpret_cast<uintptr_t>(out) & 15u) == 0;
     const int kernel = choose_conv_kernel(shape, true, out_aligned, g_forced_family.load(std::memory_order_relaxed), strip, allow_slices);
@@ -1249,10 +1255,7 @@ hipError_t launch_conv2d_f32(const ConvShape &shape, int activation, const float
     args.tiles_px = args.tiles_oc = 0;
     args.xcd_swizzle = 0;
     args.activation = activation;
-    // The offset table packs ky*dh and kx*dw into 16 bits each.
-    if ((shape.kh - 1) * static_cast<long long>(shape.dil_h) > 0x7fff ||
-        (shape.kw - 1) * static_cast<long long>(shape.dil_w) > 0x7fff)
-        return hipErrorInvalidValue;
+    if (!taps_fit(shape)) return hipErrorInvalidValue;
     const bool weight_aligned = (reinterpret_cast<uintptr_t>(weight) & 15u) == 0;
     const bool out_aligned = (reinterpret_cast<uintptr_t>(out) & 15u) == 0;
     if (scratch == kConvScratchStream && scratch_offset == 0 && conv2d_f32_split_preferred(shape, weight_aligned, out_aligned, false)) {
@@ -1339,9 +1342,7 @@ hipError_t launch_conv2d_adjoint_f32(const ConvShape &shape, const float *grad_o
     args.tiles_px = args.tiles_oc = 0;
     args.xcd_swizzle = 0;
     args.activation = ST_HIP_ACT_NONE;
-    if ((shape.kh - 1) * static_cast<long long>(shape.dil_h) > 0x7fff ||
-        (shape.kw - 1) * static_cast<long long>(shape.dil_w) > 0x7fff)
-        return hipErrorInvalidValue;
+    if (!taps_fit(shape)) return hipErrorInvalidValue;
     const bool vec = (args.K % 4 == 0) && ((reinterpret_cast<uintptr_t>(weight_ic_major) & 15u) == 0);
     if (shape.c_out > 64) return launch_tile<128, 64, 16, 4, 2, true>(args, vec, stream);
     return launch_tile<64, 64, 16, 2, 2, true>(args, vec, stream);

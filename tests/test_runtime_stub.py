@@ -241,6 +241,26 @@ print(lib.st_hip_memcpy_h2d(p, host.ctypes.data, 6000, None) == 0)  # whatever i
     assert out == ["True"] * len(out) and len(out) == 34
 
 
+@pytest.mark.parametrize("dilation,served", [(16383, True), (16384, False), (20000, False)])
+def test_a_layer_whose_taps_are_too_far_apart_is_refused_whole(stub, dilation, served):
+    """Forward and input gradient refuse the same layers, whichever kernel would run."""
+    out = run(stub, f"""
+pad = {dilation} - 20
+shape = (32, 64, 56, 96, 64, (3, 3), (1, 1), (1, pad), (1, {dilation}))
+assert hip.conv2d_output_hw(56, 96, *shape[5:]) == (56, 56)
+def refused(call, *operands):
+    try:
+        call(*operands)
+    except hip.HipErr:
+        return True
+    return False
+for family in ("auto", "tile", "strip"):
+    hip.conv2d_force_family(family)
+    print(refused(hip.conv2d_bias_act_f32_dev, *shape, 0, 1 << 20, 2 << 20, None, 3 << 20), refused(hip.conv2d_grad_input_f32_dev, *shape, 1 << 20, 2 << 20, 3 << 20))
+""")
+    assert out == [str(not served)] * 6
+
+
 def test_bf16_attention_launches_pass_their_check(stub):
     """Every grid the launchers of bf16 attention ask for passes the check made of it with the kernels' own decode."""
     out = run(stub, """
