@@ -969,7 +969,7 @@ __global__ __launch_bounds__(256) void conv2d_f32_direct_kernel(ConvArgs p)
 
 // The same for unit stride and dilation along x and a kernel width known at compile time: a thread owns four adjacent
 // pixels of an output row, so that a row segment of KW + 3 input values (one 16-byte load at any alignment plus KW - 1
-// single ones) feeds 4·KW·CO multiply-adds, and the weights (at most 144 KB) are read from LDS, every lane the same word.
+// single ones) feeds 4·KW·CO multiply-adds, and the weights (direct_weights_in_lds) are read from LDS, every lane the same word.
 // KH: the kernel height when it equals KW and is at most 5 (the loop over its rows is then unrolled, so that the loads of all rows of
 // a channel are in flight together: a thread's chain of load → multiply-add steps is what bounds this kernel), else 0.
 // GROUPS: wavefronts that share the input channels of 64 threads' worth of pixels and add their sums through LDS in a fixed order (the
@@ -1067,13 +1067,25 @@ __global__ __launch_bounds__(GROUPS == 1 ? 256 : 64 * GROUPS) void conv2d_f32_di
     }
 }
 
-constexpr size_t kDirectWeightBytes = 144 * 1024;  // the LDS, less the groups' sums (4 · 16 · 64 floats)
+size_t direct_row_items(const ConvShape &s) { return static_cast<size_t>(s.oh) * ((s.ow + 3) / 4); }  // threads with pixels of an image
+
+// Up to which size weights are read from LDS: all of it less the groups' sums (4 · 16 · 64 floats).  Beyond 64 KiB a workgroup has a compute
+// unit to itself, and loading the weights is worth it only with enough pixels beside them: at least 25 threads' worth, or, where
+// an image takes several workgroups, no nearly empty second one.  A thread a pixel without LDS / the better of the two below, µs: 5377×113, 4×7
+// -> 4, 7×7 1946 / 3150, 3924×259, 8×8 -> 4, 5×5 1585 / 2511, 3449×697, 8×11 -> 4, 3×3 3208 / 3349, 1930×182, 15×17 -> 4, 5×5 2094 / 2490;
+// 2664×772, 9×9 -> 4, 3×3 3109 / 2946, 832×447, 10×11 -> 1, 7×7 2729 / 1859, 283×340, 16×19 -> 2, 5×5 1713 / 450.
+bool direct_weights_in_lds(const ConvShape &s, size_t weight_bytes)
+{
+    if (weight_bytes <= 64 * 1024) return true;
+    const size_t items = direct_row_items(s), lanes = (items + 63) / 64 * 64;
+    return weight_bytes <= 144 * 1024 && (items <= 64 ? items >= 25 : 8 * items >= 5 * lanes);
+}
 
 template <int CO, int KW, int KH, int GROUPS>
 hipError_t launch_direct_groups(const ConvArgs &args, hipStream_t stream)
 {
     constexpr size_t kItems = GROUPS == 1 ? 256 : 64;
-    const size_t items = static_cast<size_t>(args.s.oh) * ((args.s.ow + 3) / 4);
+    const size_t items = direct_row_items(args.s);
     const dim3 grid(static_cast<unsigned>((items + kItems - 1) / kItems), static_cast<unsigned>(args.s.batch));
     const size_t lds_bytes = (static_cast<size_t>(CO) * args.K + (GROUPS == 1 ? 0 : GROUPS * CO * 4 * 64)) * sizeof(float);
     auto kernel = conv2d_f32_direct_rows_kernel<CO, KW, KH, GROUPS>;
@@ -1088,9 +1100,11 @@ hipError_t launch_direct_groups(const ConvArgs &args, hipStream_t stream)
 template <int CO, int KW>
 hipError_t launch_direct_rows(const ConvArgs &args, hipStream_t stream)
 {
-    const size_t workgroups = (static_cast<size_t>(args.s.oh) * ((args.s.ow + 3) / 4) + 255) / 256 * args.s.batch;
     // (Whole / shared are level once whole ones give the chip two workgroups a unit, 8×64, 256×256, 3×3 104 / 107, later where a channel is
-    // more work, the same with 7×7 taps 460 / 393; of 32 channels there is too little to share: 16×32, 128×128, 5×5 79 / 86.)
+    // more work, the same with 7×7 taps 460 / 393; of 32 channels there is too little to share: 16×32, 128×128, 5×5 79 / 86.  Workgroups'
+    // worth of threads that have pixels, that is: of an image of 14×14, 56 of 256 do.  600×512, 14×14 -> 3, 3×3 1041 / 352 µs, 600×1000 -> 4
+    // 3858 / 1037, 512×900, 12×12 -> 4 2129 / 639, 2048×96, 7×7 -> 3, 5×5 1514 / 370, 128×512, 64×64 -> 4 1052 / 1566.)
+    const size_t workgroups = direct_row_items(args.s) * args.s.batch / 256;
     const bool shared = (args.s.c_in >= 48 || args.s.c_in * args.s.kh > 160) && workgroups < (KW > 3 ? 2048 : 512);
     if (args.s.kh == KW && KW <= 5) return shared ? launch_direct_groups<CO, KW, KW, 4>(args, stream) : launch_direct_groups<CO, KW, KW, 1>(args, stream);
     return shared ? launch_direct_groups<CO, KW, 0, 4>(args, stream) : launch_direct_groups<CO, KW, 0, 1>(args, stream);
@@ -1112,7 +1126,7 @@ hipError_t launch_direct(const ConvArgs &args, hipStream_t stream)
 {
     const ConvShape &s = args.s;
     if (s.stride_w == 1 && s.dil_w == 1 && (s.kw == 1 || s.kw == 3 || s.kw == 5 || s.kw == 7) &&
-        static_cast<size_t>(CO) * args.K * sizeof(float) <= kDirectWeightBytes)
+        direct_weights_in_lds(s, static_cast<size_t>(CO) * args.K * sizeof(float)))
         return launch_direct_rows_for<CO>(args, stream);
     const dim3 grid(static_cast<unsigned>((args.spatial + 255) / 256), static_cast<unsigned>(args.s.batch));
     hipLaunchKernelGGL(conv2d_f32_direct_kernel<CO>, grid, dim3(256), 0, stream, args);

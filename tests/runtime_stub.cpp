@@ -54,8 +54,12 @@ hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *status) { *
 hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode *) { return hipSuccess; }
 hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
 static dim3 pushed_grid, pushed_block;
-hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t, hipStream_t)
+unsigned stub_grid = 0;            // of the last launch: workgroups along x
+unsigned long long stub_lds = 0;   // and its dynamic LDS
+hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t lds, hipStream_t)
 {
+    stub_grid = grid.x;
+    stub_lds = lds;
     pushed_grid = grid;
     pushed_block = block;
     return hipSuccess;

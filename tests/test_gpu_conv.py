@@ -159,6 +159,9 @@ def test_few_output_channels_over_many_pixels(hip, oracle, shape):
 @pytest.mark.parametrize("shape", [
     (16, 48, 64, 65, 3, (3, 3), (1, 1), (1, 1), (1, 1)), (16, 49, 64, 67, 1, (3, 3), (1, 1), (1, 1), (1, 1)), (5, 33, 115, 117, 2, (5, 5), (1, 1), (2, 2), (1, 1)),
     (3, 24, 150, 150, 4, (7, 7), (1, 1), (3, 3), (1, 1)), (4, 50, 130, 127, 2, (2, 1), (1, 1), (1, 0), (1, 1)), (16, 512, 64, 64, 4, (3, 3), (1, 1), (1, 1), (1, 1)),
+    # planes that leave most of a workgroup without pixels: a second one of 16 threads, one of 28, and too few for weights beyond 64 KiB
+    (410, 60, 10, 16, 4, (3, 3), (1, 1), (1, 1), (1, 1)), (470, 460, 14, 10, 4, (3, 3), (1, 1), (1, 1), (1, 1)), (2700, 110, 5, 5, 4, (7, 7), (1, 1), (3, 3), (1, 1)),
+    (340, 60, 13, 15, 4, (7, 7), (1, 1), (3, 3), (1, 1)), (330, 50, 20, 10, 2, (5, 5), (1, 1), (2, 2), (1, 1)),
     (16, 250, 64, 64, 3, (7, 7), (1, 1), (3, 3), (1, 1)), (16, 251, 64, 64, 3, (7, 7), (1, 1), (3, 3), (1, 1)), (8, 70, 100, 101, 3, (3, 5), (2, 1), (1, 2), (1, 1)),
 ])
 def test_few_output_channels_of_many_input_channels(hip, shape):

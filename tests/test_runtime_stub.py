@@ -241,6 +241,24 @@ print(lib.st_hip_memcpy_h2d(p, host.ctypes.data, 6000, None) == 0)  # whatever i
     assert out == ["True"] * len(out) and len(out) == 34
 
 
+# planes much smaller than a workgroup's threads, weights of up to 64 KiB and beyond, and either side of each line of the rule
+@pytest.mark.parametrize("batch,c_in,h,w,c_out,kernel,form", [
+    (600, 512, 14, 14, 3, 3, "shared"), (600, 1000, 14, 14, 4, 3, "shared"), (512, 900, 12, 12, 4, 3, "shared"), (2048, 96, 7, 7, 3, 5, "shared"), (128, 512, 64, 64, 4, 3, "whole"),
+    (127, 512, 64, 64, 4, 3, "shared"), (600, 47, 32, 32, 4, 3, "whole"), (1024, 64, 16, 32, 4, 3, "whole"), (1023, 64, 16, 32, 4, 3, "shared"), (5377, 113, 4, 7, 4, 7, "pixel"),
+    (3924, 259, 8, 8, 4, 5, "pixel"), (1024, 500, 8, 11, 4, 3, "pixel"), (1024, 500, 9, 9, 4, 3, "shared"), (1024, 500, 16, 16, 4, 3, "shared"), (1024, 500, 13, 17, 4, 3, "pixel"),
+    (1024, 500, 16, 19, 4, 3, "shared"), (1024, 455, 13, 17, 4, 3, "shared"), (64, 1025, 64, 64, 4, 3, "pixel"), (64, 1024, 64, 64, 4, 3, "shared")])
+def test_convolutions_onto_few_channels_take_the_form_for_their_planes(stub, batch, c_in, h, w, c_out, kernel, form):
+    out = run(stub, f"""
+lds = ctypes.c_ulonglong.in_dll(stub, "stub_lds")
+shape = ({batch}, {c_in}, {h}, {w}, {c_out}, ({kernel}, {kernel}), (1, 1), ({kernel // 2}, {kernel // 2}), (1, 1))
+assert hip.conv2d_planned_kernel(*shape) == "direct"
+hip.conv2d_bias_act_f32_dev(*shape, 0, 1 << 20, 2 << 20, None, 3 << 20)
+print(lds.value)
+""")
+    weights = 4 * c_out * c_in * kernel * kernel
+    assert int(out[0]) == {"pixel": 0, "whole": weights, "shared": weights + 4096 * c_out}[form]
+
+
 @pytest.mark.parametrize("dilation,served", [(16383, True), (16384, False), (20000, False)])
 def test_a_layer_whose_taps_are_too_far_apart_is_refused_whole(stub, dilation, served):
     """Forward and input gradient refuse the same layers, whichever kernel would run."""
