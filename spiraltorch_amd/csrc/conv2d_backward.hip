@@ -152,7 +152,8 @@ __global__ __launch_bounds__(256) void conv_grad_bias_partial_kernel(int planes,
 // The whole sum of a channel by one workgroup, in one launch: its sixteen wavefronts take the images' planes (planes cut in `parts`
 // where the images are fewer than they), and their sums are added in a fixed order.  Bound by what a compute unit reads, and by the
 // launch: two launches / this one, µs (a call takes the host about 4.4): 2×128 channels 6×6 6.6 / 4.4, 15×64 40×40 6.7 / 4.5, 32×32 56×56
-// 6.7 / 5.4, 32×128 56×56 11.0 / 9.5, 17×512 66×66 24.9 / 23.0.
+// 6.7 / 5.4, 32×128 56×56 11.0 / 9.5, 17×512 66×66 24.9 / 23.0.  A wavefront waits for an image before it asks for the next: of many, see
+// launch_conv2d_grad_bias_f32.
 __global__ __launch_bounds__(1024) void conv_grad_bias_channel_kernel(int batch, int c_out, int spatial, int parts, const float *grad_output,
                                                                       float scale, float *out)
 {
@@ -816,8 +817,12 @@ hipError_t launch_conv2d_grad_bias_f32(const ConvShape &shape, const float *grad
     const size_t planes = static_cast<size_t>(shape.batch) * shape.c_out;
     const int spatial = shape.oh * shape.ow;
     // (Few channels of more values leave compute units idle: 32×16 80×80 6.3 / 7.9 in one launch, 32×16 112×112 10.7 / 17.3, 32×64
-    // 112×112 17.5 / 20.1.)
-    if (planes > 0 && static_cast<size_t>(shape.batch) * spatial <= (128u << 10)) {
+    // 112×112 17.5 / 20.1.  Many images are a chain in each of a channel's wavefronts, where two launches spread the planes over the chip:
+    // 64×64 40×40 7.0 / 8.0, 112×64 28×28 6.9 / 12.3, 256×64 7×7 6.9 / 9.7, 512×16 7×7 6.8 / 16.7, 2048×64 7×7 34 / 101, 4096×16 4×4 27 / 90;
+    // 48×256 28×28 10.3 / 7.6, 112×64 20×20 7.1 / 5.7, 128×64 14×14 7.0 / 5.3.  Where the channels alone give every unit a workgroup the two
+    // read no faster: 256×256 10×10 13.0 / 10.4, 512×256 5×5 23.0 / 26.5; two a unit 1024×512 5×5 86 / 59, 2048×512 2×2 139 / 84.)
+    const int images_most = shape.c_out >= 512 ? shape.batch : shape.c_out >= 256 ? 256 : spatial <= 400 ? 128 : 48;
+    if (planes > 0 && shape.batch <= images_most && static_cast<size_t>(shape.batch) * spatial <= (128u << 10)) {
         const int parts = shape.batch >= 16 ? 1 : 16 / shape.batch;
         hipLaunchKernelGGL(conv_grad_bias_channel_kernel, dim3(static_cast<unsigned>(shape.c_out)), dim3(1024), 0, stream, shape.batch, shape.c_out, spatial, parts,
                            grad_output, scale, grad_bias);

@@ -241,6 +241,17 @@ print(lib.st_hip_memcpy_h2d(p, host.ctypes.data, 6000, None) == 0)  # whatever i
     assert out == ["True"] * len(out) and len(out) == 34
 
 
+@pytest.mark.parametrize("batch,c_out,side,launched", [
+    (48, 16, 28, 1), (49, 16, 28, 2), (128, 16, 20, 1), (129, 16, 20, 2), (128, 255, 7, 1), (129, 255, 7, 2), (48, 64, 52, 1), (49, 64, 21, 2), (256, 256, 7, 1), (257, 256, 7, 2),
+    (100, 256, 28, 1), (4096, 511, 4, 2), (4096, 512, 4, 1), (8192, 512, 4, 1), (8193, 512, 4, 2), (32, 64, 64, 1), (32, 64, 65, 2), (1, 3, 1, 1), (65536, 16, 1, 2)])
+def test_bias_gradients_of_many_images_are_spread_over_the_chip(stub, batch, c_out, side, launched):
+    out = run(stub, f"""
+hip.conv2d_grad_bias_f32_dev({batch}, 1, {side}, {side}, {c_out}, (1, 1), (1, 1), (0, 0), (1, 1), 1 << 20, 1.0, 2 << 20)
+print(launches.value)
+""")
+    assert out == [str(launched)]
+
+
 # planes much smaller than a workgroup's threads, weights of up to 64 KiB and beyond, and either side of each line of the rule
 @pytest.mark.parametrize("batch,c_in,h,w,c_out,kernel,form", [
     (600, 512, 14, 14, 3, 3, "shared"), (600, 1000, 14, 14, 4, 3, "shared"), (512, 900, 12, 12, 4, 3, "shared"), (2048, 96, 7, 7, 3, 5, "shared"), (128, 512, 64, 64, 4, 3, "whole"),
