@@ -174,7 +174,14 @@ __global__ __launch_bounds__(1024) void conv_grad_bias_channel_kernel(int batch,
 #pragma unroll
             for (int u = 0; u < 4; ++u) sums[u] += t[u];
         }
-        for (; i + 4 <= end; i += 256) sums[0] += *reinterpret_cast<const f32x4_a4 *>(src + i);
+        for (; i + 4 <= end; i += 256) {
+            // (The sums take turns: many small planes would all go into one.)
+            const f32x4_a4 next = sums[0] + *reinterpret_cast<const f32x4_a4 *>(src + i);
+            sums[0] = sums[1];
+            sums[1] = sums[2];
+            sums[2] = sums[3];
+            sums[3] = next;
+        }
         for (int e = i; e < min(i + 4, end); ++e) rest += src[e];  // (one lane's, the last quad's)
     }
     const f32x4_a4 all = (sums[0] + sums[1]) + (sums[2] + sums[3]);
@@ -816,13 +823,16 @@ hipError_t launch_conv2d_grad_bias_f32(const ConvShape &shape, const float *grad
     if (shape.c_out == 0) return hipSuccess;
     const size_t planes = static_cast<size_t>(shape.batch) * shape.c_out;
     const int spatial = shape.oh * shape.ow;
-    // (Few channels of more values leave compute units idle: 32×16 80×80 6.3 / 7.9 in one launch, 32×16 112×112 10.7 / 17.3, 32×64
-    // 112×112 17.5 / 20.1.  Many images are a chain in each of a channel's wavefronts, where two launches spread the planes over the chip:
-    // 64×64 40×40 7.0 / 8.0, 112×64 28×28 6.9 / 12.3, 256×64 7×7 6.9 / 9.7, 512×16 7×7 6.8 / 16.7, 2048×64 7×7 34 / 101, 4096×16 4×4 27 / 90;
-    // 48×256 28×28 10.3 / 7.6, 112×64 20×20 7.1 / 5.7, 128×64 14×14 7.0 / 5.3.  Where the channels alone give every unit a workgroup the two
-    // read no faster: 256×256 10×10 13.0 / 10.4, 512×256 5×5 23.0 / 26.5; two a unit 1024×512 5×5 86 / 59, 2048×512 2×2 139 / 84.)
-    const int images_most = shape.c_out >= 512 ? shape.batch : shape.c_out >= 256 ? 256 : spatial <= 400 ? 128 : 48;
-    if (planes > 0 && shape.batch <= images_most && static_cast<size_t>(shape.batch) * spatial <= (128u << 10)) {
+    // One launch or two (two / one, µs).  Many images are a chain in each of a channel's wavefronts, where two launches spread the planes over
+    // the chip: 64×64 40×40 7.0 / 8.0, 65×128 28×28 7.7 / 9.3, 112×64 28×28 6.9 / 12.3, 256×64 7×7 6.9 / 9.7, 512×16 7×7 6.8 / 17.0, 2048×64 7×7 34 / 101, 4096×16 4×4
+    // 27 / 90; 64×64 28×28 7.3 / 5.9, 112×64 20×20 7.0 / 5.6, 128×64 14×14 7.0 / 5.3.  Channels that give every unit a workgroup, or two, hide that: 256×256 10×10
+    // 13.0 / 11.1, 512×256 5×5 23.0 / 26.5, 1024×512 5×5 86 / 67, 2048×512 7×7 169 / 131.  Fewer of many values leave units idle: 32×16 112×112 10.7
+    // / 17.3, 48×64 50×50 7.1 / 8.5, 40×64 43×43 6.6 / 8.0, 32×64 61×61 7.3 / 8.5; 32×64 56×56 7.4 / 6.6, 16×64 90×90 9.8 / 8.8, 32×128 56×56 11.1
+    // / 9.8.  Planes of less than a quad add up in one sum: the error of 1024×512 1×1 would be 1.6e-7 of the sums (1.0e-7).
+    const int images_most = spatial < 4 ? 48 : shape.c_out >= 512 ? shape.batch : shape.c_out >= 256 ? 256 : spatial <= 400 ? 128 : spatial <= 800 ? 64 : 48;
+    const bool all = shape.batch <= 16 || shape.c_out >= 256 || (shape.c_out >= 128 && shape.batch <= 32);
+    const size_t values_most = all ? 128u << 10 : shape.batch <= 32 ? 104u << 10 : 64u << 10;
+    if (planes > 0 && shape.batch <= images_most && static_cast<size_t>(shape.batch) * spatial <= values_most) {
         const int parts = shape.batch >= 16 ? 1 : 16 / shape.batch;
         hipLaunchKernelGGL(conv_grad_bias_channel_kernel, dim3(static_cast<unsigned>(shape.c_out)), dim3(1024), 0, stream, shape.batch, shape.c_out, spatial, parts,
                            grad_output, scale, grad_bias);

@@ -450,3 +450,18 @@ def test_grad_bias_of_a_channel(hip, batch, c_out, oh, ow):
     # any order of f32 additions: at most one rounding a term of half an ulp of the sum of magnitudes
     bound = 2.0 ** -24 * batch * oh * ow * np.abs(terms).sum(axis=(0, 2)) + 1e-30
     assert (np.abs(got[:c_out] - 0.5 * terms.sum(axis=(0, 2))) <= bound).all()
+
+
+# the sizes above, and either side of the rule's lines: many images, channels for every unit, planes of less than a quad
+@pytest.mark.parametrize("batch,c_out,oh,ow", [(1, 3, 1, 1), (1, 5, 7, 9), (3, 2, 5, 13), (5, 17, 33, 31), (15, 4, 9, 9), (16, 3, 56, 56), (17, 3, 31, 33), (33, 2, 1, 3),
+                                               (1, 2, 256, 512), (2, 2, 257, 256), (16, 2, 64, 128), (16, 2, 91, 91), (32, 128, 60, 61), (32, 1, 64, 64), (48, 2, 29, 31), (49, 3, 29, 31),
+                                               (128, 2, 19, 21), (129, 2, 19, 21), (256, 256, 5, 7), (300, 256, 5, 7), (700, 512, 3, 3), (48, 512, 1, 3), (50, 512, 1, 2)])
+def test_grad_bias_takes_every_value_once(hip, batch, c_out, oh, ow):
+    rng = np.random.default_rng(batch * oh + ow)
+    g = rng.integers(1, 60, batch * c_out * oh * ow).astype(np.float32)  # sums below 2^24: exact in any order, and no value is zero
+    d_g, d_gb = hip.DeviceBuffer.from_array(g), hip.DeviceBuffer.from_array(np.full(c_out + 8, 7.5, np.float32))
+    hip.conv2d_grad_bias_f32_dev(batch, 1, oh, ow, c_out, (1, 1), (1, 1), (0, 0), (1, 1), d_g, 0.5, d_gb)
+    hip.device_synchronize()
+    got = d_gb.to_array(np.float32, c_out + 8)
+    assert (got[c_out:] == 7.5).all()
+    assert (got[:c_out] == 0.5 * g.astype(np.float64).reshape(batch, c_out, oh * ow).sum(axis=(0, 2))).all()

@@ -242,8 +242,9 @@ print(lib.st_hip_memcpy_h2d(p, host.ctypes.data, 6000, None) == 0)  # whatever i
 
 
 @pytest.mark.parametrize("batch,c_out,side,launched", [
-    (48, 16, 28, 1), (49, 16, 28, 2), (128, 16, 20, 1), (129, 16, 20, 2), (128, 255, 7, 1), (129, 255, 7, 2), (48, 64, 52, 1), (49, 64, 21, 2), (256, 256, 7, 1), (257, 256, 7, 2),
-    (100, 256, 28, 1), (4096, 511, 4, 2), (4096, 512, 4, 1), (8192, 512, 4, 1), (8193, 512, 4, 2), (32, 64, 64, 1), (32, 64, 65, 2), (1, 3, 1, 1), (65536, 16, 1, 2)])
+    (64, 16, 28, 1), (65, 16, 28, 2), (48, 16, 36, 1), (49, 16, 36, 2), (128, 16, 20, 1), (129, 16, 20, 2), (128, 255, 7, 1), (129, 255, 7, 2), (64, 64, 29, 2), (256, 256, 7, 1), (257, 256, 7, 2),
+    (100, 256, 28, 1), (4096, 511, 4, 2), (4096, 512, 4, 1), (8192, 512, 4, 1), (8193, 512, 4, 2), (16, 64, 90, 1), (16, 64, 91, 2), (32, 64, 57, 1), (32, 64, 58, 2), (33, 64, 44, 1), (33, 64, 45, 2),
+    (32, 128, 64, 1), (32, 128, 65, 2), (33, 128, 50, 2), (48, 255, 36, 1), (48, 255, 37, 2), (48, 512, 1, 1), (49, 512, 1, 2), (1, 3, 1, 1), (65536, 16, 1, 2)])
 def test_bias_gradients_of_many_images_are_spread_over_the_chip(stub, batch, c_out, side, launched):
     out = run(stub, f"""
 hip.conv2d_grad_bias_f32_dev({batch}, 1, {side}, {side}, {c_out}, (1, 1), (1, 1), (0, 0), (1, 1), 1 << 20, 1.0, 2 << 20)
