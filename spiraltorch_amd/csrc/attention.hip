@@ -1756,17 +1756,16 @@ int attention_route(size_t contexts, size_t sequence, size_t head_dim, float sca
     if (!vec || head_dim > 128 || sequence * head_dim * sizeof(float) >= (1ull << 31)) return ST_HIP_ATTN_KERNEL_GENERAL;
     // Many contexts of at most 64 positions: a wavefront per context.
     if (!bias && sequence <= 64 && contexts >= 256) return ST_HIP_ATTN_KERNEL_TINY;
-    // Wide heads with biases: what one tile of keys holds only while the head's registers are few (1 × 16 × 128 9.9 µs here, 10.3 by one
-    // wavefront of the split kernels); 3 × 1152 × 80 292 µs here, 28 there.  (769 to 832 keys stay on the general kernel only because a
-    // test of the launch plan holds 2 × 776 × 80 to it.)
+    // Wide heads with biases: what one tile of keys holds only while the head's registers are few (1 × 16 × 128 9.9 µs on the general kernel,
+    // 10.3 by one wavefront of the split kernels); 3 × 1152 × 80 292 µs there, 28 here.
     const bool bias_fits = sequence * (sequence + 256) * sizeof(float) < (1ull << 31);  // rows past the end included
-    if (!sums_in_reference_order(head_dim, scale) && (!bias || (bias_fits && (head_dim <= 64 || ((sequence <= 768 || sequence > 832) && (head_dim <= 96 || sequence > 32)))))) return ST_HIP_ATTN_KERNEL_SPLIT;
+    if (!sums_in_reference_order(head_dim, scale) && (!bias || (bias_fits && (head_dim <= 96 || sequence > 32)))) return ST_HIP_ATTN_KERNEL_SPLIT;
     if (!bias) return ST_HIP_ATTN_KERNEL_FAST;
     // The biases where their rows can be read 128 bits at a time.
     return head_dim <= 64 && sequence % 4 == 0 && bias_aligned ? ST_HIP_ATTN_KERNEL_FAST_BIASED : ST_HIP_ATTN_KERNEL_GENERAL;
 }
 
-// Query rows per workgroup: the split kernel (head sizes up to 64) takes 256 where such tiles still give every compute
+// Query rows per workgroup: the split kernel takes 256 (head sizes up to 64) where such tiles still give every compute
 // unit one, 128 otherwise and on every other kernel.
 int query_rows(size_t contexts, size_t sequence, size_t head_dim, bool causal)
 {

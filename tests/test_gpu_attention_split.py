@@ -57,7 +57,7 @@ def test_against_float64(hip, contexts, seq, dim, causal, biased):
 # unsplit, in pairs and with their keys cut, 32-key stages cut short; biases up to the longest that are served.
 @pytest.mark.parametrize("contexts,seq,causal,biased", [
     (1, 1, False, False), (2, 31, True, False), (3, 33, False, True), (1, 128, True, True), (5, 129, False, False), (2, 255, True, False), (7, 257, False, True),
-    (1, 300, True, False), (1, 768, False, True), (1, 833, True, True), (3, 1001, False, True), (16, 500, True, False), (40, 225, False, False), (70, 289, True, False), (33, 290, True, True)])
+    (1, 300, True, False), (1, 768, False, True), (1, 769, False, True), (2, 776, True, True), (1, 800, False, True), (1, 832, True, True), (1, 833, True, True), (3, 1001, False, True), (16, 500, True, False), (40, 225, False, False), (70, 289, True, False), (33, 290, True, True)])
 @pytest.mark.parametrize("dim", [68, 80, 96, 100, 128])
 def test_wide_heads_against_float64(hip, contexts, seq, dim, causal, biased):
     assert hip.attention_f32_launch_plan(contexts, seq, dim, causal, biased, scale=dim ** -0.5)["kernel"] == "split" or (dim > 96 and biased and seq <= 32)

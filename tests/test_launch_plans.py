@@ -67,7 +67,9 @@ def test_the_attention_plan_knows_the_scale():
     assert plan(128, 2048, 62, True)["kernel"] == "general" and plan(128, 2048, 62, True)["workgroups"] == 128 * 16
     # biases: rows the f32 kernel cannot read 16 bytes at a time, larger heads
     assert plan(2, 777, 64, False, True, scale=0.6)["kernel"] == "general" and plan(2, 776, 64, False, True, scale=0.6)["kernel"] == "fast_biased"
-    assert plan(2, 777, 64, False, True, scale=-0.5)["kernel"] == "split" and plan(2, 776, 80, False, True, scale=0.1)["kernel"] == "general"
+    assert plan(2, 777, 64, False, True, scale=-0.5)["kernel"] == "split" and plan(2, 776, 80, False, True, scale=0.6)["kernel"] == "general"
+    for seq, dim in itertools.product((33, 500, 700, 768, 769, 776, 800, 832, 833, 900, 2000), (68, 80, 96, 100, 128)):  # one kernel for all lengths
+        assert plan(2, seq, dim, False, True, scale=0.1)["kernel"] == "split", (seq, dim)
     assert plan(300, 64, 64, True, scale=0.6)["kernel"] == "tiny" and plan(300, 64, 64, True, scale=0.125)["kernel"] == "tiny"
     for contexts, seq, dim, causal, biased in itertools.product(CONTEXTS, SEQUENCES, (32, 64, 128), (False, True), (False, True)):
         got = plan(contexts, seq, dim, causal, biased, scale=0.9)
