@@ -98,6 +98,33 @@ def test_infinite_values_in_the_last_run_of_keys(hip, contexts, seq, dim, causal
     assert np.isfinite(got[1:]).all()
 
 
+# shared keys in one run and in several, 128-row tiles; every other pair masked, the last keys of all queries, the keys of a whole run, all keys of
+# some queries (zeros, as on the general kernel)
+@pytest.mark.parametrize("contexts,seq,causal", [(2, 150, False), (1, 500, True), (1, 700, False), (16, 500, False), (33, 290, True), (4, 1200, False)])
+@pytest.mark.parametrize("dim", [64, 80, 128])
+@pytest.mark.parametrize("masked", [-np.inf, np.finfo(np.float32).min])
+def test_masked_pairs(hip, contexts, seq, dim, causal, masked):
+    assert hip.attention_f32_launch_plan(contexts, seq, dim, causal, True, scale=dim ** -0.5)["kernel"] == "split"
+    rng = np.random.default_rng(seq + dim)
+    q, k, v = (rng.normal(size=(contexts, seq, dim)).astype(np.float32) for _ in range(3))
+    zb, ab = (rng.normal(0, 0.5, shape).astype(np.float32) for shape in ((contexts, seq), (contexts, seq, seq)))
+    ab[:, 0::2, 1::2] = ab[:, 1::2, 0::2] = masked
+    zb[:, seq - 20:] = masked
+    if seq > 260:
+        zb[:, 128:256] = masked
+    nothing = np.zeros(seq, bool)
+    if masked == -np.inf:
+        nothing[[3, 40, seq - 2]] = True
+        ab[:, nothing] = -np.inf
+    got = run(hip, q, k, v, dim ** -0.5, causal, zb, ab)
+    assert (got[:, nothing] == 0.0).all()
+    for c in sorted({0, contexts - 1}):
+        with np.errstate(invalid="ignore"):
+            want = exact(q[c], k[c], v[c], float(np.float32(dim ** -0.5)), causal, zb[c], ab[c])
+        error = (got[c] - want)[~nothing]
+        assert np.sqrt(np.mean(error ** 2)) <= 2.0 ** -20 * np.sqrt(np.mean(want[~nothing] ** 2)) and np.abs(error).max() <= 2.0 ** -15
+
+
 def test_values_the_pieces_cannot_carry(hip):
     rng = np.random.default_rng(9)
     q, k, v = (rng.normal(size=(4, 300, 64)).astype(np.float32) for _ in range(3))
