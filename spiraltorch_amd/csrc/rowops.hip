@@ -833,7 +833,9 @@ __global__ __launch_bounds__(256) void copy_from_pinned_kernel(size_t bytes, con
     else
         for (size_t e = at; e < bytes; ++e) device[e] = pinned[e];
     if (read == nullptr) return;
-    __syncthreads();  // (waits for this workgroup's memory accesses)
+    // A barrier does not wait for memory.  What has been stored has been read; the wait is for a copy that would hold values back.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
     if (threadIdx.x == 0) __hip_atomic_store(&read[blockIdx.x], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
