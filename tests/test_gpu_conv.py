@@ -181,6 +181,10 @@ def test_few_output_channels_of_many_input_channels(hip, shape):
     assert (np.abs(got - exact) <= bound).all()
     got = run(hip, *shape, 1, x, wt, b)
     assert (np.abs(got - np.maximum(exact, 0.0)) <= bound).all()
+    # whole numbers whose sums f32 holds (81·K < 2^24): every product once, nothing else
+    x, wt, b = rng.integers(1, 10, x.size).astype(np.float32), rng.integers(1, 10, wt.size).astype(np.float32), rng.integers(-9, 10, c_out).astype(np.float32)
+    X, W = torch.from_numpy(x).double().view(batch, c_in, h, w), torch.from_numpy(wt).double().view(c_out, c_in, *kernel)
+    assert (run(hip, *shape, 0, x, wt, b) == torch.nn.functional.conv2d(X, W, torch.from_numpy(b).double(), stride, padding, dilation).numpy().ravel()).all()
 
 
 G33 = ((3, 3), (1, 1), (1, 1), (1, 1))

@@ -525,6 +525,12 @@ def test_column_sums_from_threads_sharing_the_null_stream(hip):
                 # f32 sums in any order: at most rows roundings of half an ulp of the sum of magnitudes each
                 if np.abs(d_s.to_array(np.float32, cols) - want).max() > 2.0 ** -24 * rows * np.abs(x).reshape(rows, cols).sum(axis=0).max():
                     failures.append((index, round_))
+                x = rng.integers(1, 60, rows * cols).astype(np.float32)  # sums that f32 holds: every value once
+                d_x = hip.DeviceBuffer.from_array(x)
+                hip.sum_axis0_f32_dev(rows, cols, d_x, 1.0, d_s)
+                hip.device_synchronize()
+                if (d_s.to_array(np.float32, cols) != x.astype(np.float64).reshape(rows, cols).sum(axis=0)).any():
+                    failures.append((index, round_, "whole numbers"))
         except Exception as err:  # surfaced below
             failures.append(err)
 
