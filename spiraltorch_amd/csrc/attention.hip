@@ -314,7 +314,7 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(AttnArgs p)
 }
 
 // -------------------------------------------------------------------------------------------------
-// Fast path on the f32 matrix cores (head sizes above 64, and calls whose logits are large: see sums_in_reference_order):
+// Fast path on the f32 matrix cores (calls whose logits are large: see sums_in_reference_order; with biases head sizes up to 64):
 // head_dim a multiple of 4, 16-byte aligned operands; BIAS adds z_bias / attn_bias where their rows can
 // be read 128 bits at a time (sequence a multiple of 4), otherwise biased calls take the general kernel above.
 //

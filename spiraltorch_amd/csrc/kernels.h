@@ -270,9 +270,10 @@ HostMemory host_memory(const void *host);
 // The most that copies go through pinned memory with, where that is faster than the runtime's copy: operands of a host call (µs of
 // relu(A·B + bias) with square operands of 0.34, 0.67, 1, 2, 4 and 16 MiB and a result of the same size, staged up to 0.5 / 1 / 4 MiB: 73 / 73 / 72,
 // 114 / 111 / 111, 135 / 136 / 136, 252 / 252 / 269, 415 / 411 / 443, 2035 / 2043 / 2040; 88, 121, 156, 291, 539, 2330 without staging), its results
-// (2048×2048 of one term 585 against 1002), and st_hip_memcpy_d2h (1 KiB 13 against 21, 16 KiB 13 against 27, 256 KiB 19.5 against 20.4, 512 KiB
-// 29.5 against 30.9, 2 MiB 110 against 119; by a kernel that says what has arrived, without waiting for the stream; a read is staged whole, so that more than the ring's size would be held for it alone).  A
-// result goes through a ring: pinned memory takes 0.25 to 0.5 ms a MiB to allocate, and is then held.
+// (2048×2048 of one term 585 against 1002), and st_hip_memcpy_d2h (1 KiB 21, 16 KiB 27, 256 KiB 20.4, 512 KiB 30.9, 2 MiB 119 without staging;
+// 13.2, 13.8, 20.5, 30.4, 113 by the runtime into pinned memory; 8.4, 11.9, 19.0, 30.3, 96 by a kernel that says what has arrived, without
+// waiting for the stream; a read is staged whole, so that more than the ring's size would be held for it alone).  A result goes through
+// a ring: pinned memory takes 0.25 to 0.5 ms a MiB to allocate, and is then held.
 constexpr size_t kUploadMost = 512u << 10, kDownloadMost = 16u << 20, kDownloadRing = 2u << 20, kReadMost = kDownloadRing;
 // device[0, bytes) = pinned[0, bytes) by a kernel (device on a 16-byte boundary), and back: the piece of kCopyPiece bytes with
 // number p is in host memory when word p of `arrived` (host memory, cleared before) is not zero.
