@@ -2531,11 +2531,26 @@ hipError_t launch_transpose_u16(size_t rows, size_t cols, const uint16_t *in, ui
 // row-major, none more (448×383×2566 56 -> 12 µs, 16×663×329 16 -> 6.1).  It stays where a pass over B is most of the work: a row-major B
 // of more than 14 million values or 16384 columns for up to 64 rows (16×8192×8190 39 / 68 µs general / copies, 1×8191×8191 65 / 82,
 // 4×50257×100 11 / 26; at 16×4096×4097 they are level), and k beyond 16384, which it cuts over the chip (33×100×50257 34 / 59, packed 49 / 59).
+// A row-major B under 65 to 127 rows, one row of tiles: by the estimates below, fitted to 615 drawn products of up to 60000 columns and 130
+// million values of B (14 and 8 % in the rms).  General / copies: 65×8191×8191 78 / 97 µs, 101×6272×12491 57 / 96, 92×52864×1281 48 / 82,
+// 100×51598×218 24 / 31; 65×8191×3001 51 / 39, 127×6000×4001 48 / 37, 80×30000×1001 58 / 43, 80×20000×2001 95 / 52.  (Of the 615 the rule
+// leaves 5 more than 3 % slower than the general kernel, 92 with the copies always.)
 static bool padding_pays(size_t m, size_t n, size_t k, bool rhs_packed)
 {
     if (k <= 64) return false;
     if (m >= 128 && n >= 128 && 2.0 * m * n * k >= 2e9) return true;
-    return k <= 16384 && (rhs_packed || m > 64 || (n <= 16384 && n * k <= 14'000'000));
+    if (k > 16384) return false;
+    if (rhs_packed || m >= 128) return true;
+    const double values = static_cast<double>(n) * static_cast<double>(k) / 1e6, columns = static_cast<double>(n) / 1e4;
+    if (m <= 64) return n <= 16384 && values <= 14.0;
+    const size_t slices = general_k_slices(m, n, k), workgroups = (n + 127) / 128 * slices;
+    const double steps = static_cast<double>(((k + 31) / 32 + slices - 1) / slices), rounds = static_cast<double>((workgroups + 511) / 512);
+    const bool lines = n % 64 == 0;  // rows of B that start on cache lines
+    const double step_us = workgroups <= 256 ? (lines ? 0.72 : 0.94) : rounds * (lines ? 0.50 : 0.97);
+    const double sums_us = slices > 1 ? 2.3 + 1.17e-6 * static_cast<double>(slices * m * n) : 0.0;
+    const double general_us = 13.3 + steps * step_us + sums_us + 0.29 * values + 0.35 * columns;
+    const double copies_us = 6.7 + (lines ? 0.94 : n % 8 == 0 ? 1.15 : 1.23) * values + 0.27 * std::max(values - 50.0, 0.0) + 1.89 * columns + 0.84e-3 * static_cast<double>(k);
+    return copies_us < 0.95 * general_us;
 }
 
 hipError_t launch_gemm_bf16(size_t m, size_t n, size_t k, const uint16_t *lhs, const uint16_t *rhs,

@@ -46,7 +46,9 @@ for fail in (1, 0):
 
 # around the bounds on what is copied for up to 64 rows, and on k
 @pytest.mark.parametrize("m,n,k,launched", [(16, 663, 329, 2), (100, 1001, 300, 2), (64, 16384, 850, 2), (64, 16392, 65, 1), (64, 16384, 855, 1), (65, 40, 16383, 2),
-                                            (3000, 40, 16385, 1), (20, 40, 63, 1)])
+                                            (3000, 40, 16385, 1), (20, 40, 63, 1),
+                                            # one row of tiles: the general kernel where it reads a large B in less time than a pass over it takes
+                                            (100, 51598, 218, 1), (92, 48000, 686, 1), (80, 33600, 736, 1), (80, 30000, 1001, 2), (128, 51598, 218, 2)])
 def test_products_of_any_k_go_on_without_room_for_padded_copies(stub, m, n, k, launched):
     """A k that is no multiple of 64 is padded in scratch memory where that pays; without any to be had, the general kernel takes it as it
     is (a k it would cut over the chip needs scratch there too, as ever)."""
