@@ -832,15 +832,16 @@ hipError_t launch_conv2d_grad_bias_f32(const ConvShape &shape, const float *grad
     const int images_most = spatial < 4 ? 48 : shape.c_out >= 512 ? shape.batch : shape.c_out >= 256 ? 256 : spatial <= 400 ? 128 : spatial <= 800 ? 64 : 48;
     const bool all = shape.batch <= 16 || shape.c_out >= 256 || (shape.c_out >= 128 && shape.batch <= 32);
     const size_t values_most = all ? 128u << 10 : shape.batch <= 32 ? 104u << 10 : 64u << 10;
-    if (planes > 0 && shape.batch <= images_most && static_cast<size_t>(shape.batch) * spatial <= values_most) {
+    const bool one = planes > 0 && shape.batch <= images_most && static_cast<size_t>(shape.batch) * spatial <= values_most;
+    void *workspace = nullptr;
+    hipError_t rc = one ? hipSuccess : stream_workspace(stream, (planes ? planes : 1) * sizeof(float), &workspace);
+    if (rc != hipSuccess && !(planes > 0 && scratch_unavailable(rc))) return rc;
+    if (workspace == nullptr) {  // (the one launch needs no scratch)
         const int parts = shape.batch >= 16 ? 1 : 16 / shape.batch;
         hipLaunchKernelGGL(conv_grad_bias_channel_kernel, dim3(static_cast<unsigned>(shape.c_out)), dim3(1024), 0, stream, shape.batch, shape.c_out, spatial, parts,
                            grad_output, scale, grad_bias);
         return hipGetLastError();
     }
-    void *workspace = nullptr;
-    hipError_t rc = stream_workspace(stream, (planes ? planes : 1) * sizeof(float), &workspace);
-    if (rc != hipSuccess) return rc;
     float *partial = static_cast<float *>(workspace);
     if (planes > 0) {
         hipLaunchKernelGGL(conv_grad_bias_partial_kernel, dim3(static_cast<unsigned>((planes + 3) / 4)), dim3(256), 0, stream,

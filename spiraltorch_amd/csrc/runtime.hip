@@ -338,7 +338,7 @@ bool passes_tensor_end(const void *ptr, size_t bytes)
 }
 
 // Whether a kernel on `stream` may access `bytes` from `ptr` on: memory of the current device, which is the stream's as well, all of it in
-// one allocation.  Whatever else is left to the runtime's copy, which judges it.
+// one allocation.  Whatever else is left to the runtime's copy, which takes or refuses it.
 bool kernel_may_access(const void *ptr, size_t bytes, hipStream_t stream)
 {
     int current = 0, device = 0, streams = 0;
