@@ -264,8 +264,8 @@ int st_hip_attention_f32(size_t contexts, size_t sequence, size_t head_dim, floa
  * additionally walks the whole grid: `items` distinct work items decoded, `items_expected` what the shape calls for,
  * `out_of_range` workgroups that would read outside the operands and `duplicates` items decoded twice (both must be
  * 0), `consistent` the launcher's own check.  Operands are taken to be 16-byte aligned.  The scale decides as well: head
- * sizes up to 128 run as products of three exact bf16 pieces per value (ST_HIP_ATTN_KERNEL_SPLIT; above 96
- * not for 21 to 32 keys, with biases not for fewer either) while |scale|·sqrt(head_dim) is at most 4, on the f32 matrix cores above.
+ * sizes up to 128 run as products of three exact bf16 pieces per value (ST_HIP_ATTN_KERNEL_SPLIT; with biases
+ * head sizes above 96 from 33 keys on) while |scale|·sqrt(head_dim) is at most 4, on the f32 matrix cores above.
  * st_hip_attention_f32_launch_plan assumes the usual 1/sqrt(head_dim) and names both FAST (with biases FAST_BIASED, which for head
  * sizes above 64 always stands for SPLIT); st_hip_attention_f32_scaled_launch_plan takes the scale and tells them apart.  No reference counterpart (the reference's CPU loop, crates/st-tensor/src/pure.rs:11845-11919, has no launch
  * geometry). */

@@ -1770,12 +1770,10 @@ int attention_route(size_t contexts, size_t sequence, size_t head_dim, float sca
     if (!vec || head_dim > 128 || sequence * head_dim * sizeof(float) >= (1ull << 31)) return ST_HIP_ATTN_KERNEL_GENERAL;
     // Many contexts of at most 64 positions: a wavefront per context.
     if (!bias && sequence <= 64 && contexts >= 256) return ST_HIP_ATTN_KERNEL_TINY;
-    // Heads above 96 values and one tile of keys, a chain in one wavefront here: with biases 1 × 16 × 128 9.9 µs on the general kernel, 10.3 here,
-    // without on the f32 matrix cores 8 × 32 × 128 10.6 / 11.6, 128 × 24 × 128 10.8 / 11.2, 8 × 16 × 128 10.5 / 10.2; 40 × 33 × 128 14.6 / 11.9, biased
-    // 3 × 1152 × 80 292 / 28.
-    const bool one_tile = head_dim > 96 && sequence <= 32 && (bias || sequence > 20);
+    // Wide heads with biases: what one tile of keys holds only while the head's registers are few (1 × 16 × 128 9.9 µs on the general kernel,
+    // 10.3 by one wavefront of the split kernels); 3 × 1152 × 80 292 µs there, 28 here.
     const bool bias_fits = sequence * (sequence + 256) * sizeof(float) < (1ull << 31);  // rows past the end included
-    if (!sums_in_reference_order(head_dim, scale) && !one_tile && (!bias || bias_fits)) return ST_HIP_ATTN_KERNEL_SPLIT;
+    if (!sums_in_reference_order(head_dim, scale) && (!bias || (bias_fits && (head_dim <= 96 || sequence > 32)))) return ST_HIP_ATTN_KERNEL_SPLIT;
     if (!bias) return ST_HIP_ATTN_KERNEL_FAST;
     // The biases where their rows can be read 128 bits at a time.
     return head_dim <= 64 && sequence % 4 == 0 && bias_aligned ? ST_HIP_ATTN_KERNEL_FAST_BIASED : ST_HIP_ATTN_KERNEL_GENERAL;

@@ -70,9 +70,6 @@ def test_the_attention_plan_knows_the_scale():
     assert plan(2, 777, 64, False, True, scale=-0.5)["kernel"] == "split" and plan(2, 776, 80, False, True, scale=0.6)["kernel"] == "general"
     for seq, dim in itertools.product((33, 500, 700, 768, 769, 776, 800, 832, 833, 900, 2000), (68, 80, 96, 100, 128)):  # one kernel for all lengths
         assert plan(2, seq, dim, False, True, scale=0.1)["kernel"] == "split", (seq, dim)
-    assert [plan(8, seq, dim, False, biased, scale=0.1)["kernel"] for seq, dim, biased in ((20, 128, False), (21, 128, False), (32, 100, False), (33, 128, False), (32, 96, False),
-                                                                                           (20, 128, True), (32, 100, True), (33, 100, True), (32, 96, True))] == \
-        ["split", "fast", "fast", "split", "split", "general", "general", "split", "split"]
     assert plan(300, 64, 64, True, scale=0.6)["kernel"] == "tiny" and plan(300, 64, 64, True, scale=0.125)["kernel"] == "tiny"
     for contexts, seq, dim, causal, biased in itertools.product(CONTEXTS, SEQUENCES, (32, 64, 128), (False, True), (False, True)):
         got = plan(contexts, seq, dim, causal, biased, scale=0.9)
