@@ -1771,7 +1771,8 @@ int attention_route(size_t contexts, size_t sequence, size_t head_dim, float sca
     // Many contexts of at most 64 positions: a wavefront per context.
     if (!bias && sequence <= 64 && contexts >= 256) return ST_HIP_ATTN_KERNEL_TINY;
     // Wide heads with biases: what one tile of keys holds only while the head's registers are few (1 × 16 × 128 9.9 µs on the general kernel,
-    // 10.3 by one wavefront of the split kernels); 3 × 1152 × 80 292 µs there, 28 here.
+    // 10.3 by one wavefront of the split kernels); 3 × 1152 × 80 292 µs there, 28 here.  Without biases one kernel for all lengths: 8 × 16 × 128 10.5 µs on
+    // the f32 matrix cores, 10.2 here, 8 × 32 × 128 10.6 and 11.6, 40 × 33 × 128 14.6 and 11.9.
     const bool bias_fits = sequence * (sequence + 256) * sizeof(float) < (1ull << 31);  // rows past the end included
     if (!sums_in_reference_order(head_dim, scale) && (!bias || (bias_fits && (head_dim <= 96 || sequence > 32)))) return ST_HIP_ATTN_KERNEL_SPLIT;
     if (!bias) return ST_HIP_ATTN_KERNEL_FAST;
